@@ -238,11 +238,17 @@ void copy_blocks_peer(uintptr_t src_pool_ptr, torch::Tensor dst_pool,
       (int)src_ids.size(0), L, src_nb, dst_nb, block_bytes, cur_stream()));
 }
 
+// `chunk` chose the softmax step of an earlier kernel: it is still checked
+void check_chunk(int64_t chunk) {
+  TORCH_CHECK(chunk == 256 || chunk == 512, "chunk must be 256 or 512");
+}
+
 torch::Tensor paged_attention(torch::Tensor q, torch::Tensor k_cache,
                               torch::Tensor v_cache,
                               torch::Tensor block_tables,
                               torch::Tensor seq_lens, double scale,
-                              int64_t chunk) {
+                              int64_t chunk, int64_t waves) {
+  check_chunk(chunk);
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -252,7 +258,7 @@ torch::Tensor paged_attention(torch::Tensor q, torch::Tensor k_cache,
       q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
       out.data_ptr(), B, qh, kvh, bs, d, (int)block_tables.size(1),
-      kv_fp8_flag(k_cache), (int)chunk, (float)scale, cur_stream()));
+      kv_fp8_flag(k_cache), (int)waves, (float)scale, cur_stream()));
   return out;
 }
 
@@ -261,7 +267,8 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
                                     torch::Tensor block_tables,
                                     torch::Tensor seq_lens, int64_t n_parts,
                                     int64_t part_tokens, double scale,
-                                    int64_t chunk) {
+                                    int64_t chunk, int64_t waves) {
+  check_chunk(chunk);
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -276,7 +283,8 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
       out.data_ptr(), part_o.data_ptr<float>(), part_ml.data_ptr<float>(), B,
       qh, kvh, bs, d, (int)block_tables.size(1), (int)n_parts,
-      (int)part_tokens, kv_fp8_flag(k_cache), (int)chunk, (float)scale, cur_stream()));
+      (int)part_tokens, kv_fp8_flag(k_cache), (int)waves, (float)scale,
+      cur_stream()));
   return out;
 }
 
@@ -337,12 +345,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attention", &paged_attention,
         "GQA decode attention over paged KV", py::arg("q"),
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
-        py::arg("seq_lens"), py::arg("scale"), py::arg("chunk") = 256);
+        py::arg("seq_lens"), py::arg("scale"), py::arg("chunk") = 256,
+        py::arg("waves") = 8);
   m.def("paged_attention_split", &paged_attention_split,
         "flash-decoding GQA attention with sequence partitioning",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("n_parts"),
-        py::arg("part_tokens"), py::arg("scale"), py::arg("chunk") = 256);
+        py::arg("part_tokens"), py::arg("scale"), py::arg("chunk") = 256,
+        py::arg("waves") = 8);
   m.def("flash_prefill", &flash_prefill,
         "fused MFMA causal varlen prefill attention over paged KV");
 }

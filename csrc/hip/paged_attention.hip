@@ -2,22 +2,29 @@
 //
 // The decode-step hot kernel of the per-GPU worker engine. Memory-bound: the
 // whole point is streaming each sequence's K/V exactly once per step at
-// near-HBM rate (guide Appendix B "Attention decode").
+// near-HBM rate.
 //
-// Geometry: one workgroup (4 waves, 256 threads) per (sequence, kv_head,
-// partition). Q-heads in the GQA group (QPG = n_q_heads / n_kv_heads, <= 8)
-// are scored together so K rows are read once for the whole group.
-//   Phase A  each wave owns 64 tokens of a 256-token chunk; a lane streams
-//            its token's K row (short8 loads) against the group's Q vectors
-//            staged in LDS (broadcast reads) -> logits in LDS.
-//   Phase B  online-softmax update per q-head (wave-parallel reductions).
-//   Phase C  V accumulation: lane owns a dim pair, wave owns its 64 tokens;
-//            V rows stream fully coalesced (64 lanes x 4 B = one 256 B row).
-//   Final    cross-wave combine via LDS, normalize, bf16 store.
+// Geometry: one workgroup per (sequence, kv_head, partition). Its waves take
+// tiles of 32 tokens in turn, each with an online softmax of its own, and meet
+// once at the end: no LDS and no barrier while the cache streams by. Both
+// products run on the matrix cores, with the operands as they come from
+// memory:
+//   S' = K Q'  a lane holds 16 bytes of a token's key (bf16 matrix cores; the
+//              order of the key's channels inside a step is free, Q follows).
+//              It gets back the scores of 4 + 4 tokens for one head.
+//   O  = P V   32-bit matrix cores: probabilities stay 32-bit, as the scores
+//              left them in the lane; a lane holds 8 channels of one token's
+//              value, widened to 32-bit (exact for bf16 and fp8).
+// A tile's matrix work is a quarter of the time its bytes take at 5 TB/s, so
+// the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost nothing.
 //
-// Flash-decoding sequence split (SPLIT=true): long sequences are cut into
-// gridDim.z partitions so the launch has >> 256 workgroups (the chip needs
-// ~2 WGs/CU just to be full; B*KVH alone is often < 512). Each partition
+// Measured (8 key heads, ragged; before: scores and sums on the vector units,
+// three barriers per 256 tokens): 256 sequences of 1500 tokens, groups of 4:
+// 279 us, 5.6 TB/s (before 546); 30 of 1100, groups of 8: 27 us (67); 17 of
+// 6800, fp8, in 4 partitions: 61 us, 3.8 TB/s (137); one of 777: 11 us (18).
+//
+// Flash-decoding sequence split (SPLIT): long sequences are cut into
+// gridDim.z partitions so that small batches fill the chip. Each partition
 // writes an UNNORMALIZED partial (o_acc, m, l) and a tiny combine kernel
 // merges partitions: m* = max m_p; o = sum o_p*exp(m_p-m*); l likewise.
 #include "hip_common.h"
@@ -25,12 +32,77 @@
 namespace {
 
 constexpr int D = 128;        // head_dim (Llama-3 family)
-constexpr int DEF_CHUNK = 256;  // default tokens per online-softmax chunk
-constexpr int NW = 4;         // waves per workgroup
+constexpr int TILE = 32;      // tokens per wave and step
+constexpr int MAX_QPG = 8;
 constexpr float NEG = -1e30f;
+constexpr float LOG2E = 1.4426950408889634f;
+// The running maximum moves only when a score passes it by this much (log2):
+// sums stay below 2^8 times a tile's, far inside 32-bit range, and the
+// accumulators are rarely rescaled.
+constexpr float SLACK = 8.f;
 
-template <int QPG, bool SPLIT, typename CT, int CHUNK = DEF_CHUNK>
-__global__ __launch_bounds__(NW * WAVE) void paged_attention_kernel(
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) unsigned int uint4v;
+typedef __attribute__((ext_vector_type(2))) unsigned int uint2v;
+
+// How a cache type's loads map to operands.
+//   KL loads of 16 bytes make up a lane's share of a key (its 4 steps)
+//   dim(s, g): first of the 8 channels that lane group g holds in step s
+template <typename CT> struct Cache;
+
+template <> struct Cache<short> {
+  static constexpr int KL = 4;
+  typedef uint4v VReg;
+  static __device__ __forceinline__ int dim(int s, int g) {
+    return s * 32 + g * 8;
+  }
+  static __device__ __forceinline__ bf16x8 key(const uint4v* k, int s) {
+    return __builtin_bit_cast(bf16x8, k[s]);
+  }
+  static __device__ __forceinline__ void value(VReg v, float* f) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f[2 * i] = __builtin_bit_cast(float, v[i] << 16);
+      f[2 * i + 1] = __builtin_bit_cast(float, v[i] & 0xffff0000u);
+    }
+  }
+};
+
+template <> struct Cache<unsigned char> {
+  static constexpr int KL = 2;
+  typedef uint2v VReg;
+  static __device__ __forceinline__ int dim(int s, int g) {
+    return s / 2 * 64 + g * 16 + s % 2 * 8;
+  }
+  static __device__ __forceinline__ void value(VReg v, float* f) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const float2v a = __builtin_amdgcn_cvt_pk_f32_fp8(v[i], false);
+      const float2v b = __builtin_amdgcn_cvt_pk_f32_fp8(v[i], true);
+      f[4 * i] = a[0];
+      f[4 * i + 1] = a[1];
+      f[4 * i + 2] = b[0];
+      f[4 * i + 3] = b[1];
+    }
+  }
+  // e4m3 values are bf16 values: the upper halves of the floats
+  static __device__ __forceinline__ bf16x8 key(const uint4v* k, int s) {
+    float f[8];
+    value((uint2v){k[s / 2][s % 2 * 2], k[s / 2][s % 2 * 2 + 1]}, f);
+    uint4v r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[2 * i + 1]),
+                                   __builtin_bit_cast(uint32_t, f[2 * i]),
+                                   0x07060302);
+    return __builtin_bit_cast(bf16x8, r);
+  }
+};
+
+// PAGE16: pages of 16 tokens and partitions that begin on a page, so half a
+// tile lies in one page; else every lane looks its tokens up one by one.
+template <typename CT, bool SPLIT, bool PAGE16, int NW>
+__global__ __launch_bounds__(NW * WAVE, 3) void paged_attention_kernel(
     const short* __restrict__ q,        // [B, QH, D]
     const CT* __restrict__ k_cache,     // [NB, KVH, BS, D] bf16|fp8
     const CT* __restrict__ v_cache,     // [NB, KVH, BS, D] bf16|fp8
@@ -38,246 +110,280 @@ __global__ __launch_bounds__(NW * WAVE) void paged_attention_kernel(
     const int32_t* __restrict__ seq_lens,      // [B]
     short* __restrict__ out,                   // [B, QH, D]
     float* __restrict__ part_o,   // [B, KVH, NP, QPG, D] (SPLIT)
-    float* __restrict__ part_ml,  // [B, KVH, NP, QPG, 2] (SPLIT)
-    int kvh, int bs, int max_blocks, int part_tokens, float scale) {
+    float* __restrict__ part_ml,  // [B, KVH, NP, QPG, 2] (SPLIT), m in log2
+    int kvh, int qpg, int bs, int max_blocks, int part_tokens, float scale) {
+  typedef Cache<CT> C;
   const int b = blockIdx.x;
   const int kh = blockIdx.y;
   const int part = SPLIT ? blockIdx.z : 0;
   const int np = SPLIT ? gridDim.z : 1;
-  const int qh0 = kh * QPG;
-  const int n_q_heads = kvh * QPG;
+  const int64_t group = (int64_t)b * kvh + kh;
   const int seq_len = seq_lens[b];
   const int t_begin = SPLIT ? part * part_tokens : 0;
   const int t_end = SPLIT ? min(seq_len, t_begin + part_tokens) : seq_len;
 
-  __shared__ float q_lds[QPG][D];
-  __shared__ float logits[QPG][CHUNK];
-  __shared__ float m_sh[QPG], l_sh[QPG], alpha_sh[QPG];
-  __shared__ float comb[NW][QPG][D];
-
   const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = tid % WAVE;
+  const int col = lane % 16, g = lane / 16;
 
   if (SPLIT && t_begin >= seq_len) {
     // empty partition: publish l=0 so the combiner skips it
-    if (tid < QPG) {
-      float* ml = part_ml + ((((int64_t)b * kvh + kh) * np + part) * QPG +
-                             tid) * 2;
+    if (tid < qpg) {
+      float* ml = part_ml + ((group * np + part) * qpg + tid) * 2;
       ml[0] = NEG;
       ml[1] = 0.f;
     }
     return;
   }
 
-  // stage scaled Q for the group into LDS
-  for (int i = tid; i < QPG * D; i += NW * WAVE) {
-    int h = i / D, d = i % D;
-    q_lds[h][d] =
-        bf16_to_f32(q[((int64_t)b * n_q_heads + qh0 + h) * D + d]) * scale;
-  }
-  if (tid < QPG) {
-    m_sh[tid] = NEG;
-    l_sh[tid] = 0.f;
-  }
-  __syncthreads();
-
-  float o_acc[QPG][2];
+  // column `col` of the scores is a head of the group; the others are zero
+  bf16x8 qf[4];
 #pragma unroll
-  for (int h = 0; h < QPG; ++h) o_acc[h][0] = o_acc[h][1] = 0.f;
+  for (int s = 0; s < 4; ++s) {
+    short8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (col < qpg) z = *(const short8*)(q + (group * qpg + col) * D + C::dim(s, g));
+    qf[s] = __builtin_bit_cast(bf16x8, z);
+  }
+  const float scale_log2 = scale * LOG2E;
+
+  float m = NEG, l = 0.f;       // of head `col`; l: this lane's tokens only
+  float4v acc[8];               // heads 4g + r, channels 8 col + i
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = (float4v){0.f, 0.f, 0.f, 0.f};
 
   const int32_t* bt = block_tables + (int64_t)b * max_blocks;
+  uint4v kr[2][C::KL];
+  typename C::VReg vr[2][4];
+  int page[2];
+  // pages of the tile at t0, none past the sequence's last
+  auto find = [&](int t0) {
+    if constexpr (PAGE16) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        page[h] = bt[min(t0 / 16 + h, (t_end - 1) / 16)];
+    }
+  };
+  // a token's row; past the end the last one's (only in the lookup form)
+  auto row_of = [&](int t) {
+    const int tc = min(t, t_end - 1);
+    return (((int64_t)bt[tc / bs] * kvh + kh) * bs + tc % bs) * D;
+  };
+  auto fetch_k = [&](int t0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const CT* row;
+      if constexpr (PAGE16)
+        row = k_cache + ((int64_t)page[h] * kvh + kh) * (16 * D) + col * D;
+      else
+        row = k_cache + row_of(t0 + h * 16 + col);
+#pragma unroll
+      for (int i = 0; i < C::KL; ++i)
+        kr[h][i] = *(const uint4v*)((const char*)row + i * 64 + g * 16);
+    }
+  };
+  auto fetch_v = [&](int t0) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const CT* row;
+        if constexpr (PAGE16)
+          row = v_cache + ((int64_t)page[h] * kvh + kh) * (16 * D) +
+                (g * 4 + j) * D;
+        else
+          row = v_cache + row_of(t0 + h * 16 + g * 4 + j);
+        vr[h][j] = *(const typename C::VReg*)(row + col * 8);
+      }
+  };
 
-  for (int chunk0 = t_begin; chunk0 < t_end; chunk0 += CHUNK) {
-    const int n_t = min(CHUNK, t_end - chunk0);
-    // ---- Phase A: logits[h][t_local] (CHUNK may exceed one row/lane:
-    // each pass of the tb loop covers NW*WAVE tokens) ----
-    for (int tb = 0; tb < CHUNK; tb += NW * WAVE) {
-      const int t_local = tb + wave * WAVE + lane;
-      float dot[QPG];
-#pragma unroll
-      for (int h = 0; h < QPG; ++h) dot[h] = 0.f;
-      if (t_local < n_t) {
-        const int t = chunk0 + t_local;
-        const int64_t blk = bt[t / bs];
-        const int row = t % bs;
-        const CT* krow = k_cache + (((blk * kvh + kh) * bs) + row) * D;
-#pragma unroll 8
-        for (int c = 0; c < D / 8; ++c) {
-          float kf[8];
-          load_kv8(krow + c * 8, kf);
-#pragma unroll
-          for (int h = 0; h < QPG; ++h) {
-            const float4v* q4 = (const float4v*)&q_lds[h][c * 8];
-            float4v qa = q4[0], qb = q4[1];
-            dot[h] += qa[0] * kf[0] + qa[1] * kf[1] + qa[2] * kf[2] +
-                      qa[3] * kf[3] + qb[0] * kf[4] + qb[1] * kf[5] +
-                      qb[2] * kf[6] + qb[3] * kf[7];
-          }
-        }
-      }
-#pragma unroll
-      for (int h = 0; h < QPG; ++h)
-        logits[h][t_local] = (t_local < n_t) ? dot[h] : NEG;
-    }
-    __syncthreads();
-
-    // ---- Phase B: online softmax per head (wave w handles head w, w+NW..) ----
-    for (int h = wave; h < QPG; h += NW) {
-      float lmax = NEG;
-#pragma unroll
-      for (int i = 0; i < CHUNK / WAVE; ++i)
-        lmax = fmaxf(lmax, logits[h][i * WAVE + lane]);
-      lmax = wave_reduce_max(lmax);
-      const float m_old = m_sh[h];
-      const float m_new = fmaxf(m_old, lmax);
-      float lsum = 0.f;
-#pragma unroll
-      for (int i = 0; i < CHUNK / WAVE; ++i) {
-        const int idx = i * WAVE + lane;
-        float p = (logits[h][idx] <= NEG) ? 0.f : __expf(logits[h][idx] - m_new);
-        logits[h][idx] = p;
-        lsum += p;
-      }
-      lsum = wave_reduce_sum(lsum);
-      if (lane == 0) {
-        const float alpha = (m_old <= NEG) ? 0.f : __expf(m_old - m_new);
-        alpha_sh[h] = alpha;
-        l_sh[h] = l_sh[h] * alpha + lsum;
-        m_sh[h] = m_new;
-      }
-    }
-    __syncthreads();
-
-    // ---- Phase C: V accumulation (wave owns its 64 tokens, lane owns 2 dims) ----
-#pragma unroll
-    for (int h = 0; h < QPG; ++h) {
-      const float a = alpha_sh[h];
-      o_acc[h][0] *= a;
-      o_acc[h][1] *= a;
-    }
-    {
-      const int t_base = wave * (CHUNK / NW);
-      const int t_cnt = min(CHUNK / NW, n_t - t_base);
-      // batch the V row loads 8 deep so they overlap (each row is one
-      // coalesced 256-B wave read; a load-use loop serializes on latency)
-      int i = 0;
-      for (; i + 8 <= t_cnt; i += 8) {
-        const CT* vrows[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int t = chunk0 + t_base + i + j;
-          const int64_t blk = bt[t / bs];
-          vrows[j] = v_cache + (((blk * kvh + kh) * bs) + t % bs) * D +
-                     lane * 2;
-        }
-        float vv[8][2];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) load_kv2(vrows[j], vv[j][0], vv[j][1]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-#pragma unroll
-          for (int h = 0; h < QPG; ++h) {
-            const float p = logits[h][t_base + i + j];
-            o_acc[h][0] += p * vv[j][0];
-            o_acc[h][1] += p * vv[j][1];
-          }
-        }
-      }
-      for (; i < t_cnt; ++i) {
-        const int t = chunk0 + t_base + i;
-        const int64_t blk = bt[t / bs];
-        float v0, v1;
-        load_kv2(v_cache + (((blk * kvh + kh) * bs) + t % bs) * D + lane * 2,
-                 v0, v1);
-#pragma unroll
-        for (int h = 0; h < QPG; ++h) {
-          const float p = logits[h][t_base + i];
-          o_acc[h][0] += p * v0;
-          o_acc[h][1] += p * v1;
-        }
-      }
-    }
-    __syncthreads();  // logits reused next chunk
+  int t0 = t_begin + wave * TILE;
+  if (t0 < t_end) {
+    find(t0);
+    fetch_k(t0);
+    fetch_v(t0);
   }
-
-  // ---- combine partial o across waves ----
+  for (; t0 < t_end; t0 += NW * TILE) {
+    const int next = t0 + NW * TILE;
+    const bool more = next < t_end;
+    if (more) find(next);
+    float4v sc[2];
 #pragma unroll
-  for (int h = 0; h < QPG; ++h) {
-    comb[wave][h][2 * lane] = o_acc[h][0];
-    comb[wave][h][2 * lane + 1] = o_acc[h][1];
+    for (int h = 0; h < 2; ++h) {
+      sc[h] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(C::key(kr[h], s),
+                                                        qf[s], sc[h], 0, 0, 0);
+    }
+    if (more) fetch_k(next);
+
+    const bool tail = t0 + TILE > t_end;      // wave-uniform
+    float mx = NEG;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sc[h][r] *= scale_log2;
+        if (tail && t0 + h * 16 + g * 4 + r >= t_end) sc[h][r] = -INFINITY;
+        mx = fmaxf(mx, sc[h][r]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    const bool moved = mx > m + SLACK;
+    if (__any(moved)) {
+      const float to = moved ? mx : m;
+      const float alpha = __builtin_amdgcn_exp2f(m - to);
+      m = to;
+      l *= alpha;
+      float4v a;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) a[r] = __shfl(alpha, g * 4 + r, WAVE);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] *= a;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sc[h][r] = __builtin_amdgcn_exp2f(sc[h][r] - m);
+        l += sc[h][r];
+      }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float f[8];
+        C::value(vr[h][j], f);
+        // a page's rows past the sequence may hold anything
+        const bool gone = tail && t0 + h * 16 + g * 4 + j >= t_end;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              sc[h][j], gone ? 0.f : f[i], acc[i], 0, 0, 0);
+      }
+    if (more) fetch_v(next);
+  }
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+
+  // ---- the waves meet ----
+  __shared__ float ml_sh[NW][MAX_QPG][2];
+  __shared__ __align__(16) float o_sh[NW][MAX_QPG][D];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int h = g * 4 + r;
+    if (h >= qpg) continue;
+    float4v lo, hi;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      lo[i] = acc[i][r];
+      hi[i] = acc[4 + i][r];
+    }
+    *(float4v*)&o_sh[wave][h][col * 8] = lo;
+    *(float4v*)&o_sh[wave][h][col * 8 + 4] = hi;
+  }
+  if (g == 0 && col < qpg) {
+    ml_sh[wave][col][0] = m;
+    ml_sh[wave][col][1] = l;
   }
   __syncthreads();
-  if (SPLIT) {
-    float* po = part_o + ((((int64_t)b * kvh + kh) * np + part) * QPG) * D;
-    for (int i = tid; i < QPG * D; i += NW * WAVE) {
-      const int h = i / D, d = i % D;
-      float s = 0.f;
+  for (int i = tid; i < qpg * D; i += NW * WAVE) {
+    const int h = i / D, d = i % D;
+    float top = NEG;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) s += comb[w][h][d];
-      po[h * D + d] = s;                     // unnormalized
-    }
-    if (tid < QPG) {
-      float* ml = part_ml + ((((int64_t)b * kvh + kh) * np + part) * QPG +
-                             tid) * 2;
-      ml[0] = m_sh[tid];
-      ml[1] = l_sh[tid];
-    }
-  } else {
-    // 256 threads cover QPG*D outputs (QPG<=8 -> <=1024 values, loop)
-    for (int i = tid; i < QPG * D; i += NW * WAVE) {
-      const int h = i / D, d = i % D;
-      float s = 0.f;
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, ml_sh[w][h][0]);
+    float s = 0.f, sum = 0.f;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) s += comb[w][h][d];
-      const float l = l_sh[h];
-      out[((int64_t)b * n_q_heads + qh0 + h) * D + d] =
-          f32_to_bf16(l > 0.f ? s / l : 0.f);
+    for (int w = 0; w < NW; ++w) {
+      const float a = __builtin_amdgcn_exp2f(ml_sh[w][h][0] - top);
+      s += a * o_sh[w][h][d];
+      sum += a * ml_sh[w][h][1];
+    }
+    if (SPLIT) {
+      part_o[((group * np + part) * qpg + h) * D + d] = s;   // unnormalized
+      if (d == 0) {
+        float* ml = part_ml + ((group * np + part) * qpg + h) * 2;
+        ml[0] = top;
+        ml[1] = sum;
+      }
+    } else {
+      out[(group * qpg + h) * D + d] = f32_to_bf16(sum > 0.f ? s / sum : 0.f);
     }
   }
 }
 
-// Merge the NP partitions of one (seq, kv_head): one workgroup per
-// (seq, kv_head), each thread owns (head, dim) outputs striding QPG*D.
-template <int QPG>
-__global__ __launch_bounds__(256) void paged_attention_combine_kernel(
+// Merge the NP partitions: one workgroup per (seq, q head), a thread per dim.
+// The first wave weighs the partitions (a lane each), then every thread sums
+// its column; the loads of a step do not wait for each other.
+__global__ __launch_bounds__(D) void paged_attention_combine_kernel(
     const float* __restrict__ part_o,   // [B, KVH, NP, QPG, D]
     const float* __restrict__ part_ml,  // [B, KVH, NP, QPG, 2]
     short* __restrict__ out,            // [B, QH, D]
-    int kvh, int np) {
-  const int b = blockIdx.x;
-  const int kh = blockIdx.y;
-  const int n_q_heads = kvh * QPG;
-  __shared__ float m_g[QPG], scale_p[64][QPG];  // np <= 64
+    int qpg, int np) {
+  __shared__ float weight[64];          // np <= 64
+  const int64_t group = (int64_t)blockIdx.x * (gridDim.y / qpg) +
+                        blockIdx.y / qpg;
+  const int h = blockIdx.y % qpg, d = threadIdx.x;
+  const int64_t first = group * np * qpg + h;
+  if (d < WAVE) {
+    const float* ml = part_ml + (first + (int64_t)min(d, np - 1) * qpg) * 2;
+    const float m = d < np ? ml[0] : NEG, l = d < np ? ml[1] : 0.f;
+    const float top = wave_reduce_max(m);
+    const float w = l > 0.f ? __builtin_amdgcn_exp2f(m - top) : 0.f;
+    const float sum = wave_reduce_sum(w == 0.f ? 0.f : w * l);
+    weight[d] = w == 0.f ? 0.f : w / sum;
+  }
+  __syncthreads();
+  float o = 0.f;
+#pragma unroll 8
+  for (int p = 0; p < np; ++p) {
+    const float x = part_o[(first + (int64_t)p * qpg) * D + d];
+    const float w = weight[p];
+    o += w == 0.f ? 0.f : w * x;        // an empty partition wrote no sums
+  }
+  out[((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * D + d] = f32_to_bf16(o);
+}
 
-  const int tid = threadIdx.x;
-  if (tid < QPG) {
-    float m = NEG;
-    for (int p = 0; p < np; ++p)
-      m = fmaxf(m, part_ml[((((int64_t)b * kvh + kh) * np + p) * QPG + tid)
-                           * 2]);
-    m_g[tid] = m;
-  }
-  __syncthreads();
-  for (int i = tid; i < QPG * np; i += 256) {
-    const int p = i / QPG, h = i % QPG;
-    const float* ml =
-        part_ml + ((((int64_t)b * kvh + kh) * np + p) * QPG + h) * 2;
-    scale_p[p][h] = (ml[1] > 0.f) ? __expf(ml[0] - m_g[h]) : 0.f;
-  }
-  __syncthreads();
-  for (int i = tid; i < QPG * D; i += 256) {
-    const int h = i / D, d = i % D;
-    float o = 0.f, l = 0.f;
-    for (int p = 0; p < np; ++p) {
-      const float s = scale_p[p][h];
-      if (s == 0.f) continue;
-      o += s * part_o[((((int64_t)b * kvh + kh) * np + p) * QPG + h) * D + d];
-      l += s * part_ml[((((int64_t)b * kvh + kh) * np + p) * QPG + h) * 2 + 1];
-    }
-    out[((int64_t)b * n_q_heads + kh * QPG + h) * D + d] =
-        f32_to_bf16(l > 0.f ? o / l : 0.f);
-  }
+template <bool SPLIT>
+hipError_t attend(const void* q, const void* k_cache, const void* v_cache,
+                  const int32_t* block_tables, const int32_t* seq_lens,
+                  void* out, float* part_o, float* part_ml, int n_seqs,
+                  int n_q_heads, int kvh, int bs, int head_dim, int max_blocks,
+                  int n_parts, int part_tokens, int kv_fp8, int waves,
+                  float scale, hipStream_t stream) {
+  if (n_seqs == 0) return hipSuccess;
+  const int qpg = n_q_heads / kvh;
+  if (head_dim != D || n_parts > 64 || (waves != 4 && waves != 8) ||
+      (qpg != 1 && qpg != 2 && qpg != 4 && qpg != 8))
+    return hipErrorInvalidValue;
+  const dim3 grid(n_seqs, kvh, n_parts);
+#define GO(CT, PAGE16, NW)                                                   \
+  hipLaunchKernelGGL((paged_attention_kernel<CT, SPLIT, PAGE16, NW>), grid,  \
+                     dim3(NW * WAVE), 0, stream, (const short*)q,            \
+                     (const CT*)k_cache, (const CT*)v_cache, block_tables,   \
+                     seq_lens, (short*)out, part_o, part_ml, kvh, qpg, bs,   \
+                     max_blocks, part_tokens, scale)
+#define GO_NW(CT, PAGE16)                                                    \
+  do {                                                                       \
+    if (waves == 8) GO(CT, PAGE16, 8); else GO(CT, PAGE16, 4);               \
+  } while (0)
+#define GO_PAGE(CT)                                                          \
+  do {                                                                       \
+    if (bs == 16 && part_tokens % 16 == 0) GO_NW(CT, true);                  \
+    else GO_NW(CT, false);                                                   \
+  } while (0)
+  if (kv_fp8) GO_PAGE(unsigned char);
+  else GO_PAGE(short);
+#undef GO_PAGE
+#undef GO_NW
+#undef GO
+  if (SPLIT)
+    hipLaunchKernelGGL(paged_attention_combine_kernel,
+                       dim3(n_seqs, n_q_heads), dim3(D), 0, stream, part_o,
+                       part_ml, (short*)out, qpg, n_parts);
+  HIP_CHECK_LAST();
+  return hipSuccess;
 }
 
 }  // namespace
@@ -288,44 +394,11 @@ hipError_t lds_paged_attention(const void* q, const void* k_cache,
                                const void* v_cache, const int32_t* block_tables,
                                const int32_t* seq_lens, void* out, int n_seqs,
                                int n_q_heads, int kvh, int bs, int head_dim,
-                               int max_blocks, int kv_fp8, int chunk,
+                               int max_blocks, int kv_fp8, int waves,
                                float scale, hipStream_t stream) {
-  if (n_seqs == 0) return hipSuccess;
-  if (head_dim != D) return hipErrorInvalidValue;
-  if (chunk != 256 && chunk != 512) return hipErrorInvalidValue;
-  const int qpg = n_q_heads / kvh;
-  dim3 grid(n_seqs, kvh), block(NW * WAVE);
-#define LAUNCH_CT(QPG, CT)                                                    \
-  do {                                                                        \
-    if (chunk == 512)                                                         \
-      hipLaunchKernelGGL((paged_attention_kernel<QPG, false, CT, 512>),       \
-                         grid, block, 0, stream, (const short*)q,             \
-                         (const CT*)k_cache, (const CT*)v_cache,              \
-                         block_tables, seq_lens, (short*)out, nullptr,        \
-                         nullptr, kvh, bs, max_blocks, 0, scale);             \
-    else                                                                      \
-      hipLaunchKernelGGL((paged_attention_kernel<QPG, false, CT, 256>),       \
-                         grid, block, 0, stream, (const short*)q,             \
-                         (const CT*)k_cache, (const CT*)v_cache,              \
-                         block_tables, seq_lens, (short*)out, nullptr,        \
-                         nullptr, kvh, bs, max_blocks, 0, scale);             \
-  } while (0)
-#define LAUNCH(QPG)                                                           \
-  do {                                                                        \
-    if (kv_fp8) LAUNCH_CT(QPG, unsigned char);                                \
-    else LAUNCH_CT(QPG, short);                                               \
-  } while (0)
-  switch (qpg) {
-    case 1: LAUNCH(1); break;
-    case 2: LAUNCH(2); break;
-    case 4: LAUNCH(4); break;
-    case 8: LAUNCH(8); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef LAUNCH
-#undef LAUNCH_CT
-  HIP_CHECK_LAST();
-  return hipSuccess;
+  return attend<false>(q, k_cache, v_cache, block_tables, seq_lens, out,
+                       nullptr, nullptr, n_seqs, n_q_heads, kvh, bs, head_dim,
+                       max_blocks, 1, 0, kv_fp8, waves, scale, stream);
 }
 
 hipError_t lds_paged_attention_split(
@@ -333,46 +406,11 @@ hipError_t lds_paged_attention_split(
     const int32_t* block_tables, const int32_t* seq_lens, void* out,
     float* part_o, float* part_ml, int n_seqs, int n_q_heads, int kvh, int bs,
     int head_dim, int max_blocks, int n_parts, int part_tokens, int kv_fp8,
-    int chunk, float scale, hipStream_t stream) {
-  if (n_seqs == 0) return hipSuccess;
-  if (head_dim != D || n_parts > 64) return hipErrorInvalidValue;
-  if (chunk != 256 && chunk != 512) return hipErrorInvalidValue;
-  const int qpg = n_q_heads / kvh;
-  dim3 grid(n_seqs, kvh, n_parts), block(NW * WAVE);
-  dim3 cgrid(n_seqs, kvh), cblock(256);
-#define LAUNCH_CT(QPG, CT)                                                    \
-  do {                                                                        \
-    if (chunk == 512)                                                         \
-      hipLaunchKernelGGL((paged_attention_kernel<QPG, true, CT, 512>), grid,  \
-                         block, 0, stream, (const short*)q,                   \
-                         (const CT*)k_cache, (const CT*)v_cache,              \
-                         block_tables, seq_lens, (short*)out, part_o,         \
-                         part_ml, kvh, bs, max_blocks, part_tokens, scale);   \
-    else                                                                      \
-      hipLaunchKernelGGL((paged_attention_kernel<QPG, true, CT, 256>), grid,  \
-                         block, 0, stream, (const short*)q,                   \
-                         (const CT*)k_cache, (const CT*)v_cache,              \
-                         block_tables, seq_lens, (short*)out, part_o,         \
-                         part_ml, kvh, bs, max_blocks, part_tokens, scale);   \
-  } while (0)
-#define LAUNCH(QPG)                                                           \
-  do {                                                                        \
-    if (kv_fp8) LAUNCH_CT(QPG, unsigned char);                                \
-    else LAUNCH_CT(QPG, short);                                               \
-    hipLaunchKernelGGL((paged_attention_combine_kernel<QPG>), cgrid, cblock,  \
-                       0, stream, part_o, part_ml, (short*)out, kvh,          \
-                       n_parts);                                              \
-  } while (0)
-  switch (qpg) {
-    case 1: LAUNCH(1); break;
-    case 2: LAUNCH(2); break;
-    case 4: LAUNCH(4); break;
-    case 8: LAUNCH(8); break;
-    default: return hipErrorInvalidValue;
-  }
-#undef LAUNCH
-  HIP_CHECK_LAST();
-  return hipSuccess;
+    int waves, float scale, hipStream_t stream) {
+  return attend<true>(q, k_cache, v_cache, block_tables, seq_lens, out, part_o,
+                      part_ml, n_seqs, n_q_heads, kvh, bs, head_dim,
+                      max_blocks, n_parts, part_tokens, kv_fp8, waves, scale,
+                      stream);
 }
 
 }  // extern "C"

@@ -5,7 +5,7 @@ CUDA-device tensor with `_hip_ops` missing raises immediately rather than
 silently falling back to eager torch. CPU tensors (tests, tiny gloo runs)
 use ops.ref.
 """
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -65,11 +65,18 @@ def reshape_and_cache(k_new: torch.Tensor, v_new: torch.Tensor,
     ref.reshape_and_cache(k_new, v_new, k_cache, v_cache, slots)
 
 
-import os as _os
-
-# online-softmax chunk of the decode kernel: 512 halves barrier count
-# (bisect knob; 256 is the measured default)
-_ATTN_CHUNK = int(_os.environ.get("LLMD_ATTN_CHUNK", "256"))
+def decode_parts(groups: int, max_len: int) -> Tuple[int, int]:
+    """-> (parts, tokens per part) of the decode attention of `groups`
+    (sequence, key head) pairs. A workgroup of 8 waves takes 256 tokens a
+    step, and about 512 of them fill the chip: parts make up for fewer groups
+    as long as each has a step of its own. From 200 groups on, the partial
+    sums and the second launch cost more than the idle compute units (240
+    groups of 1100 tokens: 27 us in one part, 38 in two; 136 groups of 6800
+    tokens, 8-bit: 108 us in one part, 62 in four)."""
+    parts = 1 if groups >= 200 else \
+        max(1, min(64, -(-512 // max(1, groups)), -(-max_len // 256)))
+    part = -(-(-(-max_len // parts)) // 32) * 32
+    return -(-max_len // part), part
 
 
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
@@ -79,25 +86,19 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
     if _use_hip(q):
         bt = block_tables.to(torch.int32)
         sl = seq_lens.to(torch.int32)
-        # flash-decoding sequence split: the plain kernel launches only
-        # B*KVH workgroups — far short of the 256-CU chip's >=2 WG/CU need.
-        # Partition long sequences so the grid fills the chip; a combine
-        # kernel merges the unnormalized partials.
-        n_wgs = q.shape[0] * k_cache.shape[1]
-        if max_seq_len is not None and n_wgs < 1024 and max_seq_len > 512:
-            target_np = min(64, max(1, 1024 // max(1, n_wgs)))
-            # partition size: ceil-divide then round up to the kernel's
-            # 256-token online-softmax chunk
-            c = _ATTN_CHUNK
-            part = max(c, ((max_seq_len + target_np - 1) // target_np
-                           + c - 1) // c * c)
-            np_ = (max_seq_len + part - 1) // part
-            if np_ > 1:
+        waves = 8
+        if max_seq_len is not None and max_seq_len > 0:
+            # short sequences leave half of 8 waves without a tile (100
+            # sequences of 120 tokens: 19 us with 8 waves, 15 with 4)
+            waves = 4 if max_seq_len <= 256 else 8
+            parts, part = decode_parts(q.shape[0] * k_cache.shape[1],
+                                       max_seq_len)
+            if parts > 1:
                 return _ext.paged_attention_split(q, k_cache, v_cache, bt,
-                                                  sl, np_, part, scale,
-                                                  _ATTN_CHUNK)
+                                                  sl, parts, part, scale,
+                                                  waves=waves)
         return _ext.paged_attention(q, k_cache, v_cache, bt, sl, scale,
-                                    _ATTN_CHUNK)
+                                    waves=waves)
     return ref.paged_attention(q, k_cache, v_cache, block_tables, seq_lens,
                                scale)
 

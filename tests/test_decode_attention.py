@@ -1,0 +1,83 @@
+"""Decode attention over the paged pool: edges of tiles, pages, partitions and
+head groups against float64."""
+import pytest
+import torch
+
+from llm_d_inference_scheduler_amd.ops import dispatch
+
+KVH, D = 2, 128
+
+
+@pytest.mark.parametrize("groups", [1, 7, 64, 199, 200, 5000])
+@pytest.mark.parametrize("max_len", [1, 31, 256, 257, 5000, 131072])
+def test_parts_cover_the_context(groups, max_len):
+    parts, part = dispatch.decode_parts(groups, max_len)
+    assert 1 <= parts <= 64                   # the kernel's limit
+    assert part % 32 == 0                     # parts begin on a page
+    assert (parts - 1) * part < max_len <= parts * part
+
+
+def _case(lens, qpg, bs, fp8):
+    g = torch.Generator().manual_seed(sum(lens) + qpg + bs)
+    pages = [-(-n // bs) for n in lens]
+    width = max(pages) + 1
+    nb = sum(pages) + 1
+    dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    kc, vc = (torch.randn(nb, KVH, bs, D, generator=g).to(dtype)
+              for _ in range(2))
+    q = torch.randn(len(lens), KVH * qpg, D, generator=g).bfloat16()
+    perm, at = torch.randperm(nb, generator=g).int(), 0
+    bt = torch.zeros(len(lens), width, dtype=torch.int32)
+    want = torch.zeros(q.shape, dtype=torch.float64)
+    for i, (n, p) in enumerate(zip(lens, pages)):
+        rows = perm[at:at + p]
+        bt[i, :p], at = rows, at + p
+        if n == 0:
+            continue
+        k, v = (c[rows.long()].double().permute(1, 0, 2, 3)
+                .reshape(KVH, -1, D)[:, :n] for c in (kc, vc))
+        s = q[i].double().view(KVH, qpg, D) @ k.transpose(1, 2) * D ** -0.5
+        want[i] = (s.softmax(-1) @ v).view(-1, D)
+        if n % bs:                            # the rest of a page is unused
+            kc[rows[-1].long(), :, n % bs:] = float("nan")
+            vc[rows[-1].long(), :, n % bs:] = float("nan")
+    lens = torch.tensor(lens, dtype=torch.int32)
+    return [t.cuda() for t in (q, kc, vc, bt, lens)], want
+
+
+def _close(got, want):
+    # half a step of bf16, and the 32-bit sums' error over the context
+    torch.testing.assert_close(got.double().cpu(), want, rtol=2 ** -8,
+                               atol=1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("qpg,bs", [(1, 16), (2, 16), (4, 16), (8, 16),
+                                    (4, 8), (2, 32), (8, 5)])
+@pytest.mark.parametrize("waves", [4, 8])
+def test_edges(qpg, bs, fp8, waves):
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case([1, 15, 16, 17, 31, 32, 33, 0, 127, 128, 129, 255, 256,
+                        257, 700], qpg, bs, fp8)
+    _close(ext.paged_attention(*args, D ** -0.5, waves=waves), want)
+    for parts, part in [(3, 256), (64, 11), (8, 96)]:
+        _close(ext.paged_attention_split(*args, parts, part, D ** -0.5,
+                                         waves=waves), want)
+
+
+@pytest.mark.gpu
+def test_running_maximum_far_apart():
+    """Scores that grow along the context move the maximum at every tile."""
+    args, _ = _case([600], 4, 16, False)
+    q, kc, vc, bt, lens = args
+    order = bt[0, :38].long()
+    for i, page in enumerate(order.tolist()):
+        kc[page] = q[0, 0] * (i - 20) * 0.2
+    k, v = (c[order].double().permute(1, 0, 2, 3).reshape(KVH, -1, D)[:, :600]
+            for c in (kc, vc))
+    s = q[0].double().view(KVH, 4, D) @ k.transpose(1, 2).contiguous() \
+        * D ** -0.5
+    want = (s.softmax(-1) @ v).view(1, -1, D).cpu()
+    _close(dispatch.paged_attention(*args, D ** -0.5, 600), want)
+    _close(dispatch.paged_attention(*args, D ** -0.5), want)
