@@ -1,5 +1,6 @@
 // ops.hip — torch binding of the layered-model kernels (`_hip_layered`).
 #include "check.h"
+#include "../linear_bind.h"
 
 extern "C" {
 hipError_t lds_stream_norm(int, int, const void* const*, int64_t, int, int,
@@ -485,6 +486,7 @@ void latent_prefill(Tensor q, Tensor kv, Tensor lat, Tensor positions,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "gfx950 kernels of the layer-listed designs";
+  linear_bind::bind(m);
   m.def("stream_norm", &stream_norm);
   m.def("embed_norm", &embed_norm);
   m.def("loop_norm", &loop_norm);

@@ -1,0 +1,130 @@
+// linear_bind.h — torch binding of linear_rows.hip, shared by the extensions.
+// Products go to the streaming kernel where its rule holds, else to the
+// library.
+#pragma once
+#include <torch/extension.h>
+#include <ATen/hip/HIPContext.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <torch/csrc/jit/frontend/tracer.h>
+
+#include <hip/hip_runtime.h>
+
+extern "C" {
+int lds_linear_rows_parts(int M, int N, int K);
+int lds_linear_rows_takes(int M, int N, int K, int gated, int parts);
+hipError_t lds_linear_rows(const void*, int64_t, const void*, int64_t, void*,
+                           float*, int, int, int, int, int, hipStream_t);
+hipError_t lds_gated_rows(const void*, int64_t, const void*, int64_t, void*,
+                          int, int, int, int, hipStream_t);
+hipError_t lds_lay_weights(const float*, void*, int, int, hipStream_t);
+}
+
+namespace linear_bind {
+
+using torch::Tensor;
+
+inline bool rows_of_16_bytes(const Tensor& t) {
+  return t.stride(1) == 1 && t.stride(0) % 8 == 0 &&
+         t.stride(0) >= t.size(1) && (uintptr_t)t.data_ptr() % 16 == 0;
+}
+
+enum Use { PLAIN, GATED, PARTS };
+
+// Whether x w' goes to the streaming kernel (where it is the faster one:
+// lds_linear_rows_takes). Tensors that autograd, a trace or a functional
+// transform follows stay with the library, as do odd layouts.
+inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
+  if (x.dim() != 2 || w.dim() != 2 || !x.is_cuda() ||
+      x.device() != w.device() || x.scalar_type() != at::kBFloat16 ||
+      w.scalar_type() != at::kBFloat16)
+    return false;
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  if (M < 1 || M > 128 || K < 8 || K % 8 || N < 8 || N % 8 ||
+      w.size(1) != K || N > (1 << 24) || K > (1 << 24) ||
+      (use == GATED && N % 16) ||
+      !lds_linear_rows_takes((int)M, (int)(use == GATED ? N / 2 : N), (int)K,
+                             use == GATED, use == PARTS))
+    return false;
+  if (at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad()))
+    return false;
+  for (const Tensor* t : {&x, &w})
+    if (!t->has_storage() || t->layout() != at::kStrided || t->is_neg() ||
+        t->_fw_grad(0).defined() ||
+        t->key_set().has(c10::DispatchKey::Python))
+      return false;
+  return !torch::jit::tracer::isTracing() && rows_of_16_bytes(x) &&
+         rows_of_16_bytes(w);
+}
+
+inline void check(hipError_t e) {
+  TORCH_CHECK(e == hipSuccess, "linear_rows: ", hipGetErrorString(e));
+}
+
+inline Tensor linear_rows(const Tensor& x, const Tensor& w, bool f32) {
+  const c10::DeviceGuard guard(x.device());
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  const auto wide = x.options().dtype(at::kFloat);
+  Tensor y = torch::empty({M, N}, f32 ? wide : x.options()), part;
+  const int parts = lds_linear_rows_parts(M, N, K);
+  if (parts > 1) part = torch::empty({parts, M, N}, wide);
+  check(lds_linear_rows(
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
+      parts > 1 ? part.data_ptr<float>() : nullptr, parts, M, N, K, f32,
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return y;
+}
+
+// x [M, K] @ w' of w [N, K]
+inline Tensor linear(const Tensor& x, const Tensor& w) {
+  return few_rows(x, w, PLAIN) ? linear_rows(x, w, false) : at::matmul(x, w.t());
+}
+
+// the same with a 32-bit result; None where the library has to do it
+inline c10::optional<Tensor> linear32(const Tensor& x, const Tensor& w) {
+  if (!few_rows(x, w, PLAIN)) return c10::nullopt;
+  return linear_rows(x, w, true);
+}
+
+// act(x gate') * (x up') of w [2 N, K] = [gate; up]; None where the product
+// and the activation have to be two calls
+inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
+                                          int64_t act) {
+  if (!few_rows(x, w, GATED)) return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0) / 2;
+  Tensor y = torch::empty({M, N}, x.options());
+  check(lds_gated_rows(
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), M, N,
+      K, (int)act, at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return y;
+}
+
+// drawn weights [in, out] in 32-bit -> [out, in] in bf16
+inline Tensor lay_weights(const Tensor& w) {
+  TORCH_CHECK(w.dim() == 2 && w.is_cuda() && w.is_contiguous() &&
+                  w.scalar_type() == at::kFloat,
+              "lay_weights takes contiguous 32-bit weights on the GPU");
+  if (w.size(0) % 8 || w.size(1) % 4 || w.numel() == 0 ||
+      w.size(0) > (1 << 21) || (uintptr_t)w.data_ptr() % 16)
+    return w.to(at::kBFloat16).t().contiguous();
+  const c10::DeviceGuard guard(w.device());
+  Tensor out = torch::empty({w.size(1), w.size(0)},
+                            w.options().dtype(at::kBFloat16));
+  check(lds_lay_weights(
+      w.data_ptr<float>(), out.data_ptr(), (int)w.size(0), (int)w.size(1),
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return out;
+}
+
+inline void bind(pybind11::module& m) {
+  m.def("lay_weights", &lay_weights, "[in, out] 32-bit -> [out, in] bf16");
+  m.def("linear", &linear, "x @ w' of w [N, K]");
+  m.def("linear32", &linear32, "the same with a 32-bit result, or None");
+  m.def("gated_linear", &gated_linear,
+        "act(x gate') * (x up') of w = [gate; up], or None");
+  m.def("few_rows",
+        [](const Tensor& x, const Tensor& w) { return few_rows(x, w, PLAIN); },
+        "whether x @ w' takes the streaming kernel");
+}
+
+}  // namespace linear_bind

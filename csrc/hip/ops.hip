@@ -7,6 +7,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "linear_bind.h"
+
 #define CHECK_HIP(expr)                                                    \
   do {                                                                     \
     hipError_t err__ = (expr);                                             \
@@ -326,6 +328,7 @@ torch::Tensor flash_prefill(torch::Tensor q, torch::Tensor k_cache,
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.doc() = "MI355X gfx950 kernels: prefix-cache hashing/match, paged KV, decode attention";
+  linear_bind::bind(m);
   m.def("hash_prompts", &hash_prompts, "batched chained block hashing");
   m.def("table_update", &table_update, "device prefix table insert/remove");
   m.def("match_longest", &match_longest, "device longest-prefix match");

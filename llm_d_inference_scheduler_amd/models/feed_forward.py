@@ -22,7 +22,7 @@ class GatedMLP:
         self.down = take("down").to(dtype)
 
     def __call__(self, h: torch.Tensor) -> Output:
-        return linear(ops.gated_act(linear(h, self.gate_up), self.spec.act),
+        return linear(ops.gated_linear(h, self.gate_up, self.spec.act),
                       self.down), None
 
 

@@ -1,7 +1,7 @@
 """Llama-family model runner (random-init weights, paged KV, bf16).
 
-MI355X-native execution path: plain-GEMM projections go through
-hipBLASLt/rocBLAS via torch.matmul; the fused hot ops (residual+RMSNorm,
+MI355X-native execution path: projections of few rows stream their weights
+through a HIP kernel, the rest go through hipBLASLt; the fused hot ops (residual+RMSNorm,
 RoPE, SiLU*up, GQA paged decode attention, KV scatter) are the gfx950 HIP
 kernels in csrc/hip dispatched through ops/. Prefill attention is composed
 chunked torch-matmul attention over KV gathered from the paged pool (an
@@ -20,34 +20,7 @@ import torch
 
 from .. import ops
 from ..ops import ref as ops_ref
-from ..utils.logging import get_logger
 from .configs import ModelConfig
-
-log = get_logger("models.llama")
-
-_TUNED_GEMM_LOADED = False
-
-
-def _load_tuned_gemms() -> None:
-    """Load offline hipBLASLt autotune results (tools/tune_gemms.py) so the
-    skinny decode GEMMs use tuned solutions instead of the default pick
-    (~2.6x off the weights-bound floor, profiles/r01_bench_kernel_stats_v3)."""
-    global _TUNED_GEMM_LOADED
-    if _TUNED_GEMM_LOADED:
-        return
-    _TUNED_GEMM_LOADED = True
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)),
-                        "..", "..", "profiles", "tuned_gemm_gfx950.csv")
-    if os.environ.get("LLMD_NO_TUNED_GEMM", "0") == "1":
-        # bisect knob: TunableOp is the prime suspect for the
-        # multi-stream wedge (profiles/r02_notes.md)
-        return
-    if os.path.exists(path):
-        import torch.cuda.tunable as tunable
-        tunable.enable(True)
-        tunable.tuning_enable(False)
-        tunable.read_file(path)
-        log.info("loaded tuned GEMM solutions", path=path)
 
 
 @dataclass
@@ -90,24 +63,31 @@ class LlamaRunner:
         self.scale = 1.0 / math.sqrt(config.head_dim)
         c = config
         if self.device.type == "cuda":
-            _load_tuned_gemms()
             # init directly on the GPU (16 GB of weights for Llama-3-8B —
             # CPU-side init would dominate startup). Same seed => identical
             # weights on every rank (required by the P/D KV hand-off).
             torch.cuda.manual_seed_all(seed)
 
-            def w(*shape, std=0.02):
-                t = torch.empty(*shape, dtype=torch.float32,
-                                device=self.device)
-                t.normal_(0.0, std)
-                return t.to(dtype)
+            def draw(shape, std):
+                return torch.empty(*shape, dtype=torch.float32,
+                                   device=self.device).normal_(0.0, std)
         else:
             gen = torch.Generator(device="cpu").manual_seed(seed)
 
-            def w(*shape, std=0.02):
-                t = torch.empty(*shape, dtype=torch.float32)
-                t.normal_(0.0, std, generator=gen)
-                return t.to(dtype).to(device)
+            def draw(shape, std):
+                return torch.empty(*shape, dtype=torch.float32).normal_(
+                    0.0, std, generator=gen)
+
+        def w(*shape, std=0.02):
+            return draw(shape, std).to(dtype).to(device)
+
+        def linear(n_in, n_out, std=0.02):
+            """[in, out] weights; on the GPU an output's weights lie together
+            in memory: the streaming kernel needs that, and the library's
+            large products run at 1490 TFLOP/s with it, 1280 without."""
+            if self.device.type != "cuda" or dtype != torch.bfloat16:
+                return w(n_in, n_out, std=std)
+            return ops.lay_weights(draw((n_in, n_out), std)).t()
 
         out_std = 0.02 / math.sqrt(2 * c.num_layers)
         self.embed = w(c.vocab_size, c.hidden_size)
@@ -116,8 +96,8 @@ class LlamaRunner:
             self.layers.append({
                 "input_norm": torch.ones(c.hidden_size, dtype=dtype,
                                          device=device),
-                "wqkv": w(c.hidden_size, c.q_size + 2 * c.kv_size),
-                "wo": w(c.q_size, c.hidden_size, std=out_std),
+                "wqkv": linear(c.hidden_size, c.q_size + 2 * c.kv_size),
+                "wo": linear(c.q_size, c.hidden_size, std=out_std),
                 "post_norm": torch.ones(c.hidden_size, dtype=dtype,
                                         device=device),
                 **({"q_norm": torch.ones(c.head_dim, dtype=dtype,
@@ -125,8 +105,9 @@ class LlamaRunner:
                     "k_norm": torch.ones(c.head_dim, dtype=dtype,
                                          device=device)}
                    if c.qk_norm else {}),
-                "wgate_up": w(c.hidden_size, 2 * c.intermediate_size),
-                "wdown": w(c.intermediate_size, c.hidden_size, std=out_std),
+                "wgate_up": linear(c.hidden_size, 2 * c.intermediate_size),
+                "wdown": linear(c.intermediate_size, c.hidden_size,
+                                std=out_std),
             })
         self.final_norm = torch.ones(c.hidden_size, dtype=dtype, device=device)
         self.lm_head = self.embed if c.tie_embeddings else \
@@ -159,7 +140,7 @@ class LlamaRunner:
             else:
                 normed = ops.rmsnorm(hidden, layer["input_norm"], c.rms_eps,
                                      residual=residual)
-            qkv = normed @ layer["wqkv"]
+            qkv = ops.linear(normed, layer["wqkv"].t())
             q, k, v = qkv.split([c.q_size, c.kv_size, c.kv_size], dim=-1)
             T = q.shape[0]
             q = q.view(T, c.num_heads, c.head_dim).contiguous()
@@ -187,12 +168,11 @@ class LlamaRunner:
                                            max_seq_len=batch.max_seq_len)
             else:
                 attn = self._prefill_attention(batch, q, k_cache, v_cache)
-            o = attn.view(T, c.q_size) @ layer["wo"]
+            o = ops.linear(attn.view(T, c.q_size), layer["wo"].t())
             normed2 = ops.rmsnorm(o, layer["post_norm"], c.rms_eps,
                                   residual=residual)
-            gate_up = normed2 @ layer["wgate_up"]
-            act = ops.silu_mul(gate_up)
-            hidden = act @ layer["wdown"]
+            act = ops.gated_linear(normed2, layer["wgate_up"].t())
+            hidden = ops.linear(act, layer["wdown"].t())
         final = ops.rmsnorm(hidden, self.final_norm, c.rms_eps,
                             residual=residual)
         # `residual` now holds the pre-norm sum; `final` the normed states
@@ -200,7 +180,7 @@ class LlamaRunner:
             return final
         rows = batch.logit_rows
         sel = final if rows is None else final[rows]
-        return sel @ self.lm_head.t()
+        return ops.linear(sel, self.lm_head)
 
     def _prefill_attention(self, batch: ForwardBatch, q: torch.Tensor,
                            k_cache: torch.Tensor,

@@ -34,6 +34,29 @@ def _use_hip(t: torch.Tensor) -> bool:
     return True
 
 
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x @ w' of w [out, in]: few rows stream the weights through the HIP
+    kernel, the rest is a library product."""
+    return _ext.linear(x, w) if _use_hip(x) else x @ w.t()
+
+
+def lay_weights(w: torch.Tensor) -> torch.Tensor:
+    """Weights drawn as [in, out] in 32-bit -> bf16 [out, in] on the GPU."""
+    return hip_ops().lay_weights(w)
+
+
+def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x gate') * (x up') of w = [gate; up], one call for few rows."""
+    if _use_hip(x):
+        y = _ext.gated_linear(x, w, _SILU)
+        if y is not None:
+            return y
+    return silu_mul(linear(x, w))
+
+
+_SILU = 1       # activation code of the kernels
+
+
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
             residual: Optional[torch.Tensor] = None) -> torch.Tensor:
     if _use_hip(x):

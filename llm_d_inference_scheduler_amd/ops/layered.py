@@ -28,11 +28,26 @@ ACTS = {"gelu_tanh": 0, "silu": 1, "relu_squared": 2}
 
 
 def linear(x, w):
-    return x @ w.t()
+    """x @ w': few rows stream the weights through the HIP kernel, the rest
+    is a library product."""
+    return hip_layered().linear(x, w) if x.is_cuda else x @ w.t()
+
+
+def gated_linear(x, w, act):
+    """act(x gate') * (x up') of w = [gate; up], one call for few rows."""
+    if x.is_cuda:
+        y = hip_layered().gated_linear(x, w, ACTS[act])
+        if y is not None:
+            return y
+    return gated_act(linear(x, w), act)
 
 
 def linear32(x, w):
     """x @ w' with a 32-bit result."""
+    if x.is_cuda:
+        y = hip_layered().linear32(x, w)
+        if y is not None:
+            return y
     if x.is_cuda and x.dtype != torch.float32:
         return torch.mm(x, w.t(), out_dtype=torch.float32)
     return x.float() @ w.float().t()

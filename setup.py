@@ -13,8 +13,8 @@ files live inside the package and travel with the repo snapshot:
 
 LDS_AMD_ONLY=name,... builds only the named modules (e.g. _hip_layered).
 """
+import glob
 import os
-import sys
 
 from setuptools import setup
 
@@ -25,6 +25,22 @@ from torch.utils import cpp_extension
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
 
+
+
+def drop_stale_objects():
+    """The compile rules of HIP sources do not follow includes: an object
+    older than a header is deleted, so that it is made again."""
+    headers = glob.glob(os.path.join(ROOT, "csrc", "**", "*.h"),
+                        recursive=True)
+    newest = max(os.path.getmtime(h) for h in headers
+                 if not h.endswith("_hip.h"))       # made by the build
+    for o in glob.glob(os.path.join(ROOT, "build", "**", "*.o"),
+                       recursive=True):
+        if os.path.getmtime(o) < newest:
+            os.remove(o)
+
+
+drop_stale_objects()
 router_core = Pybind11Extension(
     "llm_d_inference_scheduler_amd._router_core",
     sources=["csrc/router/bindings.cpp"],
@@ -44,6 +60,7 @@ hip_ops = cpp_extension.CUDAExtension(
     name="llm_d_inference_scheduler_amd._hip_ops",
     sources=[
         "csrc/hip/ops.hip",
+        "csrc/hip/linear_rows.hip",
         "csrc/hip/prefix_kernels.hip",
         "csrc/hip/norm_rope_act.hip",
         "csrc/hip/kv_cache.hip",
@@ -58,6 +75,7 @@ hip_layered = cpp_extension.CUDAExtension(
     name="llm_d_inference_scheduler_amd._hip_layered",
     sources=[
         "csrc/hip/layered/ops.hip",
+        "csrc/hip/linear_rows.hip",
         "csrc/hip/layered/residual_norm.hip",
         "csrc/hip/layered/delta_rule.hip",
         "csrc/hip/layered/delta_chunk.hip",

@@ -1,0 +1,137 @@
+"""Products of few rows that stream their weights: edges of row tiles, channel
+blocks, steps and parts of K, and the calls that stay with the library,
+against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EXTENSIONS = ["_hip_ops", "_hip_layered"]
+
+
+def _ext(name):
+    import importlib
+    return importlib.import_module(f"llm_d_inference_scheduler_amd.{name}")
+
+
+def _draw(*shape, seed=0, scale=1.0):
+    g = torch.Generator("cuda").manual_seed(seed)
+    return (torch.randn(*shape, device="cuda", generator=g) *
+            scale).bfloat16()
+
+
+def _same(got, want, bits):
+    """Sums of 32 bits over K products of size 1 / sqrt(K): far below 1e-5;
+    the result is rounded to `bits` bits."""
+    torch.testing.assert_close(got.double(), want, rtol=2.0 ** -bits,
+                               atol=2e-5)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 15, 16, 17, 32, 33, 63, 64, 65, 96,
+                                  97, 128, 129])
+@pytest.mark.parametrize("n,k", [(8, 8), (120, 64), (128, 136), (136, 520),
+                                 (1032, 1000), (264, 4096), (33032, 72),
+                                 (4104, 256), (30000, 264)])
+def test_product(rows, n, k):
+    ext = _ext("_hip_ops")
+    x, w = _draw(rows, k, seed=rows), _draw(n, k, seed=n, scale=k ** -0.5)
+    want = x.double() @ w.double().t()
+    _same(ext.linear(x, w), want, 8)
+    wide = ext.linear32(x, w)
+    assert (wide is None) == (not ext.few_rows(x, w))
+    assert ext.few_rows(x, w) or rows > 32
+    if wide is not None:
+        _same(wide, want, 16)
+
+
+@pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("rows", [1, 17, 40, 64, 65])
+@pytest.mark.parametrize("n,k", [(8, 64), (72, 200), (520, 128),
+                                 (16384, 48), (16400, 48)])
+def test_gated(name, rows, n, k):
+    """The last block partly empty; what the library does better gives
+    None."""
+    F = torch.nn.functional
+    x = _draw(rows, k, seed=rows)
+    w = _draw(2 * n, k, seed=n, scale=k ** -0.5)
+    g, u = (x.double() @ w.double().t()).chunk(2, -1)
+    for act, fn in enumerate([lambda z: F.gelu(z, approximate="tanh"), F.silu,
+                              lambda z: z.relu().square()]):
+        y = _ext(name).gated_linear(x, w, act)
+        assert (y is None) == (rows > 64 or n > 16384)
+        if y is not None:
+            _same(y, fn(g) * u, 8)
+
+
+def test_rows_apart():
+    """Slices of wider tensors, as the decay and gate projections take."""
+    ext = _ext("_hip_layered")
+    x, w = _draw(30, 400, seed=1), _draw(64, 304, seed=2)
+    a, b = x[:, 16:16 + 136], w[:, 8:8 + 136]
+    assert ext.few_rows(a, b)
+    torch.testing.assert_close(ext.linear(a, b).double(),
+                               a.double() @ b.double().t(), rtol=2 ** -8,
+                               atol=1e-3)
+
+
+def test_calls_that_stay_with_the_library():
+    ext = _ext("_hip_layered")
+    x, w = _draw(20, 256, seed=3), _draw(64, 256, seed=4, scale=1 / 16)
+    want = x.double() @ w.double().t()
+    flat = _draw(20 * 256 + 8, seed=5)
+    odd = flat[1:1 + 20 * 256].view(20, 256).copy_(x)   # not 16-byte aligned
+    across = x.t().contiguous().t()
+    for a in (odd, across):
+        assert not ext.few_rows(a, w)
+        _same(ext.linear(a, w), want, 8)
+    assert not ext.few_rows(x, w.t().contiguous().t())
+    _same(ext.linear(x, w.t().contiguous().t()), want, 8)
+    _same(ext.linear(x.view(4, 5, 256), w).view(20, 64), want, 8)
+    _same(ext.linear(x[3], w), want[3], 8)
+    assert ext.linear(x[:0], w).shape == (0, 64)
+    f = ext.linear(x.float(), w.float())
+    assert f.dtype == torch.float32 and not ext.few_rows(x.float(), w.float())
+    for k, n in ((252, 64), (256, 60)):
+        a, b = _draw(5, k, seed=6), _draw(n, k, seed=7, scale=1 / 16)
+        assert not ext.few_rows(a, b)
+        _same(ext.linear(a, b), a.double() @ b.double().t(), 8)
+    with pytest.raises(RuntimeError):
+        ext.linear(x, w[:, :128])
+    with pytest.raises(RuntimeError):
+        ext.linear(x, w.float())
+
+
+def test_gradients_pass():
+    ext = _ext("_hip_layered")
+    x = _draw(6, 64, seed=8).requires_grad_()
+    w = _draw(32, 64, seed=9).requires_grad_()
+    ext.linear(x, w).float().sum().backward()
+    assert x.grad.shape == x.shape and w.grad.shape == w.shape
+    with torch.no_grad():
+        assert ext.few_rows(x, w)
+
+
+def test_capture_and_replay():
+    """Partial sums are written anew by every replay."""
+    ext = _ext("_hip_ops")
+    x, w = _draw(12, 2048, seed=10), _draw(256, 2048, seed=11, scale=1 / 45)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        ext.linear(x, w)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = ext.linear(x, w)
+    for i in range(3):
+        x.copy_(_draw(12, 2048, seed=20 + i))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ext.linear(x, w))
+
+
+@pytest.mark.parametrize("r,c", [(8, 4), (64, 64), (72, 132), (200, 68),
+                                 (12, 20), (8, 6)])
+def test_lay_weights(r, c):
+    w = _draw(r, c, seed=r).float() * 1.2345
+    got = _ext("_hip_ops").lay_weights(w)
+    assert got.is_contiguous() and torch.equal(got, w.bfloat16().t())

@@ -1,4 +1,4 @@
-"""hipBLASLt GEMM throughput at the serving shapes (run on a GPU box)."""
+"""Throughput of the projections at the serving shapes (run on a GPU)."""
 import os
 import sys
 import time
@@ -8,8 +8,7 @@ sys.path.insert(0, os.path.join(os.path.dirname(
 
 import torch  # noqa: E402
 
-from llm_d_inference_scheduler_amd.models.llama import \
-    _load_tuned_gemms  # noqa: E402
+from llm_d_inference_scheduler_amd import ops  # noqa: E402
 
 SHAPES = [(4096, 6144, "qkv"), (4096, 4096, "wo"),
           (4096, 28672, "gate_up"), (14336, 4096, "down")]
@@ -17,13 +16,13 @@ SHAPES = [(4096, 6144, "qkv"), (4096, 4096, "wo"),
 
 def bench(m, k, n, tag, iters=30):
     a = torch.randn(m, k, device="cuda", dtype=torch.bfloat16)
-    b = torch.randn(k, n, device="cuda", dtype=torch.bfloat16)
+    b = torch.randn(n, k, device="cuda", dtype=torch.bfloat16)
     for _ in range(5):
-        a @ b
+        ops.linear(a, b)
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for _ in range(iters):
-        a @ b
+        ops.linear(a, b)
     torch.cuda.synchronize()
     us = (time.perf_counter() - t0) / iters * 1e6
     tf = 2 * m * k * n / (us / 1e6) / 1e12
@@ -31,8 +30,7 @@ def bench(m, k, n, tag, iters=30):
 
 
 if __name__ == "__main__":
-    _load_tuned_gemms()
-    for m in (1024, 2048, 4096, 8192):
+    for m in (1, 16, 64, 128, 256, 1024, 2048, 4096, 8192):
         for k, n, tag in SHAPES:
             bench(m, k, n, tag)
         print()
