@@ -4,7 +4,7 @@
 
 extern "C" {
 hipError_t lds_stream_norm(int, int, const void* const*, int64_t, int, int,
-                           float, float, float, hipStream_t);
+                           int, float, float, float, hipStream_t);
 hipError_t lds_act(int, int, const void*, void*, int64_t, int, int,
                    hipStream_t);
 hipError_t lds_delta_prep(int, const void*, int64_t, const float*, void*,
@@ -74,7 +74,13 @@ Tensor stream_norm(Tensor x, OptTensor y, OptTensor wb, OptTensor wn,
   const int64_t rows = x.size(0), H = x.size(1);
   check_norm(wn, H, "wn");
   check_norm(wb, H, "wb");
-  if (y) {
+  int parts = 0;
+  if (y && y->dim() == 3) {      // partial sums of a product
+    check(*y, at::kFloat, "y");
+    TORCH_CHECK(y->size(0) > 0, "y");
+    parts = (int)y->size(0);
+    sized(*y, {parts, rows, H}, "y");
+  } else if (y) {
     same_act(*y, f32, "y");
     sized(*y, {rows, H}, "y");
   }
@@ -90,8 +96,8 @@ Tensor stream_norm(Tensor x, OptTensor y, OptTensor wb, OptTensor wn,
   const void* ptr[12] = {x.data_ptr(), ptr_or_null(y), nullptr, nullptr,
                          nullptr, ptr_or_null(wb), ptr_or_null(added), nullptr,
                          nullptr, nullptr, ptr_or_null(wn), h.data_ptr()};
-  check_hip(lds_stream_norm(f32, wb ? POST : ADD, ptr, rows, (int)n, (int)H,
-                            1.f, (float)offset, (float)eps, cur_stream()),
+  check_hip(lds_stream_norm(f32, wb ? POST : ADD, ptr, rows, parts, (int)n,
+                            (int)H, 1.f, (float)offset, (float)eps, cur_stream()),
             "stream_norm");
   return h;
 }
@@ -117,7 +123,7 @@ std::vector<Tensor> embed_norm(Tensor ids, Tensor table, double scale,
                          pos ? positions->data_ptr() : nullptr, nullptr,
                          nullptr, nullptr, nullptr, nullptr, ptr_or_null(wn),
                          h.data_ptr()};
-  check_hip(lds_stream_norm(f32, EMBED, ptr, rows, 0, (int)H, (float)scale,
+  check_hip(lds_stream_norm(f32, EMBED, ptr, rows, 0, 0, (int)H, (float)scale,
                             (float)offset, (float)eps, cur_stream()),
             "embed_norm");
   return {x, h};
@@ -140,7 +146,7 @@ Tensor loop_norm(Tensor x, Tensor a, Tensor b, Tensor v, OptTensor wn,
   const void* ptr[12] = {x.data_ptr(), nullptr, nullptr, nullptr, nullptr,
                          nullptr, nullptr, a.data_ptr(), b.data_ptr(),
                          v.data_ptr(), ptr_or_null(wn), h.data_ptr()};
-  check_hip(lds_stream_norm(f32, LOOP, ptr, rows, 0, (int)H, 1.f,
+  check_hip(lds_stream_norm(f32, LOOP, ptr, rows, 0, 0, (int)H, 1.f,
                             (float)offset, (float)eps, cur_stream()),
             "loop_norm");
   return h;

@@ -79,6 +79,22 @@ inline Tensor linear(const Tensor& x, const Tensor& w) {
   return few_rows(x, w, PLAIN) ? linear_rows(x, w, false) : at::matmul(x, w.t());
 }
 
+// the same for a caller that sums the parts of K itself: [M, N], or 32-bit
+// [parts, M, N]
+inline Tensor linear_parts(const Tensor& x, const Tensor& w) {
+  if (!few_rows(x, w, PARTS)) return linear_bind::linear(x, w);
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  const int parts = lds_linear_rows_parts(M, N, K);
+  if (parts == 1) return linear_rows(x, w, false);
+  const c10::DeviceGuard guard(x.device());
+  Tensor part = torch::empty({parts, M, N}, x.options().dtype(at::kFloat));
+  check(lds_linear_rows(
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), nullptr,
+      part.data_ptr<float>(), parts, M, N, K, 0,
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return part;
+}
+
 // the same with a 32-bit result; None where the library has to do it
 inline c10::optional<Tensor> linear32(const Tensor& x, const Tensor& w) {
   if (!few_rows(x, w, PLAIN)) return c10::nullopt;
@@ -119,6 +135,7 @@ inline Tensor lay_weights(const Tensor& w) {
 inline void bind(pybind11::module& m) {
   m.def("lay_weights", &lay_weights, "[in, out] 32-bit -> [out, in] bf16");
   m.def("linear", &linear, "x @ w' of w [N, K]");
+  m.def("linear_parts", &linear_parts, "the same, or its parts of K");
   m.def("linear32", &linear32, "the same with a 32-bit result, or None");
   m.def("gated_linear", &gated_linear,
         "act(x gate') * (x up') of w = [gate; up], or None");

@@ -14,72 +14,208 @@ namespace {
 //   if residual: r = r + x  (written back);  src = r
 //   else:        src = x
 //   y = src * rsqrt(mean(src^2) + eps) * w
-// One block (256 threads) per token row; row length H % 8 == 0.
-// Values are cached in registers between the sum-of-squares pass and the
-// normalize pass (up to CACHE_CHUNKS*8 elems/thread), avoiding a second HBM
-// read for H <= 256*CACHE_CHUNKS*8 (= 16384 at CACHE_CHUNKS=8).
+// x is bf16, or the partial sums of a product that split K: [parts, rows, H]
+// 32-bit, summed here instead of by a launch of their own (8 parts, one row of
+// 4096: 6.5 us; sum and norm apart 8.7).
+// One block (256 threads) per token row; row length H % 8 == 0. The first KEEP
+// vectors of a thread stay in registers between the two passes, the rest are
+// read again. Their number is known at compile time: an index that is not puts
+// the array into scratch memory (8013 rows of 4096 with residual: 84 us, now
+// 44, 5.9 TB/s).
 // ---------------------------------------------------------------------------
-template <bool RESIDUAL>
-__global__ void rmsnorm_kernel(const short* __restrict__ x,
-                               short* __restrict__ residual,
-                               const short* __restrict__ w,
-                               short* __restrict__ y, int H, float eps) {
-  constexpr int CACHE_CHUNKS = 8;
-  __shared__ float red[16];
-  const int64_t row = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int nthreads = blockDim.x;
-  const short8* x8 = (const short8*)(x + row * H);
-  short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
-  const short8* w8 = (const short8*)w;
-  short8* y8 = (short8*)(y + row * H);
-  const int nchunks = H / 8;
+constexpr int NT = 256;
 
-  float vals[CACHE_CHUNKS][8];
-  float ss = 0.f;
-  int ci = 0;
-  for (int c = tid; c < nchunks; c += nthreads, ++ci) {
-    short8 v = x8[c];
-    float f[8];
+template <int KEEP, bool RESIDUAL, bool PARTS>
+__global__ __launch_bounds__(NT) void rmsnorm_kernel(
+    const void* __restrict__ x, int parts, short* __restrict__ residual,
+    const short* __restrict__ w, short* __restrict__ y, int H, float eps) {
+  __shared__ float red[NT / WAVE];
+  const int64_t row = blockIdx.x;
+  const int nchunks = H / 8;
+  short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
+  auto source = [&](int c, float* f) {
+    if constexpr (PARTS) {
+      const float4v* p = (const float4v*)x + (row * H + c * 8) / 4;
+      const int64_t apart = (int64_t)gridDim.x * H / 4;
+      float4v a = p[0], b = p[1];
+#pragma unroll 4
+      for (int i = 1; i < parts; ++i) {
+        a += p[i * apart];
+        b += p[i * apart + 1];
+      }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
+      for (int j = 0; j < 4; ++j) {
+        f[j] = a[j];
+        f[4 + j] = b[j];
+      }
+    } else {
+      const short8 v = ((const short8*)((const short*)x + row * H))[c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
+    }
+  };
+  float vals[KEEP][8], ss = 0.f;
+  auto first = [&](int c, float* f) {
+    source(c, f);
     if constexpr (RESIDUAL) {
-      short8 r = r8[c];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] += bf16_to_f32(r[j]);
+      const short8 r = r8[c];
       short8 ro;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ro[j] = f32_to_bf16(f[j]);
+      for (int j = 0; j < 8; ++j) {
+        f[j] += bf16_to_f32(r[j]);
+        ro[j] = f32_to_bf16(f[j]);
+      }
       r8[c] = ro;  // residual stream updated in place
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss += f[j] * f[j];
-    if (ci < CACHE_CHUNKS) {
+  };
 #pragma unroll
-      for (int j = 0; j < 8; ++j) vals[ci][j] = f[j];
-    }
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < nchunks) first(c, vals[i]);
   }
-  float total = block_reduce_sum<4>(ss, red);
-  const float inv = rsqrtf(total / (float)H + eps);
-
-  ci = 0;
-  for (int c = tid; c < nchunks; c += nthreads, ++ci) {
+  for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
     float f[8];
-    if (ci < CACHE_CHUNKS) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = vals[ci][j];
-    } else {
-      // overflow path for very large H: re-read (residual already folded in)
-      short8 v = RESIDUAL ? r8[c] : x8[c];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
-    }
-    short8 wv = w8[c];
+    first(c, f);
+  }
+  const float inv =
+      rsqrtf(block_reduce_sum<NT / WAVE>(ss, red) / (float)H + eps);
+  auto second = [&](int c, const float* f) {
+    const short8 wv = ((const short8*)w)[c];
     short8 o;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = f32_to_bf16(f[j] * inv * bf16_to_f32(wv[j]));
-    y8[c] = o;
+    for (int j = 0; j < 8; ++j)
+      o[j] = f32_to_bf16(f[j] * inv * bf16_to_f32(wv[j]));
+    ((short8*)(y + row * H))[c] = o;
+  };
+#pragma unroll
+  for (int i = 0; i < KEEP; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < nchunks) second(c, vals[i]);
   }
+  for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
+    float f[8];
+    if constexpr (RESIDUAL) {   // this thread's own store above
+      const short8 v = r8[c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
+    } else {
+      source(c, f);
+    }
+    second(c, f);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// What lies between a decoder layer's qkv product and its attention, in one
+// pass: heads of q and k are normed (Qwen3; where qw is set), rotated
+// (rotate-half, angles from the host's table) and rounded; q goes to a packed
+// [T, QH, D], k and v to their slots in the paged cache.
+//   qkv: [T, QH + 2 KVH heads, D] bf16, rows apart by `stride` elements, or
+//   the 32-bit partial sums [parts, T, ..] of the product
+// A thread owns 8 channels of a head's first half and the 8 they rotate with;
+// D / 16 threads share a head. Bound by its bytes: it reads and writes each
+// value once, where separate copies, rotation and scatter took five passes
+// (8013 rows of 48 heads: 37 us, was 142).
+// ---------------------------------------------------------------------------
+struct Heads {
+  const void* qkv;
+  int parts;
+  int64_t stride;
+  const short *qw, *kw;          // [D] or null
+  const float* cos_sin;          // [max_pos, D / 2, 2]
+  const int32_t* positions;      // [T]
+  const int64_t* slots;          // [T], below 0: not cached
+  short* q;                      // [T, QH, D]
+  void *k_cache, *v_cache;       // [NB, KVH, BS, D]
+  int T, qh, kvh, bs, d;
+  float eps;
+};
+
+template <typename CT, bool PARTS, bool NORM>
+__global__ __launch_bounds__(NT) void heads_kernel(const Heads p) {
+  const int per = p.d / 16, heads = p.qh + 2 * p.kvh, half = p.d / 2;
+  const uint32_t i = blockIdx.x * NT + threadIdx.x, hd = i / per;
+  const int t = hd / heads, h = hd % heads, c = i % per * 8;
+  if (t >= p.T) return;          // whole heads: lanes of one stay together
+  float f[2][8];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int64_t at = t * p.stride + h * p.d + s * half + c;
+    if constexpr (PARTS) {
+      const float4v* src = (const float4v*)((const float*)p.qkv + at);
+      const int64_t apart = p.T * p.stride / 4;
+      float4v a = src[0], b = src[1];
+#pragma unroll 4
+      for (int k = 1; k < p.parts; ++k) {
+        a += src[k * apart];
+        b += src[k * apart + 1];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        f[s][j] = a[j];
+        f[s][4 + j] = b[j];
+      }
+    } else {
+      const short8 v = *(const short8*)((const short*)p.qkv + at);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[s][j] = bf16_to_f32(v[j]);
+    }
+  }
+  const bool value = h >= p.qh + p.kvh, key = !value && h >= p.qh;
+  if (NORM) {
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      ss += f[0][j] * f[0][j] + f[1][j] * f[1][j];
+    for (int o = 1; o < per; o <<= 1) ss += __shfl_xor(ss, o, WAVE);
+    if (!value) {
+      const float inv = rsqrtf(ss / (float)p.d + p.eps);
+      const short* w = key ? p.kw : p.qw;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const short8 wv = *(const short8*)(w + s * half + c);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[s][j] *= inv * bf16_to_f32(wv[j]);
+      }
+    }
+  }
+  short8 lo, hi;
+  if (value) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      lo[j] = f32_to_bf16(f[0][j]);
+      hi[j] = f32_to_bf16(f[1][j]);
+    }
+  } else {
+    const float4v* cs = (const float4v*)(
+        p.cos_sin + ((int64_t)p.positions[t] * half + c) * 2);
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      const float4v a = cs[j / 2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float co = a[2 * k], si = a[2 * k + 1];
+        const float u = f[0][j + k], v = f[1][j + k];
+        lo[j + k] = f32_to_bf16(u * co - v * si);
+        hi[j + k] = f32_to_bf16(v * co + u * si);
+      }
+    }
+  }
+  if (h < p.qh) {
+    short* o = p.q + ((int64_t)t * p.qh + h) * p.d + c;
+    *(short8*)o = lo;
+    *(short8*)(o + half) = hi;
+    return;
+  }
+  const int64_t slot = p.slots[t];
+  if (slot < 0) return;          // padding token
+  const int kh = h - p.qh - (value ? p.kvh : 0);
+  CT* o = (CT*)(value ? p.v_cache : p.k_cache) +
+          ((slot / p.bs * p.kvh + kh) * p.bs + slot % p.bs) * p.d + c;
+  store_kv8(o, lo);
+  store_kv8(o + half, hi);
 }
 
 // ---------------------------------------------------------------------------
@@ -142,19 +278,68 @@ __global__ void silu_mul_kernel(const short* __restrict__ gate_up,
 
 extern "C" {
 
-hipError_t lds_rmsnorm(const void* x, void* residual, const void* w, void* y,
-                       int64_t n_rows, int H, float eps, hipStream_t stream) {
+// parts > 0: x are that many partial sums in 32-bit
+hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
+                       void* y, int64_t n_rows, int H, float eps,
+                       hipStream_t stream) {
   if (n_rows == 0) return hipSuccess;
-  dim3 grid((uint32_t)n_rows), block(256);
-  if (residual) {
-    hipLaunchKernelGGL(rmsnorm_kernel<true>, grid, block, 0, stream,
-                       (const short*)x, (short*)residual, (const short*)w,
-                       (short*)y, H, eps);
+#define GO(KEEP, RES, PARTS)                                                 \
+  hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS>),                     \
+                     dim3((uint32_t)n_rows), dim3(NT), 0, stream, x, parts,  \
+                     (short*)residual, (const short*)w, (short*)y, H, eps)
+#define GO_K(RES, PARTS)                                                     \
+  do {                                                                       \
+    if (H <= 1 * NT * 8) GO(1, RES, PARTS);                                  \
+    else if (H <= 2 * NT * 8) GO(2, RES, PARTS);                             \
+    else GO(4, RES, PARTS);                                                  \
+  } while (0)
+  if (parts > 0) {
+    if (residual) GO_K(true, true); else GO_K(false, true);
   } else {
-    hipLaunchKernelGGL(rmsnorm_kernel<false>, grid, block, 0, stream,
-                       (const short*)x, nullptr, (const short*)w, (short*)y, H,
-                       eps);
+    if (residual) GO_K(true, false); else GO_K(false, false);
   }
+#undef GO_K
+#undef GO
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
+// 1 if heads of D channels have the one-pass form
+int lds_heads_ok(int d, int norm) {
+  const int per = d / 16;
+  return d >= 16 && d % 16 == 0 &&
+         (!norm || (per <= WAVE && (per & (per - 1)) == 0));
+}
+
+// see Heads; parts > 0: qkv are that many partial sums in 32-bit
+hipError_t lds_heads(const void* qkv, int parts, int64_t stride,
+                     const void* qw, const void* kw, const float* cos_sin,
+                     const int32_t* positions, const int64_t* slots, void* q,
+                     void* k_cache, void* v_cache, int T, int qh, int kvh,
+                     int bs, int d, int kv_fp8, float eps,
+                     hipStream_t stream) {
+  if (T == 0) return hipSuccess;
+  const int64_t n = (int64_t)T * (qh + 2 * kvh) * (d / 16);
+  if (!lds_heads_ok(d, qw != nullptr) || stride % 8 || n >= 1ll << 31)
+    return hipErrorInvalidValue;
+  const Heads p{qkv, parts, stride, (const short*)qw, (const short*)kw,
+                cos_sin, positions, slots, (short*)q, k_cache, v_cache, T, qh,
+                kvh, bs, d, eps};
+  const dim3 grid((uint32_t)((n + NT - 1) / NT));
+#define GO(CT, PARTS, NORM)                                                  \
+  hipLaunchKernelGGL((heads_kernel<CT, PARTS, NORM>), grid, dim3(NT), 0,     \
+                     stream, p)
+#define GO_CT(PARTS, NORM)                                                   \
+  do {                                                                       \
+    if (kv_fp8) GO(unsigned char, PARTS, NORM); else GO(short, PARTS, NORM); \
+  } while (0)
+  if (parts > 0) {
+    if (qw) GO_CT(true, true); else GO_CT(true, false);
+  } else {
+    if (qw) GO_CT(false, true); else GO_CT(false, false);
+  }
+#undef GO_CT
+#undef GO
   HIP_CHECK_LAST();
   return hipSuccess;
 }

@@ -25,8 +25,13 @@ hipError_t lds_table_update(uint64_t*, unsigned long long*, uint32_t,
 hipError_t lds_match_longest(const uint64_t*, const unsigned long long*,
                              uint32_t, const uint64_t*, const int32_t*, int,
                              int, int, int32_t*, hipStream_t);
-hipError_t lds_rmsnorm(const void*, void*, const void*, void*, int64_t, int,
-                       float, hipStream_t);
+hipError_t lds_rmsnorm(const void*, int, void*, const void*, void*, int64_t,
+                       int, float, hipStream_t);
+int lds_heads_ok(int, int);
+hipError_t lds_heads(const void*, int, int64_t, const void*, const void*,
+                     const float*, const int32_t*, const int64_t*, void*,
+                     void*, void*, int, int, int, int, int, int, float,
+                     hipStream_t);
 hipError_t lds_rope(void*, void*, const float*, const int32_t*, int, int, int,
                     int, hipStream_t);
 hipError_t lds_silu_mul(const void*, void*, int64_t, int, hipStream_t);
@@ -114,21 +119,76 @@ torch::Tensor match_longest(torch::Tensor keys, torch::Tensor masks,
 
 // ---- engine kernels ----
 
+// x: bf16 rows, or 32-bit partial sums [parts, rows, H] of a product
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
                       c10::optional<torch::Tensor> residual) {
   CHECK_GPU(x); CHECK_GPU(w);
-  TORCH_CHECK(x.dtype() == torch::kBFloat16, "rmsnorm expects bf16");
-  auto y = torch::empty_like(x);
+  const bool parts = x.dim() == 3 && x.dtype() == torch::kFloat32;
+  TORCH_CHECK(parts || x.dtype() == torch::kBFloat16, "rmsnorm expects bf16");
+  TORCH_CHECK(!parts || (x.size(0) > 0 && x.size(2) % 8 == 0 &&
+                         w.numel() == x.size(2)), "rmsnorm parts");
+  auto y = parts ? torch::empty({x.size(1), x.size(2)},
+                                x.options().dtype(torch::kBFloat16))
+                 : torch::empty_like(x);
   int H = (int)x.size(-1);
-  int64_t rows = x.numel() / H;
+  int64_t rows = y.numel() / H;
   void* res_ptr = nullptr;
   if (residual.has_value()) {
     CHECK_GPU(*residual);
+    TORCH_CHECK(!parts || residual->numel() == y.numel(), "residual");
     res_ptr = residual->data_ptr();
   }
-  CHECK_HIP(lds_rmsnorm(x.data_ptr(), res_ptr, w.data_ptr(), y.data_ptr(),
-                        rows, H, (float)eps, cur_stream()));
+  CHECK_HIP(lds_rmsnorm(x.data_ptr(), parts ? (int)x.size(0) : 0, res_ptr,
+                        w.data_ptr(), y.data_ptr(), rows, H, (float)eps,
+                        cur_stream()));
   return y;
+}
+
+// qkv [T, heads * D] bf16 or 32-bit partial sums [parts, T, heads * D]: q and
+// k normed (optional) and rotated, k and v into the cache -> q [T, QH, D];
+// None where the heads have no such form
+c10::optional<torch::Tensor> rope_and_cache(
+    torch::Tensor qkv, int64_t qh, torch::Tensor cos_sin,
+    torch::Tensor positions, torch::Tensor k_cache, torch::Tensor v_cache,
+    torch::Tensor slots, c10::optional<torch::Tensor> q_norm,
+    c10::optional<torch::Tensor> k_norm, double eps) {
+  CHECK_GPU(qkv); CHECK_GPU(cos_sin); CHECK_GPU(positions);
+  CHECK_GPU(k_cache); CHECK_GPU(v_cache); CHECK_GPU(slots);
+  const bool parts = qkv.dim() == 3;
+  TORCH_CHECK(qkv.dtype() == (parts ? torch::kFloat32 : torch::kBFloat16) &&
+                  (parts || qkv.dim() == 2),
+              "qkv is bf16 rows or 32-bit parts of them");
+  TORCH_CHECK(positions.dtype() == torch::kInt32 &&
+                  slots.dtype() == torch::kInt64 &&
+                  cos_sin.dtype() == torch::kFloat32 && k_cache.dim() == 4 &&
+                  k_cache.sizes() == v_cache.sizes(),
+              "rope_and_cache types");
+  const int64_t T = qkv.size(-2), stride = qkv.size(-1);
+  const int kvh = (int)k_cache.size(1), bs = (int)k_cache.size(2);
+  const int d = (int)k_cache.size(3);
+  TORCH_CHECK(stride == (qh + 2 * kvh) * d && positions.numel() == T &&
+                  slots.numel() == T && cos_sin.dim() == 3 &&
+                  cos_sin.size(1) * 2 == d, "rope_and_cache sizes");
+  TORCH_CHECK(q_norm.has_value() == k_norm.has_value(), "q_norm, k_norm");
+  for (auto& w : {q_norm, k_norm})
+    if (w) {
+      CHECK_GPU(*w);
+      TORCH_CHECK(w->dtype() == torch::kBFloat16 && w->numel() == d, "norm");
+    }
+  if (!lds_heads_ok(d, q_norm.has_value()) ||
+      T * (qh + 2 * kvh) * (d / 16) >= (1ll << 31) ||
+      ((uintptr_t)qkv.data_ptr() | (uintptr_t)k_cache.data_ptr() |
+       (uintptr_t)v_cache.data_ptr() | (uintptr_t)cos_sin.data_ptr()) % 16)
+    return c10::nullopt;
+  auto q = torch::empty({T, qh, d}, qkv.options().dtype(torch::kBFloat16));
+  CHECK_HIP(lds_heads(
+      qkv.data_ptr(), parts ? (int)qkv.size(0) : 0, stride,
+      q_norm ? q_norm->data_ptr() : nullptr,
+      k_norm ? k_norm->data_ptr() : nullptr, cos_sin.data_ptr<float>(),
+      positions.data_ptr<int32_t>(), slots.data_ptr<int64_t>(), q.data_ptr(),
+      k_cache.data_ptr(), v_cache.data_ptr(), (int)T, (int)qh, kvh, bs, d,
+      kv_fp8_flag(k_cache), (float)eps, cur_stream()));
+  return q;
 }
 
 void rope(torch::Tensor q, torch::Tensor k, torch::Tensor cos_sin,
@@ -335,6 +395,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm, py::arg("x"), py::arg("w"), py::arg("eps"),
         py::arg("residual") = py::none());
   m.def("rope", &rope, "in-place NeoX RoPE");
+  m.def("rope_and_cache", &rope_and_cache,
+        "heads of a qkv product: normed, rotated, k and v into the cache",
+        py::arg("qkv"), py::arg("n_q_heads"), py::arg("cos_sin"),
+        py::arg("positions"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("slots"), py::arg("q_norm") = py::none(),
+        py::arg("k_norm") = py::none(), py::arg("eps") = 1e-5);
   m.def("silu_mul", &silu_mul, "fused SiLU*up on packed gate_up");
   m.def("reshape_and_cache", &reshape_and_cache, "scatter K/V into paged pool");
   m.def("move_blocks", &move_blocks, "gather/scatter KV blocks for xGMI transfer");

@@ -22,8 +22,8 @@ class GatedMLP:
         self.down = take("down").to(dtype)
 
     def __call__(self, h: torch.Tensor) -> Output:
-        return linear(ops.gated_linear(h, self.gate_up, self.spec.act),
-                      self.down), None
+        return ops.linear_parts(
+            ops.gated_linear(h, self.gate_up, self.spec.act), self.down), None
 
 
 class Experts:
@@ -55,8 +55,9 @@ class Experts:
         rows = ops.experts(h, ids, weights, self.up, self.down, s.act)
         if self.shared_up is None:
             return None, rows
-        return linear(ops.activate(linear(h, self.shared_up), s.act),
-                      self.shared_down), rows
+        return ops.linear_parts(
+            ops.activate(linear(h, self.shared_up), s.act),
+            self.shared_down), rows
 
 
 def build(spec: FeedForwardSpec, take: Callable, dtype: torch.dtype):

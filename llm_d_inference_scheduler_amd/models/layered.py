@@ -159,7 +159,7 @@ class ChannelDelta:
                                 self.dt_bias, self.neg_a, state, g, ws, o)
             ops.delta_gate(o, gate, self.norm, out, batch.n_step_rows,
                            self.eps)
-        return linear(out, self.w_o)
+        return ops.linear_parts(out, self.w_o)
 
 
 class LatentAttention:
@@ -210,7 +210,7 @@ class LatentAttention:
                                batch.seq_meta, origin,
                                ctx["tiles", QUERY_TILE],
                                s.rot_dim, s.window, s.scale, out)
-        return linear(out, self.w_o)
+        return ops.linear_parts(out, self.w_o)
 
 
 class GroupedAttention:
@@ -245,7 +245,7 @@ class GroupedAttention:
                                 batch.block_tables, n, batch.seq_meta,
                                 ctx["tiles", self.tile_rows], s.heads, s.dim,
                                 s.scale, s.sink, out)
-        return linear(out, self.w_o)
+        return ops.linear_parts(out, self.w_o)
 
 
 class LayeredRunner:

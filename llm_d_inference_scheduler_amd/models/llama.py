@@ -135,32 +135,19 @@ class LlamaRunner:
         pos32 = batch.positions.to(torch.int32)
         for li, layer in enumerate(self.layers):
             if residual is None:
-                residual = hidden.clone()
+                residual = hidden
                 normed = ops.rmsnorm(hidden, layer["input_norm"], c.rms_eps)
             else:
                 normed = ops.rmsnorm(hidden, layer["input_norm"], c.rms_eps,
                                      residual=residual)
-            qkv = ops.linear(normed, layer["wqkv"].t())
-            q, k, v = qkv.split([c.q_size, c.kv_size, c.kv_size], dim=-1)
-            T = q.shape[0]
-            q = q.view(T, c.num_heads, c.head_dim).contiguous()
-            k = k.view(T, c.num_kv_heads, c.head_dim).contiguous()
-            v = v.view(T, c.num_kv_heads, c.head_dim).contiguous()
-            if c.qk_norm:
-                # Qwen3 per-head QK-RMSNorm before RoPE: each head's
-                # D-vector normalized with a learned gain (the rmsnorm
-                # kernel treats [T*H, D] rows like any hidden dim)
-                q = ops.rmsnorm(q.view(T * c.num_heads, c.head_dim),
-                                layer["q_norm"],
-                                c.rms_eps).view(T, c.num_heads, c.head_dim)
-                k = ops.rmsnorm(k.view(T * c.num_kv_heads, c.head_dim),
-                                layer["k_norm"],
-                                c.rms_eps).view(T, c.num_kv_heads,
-                                                c.head_dim)
-            ops.rope(q, k, self.cos_sin, pos32)
+            T = normed.shape[0]
             k_cache = kv_pool[li, 0]
             v_cache = kv_pool[li, 1]
-            ops.reshape_and_cache(k, v, k_cache, v_cache, batch.slot_mapping)
+            # Qwen3 norms every head of q and k before RoPE
+            q = ops.rope_and_cache(
+                ops.linear_parts(normed, layer["wqkv"].t()), c.num_heads,
+                self.cos_sin, pos32, k_cache, v_cache, batch.slot_mapping,
+                layer.get("q_norm"), layer.get("k_norm"), c.rms_eps)
             if batch.is_decode:
                 attn = ops.paged_attention(q, k_cache, v_cache,
                                            batch.block_tables, batch.seq_lens,
@@ -168,11 +155,11 @@ class LlamaRunner:
                                            max_seq_len=batch.max_seq_len)
             else:
                 attn = self._prefill_attention(batch, q, k_cache, v_cache)
-            o = ops.linear(attn.view(T, c.q_size), layer["wo"].t())
+            o = ops.linear_parts(attn.view(T, c.q_size), layer["wo"].t())
             normed2 = ops.rmsnorm(o, layer["post_norm"], c.rms_eps,
                                   residual=residual)
             act = ops.gated_linear(normed2, layer["wgate_up"].t())
-            hidden = ops.linear(act, layer["wdown"].t())
+            hidden = ops.linear_parts(act, layer["wdown"].t())
         final = ops.rmsnorm(hidden, self.final_norm, c.rms_eps,
                             residual=residual)
         # `residual` now holds the pre-norm sum; `final` the normed states

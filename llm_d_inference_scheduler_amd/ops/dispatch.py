@@ -40,6 +40,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return _ext.linear(x, w) if _use_hip(x) else x @ w.t()
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """The same for rmsnorm or rope_and_cache, which also take the 32-bit
+    partial sums [parts, rows, out] of a product that split K."""
+    return _ext.linear_parts(x, w) if _use_hip(x) else x @ w.t()
+
+
 def lay_weights(w: torch.Tensor) -> torch.Tensor:
     """Weights drawn as [in, out] in 32-bit -> bf16 [out, in] on the GPU."""
     return hip_ops().lay_weights(w)
@@ -70,6 +76,34 @@ def rope(q: torch.Tensor, k: torch.Tensor, cos_sin: torch.Tensor,
         _ext.rope(q, k, cos_sin, positions.to(torch.int32))
         return
     ref.rope(q, k, cos_sin, positions)
+
+
+def rope_and_cache(qkv: torch.Tensor, n_q_heads: int, cos_sin: torch.Tensor,
+                   positions: torch.Tensor, k_cache: torch.Tensor,
+                   v_cache: torch.Tensor, slots: torch.Tensor,
+                   q_norm: Optional[torch.Tensor] = None,
+                   k_norm: Optional[torch.Tensor] = None,
+                   eps: float = 1e-5) -> torch.Tensor:
+    """Packed heads of a qkv product (or its partial sums): q and k normed
+    per head (where weights are given) and rotated, k and v stored in the
+    cache. -> q [T, n_q_heads, D]."""
+    if _use_hip(qkv):
+        q = _ext.rope_and_cache(qkv, n_q_heads, cos_sin,
+                                positions.to(torch.int32), k_cache, v_cache,
+                                slots.to(torch.int64), q_norm, k_norm, eps)
+        if q is not None:
+            return q
+        if qkv.dim() == 3:
+            qkv = qkv.sum(0).to(torch.bfloat16)
+    T, D, kvh = qkv.shape[0], k_cache.shape[3], k_cache.shape[1]
+    q, k, v = (t.reshape(T, -1, D).contiguous() for t in qkv.split(
+        [n_q_heads * D, kvh * D, kvh * D], dim=-1))
+    if q_norm is not None:
+        q = rmsnorm(q.view(-1, D), q_norm, eps).view(T, -1, D)
+        k = rmsnorm(k.view(-1, D), k_norm, eps).view(T, -1, D)
+    rope(q, k, cos_sin, positions)
+    reshape_and_cache(k, v, k_cache, v_cache, slots)
+    return q
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:

@@ -33,6 +33,12 @@ def linear(x, w):
     return hip_layered().linear(x, w) if x.is_cuda else x @ w.t()
 
 
+def linear_parts(x, w):
+    """The same for stream_norm, which also takes the 32-bit partial sums
+    [parts, rows, out] of a product that split K."""
+    return hip_layered().linear_parts(x, w) if x.is_cuda else x @ w.t()
+
+
 def gated_linear(x, w, act):
     """act(x gate') * (x up') of w = [gate; up], one call for few rows."""
     if x.is_cuda:
@@ -62,7 +68,7 @@ def embed_norm(ids, table, scale, wn, offset, eps, pos=None, positions=None):
 
 def stream_norm(x, y, wb, wn, offset, eps, dtype, rows=None):
     """In place: x += rms_norm(y) * (wb + offset), without wb x += y, without
-    y nothing; with rows [T * n, width] also each token's n rows.
+    y nothing (y: also from linear_parts); with rows [T * n, width] also each token's n rows.
     -> rms_norm(x) * (wn + offset) as dtype; without wn x as dtype."""
     return _impl(x).stream_norm(x, y, wb, wn, offset, eps,
                                 dtype == torch.float32, rows)

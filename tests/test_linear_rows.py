@@ -135,3 +135,92 @@ def test_lay_weights(r, c):
     w = _draw(r, c, seed=r).float() * 1.2345
     got = _ext("_hip_ops").lay_weights(w)
     assert got.is_contiguous() and torch.equal(got, w.bfloat16().t())
+
+
+@pytest.mark.parametrize("rows", [1, 40, 128, 130])
+def test_parts_in_norms(rows):
+    """rmsnorm and stream_norm sum the parts of a product themselves."""
+    from llm_d_inference_scheduler_amd.ops import layered
+    hip = _ext("_hip_ops")
+    x, w = _draw(rows, 2048, seed=1), _draw(520, 2048, seed=2, scale=1 / 45)
+    gain = _draw(520, seed=3)
+    y = hip.linear_parts(x, w)
+    assert y.dim() == (3 if rows <= 128 else 2)
+    if rows <= 128:
+        assert y.shape[0] > 1 and y.dtype == torch.float32
+    # a library product is rounded to bf16 before anything is added to it
+    full = x.double() @ w.double().t() if y.dim() == 3 else y.double()
+    for start in (None, _draw(rows, 520, seed=4)):
+        residual = None if start is None else start.clone()
+        got = hip.rmsnorm(y, gain, 1e-5, residual)
+        src = full if start is None else full + start.double()
+        if residual is not None:
+            _same(residual, src, 8)
+        _same(got, src * (src.square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+              * gain.double(), 8)
+    wb, wn = gain.float(), _draw(520, seed=5).float()
+    stream = _draw(rows, 520, seed=6).float()
+    for post in (None, wb):
+        z = full if post is None else full * (
+            full.square().mean(-1, keepdim=True) + 1e-5).rsqrt() * (
+            post.double() + 0.5)
+        s = stream.double() + z
+        mine = stream.clone()
+        h = layered.stream_norm(mine, layered.linear_parts(x, w), post, wn,
+                                0.5, 1e-5, torch.bfloat16)
+        torch.testing.assert_close(mine.double(), s, rtol=1e-5, atol=1e-4)
+        _same(h, s * (s.square().mean(-1, keepdim=True) + 1e-5).rsqrt() *
+              (wn.double() + 0.5), 8)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("T,qh,kvh,d,bs", [(1, 4, 1, 128, 16),
+                                           (37, 8, 8, 64, 16),
+                                           (130, 6, 2, 32, 8),
+                                           (5, 2, 1, 16, 4),
+                                           (3, 3, 3, 96, 16)])
+@pytest.mark.parametrize("parts", [0, 3])
+def test_rope_and_cache(T, qh, kvh, d, bs, norm, fp8, parts):
+    """One pass against its steps apart in float64; a slot below 0 is not
+    cached; 96 channels have no normed form and go step by step."""
+    from llm_d_inference_scheduler_amd import ops
+    from llm_d_inference_scheduler_amd.ops import ref
+    n = (qh + 2 * kvh) * d
+    if parts:
+        qkv = _draw(parts, T, n, seed=T).float() / 2
+        x = qkv.double().sum(0)
+    else:
+        qkv = _draw(T, n, seed=T)
+        x = qkv.double()
+    pos = torch.randint(0, 300, (T,), device="cuda", dtype=torch.int32)
+    cs = ref.rope_table(300, d, 1e4, device="cuda")
+    blocks = T // bs + 2
+    slots = torch.randperm(blocks * bs, device="cuda")[:T]
+    slots[T // 2] = -1
+    dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    kc, vc = (torch.zeros(blocks, kvh, bs, d, device="cuda").to(dtype)
+              for _ in range(2))
+    qn, kn = (_draw(d, seed=7), _draw(d, seed=8)) if norm else (None, None)
+    got = ops.rope_and_cache(qkv, qh, cs, pos, kc, vc, slots, qn, kn, 1e-5)
+    q, k, v = (t.reshape(T, -1, d) for t in x.split(
+        [qh * d, kvh * d, kvh * d], -1))
+    if norm:
+        q, k = (t * (t.square().mean(-1, keepdim=True) + 1e-5).rsqrt() *
+                w.double() for t, w in ((q, qn), (k, kn)))
+    c, s = (cs.double()[pos.long()][:, None, :, i] for i in (0, 1))
+
+    def rotate(t):
+        a, b = t[..., :d // 2], t[..., d // 2:]
+        return torch.cat([a * c - b * s, b * c + a * s], -1)
+    # bf16, and the steps apart round twice; fp8: half a step of 2^-3
+    torch.testing.assert_close(got.double(), rotate(q), rtol=2 ** -6,
+                               atol=2e-2)
+    keep = slots >= 0
+    for cache, want in ((kc, rotate(k)), (vc, v)):
+        rows = cache.float().permute(0, 2, 1, 3).reshape(-1, kvh, d)
+        torch.testing.assert_close(
+            rows[slots[keep]].double(), want[keep],
+            rtol=2 ** -3.5 if fp8 else 2 ** -6, atol=2e-2)
+        rows[slots[keep]] = 0
+        assert not rows.any()            # nothing else was written
