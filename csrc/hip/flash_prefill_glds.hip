@@ -1,315 +1,318 @@
 // flash_prefill_glds.hip — the bf16-KV variant of the fused MFMA prefill
-// attention with a glds staging pipeline (guide §5 "glds with >1 tile in
-// flight"): K/V tiles are DMA'd straight to LDS (`global_load_lds`) into a
-// 3-deep ring, one tile ahead, with COUNTED `s_waitcnt vmcnt(N)` and raw
-// `s_barrier` (a `__syncthreads()` would drain the in-flight DMA; hipcc
-// also drains glds at any ordinary in-loop global load, so the block table
-// is staged into LDS up front and the hot loop touches global memory ONLY
-// through glds). The LDS image stays lane-linear (a glds constraint); the
-// XOR bank swizzle is applied by permuting the per-lane SOURCE addresses.
+// attention with a glds staging pipeline: K/V tiles are DMA'd straight to LDS
+// (`global_load_lds`) into a ring, ahead of their use, with COUNTED
+// `s_waitcnt vmcnt(N)` (hipcc drains glds at any ordinary in-loop global load,
+// so the block table is staged into LDS up front and the hot loop touches
+// global memory ONLY through glds). The LDS image stays lane-linear (a glds
+// constraint); the XOR bank swizzle is applied by permuting the per-lane
+// SOURCE addresses. The attention of a tile is flash_core.h's.
 //
-// Ring safety: iteration order is [counted vmcnt][raw barrier]
-// [compute tile n][issue tile n+2] — barrier C_n separates every wave's
-// last read of buffer (n-1)%3 (its compute at iteration n-1, before C_n)
-// from the buffer's rewrite for tile n+2 (after C_n in every wave).
+// A workgroup has 4 waves and one of two shapes:
+//   rows   128 query rows, 32 per wave; all waves share tiles of 32 keys in a
+//          3-deep ring, two tiles ahead. Order: [counted vmcnt][raw barrier]
+//          [compute tile n][issue tile n+2] — barrier n separates every wave's
+//          last read of buffer (n-1)%3 from its rewrite for tile n+2.
+//   keys   32 query rows; every wave takes each fourth tile of keys through a
+//          2-deep ring of its own, without barriers, and the waves' results
+//          meet in LDS at the end. Four times the workgroups, a quarter of the
+//          serial chain: for calls whose rows leave the chip idle. These have
+//          matrix cores to spare, so that probabilities keep 17 bits: a
+//          prompt's last tokens come out as decoding them would.
+// Key heads run fastest over the grid: with 8 of them each XCD's L2 holds the
+// keys and values of one. Tiles run from the last to the first: under the
+// causal mask the last of a sequence has the most keys.
 //
-// fp8 KV cannot ride glds (raw byte copy, no conversion point), so the
-// fp8 path keeps the convert-on-stage kernel in flash_prefill.hip; the
-// launcher in ops.hip picks per cache dtype. Attention math, fragment
-// layouts, masking and the swapped-QK^T softmax are identical to
-// flash_prefill.hip (see its header comments).
-#include "hip_common.h"
+// Measured (groups of 4, 8 key heads; before: masks, packing and rescaling of
+// every tile on the vector units): one prompt of 7900 tokens 650 us, 785
+// TFLOP/s (before 1170); 8 of 1000 135 us (265); 150 tokens behind 1000, by
+// keys: 22 us, by rows 42 (59).
+//
+// fp8 KV cannot ride glds (raw byte copy, no conversion point), so the fp8
+// path keeps the convert-on-stage kernel in flash_prefill.hip; the launcher in
+// ops.hip picks per cache dtype.
+#include "flash_core.h"
 
 namespace {
 
+using namespace flash;
+
 constexpr int D = 128;
 constexpr int KVBLK = 32;    // tokens per KV tile (ring granularity)
-constexpr int NBUF = 3;
 constexpr int NW = 4;
 constexpr int QROWS = 32;
 constexpr int BT_CAP = 1024;  // staged block-table entries (16K-token ctx)
-constexpr float NEG = -1e30f;
 
-constexpr int TILE_SHORTS = KVBLK * D;           // 4096 shorts = 8 KB
-constexpr int GLDS_PER_WAVE = KVBLK * 16 / 64 / NW;  // K instrs/wave (=2)
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) unsigned int uint4v;
-typedef __attribute__((ext_vector_type(4))) short short4v;
-
-// Bank swizzle S(row): swap the two 2-bit halves of row&15. Chosen from
-// the CDNA4 bank model (MI355X_MICROARCH.md "LDS"): the K ds_read_b128
-// only needs S bijective on row&15 (its 16-lane groups cover all 16
-// values of qcol&15, so any bijection spreads the 16 slots); the V
-// ds_read_b64_tr_b16 (32-lane groups) additionally needs kv0&3 steered
-// into address bits [7:6] so the 8-byte granule index
-// (dt | g | r) ^ (S << 1) is injective over the group's (g, kv0, r) —
-// the previous S(row)=row&15 left granule bits [4:3] untouched and put
-// FOUR lanes on every granule (the measured 47%-of-LDS-active conflict
-// cycles, profiles/r01_pmc_final.md).
-__device__ __forceinline__ int swz4(int row) {
-  return ((row & 3) << 2) | ((row >> 2) & 3);
-}
-
-__device__ __forceinline__ int g_swz(int row, int byte_off) {
-  return row * 256 + (byte_off ^ (swz4(row) << 4));
-}
-
-__device__ __forceinline__ unsigned int pack2_bf16(float a, float b) {
-  return ((unsigned int)(unsigned short)f32_to_bf16(b) << 16) |
-         (unsigned int)(unsigned short)f32_to_bf16(a);
-}
+constexpr int TILE_BYTES = KVBLK * D * 2;        // of K, and of V
+constexpr int RING_ROWS = 3, RING_KEYS = 2;      // tiles per ring
 
 __device__ __forceinline__ void raw_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
-template <int QPG>
-__global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_glds_kernel(
+constexpr int lds_bytes(bool keys) {
+  return BT_CAP * 4 + 2 * TILE_BYTES * (keys ? RING_KEYS * NW : RING_ROWS);
+}
+
+// SHIFT: block size 1 << shift; else any
+template <int QPG, bool KEYS, bool SHIFT>
+__global__ __launch_bounds__(NW * WAVE, KEYS ? 1 : 2)
+void flash_prefill_glds_kernel(
     const short* __restrict__ q, const short* __restrict__ k_cache,
     const short* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables,
     const int32_t* __restrict__ seq_meta, const int32_t* __restrict__ tiles,
-    short* __restrict__ out, int kvh, int bs, int max_blocks, float scale) {
-  const int kh = blockIdx.y;
-  const int seq = tiles[2 * blockIdx.x];
-  const int vrow0 = tiles[2 * blockIdx.x + 1];
+    short* __restrict__ out, int n_tiles, int kvh, int bs, int shift,
+    int max_blocks, float scale) {
+  const int kh = blockIdx.x % kvh, at_tile = blockIdx.x / kvh;
+  const int tile = n_tiles - 1 - at_tile / (KEYS ? NW : 1);
+  const int sub = KEYS ? at_tile % NW : 0;
+  const int seq = tiles[2 * tile];
+  const int vrow0 = tiles[2 * tile + 1] + sub * QROWS;
   const int seq_start = seq_meta[3 * seq];
   const int chunk = seq_meta[3 * seq + 1];
   const int prior = seq_meta[3 * seq + 2];
-  const int ctx = prior + chunk;
+  const int ctx = prior + chunk, rows = chunk * QPG;
   const int n_q_heads = kvh * QPG;
+  if (KEYS && vrow0 >= rows) return;            // workgroup-uniform
 
   // ONE shared object (a second __shared__ symbol makes hipcc emit
-  // vmcnt(0) before every ds_read — guide §5 trap (a))
-  __shared__ __align__(16) char lds_raw[BT_CAP * 4 +
-                                        NBUF * 2 * TILE_SHORTS * 2];
+  // vmcnt(0) before every ds_read)
+  extern __shared__ __align__(16) char lds_raw[];
   int32_t* bt_lds = (int32_t*)lds_raw;
-  auto kbuf = [&](int b) -> short* {
-    return (short*)(lds_raw + BT_CAP * 4) + b * 2 * TILE_SHORTS;
-  };
-  auto vbuf = [&](int b) -> short* { return kbuf(b) + TILE_SHORTS; };
 
   const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = tid % WAVE;
   const int qcol = lane & 31;
   const int hi = lane >> 5;
+  // a ring of this wave's, or of all waves'
+  char* ring = lds_raw + BT_CAP * 4 +
+               (KEYS ? wave * RING_KEYS * 2 * TILE_BYTES : 0);
 
-  const int vrow = vrow0 + wave * QROWS + qcol;
-  const bool active = vrow < chunk * QPG;
-  const int p = active ? vrow / QPG : -1;
-  const int g = active ? vrow % QPG : 0;
-  const int p_c = active ? p : chunk - 1;
-  const int qh = kh * QPG + g;
-  const int64_t q_row = (int64_t)(seq_start + p_c) * n_q_heads + qh;
+  // rows past the last repeat it and are not stored
+  const int w0 = vrow0 + (KEYS ? 0 : wave * QROWS);
+  const int vrow = w0 + qcol;
+  const bool active = vrow < rows;
+  const int p = (active ? vrow : rows - 1) / QPG;
+  const int qh = kh * QPG + (active ? vrow : rows - 1) % QPG;
+  const int64_t q_row = (int64_t)(seq_start + p) * n_q_heads + qh;
 
-  const int p_max_wg =
-      min((min(vrow0 + NW * QROWS, chunk * QPG) - 1) / QPG, chunk - 1);
-  const int p_max_w =
-      min((min(vrow0 + (wave + 1) * QROWS, chunk * QPG) - 1) / QPG, chunk - 1);
-  const int kv_end_wg = min(ctx, prior + p_max_wg + 1);
-  const int kv_end_w = prior + p_max_w + 1;
-  const int n_kv_tiles = (kv_end_wg + KVBLK - 1) / KVBLK;
+  const int last_wg = (min(vrow0 + (KEYS ? QROWS : NW * QROWS), rows) - 1) / QPG;
+  const int first_w = min(w0, rows - 1) / QPG;
+  const int last_w = (min(w0 + QROWS, rows) - 1) / QPG;
+  const int kv_end = prior + last_wg + 1;       // keys that a row here may see
+  const int kv_end_w = w0 < rows ? prior + last_w + 1 : 0;
+  const int n_kv_tiles = (kv_end + KVBLK - 1) / KVBLK;
 
   // ---- prologue: Q fragments + block table; every ordinary global load
   //      completes before the first glds issues ----
-  bf16x8 q_frag[D / 16];
+  bf16x8 qf[D / 16];
+  const unsigned int flip = scale < 0.f ? 0x80008000u : 0u;
 #pragma unroll
-  for (int kk = 0; kk < D / 16; ++kk)
-    q_frag[kk] = *(const bf16x8*)(q + q_row * D + kk * 16 + hi * 8);
-  // stage enough entries to cover the final tile's clamped pad rows
-  // (t = min(tile0+row, ctx-1) can reach up to kv_end_wg + KVBLK - 1)
-  const int n_bt = min(max_blocks,
-                       (min(kv_end_wg + KVBLK, ctx) + bs - 1) / bs);
+  for (int kk = 0; kk < D / 16; ++kk) {
+    const uint4v v = *(const uint4v*)(q + q_row * D + kk * 16 + hi * 8);
+    qf[kk] = __builtin_bit_cast(bf16x8, v ^ flip);
+  }
+  const float scale_log2 = fabsf(scale) * LOG2E;
+  auto page_of = [&](int t) { return SHIFT ? t >> shift : t / bs; };
+  const int n_bt = min(max_blocks, page_of(kv_end - 1) + 1);
   for (int i = tid; i < n_bt; i += NW * WAVE)
     bt_lds[i] = block_tables[(int64_t)seq * max_blocks + i];
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // publish bt_lds (no glds in flight yet)
 
-  auto stage_tile = [&](int n) {
-    const int tile0 = n * KVBLK;
-    const int buf = n % NBUF;
+  // rows of a tile that a wave fetches, 4 per instruction
+  constexpr int LOADS = KVBLK / 4 / (KEYS ? 1 : NW);
+  auto stage = [&](int n, int buf) {
+    char* kb = ring + buf * 2 * TILE_BYTES;
 #pragma unroll
-    for (int j = 0; j < GLDS_PER_WAVE; ++j) {
-      const int piece = (wave * GLDS_PER_WAVE + j) * 64 + lane;
-      const int row = piece / 16, c16 = piece % 16;
-      const int src16 = c16 ^ swz4(row);        // source-side swizzle
-      const int t = min(tile0 + row, ctx - 1);  // clamp: no garbage bf16
+    for (int j = 0; j < LOADS; ++j) {
+      const int part = (KEYS ? 0 : wave * LOADS) + j;
+      const int row = part * 4 + lane / 16;
+      const int src = lane % 16 ^ swizzle(row) >> 4;    // source-side swizzle
+      // keys past the last that is seen repeat it: no garbage bf16
+      const int t = min(n * KVBLK + row, kv_end - 1), pg = page_of(t);
+      const int at = t - (SHIFT ? pg << shift : pg * bs);
       const int64_t base =
-          (((int64_t)bt_lds[t / bs] * kvh + kh) * bs + t % bs) * D;
+          (((int64_t)bt_lds[pg] * kvh + kh) * bs + at) * D + src * 8;
+      typedef const __attribute__((address_space(1))) unsigned int gmem;
+      typedef __attribute__((address_space(3))) unsigned int smem;
+      __builtin_amdgcn_global_load_lds((gmem*)(k_cache + base),
+                                       (smem*)(kb + part * 1024), 16, 0, 0);
       __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)(
-              k_cache + base + src16 * 8),
-          (__attribute__((address_space(3))) unsigned int*)(
-              (char*)kbuf(buf) + (wave * GLDS_PER_WAVE + j) * 1024),
-          16, 0, 0);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) unsigned int*)(
-              v_cache + base + src16 * 8),
-          (__attribute__((address_space(3))) unsigned int*)(
-              (char*)vbuf(buf) + (wave * GLDS_PER_WAVE + j) * 1024),
-          16, 0, 0);
+          (gmem*)(v_cache + base), (smem*)(kb + TILE_BYTES + part * 1024), 16,
+          0, 0);
     }
   };
 
-  float m_run = NEG, l_run = 0.f;
-  f32x16 acc_o[D / 32];
+  Softmax st;
+  f32x16 acc[D / 32];
 #pragma unroll
-  for (int dt = 0; dt < D / 32; ++dt) acc_o[dt] = (f32x16)(0.f);
+  for (int t = 0; t < D / 32; ++t) acc[t] = (f32x16)(0.f);
 
-  stage_tile(0);
-  if (n_kv_tiles > 1) stage_tile(1);
-
+  // the lane's share of addresses in a tile
   const int i16 = lane % 16;
-  const int d_grp = 16 * ((lane & 31) >> 4);
-  const int dim_col = d_grp + (i16 % 4) * 4;
-
-  for (int n = 0; n < n_kv_tiles; ++n) {
+  const int k_row = qcol * 256, k_swz = swizzle(qcol);
+  const int v_col = (16 * ((lane & 31) >> 4) + (i16 % 4) * 4) * 2;
+  auto compute = [&](int n, int buf) {
     const int tile0 = n * KVBLK;
-    const int buf = n % NBUF;
-    // tile n has landed when at most the NEXT tile's DMA remains in
-    // flight (counted per-wave wait; vmcnt retires in order)
-    if (n + 1 < n_kv_tiles)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * GLDS_PER_WAVE)
-                   : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    raw_barrier();
+    const char* kb = ring + buf * 2 * TILE_BYTES;
+    const char* vb = kb + TILE_BYTES;
+    attend32<D / 16, D / 32, KEYS>(
+        [&](int kk) {
+          return *(const bf16x8*)(kb + k_row +
+                                  ((kk * 32 + hi * 16) ^ k_swz));
+        },
+        [&](int row, int t) {
+          return vb + row * 256 + ((t * 64 + v_col) ^ swizzle(row));
+        },
+        qf, scale_log2, tile0 + KVBLK - 1 <= prior + first_w, 0,
+        prior + p - tile0, st, acc);
+  };
 
-    if (tile0 < kv_end_w) {
-      const short* k_lds = kbuf(buf);
-      const short* v_lds = vbuf(buf);
-      f32x16 acc_s = (f32x16)(0.f);
-#pragma unroll
-      for (int kk = 0; kk < D / 16; ++kk) {
-        const bf16x8 k_frag = *(const bf16x8*)(
-            (const char*)k_lds + g_swz(qcol, (kk * 16 + hi * 8) * 2));
-        acc_s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(k_frag, q_frag[kk],
-                                                        acc_s, 0, 0, 0);
-      }
-
-      float s[16];
-      float tmax = NEG;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int kv = tile0 + (r & 3) + 8 * (r >> 2) + 4 * hi;
-        const bool valid = active && kv <= prior + p;
-        s[r] = valid ? acc_s[r] * scale : NEG;
-        tmax = fmaxf(tmax, s[r]);
-      }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-      const float m_new = fmaxf(m_run, tmax);
-      // MFMA reads operands from all 64 lanes regardless of EXEC: run the
-      // PV block wave-uniformly, inactive lanes contribute zero P columns
-      const bool has = m_new > NEG * 0.5f;
-      if (__any(has)) {
-        const float m_eff = has ? m_new : 0.f;
-        const float alpha =
-            (m_run <= NEG * 0.5f) ? 0.f : __expf(m_run - m_eff);
-        float tsum = 0.f;
-        float pr[16];
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          pr[r] = (s[r] <= NEG * 0.5f) ? 0.f : __expf(s[r] - m_eff);
-          tsum += pr[r];
-        }
-        tsum += __shfl_xor(tsum, 32, WAVE);
-        l_run = l_run * alpha + tsum;
-        if (has) m_run = m_new;
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc_o[dt][e] *= alpha;
-
-        unsigned int w[8], x[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          w[i] = pack2_bf16(pr[2 * i], pr[2 * i + 1]);
-          x[i] = __shfl_xor((int)w[i], 32, WAVE);
-        }
-        uint4v f0 = hi ? (uint4v){x[2], x[3], w[2], w[3]}
-                       : (uint4v){w[0], w[1], x[0], x[1]};
-        uint4v f1 = hi ? (uint4v){x[6], x[7], w[6], w[7]}
-                       : (uint4v){w[4], w[5], x[4], x[5]};
-        const bf16x8 p_frag0 = __builtin_bit_cast(bf16x8, f0);
-        const bf16x8 p_frag1 = __builtin_bit_cast(bf16x8, f1);
-
-#pragma unroll
-        for (int dt = 0; dt < D / 32; ++dt) {
-#pragma unroll
-          for (int ks = 0; ks < 2; ++ks) {
-            const int kv0 = ks * 16 + hi * 8 + i16 / 4;
-            const int dc = (dt * 32 + dim_col) * 2;
-            short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) short4v*)(
-                    (const char*)v_lds + kv0 * 256 +
-                    (dc ^ (swz4(kv0) << 4))));
-            const int kv1 = kv0 + 4;
-            short4v hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (__attribute__((address_space(3))) short4v*)(
-                    (const char*)v_lds + kv1 * 256 +
-                    (dc ^ (swz4(kv1) << 4))));
-            short8 vfrag8 = {lo[0], lo[1], lo[2], lo[3],
-                             hi4[0], hi4[1], hi4[2], hi4[3]};
-            acc_o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                __builtin_bit_cast(bf16x8, vfrag8),
-                ks == 0 ? p_frag0 : p_frag1, acc_o[dt], 0, 0, 0);
-          }
-        }
-      }
+  if constexpr (KEYS) {
+    // tiles wave, wave + NW, ..
+    const int mine = n_kv_tiles > wave ? (n_kv_tiles - wave + NW - 1) / NW : 0;
+    for (int i = 0; i < min(mine, RING_KEYS); ++i) stage(wave + i * NW, i);
+    for (int i = 0; i < mine; ++i) {
+      if (i + 1 < mine)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * LOADS) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      compute(wave + i * NW, i % RING_KEYS);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads are done
+      if (i + RING_KEYS < mine)
+        stage(wave + (i + RING_KEYS) * NW, i % RING_KEYS);
     }
-    if (n + 2 < n_kv_tiles) stage_tile(n + 2);
-  }
-
-  if (active && l_run > 0.f) {
-    const float inv_l = 1.f / l_run;
-    const int64_t out_row = ((int64_t)(seq_start + p) * n_q_heads + qh) * D;
-#pragma unroll
-    for (int dt = 0; dt < D / 32; ++dt) {
-#pragma unroll
-      for (int rq = 0; rq < 4; ++rq) {
-        const int dim = dt * 32 + 8 * rq + 4 * hi;
-        unsigned int lo = pack2_bf16(acc_o[dt][4 * rq] * inv_l,
-                                     acc_o[dt][4 * rq + 1] * inv_l);
-        unsigned int hi2 = pack2_bf16(acc_o[dt][4 * rq + 2] * inv_l,
-                                      acc_o[dt][4 * rq + 3] * inv_l);
-        *(uint2*)(out + out_row + dim) = make_uint2(lo, hi2);
-      }
+  } else {
+    stage(0, 0);
+    if (n_kv_tiles > 1) stage(1, 1);
+    int buf = 0, fill = 2;
+    for (int n = 0; n < n_kv_tiles; ++n) {
+      // tile n has landed when at most the NEXT tile's DMA remains in
+      // flight (counted per-wave wait; vmcnt retires in order)
+      if (n + 1 < n_kv_tiles)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * LOADS) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      raw_barrier();
+      if (n * KVBLK < kv_end_w) compute(n, buf);
+      if (n + 2 < n_kv_tiles) stage(n + 2, fill);
+      buf = buf + 1 == RING_ROWS ? 0 : buf + 1;
+      fill = fill + 1 == RING_ROWS ? 0 : fill + 1;
     }
   }
+  st.l = st.join();
+
+  if constexpr (KEYS) {
+    // the waves meet: wave w sums channels 32 w .. of all four
+    float* o_sh = (float*)(lds_raw + BT_CAP * 4);   // [wave][t][r][lane]
+    float2* ml_sh = (float2*)lds_raw;               // [wave][lane]
+    __syncthreads();                                // rings and table are done
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        o_sh[((wave * (D / 32) + t) * 16 + r) * WAVE + lane] = acc[t][r];
+    ml_sh[wave * WAVE + lane] = make_float2(st.m, st.l);
+    __syncthreads();
+    float m = NEG, l = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, ml_sh[w * WAVE + lane].x);
+    f32x16 o = (f32x16)(0.f);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float2 ml = ml_sh[w * WAVE + lane];
+      const float a = __builtin_amdgcn_exp2f(ml.x - m);
+      l += a * ml.y;
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        o[r] += a * o_sh[((w * (D / 32) + wave) * 16 + r) * WAVE + lane];
+    }
+    if (!active || !(l > 0.f)) return;
+    const float inv = 1.f / l;
+    short* dst = out + q_row * D + wave * 32 + 4 * hi;
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(uint2*)(dst + 8 * g) = make_uint2(
+          pack2(o[4 * g] * inv, o[4 * g + 1] * inv),
+          pack2(o[4 * g + 2] * inv, o[4 * g + 3] * inv));
+  } else if (active && st.l > 0.f) {
+    const float inv = 1.f / st.l;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(uint2*)(out + q_row * D + t * 32 + 8 * g + 4 * hi) = make_uint2(
+            pack2(acc[t][4 * g] * inv, acc[t][4 * g + 1] * inv),
+            pack2(acc[t][4 * g + 2] * inv, acc[t][4 * g + 3] * inv));
+  }
+}
+
+template <int QPG, bool KEYS, bool SHIFT>
+hipError_t go(const void* q, const void* k_cache, const void* v_cache,
+              const int32_t* block_tables, const int32_t* seq_meta,
+              const int32_t* tiles, void* out, int n_tiles, int kvh, int bs,
+              int shift, int max_blocks, float scale, hipStream_t stream) {
+  auto fn = flash_prefill_glds_kernel<QPG, KEYS, SHIFT>;
+  hipError_t e = hipFuncSetAttribute(
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+      lds_bytes(KEYS));
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3((uint32_t)kvh * n_tiles * (KEYS ? NW : 1)),
+                     dim3(NW * WAVE), lds_bytes(KEYS), stream, (const short*)q,
+                     (const short*)k_cache, (const short*)v_cache,
+                     block_tables, seq_meta, tiles, (short*)out, n_tiles, kvh,
+                     bs, shift, max_blocks, scale);
+  HIP_CHECK_LAST();
+  return hipSuccess;
 }
 
 }  // namespace
 
 extern "C" {
 
+// `keys`: the waves share query rows and split the keys (0, 1; below 0: by the
+// number of workgroups). Fewer than one per compute unit with 128 rows each
+// leave the chip idle.
 hipError_t lds_flash_prefill_glds(
     const void* q, const void* k_cache, const void* v_cache,
     const int32_t* block_tables, const int32_t* seq_meta,
     const int32_t* tiles, void* out, int n_tiles, int n_q_heads, int kvh,
-    int bs, int head_dim, int max_blocks, float scale, hipStream_t stream) {
+    int bs, int head_dim, int max_blocks, float scale, int keys,
+    hipStream_t stream) {
   if (n_tiles == 0) return hipSuccess;
-  if (head_dim != D || max_blocks > BT_CAP) return hipErrorInvalidValue;
+  if (head_dim != D || max_blocks > BT_CAP || bs < 1 ||
+      (int64_t)n_tiles * kvh * NW > 0x7fffffff)
+    return hipErrorInvalidValue;
   const int qpg = n_q_heads / kvh;
-  dim3 grid(n_tiles, kvh), block(NW * WAVE);
-#define LAUNCH_G(QPG)                                                        \
-  hipLaunchKernelGGL((flash_prefill_glds_kernel<QPG>), grid, block, 0,       \
-                     stream, (const short*)q, (const short*)k_cache,         \
-                     (const short*)v_cache, block_tables, seq_meta, tiles,   \
-                     (short*)out, kvh, bs, max_blocks, scale)
+  const bool split = keys < 0 ? (int64_t)n_tiles * kvh < 256 : keys != 0;
+  int shift = 0;
+  while (1 << shift < bs && shift < 20) ++shift;
+  const bool pow2 = 1 << shift == bs;
+#define GO(QPG, KEYS, SHIFT)                                                 \
+  return go<QPG, KEYS, SHIFT>(q, k_cache, v_cache, block_tables, seq_meta,   \
+                              tiles, out, n_tiles, kvh, bs, shift,           \
+                              max_blocks, scale, stream)
+#define GO_Q(QPG)                                                            \
+  do {                                                                       \
+    if (split) {                                                             \
+      if (pow2) GO(QPG, true, true); else GO(QPG, true, false);              \
+    } else {                                                                 \
+      if (pow2) GO(QPG, false, true); else GO(QPG, false, false);            \
+    }                                                                        \
+  } while (0)
   switch (qpg) {
-    case 1: LAUNCH_G(1); break;
-    case 2: LAUNCH_G(2); break;
-    case 4: LAUNCH_G(4); break;
-    case 8: LAUNCH_G(8); break;
+    case 1: GO_Q(1);
+    case 2: GO_Q(2);
+    case 4: GO_Q(4);
+    case 8: GO_Q(8);
     default: return hipErrorInvalidValue;
   }
-#undef LAUNCH_G
-  HIP_CHECK_LAST();
-  return hipSuccess;
+#undef GO_Q
+#undef GO
 }
 
 }  // extern "C"

@@ -7,11 +7,13 @@
 //                of everything a portion may see, the rotated key part shared
 //                by all heads; a sequence's context row 0 sits at ctx.pos0
 //
-// S' = K Q' keeps a query per lane: the online softmax is in-lane work plus
-// one exchange between the wave's halves, as in flash_prefill.hip. Rows of
-// the LDS tiles are padded instead of swizzled: 16 bytes for K (16-byte row
-// reads hit distinct banks), 64 bytes for V (the transposing reads of four
-// rows do). The next tile waits in registers while this one is computed.
+// The attention of 32 queries and 32 keys is flash_core.h's: S' = K Q' keeps a
+// query per lane. Rows of the LDS tiles are padded instead of swizzled: 16
+// bytes for K (16-byte row reads hit distinct banks), 64 bytes for V (the
+// transposing reads of four rows do). The next tile waits in registers while
+// this one is computed. Tiles run from the last to the first: under the causal
+// mask the last of a sequence has the most keys.
+#include "../flash_core.h"
 #include "elem.h"
 
 namespace {
@@ -19,16 +21,8 @@ namespace {
 constexpr int NW = 4, NT = NW * WAVE;
 constexpr int QW = 32;          // query rows per wave
 constexpr int KB = 64;          // keys per tile
-constexpr float NEG = -1e30f;
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) unsigned int uint4v;
-
-__device__ __forceinline__ unsigned int pack2(float a, float b) {
-  return ((unsigned int)(unsigned short)f32_to_bf16(b) << 16) |
-         (unsigned int)(unsigned short)f32_to_bf16(a);
-}
+using namespace flash;
 
 struct Prefill {
   const short* q;
@@ -58,7 +52,8 @@ void context_prefill_kernel(const Prefill a_) {
   short* k_lds = lds;                           // [KB][KS]
   short* v_lds = lds + KB * KS;                 // [KB][VS]
   const int kvh = blockIdx.x, rep = a_.rep;
-  const int seq = a_.tiles[2 * blockIdx.y], p0 = a_.tiles[2 * blockIdx.y + 1];
+  const int tile = gridDim.y - 1 - blockIdx.y;
+  const int seq = a_.tiles[2 * tile], p0 = a_.tiles[2 * tile + 1];
   const Seq sq = load_seq(a_.seq_meta, seq);
   const int64_t ctx0 = PAGED ? 0 : a_.ctx[2 * seq];
   // query p sees keys <= off + p
@@ -77,17 +72,23 @@ void context_prefill_kernel(const Prefill a_) {
   const int window = a_.window;
 
   bf16x8 qf[DK / 16];
+  const unsigned int flip = a_.scale_log2 < 0.f ? 0x80008000u : 0u;
+  const float scale_log2 = fabsf(a_.scale_log2);
   {
     const short* qr = a_.q + (sq.row0 + p) * a_.q_row + h * QD;
 #pragma unroll
     for (int kk = 0; kk < DK / 16; ++kk) {
       const int d = kk * 16 + hi * 8;
-      short8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (d < QD) z = *(const short8*)(qr + d);
-      qf[kk] = __builtin_bit_cast(bf16x8, z);
+      uint4v z = {0, 0, 0, 0};
+      if (d < QD) z = *(const uint4v*)(qr + d);
+      qf[kk] = __builtin_bit_cast(bf16x8, z ^ flip);
     }
   }
-  float m_run = a_.has_sink ? a_.sink : NEG, l_run = a_.has_sink ? 1.f : 0.f;
+  Softmax st;
+  if (a_.has_sink) {             // one of the halves' sums has it
+    st.m = a_.sink;
+    st.l = hi ? 0.f : 1.f;
+  }
   f32x16 acc[DV / 32];
 #pragma unroll
   for (int t = 0; t < DV / 32; ++t) acc[t] = (f32x16)(0.f);
@@ -177,93 +178,21 @@ void context_prefill_kernel(const Prefill a_) {
     for (int half = 0; half < 2; ++half) {
       const int sub = t0 + 32 * half;
       if (sub >= hi_w || sub + 32 <= lo_w) continue;   // wave-uniform
-      f32x16 s = (f32x16)(0.f);
-#pragma unroll
-      for (int kk = 0; kk < DK / 16; ++kk) {
-        const bf16x8 kf = *(const bf16x8*)(k_lds + (32 * half + qc) * KS +
-                                           kk * 16 + hi * 8);
-        s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s, 0, 0, 0);
-      }
-      // scores in units of log2; keys outside the mask drop out
-      float x[16], mx = NEG;
-      const bool inside =
-          sub + 31 <= off + pw0 && sub >= first_key(pw1);
-      if (inside) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          x[r] = s[r] * a_.scale_log2;
-          mx = fmaxf(mx, x[r]);
-        }
-      } else {
-        const int last = off + p, first = first_key(p);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int t = sub + (r & 3) + 8 * (r >> 2) + 4 * hi;
-          x[r] = t <= last && t >= first ? s[r] * a_.scale_log2 : NEG;
-          mx = fmaxf(mx, x[r]);
-        }
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-      const float mn = fmaxf(m_run, mx);
-      // a query without a key so far keeps m at NEG: its exponents are taken
-      // against 0 and underflow to 0
-      const float base = mn <= NEG * 0.5f ? 0.f : mn;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - base);
-      float sum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        x[r] = __builtin_amdgcn_exp2f(x[r] - base);
-        sum += x[r];
-      }
-      sum += __shfl_xor(sum, 32, WAVE);
-      l_run = l_run * alpha + sum;
-      if (__any(mn > m_run)) {
-#pragma unroll
-        for (int t = 0; t < DV / 32; ++t)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[t][e] *= alpha;
-      }
-      m_run = mn;
-
-      // P' as B operands: the halves exchange the rows they lack
-      unsigned int w[8], y[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        w[i] = pack2(x[2 * i], x[2 * i + 1]);
-        y[i] = __shfl_xor((int)w[i], 32, WAVE);
-      }
-      const uint4v f0 = hi ? (uint4v){y[2], y[3], w[2], w[3]}
-                           : (uint4v){w[0], w[1], y[0], y[1]};
-      const uint4v f1 = hi ? (uint4v){y[6], y[7], w[6], w[7]}
-                           : (uint4v){w[4], w[5], y[4], y[5]};
-      const bf16x8 pf[2] = {__builtin_bit_cast(bf16x8, f0),
-                            __builtin_bit_cast(bf16x8, f1)};
-
-      // O' += V' P': transposing reads give V' fragments
       const int i16 = lane % 16;
-      const int dcol = 16 * ((lane & 31) >> 4) + (i16 % 4) * 4;
-#pragma unroll
-      for (int t = 0; t < DV / 32; ++t) {
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const short* a = v_lds +
-                           (32 * half + ks * 16 + hi * 8 + i16 / 4) * VS +
-                           t * 32 + dcol;
-          typedef __attribute__((address_space(3))) short4v lds4;
-          const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)a);
-          const short4v up =
-              __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)(a + 4 * VS));
-          const short8 vf = {lo[0], lo[1], lo[2], lo[3],
-                             up[0], up[1], up[2], up[3]};
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              __builtin_bit_cast(bf16x8, vf), pf[ks], acc[t], 0, 0, 0);
-        }
-      }
+      const short* kb = k_lds + (32 * half + qc) * KS + hi * 8;
+      const short* vb = v_lds + 32 * half * VS + 16 * ((lane & 31) >> 4) +
+                        (i16 % 4) * 4;
+      attend32<DK / 16, DV / 32, false>(
+          [&](int kk) { return *(const bf16x8*)(kb + kk * 16); },
+          [&](int row, int t) { return vb + row * VS + t * 32; }, qf,
+          scale_log2, sub + 31 <= off + pw0 && sub >= first_key(pw1),
+          first_key(p) - sub, off + p - sub, st, acc);
     }
   }
+  st.l = st.join();
 
   if (active) {
-    const float inv = 1.f / l_run;
+    const float inv = 1.f / st.l;
     short* o = a_.out + ((int64_t)(sq.row0 + p) * a_.H + h) * V;
 #pragma unroll
     for (int t = 0; t < DV / 32; ++t)
@@ -291,8 +220,6 @@ hipError_t launch(const Prefill& a, int kv_heads, int n_tiles,
   HIP_CHECK_LAST();
   return hipSuccess;
 }
-
-constexpr float LOG2E = 1.4426950408889634f;
 
 }  // namespace
 

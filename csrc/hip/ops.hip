@@ -56,7 +56,7 @@ hipError_t lds_flash_prefill(const void*, const void*, const void*,
 hipError_t lds_flash_prefill_glds(const void*, const void*, const void*,
                                   const int32_t*, const int32_t*,
                                   const int32_t*, void*, int, int, int, int,
-                                  int, int, float, hipStream_t);
+                                  int, int, float, int, hipStream_t);
 }
 
 namespace {
@@ -353,7 +353,7 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
 torch::Tensor flash_prefill(torch::Tensor q, torch::Tensor k_cache,
                             torch::Tensor v_cache, torch::Tensor block_tables,
                             torch::Tensor seq_meta, torch::Tensor tiles,
-                            double scale) {
+                            double scale, int64_t keys) {
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_meta); CHECK_GPU(tiles);
   TORCH_CHECK(q.dtype() == torch::kBFloat16, "flash_prefill expects bf16");
@@ -372,7 +372,8 @@ torch::Tensor flash_prefill(torch::Tensor q, torch::Tensor k_cache,
         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
         block_tables.data_ptr<int32_t>(), seq_meta.data_ptr<int32_t>(),
         tiles.data_ptr<int32_t>(), out.data_ptr(), (int)tiles.size(0), qh,
-        kvh, bs, d, (int)block_tables.size(1), (float)scale, cur_stream()));
+        kvh, bs, d, (int)block_tables.size(1), (float)scale, (int)keys,
+        cur_stream()));
     return out;
   }
   CHECK_HIP(lds_flash_prefill(
@@ -423,5 +424,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("part_tokens"), py::arg("scale"), py::arg("chunk") = 256,
         py::arg("waves") = 8);
   m.def("flash_prefill", &flash_prefill,
-        "fused MFMA causal varlen prefill attention over paged KV");
+        "fused MFMA causal varlen prefill attention over paged KV",
+        py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
+        py::arg("block_tables"), py::arg("seq_meta"), py::arg("tiles"),
+        py::arg("scale"), py::arg("keys") = -1);
 }

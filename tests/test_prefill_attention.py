@@ -1,0 +1,95 @@
+"""Prefill attention over the paged pool: edges of tiles, pages, heads and
+masks, both shapes of the workgroup, against float64."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+def _case(seqs, qpg, kvh, bs, fp8, scale):
+    """seqs: (new tokens, tokens before). Unused rows of pages hold NaN."""
+    g = torch.Generator("cuda").manual_seed(len(seqs) * qpg + bs)
+
+    def draw(*shape):
+        return torch.randn(*shape, device="cuda", generator=g)
+    pages = [-(-(c + p) // bs) for c, p in seqs]
+    dtype = torch.float8_e4m3fn if fp8 else torch.bfloat16
+    kc, vc = (draw(sum(pages) + 1, kvh, bs, D).to(dtype) for _ in range(2))
+    perm = torch.randperm(sum(pages) + 1, generator=g, device="cuda").int()
+    bt = torch.zeros(len(seqs), max(pages), dtype=torch.int32, device="cuda")
+    rows = sum(c for c, _ in seqs)
+    q = draw(rows, kvh * qpg, D).bfloat16()
+    want = torch.empty(q.shape, dtype=torch.float64, device="cuda")
+    meta, at, row = [], 0, 0
+    for i, (c, p) in enumerate(seqs):
+        mine = perm[at:at + pages[i]]
+        bt[i, :pages[i]], at = mine, at + pages[i]
+        k, v = (x[mine.long()].double().permute(1, 0, 2, 3)
+                .reshape(kvh, -1, D)[:, :c + p] for x in (kc, vc))
+        see = torch.arange(c + p, device="cuda") <= p + torch.arange(
+            c, device="cuda")[:, None]
+        for h in range(kvh * qpg):
+            s = q[row:row + c, h].double() @ k[h // qpg].t().contiguous()
+            s = (s * scale).masked_fill(~see, -torch.inf)
+            want[row:row + c, h] = s.softmax(-1) @ v[h // qpg]
+        if (c + p) % bs:
+            for x in (kc, vc):
+                x[mine[-1].long(), :, (c + p) % bs:] = float("nan")
+        meta.append((row, c, p))
+        row += c
+    tiles = [(i, v) for i, (c, _) in enumerate(seqs)
+             for v in range(0, c * qpg, 128)]
+    ints = [torch.tensor(t, dtype=torch.int32, device="cuda")
+            for t in (meta, tiles)]
+    return (q, kc, vc, bt, *ints, scale), want
+
+
+def _close(got, want):
+    # probabilities and results are rounded to bf16: 2^-9 each, over sums of
+    # values of size 1 whose weights add up to 1
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -7,
+                               atol=2 ** -7)
+
+
+SEQS = [[(1, 0)], [(1, 700), (31, 0), (32, 1), (33, 31)],
+        [(127, 65), (129, 0), (5, 1023)], [(260, 0), (64, 64), (95, 33)]]
+
+
+@pytest.mark.parametrize("seqs", SEQS)
+@pytest.mark.parametrize("qpg,kvh", [(1, 3), (2, 8), (4, 2), (8, 1)])
+@pytest.mark.parametrize("bs", [16, 5])
+@pytest.mark.parametrize("keys", [0, 1, -1])
+def test_pages_in_bf16(seqs, qpg, kvh, bs, keys):
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case(seqs, qpg, kvh, bs, False, D ** -0.5)
+    _close(ext.flash_prefill(*args, keys=keys), want)
+
+
+@pytest.mark.parametrize("seqs", SEQS)
+@pytest.mark.parametrize("qpg,kvh", [(1, 3), (4, 2), (8, 1)])
+@pytest.mark.parametrize("bs", [16, 5])
+def test_pages_in_fp8(seqs, qpg, kvh, bs):
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case(seqs, qpg, kvh, bs, True, D ** -0.5)
+    _close(ext.flash_prefill(*args), want)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("keys", [0, 1])
+@pytest.mark.parametrize("scale", [-0.1, 0.0, 2.0])
+def test_scales(fp8, keys, scale):
+    """A negative scale turns the order of the scores round, a large one
+    moves the maximum at every tile."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case([(70, 300), (40, 0)], 4, 2, 16, fp8, scale)
+    _close(ext.flash_prefill(*args, keys=keys), want)
+
+
+def test_long_tables_stage_through_registers():
+    """More pages than the table of the direct kernel holds, in bf16."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case([(150, 40), (3, 90)], 4, 2, 16, False, D ** -0.5)
+    wide = torch.zeros(2, 1025, dtype=torch.int32, device="cuda")
+    wide[:, :args[3].shape[1]] = args[3]
+    _close(ext.flash_prefill(*args[:3], wide, *args[4:]), want)
