@@ -51,6 +51,11 @@ class GpuPrefixIndex:
                            max_blocks: int, seed0: int):
         """Hash a whole admission batch in one launch.
         Returns (hashes [R, max_blocks] uint64 on device, counts [R])."""
+        out = self.ext.hash_lists(token_lists, block_tokens, max_blocks,
+                                  _i64(seed0), self.keys) \
+            if type(token_lists) is list else None
+        if out is not None:        # lists of plain ints
+            return out
         lens = [len(t) for t in token_lists]
         flat = np.concatenate([np.asarray(t, dtype=np.int32)
                                for t in token_lists]) if token_lists else \
