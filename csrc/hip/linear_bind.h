@@ -39,7 +39,7 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
       w.scalar_type() != at::kBFloat16)
     return false;
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
-  if (M < 1 || M > 128 || K < 8 || K % 8 || N < 8 || N % 8 ||
+  if (M < 1 || M > 256 || K < 8 || K % 8 || N < 8 || N % 8 ||
       w.size(1) != K || N > (1 << 24) || K > (1 << 24) ||
       (use == GATED && N % 16) ||
       !lds_linear_rows_takes((int)M, (int)(use == GATED ? N / 2 : N), (int)K,

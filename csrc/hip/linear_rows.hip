@@ -1,21 +1,23 @@
-// linear_rows.hip — y = x w' for up to 128 rows of x (bf16, 32-bit sums).
+// linear_rows.hip — y = x w' for few rows of x (bf16, 32-bit sums): the kernel
+// for up to 16 rows, and which product goes where. Products of up to 256 rows
+// go to linear_tiles.hip.
 //
 // The weights' bytes are what counts, so they go straight from memory into
 // matrix-core operands, once, with plain loads (marked non-temporal they come
 // at three quarters of the rate). A workgroup owns 128 or 256 output channels
 // (8 waves of 16 CT) and walks K in steps of 128; a wave reads 256 bytes of 16
 // weight rows per step, two steps ahead. x goes through LDS: the waves share
-// it, since a workgroup that reads x for each wave (or few channels for each
-// x) spends as much of the caches' rate on x as on weights. Loads retire in
-// order, so x of a step is asked for ahead of the weights of that step. The
-// order of K inside a step is the same for both operands, and workgroups start
-// at different steps: in step they would hit the same few memory channels
-// where rows are a power of two apart.
+// it, since a workgroup that reads x for each wave spends as much of the
+// caches' rate on x as on weights. Loads retire in order, so x of a step is
+// asked for ahead of the weights of that step. Workgroups start at different
+// steps: in step they would hit the same few memory channels where rows are a
+// power of two apart. linear_tiles.hip adds up in the same order, so a row
+// comes out the same, to the bit, whichever of the two took it: as the one row
+// of a decode step or within a short prompt.
 //
-// Measured, cold weights, without the sum of the parts (library call: its time
-// on the device): 4096 -> 28672, 30 rows: 45 us, 5.3 TB/s (49); 14336 -> 4096,
-// 30 rows: 24 us, 5.0 TB/s (31; 69 with weights stored [in, out]); 25600 ->
-// 5120, 30 rows: 50 us, 5.2 TB/s (145); 4096 -> 4096, 1 row: 9 us (15).
+// Measured, 1 row, cold weights, without the sum of the parts (library: its
+// time on the device): 4096 -> 28672: 43 us, 5.5 TB/s (58); 14336 -> 4096 22 us
+// (26); 25600 -> 5120: 47 us (134); 4096 -> 4096: 8.4 us (15).
 #include "layered/elem.h"
 
 namespace {
@@ -36,11 +38,10 @@ enum Out { BF16, F32, GATED };
 
 constexpr int NW = 8, KS = 128, XS = KS + 8;   // XS: row of x in LDS
 
-template <int CT, int MT, int OUT>
+template <int CT, int OUT>
 __global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
-  __shared__ __align__(16) short xl[2][16 * MT * XS];
-  constexpr int WI = KS / 32, XR = NW * WAVE / (KS / 8);
-  constexpr int XT = (16 * MT + XR - 1) / XR;      // pieces of x per thread
+  __shared__ __align__(16) short xl[2][16 * XS];
+  constexpr int WI = KS / 32;
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane % 16, grp = lane / 16, M = p.M, N = p.N;
   const int k_lo = blockIdx.y * p.k_part, k_hi = min(p.K, k_lo + p.k_part);
@@ -52,23 +53,21 @@ __global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
 #pragma unroll
   for (int c = 0; c < CT; ++c)
     wr[c] = p.w + (min(n0 + c * 16 + col, N - 1) + wave / NC * N) * p.w_row +
-            grp * 16;
+            grp * 8;
+  // half of the threads bring 16 bytes of x each
   const int xr = threadIdx.x / (KS / 8), xp = threadIdx.x % (KS / 8);
-  const short* xg[XT];
+  const bool x_mine = xr < 16;
+  const short* xg = p.x + min(xr, M - 1) * p.x_row + xp * 8;
+  float4v acc[CT];
 #pragma unroll
-  for (int j = 0; j < XT; ++j)
-    xg[j] = p.x + min(xr + j * XR, M - 1) * p.x_row + xp * 8;
-  float4v acc[CT][MT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < CT; ++c) acc[c] = (float4v){0.f, 0.f, 0.f, 0.f};
   const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  short8 w0[CT][WI], w1[CT][WI], xn[XT];
+  short8 w0[CT][WI], w1[CT][WI], xn = zero;
   const int steps = (k_hi - k_lo + KS - 1) / KS;
-  const int first = blockIdx.x * 3u % steps;   // 1 instead of 3: gate and up
-                                               // of a wave pair collide, 60 us
-                                               // for 44
+  // where rows are 8 KB apart, 1 of 4096 -> 28672: a start of 3 blockIdx.x 43
+  // us, 1: 44, 2: 72, 6: 51, none: 52; gated, with twice the streams, 6: 42.5,
+  // 3: 45, 1: 67, none: 52. Other sizes hardly mind.
+  const int first = blockIdx.x * (OUT == GATED ? 6u : 3u) % steps;
   auto at = [&](int s) {
     s += first;
     return k_lo + (s >= steps ? s - steps : s) * KS;
@@ -80,37 +79,27 @@ __global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
     for (int c = 0; c < CT; ++c)
 #pragma unroll
       for (int i = 0; i < WI; ++i) {
-        const int k = k0 + i / 2 * 64 + i % 2 * 8;
-        r[c][i] = whole || k + grp * 16 < k_hi ? *(const short8*)(wr[c] + k)
+        const int k = k0 + i * 32;
+        r[c][i] = whole || k + grp * 8 < k_hi ? *(const short8*)(wr[c] + k)
                                                : zero;
       }
   };
   auto fetch_x = [&](int s) {
     const int k0 = at(s);
-#pragma unroll
-    for (int j = 0; j < XT; ++j)
-      xn[j] = k0 + xp * 8 < k_hi ? *(const short8*)(xg[j] + k0) : zero;
+    if (x_mine) xn = k0 + xp * 8 < k_hi ? *(const short8*)(xg + k0) : zero;
   };
   auto put_x = [&](int b) {
-#pragma unroll
-    for (int j = 0; j < XT; ++j)
-      if (16 * MT % XR == 0 || xr + j * XR < 16 * MT)
-        *(short8*)(xl[b] + (xr + j * XR) * XS + xp * 8) = xn[j];
+    if (x_mine) *(short8*)(xl[b] + xr * XS + xp * 8) = xn;
   };
   auto step = [&](auto& r, int b, int s) {
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
-      bf16x8 xf[MT];
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-        xf[t] = *(const bf16x8*)(xl[b] + (t * 16 + col) * XS + i / 2 * 64 +
-                                 grp * 16 + i % 2 * 8);
+      const bf16x8 xf =
+          *(const bf16x8*)(xl[b] + col * XS + i * 32 + grp * 8);
 #pragma unroll
       for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, r[c][i]), xf[t], acc[c][t], 0, 0, 0);
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, r[c][i]), xf, acc[c], 0, 0, 0);
     }
     if (s + 1 < steps) put_x(b ^ 1);
     if (s + 2 < steps) fetch_x(s + 2);
@@ -131,39 +120,34 @@ __global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
   }
   float4v* up = (float4v*)xl;              // no longer read: the loop's end
   if constexpr (OUT == GATED) {
-    static_assert(sizeof(xl) >= NC * CT * MT * WAVE * sizeof(float4v));
+    static_assert(sizeof(xl) >= NC * CT * WAVE * sizeof(float4v));
     if (wave >= NC) {
 #pragma unroll
       for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          up[(((wave - NC) * CT + c) * MT + t) * WAVE + lane] = acc[c][t];
+        up[((wave - NC) * CT + c) * WAVE + lane] = acc[c];
     }
     __syncthreads();
     if (wave >= NC) return;
   }
 #pragma unroll
-  for (int c = 0; c < CT; ++c)
+  for (int c = 0; c < CT; ++c) {
+    const int n = n0 + c * 16 + grp * 4, m = col;
+    if (n >= N || m >= M) continue;        // N is a multiple of 4
+    const float4v a = acc[c];
+    const int64_t o = ((int64_t)blockIdx.y * M + m) * N + n;
+    if constexpr (OUT == F32) {
+      *(float4v*)((float*)p.y + o) = a;
+    } else {
+      short4v v;
+      float4v u = a;
+      if constexpr (OUT == GATED) u = up[(wave * CT + c) * WAVE + lane];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int n = n0 + c * 16 + grp * 4, m = t * 16 + col;
-      if (n >= N || m >= M) continue;      // N is a multiple of 4
-      const float4v a = acc[c][t];
-      const int64_t o = ((int64_t)blockIdx.y * M + m) * N + n;
-      if constexpr (OUT == F32) {
-        *(float4v*)((float*)p.y + o) = a;
-      } else {
-        short4v v;
-        float4v u = a;
-        if constexpr (OUT == GATED)
-          u = up[((wave * CT + c) * MT + t) * WAVE + lane];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          v[r] = f32_to_bf16(OUT == GATED ? activate(p.act, a[r]) * u[r]
-                                          : a[r]);
-        *(short4v*)((short*)p.y + o) = v;
-      }
+      for (int r = 0; r < 4; ++r)
+        v[r] = f32_to_bf16(OUT == GATED ? activate(p.act, a[r]) * u[r]
+                                        : a[r]);
+      *(short4v*)((short*)p.y + o) = v;
     }
+  }
 }
 
 // sum of the parts; n4: float4s of one
@@ -212,68 +196,73 @@ __global__ __launch_bounds__(256) void lay_weights_kernel(
   }
 }
 
-// 16-channel tiles per wave. 256 channels per workgroup halve what x costs
-// beside the weights: from 33 rows on that is worth it, unless the output is
-// so narrow that K falls into many parts (50 rows: 4096 -> 28672 45 us with
-// 256 in two parts, 50 with 128; 14336 -> 4096 27 in 16 parts, 26 in 8), and
-// where 128 would make more than one round of the 256 compute units.
-int channel_tiles(int M, int weight_rows) {
-  if (weight_rows > 128 * 256) return 2;
-  return M > 32 && weight_rows > 4096 ? 2 : 1;
-}
+// 16-channel tiles per wave: two where 128 channels per workgroup would make
+// more than one round of the 256 compute units
+int channel_tiles(int weight_rows) { return weight_rows > 128 * 256 ? 2 : 1; }
 
-template <int CT, int MT, int OUT>
+template <int CT, int OUT>
 hipError_t go(const Rows& p, int parts, hipStream_t stream) {
   constexpr int width = NW * 16 * CT / (OUT == GATED ? 2 : 1);
-  hipLaunchKernelGGL((linear_rows_kernel<CT, MT, OUT>),
+  hipLaunchKernelGGL((linear_rows_kernel<CT, OUT>),
                      dim3((p.N + width - 1) / width, parts), dim3(NW * WAVE),
                      0, stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }
 
-template <int CT, int OUT>
-hipError_t go_rows(const Rows& p, int parts, hipStream_t stream) {
-  if (p.M <= 16) return go<CT, 1, OUT>(p, parts, stream);
-  if (p.M <= 32) return go<CT, 2, OUT>(p, parts, stream);
-  if (OUT == GATED || p.M <= 64) return go<CT, 4, OUT>(p, parts, stream);
-  if (p.M <= 96) return go<CT, 6, OUT>(p, parts, stream);
-  return go<CT, 8, OUT>(p, parts, stream);
+// up to 16 rows come here, more go to linear_tiles.hip
+constexpr int ROWS = 16, TILE_ROWS = 256;
+
+// of one part of K
+int workgroups(int M, int N) {
+  const int width = M <= ROWS ? 128 * channel_tiles(N) : 128;
+  return (N + width - 1) / width;
 }
 
 }  // namespace
 
 extern "C" {
 
+hipError_t lds_linear_tiles(const void*, int64_t, const void*, int64_t, void*,
+                            int, int, int, int, int, int, hipStream_t);
+
 // Parts of K of a product: as many as make up one round of the 256 compute
-// units, each with two steps of K at least. (4096 -> 4096, 1 row: 9 us in 8
-// parts and 4 for their sum, 25 in one.)
+// units, each with 256 of K at least. (4096 -> 4096, 1 row: 9 us in 8 parts
+// and 4 for their sum, 25 in one; 150 rows: 14 us in 8 parts, 17 in 4, 18 in
+// 16.)
 int lds_linear_rows_parts(int M, int N, int K) {
-  const int width = 128 * channel_tiles(M, N);
-  int parts = 256 / ((N + width - 1) / width);
-  if (parts > K / (2 * KS)) parts = K / (2 * KS);
+  int parts = 256 / workgroups(M, N);
+  if (parts > K / 256) parts = K / 256;
   if (parts < 1) parts = 1;
   const int k_part = ((K + parts - 1) / parts + KS - 1) / KS * KS;
   return (K + k_part - 1) / k_part;
 }
 
-// Whether a product of M rows is faster here than in the library (device
-// times, here / there, of 4096 -> 4096 W, 4096 -> 12576 I, 14336 -> 4096 D,
-// 4096 -> 32768 H and 4096 -> [2 x 14336] G).
-//   parts: the caller sums the parts itself: always. 1 row: W 9 / 15, I 21 /
-//     28, D 22 / 26; 64 rows: W 11 / 15, I 26 / 26, D 28 / 39.
-//   plain, in parts: their sum is a launch of 4.5 us. Up to 32 rows the call
-//     is as fast or faster and costs the host half as much; above only where
-//     the output is narrow: 50 rows W 15 / 14, I 30 / 25, D 31 / 36; 128 rows
-//     D 43 / 75.
-//   plain, in one: 96 rows H 62 / 63, 128 rows H 69 / 64.
-//   gated: 64 rows G 52 / 53 (with its activation), 96 rows G 60 / 58. The
-//     library is better in wide ones: 5120 -> [2 x 25600], 30 rows, 106 / 97.
+// Whether a product of M rows is faster here than in the library. Device
+// times, here / there, in us:
+//   parts the caller sums itself: always. 4096 -> 4096: 1 row 8 / 15, 96 rows
+//     12 / 22, 256 rows 18 / 23; 14336 -> 4096: 64 rows 23 / 40, 256 rows
+//     41 / 63; 4096 -> 12576: 64 rows 24 / 25, 256 rows 42 / 50.
+//   one part, and gated ones (there with their activation): if the workgroups
+//     fill at least 7/8 of their rounds, up to 128 rows. 4096 -> 32768: 32 rows
+//     46 / 62, 128 rows 55 / 64, 160 rows 66 / 67; -> 128256 (98 %): 64 rows
+//     182 / 208; 5120 -> 51200 (78 %): 64 rows 110 / 98. 4096 -> [2 x 14336]:
+//     64 rows 44 / 58, 128 rows 53 / 60, 160 rows 65 / 63; 2048 -> [2 x 4096]
+//     (25 %): 32 rows 18 / 16.
+//   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
+//     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
+//     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
+//     narrow ones up to 64 rows (4096 -> 1024: 64 rows 11 / 15, 96 rows
+//     13 / 12; 4096 -> 12576, 77 %: 64 rows 27 / 25).
 int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
-  if (parts) return M <= 128;
-  if (gated) return M <= 64 && 2 * N <= 128 * 256;
-  if (lds_linear_rows_parts(M, N, K) == 1) return M <= 96;
-  return M <= 32 || (M <= 128 && K >= 2 * N);
+  if (M > TILE_ROWS) return 0;
+  const int n = gated ? 1 : lds_linear_rows_parts(M, N, K);
+  if (parts && n > 1) return 1;
+  const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
+  const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
+  if (gated || N > 128 * 128) return full && M <= 128;
+  if (full) return M <= 64 || K >= 4096;
+  return M <= 64 && N <= 4096;
 }
 
 // x [M, K], w [N, K], rows x_row and w_row apart and 16-byte aligned; y [M, N]
@@ -282,21 +271,25 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
 hipError_t lds_linear_rows(const void* x, int64_t x_row, const void* w,
                            int64_t w_row, void* y, float* part, int parts,
                            int M, int N, int K, int f32, hipStream_t stream) {
-  if (M < 1 || M > 128 || N < 1 || N % 4 || K < 8 || K % 8 || x_row % 8 ||
-      w_row % 8 || parts < 1 || (!part && (parts > 1 || !y)))
+  if (M < 1 || M > TILE_ROWS || N < 1 || N % 4 || K < 8 || K % 8 ||
+      x_row % 8 || w_row % 8 || parts < 1 || (!part && (parts > 1 || !y)))
     return hipErrorInvalidValue;
-  Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K, K, 0};
-  p.k_part = ((K + parts - 1) / parts + KS - 1) / KS * KS;
-  if (parts > 1 || !y) p.y = part;
-  const bool two = channel_tiles(M, N) == 2;
+  const bool in_part = parts > 1 || !y;
   hipError_t e;
-  if (f32 || p.y == part)
-    e = two ? go_rows<2, F32>(p, parts, stream)
-            : go_rows<1, F32>(p, parts, stream);
-  else
-    e = two ? go_rows<2, BF16>(p, 1, stream) : go_rows<1, BF16>(p, 1, stream);
-  if (e != hipSuccess || p.y == y) return e;
-  if (!y) return hipSuccess;
+  if (M > ROWS) {
+    e = lds_linear_tiles(x, x_row, w, w_row, in_part ? part : y, parts, M, N,
+                         K, in_part || f32, -1, stream);
+  } else {
+    Rows p{(const short*)x, (const short*)w, x_row, w_row,
+           in_part ? part : y, M, N, K, K, 0};
+    p.k_part = ((K + parts - 1) / parts + KS - 1) / KS * KS;
+    const bool two = channel_tiles(N) == 2;
+    if (in_part || f32)
+      e = two ? go<2, F32>(p, parts, stream) : go<1, F32>(p, parts, stream);
+    else
+      e = two ? go<2, BF16>(p, 1, stream) : go<1, BF16>(p, 1, stream);
+  }
+  if (e != hipSuccess || !in_part || !y) return e;
   const int64_t n4 = (int64_t)M * N / 4;
   const dim3 grid((uint32_t)((n4 + 255) / 256));
   if (f32)
@@ -325,13 +318,15 @@ hipError_t lds_lay_weights(const float* in, void* out, int R, int C,
 hipError_t lds_gated_rows(const void* x, int64_t x_row, const void* w,
                           int64_t w_row, void* y, int M, int N, int K, int act,
                           hipStream_t stream) {
-  if (M < 1 || M > 64 || N < 1 || N % 4 || K < 8 || K % 8 || x_row % 8 ||
-      w_row % 8 || act < 0 || act >= ACTS)
+  if (M < 1 || M > TILE_ROWS || N < 1 || N % 4 || K < 8 || K % 8 ||
+      x_row % 8 || w_row % 8 || act < 0 || act >= ACTS)
     return hipErrorInvalidValue;
+  if (M > ROWS)
+    return lds_linear_tiles(x, x_row, w, w_row, y, 1, M, N, K, 0, act, stream);
   // 64 channels per workgroup: 128 rows of weights
   const Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K,
                (K + KS - 1) / KS * KS, act};
-  return go_rows<1, GATED>(p, 1, stream);
+  return go<1, GATED>(p, 1, stream);
 }
 
 }  // extern "C"
