@@ -6,7 +6,7 @@
 // Pairs are sorted by expert (stable, so results do not depend on timing) and
 // cut into tiles of one expert each; the product kernels take one tile and a
 // block of output channels per workgroup:
-//   expert_tiles   128 pairs and 256 channels through LDS, for many pairs
+//   expert_tiles   256 pairs and 256 channels through LDS, for many pairs
 //   expert_rows    up to 64 pairs, weights straight into registers, for few:
 //                  there the weights' bytes are what counts
 //   expert_plain   any size, bf16 or float
@@ -134,12 +134,13 @@ __device__ __forceinline__ void load_ids(const int32_t* ids, int i, int P,
 }
 
 // One workgroup per expert. order [P]: pairs by expert; tiles [1 + max_tiles]
-// = (number of tiles, ..), then (expert, first place in order, pairs, 0).
+// = (number of tiles, those more than half full, ..), then (expert, first
+// place in order, pairs, 0), those more than half full ahead.
 __global__ __launch_bounds__(ST) void sort_pairs_kernel(
     const int32_t* __restrict__ ids, int32_t* __restrict__ order,
     int4* __restrict__ tiles, int P, int E, int tile) {
   extern __shared__ int hist[];        // [E]
-  __shared__ int sums[ST / WAVE], at[2];
+  __shared__ int sums[ST / WAVE], at[4];
   const int e = blockIdx.x, tid = threadIdx.x;
   const int wave = tid / WAVE, lane = tid % WAVE;
   for (int i = tid; i < E; i += ST) hist[i] = 0;
@@ -152,28 +153,40 @@ __global__ __launch_bounds__(ST) void sort_pairs_kernel(
       if (x[j] >= 0 && x[j] < E) atomicAdd(&hist[x[j]], 1);
   }
   __syncthreads();
-  if (wave == 0) {                     // pairs and tiles of lower experts
-    int n = 0, t = 0;
-    for (int i = lane; i < e; i += WAVE) {
-      n += hist[i];
-      t += (hist[i] + tile - 1) / tile;
+  if (wave == 0) {       // pairs and tiles of lower experts, full ones of all
+    int n = 0, full = 0, rest = 0, all = 0;
+    for (int i = lane; i < E; i += WAVE) {
+      const int f = (hist[i] + (tile - 1) / 2) / tile;
+      all += f;
+      if (i < e) {
+        n += hist[i];
+        full += f;
+        rest += (hist[i] + tile - 1) / tile - f;
+      }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       n += __shfl_xor(n, o, WAVE);
-      t += __shfl_xor(t, o, WAVE);
+      full += __shfl_xor(full, o, WAVE);
+      rest += __shfl_xor(rest, o, WAVE);
+      all += __shfl_xor(all, o, WAVE);
     }
     if (lane == 0) {
       at[0] = n;
-      at[1] = t;
+      at[1] = full;
+      at[2] = rest;
+      at[3] = all;
     }
   }
   __syncthreads();
-  const int first = at[0], count = hist[e], nt = (count + tile - 1) / tile;
+  const int first = at[0], count = hist[e];
+  const int nt = (count + tile - 1) / tile;
+  const int nf = (count + (tile - 1) / 2) / tile;
   for (int j = tid; j < nt; j += ST)
-    tiles[1 + at[1] + j] =
+    tiles[1 + (j < nf ? at[1] + j : at[3] + at[2])] =
         make_int4(e, first + j * tile, min(tile, count - j * tile), 0);
-  if (e == E - 1 && tid == 0) tiles[0] = make_int4(at[1] + nt, 0, 0, 0);
+  if (e == E - 1 && tid == 0)
+    tiles[0] = make_int4(at[3] + at[2] + nt - nf, at[3], 0, 0);
   int base = first;
   for (int i0 = 0; i0 < P; i0 += ST * SV) {   // workgroup-uniform
     const int i = i0 + tid * SV;
@@ -337,109 +350,132 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
   }
 }
 
-// 256 channels x 128 pairs, K in steps of 64 through three LDS buffers that are
-// filled straight from memory, two steps ahead. A row of a step is 128 bytes =
-// 8 pieces; piece c of row r lies at place c ^ (r / 2 % 8): the 16 rows a read
-// serves at once then meet all 64 banks. 4 waves, 128 x 64 each, CT x PT tiles
-// of 32 x 32. Loads and LDS reads are spread between the matrix instructions:
-// issued in a row they would hold the wave up.
-constexpr int CT = 4, PT = 2, NB = 3, BK = 64;
-constexpr int TC = 64 * CT, TILE = 64 * PT;
-constexpr int BUF = (TC + TILE) * BK;
-constexpr int TILES_LDS = NB * BUF * (int)sizeof(short);
-constexpr int TG = 8;                // tiles of pairs that run side by side
+// 256 channels x 256 pairs, K in steps of 64, both operands loaded straight to
+// LDS. What bounds it is the way from the L2s to LDS and the power that it
+// takes (without the loads 28000 pairs of 4096 x 3584 take 1230 us for 1960,
+// without the LDS reads 1910), hence the size of the tile, and whole lines of
+// 128 bytes. LDS holds five chunks of 256 rows, those of weights and of pairs
+// in turn: two and a half steps. 4 waves, CT x PT tiles of 32 x 32 each:
+// 128 x 128, or, where a tile has no more than 128 pairs, 64 x 128 (so nothing
+// is lost by the larger tile). A row of a step is 8 pieces; piece c of row r
+// lies at place c ^ (r / 2 % 8): the 16 rows a read serves at once then meet
+// all 64 banks. Loads and LDS reads are spread between the matrix instructions:
+// issued in a row they would hold the wave up. Operands are read 16 of K ahead,
+// across the one barrier of a step.
+//
+// Both products: 7032 rows, 32 experts of 4096 x 3584, 4 each: 1670 us, 990
+// TFLOP/s (128 pairs per tile and the reads of a step behind its barrier:
+// 1840; 256 with half lines in steps of 32: 1900; 8 waves of 64 x 64: 1800);
+// 1000 rows, 2048 x 1536: 129 (165).
+constexpr int NB = 5, BK = 64;       // chunks; K of a step
+constexpr int TC = 256, TILE = 256, HALF = 128;
+constexpr int CHUNK = 256 * BK;
+constexpr int TILES_LDS = NB * CHUNK * (int)sizeof(short);
+constexpr int TG = 3;                // tiles of pairs that run side by side
 
-template <bool UP>
-__global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
-  extern __shared__ __align__(16) short tile_lds[];  // NB x [weights, pairs]
+// WC waves across the channels, the others across the pairs
+template <bool UP, int CT, int PT, int WC>
+__device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
+                                             const int4 tile, int n0) {
+  static_assert(32 * CT * WC == TC, "");
+  constexpr int LW = TC / 32, LP = PT * (4 / WC);      // loads per step
+  static_assert(LW == 8 && LP <= CT + PT, "");
   const int N = p.N, K = p.K;
-  // Workgroups go round the 8 XCDs in turn: each XCD gets a contiguous share
-  // of the work, in which TG tiles of pairs walk the channels together.
-  const int nx = (N + TC - 1) / TC, total = p.tiles[0].x * nx;
-  const int share = (total + 7) / 8;
-  const int id = blockIdx.x % 8 * share + blockIdx.x / 8;
-  if ((int)blockIdx.x / 8 >= share || id >= total) return;
-  const int g = id / (TG * nx), in = id % (TG * nx);
-  const int width = min(TG, p.tiles[0].x - g * TG);
-  const int4 tile = p.tiles[1 + g * TG + in % width];
-  const int n0 = in / width * TC;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int col = lane & 31, hi = lane >> 5;
-  const int wc = wave & 1, wp = wave >> 1;    // its channels, its pairs
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, col = lane & 31, hi = lane >> 5;
+  const int wc = wave % WC, wp = wave / WC;    // its channels, its pairs
 
   // A wave fills a quarter of the rows of both, 8 rows per instruction, from
   // byte offsets within the expert's weights and p.a (both under 4 GiB).
   // Rows past the tile repeat its last one: they are computed and dropped.
-  constexpr int LW = 2 * CT, LOADS = 2 * CT + 2 * PT;
   const char* wbase = (const char*)p.w + (int64_t)tile.x * N * K * 2;
   const char* abase = (const char*)p.a;
-  uint32_t src[LOADS];
-  int64_t rows[2 * PT];
-#pragma unroll
-  for (int j = 0; j < 2 * PT; ++j)
-    rows[j] = source<UP>(p, tile.y + min(wave * 16 * PT + j * 8 + lane / 8,
-                                         tile.z - 1));
   auto piece = [&](int j) {
     return (lane % 8 ^ (lane / 16 + j % 2 * 4)) * 8;
   };
+  uint32_t wsrc[LW], asrc[LP];
+  int64_t rows[LP];
+#pragma unroll
+  for (int j = 0; j < LP; ++j)
+    rows[j] = source<UP>(p, tile.y + min((wave * LP + j) * 8 + lane / 8,
+                                         tile.z - 1));
 #pragma unroll
   for (int j = 0; j < LW; ++j)
-    src[j] = ((uint32_t)min(n0 + wave * 16 * CT + j * 8 + lane / 8, N - 1) *
-                  K + piece(j)) * 2;
+    wsrc[j] = ((uint32_t)min(n0 + (wave * LW + j) * 8 + lane / 8, N - 1) * K +
+               piece(j)) * 2;
   const int steps = K / BK;
-  auto column = [&](int s) { return min(s, steps - 1) * BK * 2; };
-  auto load = [&](int buf, int k, int j) {
-    typedef __attribute__((address_space(1))) const unsigned int gmem;
-    typedef __attribute__((address_space(3))) unsigned int smem;
-    const int row = j < LW ? wave * 16 * CT + j * 8
-                           : TC + wave * 16 * PT + (j - LW) * 8;
+  typedef __attribute__((address_space(1))) const unsigned int gmem;
+  typedef __attribute__((address_space(3))) unsigned int smem;
+  // past the end the last step repeats
+  auto load_w = [&](int s, int chunk, int j) {
     __builtin_amdgcn_global_load_lds(
-        (gmem*)((j < LW ? wbase : abase) + k + src[j]),
-        (smem*)(tile_lds + buf * BUF + row * BK), 16, 0, 0);
+        (gmem*)(wbase + min(s, steps - 1) * BK * 2 + wsrc[j]),
+        (smem*)(lds + chunk * CHUNK + (wave * LW + j) * 8 * BK), 16, 0, 0);
+  };
+  auto load_a = [&](int s, int chunk, int j) {
+    __builtin_amdgcn_global_load_lds(
+        (gmem*)(abase + min(s, steps - 1) * BK * 2 + asrc[j]),
+        (smem*)(lds + chunk * CHUNK + (wave * LP + j) * 8 * BK), 16, 0, 0);
   };
 #pragma unroll
-  for (int j = 0; j < LW; ++j) load(0, column(0), j);
+  for (int j = 0; j < LW; ++j) load_w(0, 0, j);
 #pragma unroll
-  for (int j = 0; j < 2 * PT; ++j)
-    src[LW + j] = ((uint32_t)rows[j] * K + piece(j)) * 2;
+  for (int j = 0; j < LP; ++j)
+    asrc[j] = ((uint32_t)rows[j] * K + piece(j)) * 2;
 #pragma unroll
-  for (int j = LW; j < LOADS; ++j) load(0, column(0), j);
+  for (int j = 0; j < LP; ++j) load_a(0, 1, j);
 #pragma unroll
-  for (int j = 0; j < LOADS; ++j) load(1, column(1), j);
+  for (int j = 0; j < LW; ++j) load_w(1, 2, j);
+#pragma unroll
+  for (int j = 0; j < LP; ++j) load_a(1, 3, j);
 
   f32x16 acc[CT][PT];
 #pragma unroll
   for (int c = 0; c < CT; ++c)
 #pragma unroll
     for (int t = 0; t < PT; ++t) acc[c][t] = (f32x16)(0.f);
-  int buf = 0, fill = NB - 1;
+  bf16x8 wf[2][CT], af[2][PT];
+  const short* wl = lds + (wc * 32 * CT + col) * BK;
+  const short* al = lds + (wp * 32 * PT + col) * BK;
+  auto read = [&](int x, int w_chunk, int a_chunk, int kk) {
+    const int at = ((kk * 2 + hi) ^ (col / 2 & 7)) * 8;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+      wf[x][c] = *(const bf16x8*)(wl + w_chunk * CHUNK + c * 32 * BK + at);
+#pragma unroll
+    for (int t = 0; t < PT; ++t)
+      af[x][t] = *(const bf16x8*)(al + a_chunk * CHUNK + t * 32 * BK + at);
+  };
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LW + LP) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  read(0, 0, 1, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto after = [](int chunk, int n) {
+    return chunk + n < NB ? chunk + n : chunk + n - NB;
+  };
+  int at = 0;                  // chunk of this step's weights
   for (int s = 0; s < steps; ++s) {
-    // this step has landed (the next may be on its way), and the buffer that
-    // is filled now is no longer read
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LOADS) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    const int k = column(s + NB - 1);          // the last step repeats
-    const short* wl = tile_lds + buf * BUF + (wc * 32 * CT + col) * BK;
-    const short* al = tile_lds + buf * BUF + (TC + wp * 32 * PT + col) * BK;
-    bf16x8 wf[2][CT], af[2][PT];
-    auto read = [&](int x, int kk) {
-      const int at = ((kk * 2 + hi) ^ (col / 2 & 7)) * 8;
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
-        wf[x][c] = *(const bf16x8*)(wl + c * 32 * BK + at);
+    for (int kk = 0; kk < 4; ++kk) {
+      if (kk == 3) {
+        // All operands of this step are in registers: its chunks can be
+        // filled. The next step has landed, the weights after it may not.
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(0, after(at, 2), after(at, 3), 0);
+      } else {
+        read(kk + 1 & 1, at, after(at, 1), kk + 1);
+      }
+      if (kk == 3) {
 #pragma unroll
-      for (int t = 0; t < PT; ++t)
-        af[x][t] = *(const bf16x8*)(al + t * 32 * BK + at);
-    };
-    read(0, 0);
-    __builtin_amdgcn_sched_barrier(0);
+        for (int j = 0; j < LP; ++j) load_a(s + 2, at, j);
+      } else if (kk < 2) {
 #pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const bool more = kk + 1 < BK / 16;
-      if (more) read(kk + 1 & 1, kk + 1);
-#pragma unroll
-      for (int j = 0; j < LOADS / 4; ++j) load(fill, k, kk * LOADS / 4 + j);
+        for (int j = 0; j < LW / 2; ++j)
+          load_w(s + 2, after(at, 4), kk * LW / 2 + j);
+      }
 #pragma unroll
       for (int c = 0; c < CT; ++c)
 #pragma unroll
@@ -447,42 +483,60 @@ __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
           acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
               wf[kk & 1][c], af[kk & 1][t], acc[c][t], 0, 0, 0);
       // the order: matrix, read, (load), ... matrix
+      const int loads = kk == 3 ? LP : kk < 2 ? LW / 2 : 0;
 #pragma unroll
       for (int i = 0; i < CT + PT; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (more) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (i % 2 == 0) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        if (i < loads) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
       }
       __builtin_amdgcn_sched_group_barrier(0x008, CT * PT - CT - PT, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
-    buf = buf + 1 == NB ? 0 : buf + 1;
-    fill = fill + 1 == NB ? 0 : fill + 1;
+    at = after(at, 2);
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the repeated loads
+  // no wave reads a buffer any more, and the repeated loads are in
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 
+  // The results turn round in the wave's share of LDS, so that a row of them
+  // is written in pieces of 16 bytes side by side (8 bytes of 32 rows at a
+  // time take 9 us, 8 % of the products' time).
+  constexpr int G = 4 * CT;                  // pieces of 8 channels in a row
+  static_assert(32 * PT * 8 * G * 4 <= NB * CHUNK, "");
+  short* mine = lds + wave * 32 * PT * 8 * G;
+  auto place = [](int row, int g) {
+    return (row * G + (g ^ (G == 16 ? row & 15 : row / 2 & 7))) * 8;
+  };
+  static_assert(G == 16 || G == 8, "");
   auto write = [&](auto act) {
 #pragma unroll
     for (int t = 0; t < PT; ++t) {
-      const int i = wp * 32 * PT + t * 32 + col;
-      if (i >= tile.z) continue;
-      const int pair = p.order[tile.y + i];
-      const float wt = UP ? p.weights[pair] : 1.f;
-      short* o = (short*)p.out + (int64_t)(UP ? tile.y + i : pair) * N;
+      const int i = min(wp * 32 * PT + t * 32 + col, tile.z - 1);
+      const float wt = UP ? p.weights[p.order[tile.y + i]] : 1.f;
 #pragma unroll
       for (int c = 0; c < CT; ++c)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int n = n0 + wc * 32 * CT + c * 32 + q * 8 + hi * 4;
-          if (n >= N) continue;
           short4v v;
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
             const float f = acc[c][t][4 * q + x];
             v[x] = f32_to_bf16(UP ? activate(act, f * wt) : f);
           }
-          *(short4v*)(o + n) = v;
+          *(short4v*)(mine + place(t * 32 + col, c * 4 + q) + hi * 4) = v;
         }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const int n = n0 + wc * 32 * CT + lane % G * 8;
+#pragma unroll 8
+    for (int j = 0; j < 32 * PT; j += WAVE / G) {
+      const int row = j + lane / G, i = wp * 32 * PT + row;
+      if (i >= tile.z || n >= N) continue;   // N is a multiple of 8
+      const int64_t to = UP ? tile.y + i : p.order[tile.y + i];
+      *(short8*)((short*)p.out + to * N + n) =
+          *(const short8*)(mine + place(row, lane % G));
     }
   };
   using std::integral_constant;
@@ -495,9 +549,38 @@ __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
 }
 
 template <bool UP>
+__global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
+  extern __shared__ __align__(16) short tile_lds[];  // NB x [weights, pairs]
+  // Workgroups go round the 8 XCDs in turn: each XCD gets a contiguous share
+  // of the tiles more than half full, then one of the others (the shorter
+  // work last), in which TG tiles of pairs walk the channels together.
+  const int nx = (p.N + TC - 1) / TC;
+  const int4 counts = p.tiles[0];
+  int n = counts.y, base = 1, at = blockIdx.x / 8;
+  int share = (n * nx + 7) / 8;
+  if (at >= share) {
+    at -= share;
+    base += n;
+    n = counts.x - n;
+    share = (n * nx + 7) / 8;
+  }
+  const int id = blockIdx.x % 8 * share + at;
+  if (at >= share || id >= n * nx) return;
+  const int g = id / (TG * nx), in = id % (TG * nx);
+  const int width = min(TG, n - g * TG);
+  const int4 tile = p.tiles[base + g * TG + in % width];
+  const int n0 = in / width * TC;
+  if (tile.z > HALF)
+    tile_product<UP, 4, 4, 2>(p, tile_lds, tile, n0);
+  else
+    tile_product<UP, 2, 4, 4>(p, tile_lds, tile, n0);
+}
+
+template <bool UP>
 hipError_t launch_tiles(const Pairs& p, int max_tiles, hipStream_t stream) {
-  // every XCD's share is rounded up
-  const int64_t n = ((int64_t)max_tiles * ((p.N + TC - 1) / TC) + 7) / 8 * 8;
+  // every XCD's two shares are rounded up
+  const int64_t n =
+      (((int64_t)max_tiles * ((p.N + TC - 1) / TC) + 7) / 8 + 1) * 8;
   if (n > 0x7fffffff || p.N % 8 || p.K % BK || p.K < 2 * BK ||
       (int64_t)p.N * p.K >= 1ll << 31)
     return hipErrorInvalidValue;

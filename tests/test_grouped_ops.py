@@ -357,3 +357,26 @@ def test_forms_agree_at_a_large_size():
     a = ops.experts(h, ids, wt, up, down, "relu_squared")
     b = ops.experts(h, ids, wt, up, down, "relu_squared", plain=True)
     close(a, f64(b), ("", torch.bfloat16), bf16=1e-2)
+
+
+@GPU
+@pytest.mark.parametrize("K,F", [(128, 192), (192, 128), (320, 576)])
+@pytest.mark.parametrize("act", ["relu_squared", "silu", "gelu_tanh"])
+def test_tiles_at_their_edges(K, F, act):
+    """Pairs of an expert around half and whole tiles, K of two steps and of
+    more, channels that end inside a tile; against the plain kernel."""
+    counts = [1, 128, 129, 0, 255, 256, 257, 384, 385, 512]
+    dev, E, T = "cuda:0", len(counts), sum(counts)
+    g = torch.Generator(device=dev).manual_seed(K + F)
+
+    def normal(*shape, std=1.0):
+        return torch.empty(shape, device=dev).normal_(
+            0, std, generator=g).bfloat16()
+    up, down = normal(E, F, K, std=K ** -0.5), normal(E, K, F, std=F ** -0.5)
+    h = normal(T, K)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    ids = ids[torch.randperm(T)].int().to(dev)[:, None].contiguous()
+    wt = torch.rand(T, 1, device=dev, generator=g) * 0.9 + 0.05
+    a = ops.experts(h, ids, wt, up, down, act)
+    b = ops.experts(h, ids, wt, up, down, act, plain=True)
+    close(a, f64(b), ("", torch.bfloat16), bf16=1e-2)
