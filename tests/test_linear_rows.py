@@ -59,7 +59,7 @@ def test_gated(name, rows, n, k):
     for act, fn in enumerate([lambda z: F.gelu(z, approximate="tanh"), F.silu,
                               lambda z: z.relu().square()]):
         y = _ext(name).gated_linear(x, w, act)
-        assert (y is None) == (rows > 128 or n not in (14400, 16384))
+        assert (y is None) == (rows > 192 or n not in (14400, 16384))
         if y is not None:
             _same(y, fn(g) * u, 8)
 
