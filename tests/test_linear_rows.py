@@ -64,6 +64,26 @@ def test_gated(name, rows, n, k):
             _same(y, fn(g) * u, 8)
 
 
+@pytest.mark.parametrize("rows", [2048, 4095, 4096, 4097, 4352, 4500, 8193])
+@pytest.mark.parametrize("n,k", [(4096, 96), (4090, 72), (16384, 64),
+                                 (300, 64)])
+def test_whole_rounds_apart(rows, n, k):
+    """Many rows in two calls, of which the second may have one row; rows that
+    lie apart; errors and other types as ever."""
+    ext = _ext("_hip_ops")
+    x, w = _draw(rows, k + 8, seed=rows)[:, 8:], _draw(n, k, seed=n,
+                                                       scale=k ** -0.5)
+    _same(ext.linear(x, w), x.double() @ w.double().t(), 8)
+    if n == 4096 and rows == 4500:
+        y = ext.linear(x.float(), w.float())
+        assert y.dtype == torch.float32
+        with pytest.raises(RuntimeError):
+            ext.linear(x, w[:, 1:])
+        a = x.detach().clone().requires_grad_()
+        ext.linear(a, w).float().sum().backward()
+        assert a.grad.shape == x.shape
+
+
 def test_rows_apart():
     """Slices of wider tensors, as the decay and gate projections take."""
     ext = _ext("_hip_layered")
