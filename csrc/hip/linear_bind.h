@@ -61,19 +61,22 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
 }
 
 // Rows of a product of many that make up whole rounds of tiles of 256 x 256
-// over the 256 compute units; 0 if all of them do, or none. The library often
+// over the 256 compute units; 0 if there are none or if the others nearly make
+// up the next ones (8 layers of the delta design, 7749 rows: 4096 and 15 more
+// tiles of 16, 31.7 ms in one call each, 31.95 in two). The library often
 // takes a kernel of half the rate where a round is nearly empty, so these rows
 // go in a call of their own and the others in a second one: 14336 -> 4096,
 // 8533 rows 658 us for 1074, 6540 rows 510 for 841; 4096 -> 6144, 8533 rows
-// 290 for 399; 4096 -> 28672, 8533 rows 1312 for 1444. Over 103 draws of 12
-// sizes and 1000 to 12000 rows 1.19 times as fast, 0.96 at the least (a short
-// K, and under 2048 rows, which are left alone).
+// 290 for 399; 4096 -> 28672, 8533 rows 1312 for 1444. Over draws of 15 sizes
+// and 2048 to 12000 rows 1.16 to 1.2 times as fast; where the others are many
+// and the one call had a good kernel up to 4 % slower (4096 -> 14336, 11456
+// rows: 16 %, the library's pick for the 3264 others being a poor one).
 inline int64_t whole_rounds(int64_t M, int64_t N) {
   const int64_t across = (N + 255) / 256;
   int64_t down = 256;                     // tiles of rows in whole rounds
   while (down > 1 && across * (down / 2) % 256 == 0) down /= 2;
-  if ((M + 255) / 256 % down == 0) return 0;
   const int64_t rows = M / (down * 256) * (down * 256);
+  if ((M - rows + 255) / 256 * 16 >= down * 15 || rows == M) return 0;
   return rows < 2048 ? 0 : rows;
 }
 
