@@ -406,18 +406,25 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
   for (int d = tid; d < KP; d += LT) wk.gl[d] = __expf(blocks(0, 4, d));
 }
 
-// grid (H, VP / 16, sequences); walk [n, 4] = first row, tokens, slot, first
-// chunk | (1 << 30 if the state starts at zero)
-template <int KT>
-__global__ __launch_bounds__(ST) void delta_chunk_scan_kernel(
+// grid (H, VP / (16 NC), sequences); walk [n, 4] = first row, tokens, slot,
+// first chunk | (1 << 30 if the state starts at zero). A workgroup has NC tiles
+// of 16 columns. S lies in LDS between the chunks, as operands; a wave keeps
+// the tiles of it that it brings up to date, takes 16 tokens of the products
+// with it, and asks for a chunk's operands of these during the chunk before.
+// The matrix instructions bound it (60 us of 94 for 32 chunks of 8 sequences,
+// 32 heads of 128 x 128; 111 with one tile, 125 with all of S in the registers
+// of every wave and loads under conditions).
+template <int KT, int NC>
+__global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     float* __restrict__ ws, float* __restrict__ state,  // [slots, H, K, V]
     const int32_t* __restrict__ walk, float* __restrict__ out,  // [rows, H V]
     int H, int K, int V, int VP) {
   constexpr int KP = KT * 16;
-  __shared__ float4v s_lds[KT][WAVE], u_lds[4][WAVE];
+  constexpr int MY = (KT + 3) / 4;    // tiles of 16 rows of S per wave
+  __shared__ float4v s_lds[NC][KT][WAVE], u_lds[NC][4][WAVE];
   const int h = blockIdx.x, lane = threadIdx.x % WAVE;
   const int wave = threadIdx.x / WAVE, col = lane % 16, g4 = 4 * (lane / 16);
-  const int c = blockIdx.y * 16 + col;
+  const int c0 = blockIdx.y * 16 * NC + col;
   const int4 m = ((const int4*)walk)[blockIdx.z];
   const int64_t row0 = m.x;
   const int n = m.y;
@@ -425,104 +432,145 @@ __global__ __launch_bounds__(ST) void delta_chunk_scan_kernel(
   const int64_t chunk0 = m.w & ((1 << 30) - 1);
   float* Sp = state + ((int64_t)m.z * H + h) * K * V;
 
-  float4v S[KT];      // every wave has all of its 16 columns
+  float4v S[NC][MY];
 #pragma unroll
-  for (int t = 0; t < KT; ++t)
+  for (int x = 0; x < NC; ++x)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int d = 16 * t + g4 + r;
-      S[t][r] = !fresh && d < K && c < V ? Sp[(int64_t)d * V + c] : 0.f;
+    for (int i = 0; i < MY; ++i) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = 16 * (wave + 4 * i) + g4 + r, c = c0 + 16 * x;
+        S[x][i][r] = !fresh && d < K && c < V ? Sp[(int64_t)d * V + c] : 0.f;
+      }
+      if (wave + 4 * i < KT) s_lds[x][wave + 4 * i][lane] = S[x][i];
     }
+  lds_barrier();
 
   // uniform bases, per-lane offsets that stay the same for every chunk
   const int tw = wave * B;            // this wave's 16 tokens
   const int64_t stride = (int64_t)H * work_size(KP, VP);
   const float* base = ws + (chunk0 * H + h) * work_size(KP, VP);
-  const unsigned at_w = wave * KT * 256 + lane * 4, at_g = tw + g4;
-  const unsigned at_u = (blockIdx.y * 4 + wave) * 256 + lane * 4;
-  const unsigned at_k = wave * 4 * 256 + lane * 4;
-  float4v w[KT], qe[KT], u;
-  auto fetch = [&](const float* p) {
+  const unsigned at_w = wave * KT * 256 + lane * 4;
+  unsigned at_u[NC];                  // past the last tile: that one's
+#pragma unroll
+  for (int x = 0; x < NC; ++x)
+    at_u[x] = (min((int)blockIdx.y * NC + x, VP / 16 - 1) * 4 + wave) * 256 +
+              lane * 4;
+  const unsigned at_p = wave * 4 * 256 + lane * 4;
+  // of 32 channels, the third and fourth wave have no tile of their own
+  const unsigned at_k = wave % KT * 4 * 256 + lane * 4;
+  const unsigned at_g = wave % KT * B + g4;
+  float4v w[KT], qe[KT], u[NC];
+  auto fetch = [&](const float* p) {  // in the order of their use
     const float* pw = p + C * VP;
     const float* pq = pw + C * KP;
+#pragma unroll
+    for (int x = 0; x < NC; ++x) u[x] = *(const float4v*)(p + at_u[x]);
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
       w[t] = *(const float4v*)(pw + (at_w + 256 * t));
       qe[t] = *(const float4v*)(pq + (at_w + 256 * t));
     }
-    u = *(const float4v*)(p + at_u);
+    __builtin_amdgcn_sched_barrier(0);
   };
   fetch(base);
   float* oc = out + (row0 * H + h) * V;
-  const unsigned at_o = (tw + g4) * (H * V) + c, orow = H * V;
-  for (int t0 = 0; t0 < n; t0 += C, base += stride, oc += C * orow) {
+  const unsigned at_o = (tw + g4) * (H * V) + c0, orow = H * V;
+  // No load of the loop is under a condition: the compiler could not count
+  // what is under way, and would wait for all of it.
+  for (int t0 = 0; t0 < n; t0 += C, oc += C * orow) {
     // operands of the state update and of P U, used after the first products
-    constexpr int MY = (KT + 3) / 4;
     float4v kt[MY][4], decay[MY], p[4];
     const float* pk = base + C * VP + 2 * C * KP;
     const float* pp = pk + C * KP;
     const float* pg = pp + C * C;
 #pragma unroll
-    for (int i = 0; i < MY; ++i)
-      if (wave + 4 * i < KT) {
+    for (int i = 0; i < MY; ++i) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x)
-          kt[i][x] = *(const float4v*)(pk + (at_k + i * 4096 + 256 * x));
-        decay[i] = *(const float4v*)(pg + (at_g + i * 4 * B));
-      }
+      for (int x = 0; x < 4; ++x)
+        kt[i][x] = *(const float4v*)(pk + (at_k + i * 4096 + 256 * x));
+      decay[i] = *(const float4v*)(pg + (at_g + i * 4 * B));
+    }
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
-      if (x <= wave) p[x] = *(const float4v*)(pp + (at_k + 256 * x));
-    float4v o = {0.f, 0.f, 0.f, 0.f};
+    for (int x = 0; x < 4; ++x)       // those past the wave's own are not used
+      p[x] = *(const float4v*)(pp + (at_p + 256 * x));
+    __builtin_amdgcn_sched_barrier(0);    // now, not where they are used
+    float4v o[NC];
+#pragma unroll
+    for (int x = 0; x < NC; ++x) o[x] = (float4v){0.f, 0.f, 0.f, 0.f};
+    // sums take turns: a product waits for the one before it on its sum
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      u = mfma4(w[t], S[t], u);
-      o = mfma4(qe[t], S[t], o);
+      float4v s[NC];
+#pragma unroll
+      for (int x = 0; x < NC; ++x) s[x] = s_lds[x][t][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int x = 0; x < NC; ++x) {
+          u[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][r], s[x][r], u[x],
+                                                      0, 0, 0);
+          o[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(qe[t][r], s[x][r], o[x],
+                                                      0, 0, 0);
+        }
     }
-    u_lds[wave][lane] = u;
-    // w, qe and u are free now: the next chunk's arrive during the rest
-    if (t0 + C < n) fetch(base + stride);
+#pragma unroll
+    for (int x = 0; x < NC; ++x) u_lds[x][wave][lane] = u[x];
+    // w, qe and u are free now: the next chunk's arrive during the rest (the
+    // last one's once more)
+    if (t0 + C < n) base += stride;
+    fetch(base);
     lds_barrier();
-    float4v us[4];
 #pragma unroll
-    for (int x = 0; x < 4; ++x) us[x] = u_lds[x][lane];
+    for (int x = 0; x < NC; ++x)
 #pragma unroll
-    for (int i = 0; i < MY; ++i) {
-      const int t = wave + 4 * i;
-      if (t < KT) {
-        // S[t] with a register index that depends on the wave would spill
-        float4v s = {0.f, 0.f, 0.f, 0.f};
+      for (int i = 0; i < MY; ++i) S[x][i] = S[x][i] * decay[i];
 #pragma unroll
-        for (int y = 0; y < KT; ++y)
-          if (y == t) s = S[y];
-        s = s * decay[i];
+    for (int y = 0; y < 4; ++y) {
+      float4v us[NC];
 #pragma unroll
-        for (int x = 0; x < 4; ++x) s = mfma4(kt[i][x], us[x], s);
-        s_lds[t][lane] = s;
+      for (int x = 0; x < NC; ++x) us[x] = u_lds[x][y][lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int x = 0; x < NC; ++x)
+#pragma unroll
+          for (int i = 0; i < MY; ++i)
+            S[x][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                kt[i][y][r], us[x][r], S[x][i], 0, 0, 0);
+      if (y <= wave) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int x = 0; x < NC; ++x)
+            o[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[y][r], us[x][r],
+                                                        o[x], 0, 0, 0);
       }
     }
 #pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      if (x <= wave) o = mfma4(p[x], us[x], o);
-    }
+    for (int x = 0; x < NC; ++x)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if (t0 + tw + g4 + r < n && c < V) oc[at_o + r * orow] = o[r];
-    }
+      for (int i = 0; i < MY; ++i)
+        if (wave + 4 * i < KT) s_lds[x][wave + 4 * i][lane] = S[x][i];
+#pragma unroll
+    for (int x = 0; x < NC; ++x)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (t0 + tw + g4 + r < n && c0 + 16 * x < V)
+          oc[at_o + r * orow + 16 * x] = o[x][r];
     lds_barrier();
-#pragma unroll
-    for (int t = 0; t < KT; ++t) S[t] = s_lds[t][lane];
   }
 
-  if (wave == 0) {
 #pragma unroll
-    for (int t = 0; t < KT; ++t)
+  for (int x = 0; x < NC; ++x)
+#pragma unroll
+    for (int i = 0; i < MY; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int d = 16 * t + g4 + r;
-        if (d < K && c < V) Sp[(int64_t)d * V + c] = S[t][r];
+        const int d = 16 * (wave + 4 * i) + g4 + r, c = c0 + 16 * x;
+        if (wave + 4 * i < KT && d < K && c < V)
+          Sp[(int64_t)d * V + c] = S[x][i][r];
       }
-  }
 }
 
 // out = o / rms(o) * w * sigmoid(gate) per head; LANES threads per (row,
@@ -583,7 +631,10 @@ hipError_t lds_delta_chunk(int f32, const float* q, const float* k,
   const int KP = padded_k(K), VP = (V + 15) / 16 * 16;
   const size_t lds =
       (2 * C * (KP + 4) + 10 * AB + C + LT / WAVE) * sizeof(float);
-  const dim3 g1(H, n_chunks), g2(H, VP / 16, n_seqs);
+  const dim3 g1(H, n_chunks);
+  const int tiles = VP / 16, pairs = (tiles + 1) / 2;
+  // two workgroups per compute unit at least, else one tile each
+  const bool two = (int64_t)H * pairs * n_seqs >= 512;
 #define LOCAL(T, KPV)                                                         \
   do {                                                                        \
     auto fn = delta_chunk_local_kernel<T, KPV>;                               \
@@ -598,8 +649,14 @@ hipError_t lds_delta_chunk(int f32, const float* q, const float* k,
 #define GO(KPV)                                                               \
   do {                                                                        \
     if (f32) LOCAL(float, KPV); else LOCAL(short, KPV);                       \
-    hipLaunchKernelGGL(delta_chunk_scan_kernel<KPV / 16>, g2, dim3(ST), 0,    \
-                       stream, ws, state, walk, out, H, K, V, VP);            \
+    if (two)                                                                  \
+      hipLaunchKernelGGL((delta_chunk_scan_kernel<KPV / 16, 2>),              \
+                         dim3(H, pairs, n_seqs), dim3(ST), 0, stream, ws,     \
+                         state, walk, out, H, K, V, VP);                      \
+    else                                                                      \
+      hipLaunchKernelGGL((delta_chunk_scan_kernel<KPV / 16, 1>),              \
+                         dim3(H, tiles, n_seqs), dim3(ST), 0, stream, ws,     \
+                         state, walk, out, H, K, V, VP);                      \
   } while (0)
   if (KP == 32) GO(32); else if (KP == 64) GO(64); else GO(128);
 #undef GO

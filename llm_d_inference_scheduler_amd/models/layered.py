@@ -60,27 +60,33 @@ class ChunkGroup:
 def chunk_groups(long: List[Portion], per_group: int,
                  device: torch.device) -> List[ChunkGroup]:
     """Cut long portions into chunks, at most `per_group` a group. A group
-    takes a stretch of every portion in turn (they run side by side); the
-    next group goes on from the stored states."""
-    total = sum(-(-p.n // CHUNK) for p in long)
+    takes a stretch of every portion (they run side by side), as even as the
+    portions allow; the next group goes on from the stored states. (A last
+    group of two chunks took 50 us a layer.)"""
+    rest = [-(-p.n // CHUNK) for p in long]
+    total = sum(rest)
     per_group = -(-total // -(-total // per_group))     # groups of like size
     groups = []
     at = [0] * len(long)
-    while any(a < p.n for a, p in zip(at, long)):
-        left = sum(a < p.n for a, p in zip(at, long))
+    while any(rest):
+        room, share = per_group, [0] * len(long)
+        while room and share != rest:
+            for i, r in enumerate(rest):
+                if room and share[i] < r:
+                    share[i] += 1
+                    room -= 1
         chunks, walk = [], []
-        for i, p in enumerate(long):
-            if at[i] == p.n or len(chunks) == per_group:
+        for i, (p, some) in enumerate(zip(long, share)):
+            if not some:
                 continue
-            share = max(1, (per_group - len(chunks)) // left)
-            left -= 1
-            n = min(p.n - at[i], share * CHUNK)
+            n = min(p.n - at[i], some * CHUNK)
             row = p.row0 + at[i]
             fresh = p.prior + at[i] == 0
             walk.append((row, n, p.slot, len(chunks) | fresh << 30))
             chunks.extend((row + a, min(CHUNK, n - a))
                           for a in range(0, n, CHUNK))
             at[i] += n
+            rest[i] -= some
         c = torch.tensor(chunks, dtype=torch.int32)
         w = torch.tensor(walk, dtype=torch.int32)
         groups.append(ChunkGroup(c.to(device), w.to(device), c, w))

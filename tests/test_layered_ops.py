@@ -246,6 +246,51 @@ class TestDelta:
         close(got[loud[64:].to(run[0])], ref[loud[64:]], run, f32=3e-3)
 
 
+@GPU
+@pytest.mark.parametrize("K,V,n", [(32, 40, 32), (64, 128, 16), (128, 16, 64),
+                                   (100, 72, 22)])
+@pytest.mark.parametrize("shift", DECAYS[:2])
+@pytest.mark.parametrize("run", RUNS[-1:])
+def test_chunks_of_many_sequences(run, K, V, n, shift):
+    """Enough sequences that a workgroup takes two tiles of columns of the
+    state, the last of which may not exist; lengths around a chunk."""
+    KH, H = 2, 8
+    seqs = [((63, 64, 65, 9, 130)[i % 5], i % 2, i) for i in range(n)]
+    if sum(s[0] for s in seqs) % 2:          # delta_case halves the rows
+        seqs[-1] = (seqs[-1][0] + 1,) + seqs[-1][1:]
+    d = delta_case(run, seqs, KH, H, K, V, shift, seed=70)
+    d["state"] = rnd(n, H, K, V, seed=79).to(run[0])
+    _, raw, states = delta_oracle(d, seqs, 1e-5)
+    row, long = 0, []
+    for i, (rows, prior, slot) in enumerate(seqs):
+        long.append(layered.Portion(i, row, rows, prior, [], slot))
+        row += rows
+    o = torch.zeros(row, H * V, device=run[0])
+    work = ops.delta_chunk_work(K, V, torch.device("cuda"))
+    g, = layered.chunk_groups(long, 1000, torch.device(run[0]))
+    ws = torch.full((work * H * len(g.chunks_host),), float("nan"),
+                    device=run[0])
+    ops.delta_chunk(d["q"], d["k"], d["v"], d["proj"], 5, d["decay"],
+                    d["bias"], d["neg_a"], d["state"], g, ws, o)
+    close(o.view(row, H, V), raw, ("", torch.float32), f32=3e-5)
+    for slot, S in states.items():
+        close(d["state"][slot], S, ("", torch.float32), f32=3e-5)
+
+
+def test_groups_are_full():
+    """As few groups as hold all chunks, whatever the portions' lengths."""
+    cpu = torch.device("cpu")
+    for lengths in ([750, 1250, 1000, 64, 1], [5000], [70] * 40, [1, 9000]):
+        long = [layered.Portion(i, 0, n, 0, [], i)
+                for i, n in enumerate(lengths)]
+        total = sum(-(-n // 64) for n in lengths)
+        for per in (1, 7, 33, 500):
+            groups = layered.chunk_groups(long, per, cpu)
+            assert len(groups) == -(-total // per)
+            assert sum(len(g.chunks_host) for g in groups) == total
+            assert all(len(g.chunks_host) <= per for g in groups)
+
+
 class TestRotary:
     @pytest.mark.parametrize("scaling", [
         None, {"factor": 4.0, "original": 64, "fast": 32.0, "slow": 1.0},
