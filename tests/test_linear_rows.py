@@ -132,10 +132,12 @@ def test_gradients_pass():
         assert ext.few_rows(x, w)
 
 
-def test_capture_and_replay():
+@pytest.mark.parametrize("rows", [12, 60, 200])
+def test_capture_and_replay(rows):
     """Partial sums are written anew by every replay."""
     ext = _ext("_hip_ops")
-    x, w = _draw(12, 2048, seed=10), _draw(256, 2048, seed=11, scale=1 / 45)
+    x, w = _draw(rows, 4096, seed=10), _draw(4096, 4096, seed=11, scale=1 / 64)
+    assert ext.few_rows(x, w)
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         ext.linear(x, w)
@@ -144,7 +146,7 @@ def test_capture_and_replay():
     with torch.cuda.graph(graph):
         y = ext.linear(x, w)
     for i in range(3):
-        x.copy_(_draw(12, 2048, seed=20 + i))
+        x.copy_(_draw(rows, 4096, seed=20 + i))
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ext.linear(x, w))
