@@ -3,8 +3,10 @@
 // library.
 #pragma once
 #include <torch/extension.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 
 #include <hip/hip_runtime.h>
@@ -28,8 +30,10 @@ inline bool rows_of_16_bytes(const Tensor& t) {
          t.stride(0) >= t.size(1) && (uintptr_t)t.data_ptr() % 16 == 0;
 }
 
-// bf16 matrices on one GPU that autograd, a trace or a functional transform
-// does not follow, of matching sizes
+// bf16 matrices on one GPU, of matching sizes, whose product is what this
+// header computes and nothing else: autograd, a trace, a dispatch mode or a
+// functional transform does not follow it, autocast gives it no other type, and
+// both have memory (a tensor known to be zero has none)
 inline bool plain_matrices(const Tensor& x, const Tensor& w) {
   if (x.dim() != 2 || w.dim() != 2 || !x.is_cuda() ||
       x.device() != w.device() || x.scalar_type() != at::kBFloat16 ||
@@ -37,9 +41,13 @@ inline bool plain_matrices(const Tensor& x, const Tensor& w) {
     return false;
   if (at::GradMode::is_enabled() && (x.requires_grad() || w.requires_grad()))
     return false;
+  if (c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+      (at::autocast::is_autocast_enabled(at::kCUDA) &&
+       at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16))
+    return false;
   for (const Tensor* t : {&x, &w})
     if (!t->has_storage() || t->layout() != at::kStrided || t->is_neg() ||
-        t->_fw_grad(0).defined() ||
+        t->_is_zerotensor() || t->_fw_grad(0).defined() ||
         t->key_set().has(c10::DispatchKey::Python))
       return false;
   return !torch::jit::tracer::isTracing();

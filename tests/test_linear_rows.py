@@ -132,6 +132,49 @@ def test_gradients_pass():
         assert ext.few_rows(x, w)
 
 
+@pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("rows", [1, 20, 4500])
+def test_calls_that_something_follows(name, rows):
+    """A dispatch mode sees the product, a graph traced through one computes
+    it anew, and autocast gives it its type."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+    ext, seen = _ext(name), []
+
+    class Record(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func.overloadpacket)
+            return func(*args, **(kwargs or {}))
+    n, k = (4096, 64) if rows > 256 else (28672, 256)
+    x, w = _draw(rows, k, seed=1), _draw(n, k, seed=2, scale=k ** -0.5)
+    want = x.double() @ w.double().t()
+    with Record():
+        y = ext.linear(x, w)
+        parts = ext.linear_parts(x, w)
+        assert ext.linear32(x, w) is None
+        assert ext.gated_linear(x, w, 1) is None
+    assert seen.count(torch.ops.aten.mm) == 2
+    _same(y, want, 8)
+    _same(parts, want, 8)
+    traced = make_fx(lambda a: ext.linear(a, w))(_draw(rows, k, seed=3))
+    _same(traced(x), want, 8)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ext.linear(x, w).dtype == torch.float16
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        _same(ext.linear(x, w), want, 8)
+
+
+def test_zeros_without_memory():
+    ext = _ext("_hip_ops")
+    w = _draw(64, 256, seed=4)
+    for rows in (20, 4500):
+        x = torch._efficientzerotensor((rows, 256), dtype=torch.bfloat16,
+                                       device="cuda")
+        assert not ext.few_rows(x, w)
+        y = ext.linear(x, w)
+        assert y.shape == (rows, 64) and not y.any()
+
+
 @pytest.mark.parametrize("rows", [12, 60, 200])
 def test_capture_and_replay(rows):
     """Partial sums are written anew by every replay."""
