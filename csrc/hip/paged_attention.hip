@@ -113,7 +113,10 @@ __global__ __launch_bounds__(NW * WAVE, 3) void paged_attention_kernel(
     float* __restrict__ part_ml,  // [B, KVH, NP, QPG, 2] (SPLIT), m in log2
     int kvh, int qpg, int bs, int max_blocks, int part_tokens, float scale) {
   typedef Cache<CT> C;
-  const int b = blockIdx.x;
+  // Workgroups go round the XCDs in turn: with an even number of sequences all
+  // parts of one would run on the same few, so sequences take turns by part.
+  const int turn = SPLIT && gridDim.x % 2 == 0 ? blockIdx.z : 0;
+  const int b = (blockIdx.x + turn) % gridDim.x;
   const int kh = blockIdx.y;
   const int part = SPLIT ? blockIdx.z : 0;
   const int np = SPLIT ? gridDim.z : 1;

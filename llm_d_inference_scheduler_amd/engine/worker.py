@@ -778,11 +778,11 @@ class EngineWorker:
             return self._nothing_to_decode(finals)
         rows_t, ids, pos, slot, bt_rows, new_len = self._decode_rows(
             [r.request_id for r in active])
+        lens = [self.mgr.seq_lens[r.request_id] for r in active]
         batch = ForwardBatch(
             input_ids=ids, positions=pos, slot_mapping=slot, is_decode=True,
-            block_tables=bt_rows, seq_lens=new_len,
-            max_seq_len=max(self.mgr.seq_lens[r.request_id]
-                            for r in active))
+            block_tables=bt_rows, seq_lens=new_len, max_seq_len=max(lens),
+            mean_seq_len=sum(lens) / len(lens))
         logits = self.model.forward(batch, self.pool.model_view())
         return self._emit_decode(active, rows_t, logits) + finals
 

@@ -38,6 +38,7 @@ class ForwardBatch:
     block_tables: Optional[torch.Tensor] = None   # [B, max_blocks] int32
     seq_lens: Optional[torch.Tensor] = None       # [B] int32 (incl. new token)
     max_seq_len: Optional[int] = None             # host-known max (no sync)
+    mean_seq_len: Optional[float] = None          # and mean, if known
     # prefill-only:
     seq_starts: Optional[List[int]] = None        # len B+1 offsets into T
     ctx_lens: Optional[List[int]] = None          # [B] total ctx after chunk
@@ -152,7 +153,8 @@ class LlamaRunner:
                 attn = ops.paged_attention(q, k_cache, v_cache,
                                            batch.block_tables, batch.seq_lens,
                                            self.scale,
-                                           max_seq_len=batch.max_seq_len)
+                                           max_seq_len=batch.max_seq_len,
+                                           mean_seq_len=batch.mean_seq_len)
             else:
                 attn = self._prefill_attention(batch, q, k_cache, v_cache)
             o = ops.linear_parts(attn.view(T, c.q_size), layer["wo"].t())

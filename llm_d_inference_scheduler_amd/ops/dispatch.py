@@ -5,6 +5,7 @@ CUDA-device tensor with `_hip_ops` missing raises immediately rather than
 silently falling back to eager torch. CPU tensors (tests, tiny gloo runs)
 use ops.ref.
 """
+import math
 from typing import Optional, Tuple
 
 import torch
@@ -122,16 +123,33 @@ def reshape_and_cache(k_new: torch.Tensor, v_new: torch.Tensor,
     ref.reshape_and_cache(k_new, v_new, k_cache, v_cache, slots)
 
 
-def decode_parts(groups: int, max_len: int) -> Tuple[int, int]:
+def decode_parts(groups: int, max_len: int,
+                 mean_len: Optional[float] = None) -> Tuple[int, int]:
     """-> (parts, tokens per part) of the decode attention of `groups`
-    (sequence, key head) pairs. A workgroup of 8 waves takes 256 tokens a
-    step, and about 512 of them fill the chip: parts make up for fewer groups
-    as long as each has a step of its own. From 200 groups on, the partial
-    sums and the second launch cost more than the idle compute units (240
-    groups of 1100 tokens: 27 us in one part, 38 in two; 136 groups of 6800
-    tokens, 8-bit: 108 us in one part, 62 in four)."""
-    parts = 1 if groups >= 200 else \
-        max(1, min(64, -(-512 // max(1, groups)), -(-max_len // 256)))
+    (sequence, key head) pairs of up to max_len tokens, and of mean_len on
+    average (None: all about as long). A workgroup of 8 waves takes 256 tokens
+    a step, and about 512 of them fill the chip: parts make up for fewer groups
+    as long as each has a step of its own. From 200 groups of like length on,
+    the partial sums and the second launch cost more than the idle compute
+    units (240 groups of 1100 tokens: 27 us in one part, 38 in two; 136 groups
+    of 6800 tokens, 8-bit: 108 us in one part, 62 in four).
+
+    One long sequence among short ones would hold the batch up: 14 us per 1000
+    tokens that a workgroup walks alone. It is cut so that none walks more than
+    one and a half shares of a compute unit; up to 1000 tokens past these, or
+    for less than twice the parts, the second launch costs as much. A sequence
+    of 8000 among 24 of 100: 108 us in one part, 24 in 17; among 255 of 300: 258
+    and 140 in 3; of 3000 among 16 of 300: 21 in 4, 17 in 8; of 1500 among 24 of
+    1000: 27 in one, 34 in two."""
+    parts = 1 if groups >= 200 else -(-512 // max(1, groups))
+    if mean_len is not None:
+        # tokens that one workgroup may walk while each compute unit takes one
+        # and a half shares of the whole
+        walk = max(256., 1.5 * mean_len * groups / 256)
+        ragged = math.ceil(max_len / walk)
+        if max_len - walk >= 1000 and ragged >= 2 * parts:
+            parts = ragged
+    parts = max(1, min(64, parts, -(-max_len // 256)))
     part = -(-(-(-max_len // parts)) // 32) * 32
     return -(-max_len // part), part
 
@@ -139,7 +157,8 @@ def decode_parts(groups: int, max_len: int) -> Tuple[int, int]:
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
                     v_cache: torch.Tensor, block_tables: torch.Tensor,
                     seq_lens: torch.Tensor, scale: float,
-                    max_seq_len: Optional[int] = None) -> torch.Tensor:
+                    max_seq_len: Optional[int] = None,
+                    mean_seq_len: Optional[float] = None) -> torch.Tensor:
     if _use_hip(q):
         bt = block_tables.to(torch.int32)
         sl = seq_lens.to(torch.int32)
@@ -149,7 +168,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # sequences of 120 tokens: 19 us with 8 waves, 15 with 4)
             waves = 4 if max_seq_len <= 256 else 8
             parts, part = decode_parts(q.shape[0] * k_cache.shape[1],
-                                       max_seq_len)
+                                       max_seq_len, mean_seq_len)
             if parts > 1:
                 return _ext.paged_attention_split(q, k_cache, v_cache, bt,
                                                   sl, parts, part, scale,

@@ -17,6 +17,26 @@ def test_parts_cover_the_context(groups, max_len):
     assert (parts - 1) * part < max_len <= parts * part
 
 
+@pytest.mark.parametrize("batch", [2, 5, 17, 24, 25, 32, 64, 127, 256])
+@pytest.mark.parametrize("short", [1, 100, 300, 1000])
+@pytest.mark.parametrize("long", [1500, 3000, 8000, 131072])
+def test_a_long_sequence_among_short_ones(batch, short, long):
+    """No workgroup walks 2000 tokens more than a compute unit's share, and
+    batches of like lengths are cut as without their mean."""
+    lens = [short] * (batch - 1) + [long]
+    mean, groups = sum(lens) / batch, batch * 8
+    parts, part = dispatch.decode_parts(groups, long, mean)
+    assert 1 <= parts <= 64 and part % 32 == 0
+    assert (parts - 1) * part < long <= parts * part
+    even = dispatch.decode_parts(groups, long)
+    assert parts >= even[0]
+    share = sum(lens) * 8 / 256
+    assert part <= 1.5 * share + 2000 or parts == 64 or parts < 2 * even[0]
+    for like in (short, min(long, 8000)):
+        assert dispatch.decode_parts(groups, int(like * 1.25), like) == \
+            dispatch.decode_parts(groups, int(like * 1.25))
+
+
 def _case(lens, qpg, bs, fp8):
     g = torch.Generator().manual_seed(sum(lens) + qpg + bs)
     pages = [-(-n // bs) for n in lens]
@@ -64,6 +84,21 @@ def test_edges(qpg, bs, fp8, waves):
     for parts, part in [(3, 256), (64, 11), (8, 96)]:
         _close(ext.paged_attention_split(*args, parts, part, D ** -0.5,
                                          waves=waves), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("batch", [1, 2, 3, 8, 24, 25, 104])
+def test_lengths_far_apart(batch, fp8):
+    """Every sequence has its parts, whichever order the grid takes them in."""
+    lens = [1 + 37 * i % 90 for i in range(batch - 1)] + [2900]
+    args, want = _case(lens, 4, 16, fp8)
+    mean = sum(lens) / batch
+    _close(dispatch.paged_attention(*args, D ** -0.5, 2900, mean), want)
+    assert batch == 1 or dispatch.decode_parts(batch * KVH, 2900, mean)[0] > 1
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    for parts, part in [(2, 1472), (12, 256), (64, 48)]:
+        _close(ext.paged_attention_split(*args, parts, part, D ** -0.5), want)
 
 
 @pytest.mark.gpu
