@@ -14,18 +14,22 @@
 //          last read of buffer (n-1)%3 from its rewrite for tile n+2.
 //   keys   32 query rows; every wave takes each fourth tile of keys through a
 //          2-deep ring of its own, without barriers, and the waves' results
-//          meet in LDS at the end. Four times the workgroups, a quarter of the
-//          serial chain: for calls whose rows leave the chip idle. These have
-//          matrix cores to spare, so that probabilities keep 17 bits: a
-//          prompt's last tokens come out as decoding them would.
+//          meet in LDS at the end. Four times the workgroups, half the serial
+//          chain, one workgroup per compute unit (132 KB of LDS).
+// Where the workgroups of the first shape leave compute units idle, one of the
+// two takes the call by its work (see prefill_shape in ops/dispatch.py), and
+// probabilities keep 17 bits in both: the matrix cores have the time, and a
+// prompt's last tokens come out as decoding them would.
 // Key heads run fastest over the grid: with 8 of them each XCD's L2 holds the
 // keys and values of one. Tiles run from the last to the first: under the
 // causal mask the last of a sequence has the most keys.
 //
-// Measured (groups of 4, 8 key heads; before: masks, packing and rescaling of
-// every tile on the vector units): one prompt of 7900 tokens 650 us, 785
-// TFLOP/s (before 1170); 8 of 1000 135 us (265); 150 tokens behind 1000, by
-// keys: 22 us, by rows 42 (59).
+// Measured (groups of 4, 8 key heads, alone; before: masks, packing and
+// rescaling of every tile on the vector units): one prompt of 7900 tokens 650
+// us, 785 TFLOP/s (before 1170); 8 of 1000 135 us (265). By keys / by rows with
+// 17 bits (with 8): 150 tokens behind 1000 24 / 48 us (44; before 61); 500
+// behind 1000 52 / 66 (57; 79); 600 behind 4000 195 / 175 (159; 235); 12
+// prompts of 20 13 / 7 (6; 7).
 //
 // fp8 KV cannot ride glds (raw byte copy, no conversion point), so the fp8
 // path keeps the convert-on-stage kernel in flash_prefill.hip; the launcher in
@@ -55,8 +59,8 @@ constexpr int lds_bytes(bool keys) {
   return BT_CAP * 4 + 2 * TILE_BYTES * (keys ? RING_KEYS * NW : RING_ROWS);
 }
 
-// SHIFT: block size 1 << shift; else any
-template <int QPG, bool KEYS, bool SHIFT>
+// FINE: see attend32. SHIFT: block size 1 << shift; else any
+template <int QPG, bool KEYS, bool FINE, bool SHIFT>
 __global__ __launch_bounds__(NW * WAVE, KEYS ? 1 : 2)
 void flash_prefill_glds_kernel(
     const short* __restrict__ q, const short* __restrict__ k_cache,
@@ -160,7 +164,7 @@ void flash_prefill_glds_kernel(
     const int tile0 = n * KVBLK;
     const char* kb = ring + buf * 2 * TILE_BYTES;
     const char* vb = kb + TILE_BYTES;
-    attend32<D / 16, D / 32, KEYS>(
+    attend32<D / 16, D / 32, FINE>(
         [&](int kk) {
           return *(const bf16x8*)(kb + k_row +
                                   ((kk * 32 + hi * 16) ^ k_swz));
@@ -251,12 +255,12 @@ void flash_prefill_glds_kernel(
   }
 }
 
-template <int QPG, bool KEYS, bool SHIFT>
+template <int QPG, bool KEYS, bool FINE, bool SHIFT>
 hipError_t go(const void* q, const void* k_cache, const void* v_cache,
               const int32_t* block_tables, const int32_t* seq_meta,
               const int32_t* tiles, void* out, int n_tiles, int kvh, int bs,
               int shift, int max_blocks, float scale, hipStream_t stream) {
-  auto fn = flash_prefill_glds_kernel<QPG, KEYS, SHIFT>;
+  auto fn = flash_prefill_glds_kernel<QPG, KEYS, FINE, SHIFT>;
   hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
       lds_bytes(KEYS));
@@ -274,34 +278,45 @@ hipError_t go(const void* q, const void* k_cache, const void* v_cache,
 
 extern "C" {
 
-// `keys`: the waves share query rows and split the keys (0, 1; below 0: by the
-// number of workgroups). Fewer than one per compute unit with 128 rows each
-// leave the chip idle.
+// shape: 0 by rows, 1 by keys, 2 by rows with probabilities of 17 bits; below
+// 0, for callers that do not know the lengths: rows if these fill the chip,
+// else keys in one round of workgroups, or in two where prompts are long enough
+// to make up for the second (300 tokens behind 300 23 us by keys, 28 by rows; 4
+// x 100 13 and 10).
 hipError_t lds_flash_prefill_glds(
     const void* q, const void* k_cache, const void* v_cache,
     const int32_t* block_tables, const int32_t* seq_meta,
     const int32_t* tiles, void* out, int n_tiles, int n_q_heads, int kvh,
-    int bs, int head_dim, int max_blocks, float scale, int keys,
-    hipStream_t stream) {
+    int bs, int head_dim, int max_blocks, float scale, int shape, int n_tokens,
+    int n_seqs, hipStream_t stream) {
   if (n_tiles == 0) return hipSuccess;
   if (head_dim != D || max_blocks > BT_CAP || bs < 1 ||
       (int64_t)n_tiles * kvh * NW > 0x7fffffff)
     return hipErrorInvalidValue;
   const int qpg = n_q_heads / kvh;
-  const bool split = keys < 0 ? (int64_t)n_tiles * kvh < 256 : keys != 0;
+  const int64_t groups = (int64_t)n_tiles * kvh;
+  if (shape < 0)
+    shape = groups >= 256  ? 0
+            : groups <= 64 ? 1
+            : groups <= 128 && n_tokens / 256 >= n_seqs ? 1
+                                                        : 2;
   int shift = 0;
   while (1 << shift < bs && shift < 20) ++shift;
   const bool pow2 = 1 << shift == bs;
-#define GO(QPG, KEYS, SHIFT)                                                 \
-  return go<QPG, KEYS, SHIFT>(q, k_cache, v_cache, block_tables, seq_meta,   \
+#define GO(QPG, KEYS, FINE, SHIFT)                                           \
+  return go<QPG, KEYS, FINE, SHIFT>(q, k_cache, v_cache, block_tables, seq_meta,   \
                               tiles, out, n_tiles, kvh, bs, shift,           \
                               max_blocks, scale, stream)
 #define GO_Q(QPG)                                                            \
   do {                                                                       \
-    if (split) {                                                             \
-      if (pow2) GO(QPG, true, true); else GO(QPG, true, false);              \
+    if (shape == 1) {                                                        \
+      if (pow2) GO(QPG, true, true, true); else GO(QPG, true, true, false);  \
+    } else if (shape == 2) {                                                 \
+      if (pow2) GO(QPG, false, true, true);                                  \
+      else GO(QPG, false, true, false);                                      \
     } else {                                                                 \
-      if (pow2) GO(QPG, false, true); else GO(QPG, false, false);            \
+      if (pow2) GO(QPG, false, false, true);                                 \
+      else GO(QPG, false, false, false);                                     \
     }                                                                        \
   } while (0)
   switch (qpg) {

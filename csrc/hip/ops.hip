@@ -56,7 +56,8 @@ hipError_t lds_flash_prefill(const void*, const void*, const void*,
 hipError_t lds_flash_prefill_glds(const void*, const void*, const void*,
                                   const int32_t*, const int32_t*,
                                   const int32_t*, void*, int, int, int, int,
-                                  int, int, float, int, hipStream_t);
+                                  int, int, float, int, int, int,
+                                  hipStream_t);
 }
 
 namespace {
@@ -425,7 +426,7 @@ torch::Tensor flash_prefill(torch::Tensor q, torch::Tensor k_cache,
         block_tables.data_ptr<int32_t>(), seq_meta.data_ptr<int32_t>(),
         tiles.data_ptr<int32_t>(), out.data_ptr(), (int)tiles.size(0), qh,
         kvh, bs, d, (int)block_tables.size(1), (float)scale, (int)keys,
-        cur_stream()));
+        (int)q.size(0), (int)seq_meta.size(0), cur_stream()));
     return out;
   }
   CHECK_HIP(lds_flash_prefill(

@@ -134,6 +134,13 @@ class LlamaRunner:
             hidden[batch.embed_rows] = batch.embed_values.to(hidden.dtype)
         residual = None
         pos32 = batch.positions.to(torch.int32)
+        shape = -1
+        if batch.prefill_tiles is not None and batch.seq_starts and \
+                batch.ctx_lens:
+            shape = ops.prefill_shape(
+                [e - s for s, e in zip(batch.seq_starts,
+                                       batch.seq_starts[1:])],
+                batch.ctx_lens, c.num_heads // c.num_kv_heads, c.num_kv_heads)
         for li, layer in enumerate(self.layers):
             if residual is None:
                 residual = hidden
@@ -156,7 +163,8 @@ class LlamaRunner:
                                            max_seq_len=batch.max_seq_len,
                                            mean_seq_len=batch.mean_seq_len)
             else:
-                attn = self._prefill_attention(batch, q, k_cache, v_cache)
+                attn = self._prefill_attention(batch, q, k_cache, v_cache,
+                                               shape)
             o = ops.linear_parts(attn.view(T, c.q_size), layer["wo"].t())
             normed2 = ops.rmsnorm(o, layer["post_norm"], c.rms_eps,
                                   residual=residual)
@@ -172,8 +180,8 @@ class LlamaRunner:
         return ops.linear(sel, self.lm_head)
 
     def _prefill_attention(self, batch: ForwardBatch, q: torch.Tensor,
-                           k_cache: torch.Tensor,
-                           v_cache: torch.Tensor) -> torch.Tensor:
+                           k_cache: torch.Tensor, v_cache: torch.Tensor,
+                           shape: int = -1) -> torch.Tensor:
         """Causal varlen attention per sequence. GPU: fused MFMA flash
         kernel (flash_prefill.hip) — S never materialized. CPU fallback:
         composed chunked torch attention over pool-gathered KV."""
@@ -183,7 +191,7 @@ class LlamaRunner:
                 and c.num_heads // c.num_kv_heads in (1, 2, 4, 8)):
             return ops.flash_prefill(
                 q, k_cache, v_cache, batch.prefill_bt, batch.prefill_meta,
-                batch.prefill_tiles, self.scale)
+                batch.prefill_tiles, self.scale, shape)
         qpg = c.num_heads // c.num_kv_heads
         out = torch.empty_like(q)
         starts = batch.seq_starts

@@ -6,7 +6,7 @@ silently falling back to eager torch. CPU tensors (tests, tiny gloo runs)
 use ops.ref.
 """
 import math
-from typing import Optional, Tuple
+from typing import List, Optional, Tuple
 
 import torch
 
@@ -179,14 +179,38 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
                                scale)
 
 
+def prefill_shape(news: List[int], ctxs: List[int], group: int,
+                  kv_heads: int) -> int:
+    """Shape of the prefill attention's workgroups (flash_prefill_glds.hip) for
+    prompts of `news` tokens that end contexts of `ctxs`: 0 by rows, 1 by keys,
+    2 by rows with probabilities of 17 bits. From 256 workgroups by rows on the
+    chip is full (1000 tokens behind 1000: 75 us by rows, 109 by keys). Below,
+    the two with 17 bits are weighed in us, as measured: a workgroup by rows
+    takes 6 + 0.042 per key, one by keys 4.2 + 0.0167, one per compute unit,
+    those with the most keys first. One round of these is always faster."""
+    rows = sum(-(-n * group // 128) for n in news) * kv_heads
+    if rows >= 256:
+        return 0
+    some = [-(-n * group // 32) * kv_heads for n in news]
+    if sum(some) <= 256:
+        return 1
+    work = sum(k * (4.2 + 0.0167 * (c - n / 2))
+               for k, n, c in zip(some, news, ctxs)) / 256
+    least = 4.2 + 0.0167 * min(c - n for n, c in zip(news, ctxs))
+    most = max(ctxs)
+    keys = 3 + max(4.2 + 0.0167 * most, work + 0.6 * least)
+    return 1 if keys <= 6 + 0.042 * most else 2
+
+
 def flash_prefill(q: torch.Tensor, k_cache: torch.Tensor,
                   v_cache: torch.Tensor, block_tables: torch.Tensor,
                   seq_meta: torch.Tensor, tiles: torch.Tensor,
-                  scale: float) -> torch.Tensor:
+                  scale: float, shape: int = -1) -> torch.Tensor:
     """Fused MFMA causal varlen prefill attention (GPU-only; callers fall
-    back to the composed reference path when unsupported)."""
+    back to the composed reference path when unsupported). shape: of its
+    workgroups, from prefill_shape; below 0 by their number alone."""
     return hip_ops().flash_prefill(q, k_cache, v_cache, block_tables,
-                                   seq_meta, tiles, scale)
+                                   seq_meta, tiles, scale, shape)
 
 
 def move_blocks(pool: torch.Tensor, staging: torch.Tensor,

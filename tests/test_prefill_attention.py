@@ -52,6 +52,12 @@ def _close(got, want):
                                atol=2 ** -7)
 
 
+def _as_decoded(got, want):
+    # results rounded to bf16 and probabilities of 17 bits: half a step of
+    # bf16, and 2^-17 over values of size 1
+    torch.testing.assert_close(got.double(), want, rtol=2 ** -8, atol=1e-4)
+
+
 SEQS = [[(1, 0)], [(1, 700), (31, 0), (32, 1), (33, 31)],
         [(127, 65), (129, 0), (5, 1023)], [(260, 0), (64, 64), (95, 33)]]
 
@@ -59,7 +65,7 @@ SEQS = [[(1, 0)], [(1, 700), (31, 0), (32, 1), (33, 31)],
 @pytest.mark.parametrize("seqs", SEQS)
 @pytest.mark.parametrize("qpg,kvh", [(1, 3), (2, 8), (4, 2), (8, 1)])
 @pytest.mark.parametrize("bs", [16, 5])
-@pytest.mark.parametrize("keys", [0, 1, -1])
+@pytest.mark.parametrize("keys", [0, 1, 2, -1])
 def test_pages_in_bf16(seqs, qpg, kvh, bs, keys):
     from llm_d_inference_scheduler_amd import _hip_ops as ext
     args, want = _case(seqs, qpg, kvh, bs, False, D ** -0.5)
@@ -76,7 +82,7 @@ def test_pages_in_fp8(seqs, qpg, kvh, bs):
 
 
 @pytest.mark.parametrize("fp8", [False, True])
-@pytest.mark.parametrize("keys", [0, 1])
+@pytest.mark.parametrize("keys", [0, 1, 2])
 @pytest.mark.parametrize("scale", [-0.1, 0.0, 2.0])
 def test_scales(fp8, keys, scale):
     """A negative scale turns the order of the scores round, a large one
@@ -93,3 +99,21 @@ def test_long_tables_stage_through_registers():
     wide = torch.zeros(2, 1025, dtype=torch.int32, device="cuda")
     wide[:, :args[3].shape[1]] = args[3]
     _close(ext.flash_prefill(*args[:3], wide, *args[4:]), want)
+
+
+@pytest.mark.parametrize("seqs,qpg,kvh", [
+    ([(300, 0)], 4, 8), ([(400, 300)], 4, 8), ([(100, 40)] * 4, 4, 8),
+    ([(20, 300)] * 12, 4, 8), ([(250, 0)], 8, 8), ([(900, 0)], 4, 8),
+    ([(500, 0), (100, 600)], 4, 8), ([(1020, 0)], 1, 16)])
+def test_workgroups_fewer_than_compute_units(seqs, qpg, kvh):
+    """64 to 255 workgroups by rows: both shapes, and the one that is taken,
+    are as exact as decoding."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    from llm_d_inference_scheduler_amd import ops
+    args, want = _case(seqs, qpg, kvh, 16, False, D ** -0.5)
+    assert 64 < args[5].shape[0] * kvh < 256
+    shape = ops.prefill_shape([n for n, _ in seqs], [n + p for n, p in seqs],
+                              qpg, kvh)
+    assert shape in (1, 2)
+    for keys in (1, 2, shape, -1):
+        _as_decoded(ext.flash_prefill(*args, keys=keys), want)
