@@ -68,24 +68,32 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
          rows_of_16_bytes(x) && rows_of_16_bytes(w);
 }
 
-// Rows of a product of many that make up whole rounds of tiles of 256 x 256
-// over the 256 compute units; 0 if there are none or if the others nearly make
-// up the next ones (8 layers of the delta design, 7749 rows: 4096 and 15 more
-// tiles of 16, 31.7 ms in one call each, 31.95 in two). The library often
-// takes a kernel of half the rate where a round is nearly empty, so these rows
-// go in a call of their own and the others in a second one: 14336 -> 4096,
-// 8533 rows 658 us for 1074, 6540 rows 510 for 841; 4096 -> 6144, 8533 rows
-// 290 for 399; 4096 -> 28672, 8533 rows 1312 for 1444. Over draws of 15 sizes
-// and 2048 to 12000 rows 1.16 to 1.2 times as fast; where the others are many
-// and the one call had a good kernel up to 4 % slower (4096 -> 14336, 11456
-// rows: 16 %, the library's pick for the 3264 others being a poor one).
-inline int64_t whole_rounds(int64_t M, int64_t N) {
+// Rows of a product of many that go in a call of their own: those that make up
+// whole rounds of tiles of 256 x 256 over the 256 compute units. The library
+// often takes a kernel of half the rate where the rest is little (14336 ->
+// 4096: 8533 rows 1074 us in one call, 658 in two; 6540 rows 841 and 510; 4096
+// -> 28672: 8533 rows 1444 and 1312). 0, one call, where
+//   - the rest is two rounds of tiles or more: the second call is as likely as
+//     the one to get the poor kernel (5120 -> 10240, 12852 rows: 869 us in one
+//     call, 1065 in two; 4096 -> 14336, 11518 rows: 878 and 1039);
+//   - it ends in a round that is full but for 1/16: nothing to gain (4096 ->
+//     12576, 7749 rows: 31.7 ms a pass of 8 layers, 31.95 in two calls each);
+//   - it is more than half a round beside a single whole one and K is short:
+//     the second call costs what the round would (2048 -> 4096, 6266 rows: 88
+//     us and 95).
+// Over 1519 draws of 32 sizes and 2048 to 24000 rows: 1.12 times as fast as in
+// one call, 0.94 at the least (2048 -> 6144, 9515 rows), where calls of one
+// kind differ by 0.03.
+inline int64_t whole_rounds(int64_t M, int64_t N, int64_t K) {
   const int64_t across = (N + 255) / 256;
   int64_t down = 256;                     // tiles of rows in whole rounds
   while (down > 1 && across * (down / 2) % 256 == 0) down /= 2;
   const int64_t rows = M / (down * 256) * (down * 256);
-  if ((M - rows + 255) / 256 * 16 >= down * 15 || rows == M) return 0;
-  return rows < 2048 ? 0 : rows;
+  const int64_t rest = (M - rows + 255) / 256 * across, last = rest % 256;
+  if (rows < 2048 || rest == 0 || rest >= 512) return 0;
+  if (rest <= 128) return rows;
+  const bool worth = K >= 4096 || rows / 256 * across >= 512;
+  return worth && last > 0 && last <= 240 ? rows : 0;
 }
 
 inline void check(hipError_t e) {
@@ -118,7 +126,7 @@ inline Tensor linear_rows(const Tensor& x, const Tensor& w, bool f32) {
 inline Tensor linear(const Tensor& x, const Tensor& w) {
   if (few_rows(x, w, PLAIN)) return linear_rows(x, w, false);
   int64_t whole = 0;
-  if (plain_matrices(x, w)) whole = whole_rounds(x.size(0), w.size(0));
+  if (plain_matrices(x, w)) whole = whole_rounds(x.size(0), w.size(0), x.size(1));
   if (whole == 0) return at::matmul(x, w.t());
   Tensor y = torch::empty({x.size(0), w.size(0)}, x.options());
   const int64_t left = x.size(0) - whole;
@@ -195,6 +203,8 @@ inline void bind(pybind11::module& m) {
   m.def("few_rows",
         [](const Tensor& x, const Tensor& w) { return few_rows(x, w, PLAIN); },
         "whether x @ w' takes the streaming kernel");
+  m.def("whole_rounds", &whole_rounds,
+        "rows of [M, K] @ [K, N] that go in a call of their own");
 }
 
 }  // namespace linear_bind

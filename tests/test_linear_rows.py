@@ -64,6 +64,20 @@ def test_gated(name, rows, n, k):
             _same(y, fn(g) * u, 8)
 
 
+@pytest.mark.parametrize("rows,n,k,whole", [
+    (2047, 4096, 4096, 0), (4096, 4096, 4096, 0), (4097, 4096, 96, 4096),
+    (4096 + 2048, 4096, 96, 4096), (4096 + 2049, 4096, 96, 0),
+    (4096 + 2049, 4096, 4096, 4096), (8192 + 2049, 4096, 96, 8192),
+    (4096 + 3840, 4096, 4096, 4096), (4096 + 3841, 4096, 4096, 0),
+    (8192 + 3072, 10240, 5120, 8192), (8192 + 3073, 10240, 5120, 0),
+    (11456, 14336, 4096, 0), (8533, 14336, 4096, 8192),
+    (7749, 12576, 4096, 0), (40000, 12576, 4096, 0)])
+def test_which_rows_go_apart(rows, n, k, whole):
+    """Up to half a round of tiles behind the whole ones; up to two of them
+    that do not end full, where K or the whole ones are large."""
+    assert _ext("_hip_ops").whole_rounds(rows, n, k) == whole
+
+
 @pytest.mark.parametrize("rows", [2048, 4095, 4096, 4097, 4352, 4500, 8193])
 @pytest.mark.parametrize("n,k", [(4096, 96), (4090, 72), (16384, 64),
                                  (300, 64)])
