@@ -119,6 +119,7 @@ __global__ __launch_bounds__(NW * WAVE) void route_kernel(
 
 // ---- sorting ---------------------------------------------------------------
 constexpr int ST = 1024, SV = 8;   // threads; pairs per thread and sweep
+constexpr int TILE = 256;          // pairs of a tile of expert_tiles
 
 // SV experts from place i on; -1 past the end (i is a multiple of SV)
 __device__ __forceinline__ void load_ids(const int32_t* ids, int i, int P,
@@ -134,13 +135,20 @@ __device__ __forceinline__ void load_ids(const int32_t* ids, int i, int P,
 }
 
 // One workgroup per expert. order [P]: pairs by expert; tiles [1 + max_tiles]
-// = (number of tiles, those more than half full, ..), then (expert, first
-// place in order, pairs, 0), those more than half full ahead.
+// = (number of tiles, those ahead, ..), then (expert, first place in order,
+// pairs, 0). Those more than half full go ahead, so that the shorter work comes
+// last (2000 rows, 32 experts of 4096 x 3584, 4 each: 638 us, by expert 660;
+// 2048 x 1536: 157 and 171). `share`: the weights are too many to stay in the
+// last-level cache, and tiles of one expert want to run together. So they do,
+// by expert, where workgroups read weights straight from memory (tiles of up to
+// 64 pairs) and some expert has several (380 rows of uneven loads: 592 us for
+// 617), and where every expert has several of the large ones (2500 rows: 812 us
+// for 877).
 __global__ __launch_bounds__(ST) void sort_pairs_kernel(
     const int32_t* __restrict__ ids, int32_t* __restrict__ order,
-    int4* __restrict__ tiles, int P, int E, int tile) {
+    int4* __restrict__ tiles, int P, int E, int tile, int share) {
   extern __shared__ int hist[];        // [E]
-  __shared__ int sums[ST / WAVE], at[4];
+  __shared__ int sums[ST / WAVE], at[5];
   const int e = blockIdx.x, tid = threadIdx.x;
   const int wave = tid / WAVE, lane = tid % WAVE;
   for (int i = tid; i < E; i += ST) hist[i] = 0;
@@ -153,10 +161,18 @@ __global__ __launch_bounds__(ST) void sort_pairs_kernel(
       if (x[j] >= 0 && x[j] < E) atomicAdd(&hist[x[j]], 1);
   }
   __syncthreads();
-  if (wave == 0) {       // pairs and tiles of lower experts, full ones of all
-    int n = 0, full = 0, rest = 0, all = 0;
+  if (wave == 0) {       // pairs and tiles of lower experts, those ahead of all
+    int n = 0, full = 0, rest = 0, all = 0, ahead = tile / 2 + 1;
+    if (share) {
+      bool all_do = true, some_do = false;       // have several tiles
+      for (int i = lane; i < E; i += WAVE) {
+        all_do &= hist[i] > tile;
+        some_do |= hist[i] > tile;
+      }
+      if (tile < TILE ? __any(some_do) : __all(all_do)) ahead = 1;
+    }
     for (int i = lane; i < E; i += WAVE) {
-      const int f = (hist[i] + (tile - 1) / 2) / tile;
+      const int f = (hist[i] + tile - ahead) / tile;
       all += f;
       if (i < e) {
         n += hist[i];
@@ -176,12 +192,13 @@ __global__ __launch_bounds__(ST) void sort_pairs_kernel(
       at[1] = full;
       at[2] = rest;
       at[3] = all;
+      at[4] = ahead;
     }
   }
   __syncthreads();
   const int first = at[0], count = hist[e];
   const int nt = (count + tile - 1) / tile;
-  const int nf = (count + (tile - 1) / 2) / tile;
+  const int nf = (count + tile - at[4]) / tile;
   for (int j = tid; j < nt; j += ST)
     tiles[1 + (j < nf ? at[1] + j : at[3] + at[2])] =
         make_int4(e, first + j * tile, min(tile, count - j * tile), 0);
@@ -368,7 +385,7 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
 // 1840; 256 with half lines in steps of 32: 1900; 8 waves of 64 x 64: 1800);
 // 1000 rows, 2048 x 1536: 129 (165).
 constexpr int NB = 5, BK = 64;       // chunks; K of a step
-constexpr int TC = 256, TILE = 256, HALF = 128;
+constexpr int TC = 256, HALF = 128;
 constexpr int CHUNK = 256 * BK;
 constexpr int TILES_LDS = NB * CHUNK * (int)sizeof(short);
 constexpr int TG = 3;                // tiles of pairs that run side by side
@@ -666,13 +683,14 @@ int lds_expert_max_tiles(int P, int E, int tile) {
   return n < P ? n : P;
 }
 
-// order [P], tiles [1 + max_tiles, 4]
+// order [P], tiles [1 + max_tiles, 4]; share: see sort_pairs_kernel
 hipError_t lds_sort_pairs(const int32_t* ids, int32_t* order, void* tiles,
-                          int P, int E, int tile, hipStream_t stream) {
+                          int P, int E, int tile, int share,
+                          hipStream_t stream) {
   if (P == 0) return hipSuccess;
   if (E > 8192) return hipErrorInvalidValue;
   hipLaunchKernelGGL(sort_pairs_kernel, dim3(E), dim3(ST), E * sizeof(int),
-                     stream, ids, order, (int4*)tiles, P, E, tile);
+                     stream, ids, order, (int4*)tiles, P, E, tile, share);
   HIP_CHECK_LAST();
   return hipSuccess;
 }

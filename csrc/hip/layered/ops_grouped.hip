@@ -20,7 +20,7 @@ hipError_t lds_route(int, const void*, const void*, int32_t*, float*, int64_t,
                      int, int, int, hipStream_t);
 int lds_expert_tile(int, int, int, int, int, int, int);
 int lds_expert_max_tiles(int, int, int);
-hipError_t lds_sort_pairs(const int32_t*, int32_t*, void*, int, int, int,
+hipError_t lds_sort_pairs(const int32_t*, int32_t*, void*, int, int, int, int,
                           hipStream_t);
 hipError_t lds_expert_product(int, int, int, const void*, const void*, void*,
                               const int32_t*, const void*, int, int,
@@ -175,6 +175,23 @@ std::vector<Tensor> route(Tensor h, Tensor w, int64_t top) {
   return {ids, wt};
 }
 
+// ids [T, top] below E -> pairs by expert; (number of tiles, those ahead, ..),
+// then the tiles
+std::tuple<Tensor, Tensor> sort_pairs(Tensor ids, int64_t E, int64_t tile,
+                                      bool share) {
+  check(ids, at::kInt, "ids");
+  const int64_t P = ids.numel();
+  TORCH_CHECK(P > 0 && P < (1 << 30) && E > 0 && E <= 8192 && tile > 0 &&
+                  tile <= 256, "sort_pairs");
+  const int max_tiles = lds_expert_max_tiles((int)P, (int)E, (int)tile);
+  auto order = torch::empty({P}, ids.options());
+  auto tiles = torch::empty({1 + max_tiles, 4}, ids.options());
+  check_hip(lds_sort_pairs(ip(ids), ip(order), tiles.data_ptr(), (int)P,
+                           (int)E, (int)tile, share, cur_stream()),
+            "sort_pairs");
+  return {order, tiles};
+}
+
 // h [T, K], ids and weights [T, top], up [E, F, K], down [E, K, F]
 // -> [T top, K]
 Tensor experts(Tensor h, Tensor ids, Tensor weights, Tensor up, Tensor down,
@@ -198,12 +215,10 @@ Tensor experts(Tensor h, Tensor ids, Tensor weights, Tensor up, Tensor down,
   const int tile = lds_expert_tile(f32, plain, (int)P, (int)T, (int)E, (int)F,
                                    (int)K);
   const int max_tiles = lds_expert_max_tiles((int)P, (int)E, tile);
-  auto order = torch::empty({P}, ids.options());
-  auto tiles = torch::empty({1 + max_tiles, 4}, ids.options());
   auto inner = torch::empty({P, F}, h.options());
-  check_hip(lds_sort_pairs(ip(ids), ip(order), tiles.data_ptr(), (int)P,
-                           (int)E, tile, cur_stream()),
-            "sort_pairs");
+  // the last-level cache has 256 MB
+  const auto [order, tiles] =
+      sort_pairs(ids, E, tile, E * F * K * h.element_size() > 512ll << 20);
   check_hip(lds_expert_product(f32, plain, 1, h.data_ptr(), up.data_ptr(),
                                inner.data_ptr(), ip(order), tiles.data_ptr(),
                                max_tiles, tile, fp(weights), (int)F, (int)K,
@@ -225,5 +240,6 @@ void bind_grouped(pybind11::module& m) {
   m.def("grouped_decode", &grouped_decode);
   m.def("grouped_prefill", &grouped_prefill);
   m.def("route", &route);
+  m.def("sort_pairs", &sort_pairs);
   m.def("experts", &experts);
 }

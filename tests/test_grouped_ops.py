@@ -380,3 +380,53 @@ def test_tiles_at_their_edges(K, F, act):
     a = ops.experts(h, ids, wt, up, down, act)
     b = ops.experts(h, ids, wt, up, down, act, plain=True)
     close(a, f64(b), ("", torch.bfloat16), bf16=1e-2)
+
+
+@GPU
+@pytest.mark.parametrize("tile", [16, 32, 64, 256])
+@pytest.mark.parametrize("share", [False, True])
+@pytest.mark.parametrize("times", [-1, 0, 1, 2])
+def test_order_of_tiles(tile, share, times):
+    """Tiles more than half full first; by expert where they share weights: if
+    some expert has several, of the large ones if every one has."""
+    from llm_d_inference_scheduler_amd import _hip_layered as ext
+    counts = [1, tile // 2, tile // 2 + 1, 0, tile - 1, tile, tile + 1]
+    counts = counts[:6] + [0] * 70 if times < 0 else \
+        [n + times * tile for n in counts]
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    ids = ids[torch.randperm(len(ids))].int()
+    order, tiles = ext.sort_pairs(ids.cuda()[:, None], len(counts), tile,
+                                  share)
+    assert torch.equal(order.cpu().long(), ids.argsort(stable=True))
+    cut, first = [], 0
+    for e, n in enumerate(counts):
+        cut += [[e, first + j, min(tile, n - j), 0] for j in range(0, n, tile)]
+        first += n
+    together = share and (max if tile < 256 else min)(counts) > tile
+    if not together:
+        cut.sort(key=lambda c: 2 * c[2] <= tile)
+    ahead = sum(together or 2 * c[2] > tile for c in cut)
+    assert tiles[0, :2].tolist() == [len(cut), ahead]
+    assert tiles[1:1 + len(cut)].tolist() == cut
+
+
+@GPU
+def test_tiles_that_share_weights():
+    """Experts whose weights do not stay in a cache, several tiles each."""
+    dev, E, K, F = "cuda:0", 5, 8192, 8192
+    counts = [257, 300, 384, 400, 512]
+    g = torch.Generator(device=dev).manual_seed(0)
+
+    def normal(*shape, std=1.0):
+        return torch.empty(shape, device=dev).normal_(
+            0, std, generator=g).bfloat16()
+    up, down = normal(E, F, K, std=K ** -0.5), normal(E, K, F, std=F ** -0.5)
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    ids = ids[torch.randperm(len(ids))].int().to(dev)[:, None].contiguous()
+    h, wt = normal(len(ids), K), torch.ones(len(ids), 1, device=dev)
+    got = ops.experts(h, ids, wt, up, down, "silu")
+    for e in range(E):
+        rows = (ids[:, 0] == e).nonzero()[:, 0]
+        inner = torch.nn.functional.silu(h[rows].float() @ up[e].float().t())
+        close(got[rows], f64(inner @ down[e].float().t()),
+              ("", torch.bfloat16), bf16=1e-2)
