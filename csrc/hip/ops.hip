@@ -47,7 +47,7 @@ hipError_t lds_paged_attention(const void*, const void*, const void*,
 hipError_t lds_paged_attention_split(const void*, const void*, const void*,
                                      const int32_t*, const int32_t*, void*,
                                      float*, float*, int, int, int, int, int,
-                                     int, int, int, int, int, float,
+                                     int, int, int, int, int, int, float,
                                      hipStream_t);
 hipError_t lds_flash_prefill(const void*, const void*, const void*,
                              const int32_t*, const int32_t*, const int32_t*,
@@ -382,7 +382,8 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
                                     torch::Tensor block_tables,
                                     torch::Tensor seq_lens, int64_t n_parts,
                                     int64_t part_tokens, double scale,
-                                    int64_t chunk, int64_t waves) {
+                                    int64_t chunk, int64_t waves,
+                                    bool spread) {
   check_chunk(chunk);
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
@@ -398,7 +399,7 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
       out.data_ptr(), part_o.data_ptr<float>(), part_ml.data_ptr<float>(), B,
       qh, kvh, bs, d, (int)block_tables.size(1), (int)n_parts,
-      (int)part_tokens, kv_fp8_flag(k_cache), (int)waves, (float)scale,
+      (int)part_tokens, spread, kv_fp8_flag(k_cache), (int)waves, (float)scale,
       cur_stream()));
   return out;
 }
@@ -476,7 +477,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("n_parts"),
         py::arg("part_tokens"), py::arg("scale"), py::arg("chunk") = 256,
-        py::arg("waves") = 8);
+        py::arg("waves") = 8, py::arg("spread") = false);
   m.def("flash_prefill", &flash_prefill,
         "fused MFMA causal varlen prefill attention over paged KV",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),

@@ -111,12 +111,14 @@ __global__ __launch_bounds__(NW * WAVE, 3) void paged_attention_kernel(
     short* __restrict__ out,                   // [B, QH, D]
     float* __restrict__ part_o,   // [B, KVH, NP, QPG, D] (SPLIT)
     float* __restrict__ part_ml,  // [B, KVH, NP, QPG, 2] (SPLIT), m in log2
-    int kvh, int qpg, int bs, int max_blocks, int part_tokens, float scale) {
+    int kvh, int qpg, int bs, int max_blocks, int part_tokens, int spread,
+    float scale) {
   typedef Cache<CT> C;
   // Workgroups go round the XCDs in turn: with an even number of sequences all
-  // parts of one would run on the same few, so sequences take turns by part.
-  const int turn = SPLIT && gridDim.x % 2 == 0 ? blockIdx.z : 0;
-  const int b = (blockIdx.x + turn) % gridDim.x;
+  // parts of one run on the same few. Where one is far longer than the others,
+  // sequences take turns by part.
+  const int b = SPLIT && spread ? (blockIdx.x + blockIdx.z) % gridDim.x
+                                : blockIdx.x;
   const int kh = blockIdx.y;
   const int part = SPLIT ? blockIdx.z : 0;
   const int np = SPLIT ? gridDim.z : 1;
@@ -353,8 +355,8 @@ hipError_t attend(const void* q, const void* k_cache, const void* v_cache,
                   const int32_t* block_tables, const int32_t* seq_lens,
                   void* out, float* part_o, float* part_ml, int n_seqs,
                   int n_q_heads, int kvh, int bs, int head_dim, int max_blocks,
-                  int n_parts, int part_tokens, int kv_fp8, int waves,
-                  float scale, hipStream_t stream) {
+                  int n_parts, int part_tokens, int spread, int kv_fp8,
+                  int waves, float scale, hipStream_t stream) {
   if (n_seqs == 0) return hipSuccess;
   const int qpg = n_q_heads / kvh;
   if (head_dim != D || n_parts > 64 || (waves != 4 && waves != 8) ||
@@ -366,7 +368,8 @@ hipError_t attend(const void* q, const void* k_cache, const void* v_cache,
                      dim3(NW * WAVE), 0, stream, (const short*)q,            \
                      (const CT*)k_cache, (const CT*)v_cache, block_tables,   \
                      seq_lens, (short*)out, part_o, part_ml, kvh, qpg, bs,   \
-                     max_blocks, part_tokens, scale)
+                     max_blocks, part_tokens, spread && n_seqs % 2 == 0,     \
+                     scale)
 #define GO_NW(CT, PAGE16)                                                    \
   do {                                                                       \
     if (waves == 8) GO(CT, PAGE16, 8); else GO(CT, PAGE16, 4);               \
@@ -401,19 +404,19 @@ hipError_t lds_paged_attention(const void* q, const void* k_cache,
                                float scale, hipStream_t stream) {
   return attend<false>(q, k_cache, v_cache, block_tables, seq_lens, out,
                        nullptr, nullptr, n_seqs, n_q_heads, kvh, bs, head_dim,
-                       max_blocks, 1, 0, kv_fp8, waves, scale, stream);
+                       max_blocks, 1, 0, 0, kv_fp8, waves, scale, stream);
 }
 
 hipError_t lds_paged_attention_split(
     const void* q, const void* k_cache, const void* v_cache,
     const int32_t* block_tables, const int32_t* seq_lens, void* out,
     float* part_o, float* part_ml, int n_seqs, int n_q_heads, int kvh, int bs,
-    int head_dim, int max_blocks, int n_parts, int part_tokens, int kv_fp8,
-    int waves, float scale, hipStream_t stream) {
+    int head_dim, int max_blocks, int n_parts, int part_tokens, int spread,
+    int kv_fp8, int waves, float scale, hipStream_t stream) {
   return attend<true>(q, k_cache, v_cache, block_tables, seq_lens, out, part_o,
                       part_ml, n_seqs, n_q_heads, kvh, bs, head_dim,
-                      max_blocks, n_parts, part_tokens, kv_fp8, waves, scale,
-                      stream);
+                      max_blocks, n_parts, part_tokens, spread, kv_fp8, waves,
+                      scale, stream);
 }
 
 }  // extern "C"

@@ -170,9 +170,12 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
             parts, part = decode_parts(q.shape[0] * k_cache.shape[1],
                                        max_seq_len, mean_seq_len)
             if parts > 1:
+                far_apart = mean_seq_len is not None and \
+                    max_seq_len > 2 * mean_seq_len
                 return _ext.paged_attention_split(q, k_cache, v_cache, bt,
                                                   sl, parts, part, scale,
-                                                  waves=waves)
+                                                  waves=waves,
+                                                  spread=far_apart)
         return _ext.paged_attention(q, k_cache, v_cache, bt, sl, scale,
                                     waves=waves)
     return ref.paged_attention(q, k_cache, v_cache, block_tables, seq_lens,

@@ -98,7 +98,9 @@ def test_lengths_far_apart(batch, fp8):
     assert batch == 1 or dispatch.decode_parts(batch * KVH, 2900, mean)[0] > 1
     from llm_d_inference_scheduler_amd import _hip_ops as ext
     for parts, part in [(2, 1472), (12, 256), (64, 48)]:
-        _close(ext.paged_attention_split(*args, parts, part, D ** -0.5), want)
+        for spread in (False, True):
+            _close(ext.paged_attention_split(*args, parts, part, D ** -0.5,
+                                             spread=spread), want)
 
 
 @pytest.mark.gpu
