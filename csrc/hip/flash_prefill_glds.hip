@@ -26,10 +26,10 @@
 //
 // Measured (groups of 4, 8 key heads, alone; before: masks, packing and
 // rescaling of every tile on the vector units): one prompt of 7900 tokens 650
-// us, 785 TFLOP/s (before 1170); 8 of 1000 135 us (265). By keys / by rows with
-// 17 bits (with 8): 150 tokens behind 1000 24 / 48 us (44; before 61); 500
-// behind 1000 52 / 66 (57; 79); 600 behind 4000 195 / 175 (159; 235); 12
-// prompts of 20 13 / 7 (6; 7).
+// us, 785 TFLOP/s (before 1170); 8 of 1000 135 us (265); in a pass of layers one
+// of 8190 takes 812, 676 TFLOP/s. By keys / by rows with 17 bits (with 8): 150
+// tokens behind 1000 24 / 48 us (44; before 61); 500 behind 1000 52 / 66 (57;
+// 79); 600 behind 4000 195 / 175 (159; 235); 12 prompts of 20 13 / 7 (6; 7).
 //
 // fp8 KV cannot ride glds (raw byte copy, no conversion point), so the fp8
 // path keeps the convert-on-stage kernel in flash_prefill.hip; the launcher in

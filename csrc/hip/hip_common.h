@@ -34,13 +34,7 @@ __device__ __forceinline__ short f32_to_bf16(float f) {
 // dword. Cache element type CT is short (bf16) or unsigned char (fp8).
 typedef __attribute__((ext_vector_type(8))) unsigned char uchar8;
 
-// load 8 cache elements -> f32[8]
-__device__ __forceinline__ void load_kv8(const short* p, float* f) {
-  short8 v = *(const short8*)p;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
-}
-
+// load 8 fp8 cache elements -> f32[8]
 __device__ __forceinline__ void load_kv8(const unsigned char* p, float* f) {
   const uint32_t* w = (const uint32_t*)p;   // two dwords = 8 fp8
   uint32_t a = w[0], b = w[1];
@@ -52,20 +46,6 @@ __device__ __forceinline__ void load_kv8(const unsigned char* p, float* f) {
   f[5] = __builtin_amdgcn_cvt_f32_fp8(b, 1);
   f[6] = __builtin_amdgcn_cvt_f32_fp8(b, 2);
   f[7] = __builtin_amdgcn_cvt_f32_fp8(b, 3);
-}
-
-// load 2 consecutive cache elements (phase-C dim pair per lane)
-__device__ __forceinline__ void load_kv2(const short* p, float& a, float& b) {
-  const int32_t pair = *(const int32_t*)p;
-  a = bf16_to_f32((short)(pair & 0xFFFF));
-  b = bf16_to_f32((short)((pair >> 16) & 0xFFFF));
-}
-
-__device__ __forceinline__ void load_kv2(const unsigned char* p, float& a,
-                                         float& b) {
-  const uint32_t pair = *(const uint16_t*)p;
-  a = __builtin_amdgcn_cvt_f32_fp8(pair, 0);
-  b = __builtin_amdgcn_cvt_f32_fp8(pair, 1);
 }
 
 // store 8 bf16 source elements as cache elements
@@ -86,20 +66,6 @@ __device__ __forceinline__ void store_kv8(unsigned char* p, short8 v) {
   uint32_t* w = (uint32_t*)p;
   w[0] = lo;
   w[1] = hi;
-}
-
-// load 8 cache elements as bf16 (LDS staging in the flash-prefill kernel)
-__device__ __forceinline__ short8 load_kv8_bf16(const short* p) {
-  return *(const short8*)p;
-}
-
-__device__ __forceinline__ short8 load_kv8_bf16(const unsigned char* p) {
-  float f[8];
-  load_kv8(p, f);
-  short8 out;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) out[j] = f32_to_bf16(f[j]);
-  return out;
 }
 
 // full-wave f32 sum reduction (6 xor-shuffle steps over 64 lanes)

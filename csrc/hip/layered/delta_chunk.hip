@@ -16,8 +16,8 @@
 // delta_chunk_local  everything that does not need S0, one workgroup per
 //                    (head, chunk): U0 and W with U = U0 - W S0, P, the
 //                    scaled q and k -> workspace
-// delta_chunk_scan   one workgroup per (head, 16 columns of S, sequence)
-//                    walks the chunks with S in registers
+// delta_chunk_scan   one workgroup per (head, 16 or 32 columns of S, sequence)
+//                    walks the chunks with S in LDS
 // delta_gate         gated output norm
 //
 // MFMA operands: lane l gives A[l % 16][k] and B[k][l % 16] with k = l / 16,

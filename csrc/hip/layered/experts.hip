@@ -368,10 +368,11 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
 }
 
 // 256 channels x 256 pairs, K in steps of 64, both operands loaded straight to
-// LDS. What bounds it is the way from the L2s to LDS and the power that it
-// takes (without the loads 28000 pairs of 4096 x 3584 take 1230 us for 1960,
-// without the LDS reads 1910), hence the size of the tile, and whole lines of
-// 128 bytes. LDS holds five chunks of 256 rows, those of weights and of pairs
+// LDS. What bounds it is the way from the L2s to LDS (without the loads 28000
+// pairs of 4096 x 3584 take 1230 us for 1960, without the LDS reads 1910), hence
+// the size of the tile, and whole lines of 128 bytes; 160 KB of LDS leave one
+// workgroup per compute unit, so nothing covers a tile's first loads and its
+// turning round of the results. LDS holds five chunks of 256 rows, those of weights and of pairs
 // in turn: two and a half steps. 4 waves, CT x PT tiles of 32 x 32 each:
 // 128 x 128, or, where a tile has no more than 128 pairs, 64 x 128 (so nothing
 // is lost by the larger tile). A row of a step is 8 pieces; piece c of row r

@@ -1,6 +1,6 @@
-// linear_bind.h — torch binding of linear_rows.hip, shared by the extensions.
-// Products go to the streaming kernel where its rule holds, else to the
-// library.
+// linear_bind.h — torch binding of linear_rows.hip and linear_tiles.hip, shared
+// by the extensions. Products go to these kernels where their rule holds, else
+// to the library, of many rows in two calls where that is faster.
 #pragma once
 #include <torch/extension.h>
 #include <ATen/autocast_mode.h>
@@ -76,8 +76,9 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
 //   - the rest is two rounds of tiles or more: the second call is as likely as
 //     the one to get the poor kernel (5120 -> 10240, 12852 rows: 869 us in one
 //     call, 1065 in two; 4096 -> 14336, 11518 rows: 878 and 1039);
-//   - it ends in a round that is full but for 1/16: nothing to gain (4096 ->
-//     12576, 7749 rows: 31.7 ms a pass of 8 layers, 31.95 in two calls each);
+//   - it ends in a round that is full but for 1/16: nothing to gain (a pass of
+//     8 delta layers, 7749 rows: 31.7 ms, 31.95 with its products to 4096
+//     channels in two calls);
 //   - it is more than half a round beside a single whole one and K is short:
 //     the second call costs what the round would (2048 -> 4096, 6266 rows: 88
 //     us and 95).

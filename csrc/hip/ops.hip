@@ -353,17 +353,11 @@ void copy_blocks_peer(uintptr_t src_pool_ptr, torch::Tensor dst_pool,
       (int)src_ids.size(0), L, src_nb, dst_nb, block_bytes, cur_stream()));
 }
 
-// `chunk` chose the softmax step of an earlier kernel: it is still checked
-void check_chunk(int64_t chunk) {
-  TORCH_CHECK(chunk == 256 || chunk == 512, "chunk must be 256 or 512");
-}
-
 torch::Tensor paged_attention(torch::Tensor q, torch::Tensor k_cache,
                               torch::Tensor v_cache,
                               torch::Tensor block_tables,
                               torch::Tensor seq_lens, double scale,
-                              int64_t chunk, int64_t waves) {
-  check_chunk(chunk);
+                              int64_t waves) {
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -382,9 +376,7 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
                                     torch::Tensor block_tables,
                                     torch::Tensor seq_lens, int64_t n_parts,
                                     int64_t part_tokens, double scale,
-                                    int64_t chunk, int64_t waves,
-                                    bool spread) {
-  check_chunk(chunk);
+                                    int64_t waves, bool spread) {
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -470,14 +462,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attention", &paged_attention,
         "GQA decode attention over paged KV", py::arg("q"),
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
-        py::arg("seq_lens"), py::arg("scale"), py::arg("chunk") = 256,
-        py::arg("waves") = 8);
+        py::arg("seq_lens"), py::arg("scale"), py::arg("waves") = 8);
   m.def("paged_attention_split", &paged_attention_split,
         "flash-decoding GQA attention with sequence partitioning",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("n_parts"),
-        py::arg("part_tokens"), py::arg("scale"), py::arg("chunk") = 256,
-        py::arg("waves") = 8, py::arg("spread") = false);
+        py::arg("part_tokens"), py::arg("scale"), py::arg("waves") = 8,
+        py::arg("spread") = false);
   m.def("flash_prefill", &flash_prefill,
         "fused MFMA causal varlen prefill attention over paged KV",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),

@@ -18,10 +18,11 @@
 // A tile's matrix work is a quarter of the time its bytes take at 5 TB/s, so
 // the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost nothing.
 //
-// Measured (8 key heads, ragged; before: scores and sums on the vector units,
-// three barriers per 256 tokens): 256 sequences of 1500 tokens, groups of 4:
-// 279 us, 5.6 TB/s (before 546); 30 of 1100, groups of 8: 27 us (67); 17 of
-// 6800, fp8, in 4 partitions: 61 us, 3.8 TB/s (137); one of 777: 11 us (18).
+// Measured alone (8 key heads, ragged; before: scores and sums on the vector
+// units, three barriers per 256 tokens): 256 sequences of 1500 tokens, groups of
+// 4: 279 us, 5.6 TB/s (before 546); 30 of 1100, groups of 8: 27 us (67); 17 of
+// 6800, fp8, in 4 partitions: 61 us, 3.8 TB/s (137), in a pass of layers 82, 2.9
+// TB/s; one of 777: 11 us (18).
 //
 // Flash-decoding sequence split (SPLIT): long sequences are cut into
 // gridDim.z partitions so that small batches fill the chip. Each partition

@@ -1,18 +1,17 @@
 """Llama-family model runner (random-init weights, paged KV, bf16).
 
 MI355X-native execution path: projections of few rows stream their weights
-through a HIP kernel, the rest go through hipBLASLt; the fused hot ops (residual+RMSNorm,
-RoPE, SiLU*up, GQA paged decode attention, KV scatter) are the gfx950 HIP
-kernels in csrc/hip dispatched through ops/. Prefill attention is composed
-chunked torch-matmul attention over KV gathered from the paged pool (an
-LDS-tiled MFMA flash kernel is the planned replacement; no Triton, no SDPA
-multi-backend dispatch is used anywhere).
+through a HIP kernel, the rest go through hipBLASLt; the fused hot ops
+(residual+RMSNorm, RoPE with the KV scatter, SiLU*up, GQA paged decode and
+prefill attention) are the gfx950 HIP kernels in csrc/hip dispatched through
+ops/. On the CPU, and for head sizes that the prefill kernels do not take,
+prefill attention is composed of torch products over KV gathered from the paged
+pool.
 
 The reference router never runs a model — its pods do (vLLM). This runner
 is the per-GPU worker engine's model, SURVEY.md §2.12 "worker shim".
 """
 import math
-import os
 from dataclasses import dataclass
 from typing import Dict, List, Optional
 

@@ -1,7 +1,5 @@
 """Decode paged-attention kernel microbenchmark (run on a GPU box).
-Times the production kernel at serving shapes with/without sequence split,
-against the pipelined v4 (producer/consumer waves, double-buffered logits).
-Also checks v4 numerics against v1 before timing.
+Times the kernel at serving shapes with and without sequence split.
 """
 import os
 import sys
@@ -34,22 +32,7 @@ def make(B, ctx, qpg, fp8=False, seed=0):
     return q, kc, vc, bt, sl
 
 
-def check(kernel, qpg=4, fp8=False):
-    fn = getattr(ext, f"paged_attention_{kernel}")
-    for B, ctx, np_, part in ((4, 300, 1, 0), (8, 1152, 1, 0),
-                              (8, 1152, 4, 320), (3, 70, 1, 0)):
-        q, kc, vc, bt, sl = make(B, ctx, qpg, fp8)
-        scale = D ** -0.5
-        ref = ext.paged_attention(q, kc, vc, bt, sl, scale)
-        got = fn(q, kc, vc, bt, sl, np_,
-                 part if np_ > 1 else ctx + 256, scale)
-        diff = (ref.float() - got.float()).abs().max().item()
-        status = "OK" if diff < 3e-2 else "FAIL"
-        print(f"{kernel} numerics qpg={qpg} fp8={int(fp8)} B={B} ctx={ctx} "
-              f"np={np_}: max|d|={diff:.4f} {status}")
-
-
-def bench(B, ctx, np_=None, part=512, iters=50, kernel="v1", qpg=4):
+def bench(B, ctx, np_=None, part=512, iters=50, qpg=4):
     q, kc, vc, bt, sl = make(B, ctx, qpg)
     scale = D ** -0.5
 
@@ -68,7 +51,7 @@ def bench(B, ctx, np_=None, part=512, iters=50, kernel="v1", qpg=4):
     torch.cuda.synchronize()
     us = (time.perf_counter() - t0) / iters * 1e6
     kv_gb = B * ctx * KVH * D * 2 * 2 / 1e9
-    print(f"B={B:4d} ctx={ctx:5d} np={np_ or 1:2d} {kernel}: {us:8.1f} us  "
+    print(f"B={B:4d} ctx={ctx:5d} np={np_ or 1:2d}: {us:8.1f} us  "
           f"({kv_gb / (us / 1e6) / 1e3:6.2f} TB/s effective)")
 
 
