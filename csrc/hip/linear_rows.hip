@@ -242,7 +242,9 @@ int lds_linear_rows_parts(int M, int N, int K) {
 // times, here / there, in us:
 //   parts the caller sums itself: always. 4096 -> 4096: 1 row 8 / 15, 96 rows
 //     12 / 22, 256 rows 18 / 23; 14336 -> 4096: 64 rows 23 / 40, 256 rows
-//     41 / 63; 4096 -> 12576: 64 rows 24 / 25, 256 rows 42 / 50.
+//     41 / 63; 4096 -> 12576: 64 rows 24 / 25, 256 rows 42 / 50. (Above 128 rows
+//     a K below 1600 takes up to 3 us more here, 688 -> 1680, 256 rows 13 / 10;
+//     that it comes out as a single row does is worth it.)
 //   one part, and gated ones (there with their activation): if the workgroups
 //     fill at least 7/8 of their rounds, up to 128 rows, gated up to 192. 4096 -> 32768: 32 rows
 //     46 / 62, 128 rows 55 / 64, 160 rows 66 / 67; -> 128256 (98 %): 64 rows
