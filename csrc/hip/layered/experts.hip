@@ -11,13 +11,9 @@
 //                  there the weights' bytes are what counts
 //   expert_plain   any size, bf16 or float
 #include "elem.h"
-
-#include <type_traits>
+#include "../tile_core.h"
 
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 // ---- router ----------------------------------------------------------------
 // The `top` largest of z[0, E) by one wave: experts and sigmoids of their
@@ -367,195 +363,71 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
   }
 }
 
-// 256 channels x 256 pairs, K in steps of 64, both operands loaded straight to
-// LDS. What bounds it is the way from the L2s to LDS (without the loads 28000
-// pairs of 4096 x 3584 take 1230 us for 1960, without the LDS reads 1910), hence
-// the size of the tile, and whole lines of 128 bytes; 160 KB of LDS leave one
-// workgroup per compute unit, so nothing covers a tile's first loads and its
-// turning round of the results. LDS holds five chunks of 256 rows, those of weights and of pairs
-// in turn: two and a half steps. 4 waves, CT x PT tiles of 32 x 32 each:
-// 128 x 128, or, where a tile has no more than 128 pairs, 64 x 128 (so nothing
-// is lost by the larger tile). A row of a step is 8 pieces; piece c of row r
-// lies at place c ^ (r / 2 % 8): the 16 rows a read serves at once then meet
-// all 64 banks. Loads and LDS reads are spread between the matrix instructions:
-// issued in a row they would hold the wave up. Operands are read 16 of K ahead,
-// across the one barrier of a step.
-//
-// Both products: 7032 rows, 32 experts of 4096 x 3584, 4 each: 1670 us, 990
-// TFLOP/s (128 pairs per tile and the reads of a step behind its barrier:
-// 1840; 256 with half lines in steps of 32: 1900; 8 waves of 64 x 64: 1800);
-// 1000 rows, 2048 x 1536: 129 (165).
-constexpr int NB = 5, BK = 64;       // chunks; K of a step
-constexpr int TC = 256, HALF = 128;
-constexpr int CHUNK = 256 * BK;
-constexpr int TILES_LDS = NB * CHUNK * (int)sizeof(short);
-constexpr int TG = 3;                // tiles of pairs that run side by side
+// 256 channels x 256 pairs, or 128 where a tile has no more (so nothing is lost by
+// the larger tile): see tile_core.h for the loop and what bounds it. Both products,
+// 7032 rows, 32 experts of 4096 x 3584, 4 each: 1290 us, 1280 TFLOP/s of useful
+// work (1655 with 32x32 instructions, address arithmetic in the loop and places
+// read while the results leave); 2000 rows 580 us (652); 16000 rows, 64 experts of
+// 2048 x 1024, 2 each: 311 us (378). Four tiles of pairs side by side: a compute
+// die's 32 workgroups share the loads of 4 + 8 tiles (8192 x 4096 -> 28672 in 1320
+// us, 1366 with 3).
+constexpr int TC = TILE_C, BK = TILE_K, HALF = 128;
+constexpr int TG = 4;                // tiles of pairs that run side by side
 
 // WC waves across the channels, the others across the pairs
 template <bool UP, int CT, int PT, int WC>
 __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
                                              const int4 tile, int n0) {
-  static_assert(32 * CT * WC == TC, "");
-  constexpr int LW = TC / 32, LP = PT * (4 / WC);      // loads per step
-  static_assert(LW == 8 && LP <= CT + PT, "");
+  TileCore<CT, PT, WC> core;
+  constexpr int LW = core.LW, LP = core.LP;
   const int N = p.N, K = p.K;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-  const int lane = threadIdx.x % WAVE, col = lane & 31, hi = lane >> 5;
-  const int wc = wave % WC, wp = wave / WC;    // its channels, its pairs
-
-  // A wave fills a quarter of the rows of both, 8 rows per instruction, from
-  // byte offsets within the expert's weights and p.a (both under 4 GiB).
-  // Rows past the tile repeat its last one: they are computed and dropped.
-  const char* wbase = (const char*)p.w + (int64_t)tile.x * N * K * 2;
-  const char* abase = (const char*)p.a;
-  auto piece = [&](int j) {
-    return (lane % 8 ^ (lane / 16 + j % 2 * 4)) * 8;
-  };
-  uint32_t wsrc[LW], asrc[LP];
-  int64_t rows[LP];
+  const auto wres = __builtin_amdgcn_make_buffer_rsrc(
+      (char*)p.w + (int64_t)tile.x * N * K * 2, 0, (uint32_t)N * K * 2,
+      BUFFER_BYTES);
+  const auto ares = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, 0xffffffffu,
+                                                      BUFFER_BYTES);
+  // channels past the end and rows past the tile repeat the last one: they are
+  // computed and dropped
+  uint32_t wsrc[2 * LW], asrc[2 * LP];
 #pragma unroll
-  for (int j = 0; j < LP; ++j)
-    rows[j] = source<UP>(p, tile.y + min((wave * LP + j) * 8 + lane / 8,
+  for (int j = 0; j < 2 * LP; ++j)
+    asrc[j] = source<UP>(p, tile.y + min(core.template loaded<LP>(j),
                                          tile.z - 1));
 #pragma unroll
-  for (int j = 0; j < LW; ++j)
-    wsrc[j] = ((uint32_t)min(n0 + (wave * LW + j) * 8 + lane / 8, N - 1) * K +
-               piece(j)) * 2;
-  const int steps = K / BK;
-  typedef __attribute__((address_space(1))) const unsigned int gmem;
-  typedef __attribute__((address_space(3))) unsigned int smem;
-  // past the end the last step repeats
-  auto load_w = [&](int s, int chunk, int j) {
-    __builtin_amdgcn_global_load_lds(
-        (gmem*)(wbase + min(s, steps - 1) * BK * 2 + wsrc[j]),
-        (smem*)(lds + chunk * CHUNK + (wave * LW + j) * 8 * BK), 16, 0, 0);
-  };
-  auto load_a = [&](int s, int chunk, int j) {
-    __builtin_amdgcn_global_load_lds(
-        (gmem*)(abase + min(s, steps - 1) * BK * 2 + asrc[j]),
-        (smem*)(lds + chunk * CHUNK + (wave * LP + j) * 8 * BK), 16, 0, 0);
-  };
+  for (int j = 0; j < 2 * LW; ++j)
+    wsrc[j] = ((uint32_t)min(n0 + core.template loaded<LW>(j), N - 1) * K +
+               core.piece(j)) * 2;
 #pragma unroll
-  for (int j = 0; j < LW; ++j) load_w(0, 0, j);
-#pragma unroll
-  for (int j = 0; j < LP; ++j)
-    asrc[j] = ((uint32_t)rows[j] * K + piece(j)) * 2;
-#pragma unroll
-  for (int j = 0; j < LP; ++j) load_a(0, 1, j);
-#pragma unroll
-  for (int j = 0; j < LW; ++j) load_w(1, 2, j);
-#pragma unroll
-  for (int j = 0; j < LP; ++j) load_a(1, 3, j);
-
-  f32x16 acc[CT][PT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c)
-#pragma unroll
-    for (int t = 0; t < PT; ++t) acc[c][t] = (f32x16)(0.f);
-  bf16x8 wf[2][CT], af[2][PT];
-  const short* wl = lds + (wc * 32 * CT + col) * BK;
-  const short* al = lds + (wp * 32 * PT + col) * BK;
-  auto read = [&](int x, int w_chunk, int a_chunk, int kk) {
-    const int at = ((kk * 2 + hi) ^ (col / 2 & 7)) * 8;
-#pragma unroll
-    for (int c = 0; c < CT; ++c)
-      wf[x][c] = *(const bf16x8*)(wl + w_chunk * CHUNK + c * 32 * BK + at);
+  for (int j = 0; j < 2 * LP; ++j) asrc[j] = (asrc[j] * K + core.piece(j)) * 2;
+  // what the results need is on its way while the products run: weights by row,
+  // or the places that 64 rows go to
+  float wt[PT];
+  int32_t to[PT / 4];
+  if constexpr (UP) {
 #pragma unroll
     for (int t = 0; t < PT; ++t)
-      af[x][t] = *(const bf16x8*)(al + a_chunk * CHUNK + t * 32 * BK + at);
-  };
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(LW + LP) : "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  read(0, 0, 1, 0);
-  __builtin_amdgcn_sched_barrier(0);
-  auto after = [](int chunk, int n) {
-    return chunk + n < NB ? chunk + n : chunk + n - NB;
-  };
-  int at = 0;                  // chunk of this step's weights
-  for (int s = 0; s < steps; ++s) {
+      wt[t] = p.weights[p.order[tile.y + min(core.row_of(t * 16 + core.col),
+                                             tile.z - 1)]];
+  } else {
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      if (kk == 3) {
-        // All operands of this step are in registers: its chunks can be
-        // filled. The next step has landed, the weights after it may not.
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(LW) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        read(0, after(at, 2), after(at, 3), 0);
-      } else {
-        read(kk + 1 & 1, at, after(at, 1), kk + 1);
-      }
-      if (kk == 3) {
-#pragma unroll
-        for (int j = 0; j < LP; ++j) load_a(s + 2, at, j);
-      } else if (kk < 2) {
-#pragma unroll
-        for (int j = 0; j < LW / 2; ++j)
-          load_w(s + 2, after(at, 4), kk * LW / 2 + j);
-      }
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int t = 0; t < PT; ++t)
-          acc[c][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-              wf[kk & 1][c], af[kk & 1][t], acc[c][t], 0, 0, 0);
-      // the order: matrix, read, (load), ... matrix
-      const int loads = kk == 3 ? LP : kk < 2 ? LW / 2 : 0;
-#pragma unroll
-      for (int i = 0; i < CT + PT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        if (i < loads) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-      }
-      __builtin_amdgcn_sched_group_barrier(0x008, CT * PT - CT - PT, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    at = after(at, 2);
+    for (int t = 0; t < PT / 4; ++t)
+      to[t] = p.order[tile.y + min(core.row_of(t * 64 + core.lane),
+                                   tile.z - 1)];
   }
-  // no wave reads a buffer any more, and the repeated loads are in
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  core.run(lds, wres, wsrc, ares, asrc, K / BK);
 
-  // The results turn round in the wave's share of LDS, so that a row of them
-  // is written in pieces of 16 bytes side by side (8 bytes of 32 rows at a
-  // time take 9 us, 8 % of the products' time).
-  constexpr int G = 4 * CT;                  // pieces of 8 channels in a row
-  static_assert(32 * PT * 8 * G * 4 <= NB * CHUNK, "");
-  short* mine = lds + wave * 32 * PT * 8 * G;
-  auto place = [](int row, int g) {
-    return (row * G + (g ^ (G == 16 ? row & 15 : row / 2 & 7))) * 8;
-  };
-  static_assert(G == 16 || G == 8, "");
   auto write = [&](auto act) {
 #pragma unroll
-    for (int t = 0; t < PT; ++t) {
-      const int i = min(wp * 32 * PT + t * 32 + col, tile.z - 1);
-      const float wt = UP ? p.weights[p.order[tile.y + i]] : 1.f;
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          short4v v;
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const float f = acc[c][t][4 * q + x];
-            v[x] = f32_to_bf16(UP ? activate(act, f * wt) : f);
-          }
-          *(short4v*)(mine + place(t * 32 + col, c * 4 + q) + hi * 4) = v;
-        }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const int n = n0 + wc * 32 * CT + lane % G * 8;
-#pragma unroll 8
-    for (int j = 0; j < 32 * PT; j += WAVE / G) {
-      const int row = j + lane / G, i = wp * 32 * PT + row;
-      if (i >= tile.z || n >= N) continue;   // N is a multiple of 8
-      const int64_t to = UP ? tile.y + i : p.order[tile.y + i];
-      *(short8*)((short*)p.out + to * N + n) =
-          *(const short8*)(mine + place(row, lane % G));
-    }
+    for (int b = 0; b < PT / 2; ++b)
+      core.turn(
+          lds, b,
+          [&](float f, int t) { return UP ? activate(act, f * wt[t]) : f; },
+          [&](int row, int i, int c, short8 v) {
+            int64_t at = tile.y + i;
+            if constexpr (!UP) at = __shfl(to[b / 2], b % 2 * 32 + row, WAVE);
+            if (i < tile.z && n0 + c < N)       // N is a multiple of 8
+              *(short8*)((short*)p.out + at * N + n0 + c) = v;
+          });
   };
   using std::integral_constant;
   if (!UP || p.act == ACT_RELU_SQUARED)
@@ -568,7 +440,7 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
 
 template <bool UP>
 __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
-  extern __shared__ __align__(16) short tile_lds[];  // NB x [weights, pairs]
+  extern __shared__ __align__(16) short tile_lds[];  
   // Workgroups go round the 8 XCDs in turn: each XCD gets a contiguous share
   // of the tiles more than half full, then one of the others (the shorter
   // work last), in which TG tiles of pairs walk the channels together.
@@ -589,9 +461,9 @@ __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
   const int4 tile = p.tiles[base + g * TG + in % width];
   const int n0 = in / width * TC;
   if (tile.z > HALF)
-    tile_product<UP, 4, 4, 2>(p, tile_lds, tile, n0);
+    tile_product<UP, 8, 8, 2>(p, tile_lds, tile, n0);
   else
-    tile_product<UP, 2, 4, 4>(p, tile_lds, tile, n0);
+    tile_product<UP, 4, 8, 4>(p, tile_lds, tile, n0);
 }
 
 template <bool UP>
@@ -604,9 +476,9 @@ hipError_t launch_tiles(const Pairs& p, int max_tiles, hipStream_t stream) {
     return hipErrorInvalidValue;
   auto fn = expert_tiles_kernel<UP>;
   hipError_t e = hipFuncSetAttribute(
-      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, TILES_LDS);
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, TILE_LDS);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3((uint32_t)n), dim3(256), TILES_LDS, stream, p);
+  hipLaunchKernelGGL(fn, dim3((uint32_t)n), dim3(256), TILE_LDS, stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }
