@@ -371,34 +371,41 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
 // 2048 x 1024, 2 each: 311 us (378). Four tiles of pairs side by side: a compute
 // die's 32 workgroups share the loads of 4 + 8 tiles (8192 x 4096 -> 28672 in 1320
 // us, 1366 with 3).
-constexpr int TC = TILE_C, BK = TILE_K, HALF = 128;
+constexpr int TC = 256, BK = TILE_K, HALF = 128;
 constexpr int TG = 4;                // tiles of pairs that run side by side
+typedef TileCore<8, 8, 2, 2> Whole;
+typedef TileCore<4, 8, 4, 2> Half;
+static_assert(Whole::CHANNELS == TC && Half::CHANNELS == TC &&
+                  Whole::ROWS == TILE && Half::ROWS == HALF,
+              "");
 
-// WC waves across the channels, the others across the pairs
-template <bool UP, int CT, int PT, int WC>
+template <bool UP, typename Core>
 __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
                                              const int4 tile, int n0) {
-  TileCore<CT, PT, WC> core;
-  constexpr int LW = core.LW, LP = core.LP;
+  Core core;
+  constexpr int LW = Core::LW, LP = Core::LP, PT = Core::ROWS / 16 / Core::WP;
   const int N = p.N, K = p.K;
-  const auto wres = __builtin_amdgcn_make_buffer_rsrc(
-      (char*)p.w + (int64_t)tile.x * N * K * 2, 0, (uint32_t)N * K * 2,
-      BUFFER_BYTES);
-  const auto ares = __builtin_amdgcn_make_buffer_rsrc((void*)p.a, 0, 0xffffffffu,
-                                                      BUFFER_BYTES);
   // channels past the end and rows past the tile repeat the last one: they are
   // computed and dropped
-  uint32_t wsrc[2 * LW], asrc[2 * LP];
+  uint32_t wsrc[2][LW], asrc[2][LP];
 #pragma unroll
-  for (int j = 0; j < 2 * LP; ++j)
-    asrc[j] = source<UP>(p, tile.y + min(core.template loaded<LP>(j),
-                                         tile.z - 1));
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-  for (int j = 0; j < 2 * LW; ++j)
-    wsrc[j] = ((uint32_t)min(n0 + core.template loaded<LW>(j), N - 1) * K +
-               core.piece(j)) * 2;
+    for (int j = 0; j < LP; ++j)
+      asrc[h][j] = source<UP>(
+          p, tile.y + min(h * Core::RH + core.template loaded<LP>(j),
+                          tile.z - 1));
 #pragma unroll
-  for (int j = 0; j < 2 * LP; ++j) asrc[j] = (asrc[j] * K + core.piece(j)) * 2;
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int j = 0; j < LW; ++j)
+      wsrc[h][j] =
+          ((uint32_t)min(n0 + h * Core::CH + core.template loaded<LW>(j),
+                         N - 1) * K + core.template piece<LW>(j)) * 2;
+#pragma unroll
+    for (int j = 0; j < LP; ++j)
+      asrc[h][j] = (asrc[h][j] * K + core.template piece<LP>(j)) * 2;
+  }
   // what the results need is on its way while the products run: weights by row,
   // or the places that 64 rows go to
   float wt[PT];
@@ -406,15 +413,17 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
   if constexpr (UP) {
 #pragma unroll
     for (int t = 0; t < PT; ++t)
-      wt[t] = p.weights[p.order[tile.y + min(core.row_of(t * 16 + core.col),
+      wt[t] = p.weights[p.order[tile.y + min(core.row(t) + core.col,
                                              tile.z - 1)]];
   } else {
 #pragma unroll
     for (int t = 0; t < PT / 4; ++t)
-      to[t] = p.order[tile.y + min(core.row_of(t * 64 + core.lane),
-                                   tile.z - 1)];
+      to[t] = p.order[tile.y + min(core.row(t * 4) + core.lane, tile.z - 1)];
   }
-  core.run(lds, wres, wsrc, ares, asrc, K / BK);
+  // offsets stay under 4 GiB (lds_expert_tile)
+  core.run(lds, (const char*)p.w + (int64_t)tile.x * N * K * 2,
+           (uint32_t)N * K * 2, wsrc, p.a, 0xfffffff0u, asrc, K / BK,
+           [](int s) { return s * BK * 2; });
 
   auto write = [&](auto act) {
 #pragma unroll
@@ -461,9 +470,9 @@ __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
   const int4 tile = p.tiles[base + g * TG + in % width];
   const int n0 = in / width * TC;
   if (tile.z > HALF)
-    tile_product<UP, 8, 8, 2>(p, tile_lds, tile, n0);
+    tile_product<UP, Whole>(p, tile_lds, tile, n0);
   else
-    tile_product<UP, 4, 8, 4>(p, tile_lds, tile, n0);
+    tile_product<UP, Half>(p, tile_lds, tile, n0);
 }
 
 template <bool UP>
@@ -476,9 +485,9 @@ hipError_t launch_tiles(const Pairs& p, int max_tiles, hipStream_t stream) {
     return hipErrorInvalidValue;
   auto fn = expert_tiles_kernel<UP>;
   hipError_t e = hipFuncSetAttribute(
-      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, TILE_LDS);
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, Whole::LDS_TURN);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3((uint32_t)n), dim3(256), TILE_LDS, stream, p);
+  hipLaunchKernelGGL(fn, dim3((uint32_t)n), dim3(256), Whole::LDS_TURN, stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }

@@ -246,10 +246,11 @@ int lds_linear_rows_parts(int M, int N, int K) {
 //     a K below 1600 takes up to 3 us more here, 688 -> 1680, 256 rows 13 / 10;
 //     that it comes out as a single row does is worth it.)
 //   one part, and gated ones (there with their activation): if the workgroups
-//     fill at least 7/8 of their rounds, up to 128 rows, gated up to 192. 4096 -> 32768: 32 rows
+//     fill at least 7/8 of their rounds, plain up to 128 rows. 4096 -> 32768: 32 rows
 //     46 / 62, 128 rows 55 / 64, 160 rows 66 / 67; -> 128256 (98 %): 64 rows
 //     182 / 208; 5120 -> 51200 (78 %): 64 rows 110 / 98. 4096 -> [2 x 14336]:
-//     64 rows 44 / 58, 128 rows 53 / 60, 192 rows 65 / 67, 256 rows 78 / 72;
+//     64 rows 44 / 58, 128 rows 53 / 60, 192 rows 65 / 67, 256 rows 69 / 75 (by
+//     linear_wide, for K from 1024 on in whole steps);
 //     inside a 4-layer stack of about 180 rows the pass takes 790 / 835;
 //     2048 -> [2 x 4096] (25 %): 32 rows 18 / 16.
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
@@ -263,7 +264,9 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   if (parts && n > 1) return 1;
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
-  if (gated || N > 128 * 128) return full && M <= (gated ? 192 : 128);
+  if (gated)
+    return full && (M <= 192 || (K >= 1024 && K % KS == 0));
+  if (N > 128 * 128) return full && M <= 128;
   if (full) return M <= 64 || K >= 4096;
   return M <= 64 && N <= 4096;
 }

@@ -20,10 +20,9 @@
 // 50), 256 rows 111 (260). Above 128 rows matrix cores and LDS bound it (with
 // one row of x and of w repeated, nothing to fetch, 256 rows 64 of 75 us).
 #include "layered/elem.h"
+#include "tile_core.h"
 
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 struct Tiles {
   const short *x, *w;        // [M, K], [N, K] (GATED: [2 N, K], gate first)
@@ -31,12 +30,25 @@ struct Tiles {
   void* y;                   // [M, N]; F32: [parts, M, N] 32-bit
   int M, N, K, k_part;       // k_part: K per part, a multiple of 2 KS
   int parts, act;
+  uint32_t x_bytes, w_bytes; // linear_wide
 };
 
 enum Out { BF16, F32, GATED };
 
 constexpr int NW = 8, KS = 64, BN = 128;      // BN: rows of w per workgroup
 constexpr int ROW = KS * 2;                   // bytes of a row in LDS
+
+// The order of linear_rows.hip: steps of 128, starting at one by the channels.
+template <int OUT>
+__device__ __forceinline__ int start(int blk, int N, int steps) {
+  return (OUT == GATED    ? blk * 6
+          : N > 128 * 256 ? blk / 2 * 3
+                          : blk * 3) %
+         (steps / 2) * 2;
+}
+
+// 128 channels by 256 rows, a ring of three steps
+typedef TileCore<4, 8, 2, 3> Wide;
 
 // what is past the end of K
 __device__ const float4v zeros = {0.f, 0.f, 0.f, 0.f};
@@ -55,12 +67,8 @@ __global__ __launch_bounds__(NW * WAVE, 2) void linear_tiles_kernel(
   const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
   const int part = blockIdx.x % p.parts, blk = blockIdx.x / p.parts;
   const int k_lo = part * p.k_part, k_hi = min(p.K, k_lo + p.k_part);
-  // the order of linear_rows.hip: steps of 128, starting at one by its channels
   const int steps = (k_hi - k_lo + 2 * KS - 1) / (2 * KS) * 2;
-  const int first = (OUT == GATED      ? blk * 6
-                     : p.N > 128 * 256 ? blk / 2 * 3
-                                       : blk * 3) %
-                    (steps / 2) * 2;
+  const int first = start<OUT>(blk, p.N, steps);
   const int M = p.M, N = p.N;
 
   // A load takes 8 rows of KS, 8 pieces of 16 bytes each; the pieces of a row
@@ -197,6 +205,80 @@ __global__ __launch_bounds__(NW * WAVE, 2) void linear_tiles_kernel(
     }
 }
 
+// From 193 rows on, K in parts of 1024 and more, multiples of 128: 128 rows of w by
+// all of x in four waves, by the loop of tile_core.h. The matrix cores are 75 %
+// busy, but they and the stream of weights together take the clock down to 1.25 to
+// 1.9 GHz: 4096 -> 28672, gated, 256 rows 69 us (78 above; library 65 to 69 and 6
+// for the activation), 14336 -> 4096 37 (41), 4096 -> 12576 37 (42), of 5120 ->
+// 10240 38 (42). Shorter parts end sooner in eight waves (4096 -> 4096, 512 each:
+// 18 us for 20), as do 192 rows and fewer (a stack of 178: 795 us a pass for 814).
+template <int OUT>
+__global__ __launch_bounds__(256, 1) void linear_wide_kernel(const Tiles p) {
+  extern __shared__ __align__(16) short wide_lds[];
+  constexpr int LW = Wide::LW, LP = Wide::LP, QC = Wide::QC;
+  Wide core;
+  const int part = blockIdx.x % p.parts, blk = blockIdx.x / p.parts;
+  const int k_lo = part * p.k_part, M = p.M, N = p.N;
+  const int steps = (min(p.K, k_lo + p.k_part) - k_lo) / KS;
+  const int first = start<OUT>(blk, N, steps);
+  uint32_t wsrc[2][LW], xsrc[2][LP];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int j = 0; j < LW; ++j) {
+      const int r = core.loaded<LW>(j);
+      const int n = OUT == GATED ? h * N + min(blk * Wide::CH + r, N - 1)
+                                 : min(blk * BN + h * Wide::CH + r, N - 1);
+      wsrc[h][j] = (uint32_t)(n * p.w_row + core.piece<LW>(j)) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < LP; ++j)
+      xsrc[h][j] =
+          (uint32_t)(min(h * Wide::RH + core.loaded<LP>(j), M - 1) *
+                         p.x_row + core.piece<LP>(j)) * 2;
+  }
+  core.run(wide_lds, p.w, p.w_bytes, wsrc, p.x, p.x_bytes, xsrc, steps,
+           [&](int s) {
+             s += first;
+             return (k_lo + (s >= steps ? s - steps : s) * KS) * 2;
+           });
+#pragma unroll
+  for (int t = 0; t < Wide::ROWS / 32; ++t) {
+    const int m = core.row(t) + core.col;
+    if (m >= M) continue;
+    const int64_t o = ((int64_t)part * M + m) * N;
+#pragma unroll
+    for (int c = 0; c < (OUT == GATED ? QC : 2 * QC); ++c) {
+      const int n =
+          blk * (OUT == GATED ? Wide::CH : BN) + core.channel(c) + core.grp * 4;
+      if (n >= N) continue;           // N is a multiple of 4
+      float4v v = core.acc[c][t];
+      if constexpr (OUT == F32) {
+        *(float4v*)((float*)p.y + o + n) = v;
+      } else {
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          v[x] = activate(p.act, v[x]) * core.acc[c + QC][t][x];
+        *(bf16x4*)((short*)p.y + o + n) = __builtin_convertvector(v, bf16x4);
+      }
+    }
+  }
+}
+
+template <int OUT>
+hipError_t go_wide(const Tiles& p, hipStream_t stream) {
+  constexpr int width = OUT == GATED ? BN / 2 : BN;
+  auto fn = linear_wide_kernel<OUT>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+      Wide::LDS);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3((p.N + width - 1) / width * p.parts), dim3(256),
+                     Wide::LDS, stream, p);
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
 template <int MT, int OUT>
 hipError_t go(const Tiles& p, hipStream_t stream) {
   constexpr int width = OUT == GATED ? BN / 2 : BN;
@@ -212,7 +294,17 @@ hipError_t go(const Tiles& p, hipStream_t stream) {
 }
 
 template <int OUT>
-hipError_t go_rows(const Tiles& p, hipStream_t stream) {
+hipError_t go_rows(Tiles p, hipStream_t stream) {
+  const int64_t xb = ((p.M - 1) * p.x_row + p.K) * 2;
+  const int64_t wb =
+      (((OUT == GATED ? 2 : 1) * (int64_t)p.N - 1) * p.w_row + p.K) * 2;
+  // (products of one part that are not gated go to the library)
+  if (OUT != BF16 && p.M > 192 && p.k_part >= 1024 && p.K % (2 * KS) == 0 &&
+      xb < 1ll << 32 && wb < 1ll << 32) {
+    p.x_bytes = (uint32_t)xb;
+    p.w_bytes = (uint32_t)wb;
+    if constexpr (OUT != BF16) return go_wide<OUT>(p, stream);
+  }
   if (p.M <= 64) return go<1, OUT>(p, stream);
   if (p.M <= 128) return go<2, OUT>(p, stream);
   if (p.M <= 192) return go<3, OUT>(p, stream);

@@ -64,6 +64,32 @@ def test_gated(name, rows, n, k):
             _same(y, fn(g) * u, 8)
 
 
+@pytest.mark.parametrize("rows", [192, 193, 255, 256])
+@pytest.mark.parametrize("n,k,parts", [(4088, 8320, 8), (7304, 4224, 4),
+                                       (7304, 4232, 4), (12576, 2048, 2)])
+def test_parts_of_many_steps(rows, n, k, parts):
+    """Ends of rows, channels and K of the loop for large parts (its K is a
+    multiple of 128), and the bits of a row alone."""
+    ext = _ext("_hip_ops")
+    x, w = _draw(rows, k, seed=rows), _draw(n, k, seed=n, scale=k ** -0.5)
+    y = ext.linear_parts(x, w)
+    assert y.shape == (parts, rows, n) and y.dtype == torch.float32
+    _same(y.sum(0), x.double() @ w.double().t(), 12)
+    assert torch.equal(y[:, -1:], ext.linear_parts(x[-1:], w))
+
+
+@pytest.mark.parametrize("rows", [193, 256])
+@pytest.mark.parametrize("n,k", [(14400, 1024), (16368, 1152), (14400, 1096)])
+def test_gated_of_many_steps(rows, n, k):
+    x, w = _draw(rows, k, seed=rows), _draw(2 * n, k, seed=n, scale=k ** -0.5)
+    y = _ext("_hip_ops").gated_linear(x, w, 1)
+    assert (y is None) == (k % 128 > 0)
+    if y is not None:
+        g, u = (x.double() @ w.double().t()).chunk(2, -1)
+        _same(y, torch.nn.functional.silu(g) * u, 8)
+        assert torch.equal(y[-1:], _ext("_hip_ops").gated_linear(x[-1:], w, 1))
+
+
 @pytest.mark.parametrize("rows,n,k,whole", [
     (2047, 4096, 4096, 0), (4096, 4096, 4096, 0), (4097, 4096, 96, 4096),
     (4096 + 2048, 4096, 96, 4096), (4096 + 2049, 4096, 96, 0),
