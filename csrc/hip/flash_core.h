@@ -1,15 +1,17 @@
 // flash_core.h — the part that the prefill attention kernels share: a wave's
-// 32 query rows against 32 keys in LDS, with an online softmax per query.
+// 32 query rows against 32 or 64 keys in LDS, with an online softmax per query.
 //
 // S' = K Q' on 32x32x16 tiles leaves lane (column c, half h) with the scores
 // of query c for keys (r & 3) + 8 (r >> 2) + 4 h, r = 0..15. The order of the
 // keys inside a step of O' = V' P' is free, so the probabilities of registers
 // 8 s .. 8 s + 7 are step s's operand as they are, and V' is read in the same
 // order: rows 16 s + 4 h .. + 3 and + 8 .. + 11. Nothing crosses the wave but
-// the maximum. What bounds the kernels is the vector work per score, so each
-// has one multiply-add, one exponential (the scale is in the multiply-add),
-// half a pack, and its shares of the maximum and the sum: about as many cycles
-// as the matrix cores need.
+// the maximum. Each score has one multiply-add, one exponential (the scale is in
+// the multiply-add), half a pack, and its shares of the maximum and the sum: two
+// thirds of the cycles that the matrix cores need, which the other wave of a SIMD
+// fills. LDS reads run a fixed number of operands ahead of their instructions, in
+// an order that is written out: left to the compiler, each operand of K was waited
+// for before the next was asked for.
 #pragma once
 #include "hip_common.h"
 
@@ -22,6 +24,12 @@ typedef __attribute__((ext_vector_type(4))) unsigned int uint4v;
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float NEG = -1e30f;
+
+// |scale| in log2 units. Not 0, which makes nothing of a masked -infinity: scores
+// below 1e30 come out all alike by this one as well.
+__device__ __forceinline__ float log2_scale(float scale) {
+  return fmaxf(fabsf(scale) * LOG2E, 1e-37f);
+}
 
 __device__ __forceinline__ unsigned int pack2(float a, float b) {
   const float2v v = {a, b};
@@ -56,39 +64,99 @@ struct Softmax {
   }
 };
 
-// NK = key channels / 16, NV = value channels / 32.
-//   key(kk)        16 bytes of key row (lane & 31), channels 16 kk + 8 half ..
-//   value(row, t)  address of the lane's 8 bytes of value row `row`: channels
-//                  32 t + 16 (lane / 16 & 1) + 4 (lane & 3) ..; row is this
-//                  lane's of the four that a transposing read covers
-//   FINE           probabilities as the sum of two bf16 (2^-17 of their size
-//                  off, as good as the 32-bit ones of the decode kernel)
-//   inside         every lane's query sees all 32 keys; else those with
-//                  first <= key <= last, relative to the tile
-// scale_log2 >= 0.
-template <int NK, int NV, bool FINE, class Key, class Value>
-__device__ __forceinline__ void attend32(Key key, Value value,
-                                         const bf16x8* qf, float scale_log2,
-                                         bool inside, int first, int last,
-                                         Softmax& st, f32x16* acc) {
+// the larger of three; a is known to come from a vector instruction (which the
+// compiler keeps apart from the matrix instruction that gave b and c)
+__device__ __forceinline__ float max3(float a, float b, float c) {
+  asm("v_max3_f32 %0, %0, %1, %2" : "+v"(a) : "v"(b), "v"(c));
+  return a;
+}
+
+// SUB x 32 keys. NK = key channels / 16, NV = value channels / 32.
+//   key(u, kk)        16 bytes of key row 32 u + (lane & 31), channels 16 kk + 8
+//                     half ..
+//   value(u, row, t)  address of the lane's 8 bytes of value row 32 u + row:
+//                     channels 32 t + 16 (lane / 16 & 1) + 4 (lane & 3) ..; row is
+//                     this lane's of the four that a transposing read covers
+//   FINE              probabilities as the sum of two bf16 (2^-17 of their size
+//                     off, as good as the 32-bit ones of the decode kernel)
+//   inside            every lane's query sees all keys; else those with
+//                     first <= key <= last, relative to the tile
+//   between(i)        what goes between the NK SUB matrix instructions of the
+//                     scores: the caller's loads of later tiles, which in a row
+//                     would hold the wave up
+// scale_log2 > 0: log2_scale.
+template <int NK, int NV, int SUB, bool FINE, class Key, class Value,
+          class Between>
+__device__ __forceinline__ void attend(Key key, Value value, const bf16x8* qf,
+                                       float scale_log2, bool inside, int first,
+                                       int last, Softmax& st, f32x16* acc,
+                                       Between between) {
   const int lane = threadIdx.x % WAVE, hi = lane >> 5;
-  f32x16 s = (f32x16)(0.f);
+  // operands read ahead, as many as the registers hold
+  constexpr int AHEAD = NK <= 8 && NV <= 4 ? 8 : 4;
+  f32x16 s[SUB];
 #pragma unroll
-  for (int kk = 0; kk < NK; ++kk)
-    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(key(kk), qf[kk], s, 0, 0, 0);
-  if (!inside) {
+  for (int u = 0; u < SUB; ++u) s[u] = (f32x16)(0.f);
+  {
+    constexpr int N = NK * SUB;
+    bf16x8 kf[AHEAD];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int t = (r & 3) + 8 * (r >> 2) + 4 * hi;
-      if (t < first || t > last) s[r] = -INFINITY;
+    for (int i = 0; i < (N < AHEAD ? N : AHEAD); ++i)
+      kf[i] = key(i % SUB, i / SUB);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      s[i % SUB] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          kf[i % AHEAD], qf[i / SUB], s[i % SUB], 0, 0, 0);
+      if (i + AHEAD < N)
+        kf[i % AHEAD] = key((i + AHEAD) % SUB, (i + AHEAD) / SUB);
+      between(i);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
-  float mx = fmaxf(s[0], s[1]);
+  // operand (k, t) of V': step k of 16 keys, 32 channels
+  const int row = 4 * hi + lane % 16 / 4;
+  auto operand = [&](int i) {
+    const int k = i / NV, t = i % NV;
+    typedef __attribute__((address_space(3))) short4v lds4;
+    const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds4*)value(k / 2, k % 2 * 16 + row, t));
+    const short4v up = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds4*)value(k / 2, k % 2 * 16 + row + 8, t));
+    const short8 v = {lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
+    return __builtin_bit_cast(bf16x8, v);
+  };
+  // half of the operands read ahead come in while the softmax runs, the others
+  // once its registers are free
+  constexpr int N = NV * 2 * SUB;
+  bf16x8 vf[AHEAD];
 #pragma unroll
-  for (int r = 2; r < 16; r += 2) mx = fmaxf(mx, fmaxf(s[r], s[r + 1]));
-  mx = max_halves(mx);
+  for (int i = 0; i < AHEAD / 2; ++i) vf[i] = operand(i);
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (!inside) {
+#pragma unroll
+    for (int u = 0; u < SUB; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int t = u * 32 + (r & 3) + 8 * (r >> 2) + 4 * hi;
+        if (t < first || t > last) s[u][r] = -INFINITY;
+      }
+  }
+  float mx[SUB];
+#pragma unroll
+  for (int u = 0; u < SUB; ++u) {
+    mx[u] = fmaxf(s[u][0], s[u][1]);
+#pragma unroll
+    for (int r = 2; r < 16; r += 2) mx[u] = max3(mx[u], s[u][r], s[u][r + 1]);
+  }
+  float largest = mx[0];
+#pragma unroll
+  for (int u = 1; u < SUB; ++u) largest = fmaxf(largest, mx[u]);
+  largest = max_halves(largest);
   // without a key so far m stays at NEG and every exponent underflows to 0
-  const float top = mx == -INFINITY ? NEG : mx * scale_log2;
+  const float top = largest == -INFINITY ? NEG : largest * scale_log2;
   // The largest probability is exactly 1, which bf16 holds: to let the maximum
   // lag behind would spare rescaling and cost precision (5 % more error).
   if (__any(top > st.m)) {
@@ -101,28 +169,27 @@ __device__ __forceinline__ void attend32(Key key, Value value,
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[t][e] *= alpha;
   }
-  if (inside) {
+#pragma unroll
+  for (int u = 0; u < SUB; ++u)
 #pragma unroll
     for (int r = 0; r < 16; ++r)
-      s[r] = __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2, -st.m));
-  } else {
+      s[u][r] = __builtin_amdgcn_exp2f(fmaf(s[u][r], scale_log2, -st.m));
+  float sum[SUB];
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
-      s[r] = s[r] == -INFINITY
-                 ? 0.f
-                 : __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2, -st.m));
+  for (int u = 0; u < SUB; ++u) {
+    sum[u] = s[u][0] + s[u][1];
+#pragma unroll
+    for (int r = 2; r < 16; r += 2) sum[u] += s[u][r] + s[u][r + 1];
+    st.l += sum[u];
   }
-  float sum = s[0] + s[1];
+  bf16x8 pf[2 * SUB], pr[2 * SUB];
 #pragma unroll
-  for (int r = 2; r < 16; r += 2) sum += s[r] + s[r + 1];
-  st.l += sum;
-  bf16x8 pf[2], pr[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
+  for (int k = 0; k < 2 * SUB; ++k) {
     uint4v w, v;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float a = s[8 * k + 2 * i], b = s[8 * k + 2 * i + 1];
+      const float a = s[k / 2][k % 2 * 8 + 2 * i];
+      const float b = s[k / 2][k % 2 * 8 + 2 * i + 1];
       const unsigned int ab = pack2(a, b);
       w[i] = ab;
       if (FINE) {
@@ -134,24 +201,21 @@ __device__ __forceinline__ void attend32(Key key, Value value,
     pf[k] = __builtin_bit_cast(bf16x8, w);
     if (FINE) pr[k] = __builtin_bit_cast(bf16x8, v);
   }
-  const int row = 4 * hi + lane % 16 / 4;
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int t = 0; t < NV; ++t)
+  for (int i = AHEAD / 2; i < (N < AHEAD ? N : AHEAD); ++i) vf[i] = operand(i);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      typedef __attribute__((address_space(3))) short4v lds4;
-      const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (lds4*)value(16 * k + row, t));
-      const short4v up = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (lds4*)value(16 * k + row + 8, t));
-      const short8 vf = {lo[0], lo[1], lo[2], lo[3],
-                         up[0], up[1], up[2], up[3]};
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-          __builtin_bit_cast(bf16x8, vf), pf[k], acc[t], 0, 0, 0);
-      if constexpr (FINE)
-        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-            __builtin_bit_cast(bf16x8, vf), pr[k], acc[t], 0, 0, 0);
-    }
+  for (int i = 0; i < N; ++i) {
+    const int k = i / NV, t = i % NV;
+    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % AHEAD], pf[k],
+                                                     acc[t], 0, 0, 0);
+    if constexpr (FINE)
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i % AHEAD], pr[k],
+                                                       acc[t], 0, 0, 0);
+    if (i + AHEAD < N) vf[i % AHEAD] = operand(i + AHEAD);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 }  // namespace flash

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
     const uint4v v = *(const uint4v*)(q + q_row * D + kk * 16 + hi * 8);
     qf[kk] = __builtin_bit_cast(bf16x8, v ^ flip);
   }
-  const float scale_log2 = fabsf(scale) * LOG2E;
+  const float scale_log2 = log2_scale(scale);
 
   Softmax st;
   f32x16 acc[D / 32];
@@ -153,16 +153,16 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
       if (sub0 >= kv_end_w) break;          // beyond this wave's horizon
       const char* kb = (const char*)k_lds + 32 * half * 256;
       const char* vb = (const char*)v_lds + 32 * half * 256;
-      attend32<D / 16, D / 32, false>(
-          [&](int kk) {
+      attend<D / 16, D / 32, 1, false>(
+          [&](int, int kk) {
             return *(const bf16x8*)(kb + qcol * 256 +
                                     ((kk * 32 + hi * 16) ^ swizzle(qcol)));
           },
-          [&](int row, int t) {
+          [&](int, int row, int t) {
             return vb + row * 256 + ((t * 64 + v_col) ^ swizzle(row));
           },
           qf, scale_log2, sub0 + 31 <= prior + first_w, 0, prior + p - sub0,
-          st, acc);
+          st, acc, [](int) {});
     }
   }
   st.l = st.join();

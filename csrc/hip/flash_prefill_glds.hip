@@ -1,21 +1,18 @@
-// flash_prefill_glds.hip — the bf16-KV variant of the fused MFMA prefill
-// attention with a glds staging pipeline: K/V tiles are DMA'd straight to LDS
-// (`global_load_lds`) into a ring, ahead of their use, with COUNTED
-// `s_waitcnt vmcnt(N)` (hipcc drains glds at any ordinary in-loop global load,
-// so the block table is staged into LDS up front and the hot loop touches
-// global memory ONLY through glds). The LDS image stays lane-linear (a glds
-// constraint); the XOR bank swizzle is applied by permuting the per-lane
-// SOURCE addresses. The attention of a tile is flash_core.h's.
+// flash_prefill_glds.hip — prefill attention of bf16 caches: tiles of keys and
+// values go through registers into LDS, two of them there, a third on its way. The
+// attention of a tile is flash_core.h's; the tiles' loads and LDS writes stand
+// between its matrix instructions (in a row they hold a wave up for 1200 cycles of
+// 4900 per 64 keys). Loads straight to LDS are not used: the compiler waits for all
+// of them ahead of each transposing read.
 //
 // A workgroup has 4 waves and one of two shapes:
-//   rows   128 query rows, 32 per wave; all waves share tiles of 32 keys in a
-//          3-deep ring, two tiles ahead. Order: [counted vmcnt][raw barrier]
-//          [compute tile n][issue tile n+2] — barrier n separates every wave's
-//          last read of buffer (n-1)%3 from its rewrite for tile n+2.
-//   keys   32 query rows; every wave takes each fourth tile of keys through a
-//          2-deep ring of its own, without barriers, and the waves' results
-//          meet in LDS at the end. Four times the workgroups, half the serial
-//          chain, one workgroup per compute unit (132 KB of LDS).
+//   rows   128 query rows, 32 per wave; all waves share tiles of 64 keys, with
+//          one barrier per tile: it stands between the last read of a tile and
+//          the writes of the one after the next.
+//   keys   32 query rows; every wave takes each fourth tile of 32 keys through LDS
+//          of its own, without barriers, and the waves' results meet in LDS at
+//          the end. Four times the workgroups, half the serial chain, one
+//          workgroup per compute unit (132 KB of LDS).
 // Where the workgroups of the first shape leave compute units idle, one of the
 // two takes the call by its work (see prefill_shape in ops/dispatch.py), and
 // probabilities keep 17 bits in both: the matrix cores have the time, and a
@@ -24,30 +21,32 @@
 // keys and values of one. Tiles run from the last to the first: under the
 // causal mask the last of a sequence has the most keys.
 //
-// Measured (groups of 4, 8 key heads, alone; before: masks, packing and
-// rescaling of every tile on the vector units): one prompt of 7900 tokens 650
-// us, 785 TFLOP/s (before 1170); 8 of 1000 135 us (265); in a pass of layers one
-// of 8190 takes 812, 676 TFLOP/s. By keys / by rows with 17 bits (with 8): 150
-// tokens behind 1000 24 / 48 us (44; before 61); 500 behind 1000 52 / 66 (57;
-// 79); 600 behind 4000 195 / 175 (159; 235); 12 prompts of 20 13 / 7 (6; 7).
+// What bounds it: per 64 keys the matrix cores work 1024 cycles for each of a
+// SIMD's two waves, of 4450 that a pass takes; the rest is the vector work of both
+// (650 to 850 cycles each), waits at the barrier, and the clock, which falls to 1.7
+// GHz over long prompts.
+// Measured (groups of 4, 8 key heads, alone; before: operands of K waited for one
+// by one, tiles of 32 keys in a ring of loads to LDS): one prompt of 7900 tokens
+// 553 us, 924 TFLOP/s (652); 8 of 1000 109 us (127). By keys / by rows with 17 bits
+// (with 8): 150 tokens behind 1000 17 / 35 us (30; before 21 / 45); 500 behind 1000
+// 40 / 47 (38; 49 / 59); 600 behind 4000 139 / 127 (102; 183 / 168); 12 prompts of
+// 20 12 / 7 (7).
 //
-// fp8 KV cannot ride glds (raw byte copy, no conversion point), so the fp8
-// path keeps the convert-on-stage kernel in flash_prefill.hip; the launcher in
-// ops.hip picks per cache dtype.
+// 8-bit caches take the kernel in flash_prefill.hip, which widens them; the
+// launcher in ops.hip picks per cache dtype.
 #include "flash_core.h"
+
+#include <type_traits>
 
 namespace {
 
 using namespace flash;
 
 constexpr int D = 128;
-constexpr int KVBLK = 32;    // tokens per KV tile (ring granularity)
+constexpr int tile_of(bool keys) { return keys ? 32 : 64; }   // tokens
 constexpr int NW = 4;
 constexpr int QROWS = 32;
 constexpr int BT_CAP = 1024;  // staged block-table entries (16K-token ctx)
-
-constexpr int TILE_BYTES = KVBLK * D * 2;        // of K, and of V
-constexpr int RING_ROWS = 3, RING_KEYS = 2;      // tiles per ring
 
 __device__ __forceinline__ void raw_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -55,13 +54,13 @@ __device__ __forceinline__ void raw_barrier() {
   asm volatile("" ::: "memory");
 }
 
-constexpr int lds_bytes(bool keys) {
-  return BT_CAP * 4 + 2 * TILE_BYTES * (keys ? RING_KEYS * NW : RING_ROWS);
+constexpr int lds_bytes(bool keys) {       // two tiles of keys and values
+  return BT_CAP * 4 + 4 * tile_of(keys) * D * 2 * (keys ? NW : 1);
 }
 
-// FINE: see attend32. SHIFT: block size 1 << shift; else any
+// FINE: see attend. SHIFT: block size 1 << shift; else any
 template <int QPG, bool KEYS, bool FINE, bool SHIFT>
-__global__ __launch_bounds__(NW * WAVE, KEYS ? 1 : 2)
+__global__ __launch_bounds__(NW * WAVE, 2)
 void flash_prefill_glds_kernel(
     const short* __restrict__ q, const short* __restrict__ k_cache,
     const short* __restrict__ v_cache,
@@ -69,6 +68,7 @@ void flash_prefill_glds_kernel(
     const int32_t* __restrict__ seq_meta, const int32_t* __restrict__ tiles,
     short* __restrict__ out, int n_tiles, int kvh, int bs, int shift,
     int max_blocks, float scale) {
+  constexpr int TILE = tile_of(KEYS), TILE_BYTES = TILE * D * 2;
   const int kh = blockIdx.x % kvh, at_tile = blockIdx.x / kvh;
   const int tile = n_tiles - 1 - at_tile / (KEYS ? NW : 1);
   const int sub = KEYS ? at_tile % NW : 0;
@@ -81,8 +81,6 @@ void flash_prefill_glds_kernel(
   const int n_q_heads = kvh * QPG;
   if (KEYS && vrow0 >= rows) return;            // workgroup-uniform
 
-  // ONE shared object (a second __shared__ symbol makes hipcc emit
-  // vmcnt(0) before every ds_read)
   extern __shared__ __align__(16) char lds_raw[];
   int32_t* bt_lds = (int32_t*)lds_raw;
 
@@ -93,7 +91,7 @@ void flash_prefill_glds_kernel(
   const int hi = lane >> 5;
   // a ring of this wave's, or of all waves'
   char* ring = lds_raw + BT_CAP * 4 +
-               (KEYS ? wave * RING_KEYS * 2 * TILE_BYTES : 0);
+               (KEYS ? wave * 4 * TILE_BYTES : 0);
 
   // rows past the last repeat it and are not stored
   const int w0 = vrow0 + (KEYS ? 0 : wave * QROWS);
@@ -108,10 +106,8 @@ void flash_prefill_glds_kernel(
   const int last_w = (min(w0 + QROWS, rows) - 1) / QPG;
   const int kv_end = prior + last_wg + 1;       // keys that a row here may see
   const int kv_end_w = w0 < rows ? prior + last_w + 1 : 0;
-  const int n_kv_tiles = (kv_end + KVBLK - 1) / KVBLK;
+  const int n_kv_tiles = (kv_end + TILE - 1) / TILE;
 
-  // ---- prologue: Q fragments + block table; every ordinary global load
-  //      completes before the first glds issues ----
   bf16x8 qf[D / 16];
   const unsigned int flip = scale < 0.f ? 0x80008000u : 0u;
 #pragma unroll
@@ -119,36 +115,60 @@ void flash_prefill_glds_kernel(
     const uint4v v = *(const uint4v*)(q + q_row * D + kk * 16 + hi * 8);
     qf[kk] = __builtin_bit_cast(bf16x8, v ^ flip);
   }
-  const float scale_log2 = fabsf(scale) * LOG2E;
-  auto page_of = [&](int t) { return SHIFT ? t >> shift : t / bs; };
-  const int n_bt = min(max_blocks, page_of(kv_end - 1) + 1);
+  const float scale_log2 = log2_scale(scale);
+  const int n_bt =
+      min(max_blocks, (SHIFT ? kv_end - 1 >> shift : (kv_end - 1) / bs) + 1);
   for (int i = tid; i < n_bt; i += NW * WAVE)
     bt_lds[i] = block_tables[(int64_t)seq * max_blocks + i];
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();  // publish bt_lds (no glds in flight yet)
+  __syncthreads();
 
-  // rows of a tile that a wave fetches, 4 per instruction
-  constexpr int LOADS = KVBLK / 4 / (KEYS ? 1 : NW);
-  auto stage = [&](int n, int buf) {
-    char* kb = ring + buf * 2 * TILE_BYTES;
-#pragma unroll
-    for (int j = 0; j < LOADS; ++j) {
-      const int part = (KEYS ? 0 : wave * LOADS) + j;
-      const int row = part * 4 + lane / 16;
-      const int src = lane % 16 ^ swizzle(row) >> 4;    // source-side swizzle
-      // keys past the last that is seen repeat it: no garbage bf16
-      const int t = min(n * KVBLK + row, kv_end - 1), pg = page_of(t);
-      const int at = t - (SHIFT ? pg << shift : pg * bs);
-      const int64_t base =
-          (((int64_t)bt_lds[pg] * kvh + kh) * bs + at) * D + src * 8;
-      typedef const __attribute__((address_space(1))) unsigned int gmem;
-      typedef __attribute__((address_space(3))) unsigned int smem;
-      __builtin_amdgcn_global_load_lds((gmem*)(k_cache + base),
-                                       (smem*)(kb + part * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(
-          (gmem*)(v_cache + base), (smem*)(kb + TILE_BYTES + part * 1024), 16,
-          0, 0);
+  // A tile goes through registers, one ahead of the two in LDS. A wave brings 4
+  // rows per load: all of one page where pages are multiples of 4, whose place
+  // lane g works out for load g. Rows past the last key that is seen repeat it: no
+  // garbage bf16.
+  constexpr int P = TILE / (KEYS ? 4 : 4 * NW);        // loads of a wave
+  short8 kn[P], vn[P];
+  uint64_t place = 0;
+  const int lrow = lane / 16, last = kv_end - 1;
+  const uint32_t page_bytes = (uint32_t)kvh * bs * D * 2;
+  const char* const k_head = (const char*)(k_cache + (int64_t)kh * bs * D);
+  const char* const v_head = (const char*)(v_cache + (int64_t)kh * bs * D);
+  auto token = [&](int n, int g) {
+    return n * TILE + (KEYS ? g * 4 : g * 4 * NW + wave * 4);
+  };
+  auto look = [&](int n) {
+    if constexpr (SHIFT) {
+      const int t = min(token(n, lane % P), last & ~3);
+      place = (uint64_t)(uint32_t)bt_lds[t >> shift] * page_bytes +
+              (uint32_t)(t & (bs - 1)) * (D * 2);
     }
+  };
+  auto fetch = [&](int n, int g) {
+    const int t0 = token(n, g);
+    uint64_t at;
+    uint32_t off;
+    if constexpr (SHIFT) {
+      at = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(place >> 32), g)
+               << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)place, g);
+      off = (min(lrow, max(last - t0, last & 3)) * D + lane % 16 * 8) * 2;
+    } else {
+      const int t = min(t0 + lrow, last), pg = t / bs;
+      at = ((uint64_t)(uint32_t)bt_lds[pg] * kvh * bs + (t - pg * bs)) * (D * 2);
+      off = lane % 16 * 16;
+    }
+    kn[g] = *(const short8*)(k_head + at + off);
+    vn[g] = *(const short8*)(v_head + at + off);
+  };
+  constexpr int GAP = (KEYS ? 4 : 4 * NW) * 256;       // between its loads' rows
+  const int row0 = (KEYS ? 0 : wave * 4) + lrow;
+  auto put = [&](int buf, int g) {
+    // (16 rows on, the swizzle is the same)
+    const int row = row0 + (KEYS ? g % 4 * 4 : 0);
+    char* to = ring + buf * 2 * TILE_BYTES + row0 * 256 + g * GAP +
+               ((lane % 16 * 16) ^ swizzle(row));
+    *(short8*)to = kn[g];
+    *(short8*)(to + TILE_BYTES) = vn[g];
   };
 
   Softmax st;
@@ -160,52 +180,62 @@ void flash_prefill_glds_kernel(
   const int i16 = lane % 16;
   const int k_row = qcol * 256, k_swz = swizzle(qcol);
   const int v_col = (16 * ((lane & 31) >> 4) + (i16 % 4) * 4) * 2;
-  auto compute = [&](int n, int buf) {
-    const int tile0 = n * KVBLK;
+  // Tile n from `buf`, while the next one of this wave leaves the registers and
+  // the one after it comes in.
+  auto step = [&](int n, int next2, int next3, auto buf_) {
+    constexpr int buf = decltype(buf_)::value;
+    if constexpr (!KEYS) raw_barrier();   // it is there; all are done with n - 1
+    if (!KEYS && n * TILE >= kv_end_w) {  // beyond what this wave's rows see
+#pragma unroll
+      for (int g = 0; g < P; ++g) {
+        put(buf ^ 1, g);
+        fetch(next2, g);
+      }
+      look(next3);
+      return;
+    }
+    const int tile0 = n * TILE;
     const char* kb = ring + buf * 2 * TILE_BYTES;
     const char* vb = kb + TILE_BYTES;
-    attend32<D / 16, D / 32, FINE>(
-        [&](int kk) {
-          return *(const bf16x8*)(kb + k_row +
+    attend<D / 16, D / 32, TILE / 32, FINE>(
+        [&](int u, int kk) {
+          return *(const bf16x8*)(kb + u * 32 * 256 + k_row +
                                   ((kk * 32 + hi * 16) ^ k_swz));
         },
-        [&](int row, int t) {
-          return vb + row * 256 + ((t * 64 + v_col) ^ swizzle(row));
+        [&](int u, int row, int t) {
+          return vb + (u * 32 + row) * 256 + ((t * 64 + v_col) ^ swizzle(row));
         },
-        qf, scale_log2, tile0 + KVBLK - 1 <= prior + first_w, 0,
-        prior + p - tile0, st, acc);
+        qf, scale_log2, tile0 + TILE - 1 <= prior + first_w, 0,
+        prior + p - tile0, st, acc,
+        [&](int i) {
+          constexpr int N = D / 16 * TILE / 32;
+          if (i * P % N == 0) {
+            put(buf ^ 1, i * P / N);
+            fetch(next2, i * P / N);
+          }
+          if (i == N - 1) look(next3);
+        });
   };
-
-  if constexpr (KEYS) {
-    // tiles wave, wave + NW, ..
-    const int mine = n_kv_tiles > wave ? (n_kv_tiles - wave + NW - 1) / NW : 0;
-    for (int i = 0; i < min(mine, RING_KEYS); ++i) stage(wave + i * NW, i);
-    for (int i = 0; i < mine; ++i) {
-      if (i + 1 < mine)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * LOADS) : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      compute(wave + i * NW, i % RING_KEYS);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads are done
-      if (i + RING_KEYS < mine)
-        stage(wave + (i + RING_KEYS) * NW, i % RING_KEYS);
+  // this wave's tiles: every NWth by keys
+  constexpr int EACH = KEYS ? NW : 1;
+  const int n0 = KEYS ? wave : 0;
+  if (n0 < n_kv_tiles) {
+    look(n0);
+#pragma unroll
+    for (int g = 0; g < P; ++g) fetch(n0, g);
+#pragma unroll
+    for (int g = 0; g < P; ++g) put(0, g);
+    if (n0 + EACH < n_kv_tiles) {
+      look(n0 + EACH);
+#pragma unroll
+      for (int g = 0; g < P; ++g) fetch(n0 + EACH, g);
+      look(n0 + 2 * EACH);
     }
-  } else {
-    stage(0, 0);
-    if (n_kv_tiles > 1) stage(1, 1);
-    int buf = 0, fill = 2;
-    for (int n = 0; n < n_kv_tiles; ++n) {
-      // tile n has landed when at most the NEXT tile's DMA remains in
-      // flight (counted per-wave wait; vmcnt retires in order)
-      if (n + 1 < n_kv_tiles)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(2 * LOADS) : "memory");
-      else
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      raw_barrier();
-      if (n * KVBLK < kv_end_w) compute(n, buf);
-      if (n + 2 < n_kv_tiles) stage(n + 2, fill);
-      buf = buf + 1 == RING_ROWS ? 0 : buf + 1;
-      fill = fill + 1 == RING_ROWS ? 0 : fill + 1;
+    for (int n = n0; n < n_kv_tiles; n += 2 * EACH) {
+      step(n, n + 2 * EACH, n + 3 * EACH, std::integral_constant<int, 0>{});
+      if (n + EACH < n_kv_tiles)
+        step(n + EACH, n + 3 * EACH, n + 4 * EACH,
+             std::integral_constant<int, 1>{});
     }
   }
   st.l = st.join();
@@ -281,7 +311,7 @@ extern "C" {
 // shape: 0 by rows, 1 by keys, 2 by rows with probabilities of 17 bits; below
 // 0, for callers that do not know the lengths: rows if these fill the chip,
 // else keys in one round of workgroups, or in two where prompts are long enough
-// to make up for the second (300 tokens behind 300 23 us by keys, 28 by rows; 4
+// to make up for the second (300 tokens behind 300 20 us by keys, 22 by rows; 4
 // x 100 13 and 10).
 hipError_t lds_flash_prefill_glds(
     const void* q, const void* k_cache, const void* v_cache,
@@ -302,7 +332,8 @@ hipError_t lds_flash_prefill_glds(
                                                         : 2;
   int shift = 0;
   while (1 << shift < bs && shift < 20) ++shift;
-  const bool pow2 = 1 << shift == bs;
+  const bool pow2 =
+      1 << shift == bs && bs >= 4 && (int64_t)kvh * bs * D * 2 < 1ll << 32;
 #define GO(QPG, KEYS, FINE, SHIFT)                                           \
   return go<QPG, KEYS, FINE, SHIFT>(q, k_cache, v_cache, block_tables, seq_meta,   \
                               tiles, out, n_tiles, kvh, bs, shift,           \

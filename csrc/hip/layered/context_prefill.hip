@@ -2,7 +2,8 @@
 // (bf16). A tile is 128 rows of (query, head): all heads of a key/value head
 // share its tiles of keys. Keys and values come from
 //   pages        grouped heads: cache rows [key | value], found through the
-//                block table a tile ahead
+//                block table a tile ahead (block sizes that are powers of two
+//                without divisions, which took as long as the scores)
 //   context rows latent attention: keys and values expanded from the latents
 //                of everything a portion may see, the rotated key part shared
 //                by all heads; a sequence's context row 0 sits at ctx.pos0
@@ -10,17 +11,24 @@
 // The attention of 32 queries and 32 keys is flash_core.h's: S' = K Q' keeps a
 // query per lane. Rows of the LDS tiles are padded instead of swizzled: 16
 // bytes for K (16-byte row reads hit distinct banks), 64 bytes for V (the
-// transposing reads of four rows do). The next tile waits in registers while
-// this one is computed. Tiles run from the last to the first: under the causal
-// mask the last of a sequence has the most keys.
+// transposing reads of four rows do). Two tiles are in LDS, a third on its way in
+// registers; its loads and LDS writes stand between the matrix instructions. Tiles
+// run from the last to the first: under the causal mask the last of a sequence has
+// the most keys.
+//
+// 7800 rows of 7 prompts behind 100 tokens, 32 heads of 128 on 8 key heads: 190 us
+// (232 with one tile in LDS, divisions and operands of K waited for one by one; 231
+// in tiles of 32 keys); 7750 rows of 8 prompts, 32 heads of 192 and 128: 171 us (226;
+// 253 in tiles of 64 keys, whose scores do not fit the registers beside a tile).
 #include "../flash_core.h"
 #include "elem.h"
+
+#include <type_traits>
 
 namespace {
 
 constexpr int NW = 4, NT = NW * WAVE;
 constexpr int QW = 32;          // query rows per wave
-constexpr int KB = 64;          // keys per tile
 
 using namespace flash;
 
@@ -33,24 +41,30 @@ struct Prefill {
   const int32_t* ctx;        // [n_seqs, 2] = first context row, its position
   // pages: rows of D + V elements from ka on
   const int32_t* block_tables;
-  int max_blocks, bs;
+  int max_blocks, bs, shift; // bs = 1 << shift; below 0: any
   int64_t page, head;        // strides of a page and of a head inside it
   const int32_t *seq_meta, *tiles;  // tiles [n, 2] = sequence, first query
   short* out;                // [rows, H V]
   int H, rep, D, rot, V, window;
-  float scale_log2, sink;    // sink: score (log2) of a key without a value
+  float scale, sink;         // sink: score (log2) of a key without a value
   int has_sink;
 };
+
+// keys per tile: as many as the registers hold scores of and a tile on its way
+constexpr int keys_of(int DK, int DV) { return DK + DV <= 256 ? 64 : 32; }
+constexpr int tile_of(int DK, int DV) {       // in LDS (shorts)
+  return keys_of(DK, DV) * (DK + 8 + DV + 32);
+}
 
 // grid (key/value heads, tiles)
 template <int DK, int DV, bool PAGED>
 __global__ __launch_bounds__(NT, DK + DV > 320 ? 1 : 2)
 void context_prefill_kernel(const Prefill a_) {
   constexpr int KS = DK + 8, VS = DV + 32;      // row strides in LDS (shorts)
-  constexpr int NK = DK / 32, NV = DV / 32;     // 16-byte pieces per thread
+  constexpr int KB = keys_of(DK, DV);
+  constexpr int NK = DK * KB / 8 / NT, NV = DV * KB / 8 / NT;   // loads
+  constexpr int TILE = tile_of(DK, DV);         // keys [KB][KS], values [KB][VS]
   extern __shared__ short lds[];
-  short* k_lds = lds;                           // [KB][KS]
-  short* v_lds = lds + KB * KS;                 // [KB][VS]
   const int kvh = blockIdx.x, rep = a_.rep;
   const int tile = gridDim.y - 1 - blockIdx.y;
   const int seq = a_.tiles[2 * tile], p0 = a_.tiles[2 * tile + 1];
@@ -72,8 +86,8 @@ void context_prefill_kernel(const Prefill a_) {
   const int window = a_.window;
 
   bf16x8 qf[DK / 16];
-  const unsigned int flip = a_.scale_log2 < 0.f ? 0x80008000u : 0u;
-  const float scale_log2 = fabsf(a_.scale_log2);
+  const unsigned int flip = a_.scale < 0.f ? 0x80008000u : 0u;
+  const float scale_log2 = log2_scale(a_.scale);
   {
     const short* qr = a_.q + (sq.row0 + p) * a_.q_row + h * QD;
 #pragma unroll
@@ -104,90 +118,129 @@ void context_prefill_kernel(const Prefill a_) {
   const int hi_w = pw0 <= p_last ? off + pw1 + 1 : 0;
   const int lo_w = first_key(pw0);
 
+  // A tile goes through registers: rows past the last key that is seen repeat it
+  // (they are masked), channels past the end are 0.
   short8 kn[NK], vn[NV];
-  int kp[PAGED ? NK : 1], vp[PAGED ? NV : 1];   // pages of a tile
+  int kp[PAGED ? NK : 1], vp[PAGED && DK != DV ? NV : 1];   // pages of a tile
+  const int shift = a_.shift, page_mask = bs - 1;
+  auto row_of = [&](int t0, int i, int per) {
+    return min(t0 + (tid + i * NT) / per, hi_wg - 1);
+  };
   auto find = [&](int t0) {
     if constexpr (PAGED) {
 #pragma unroll
       for (int i = 0; i < NK; ++i) {
-        const int t = t0 + (tid + i * NT) / (DK / 8);
-        kp[i] = t < hi_wg ? bt[t / bs] : 0;
+        const int t = row_of(t0, i, DK / 8);
+        kp[i] = bt[shift < 0 ? t / bs : t >> shift];
       }
+      if constexpr (DK != DV)
 #pragma unroll
-      for (int i = 0; i < NV; ++i) {
-        const int t = t0 + (tid + i * NT) / (DV / 8);
-        vp[i] = t < hi_wg ? bt[t / bs] : 0;
-      }
+        for (int i = 0; i < NV; ++i) {
+          const int t = row_of(t0, i, DV / 8);
+          vp[i] = bt[shift < 0 ? t / bs : t >> shift];
+        }
     }
   };
+  const short* const pages = a_.ka + kvh * a_.head;
   auto page_row = [&](int page, int t) {
-    return a_.ka + page * a_.page + kvh * a_.head + t % bs * (D + V);
+    const uint32_t at = (shift < 0 ? t % bs : t & page_mask) * (D + V);
+    return pages + ((uint64_t)(uint32_t)page * (uint64_t)a_.page + at);
   };
-  auto fetch = [&](int t0) {
-#pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int ch = tid + i * NT, row = ch / (DK / 8), d = ch % (DK / 8) * 8;
-      const int t = t0 + row;
+  // load i of the keys, then of the values
+  auto fetch = [&](int t0, int i) {
+    if (i < NK) {
+      const int t = row_of(t0, i, DK / 8), d = (tid + i * NT) % (DK / 8) * 8;
       kn[i] = (short8){0, 0, 0, 0, 0, 0, 0, 0};
-      if (t < hi_wg && d < QD) {
+      if (d < QD) {
         if constexpr (PAGED)
-          kn[i] = *(const short8*)(page_row(kp[i], t) + d);
+          kn[i] = *(const short8*)(page_row(kp[PAGED ? i : 0], t) + d);
         else
           kn[i] = *(const short8*)(
               d < D ? a_.ka + (ctx0 + t) * a_.ka_tok + kvh * a_.ka_head + d
                     : a_.kb + (ctx0 + t) * a_.kb_tok + (d - D));
       }
-    }
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int ch = tid + i * NT, row = ch / (DV / 8), d = ch % (DV / 8) * 8;
-      const int t = t0 + row;
+    } else {
+      i -= NK;
+      const int t = row_of(t0, i, DV / 8), d = (tid + i * NT) % (DV / 8) * 8;
       vn[i] = (short8){0, 0, 0, 0, 0, 0, 0, 0};
-      if (t < hi_wg && d < V) {
+      if (d < V) {
         if constexpr (PAGED)
-          vn[i] = *(const short8*)(page_row(vp[i], t) + D + d);
+          vn[i] = *(const short8*)(
+              page_row(DK == DV ? kp[PAGED ? i : 0]
+                                : vp[PAGED && DK != DV ? i : 0], t) + D + d);
         else
           vn[i] = *(const short8*)(a_.v + (ctx0 + t) * a_.v_tok +
                                    kvh * a_.v_head + d);
       }
     }
   };
+  auto put = [&](int buf, int i) {
+    short* to = lds + buf * TILE;
+    if (i < NK) {
+      const int ch = tid + i * NT;
+      *(short8*)(to + ch / (DK / 8) * KS + ch % (DK / 8) * 8) = kn[i];
+    } else {
+      i -= NK;
+      const int ch = tid + i * NT;
+      *(short8*)(to + KB * KS + ch / (DV / 8) * VS + ch % (DV / 8) * 8) = vn[i];
+    }
+  };
+  const int i16 = lane % 16;
+  // the tile at t0 from `buf`
+  auto compute = [&](int t0, int buf, auto between) {
+    const short* kb = lds + buf * TILE + qc * KS + hi * 8;
+    const short* vb = lds + buf * TILE + KB * KS + 16 * ((lane & 31) >> 4) +
+                      (i16 % 4) * 4;
+    attend<DK / 16, DV / 32, KB / 32, false>(
+        [&](int u, int kk) {
+          return *(const bf16x8*)(kb + u * 32 * KS + kk * 16);
+        },
+        [&](int u, int row, int t) {
+          return vb + (u * 32 + row) * VS + t * 32;
+        },
+        qf, scale_log2, t0 + KB - 1 <= off + pw0 && t0 >= first_key(pw1),
+        first_key(p) - t0, off + p - t0, st, acc, between);
+  };
+  auto skips = [&](int t0) { return t0 >= hi_w || t0 + KB <= lo_w; };
   find(lo_wg);
-  fetch(lo_wg);
-  find(lo_wg + KB);
-
-  for (int t0 = lo_wg; t0 < hi_wg; t0 += KB) {
-    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NK; ++i) {
-      const int ch = tid + i * NT;
-      *(short8*)(k_lds + ch / (DK / 8) * KS + ch % (DK / 8) * 8) = kn[i];
-    }
+  for (int i = 0; i < NK + NV; ++i) fetch(lo_wg, i);
+  // Two tiles in LDS: while one is computed, the next one leaves the registers
+  // and the one after it comes in, between the matrix instructions.
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int ch = tid + i * NT;
-      *(short8*)(v_lds + ch / (DV / 8) * VS + ch % (DV / 8) * 8) = vn[i];
-    }
-    __syncthreads();
-    if (t0 + KB < hi_wg) {
-      fetch(t0 + KB);
-      find(t0 + 2 * KB);
-    }
-
+  for (int i = 0; i < NK + NV; ++i) put(0, i);
+  if (lo_wg + KB < hi_wg) {
+    find(lo_wg + KB);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int sub = t0 + 32 * half;
-      if (sub >= hi_w || sub + 32 <= lo_w) continue;   // wave-uniform
-      const int i16 = lane % 16;
-      const short* kb = k_lds + (32 * half + qc) * KS + hi * 8;
-      const short* vb = v_lds + 32 * half * VS + 16 * ((lane & 31) >> 4) +
-                        (i16 % 4) * 4;
-      attend32<DK / 16, DV / 32, false>(
-          [&](int kk) { return *(const bf16x8*)(kb + kk * 16); },
-          [&](int row, int t) { return vb + row * VS + t * 32; }, qf,
-          scale_log2, sub + 31 <= off + pw0 && sub >= first_key(pw1),
-          first_key(p) - sub, off + p - sub, st, acc);
+    for (int i = 0; i < NK + NV; ++i) fetch(lo_wg + KB, i);
+    find(lo_wg + 2 * KB);
+  }
+  auto step = [&](int t0, auto buf_) {
+    constexpr int buf = decltype(buf_)::value;
+    lds_barrier();
+    if (skips(t0)) {                                 // wave-uniform
+#pragma unroll
+      for (int i = 0; i < NK + NV; ++i) {
+        put(buf ^ 1, i);
+        fetch(t0 + 2 * KB, i);
+      }
+      find(t0 + 3 * KB);
+      return;
     }
+    compute(t0, buf, [&](int m) {
+      constexpr int N = DK / 16 * KB / 32;           // matrix instructions
+#pragma unroll
+      for (int i = 0; i < NK + NV; ++i)
+        if (i * N / (NK + NV) == m) {
+          put(buf ^ 1, i);
+          fetch(t0 + 2 * KB, i);
+        }
+      if (m == N - 1) find(t0 + 3 * KB);
+    });
+  };
+  for (int t0 = lo_wg; t0 < hi_wg; t0 += 2 * KB) {
+    step(t0, std::integral_constant<int, 0>{});
+    if (t0 + KB < hi_wg) step(t0 + KB, std::integral_constant<int, 1>{});
   }
   st.l = st.join();
 
@@ -211,7 +264,7 @@ void context_prefill_kernel(const Prefill a_) {
 template <int DK, int DV, bool PAGED>
 hipError_t launch(const Prefill& a, int kv_heads, int n_tiles,
                   hipStream_t stream) {
-  const int lds = KB * (DK + 8 + DV + 32) * (int)sizeof(short);
+  const int lds = 2 * tile_of(DK, DV) * (int)sizeof(short);
   auto fn = context_prefill_kernel<DK, DV, PAGED>;
   hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -260,7 +313,7 @@ hipError_t lds_latent_prefill(const void* q, const void* kv, const void* lat,
   a.rot = rot;
   a.V = V;
   a.window = window;
-  a.scale_log2 = scale * LOG2E;
+  a.scale = scale;
   const int qd = D + rot;
 #define GO(DK)                                                                \
   return V <= 64 ? launch<DK, 64, false>(a, H, n_tiles, stream)               \
@@ -296,6 +349,7 @@ hipError_t lds_grouped_prefill(const void* q, int64_t q_stride,
   a.block_tables = block_tables;
   a.max_blocks = max_blocks;
   a.bs = bs;
+  a.shift = bs & bs - 1 ? -1 : __builtin_ctz(bs);
   a.head = (int64_t)bs * (D + V);
   a.page = G * a.head;
   a.seq_meta = seq_meta;
@@ -305,7 +359,7 @@ hipError_t lds_grouped_prefill(const void* q, int64_t q_stride,
   a.rep = H / G;
   a.D = D;
   a.V = V;
-  a.scale_log2 = scale * LOG2E;
+  a.scale = scale;
   a.has_sink = has_sink;
   a.sink = sink * LOG2E;
 #define GO(DK)                                                                \

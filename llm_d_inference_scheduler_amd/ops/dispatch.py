@@ -187,9 +187,9 @@ def prefill_shape(news: List[int], ctxs: List[int], group: int,
     """Shape of the prefill attention's workgroups (flash_prefill_glds.hip) for
     prompts of `news` tokens that end contexts of `ctxs`: 0 by rows, 1 by keys,
     2 by rows with probabilities of 17 bits. From 256 workgroups by rows on the
-    chip is full (1000 tokens behind 1000: 75 us by rows, 109 by keys). Below,
+    chip is full (1000 tokens behind 1000: 49 us by rows, 86 by keys). Below,
     the two with 17 bits are weighed in us, as measured: a workgroup by rows
-    takes 6 + 0.042 per key, one by keys 4.2 + 0.0167, one per compute unit,
+    takes 5 + 0.026 per key, one by keys 5 + 0.0107, one per compute unit,
     those with the most keys first. One round of these is always faster."""
     rows = sum(-(-n * group // 128) for n in news) * kv_heads
     if rows >= 256:
@@ -197,12 +197,12 @@ def prefill_shape(news: List[int], ctxs: List[int], group: int,
     some = [-(-n * group // 32) * kv_heads for n in news]
     if sum(some) <= 256:
         return 1
-    work = sum(k * (4.2 + 0.0167 * (c - n / 2))
+    work = sum(k * (5 + 0.0107 * (c - n / 2))
                for k, n, c in zip(some, news, ctxs)) / 256
-    least = 4.2 + 0.0167 * min(c - n for n, c in zip(news, ctxs))
+    least = 5 + 0.0107 * min(c - n for n, c in zip(news, ctxs))
     most = max(ctxs)
-    keys = 3 + max(4.2 + 0.0167 * most, work + 0.6 * least)
-    return 1 if keys <= 6 + 0.042 * most else 2
+    keys = 3 + max(5 + 0.0107 * most, work + 0.3 * least)
+    return 1 if keys <= 5 + 0.026 * most else 2
 
 
 def flash_prefill(q: torch.Tensor, k_cache: torch.Tensor,

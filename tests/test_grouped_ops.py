@@ -343,6 +343,31 @@ class TestExperts:
 
 
 @GPU
+@pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (192, 128), (64, 256)])
+@pytest.mark.parametrize("bs", [1, 5, 64])
+def test_prefill_in_other_pages(D, V, bs, monkeypatch):
+    """Where keys and values lie changes no bit: block sizes that are powers of
+    two and others, portions around tiles of 32 and 64 keys."""
+    run, H, G = ("cuda:0", torch.bfloat16), 8, 2
+    portions = [(0, 64), (31, 1), (200, 9), (63, 130), (0, 33)]
+    seqs = [(n, prior, 0) for prior, n in portions]
+    m, rows = meta(seqs, run)
+    pos = torch.cat([torch.arange(a, a + n) for a, n in portions]).int()
+    tiles = torch.tensor([(i, r) for i, (_, n) in enumerate(portions)
+                          for r in range(0, n, 32)], dtype=torch.int32)
+    proj = put(rnd(len(pos), H * D + G * (D + V), seed=3), run)
+    outs = []
+    for size in (16, bs):
+        monkeypatch.setitem(globals(), "BS", size)
+        cache, tables, _ = paged(run, G, D, V, [a + n for a, n in portions])
+        out = put(torch.full((len(pos), H * V), 7.0), run)
+        ops.grouped_prefill(proj, cache, pos.to(run[0]), rows, tables, 0, m,
+                            tiles.to(run[0]), H, D, D ** -0.5, 0.0, out)
+        outs.append(out)
+    assert torch.equal(*outs)
+
+
+@GPU
 def test_forms_agree_at_a_large_size():
     """The tiled products against the plain kernel."""
     dev, E, K, F, T, top = "cuda:0", 9, 512, 448, 1500, 3

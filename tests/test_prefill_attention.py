@@ -80,6 +80,18 @@ def test_pages_in_bf16(seqs, qpg, kvh, bs, keys):
                                       want)
 
 
+@pytest.mark.parametrize("bs", [1, 2, 4, 64])
+@pytest.mark.parametrize("keys", [0, 1, 2])
+def test_sizes_of_pages(bs, keys):
+    """Pages of less than a load's four rows, of as many, of a whole tile; last
+    tiles of one key, of up to three loads less, and of all."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case([(65, 0), (40, 21), (3, 125), (30, 34), (1, 256)], 4, 2,
+                       bs, False, D ** -0.5)
+    (_as_decoded if keys else _close)(ext.flash_prefill(*args, keys=keys),
+                                      want)
+
+
 @pytest.mark.parametrize("seqs", SEQS)
 @pytest.mark.parametrize("qpg,kvh", [(1, 3), (4, 2), (8, 1)])
 @pytest.mark.parametrize("bs", [16, 5])
