@@ -428,9 +428,12 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
   auto write = [&](auto act) {
 #pragma unroll
     for (int b = 0; b < PT / 2; ++b)
-      core.turn(
+      core.template turn<2 * Core::QC>(
           lds, b,
-          [&](float f, int t) { return UP ? activate(act, f * wt[t]) : f; },
+          [&](int c, int t, int x) {
+            const float f = core.acc[c][t][x];
+            return UP ? activate(act, f * wt[t]) : f;
+          },
           [&](int row, int i, int c, short8 v) {
             int64_t at = tile.y + i;
             if constexpr (!UP) at = __shfl(to[b / 2], b % 2 * 32 + row, WAVE);

@@ -1,0 +1,137 @@
+// linear_act.hip — y = act(x gate') * (x up') and y = act(x w') for many rows
+// (bf16, 32-bit sums): tiles of 256 weight rows by 256 rows of x by the loop of
+// tile_core.h, the activation in the sums' registers.
+//
+// The library's product of the same weights is 3 % faster, but its result, twice
+// as wide where a gate is in it, goes to memory and comes back for the activation:
+// a tenth of the product's time. A wave's channels of gate and up are the same ones,
+// 64 of the first and of the second half of the tile's weight rows, so that both
+// sums are in one lane.
+#include "layered/elem.h"
+#include "tile_core.h"
+
+namespace {
+
+typedef TileCore<8, 8, 2, 2> Whole;      // 256 rows
+typedef TileCore<4, 8, 4, 2> Half;       // the last tile, of up to 128
+constexpr int BC = Whole::CHANNELS, BR = Whole::ROWS;
+static_assert(Half::CHANNELS == BC && Half::CH == Whole::CH &&
+                  Half::LDS_TURN <= Whole::LDS_TURN,
+              "");
+constexpr int TG = 4;        // tiles of rows that walk the channels together
+
+struct Product {
+  const short *x, *w;        // [M, K], [N, K] (GATED: [2 N, K], gate first)
+  int64_t x_row, w_row;      // strides in elements
+  short* y;                  // [M, N]
+  int M, N, K, act;
+  uint32_t x_bytes, w_bytes;
+};
+
+// as activate() of elem.h, by the exponential and the reciprocal of the hardware:
+// a few 2^-24 of the result, which is rounded to 8 bits
+template <int ACT>
+__device__ __forceinline__ float act_f(float z) {
+  if (ACT == ACT_RELU_SQUARED) return z > 0.f ? z * z : 0.f;
+  if (ACT == ACT_SILU) return z * sigmoid_f(z);
+  return z * sigmoid_f(2.f * 0.7978845608028654f *
+                       (z + 0.044715f * z * z * z));
+}
+
+template <int ACT, bool GATED, typename Core>
+__device__ __forceinline__ void tile(const Product& p, short* lds, int m0, int blk) {
+  Core core;
+  constexpr int LW = Core::LW, LP = Core::LP, QC = Core::QC;
+  constexpr int PT = Core::ROWS / 16 / Core::WP;
+  const int M = p.M, N = p.N;
+  // rows and channels past the end repeat the last one and are dropped
+  uint32_t wsrc[2][LW], xsrc[2][LP];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int j = 0; j < LW; ++j) {
+      const int r = core.template loaded<LW>(j);
+      const int n = GATED ? h * N + min(blk * Core::CH + r, N - 1)
+                          : min(blk * BC + h * Core::CH + r, N - 1);
+      wsrc[h][j] = (uint32_t)(n * p.w_row + core.template piece<LW>(j)) * 2;
+    }
+#pragma unroll
+    for (int j = 0; j < LP; ++j) {
+      const int r = m0 + h * Core::RH + core.template loaded<LP>(j);
+      xsrc[h][j] = (uint32_t)(min(r, M - 1) * p.x_row +
+                              core.template piece<LP>(j)) * 2;
+    }
+  }
+  core.run(lds, p.w, p.w_bytes, wsrc, p.x, p.x_bytes, xsrc, p.K / TILE_K,
+           [](int s) { return s * TILE_K * 2; });
+  const int n0 = blk * (GATED ? Core::CH : BC);
+#pragma unroll
+  for (int b = 0; b < PT / 2; ++b)
+    core.template turn<GATED ? QC : 2 * QC>(
+        lds, b,
+        [&](int c, int t, int x) {
+          const float z = act_f<ACT>(core.acc[c][t][x]);
+          return GATED ? z * core.acc[GATED ? c + QC : c][t][x] : z;
+        },
+        [&](int, int r, int c, short8 v) {
+          if (m0 + r < M && n0 + c < N)         // N is a multiple of 8
+            *(short8*)(p.y + (int64_t)(m0 + r) * N + n0 + c) = v;
+        });
+}
+
+template <int ACT, bool GATED>
+__global__ __launch_bounds__(256, 1) void linear_act_kernel(const Product p) {
+  extern __shared__ __align__(16) short act_lds[];
+  // Workgroups go round the 8 XCDs in turn: each gets a contiguous share of the
+  // tiles, in which TG tiles of rows walk the channels together.
+  constexpr int width = GATED ? BC / 2 : BC;
+  const int nx = (p.N + width - 1) / width, ny = (p.M + BR - 1) / BR;
+  const int id = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+  if (id >= nx * ny) return;
+  const int g = id / (TG * nx), in = id % (TG * nx);
+  const int side = min(TG, ny - g * TG);
+  const int m0 = (g * TG + in % side) * BR, blk = in / side;
+  if (p.M - m0 > Half::ROWS)
+    tile<ACT, GATED, Whole>(p, act_lds, m0, blk);
+  else
+    tile<ACT, GATED, Half>(p, act_lds, m0, blk);
+}
+
+template <int ACT, bool GATED>
+hipError_t go(const Product& p, hipStream_t stream) {
+  constexpr int width = GATED ? BC / 2 : BC;
+  const int64_t n = (int64_t)((p.N + width - 1) / width) * ((p.M + BR - 1) / BR);
+  if (n > 1 << 24) return hipErrorInvalidValue;
+  auto fn = linear_act_kernel<ACT, GATED>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+      Whole::LDS_TURN);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3((uint32_t)((n + 7) / 8 * 8)), dim3(256),
+                     Whole::LDS_TURN, stream, p);
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
+}  // namespace
+
+// y [M, N] = act(x gate') * (x up') of w [2 N, K] = [gate; up], or (not gated)
+// act(x w') of w [N, K]; rows x_row and w_row apart, 16-byte aligned; K a multiple
+// of 64 from 128 on, N one of 8.
+extern "C" hipError_t lds_linear_act(const void* x, int64_t x_row,
+                                     const void* w, int64_t w_row, void* y,
+                                     int M, int N, int K, int act, int gated,
+                                     hipStream_t stream) {
+  const int64_t xb = ((M - 1) * x_row + K) * 2;
+  const int64_t wb = (((gated ? 2 : 1) * (int64_t)N - 1) * w_row + K) * 2;
+  if (M < 1 || N < 8 || N % 8 || K < 2 * TILE_K || K % TILE_K || x_row % 8 ||
+      w_row % 8 || act < 0 || act >= ACTS || xb >= 1ll << 32 || wb >= 1ll << 32)
+    return hipErrorInvalidValue;
+  const Product p{(const short*)x, (const short*)w, x_row, w_row, (short*)y,
+              M, N, K, act, (uint32_t)xb, (uint32_t)wb};
+#define GO(A) return gated ? go<A, true>(p, stream) : go<A, false>(p, stream)
+  if (act == ACT_SILU) GO(ACT_SILU);
+  if (act == ACT_RELU_SQUARED) GO(ACT_RELU_SQUARED);
+  GO(ACT_GELU_TANH);
+#undef GO
+}

@@ -1,6 +1,7 @@
-// linear_bind.h — torch binding of linear_rows.hip and linear_tiles.hip, shared
-// by the extensions. Products go to these kernels where their rule holds, else
-// to the library, of many rows in two calls where that is faster.
+// linear_bind.h — torch binding of linear_rows.hip, linear_tiles.hip and
+// linear_act.hip, shared by the extensions. Products go to these kernels where
+// their rule holds, else to the library, of many rows in two calls where that is
+// faster.
 #pragma once
 #include <torch/extension.h>
 #include <ATen/autocast_mode.h>
@@ -18,6 +19,8 @@ hipError_t lds_linear_rows(const void*, int64_t, const void*, int64_t, void*,
                            float*, int, int, int, int, int, hipStream_t);
 hipError_t lds_gated_rows(const void*, int64_t, const void*, int64_t, void*,
                           int, int, int, int, hipStream_t);
+hipError_t lds_linear_act(const void*, int64_t, const void*, int64_t, void*,
+                          int, int, int, int, int, hipStream_t);
 hipError_t lds_lay_weights(const float*, void*, int, int, hipStream_t);
 }
 
@@ -66,6 +69,29 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
          lds_linear_rows_takes((int)M, (int)(use == GATED ? N / 2 : N), (int)K,
                                use == GATED, use == PARTS) &&
          rows_of_16_bytes(x) && rows_of_16_bytes(w);
+}
+
+// Whether a product of many rows and its activation are one kernel
+// (linear_act.hip): where its tiles fill 7/10 of their rounds over the compute
+// units. us, library and activation / here, behind it how full: 4096 -> [2 x
+// 14336], 600 rows 149 / 165 (51 %), 1000 202 / 197 (85 %), 2000 383 / 358 (85 %),
+// 8190 1415 / 1298; 2048 -> [2 x 8192], 4200 rows 249 / 239 (82 %), 1000 68 / 51 (98
+// %); 5120 -> [2 x 25600], 1000 rows 528 / 441 (76 %); 4096 -> 7168, 3000 rows 168 /
+// 163 (64 %), 8190 376 / 352 (87 %); 2048 -> 4096, 8533 rows 138 / 137 (69 %), 6000
+// 102 / 94 (73 %), 4200 74 / 87 (51 %).
+inline bool many_rows(const Tensor& x, const Tensor& w, bool gated) {
+  if (!plain_matrices(x, w)) return false;
+  const int64_t M = x.size(0), K = x.size(1), across = gated ? 128 : 256;
+  const int64_t N = gated ? w.size(0) / 2 : w.size(0);
+  const int64_t limit = 1ll << 31;       // elements: offsets stay under 4 GiB
+  if (M <= 256 || K < 128 || K % 64 || N < 8 || N % 8 ||
+      (gated && w.size(0) % 2) || M >= limit / K || w.size(0) >= limit / K ||
+      !rows_of_16_bytes(x) || !rows_of_16_bytes(w) ||
+      M * x.stride(0) >= limit || w.size(0) * w.stride(0) >= limit)
+    return false;
+  const int64_t tiles = (M + 255) / 256 * ((N + across - 1) / across);
+  const int64_t rounds = (tiles + 255) / 256;
+  return M * N * 10 >= rounds * 256 * 256 * across * 7;
 }
 
 // Rows of a product of many that go in a call of their own: those that make up
@@ -163,10 +189,24 @@ inline c10::optional<Tensor> linear32(const Tensor& x, const Tensor& w) {
   return linear_rows(x, w, true);
 }
 
+inline Tensor linear_act(const Tensor& x, const Tensor& w, int64_t act,
+                         bool gated) {
+  const c10::DeviceGuard guard(x.device());
+  const int M = (int)x.size(0), K = (int)x.size(1);
+  const int N = (int)w.size(0) / (gated ? 2 : 1);
+  Tensor y = torch::empty({M, N}, x.options());
+  check(lds_linear_act(
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), M, N,
+      K, (int)act, gated,
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return y;
+}
+
 // act(x gate') * (x up') of w [2 N, K] = [gate; up]; None where the product
 // and the activation have to be two calls
 inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
                                           int64_t act) {
+  if (many_rows(x, w, true)) return linear_act(x, w, act, true);
   if (!few_rows(x, w, GATED)) return c10::nullopt;
   const c10::DeviceGuard guard(x.device());
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0) / 2;
@@ -175,6 +215,13 @@ inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
       x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), M, N,
       K, (int)act, at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
   return y;
+}
+
+// act(x w'), or None as above
+inline c10::optional<Tensor> activated_linear(const Tensor& x, const Tensor& w,
+                                              int64_t act) {
+  if (!many_rows(x, w, false)) return c10::nullopt;
+  return linear_act(x, w, act, false);
 }
 
 // drawn weights [in, out] in 32-bit -> [out, in] in bf16
@@ -201,6 +248,7 @@ inline void bind(pybind11::module& m) {
   m.def("linear32", &linear32, "the same with a 32-bit result, or None");
   m.def("gated_linear", &gated_linear,
         "act(x gate') * (x up') of w = [gate; up], or None");
+  m.def("activated_linear", &activated_linear, "act(x w'), or None");
   m.def("few_rows",
         [](const Tensor& x, const Tensor& w) { return few_rows(x, w, PLAIN); },
         "whether x @ w' takes the streaming kernel");

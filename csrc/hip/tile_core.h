@@ -49,7 +49,6 @@ struct TileCore {
   static_assert(CH % 32 == 0 && RH % 32 == 0 && RS >= 2, "");
   static constexpr int STEP = (CHANNELS + ROWS) * TILE_K;
   static constexpr int RING = RS * STEP;
-  static constexpr int G = 2 * CT;       // pieces of 8 channels of a wave's row
   // results that a wave turns round at a time: 32 rows
   static constexpr int TURN = 32 * 16 * CT;
   static constexpr int LDS = RING * (int)sizeof(short);
@@ -255,24 +254,27 @@ struct TileCore {
     if (s < steps) step(integral_constant<int, 0>{});
   }
 
-  // The results of rows row(2 b) to row(2 b + 1) + 15 as bf16, after f(sum, t)
-  // for those of row(t) + col. The wave's share of LDS behind the ring turns them
-  // round so that they leave in whole lines: store(row of the 32, row of the
-  // tile, channel of the tile, 8 values).
-  template <typename F, typename S>
+  // Results of rows row(2 b) to row(2 b + 1) + 15 and of the first NC tiles of
+  // channels, f(c, t, x) for what acc[c][t][x] stands for, as bf16. The wave's share
+  // of LDS behind the ring turns them round so that they leave in whole lines:
+  // store(row of the 32, row of the tile, channel of the tile, 8 values).
+  template <int NC, typename F, typename S>
   __device__ __forceinline__ void turn(short* lds, int b, F f, S store) const {
-    static_assert(QP % 2 == 0, "");
+    static_assert(QP % 2 == 0 && NC <= CT, "");
+    constexpr int G = 2 * NC;            // pieces of 8 channels in a row
+    static_assert(G == 16 || G == 8 || G == 4, "");
     short* mine = lds + RING + wave * TURN;
     auto place = [](int r, int g) {
-      return (r * G + (g ^ (G == 16 ? r & 15 : r / 2 & 7))) * 8;
+      return (r * G + (g ^ (G == 16 ? r & 15 : G == 8 ? r / 2 & 7 : r / 4 & 3))) *
+             8;
     };
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int c = 0; c < CT; ++c) {
+      for (int c = 0; c < NC; ++c) {
         float4v v;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = f(acc[c][2 * b + t][x], 2 * b + t);
+        for (int x = 0; x < 4; ++x) v[x] = f(c, 2 * b + t, x);
         *(bf16x4*)(mine + place(t * 16 + col, c * 2 + grp / 2) + grp % 2 * 4) =
             __builtin_convertvector(v, bf16x4);
       }

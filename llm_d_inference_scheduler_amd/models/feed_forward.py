@@ -9,7 +9,6 @@ from typing import Callable, Optional, Tuple
 import torch
 
 from ..ops import layered as ops
-from ..ops.layered import linear
 from .configs import ExpertsSpec, FeedForwardSpec, GatedSpec
 
 Output = Tuple[Optional[torch.Tensor], Optional[torch.Tensor]]
@@ -56,7 +55,7 @@ class Experts:
         if self.shared_up is None:
             return None, rows
         return ops.linear_parts(
-            ops.activate(linear(h, self.shared_up), s.act),
+            ops.activated_linear(h, self.shared_up, s.act),
             self.shared_down), rows
 
 

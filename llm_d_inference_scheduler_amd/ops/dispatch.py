@@ -53,7 +53,7 @@ def lay_weights(w: torch.Tensor) -> torch.Tensor:
 
 
 def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """silu(x gate') * (x up') of w = [gate; up], one call for few rows."""
+    """silu(x gate') * (x up') of w = [gate; up], mostly in one kernel."""
     if _use_hip(x):
         y = _ext.gated_linear(x, w, _SILU)
         if y is not None:

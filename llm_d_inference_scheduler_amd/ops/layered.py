@@ -48,6 +48,15 @@ def gated_linear(x, w, act):
     return gated_act(linear(x, w), act)
 
 
+def activated_linear(x, w, act):
+    """act(x @ w'), one kernel for many rows."""
+    if x.is_cuda:
+        y = hip_layered().activated_linear(x, w, ACTS[act])
+        if y is not None:
+            return y
+    return activate(linear(x, w), act)
+
+
 def linear32(x, w):
     """x @ w' with a 32-bit result."""
     if x.is_cuda:

@@ -62,6 +62,7 @@ hip_ops = cpp_extension.CUDAExtension(
         "csrc/hip/ops.hip",
         "csrc/hip/linear_rows.hip",
         "csrc/hip/linear_tiles.hip",
+        "csrc/hip/linear_act.hip",
         "csrc/hip/prefix_kernels.hip",
         "csrc/hip/norm_rope_act.hip",
         "csrc/hip/kv_cache.hip",
@@ -78,6 +79,7 @@ hip_layered = cpp_extension.CUDAExtension(
         "csrc/hip/layered/ops.hip",
         "csrc/hip/linear_rows.hip",
         "csrc/hip/linear_tiles.hip",
+        "csrc/hip/linear_act.hip",
         "csrc/hip/layered/residual_norm.hip",
         "csrc/hip/layered/delta_rule.hip",
         "csrc/hip/layered/delta_chunk.hip",

@@ -90,6 +90,46 @@ def test_gated_of_many_steps(rows, n, k):
         assert torch.equal(y[-1:], _ext("_hip_ops").gated_linear(x[-1:], w, 1))
 
 
+@pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("rows,n,k,one", [
+    (640, 10880, 128, True), (560, 10872, 192, True), (897, 8192, 320, True),
+    (1024, 8136, 256, True), (512, 16384, 64, False), (640, 10880, 136, False),
+    (512, 8192, 128, False)])
+def test_act_of_many_rows(name, gated, rows, n, k, one):
+    """Tiles of 256 rows and a last one of up to 128 or more, channels that end
+    inside a tile, even and odd numbers of steps, rows that lie apart; what does
+    not fill its rounds of tiles and other sizes of K stay apart."""
+    F, ext = torch.nn.functional, _ext(name)
+    n *= 1 if gated else 2
+    x = _draw(rows, k + 8, seed=rows)[:, :k]
+    w = _draw(2 * n if gated else n, k + 16, seed=n, scale=k ** -0.5)[:, 8:-8]
+    z = x.double() @ w.double().t()
+    call = ext.gated_linear if gated else ext.activated_linear
+    for act, fn in enumerate([lambda z: F.gelu(z, approximate="tanh"), F.silu,
+                              lambda z: z.relu().square()]):
+        y = call(x, w, act)
+        assert (y is not None) == one
+        if one:
+            g, u = z.chunk(2, -1) if gated else (z, 1)
+            _same(y, fn(g) * u, 8)
+
+
+@pytest.mark.parametrize("act", [0, 1, 2])
+def test_act_of_large_sums(act):
+    """Infinities and what overflows come out as they do apart."""
+    ext = _ext("_hip_layered")
+    x = torch.zeros(640, 128, device="cuda").bfloat16()
+    x[:, 0] = torch.tensor([1, -1, 1e4, -1e4, 1e38, -1e38, 90, -90, 0, -0.0],
+                           device="cuda").repeat(64).bfloat16()
+    w = torch.zeros(2 * 10880, 128, device="cuda").bfloat16()
+    w[::2, 0], w[1::2, 0] = 1, 1e4
+    got, want = ext.activated_linear(x, w, act), ext.activate(x @ w.t(), act)
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = ~want.isnan()
+    torch.testing.assert_close(got[ok], want[ok], rtol=2 ** -7, atol=1e-30)
+
+
 @pytest.mark.parametrize("rows,n,k,whole", [
     (2047, 4096, 4096, 0), (4096, 4096, 4096, 0), (4097, 4096, 96, 4096),
     (4096 + 2048, 4096, 96, 4096), (4096 + 2049, 4096, 96, 0),
