@@ -12,17 +12,21 @@
 //   S' = K Q'  a lane holds 16 bytes of a token's key (bf16 matrix cores; the
 //              order of the key's channels inside a step is free, Q follows).
 //              It gets back the scores of 4 + 4 tokens for one head.
-//   O  = P V   32-bit matrix cores: probabilities stay 32-bit, as the scores
-//              left them in the lane; a lane holds 8 channels of one token's
-//              value, widened to 32-bit (exact for bf16 and fp8).
-// A tile's matrix work is a quarter of the time its bytes take at 5 TB/s, so
-// the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost nothing.
+//   O  = P V   bf16 matrix cores, a step for 32 tokens and 16 channels: a
+//              probability is the sum of three bf16, all 24 bits of it, as the
+//              scores left them in the lane; values are bf16 as they are (fp8
+//              ones exactly). A lane holds 8 channels of 8 tokens and turns them
+//              round for itself.
+// A tile's matrix work is 512 cycles (2176 with P V on the 32-bit cores, which
+// for fp8 was as long as its bytes took, and the most power of a pass), its vector
+// work 700 (bf16) to 930 (fp8): less than its bytes take at 5 TB/s with three waves
+// a SIMD, so the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost
+// nothing.
 //
-// Measured alone (8 key heads, ragged; before: scores and sums on the vector
-// units, three barriers per 256 tokens): 256 sequences of 1500 tokens, groups of
-// 4: 279 us, 5.6 TB/s (before 546); 30 of 1100, groups of 8: 27 us (67); 17 of
-// 6800, fp8, in 4 partitions: 61 us, 3.8 TB/s (137), in a pass of layers 82, 2.9
-// TB/s; one of 777: 11 us (18).
+// Measured alone, cold (8 key heads, ragged; before: P V on the 32-bit cores): 256
+// sequences of 1500 tokens, groups of 4: 269 us, 5.8 TB/s (279), fp8 156 us, 5.0 TB/s
+// (191); 30 of 1100, groups of 8: 27.5 us (31.5); 17 of 6800, fp8, in 4 partitions:
+// 51 us, 4.5 TB/s (66.5); 60 of 300: 15.7 us (19.9); one of 777: 9.3 us (10.3).
 //
 // Flash-decoding sequence split (SPLIT): long sequences are cut into
 // gridDim.z partitions so that small batches fill the chip. Each partition
@@ -60,11 +64,16 @@ template <> struct Cache<short> {
   static __device__ __forceinline__ bf16x8 key(const uint4v* k, int s) {
     return __builtin_bit_cast(bf16x8, k[s]);
   }
-  static __device__ __forceinline__ void value(VReg v, float* f) {
+  // channels CH d .. of a lane's 8 tokens as operands, two tokens per register
+  static constexpr int CH = 2;
+  static __device__ __forceinline__ void values(const VReg (&v)[2][4], int d,
+                                                uint4v* o) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      f[2 * i] = __builtin_bit_cast(float, v[i] << 16);
-      f[2 * i + 1] = __builtin_bit_cast(float, v[i] & 0xffff0000u);
+      const unsigned int x = v[i / 2][i % 2 * 2][d];
+      const unsigned int y = v[i / 2][i % 2 * 2 + 1][d];
+      o[0][i] = __builtin_amdgcn_perm(y, x, 0x05040100);
+      o[1][i] = __builtin_amdgcn_perm(y, x, 0x07060302);
     }
   }
 };
@@ -75,30 +84,63 @@ template <> struct Cache<unsigned char> {
   static __device__ __forceinline__ int dim(int s, int g) {
     return s / 2 * 64 + g * 16 + s % 2 * 8;
   }
-  static __device__ __forceinline__ void value(VReg v, float* f) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const float2v a = __builtin_amdgcn_cvt_pk_f32_fp8(v[i], false);
-      const float2v b = __builtin_amdgcn_cvt_pk_f32_fp8(v[i], true);
-      f[4 * i] = a[0];
-      f[4 * i + 1] = a[1];
-      f[4 * i + 2] = b[0];
-      f[4 * i + 3] = b[1];
-    }
+  static __device__ __forceinline__ void widen(unsigned int v, float* f) {
+    const float2v a = __builtin_amdgcn_cvt_pk_f32_fp8(v, false);
+    const float2v b = __builtin_amdgcn_cvt_pk_f32_fp8(v, true);
+    f[0] = a[0];
+    f[1] = a[1];
+    f[2] = b[0];
+    f[3] = b[1];
   }
   // e4m3 values are bf16 values: the upper halves of the floats
+  static __device__ __forceinline__ unsigned int pair(float a, float b) {
+    return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b),
+                                 __builtin_bit_cast(uint32_t, a), 0x07060302);
+  }
+  static constexpr int CH = 4;
+  static __device__ __forceinline__ void values(const VReg (&v)[2][4], int d,
+                                                uint4v* o) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float x[4], y[4];
+      widen(v[i / 2][i % 2 * 2][d], x);
+      widen(v[i / 2][i % 2 * 2 + 1][d], y);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c][i] = pair(x[c], y[c]);
+    }
+  }
   static __device__ __forceinline__ bf16x8 key(const uint4v* k, int s) {
     float f[8];
-    value((uint2v){k[s / 2][s % 2 * 2], k[s / 2][s % 2 * 2 + 1]}, f);
+    widen(k[s / 2][s % 2 * 2], f);
+    widen(k[s / 2][s % 2 * 2 + 1], f + 4);
     uint4v r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      r[i] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, f[2 * i + 1]),
-                                   __builtin_bit_cast(uint32_t, f[2 * i]),
-                                   0x07060302);
+    for (int i = 0; i < 4; ++i) r[i] = pair(f[2 * i], f[2 * i + 1]);
     return __builtin_bit_cast(bf16x8, r);
   }
 };
+
+// 8 floats as sums of three bf16, exactly but for a last bit or two
+__device__ __forceinline__ void split3(const float4v* x, bf16x8* parts) {
+  float r[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r[i] = x[i / 4][i % 4];
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    uint4v w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float2v two = {r[2 * i], r[2 * i + 1]};
+      typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+      w[i] = __builtin_bit_cast(unsigned int,
+                                __builtin_convertvector(two, bf16x2));
+      const unsigned int lo = w[i] << 16, up = w[i] & 0xffff0000u;
+      r[2 * i] -= __builtin_bit_cast(float, lo);
+      r[2 * i + 1] -= __builtin_bit_cast(float, up);
+    }
+    parts[p] = __builtin_bit_cast(bf16x8, w);
+  }
+}
 
 // PAGE16: pages of 16 tokens and partitions that begin on a page, so half a
 // tile lies in one page; else every lane looks its tokens up one by one.
@@ -255,19 +297,28 @@ __global__ __launch_bounds__(NW * WAVE, 3) void paged_attention_kernel(
         sc[h][r] = __builtin_amdgcn_exp2f(sc[h][r] - m);
         l += sc[h][r];
       }
+    if (tail) {      // a page's rows past the sequence may hold anything
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float f[8];
-        C::value(vr[h][j], f);
-        // a page's rows past the sequence may hold anything
-        const bool gone = tail && t0 + h * 16 + g * 4 + j >= t_end;
+        for (int j = 0; j < 4; ++j)
+          if (t0 + h * 16 + g * 4 + j >= t_end)
+            vr[h][j] = (typename C::VReg)(0u);
+    }
+    bf16x8 parts[3];
+    split3(sc, parts);
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-              sc[h][j], gone ? 0.f : f[i], acc[i], 0, 0, 0);
-      }
+    for (int d = 0; d < 8 / C::CH; ++d) {
+      uint4v v[C::CH];
+      C::values(vr, d, v);
+#pragma unroll
+      for (int p = 2; p >= 0; --p)
+#pragma unroll
+        for (int c = 0; c < C::CH; ++c)
+          acc[d * C::CH + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              parts[p], __builtin_bit_cast(bf16x8, v[c]), acc[d * C::CH + c],
+              0, 0, 0);
+    }
     if (more) fetch_v(next);
   }
   l += __shfl_xor(l, 16, WAVE);
