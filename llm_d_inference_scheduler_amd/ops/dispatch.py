@@ -124,15 +124,18 @@ def reshape_and_cache(k_new: torch.Tensor, v_new: torch.Tensor,
 
 
 def decode_parts(groups: int, max_len: int,
-                 mean_len: Optional[float] = None) -> Tuple[int, int]:
+                 mean_len: Optional[float] = None,
+                 elem: int = 2) -> Tuple[int, int]:
     """-> (parts, tokens per part) of the decode attention of `groups`
     (sequence, key head) pairs of up to max_len tokens, and of mean_len on
-    average (None: all about as long). A workgroup of 8 waves takes 256 tokens
-    a step, and about 512 of them fill the chip: parts make up for fewer groups
-    as long as each has a step of its own. From 200 groups of like length on,
-    the partial sums and the second launch cost more than the idle compute
-    units (240 groups of 1100 tokens: 27 us in one part, 38 in two; 136 groups
-    of 6800 tokens, 8-bit: 108 us in one part, 62 in four).
+    average (None: all about as long), of `elem` bytes a value. A workgroup of 8
+    waves takes 256 tokens a step, and about 512 of them fill the chip: parts make
+    up for fewer groups as long as each has a step of its own. They cost their
+    sums and a second launch. In us, as measured: one part takes 3 and as long as
+    a workgroup walks (9.3 per 1000 tokens, 7.4 in 8 bits) or the bytes take at 4.9
+    TB/s, several 7 and the bytes at 5.2 TB/s; from 200 groups on it is always one
+    (136 groups of 6800 tokens, 8-bit: 63 in one part, 51 in four; 160 of 1500: 27
+    and 34; 96 of 800: 13 and 16; 64 of 2000: 25 and 18; 240 of 1100: 27 and 35).
 
     One long sequence among short ones would hold the batch up: 14 us per 1000
     tokens that a workgroup walks alone. It is cut so that none walks more than
@@ -141,8 +144,13 @@ def decode_parts(groups: int, max_len: int,
     of 8000 among 24 of 100: 108 us in one part, 24 in 17; among 255 of 300: 258
     and 140 in 3; of 3000 among 16 of 300: 21 in 4, 17 in 8; of 1500 among 24 of
     1000: 27 in one, 34 in two."""
-    parts = 1 if groups >= 200 else -(-512 // max(1, groups))
-    if mean_len is not None:
+    parts = 1
+    if groups < 200:
+        walk = max_len * (9.3e-3 if elem > 1 else 7.4e-3)
+        size = groups * 0.8 * max_len * 256 * elem
+        if 3 + max(walk, size / 4.9e6) > 7 + size / 5.2e6:
+            parts = -(-512 // max(1, groups))
+    if mean_len is not None and max_len > 1.4 * mean_len:
         # tokens that one workgroup may walk while each compute unit takes one
         # and a half shares of the whole
         walk = max(256., 1.5 * mean_len * groups / 256)
@@ -168,7 +176,8 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
             # sequences of 120 tokens: 19 us with 8 waves, 15 with 4)
             waves = 4 if max_seq_len <= 256 else 8
             parts, part = decode_parts(q.shape[0] * k_cache.shape[1],
-                                       max_seq_len, mean_seq_len)
+                                       max_seq_len, mean_seq_len,
+                                       k_cache.element_size())
             if parts > 1:
                 far_apart = mean_seq_len is not None and \
                     max_seq_len > 2 * mean_seq_len

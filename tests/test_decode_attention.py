@@ -17,6 +17,17 @@ def test_parts_cover_the_context(groups, max_len):
     assert (parts - 1) * part < max_len <= parts * part
 
 
+@pytest.mark.parametrize("groups,max_len,elem,one,several", [
+    (136, 8190, 1, 63, 51), (136, 8190, 2, 108, 87), (160, 1875, 2, 27, 34),
+    (176, 3750, 2, 54, 58), (96, 1000, 2, 13, 16), (64, 2500, 2, 25, 18),
+    (80, 375, 1, 5.9, 8.4), (32, 1250, 2, 13.9, 9.8), (8, 3750, 2, 31, 10),
+    (120, 650, 2, 10.3, 15.3), (8, 307, 1, 5.5, 7.8), (24, 6250, 1, 38, 13)])
+def test_one_part_or_several(groups, max_len, elem, one, several):
+    """Against the times that both took, us."""
+    parts, _ = dispatch.decode_parts(groups, max_len, None, elem)
+    assert (parts > 1) == (several < one)
+
+
 @pytest.mark.parametrize("batch", [2, 5, 17, 24, 25, 32, 64, 127, 256])
 @pytest.mark.parametrize("short", [1, 100, 300, 1000])
 @pytest.mark.parametrize("long", [1500, 3000, 8000, 131072])
