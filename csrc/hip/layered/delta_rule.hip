@@ -173,8 +173,21 @@ __global__ __launch_bounds__(NT) void delta_conv_kernel(
 // One workgroup per (head, sequence). S is spread over the threads: a thread
 // owns 4 columns (lanes_v threads cover V) and every groups-th row.
 // RPT: rows per thread. VEC: V % 4 == 0.
+//
+// The bytes of S, read and written once, are what counts; what kept it from
+// their rate were two workgroups per compute unit, each with a chain of loads.
+// So all of a token's inputs are asked for ahead of S, barriers wait for LDS
+// alone, and 16 rows per thread stay within 168 registers, for three (for four
+// they spill). S is not seen again before the next step of the model: marked
+// non-temporal, both ways, it leaves the last-level cache to the weights. us of
+// 50 sequences of 32 heads of 128 x 128, and with a gated product of 4096 -> 2 x
+// 14336 behind it: 56; 50 and 102 by the shorter chain; 47 and 103 with the
+// stores non-temporal; 42 (4.9 TB/s) and 88 with both. 200 sequences 186 -> 157,
+// 24 30 -> 17.5, 1 9.2 -> 8.7.
 template <typename T, int RPT, bool VEC>
-__global__ __launch_bounds__(NT) void delta_step_kernel(
+__global__ __launch_bounds__(NT, RPT <= 8    ? 4
+                                 : RPT == 16 ? 3
+                                             : 1) void delta_step_kernel(
     const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v,                 // [rows, KH|KH|H, K|K|V]
     const T* __restrict__ beta, int64_t bstride,  // [rows, H] before sigmoid
@@ -190,15 +203,52 @@ __global__ __launch_bounds__(NT) void delta_step_kernel(
   const Seq sq = load_seq(seq_meta, blockIdx.y);
   const int kh = h / (H / KH);
   const int groups = NT / lanes_v;
-  const int tv = threadIdx.x % lanes_v, grp = threadIdx.x / lanes_v;
-  const int c0 = tv * 4;
+  const unsigned tv = threadIdx.x % lanes_v, grp = threadIdx.x / lanes_v;
+  const unsigned c0 = tv * 4;
 
-  __shared__ float qs[512], ks[512], gs[512];
-  __shared__ float sk[4 * NT], so[4 * NT], kq[NT];
+  constexpr int KT = 512 / NT;        // channels of K per thread, at most
+  __shared__ float4v gkq[512];        // decay, k, q of a channel
+  __shared__ float4v sk[NT], so[NT];
+  __shared__ float kq[NT];
   __shared__ float red[NWV];
+
+  // a token's inputs, as they are in memory; past the end they repeat the last
+  const unsigned tid = threadIdx.x, last = V - 1, cv = VEC ? min(c0, V - 4u) : c0;
+  auto channel = [&](int j) { return VEC ? cv + j : min(cv + j, last); };
+  float qr[KT], kr[KT], vr[4], bias[KT], nw[4];
+  T dr[KT], gr[4], br;
+  auto fetch = [&](int t) {
+    const int64_t row = sq.row0 + t;
+    const float* qt = q + (row * KH + kh) * K;
+    const float* kt = k + (row * KH + kh) * K;
+    const T* dt = decay + (row * H + h) * K;
+    const float* vt = v + (row * H + h) * V;
+    const T* gt = gate + (row * H + h) * V;
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+      const unsigned d = min(tid + i * NT, K - 1u);
+      qr[i] = qt[d];
+      kr[i] = kt[d];
+      dr[i] = dt[d];
+    }
+    br = beta[row * bstride + h];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      vr[j] = vt[channel(j)];
+      gr[j] = gt[channel(j)];
+    }
+  };
+  const float na = neg_a[h];
+  const float* bt = dt_bias + (int64_t)h * K;
+#pragma unroll
+  for (int i = 0; i < KT; ++i) bias[i] = bt[min(tid + i * NT, K - 1u)];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) nw[j] = norm_w[channel(j)];
+  if (sq.n > 0) fetch(0);
 
   float S[RPT][4];
   float* Sp = state + ((int64_t)sq.slot * H + h) * K * V;
+  const unsigned at = grp * V + c0, step = groups * V;
 #pragma unroll
   for (int i = 0; i < RPT; ++i) {
     const int r = grp + i * groups;
@@ -206,69 +256,67 @@ __global__ __launch_bounds__(NT) void delta_step_kernel(
     for (int j = 0; j < 4; ++j) S[i][j] = 0.f;
     if (r < K && sq.prior > 0) {
       if constexpr (VEC) {
-        if (c0 < V) {
-          const float4v t = *(const float4v*)(Sp + (int64_t)r * V + c0);
+        if (c0 < (unsigned)V) {
+          const float4v t =
+              __builtin_nontemporal_load((const float4v*)(Sp + i * step + at));
 #pragma unroll
           for (int j = 0; j < 4; ++j) S[i][j] = t[j];
         }
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (c0 + j < V) S[i][j] = Sp[(int64_t)r * V + c0 + j];
+          if (c0 + j < (unsigned)V) S[i][j] = Sp[i * step + at + j];
       }
     }
   }
 
   for (int t = 0; t < sq.n; ++t) {
     const int64_t row = sq.row0 + t;
-    __syncthreads();  // the previous token's readers of shared memory
-    for (int d = threadIdx.x; d < K; d += NT) {
-      qs[d] = q[(row * KH + kh) * K + d];
-      ks[d] = k[(row * KH + kh) * K + d];
-      gs[d] = expf(neg_a[h] * softplus_f(ld(decay + (row * H + h) * K + d) +
-                                         dt_bias[(int64_t)h * K + d]));
+    // readers of gkq and kq of the token before are past a barrier (block_sum)
+#pragma unroll
+    for (int i = 0; i < KT; ++i) {
+      const int d = tid + i * NT;
+      if (d < K)
+        gkq[d] = (float4v){expf(na * softplus_f(ld(&dr[i]) + bias[i])), kr[i],
+                           qr[i], 0.f};
     }
-    __syncthreads();
-    float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f}, c = 0.f;
+    lds_barrier();
+    float4v a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    float c = 0.f;
 #pragma unroll
     for (int i = 0; i < RPT; ++i) {
       const int r = grp + i * groups;
       if (r < K) {
-        const float g = gs[r], kr = ks[r], qr = qs[r];
-        c += kr * qr;
+        const float4v x = gkq[r];
+        c += x[1] * x[2];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          S[i][j] *= g;
-          a[j] += S[i][j] * kr;
-          b[j] += S[i][j] * qr;
+          S[i][j] *= x[0];
+          a[j] += S[i][j] * x[1];
+          b[j] += S[i][j] * x[2];
         }
       }
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // registers
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      sk[(grp * lanes_v + tv) * 4 + j] = a[j];
-      so[(grp * lanes_v + tv) * 4 + j] = b[j];
-    }
+    sk[threadIdx.x] = a;
+    so[threadIdx.x] = b;
     if (tv == 0) kq[grp] = c;
-    __syncthreads();
+    lds_barrier();
     // S'k and S'q of the decayed state; the new write adds (k.q) u to o
-    float u[4], o[4] = {0.f, 0.f, 0.f, 0.f}, dot = 0.f;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) u[j] = 0.f;
+    float4v u = {0.f, 0.f, 0.f, 0.f}, o = u;
+    float dot = 0.f;
+#pragma unroll 2
     for (int p = 0; p < groups; ++p) {
       dot += kq[p];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u[j] += sk[(p * lanes_v + tv) * 4 + j];
-        o[j] += so[(p * lanes_v + tv) * 4 + j];
-      }
+      u += sk[p * lanes_v + tv];
+      o += so[p * lanes_v + tv];
     }
-    const float bt = sigmoid_f(ld(beta + row * bstride + h));
+    const float write = sigmoid_f(ld(&br));
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bool in = c0 + j < V;
-      u[j] = in ? bt * (v[(row * H + h) * V + c0 + j] - u[j]) : 0.f;
+      const bool in = c0 + j < (unsigned)V;
+      u[j] = in ? write * (vr[j] - u[j]) : 0.f;
       o[j] += dot * u[j];
       if (in && grp == 0) ss += o[j] * o[j];
     }
@@ -276,20 +324,25 @@ __global__ __launch_bounds__(NT) void delta_step_kernel(
     for (int i = 0; i < RPT; ++i) {
       const int r = grp + i * groups;
       if (r < K) {
+        const float kd = gkq[r][1];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) S[i][j] += ks[r] * u[j];
+        for (int j = 0; j < 4; ++j) S[i][j] += kd * u[j];
       }
+      if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
+    T gt[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) gt[j] = gr[j];
+    if (t + 1 < sq.n) fetch(t + 1);
     const float inv =
         1.f / sqrtf(block_sum<NWV>(ss, red) / (float)V + eps);
+    T* ot = out + (row * H + h) * V;
     if (grp == 0) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (c0 + j < V) {
-          const int64_t at = (row * H + h) * V + c0 + j;
-          st(out + at, o[j] * inv * norm_w[c0 + j] * sigmoid_f(ld(gate + at)));
-        }
-      }
+      for (int j = 0; j < 4; ++j)
+        if (c0 + j < (unsigned)V)
+          st(ot + c0 + j,
+             o[j] * inv * nw[j] * sigmoid_f(ld(&gt[j])));
     }
   }
 
@@ -298,13 +351,14 @@ __global__ __launch_bounds__(NT) void delta_step_kernel(
     const int r = grp + i * groups;
     if (r < K) {
       if constexpr (VEC) {
-        if (c0 < V)
-          *(float4v*)(Sp + (int64_t)r * V + c0) =
-              (float4v){S[i][0], S[i][1], S[i][2], S[i][3]};
+        if (c0 < (unsigned)V)
+          __builtin_nontemporal_store(
+              (float4v){S[i][0], S[i][1], S[i][2], S[i][3]},
+              (float4v*)(Sp + i * step + at));
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (c0 + j < V) Sp[(int64_t)r * V + c0 + j] = S[i][j];
+          if (c0 + j < (unsigned)V) Sp[i * step + at + j] = S[i][j];
       }
     }
   }

@@ -291,6 +291,23 @@ def test_groups_are_full():
             assert all(len(g.chunks_host) <= per for g in groups)
 
 
+@pytest.mark.parametrize("run", RUNS)
+@pytest.mark.parametrize("K,V", [(300, 8), (512, 3), (512, 32), (256, 256)])
+def test_steps_of_many_channels(run, K, V):
+    """More than one channel of K, or every row count, per thread."""
+    seqs = [(1, 3, 2), (4, 0, 4), (1, 2, 0)]
+    d = delta_case(run, seqs, 1, 2, K, V, DECAYS[0], seed=70)
+    m, _ = meta(seqs, run)
+    want, _, states = delta_oracle(d, seqs, 1e-5)
+    out = torch.zeros(6, 2 * V, dtype=run[1], device=run[0])
+    ops.delta_step(d["q"], d["k"], d["v"], d["proj"], 5, d["decay"], d["bias"],
+                   d["neg_a"], d["gate"], d["norm"], d["state"], m, 3, out,
+                   1e-5)
+    close(out, want, run, f32=2e-5)
+    for slot, S in states.items():
+        close(d["state"][slot], S, ("", torch.float32), f32=1e-5)
+
+
 class TestRotary:
     @pytest.mark.parametrize("scaling", [
         None, {"factor": 4.0, "original": 64, "fast": 32.0, "slow": 1.0},
