@@ -7,11 +7,11 @@
 //   P[i][j] = sum_d q_i k_j e^(G_i - G_j)   (j <= i)
 //   (I + diag(beta) A) U = diag(beta) (V - (k e^G) S0)
 //   O = (q e^G) S0 + P U,   S = e^(G_last) S0 + (k e^(G_last - G))' U
-// A and P are products of scaled rows, in blocks of 16 tokens. Off the diagonal
-// the sum before the later block is the reference, so no exponent is positive.
-// On the diagonal it is the block's middle, as long as no channel decays by
-// more than e^-DECAY_LIMIT inside a block; else every pair is taken by itself.
-// So any decay down to 0 is right.
+// A and P are products of scaled rows, in blocks of 16 tokens. The sum before
+// the later block is the reference, so off the diagonal no exponent is positive.
+// On the diagonal they are up to e^24, as long as no channel decays by more than
+// that inside a block (every term has its own relative error, whatever the
+// reference); else every pair is taken by itself. So any decay down to 0 is right.
 //
 // delta_chunk_local  everything that does not need S0, one workgroup per
 //                    (head, chunk): U0 and W with U = U0 - W S0, P, the
@@ -90,15 +90,64 @@ __device__ __forceinline__ float4v load4(const short* p, int left,
   return f;
 }
 
-constexpr float DECAY_LIMIT = 24.f;
-constexpr int AB = B * (B + 4);     // one 16 x 16 block of beta A in LDS
+constexpr float LOG2E = 1.4426950408889634f;
+constexpr float DECAY_LIMIT = 24.f * LOG2E;    // of a block, in powers of two
+// beta A in LDS, 16 x 16 blocks of the lower triangle: groups of 4 columns change
+// places by XOR with the row, so that 16 rows' groups meet all banks
+constexpr int AB = B * B;
 __device__ __forceinline__ int block_at(int bi, int bj) {
   return (bi * (bi + 1) / 2 + bj) * AB;
+}
+__device__ __forceinline__ int group_at(int r, int g) {
+  return r * B + (g ^ (r / 4)) * 4;
+}
+__device__ __forceinline__ float exp2_f(float x) {
+  return __builtin_amdgcn_exp2f(x);
+}
+
+// channels d .. d + 3 of a row of K: past the end the last ones, which come() drops.
+// No load is under a condition, so that the compiler can count those under way.
+template <typename T> struct Raw;
+template <> struct Raw<float> { typedef float4v type; };
+template <> struct Raw<short> { typedef short4v type; };
+template <typename T>
+__device__ __forceinline__ typename Raw<T>::type ask4(const T* row, int d, int K,
+                                                      bool whole) {
+  typedef typename Raw<T>::type Four;
+  if (whole) return *(const Four*)(row + min(d, K - 4));
+  Four f;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) f[x] = row[min(d + x, K - 1)];
+  return f;
+}
+template <typename F>
+__device__ __forceinline__ float4v come(F f, bool in, int d, int K) {
+  float4v o;
+#pragma unroll
+  for (int x = 0; x < 4; ++x) {
+    float v;
+    if constexpr (sizeof(F) == 16) v = f[x]; else v = bf16_to_f32(f[x]);
+    o[x] = in && d + x < K ? v : 0.f;
+  }
+  return o;
 }
 
 // grid (H, chunks); chunks [n, 2] = first row, tokens. Everything the waves
 // share goes through LDS (80 KB: two workgroups per CU), so its barriers let
 // global loads and stores run on.
+//
+// Decays are powers of two and taken once per token and channel: with g the sum
+// inside a block up to the token, t the block's whole sum, LDS keeps k 2^g, k
+// 2^(t - g) and 2^t, and all else is products of these. Four waves do the blocks
+// of A, each 16 tokens' row of them and its diagonal block's inverse, four those
+// of P, the longest of these beside the shortest of those on a SIMD; operands of
+// the row stay in registers, and results come out turned, whole groups of 4.
+// Loads of q and v are under way a phase ahead. What bounds it is no one thing:
+// loads and stores take half of a workgroup's 67000 cycles (260 KB each, 3.4 TB/s
+// over the chip), matrix instructions a third; with decays taken per pair of
+// blocks, references in the middle of diagonal ones and results stored one value
+// at a time it was 105000. 1024 chunks of 32 heads of 128 x 128, with the scan:
+// 197 -> 166 us; here alone, in a pass, 128 -> 101. Steep blocks take half as long again.
 template <typename T, int KP>
 __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
     const float* __restrict__ q, const float* __restrict__ k,
@@ -107,10 +156,12 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
     const float* __restrict__ neg_a, const int32_t* __restrict__ chunks,
     float* __restrict__ ws, int KH, int H, int K, int V, int VP) {
   constexpr int LD = KP + 4;          // row stride in LDS
+  constexpr int NT = KP / 16;
   extern __shared__ float lds[];
-  float* kl = lds;                    // [C][LD]
-  float* gl = kl + C * LD;            // log decays summed inside blocks
-  float* al = gl + C * LD;            // beta A, lower blocks; the diagonal
+  float* kl = lds;                    // [C][LD]: k, then k 2^g
+  float* gl = kl + C * LD;            // [C][LD]: g, then k 2^(t - g)
+  float* tl = gl + C * LD;            // [4][KP]: 2^t
+  float* al = tl + 4 * KP;            // beta A, lower blocks; the diagonal
                                       // ones become their inverses
   float* bl = al + 10 * AB;           // beta [C]
   int* steep = (int*)(bl + C);        // per wave: a block decays too much
@@ -119,7 +170,8 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
   const int64_t row0 = chunks[2 * blockIdx.y];
   const int n = chunks[2 * blockIdx.y + 1];
   const Work wk = work_at(ws, (int64_t)blockIdx.y * H + h, KP, VP);
-  const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int col = lane % 16, g4 = 4 * (lane / 16);
   // bases of this chunk and head; offsets from them fit 32 bits
   const float* kc = k + (row0 * KH + kh) * K;
@@ -128,54 +180,64 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
   const T* dc = decay + (row0 * H + h) * K;
   const unsigned krow = KH * K, drow = H * K, vrow = H * V;
   const bool whole = K % 4 == 0;
+  // the wave's 16 tokens: waves 0 to 3 have their rows of A, 7 to 4 of P
+  const bool of_p = wave >= 4;
+  const int bi = of_p ? 7 - wave : wave, mine = bi * B + col;
 
   // ---- load; rows and channels past the end are zero. All loads of a
   // thread are under way before the first is used ----
   constexpr int Q4 = C * KP / 4 / LT;            // groups of 4 channels
-  const int di = tid / 8, ds = tid % 8;          // diagonal part: token, slice
-  constexpr int DS = KP / 32;                    // its groups of 4 channels
+  const int d4 = tid % (KP / 4) * 4, t4 = tid / (KP / 4);
+  float4v row[NT];                               // of q or k; later times 2^g
   {
-    float4v kr[Q4], dr[Q4], bias[Q4];
+    float4v kr[Q4], bias;
+    typename Raw<T>::type dr[Q4];
+    if (of_p) {
+      const float* qrow = qc + (unsigned)min(mine, n - 1) * krow;
 #pragma unroll
-    for (int i = 0; i < Q4; ++i) {
-      const unsigned t = (tid + i * LT) / (KP / 4),
-                     d = (tid + i * LT) % (KP / 4) * 4;
-      const int left = (int)t < n ? K - (int)d : 0;
-      kr[i] = load4(kc + t * krow + d, left, whole);
-      dr[i] = load4(dc + t * drow + d, left, whole);
-      bias[i] = load4(dt_bias + (int64_t)h * K + d, left, whole);
+      for (int t = 0; t < NT; ++t) row[t] = ask4(qrow, 16 * t + g4, K, whole);
     }
-    const float na = neg_a[h];
+    const float na = neg_a[h] * LOG2E;
+    const float b0 = ld(beta + (row0 + min(tid % C, n - 1)) * bstride + h);
+    bias = ask4(dt_bias + (int64_t)h * K, d4, K, whole);
 #pragma unroll
     for (int i = 0; i < Q4; ++i) {
-      const int t = (tid + i * LT) / (KP / 4), d = (tid + i * LT) % (KP / 4) * 4;
+      const unsigned t = min(t4 + i * (LT * 4 / KP), n - 1);
+      dr[i] = ask4(dc + t * drow, d4, K, whole);
+      kr[i] = ask4(kc + t * krow, d4, K, whole);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (tid < C) bl[tid] = tid < n ? sigmoid_f(b0) : 0.f;
+#pragma unroll
+    for (int i = 0; i < Q4; ++i) {
+      const int t = t4 + i * (LT * 4 / KP);
+      const float4v d = come(dr[i], t < n, d4, K);
       float4v gv;
 #pragma unroll
       for (int x = 0; x < 4; ++x)
-        gv[x] = t < n && d + x < K ? na * softplus_f(dr[i][x] + bias[i][x])
-                                   : 0.f;
-      *(float4v*)(kl + t * LD + d) = kr[i];
-      *(float4v*)(gl + t * LD + d) = gv;
+        gv[x] = t < n && d4 + x < K ? na * softplus_f(d[x] + bias[x]) : 0.f;
+      *(float4v*)(kl + t * LD + d4) = come(kr[i], t < n, d4, K);
+      *(float4v*)(gl + t * LD + d4) = gv;
     }
   }
-  if (tid < C)
-    bl[tid] = tid < n ? sigmoid_f(ld(beta + (row0 + tid) * bstride + h)) : 0.f;
   lds_barrier();
   // ---- running sums inside blocks of 16: differences of small sums stay
   // exact where a chunk's whole sum would have swallowed them ----
   static_assert(4 * KP <= LT, "one pass");
+  const bool has = tid < 4 * KP;                 // wave-uniform
+  const int column = tid / KP % 4 * B * LD + tid % KP;
   bool over = false;
-  for (int i = tid; i < 4 * KP; i += LT) {
-    float* c = gl + (i / KP) * B * LD + i % KP;
-    float x[B];
+  if (has) {
+    float sum[B];
 #pragma unroll
-    for (int t = 0; t < B; ++t) x[t] = c[t * LD];
+    for (int t = 0; t < B; ++t) sum[t] = gl[column + t * LD];
 #pragma unroll
     for (int t = 1; t < B; ++t) {
-      x[t] += x[t - 1];
-      c[t * LD] = x[t];
+      sum[t] += sum[t - 1];
+      gl[column + t * LD] = sum[t];
     }
-    over = x[B - 1] < -DECAY_LIMIT;
+    tl[tid] = exp2_f(sum[B - 1]);
+    over = sum[B - 1] < -DECAY_LIMIT;
   }
   {
     const bool any = __any(over);
@@ -185,64 +247,11 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
   bool slow = false;
 #pragma unroll
   for (int w = 0; w < LT / WAVE; ++w) slow |= steep[w] != 0;
-  // sum over the blocks b0 <= b < b1
-  auto blocks = [&](int b0, int b1, int d) {
-    float s = 0.f;
-    for (int b = b0; b < b1; ++b) s += gl[(b * B + B - 1) * LD + d];
-    return s;
-  };
-
-  // ---- blocks of A (to LDS) and P: one wave each, bi >= bj ----
-  auto block_pair = [&](int bi, int bj) -> float4v {
-    const int i = bi * B + col, j = bj * B + col;
-    float4v qo[KP / 16];
-#pragma unroll
-    for (int t = 0; t < KP / 16; ++t)
-      qo[t] = load4(qc + i * krow + 16 * t + g4, i < n ? K - 16 * t - g4 : 0,
-                    whole);
-    float4v a = {0.f, 0.f, 0.f, 0.f}, p = a;
-#pragma unroll
-    for (int t = 0; t < KP / 16; ++t) {
-      const int o = 16 * t + g4;
-      const float4v gi = *(const float4v*)(gl + i * LD + o);
-      const float4v gj = *(const float4v*)(gl + j * LD + o);
-      const float4v ki = *(const float4v*)(kl + i * LD + o);
-      const float4v kj = *(const float4v*)(kl + j * LD + o);
-      // reference as seen from block bi and from block bj
-      float4v ri = {0.f, 0.f, 0.f, 0.f}, rj = ri;
-      if (bi == bj)
-        ri = rj = *(const float4v*)(gl + (bi * B + B / 2) * LD + o);
-      for (int b = bj; b < bi; ++b)
-        rj += *(const float4v*)(gl + (b * B + B - 1) * LD + o);
-      float4v ka, qa, kb;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        const float e = __expf(gi[x] - ri[x]);
-        ka[x] = ki[x] * e;
-        qa[x] = qo[t][x] * e;
-        kb[x] = kj[x] * __expf(rj[x] - gj[x]);
-      }
-      a = mfma4(ka, kb, a);
-      p = mfma4(qa, kb, p);
-      __builtin_amdgcn_sched_barrier(0);   // keep the reads of later steps
-    }                                      // from taking all registers
-    float* ab = al + block_at(bi, bj);
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int r = g4 + x;
-      if (bi == bj && col > r) p[x] = 0.f;
-      ab[r * (B + 4) + col] =
-          bi == bj && col >= r ? 0.f : bl[bi * B + r] * a[x];
-    }
-    return p;
-  };
-  float4v p0 = {0.f, 0.f, 0.f, 0.f}, p1 = p0;
-  const int bi = wave < 1 ? 1 : wave < 3 ? 2 : wave < 6 ? 3 : 2 * (wave - 6);
-  const int bj = wave < 6 ? wave - bi * (bi - 1) / 2 : bi;
-  if (wave < 6 || !slow) p0 = block_pair(bi, bj);
-  if (wave >= 6 && !slow) p1 = block_pair(bi + 1, bj + 1);
+  slow = __builtin_amdgcn_readfirstlane(slow);
 
   // ---- diagonal blocks pair by pair: 8 threads share token i ----
+  const int di = tid / 8, ds = tid % 8;          // token, slice
+  constexpr int DS = KP / 32;                    // its groups of 4 channels
   float pk[2] = {0.f, 0.f};          // this thread's share of P's row
   if (slow) {
     const int i = di, s = ds, b0 = i / B * B;
@@ -256,7 +265,7 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
                     i < n ? K - s * 4 - d * 32 : 0, whole);
     }
     const float beta_i = bl[i];
-    float* ab = al + block_at(i / B, i / B) + (i % B) * (B + 4);
+    float* ab = al + block_at(i / B, i / B);
 #pragma unroll 1
     for (int j = b0; j < b0 + B; ++j) {
       float a = 0.f, p = 0.f;
@@ -268,57 +277,148 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
 #pragma unroll
           for (int x = 0; x < 4; ++x) {
             // pairs with j > i are thrown away below; their exponent is cut
-            const float e = __expf(fminf(gi[d][x] - gj[x], 0.f)) * kj[x];
+            const float e = exp2_f(fminf(gi[d][x] - gj[x], 0.f)) * kj[x];
             a += ki[d][x] * e;
             p += qi[d][x] * e;
           }
-        }
+          __builtin_amdgcn_sched_barrier(0);   // keep the reads from taking
+        }                                      // all registers
 #pragma unroll
         for (int o = 1; o < 8; o *= 2) {
           a += __shfl_xor(a, o, WAVE);
           p += __shfl_xor(p, o, WAVE);
         }
       }
-      if (s == 0) ab[j - b0] = j < i ? beta_i * a : 0.f;
+      if (s == 0)
+        ab[group_at(i % B, (j - b0) / 4) + j % 4] = j < i ? beta_i * a : 0.f;
       p = j <= i ? p : 0.f;
       if (j - b0 == 2 * s) pk[0] = p;
       if (j - b0 == 2 * s + 1) pk[1] = p;
     }
   }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int o = 16 * t + g4;
+    const float4v g = *(const float4v*)(gl + mine * LD + o);
+    row[t] = of_p ? come(row[t], mine < n, o, K)
+                  : *(const float4v*)(kl + mine * LD + o);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) row[t][x] *= exp2_f(g[x]);
+  }
+  float sum[B], kcol[B];
+  if (has) {
+#pragma unroll
+    for (int t = 0; t < B; ++t) {
+      sum[t] = gl[column + t * LD];
+      kcol[t] = kl[column + t * LD];
+    }
+  }
   lds_barrier();
-
-  // ---- inverses of the unit lower triangular diagonal blocks, in place (a
-  // step reads row i before it writes row i; lanes run in step) ----
-  if (wave < 4 && lane < B) {
-    float* a = al + block_at(wave, wave);
-    float x[B];
+  if (has) {
 #pragma unroll
-    for (int i = 0; i < B; ++i) {
-      float s = i == lane ? 1.f : 0.f;
-#pragma unroll
-      for (int j = 0; j < i; ++j) s -= a[i * (B + 4) + j] * x[j];
-      x[i] = s;
-      a[i * (B + 4) + lane] = s;
+    for (int t = 0; t < B; ++t) {
+      kl[column + t * LD] = kcol[t] * exp2_f(sum[t]);
+      gl[column + t * LD] = kcol[t] * exp2_f(sum[B - 1] - sum[t]);
     }
   }
   // Loads wait for the stores issued before them, so this wave's first tile
   // of v comes now and every store after it.
-  float4v vpre[4];
+  float vpre[4][4];
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = b * B + g4 + r, c = wave * 16 + col;
-      vpre[b][r] = t < n && c < V ? vc[t * vrow + c] : 0.f;
-    }
-  // its share of q too
-  float4v qr[Q4];
+    for (int r = 0; r < 4; ++r)
+      vpre[b][r] = vc[(unsigned)min(b * B + g4 + r, n - 1) * vrow +
+                      min(wave * 16 + col, V - 1)];
+  lds_barrier();
+
+  // products of 2^t over the blocks b0 <= b < b1, of 4 channels or of one
+  auto span4 = [&](int b0, int b1, int d) {
+    float4v f = {1.f, 1.f, 1.f, 1.f};
+    for (int b = b0; b < b1; ++b) f *= *(const float4v*)(tl + b * KP + d);
+    return f;
+  };
+  auto span = [&](int b0, int b1, int d) {
+    float f = 1.f;
+    for (int b = b0; b < b1; ++b) f *= tl[b * KP + d];
+    return f;
+  };
+  // ---- one block of the wave's row, turned: lane (i, g) has columns 4 g .. ----
+  auto block = [&](int bj) -> float4v {
+    float4v a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < Q4; ++i) {
-    const int tile = wave + i * (LT / WAVE);
-    const int t = tile / (KP / 16) * 16 + col, d = tile % (KP / 16) * 16 + g4;
-    qr[i] = load4(qc + t * krow + d, t < n ? K - d : 0, whole);
+    for (int t = 0; t < NT; ++t) {
+      const int o = 16 * t + g4;
+      float4v kb = *(const float4v*)(gl + (bj * B + col) * LD + o);
+      if (bi == bj) {                            // 2^-g_j, at most e^24
+        const float4v f = *(const float4v*)(tl + bi * KP + o);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) kb[x] *= rcp_f(f[x]);
+      } else if (bi > bj + 1) {
+        kb *= span4(bj + 1, bi, o);
+      }
+      a = mfma4(kb, row[t], a);
+    }
+    return a;
+  };
+  if (!of_p) {
+    if (!slow) {
+      float4v a = block(bi);
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+        a[x] = g4 + x < col ? bl[mine] * a[x] : 0.f;
+      *(float4v*)(al + block_at(bi, bi) + group_at(col, g4 / 4)) = a;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    // inverse of the unit lower triangular diagonal block, in place
+    if (lane < B) {
+      float* a = al + block_at(bi, bi);
+      float x[B];
+#pragma unroll
+      for (int i = 0; i < B; ++i) {
+        float s = i == lane ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < i; ++j)
+          s -= a[group_at(i, j / 4) + j % 4] * x[j];
+        x[i] = s;
+      }
+#pragma unroll
+      for (int i = 0; i < B; ++i) a[group_at(i, lane / 4) + lane % 4] = x[i];
+    }
+    for (int bj = 0; bj < bi; ++bj)
+      *(float4v*)(al + block_at(bi, bj) + group_at(col, g4 / 4)) =
+          bl[mine] * block(bj);
+  } else {
+    for (int bj = 0; bj < bi + !slow; ++bj) {
+      float4v p = block(bj);
+      if (bi == bj) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x)
+          if (g4 + x > col) p[x] = 0.f;
+      }
+      *(float4v*)(wk.p + (bi * 4 + bj) * 256 + lane * 4) = p;
+    }
+    // scaled q and k
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      *(float4v*)(wk.qe + (bi * NT + t) * 256 + lane * 4) =
+          row[t] * span4(0, bi, 16 * t + g4);
+    for (int tile = wave - 4; tile < 4 * NT; tile += 4) {
+      const int d = tile / 4 * 16 + col, t = tile % 4 * 16 + g4;
+      const float after = span(tile % 4 + 1, 4, d);
+      float4v o;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) o[x] = gl[(t + x) * LD + d] * after;
+      *(float4v*)(wk.kt + tile * 256 + lane * 4) = o;
+    }
   }
+  if (slow) {
+    float* o = wk.p + di / B * (4 + 1) * 256;     // tile (b, b)
+    typedef __attribute__((ext_vector_type(2))) float f2;
+    *(f2*)(o + (di % B + 16 * (ds / 2)) * 4 + ds % 2 * 2) =
+        (f2){pk[0], pk[1]};
+  }
+  if (tid < KP) wk.gl[tid] = span(0, 4, tid);
   lds_barrier();
 
   // ---- forward substitution by blocks, 16 columns of [V | K] at a time ----
@@ -327,83 +427,40 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
     const int c = (is_v ? tile : tile - VP / 16) * 16 + col;
     float4v f[4], x[4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int b = 0; b < 4; ++b) {
+      const float before = is_v ? 1.f : span(0, b, c);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int t = b * B + g4 + r;
-        if (is_v)
-          f[b][r] = tile == wave         ? vpre[b][r]
-                    : t < n && c < V     ? vc[t * vrow + c]
-                                         : 0.f;
+        if (!is_v)
+          f[b][r] = -kl[t * LD + c] * before;
+        else if (tile == wave)
+          f[b][r] = t < n && c < V ? vpre[b][r] : 0.f;
         else
-          f[b][r] = -kl[t * LD + c] * __expf(blocks(0, b, c) + gl[t * LD + c]);
+          f[b][r] = t < n && c < V ? vc[t * vrow + c] : 0.f;
       }
+    }
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
       float4v acc = *(const float4v*)(bl + b * B + g4) * f[b];
 #pragma unroll
       for (int p = 0; p < b; ++p) {
         const float4v a =
-            *(const float4v*)(al + block_at(b, p) + col * (B + 4) + g4);
+            *(const float4v*)(al + block_at(b, p) + group_at(col, g4 / 4));
         acc = mfma4(-a, x[p], acc);
       }
       const float4v inv =
-          *(const float4v*)(al + block_at(b, b) + col * (B + 4) + g4);
+          *(const float4v*)(al + block_at(b, b) + group_at(col, g4 / 4));
       x[b] = mfma4(inv, acc, (float4v){0.f, 0.f, 0.f, 0.f});
       if (is_v) {
         *(float4v*)(wk.u0 + (tile * 4 + b) * 256 + lane * 4) = x[b];
       } else {
-        // -W, turned: rows of D are the lanes of A
-        float* o = wk.w + (b * (KP / 16) + tile - VP / 16) * 256;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          o[(g4 + r + 16 * (col / 4)) * 4 + col % 4] = x[b][r];
+        // -W, turned by taking the last product the other way round
+        *(float4v*)(wk.w + (b * NT + tile - VP / 16) * 256 + lane * 4) =
+            mfma4(acc, inv, (float4v){0.f, 0.f, 0.f, 0.f});
       }
     }
   }
-
-  // ---- P, scaled q and k, the chunk's decay ----
-  if (slow) {
-    float* o = wk.p + di / B * (4 + 1) * 256;     // tile (b, b)
-    typedef __attribute__((ext_vector_type(2))) float f2;
-    *(f2*)(o + (di % B + 16 * (ds / 2)) * 4 + ds % 2 * 2) =
-        (f2){pk[0], pk[1]};
-  }
-  if (wave < 6 || !slow) {
-    float* o = wk.p + (bi * 4 + bj) * 256;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int at = (g4 + r + 16 * (col / 4)) * 4 + col % 4;
-      o[at] = p0[r];
-      if (wave >= 6) o[at + 5 * 256] = p1[r];     // the next diagonal tile
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < Q4; ++i) {
-    const int tile = wave + i * (LT / WAVE);
-    {
-      const int t = tile / (KP / 16) * 16 + col,
-                d = tile % (KP / 16) * 16 + g4;
-      const float4v g = *(const float4v*)(gl + t * LD + d);
-      float4v o = qr[i];
-      float4v before = {0.f, 0.f, 0.f, 0.f};
-      for (int b = 0; b < tile / (KP / 16); ++b)
-        before += *(const float4v*)(gl + (b * B + B - 1) * LD + d);
-#pragma unroll
-      for (int x = 0; x < 4; ++x) o[x] *= __expf(before[x] + g[x]);
-      *(float4v*)(wk.qe + tile * 256 + lane * 4) = o;
-    }
-    {
-      const int d = tile / 4 * 16 + col, t = tile % 4 * 16 + g4;
-      const float after = blocks(tile % 4, 4, d);
-      float4v o;
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-        o[x] = kl[(t + x) * LD + d] * __expf(after - gl[(t + x) * LD + d]);
-      *(float4v*)(wk.kt + tile * 256 + lane * 4) = o;
-    }
-  }
-  for (int d = tid; d < KP; d += LT) wk.gl[d] = __expf(blocks(0, 4, d));
 }
 
 // grid (H, VP / (16 NC), sequences); walk [n, 4] = first row, tokens, slot,
@@ -630,7 +687,7 @@ hipError_t lds_delta_chunk(int f32, const float* q, const float* k,
   if (K > 128) return hipErrorInvalidValue;
   const int KP = padded_k(K), VP = (V + 15) / 16 * 16;
   const size_t lds =
-      (2 * C * (KP + 4) + 10 * AB + C + LT / WAVE) * sizeof(float);
+      (2 * C * (KP + 4) + 4 * KP + 10 * AB + C + LT / WAVE) * sizeof(float);
   const dim3 g1(H, n_chunks);
   const int tiles = VP / 16, pairs = (tiles + 1) / 2;
   // two workgroups per compute unit at least, else one tile each

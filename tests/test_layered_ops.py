@@ -277,6 +277,39 @@ def test_chunks_of_many_sequences(run, K, V, n, shift):
         close(d["state"][slot], S, ("", torch.float32), f32=3e-5)
 
 
+@GPU
+@pytest.mark.parametrize("K,V", [(128, 128), (64, 24), (36, 40), (31, 5)])
+@pytest.mark.parametrize("total", [23.9, 24.1, 90.])
+@pytest.mark.parametrize("run", RUNS[1:2])
+def test_chunks_of_steep_blocks(run, K, V, total):
+    """All channels of every second head decay by e^-total over 16 tokens: just
+    short of where blocks go pair by pair, just past it, and where a block's decay
+    is no normal number. Values as in the tests above."""
+    H, seqs = 4, [(130, 0, 1), (64, 3, 0), (16, 1, 2)]
+    d = delta_case(run, seqs, 2, H, K, V, 0., seed=90)
+    d["decay"].zero_()
+    d["bias"].zero_()                       # softplus: log 2
+    d["neg_a"][::2] = -total / 16 / math.log(2)
+    d["neg_a"][1::2] = -0.02
+    _, raw, states = delta_oracle(d, seqs, 1e-5)
+    row, long = 0, []
+    for i, (n, prior, slot) in enumerate(seqs):
+        long.append(layered.Portion(i, row, n, prior, [], slot))
+        row += n
+    o = torch.zeros(row, H * V, device=run[0])
+    work = ops.delta_chunk_work(K, V, torch.device("cuda"))
+    g, = layered.chunk_groups(long, 1000, torch.device(run[0]))
+    ws = torch.full((work * H * len(g.chunks_host),), float("nan"),
+                    device=run[0])
+    ops.delta_chunk(d["q"], d["k"], d["v"], d["proj"], 5, d["decay"],
+                    d["bias"], d["neg_a"], d["state"], g, ws, o)
+    for h in range(H):
+        close(o.view(row, H, V)[:, h], raw[:, h], ("", torch.float32),
+              f32=3e-5)
+        for slot, S in states.items():
+            close(d["state"][slot][h], S[h], ("", torch.float32), f32=3e-5)
+
+
 def test_groups_are_full():
     """As few groups as hold all chunks, whatever the portions' lengths."""
     cpu = torch.device("cpu")
