@@ -1,7 +1,7 @@
-// linear_bind.h — torch binding of linear_rows.hip, linear_tiles.hip and
-// linear_act.hip, shared by the extensions. Products go to these kernels where
-// their rule holds, else to the library, of many rows in two calls where that is
-// faster.
+// linear_bind.h — torch binding of linear_rows.hip, linear_tiles.hip,
+// linear_split.hip and linear_act.hip, shared by the extensions. Products go to
+// these kernels where their rule holds, else to the library, of many rows in two
+// calls where that is faster.
 #pragma once
 #include <torch/extension.h>
 #include <ATen/autocast_mode.h>
@@ -21,6 +21,9 @@ hipError_t lds_gated_rows(const void*, int64_t, const void*, int64_t, void*,
                           int, int, int, int, hipStream_t);
 hipError_t lds_linear_act(const void*, int64_t, const void*, int64_t, void*,
                           int, int, int, int, int, hipStream_t);
+int lds_linear_split_plan(int64_t, int64_t, int64_t);
+hipError_t lds_linear_split(const void*, int64_t, const void*, int64_t, void*,
+                            float*, int, int, int, int, hipStream_t);
 hipError_t lds_lay_weights(const float*, void*, int, int, hipStream_t);
 }
 
@@ -94,6 +97,19 @@ inline bool many_rows(const Tensor& x, const Tensor& w, bool gated) {
   return M * N * 10 >= rounds * 256 * 256 * across * 7;
 }
 
+// The plan of a product of many rows in parts of K (linear_split.hip), 0 where it
+// is not taken
+inline int split_plan(const Tensor& x, const Tensor& w) {
+  if (!plain_matrices(x, w)) return 0;
+  const int plan = lds_linear_split_plan(x.size(0), w.size(0), x.size(1));
+  const int64_t limit = 1ll << 31;       // elements: offsets stay under 4 GiB
+  return plan && rows_of_16_bytes(x) && rows_of_16_bytes(w) &&
+                 x.size(0) < limit / x.stride(0) &&
+                 w.size(0) < limit / w.stride(0)
+             ? plan
+             : 0;
+}
+
 // Rows of a product of many that go in a call of their own: those that make up
 // whole rounds of tiles of 256 x 256 over the 256 compute units. The library
 // often takes a kernel of half the rate where the rest is little (14336 ->
@@ -149,9 +165,28 @@ inline Tensor linear_rows(const Tensor& x, const Tensor& w, bool f32) {
   return y;
 }
 
+// the parts [parts, M, N] of a product with a plan, and their sum in y if there is
+// one
+inline Tensor linear_split(const Tensor& x, const Tensor& w, int plan,
+                           const Tensor* y) {
+  const c10::DeviceGuard guard(x.device());
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  Tensor part = torch::empty({plan >> 16, M, N}, x.options().dtype(at::kFloat));
+  check(lds_linear_split(
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
+      y ? y->data_ptr() : nullptr, part.data_ptr<float>(), plan, M, N, K,
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return part;
+}
+
 // x [M, K] @ w' of w [N, K]
 inline Tensor linear(const Tensor& x, const Tensor& w) {
   if (few_rows(x, w, PLAIN)) return linear_rows(x, w, false);
+  if (const int plan = split_plan(x, w)) {
+    Tensor y = torch::empty({x.size(0), w.size(0)}, x.options());
+    linear_split(x, w, plan, &y);
+    return y;
+  }
   int64_t whole = 0;
   if (plain_matrices(x, w)) whole = whole_rounds(x.size(0), w.size(0), x.size(1));
   if (whole == 0) return at::matmul(x, w.t());
@@ -162,6 +197,8 @@ inline Tensor linear(const Tensor& x, const Tensor& w) {
   at::mm_out(y0, first, w.t());
   if (few_rows(rest, w, PLAIN))
     linear_rows(rest, w, y1, false);
+  else if (const int plan = split_plan(rest, w))
+    linear_split(rest, w, plan, &y1);
   else
     at::mm_out(y1, rest, w.t());
   return y;
@@ -170,7 +207,10 @@ inline Tensor linear(const Tensor& x, const Tensor& w) {
 // the same for a caller that sums the parts of K itself: [M, N], or 32-bit
 // [parts, M, N]
 inline Tensor linear_parts(const Tensor& x, const Tensor& w) {
-  if (!few_rows(x, w, PARTS)) return linear_bind::linear(x, w);
+  if (!few_rows(x, w, PARTS)) {
+    const int plan = split_plan(x, w);
+    return plan ? linear_split(x, w, plan, nullptr) : linear_bind::linear(x, w);
+  }
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const int parts = lds_linear_rows_parts(M, N, K);
   if (parts == 1) return linear_rows(x, w, false);
@@ -252,6 +292,8 @@ inline void bind(pybind11::module& m) {
   m.def("few_rows",
         [](const Tensor& x, const Tensor& w) { return few_rows(x, w, PLAIN); },
         "whether x @ w' takes the streaming kernel");
+  m.def("split_plan", &lds_linear_split_plan,
+        "rows of a tile | parts of K << 16 of such a product of many rows, or 0");
   m.def("whole_rounds", &whole_rounds,
         "rows of [M, K] @ [K, N] that go in a call of their own");
 }

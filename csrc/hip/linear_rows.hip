@@ -271,6 +271,21 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   return M <= 64 && N <= 4096;
 }
 
+// y [n] = the sum of part [parts, n], 16-byte aligned, n a multiple of 4
+hipError_t lds_sum_parts(const float* part, void* y, int64_t n, int parts,
+                         int f32, hipStream_t stream) {
+  const int64_t n4 = n / 4;
+  const dim3 grid((uint32_t)((n4 + 255) / 256));
+  if (f32)
+    hipLaunchKernelGGL(sum_parts_kernel<float>, grid, dim3(256), 0, stream,
+                       (const float4v*)part, (float*)y, n4, parts);
+  else
+    hipLaunchKernelGGL(sum_parts_kernel<short>, grid, dim3(256), 0, stream,
+                       (const float4v*)part, (short*)y, n4, parts);
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
 // x [M, K], w [N, K], rows x_row and w_row apart and 16-byte aligned; y [M, N]
 // bf16 or (f32) 32-bit. part: [parts, M, N] floats if parts > 1; without y
 // the result stays there.
@@ -296,16 +311,7 @@ hipError_t lds_linear_rows(const void* x, int64_t x_row, const void* w,
       e = two ? go<2, BF16>(p, 1, stream) : go<1, BF16>(p, 1, stream);
   }
   if (e != hipSuccess || !in_part || !y) return e;
-  const int64_t n4 = (int64_t)M * N / 4;
-  const dim3 grid((uint32_t)((n4 + 255) / 256));
-  if (f32)
-    hipLaunchKernelGGL(sum_parts_kernel<float>, grid, dim3(256), 0, stream,
-                       (const float4v*)part, (float*)y, n4, parts);
-  else
-    hipLaunchKernelGGL(sum_parts_kernel<short>, grid, dim3(256), 0, stream,
-                       (const float4v*)part, (short*)y, n4, parts);
-  HIP_CHECK_LAST();
-  return hipSuccess;
+  return lds_sum_parts(part, y, (int64_t)M * N, parts, f32, stream);
 }
 
 // in [R, C] 32-bit -> out [C, R] bf16

@@ -63,6 +63,7 @@ hip_ops = cpp_extension.CUDAExtension(
         "csrc/hip/linear_rows.hip",
         "csrc/hip/linear_tiles.hip",
         "csrc/hip/linear_act.hip",
+        "csrc/hip/linear_split.hip",
         "csrc/hip/prefix_kernels.hip",
         "csrc/hip/norm_rope_act.hip",
         "csrc/hip/kv_cache.hip",
@@ -80,6 +81,7 @@ hip_layered = cpp_extension.CUDAExtension(
         "csrc/hip/linear_rows.hip",
         "csrc/hip/linear_tiles.hip",
         "csrc/hip/linear_act.hip",
+        "csrc/hip/linear_split.hip",
         "csrc/hip/layered/residual_norm.hip",
         "csrc/hip/layered/delta_rule.hip",
         "csrc/hip/layered/delta_chunk.hip",

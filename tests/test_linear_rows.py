@@ -91,6 +91,53 @@ def test_gated_of_many_steps(rows, n, k):
 
 
 @pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("rows,n,k", [
+    (257, 1024, 5120), (384, 1288, 5184), (385, 1032, 8192), (512, 4088, 14336),
+    (513, 5120, 6400), (1000, 4096, 7168), (1300, 5120, 25600),
+    (2560, 1024, 16384)])
+def test_split_of_many_rows(name, rows, n, k):
+    """Tiles of 192 and 256 rows that are partly empty, channels that end inside a
+    tile, uneven parts of K, rows further apart than their length: each part is a
+    sum of its own K, and all are the product. Sums as in _same."""
+    ext = _ext(name)
+    plan = ext.split_plan(rows, n, k)
+    parts = plan >> 16
+    assert parts > 1 and plan % 65536 in (192, 256)
+    x = _draw(rows, k + 72, seed=rows)[:, 8:k + 8]
+    w = _draw(n, k, seed=n, scale=k ** -0.5)
+    want = x.double() @ w.double().t()
+    _same(ext.linear(x, w), want, 8)
+    got = ext.linear_parts(x, w)
+    assert got.shape == (parts, rows, n) and got.dtype == torch.float32
+    _same(got.double().sum(0), want, 16)
+    ends = [k // 64 * i // parts * 64 for i in range(parts + 1)]
+    for i in (0, parts - 1):
+        a, b = ends[i:i + 2]
+        _same(got[i], x[:, a:b].double() @ w[:, a:b].double().t(), 16)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    (256, 4096, 14336), (257, 4096, 5056), (257, 4096, 5128), (257, 1020, 8192),
+    (257, 1016, 8192), (257, 0, 8192), (0, 4096, 8192), (257, 4096, 0),
+    (2300, 5120, 25600), (2561, 1024, 16384), (1 << 62, 1 << 62, 1 << 62)])
+def test_products_that_stay_whole(rows, n, k):
+    """Few rows, short or odd K, odd or narrow widths, many rows, and what fills the
+    compute units."""
+    assert _ext("_hip_ops").split_plan(rows, n, k) == 0
+
+
+def test_split_of_what_is_left():
+    """Rows behind whole rounds of tiles, in a call of their own."""
+    ext = _ext("_hip_ops")
+    assert ext.whole_rounds(4400, 4096, 8192) == 4096
+    assert ext.split_plan(304, 4096, 8192)
+    x, w = _draw(4400, 8192, seed=1), _draw(4096, 8192, seed=2, scale=1 / 91)
+    y = ext.linear(x, w)
+    _same(y, x.double() @ w.double().t(), 8)
+    assert torch.equal(y[4096:], ext.linear(x[4096:], w))
+
+
+@pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("rows,n,k,one", [
     (640, 10880, 128, True), (560, 10872, 192, True), (897, 8192, 320, True),
@@ -255,12 +302,13 @@ def test_zeros_without_memory():
         assert y.shape == (rows, 64) and not y.any()
 
 
-@pytest.mark.parametrize("rows", [12, 60, 200])
-def test_capture_and_replay(rows):
+@pytest.mark.parametrize("rows,k", [(12, 4096), (60, 4096), (200, 4096),
+                                    (300, 8192)])
+def test_capture_and_replay(rows, k):
     """Partial sums are written anew by every replay."""
     ext = _ext("_hip_ops")
-    x, w = _draw(rows, 4096, seed=10), _draw(4096, 4096, seed=11, scale=1 / 64)
-    assert ext.few_rows(x, w)
+    x, w = _draw(rows, k, seed=10), _draw(4096, k, seed=11, scale=1 / 64)
+    assert rows > 256 or ext.few_rows(x, w)
     side = torch.cuda.Stream()
     with torch.cuda.stream(side):
         ext.linear(x, w)
@@ -269,7 +317,7 @@ def test_capture_and_replay(rows):
     with torch.cuda.graph(graph):
         y = ext.linear(x, w)
     for i in range(3):
-        x.copy_(_draw(rows, 4096, seed=20 + i))
+        x.copy_(_draw(rows, k, seed=20 + i))
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, ext.linear(x, w))
