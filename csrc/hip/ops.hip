@@ -2,6 +2,11 @@
 // Pure HIP (no hipify, no CUDA shims): includes the ROCm-native ATen HIP
 // headers directly and drives hipStream_t launchers from the .hip kernels.
 #include <torch/extension.h>
+#if PY_VERSION_HEX < 0x030B0000
+#include <longintrepr.h>
+#elif PY_VERSION_HEX < 0x030C0000
+#include <cpython/longintrepr.h>
+#endif
 #include <ATen/hip/HIPContext.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -101,13 +106,31 @@ std::vector<torch::Tensor> hash_prompts(torch::Tensor tokens,
                    n_req, block_tokens, max_blocks, seed0, tokens);
 }
 
+// A plain int of 32 bits, or false. Token ids have one digit, which is read where
+// it lies (a call for each took 1.2 ns, half of a burst's time); from Python 3.12 on
+// the digits lie elsewhere.
+inline bool int32_of(PyObject* x, int32_t* out) {
+  if (!PyLong_CheckExact(x)) return false;
+#if PY_VERSION_HEX < 0x030C0000
+  if (Py_SIZE(x) == 1) {
+    *out = (int32_t)((PyLongObject*)x)->ob_digit[0];    // at most 30 bits
+    return true;
+  }
+#endif
+  int overflow = 0;
+  const long v = PyLong_AsLongAndOverflow(x, &overflow);
+  *out = (int32_t)v;
+  return !overflow && v == (int32_t)v;
+}
+
 // hash_prompts of lists of python ints, for the device of `like`. They are
 // unpacked here, behind the offsets, so that one copy takes all (a burst of 48
-// prompts of 1000 tokens, hashed and matched: 71 us; by way of NumPy's arrays
-// 674, most of it in unpacking); the pinned buffer is torch's to give out again
+// prompts of 1000 tokens, hashed and matched: 45 us, 72 with a call for each int;
+// by way of NumPy's arrays 674, most of it in unpacking); the pinned buffer is torch's to give out again
 // once that copy is done, and larger bursts do without one. None where an element is not a plain int
 // of 32 bits: NumPy knows what to do with that.
 constexpr int64_t PINNED_WORDS = 1 << 19;       // 4 MB, a million tokens
+constexpr Py_ssize_t AHEAD = 16;
 c10::optional<std::vector<torch::Tensor>> hash_lists(
     py::list prompts, int64_t block_tokens, int64_t max_blocks, int64_t seed0,
     torch::Tensor like) {
@@ -128,14 +151,13 @@ c10::optional<std::vector<torch::Tensor>> hash_lists(
   for (int64_t i = 0; i < n; ++i) {
     PyObject* p = PyList_GET_ITEM(prompts.ptr(), i);
     const Py_ssize_t len = PyList_GET_SIZE(p);
+    PyObject* const* items = ((PyListObject*)p)->ob_item;
     for (Py_ssize_t t = 0; t < len; ++t) {
-      PyObject* x = PyList_GET_ITEM(p, t);
-      if (!PyLong_CheckExact(x)) return c10::nullopt;
-      int overflow = 0;
-      const long v = PyLong_AsLongAndOverflow(x, &overflow);
-      if (overflow || v != (int32_t)v) return c10::nullopt;
-      tokens[at++] = (int32_t)v;
+      // ints are objects of their own: those of a new prompt are in no near cache
+      __builtin_prefetch(items[t + AHEAD < len ? t + AHEAD : t]);
+      if (!int32_of(items[t], tokens + at + t)) return c10::nullopt;
     }
+    at += len;
     offsets[i + 1] = at;
   }
   const c10::DeviceGuard guard(like.device());

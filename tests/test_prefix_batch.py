@@ -72,3 +72,15 @@ def test_other_prompts(index):
             index.hash_prompts_batch([ids, bad], 16, 8, SEED0)
     hashes, counts = index.hash_prompts_batch([], 16, 8, SEED0)
     assert hashes.shape == (0, 8) and counts.shape == (0,)
+
+
+def test_ints_of_any_size(index):
+    """None, one or two digits of 30 bits, either sign, as NumPy reads them."""
+    ids = [0, 1, -1, 255, 256, -256, 2**30 - 1, 2**30, 1 - 2**30, -2**30,
+           2**31 - 1, -2**31, 7, 2**15, 2**16, -5] * 3
+    want = index.hash_prompts_batch([np.array(ids, dtype=np.int32)], 16, 8,
+                                    SEED0)
+    got = index.hash_prompts_batch([ids], 16, 8, SEED0)
+    assert int(got[1][0]) == 3
+    for a, b in zip(got, want):
+        assert a.cpu().numpy().tolist() == b.cpu().numpy().tolist()
