@@ -1,5 +1,6 @@
 // delta_chunk.hip — the gated delta rule of delta_rule.hip over chunks of 64
-// tokens, all in 32-bit on the matrix cores (v_mfma_f32_16x16x4f32).
+// tokens on the matrix cores, in 32-bit (v_mfma_f32_16x16x4f32) or, in the scan of
+// many sequences, in bf16 with each value in three parts, 24 bits.
 //
 // With G the running sum of log decays inside a chunk (token's own included)
 // and S0 the state before it, per head:
@@ -468,9 +469,46 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
 // of 16 columns. S lies in LDS between the chunks, as operands; a wave keeps
 // the tiles of it that it brings up to date, takes 16 tokens of the products
 // with it, and asks for a chunk's operands of these during the chunk before.
-// The matrix instructions bound it (60 us of 94 for 32 chunks of 8 sequences,
-// 32 heads of 128 x 128; 111 with one tile, 125 with all of S in the registers
-// of every wave and loads under conditions).
+//
+// In 32-bit the matrix instructions bound it: 223 us of 297 for 16 chunks of 8
+// sequences, 32 heads of 128 x 128. With two tiles values are sums of three bf16
+// instead, six products of which take 3/8 of the time: 254 us, 172 of them with
+// operands that are in cache (now the splitting of operands, 2400 instructions per
+// chunk and wave, and the waits), the error of outputs 3.52e-7 instead of 4.18e-7.
+// With one tile the splitting costs more than it saves (31 chunks of one sequence
+// 112 us, in 32-bit 91); four tiles do not fit the registers (+ 7 %).
+typedef __attribute__((ext_vector_type(8))) float float8v;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+template <int N> struct Vec;
+template <> struct Vec<4> { typedef float4v F; typedef bf16x4 H; };
+template <> struct Vec<8> { typedef float8v F; typedef bf16x8 H; };
+// 32-bit values as sums of three bf16 (high, middle, low): 24 bits of them
+template <int N>
+__device__ __forceinline__ void split(typename Vec<N>::F f,
+                                      typename Vec<N>::H (&o)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    o[i] = __builtin_convertvector(f, typename Vec<N>::H);
+    if (i < 2) f -= __builtin_convertvector(o[i], typename Vec<N>::F);
+  }
+}
+__device__ __forceinline__ void split2(float4v a, float4v b, bf16x8 (&o)[3]) {
+  split<8>(__builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7), o);
+}
+// products of 32 k, without those below 2^-24 of the largest: a[i] b[term - i]
+__device__ __forceinline__ float4v mfma_split(const bf16x8 (&a)[3],
+                                              const bf16x8 (&b)[3],
+                                              float4v c) {
+#pragma unroll
+  for (int term = 2; term >= 0; --term)
+#pragma unroll
+    for (int i = term; i >= 0; --i)
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[term - i], c, 0, 0,
+                                                  0);
+  return c;
+}
+
 template <int KT, int NC>
 __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     float* __restrict__ ws, float* __restrict__ state,  // [slots, H, K, V]
@@ -478,9 +516,29 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     int H, int K, int V, int VP) {
   constexpr int KP = KT * 16;
   constexpr int MY = (KT + 3) / 4;    // tiles of 16 rows of S per wave
-  __shared__ float4v s_lds[NC][KT][WAVE], u_lds[NC][4][WAVE];
+  constexpr bool SPLIT = NC > 1;
+  // tiles of 16 rows, 32-bit or split: a lane's values of two tiles together
+  constexpr int TILE = SPLIT ? WAVE * 3 / 2 : WAVE;
+  __shared__ float4v s_lds[NC][KT * TILE], u_lds[NC][4 * TILE];
   const int h = blockIdx.x, lane = threadIdx.x % WAVE;
   const int wave = threadIdx.x / WAVE, col = lane % 16, g4 = 4 * (lane / 16);
+  auto put = [&](float4v* to, int tile, float4v f) {
+    if constexpr (SPLIT) {
+      bf16x4 o[3];
+      split<4>(f, o);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        ((bf16x4*)(to + (tile / 2 * 3 + i) * WAVE + lane))[tile % 2] = o[i];
+    } else {
+      to[tile * WAVE + lane] = f;
+    }
+  };
+  auto get = [&](const float4v* from, int tile, bf16x8 (&o)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+      o[i] = __builtin_bit_cast(bf16x8,
+                                from[(tile / 2 * 3 + i) * WAVE + lane]);
+  };
   const int c0 = blockIdx.y * 16 * NC + col;
   const int4 m = ((const int4*)walk)[blockIdx.z];
   const int64_t row0 = m.x;
@@ -499,7 +557,7 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
         const int d = 16 * (wave + 4 * i) + g4 + r, c = c0 + 16 * x;
         S[x][i][r] = !fresh && d < K && c < V ? Sp[(int64_t)d * V + c] : 0.f;
       }
-      if (wave + 4 * i < KT) s_lds[x][wave + 4 * i][lane] = S[x][i];
+      if (wave + 4 * i < KT) put(s_lds[x], wave + 4 * i, S[x][i]);
     }
   lds_barrier();
 
@@ -555,24 +613,35 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     float4v o[NC];
 #pragma unroll
     for (int x = 0; x < NC; ++x) o[x] = (float4v){0.f, 0.f, 0.f, 0.f};
-    // sums take turns: a product waits for the one before it on its sum
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int t = 0; t < KT; ++t) {
-      float4v s[NC];
-#pragma unroll
-      for (int x = 0; x < NC; ++x) s[x] = s_lds[x][t][lane];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
+      for (int t = 0; t < KT; t += 2) {
+        bf16x8 ws[3], qs[3], ss[3];
+        split2(w[t], w[t + 1], ws);
+        split2(qe[t], qe[t + 1], qs);
 #pragma unroll
         for (int x = 0; x < NC; ++x) {
-          u[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][r], s[x][r], u[x],
-                                                      0, 0, 0);
-          o[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(qe[t][r], s[x][r], o[x],
-                                                      0, 0, 0);
+          get(s_lds[x], t, ss);
+          u[x] = mfma_split(ws, ss, u[x]);
+          o[x] = mfma_split(qs, ss, o[x]);
         }
+      }
+    } else {
+      // the sums take turns: a product waits for the one before it on its sum
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+        const float4v s = s_lds[0][t * WAVE + lane];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          u[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][r], s[r], u[0], 0, 0,
+                                                      0);
+          o[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(qe[t][r], s[r], o[0], 0,
+                                                      0, 0);
+        }
+      }
     }
 #pragma unroll
-    for (int x = 0; x < NC; ++x) u_lds[x][wave][lane] = u[x];
+    for (int x = 0; x < NC; ++x) put(u_lds[x], wave, u[x]);
     // w, qe and u are free now: the next chunk's arrive during the rest (the
     // last one's once more)
     if (t0 + C < n) base += stride;
@@ -582,33 +651,46 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     for (int x = 0; x < NC; ++x)
 #pragma unroll
       for (int i = 0; i < MY; ++i) S[x][i] = S[x][i] * decay[i];
+    if constexpr (SPLIT) {
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
-      float4v us[NC];
+      for (int y = 0; y < 4; y += 2) {
+        bf16x8 us[NC][3], ks[MY][3];
 #pragma unroll
-      for (int x = 0; x < NC; ++x) us[x] = u_lds[x][y][lane];
+        for (int i = 0; i < MY; ++i) split2(kt[i][y], kt[i][y + 1], ks[i]);
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int x = 0; x < NC; ++x)
+        for (int x = 0; x < NC; ++x) {
+          get(u_lds[x], y, us[x]);
 #pragma unroll
           for (int i = 0; i < MY; ++i)
-            S[x][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                kt[i][y][r], us[x][r], S[x][i], 0, 0, 0);
-      if (y <= wave) {
+            S[x][i] = mfma_split(ks[i], us[x], S[x][i]);
+        }
+        if (y <= wave) {
+          // of columns that P does not have nothing was written
+          bf16x8 ps[3];
+          split2(p[y], y < wave ? p[y + 1] : (float4v){0.f, 0.f, 0.f, 0.f},
+                 ps);
+#pragma unroll
+          for (int x = 0; x < NC; ++x) o[x] = mfma_split(ps, us[x], o[x]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        const float4v us = u_lds[0][y * WAVE + lane];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int x = 0; x < NC; ++x)
-            o[x] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[y][r], us[x][r],
-                                                        o[x], 0, 0, 0);
+          for (int i = 0; i < MY; ++i)
+            S[0][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(kt[i][y][r], us[r],
+                                                           S[0][i], 0, 0, 0);
+        if (y <= wave) o[0] = mfma4(p[y], us, o[0]);
       }
     }
 #pragma unroll
     for (int x = 0; x < NC; ++x)
 #pragma unroll
       for (int i = 0; i < MY; ++i)
-        if (wave + 4 * i < KT) s_lds[x][wave + 4 * i][lane] = S[x][i];
+        if (wave + 4 * i < KT) put(s_lds[x], wave + 4 * i, S[x][i]);
 #pragma unroll
     for (int x = 0; x < NC; ++x)
 #pragma unroll
