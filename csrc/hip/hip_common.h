@@ -96,6 +96,58 @@ __device__ __forceinline__ float block_reduce_sum(float v, float* scratch) {
   return total;
 }
 
+// The sums of `parts` 32-bit parts of a product that split K, of the 8 values at each
+// src[i]; apart: float4s from part to part. Up to 8 parts of all N are under way
+// together: summed one by one, or in a loop that the compiler unrolls by 4, each
+// few of them cost the latency of a cache that another XCD wrote behind.
+template <int N>
+struct PartSums {
+  float4v a[N][2];
+
+  __device__ __forceinline__ PartSums(const float4v* const (&src)[N],
+                                      int64_t apart, int parts) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)          // -0 leaves what is added as it is
+      a[i][0] = a[i][1] = (float4v){-0.f, -0.f, -0.f, -0.f};
+    int k = 0;
+    for (; k + 8 <= parts; k += 8) add<8>(src, apart, k);
+    switch (parts - k) {
+      case 7: add<7>(src, apart, k); break;
+      case 6: add<6>(src, apart, k); break;
+      case 5: add<5>(src, apart, k); break;
+      case 4: add<4>(src, apart, k); break;
+      case 3: add<3>(src, apart, k); break;
+      case 2: add<2>(src, apart, k); break;
+      case 1: add<1>(src, apart, k); break;
+    }
+  }
+  template <int G>
+  __device__ __forceinline__ void add(const float4v* const (&src)[N],
+                                      int64_t apart, int first) {
+    float4v g[G][N][2];
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) g[k][i][j] = src[i][(first + k) * apart + j];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) a[i][j] += g[k][i][j];
+  }
+  __device__ __forceinline__ void get(int i, float* f) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      f[j] = a[i][0][j];
+      f[4 + j] = a[i][1][j];
+    }
+  }
+};
+
 #define HIP_CHECK_LAST()                                              \
   do {                                                                 \
     hipError_t e_ = hipGetLastError();                                 \

@@ -16,7 +16,8 @@ namespace {
 //   y = src * rsqrt(mean(src^2) + eps) * w
 // x is bf16, or the partial sums of a product that split K: [parts, rows, H]
 // 32-bit, summed here instead of by a launch of their own (8 parts, one row of
-// 4096: 6.5 us; sum and norm apart 8.7).
+// 4096: 4.5 us, 6.5 with few loads under way; sum and norm apart 8.7; 30 rows of
+// 5120 6.7, were 7.6, 256 of 4096 8.6, were 9.6).
 // One block (256 threads) per token row; row length H % 8 == 0. The first KEEP
 // vectors of a thread stay in registers between the two passes, the rest are
 // read again. Their number is known at compile time: an index that is not puts
@@ -35,19 +36,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
   auto source = [&](int c, float* f) {
     if constexpr (PARTS) {
-      const float4v* p = (const float4v*)x + (row * H + c * 8) / 4;
-      const int64_t apart = (int64_t)gridDim.x * H / 4;
-      float4v a = p[0], b = p[1];
-#pragma unroll 4
-      for (int i = 1; i < parts; ++i) {
-        a += p[i * apart];
-        b += p[i * apart + 1];
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f[j] = a[j];
-        f[4 + j] = b[j];
-      }
+      const float4v* const p[1] = {(const float4v*)x + (row * H + c * 8) / 4};
+      PartSums<1>(p, (int64_t)gridDim.x * H / 4, parts).get(0, f);
     } else {
       const short8 v = ((const short8*)((const short*)x + row * H))[c];
 #pragma unroll
@@ -55,10 +45,33 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     }
   };
   float vals[KEEP][8], ss = 0.f;
-  auto first = [&](int c, float* f) {
-    source(c, f);
+  // with parts, all that a thread keeps is asked for at once, pair by pair
+  constexpr bool EARLY = PARTS && KEEP > 1;
+  short8 rv[EARLY ? KEEP : 1], wk[EARLY ? KEEP : 1];
+  if constexpr (EARLY) {
+    const int64_t apart = (int64_t)gridDim.x * H / 4;
+#pragma unroll
+    for (int i = 0; i < KEEP; ++i) {
+      const int c = min((int)threadIdx.x + i * NT, nchunks - 1);
+      if constexpr (RESIDUAL) rv[i] = r8[c];
+      wk[i] = ((const short8*)w)[c];
+    }
+#pragma unroll
+    for (int i = 0; i < KEEP; i += 2) {
+      const float4v* p[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        p[j] = (const float4v*)x + row * H / 4 +
+               min((int)threadIdx.x + (i + j) * NT, nchunks - 1) * 2;
+      const PartSums<2> sum(p, apart, parts);
+      sum.get(0, vals[i]);
+      sum.get(1, vals[i + 1]);
+    }
+  }
+  auto first = [&](int c, float* f, int i) {
+    if (!EARLY || i < 0) source(c, f);
     if constexpr (RESIDUAL) {
-      const short8 r = r8[c];
+      const short8 r = EARLY && i >= 0 ? rv[EARLY ? i : 0] : r8[c];
       short8 ro;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -73,16 +86,17 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
     const int c = threadIdx.x + i * NT;
-    if (c < nchunks) first(c, vals[i]);
+    if (c < nchunks) first(c, vals[i], i);
   }
   for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
     float f[8];
-    first(c, f);
+    first(c, f, -1);
   }
   const float inv =
       rsqrtf(block_reduce_sum<NT / WAVE>(ss, red) / (float)H + eps);
-  auto second = [&](int c, const float* f) {
-    const short8 wv = ((const short8*)w)[c];
+  auto second = [&](int c, const float* f, int i) {
+    const short8 wv =
+        EARLY && i >= 0 ? wk[EARLY ? i : 0] : ((const short8*)w)[c];
     short8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -92,7 +106,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
     const int c = threadIdx.x + i * NT;
-    if (c < nchunks) second(c, vals[i]);
+    if (c < nchunks) second(c, vals[i], i);
   }
   for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
     float f[8];
@@ -103,7 +117,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     } else {
       source(c, f);
     }
-    second(c, f);
+    second(c, f, -1);
   }
 }
 

@@ -367,6 +367,47 @@ def test_parts_in_norms(rows):
               (wn.double() + 0.5), 8)
 
 
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 6, 7, 8, 9, 15, 16, 17])
+@pytest.mark.parametrize("rows,width", [(3, 8), (2, 2040), (2, 2056), (2, 4104),
+                                        (1, 8200), (2, 8192), (1, 16392)])
+def test_norms_of_any_parts(rows, width, parts):
+    """Whole and rest groups of 8 parts; threads that keep none, some or all of
+    their vectors. Sums of up to 17 values of size 1: 32-bit ones within 1e-5; the
+    rest as in _same."""
+    from llm_d_inference_scheduler_amd.ops import layered
+    hip = _ext("_hip_ops")
+    g = torch.Generator("cuda").manual_seed(width + parts)
+    y = torch.randn(parts, rows, width, device="cuda", generator=g)
+    y /= parts ** 0.5
+    full, gain = y.double().sum(0), _draw(width, seed=3)
+
+    def normed(z):
+        return z * (z.square().mean(-1, keepdim=True) + 1e-5).rsqrt()
+    for start in (None, _draw(rows, width, seed=4)):
+        residual = None if start is None else start.clone()
+        got = hip.rmsnorm(y, gain, 1e-5, residual)
+        src = full if start is None else full + start.double()
+        if residual is not None:
+            _same(residual, src, 8)
+        # what does not stay in registers is read again from the residual, whose
+        # rounding (2^-8) comes on top of the result's
+        twice = residual is not None and width > 8192
+        _same(got, normed(src) * gain.double(), 7 if twice else 8)
+    wb, wn = gain.float(), _draw(width, seed=5).float()
+    rows_of = _draw(2 * rows, width, seed=7)
+    for post in (None, wb):
+        for more in (None, rows_of):
+            z = full if post is None else normed(full) * (post.double() + 0.5)
+            if more is not None:
+                z = z + more.double().view(rows, 2, width).sum(1)
+            mine = _draw(rows, width, seed=6).float()
+            s = mine.double() + z
+            h = layered.stream_norm(mine, y, post, wn, 0.5, 1e-5,
+                                    torch.bfloat16, more)
+            torch.testing.assert_close(mine.double(), s, rtol=1e-5, atol=1e-5)
+            _same(h, normed(s) * (wn.double() + 0.5), 8)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("T,qh,kvh,d,bs", [(1, 4, 1, 128, 16),
