@@ -1,6 +1,6 @@
 // linear_act.hip — y = act(x gate') * (x up') and y = act(x w') for many rows
-// (bf16, 32-bit sums): tiles of 256 weight rows by 256 rows of x by the loop of
-// tile_core.h, the activation in the sums' registers.
+// (bf16, 32-bit sums): tiles of 256 weight rows by 256 or 192 rows of x by the loop
+// of tile_core.h, the activation in the sums' registers.
 //
 // The library's product of the same weights is 3 % faster, but its result, twice
 // as wide where a gate is in it, goes to memory and comes back for the activation:
@@ -12,11 +12,11 @@
 
 namespace {
 
-typedef TileCore<8, 8, 2, 2> Whole;      // 256 rows
+template <int PT> using Whole = TileCore<8, PT, 2, 2>;    // 32 PT rows
 typedef TileCore<4, 8, 4, 2> Half;       // the last tile, of up to 128
-constexpr int BC = Whole::CHANNELS, BR = Whole::ROWS;
-static_assert(Half::CHANNELS == BC && Half::CH == Whole::CH &&
-                  Half::LDS_TURN <= Whole::LDS_TURN,
+constexpr int BC = Whole<8>::CHANNELS;
+static_assert(Half::CHANNELS == BC && Half::CH == Whole<8>::CH &&
+                  Half::LDS_TURN <= Whole<6>::LDS_TURN,
               "");
 constexpr int TG = 4;        // tiles of rows that walk the channels together
 
@@ -79,9 +79,10 @@ __device__ __forceinline__ void tile(const Product& p, short* lds, int m0, int b
         });
 }
 
-template <int ACT, bool GATED>
+template <int ACT, bool GATED, int PT>
 __global__ __launch_bounds__(256, 1) void linear_act_kernel(const Product p) {
   extern __shared__ __align__(16) short act_lds[];
+  constexpr int BR = Whole<PT>::ROWS;
   // Workgroups go round the 8 XCDs in turn: each gets a contiguous share of the
   // tiles, in which TG tiles of rows walk the channels together.
   constexpr int width = GATED ? BC / 2 : BC;
@@ -92,46 +93,76 @@ __global__ __launch_bounds__(256, 1) void linear_act_kernel(const Product p) {
   const int side = min(TG, ny - g * TG);
   const int m0 = (g * TG + in % side) * BR, blk = in / side;
   if (p.M - m0 > Half::ROWS)
-    tile<ACT, GATED, Whole>(p, act_lds, m0, blk);
+    tile<ACT, GATED, Whole<PT>>(p, act_lds, m0, blk);
   else
     tile<ACT, GATED, Half>(p, act_lds, m0, blk);
 }
 
-template <int ACT, bool GATED>
+template <int ACT, bool GATED, int PT>
 hipError_t go(const Product& p, hipStream_t stream) {
-  constexpr int width = GATED ? BC / 2 : BC;
+  constexpr int width = GATED ? BC / 2 : BC, BR = Whole<PT>::ROWS;
+  constexpr int bytes = Whole<PT>::LDS_TURN;
   const int64_t n = (int64_t)((p.N + width - 1) / width) * ((p.M + BR - 1) / BR);
   if (n > 1 << 24) return hipErrorInvalidValue;
-  auto fn = linear_act_kernel<ACT, GATED>;
+  auto fn = linear_act_kernel<ACT, GATED, PT>;
   const hipError_t e = hipFuncSetAttribute(
-      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-      Whole::LDS_TURN);
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3((uint32_t)((n + 7) / 8 * 8)), dim3(256),
-                     Whole::LDS_TURN, stream, p);
+  hipLaunchKernelGGL(fn, dim3((uint32_t)((n + 7) / 8 * 8)), dim3(256), bytes,
+                     stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }
 
 }  // namespace
 
+extern "C" {
+
+// Rows of a tile with which a product of many rows and its activation are one
+// kernel: 256, or 192 where these fill their rounds over the compute units better by
+// 1.08 (they are that much slower per row); 0 below 11/20 of a round's work. us,
+// library and activation / here, behind it rows of a tile and how full. 4096 -> [2 x
+// 14336]: 283 rows 96 / 70 (192, 64 %), 391 123 / 99 (256, 67 %), 524 152 / 139 (192,
+// 60 %), 744 176 / 144 (192, 85 %; 256, 64 %: 172), 1014 213 / 180 (256, 87 %), 8190
+// 1415 / 1298. 2048 -> [2 x 8192]: 565 rows 50 / 37 (192, 74 %), 1232 92 / 75 (192, 80
+// %). 5120 -> [2 x 25600]: 320 rows 205 / 176 (192, 65 %), 1005 528 / 429 (256, 77 %;
+// 192, 82 %: 468). 4096 -> 7168: 732 rows 61 / 66 (192, 42 %), 1047 69 / 62 (192, 60 %),
+// 8190 376 / 352 (256). 2048 -> 4096: 925 rows 31 / 33 (30 %), 2809 57 / 40 (192, 91 %).
+// 5120 -> 12800: 565 rows 89 / 87 (192, 57 %).
+int lds_linear_act_rows(int64_t M, int64_t N, int64_t K, int gated) {
+  const int64_t width = gated ? BC / 2 : BC;
+  if (M <= 256 || K < 2 * TILE_K || K % TILE_K || N < 8 || N % 8) return 0;
+  auto cost = [&](int64_t rows) {
+    const int64_t tiles = (M + rows - 1) / rows * ((N + width - 1) / width);
+    return (tiles + 255) / 256 * 256 * rows * width;
+  };
+  const int rows = cost(192) * 108 < cost(256) * 100 ? 192 : 256;
+  return M * N * 20 >= cost(rows) * 11 ? rows : 0;
+}
+
 // y [M, N] = act(x gate') * (x up') of w [2 N, K] = [gate; up], or (not gated)
 // act(x w') of w [N, K]; rows x_row and w_row apart, 16-byte aligned; K a multiple
-// of 64 from 128 on, N one of 8.
-extern "C" hipError_t lds_linear_act(const void* x, int64_t x_row,
-                                     const void* w, int64_t w_row, void* y,
-                                     int M, int N, int K, int act, int gated,
-                                     hipStream_t stream) {
+// of 64 from 128 on, N one of 8; tiles of `rows` rows (192 or 256).
+hipError_t lds_linear_act(const void* x, int64_t x_row, const void* w,
+                          int64_t w_row, void* y, int rows, int M, int N,
+                          int K, int act, int gated, hipStream_t stream) {
   const int64_t xb = ((M - 1) * x_row + K) * 2;
   const int64_t wb = (((gated ? 2 : 1) * (int64_t)N - 1) * w_row + K) * 2;
   if (M < 1 || N < 8 || N % 8 || K < 2 * TILE_K || K % TILE_K || x_row % 8 ||
-      w_row % 8 || act < 0 || act >= ACTS || xb >= 1ll << 32 || wb >= 1ll << 32)
+      w_row % 8 || act < 0 || act >= ACTS || (rows != 192 && rows != 256) ||
+      xb >= 1ll << 32 || wb >= 1ll << 32)
     return hipErrorInvalidValue;
   const Product p{(const short*)x, (const short*)w, x_row, w_row, (short*)y,
               M, N, K, act, (uint32_t)xb, (uint32_t)wb};
-#define GO(A) return gated ? go<A, true>(p, stream) : go<A, false>(p, stream)
+#define GO(A)                                                                \
+  return rows == 192                                                         \
+             ? gated ? go<A, true, 6>(p, stream) : go<A, false, 6>(p, stream) \
+         : gated ? go<A, true, 8>(p, stream)                                 \
+                 : go<A, false, 8>(p, stream)
   if (act == ACT_SILU) GO(ACT_SILU);
   if (act == ACT_RELU_SQUARED) GO(ACT_RELU_SQUARED);
   GO(ACT_GELU_TANH);
 #undef GO
 }
+
+}  // extern "C"

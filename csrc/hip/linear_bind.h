@@ -19,8 +19,9 @@ hipError_t lds_linear_rows(const void*, int64_t, const void*, int64_t, void*,
                            float*, int, int, int, int, int, hipStream_t);
 hipError_t lds_gated_rows(const void*, int64_t, const void*, int64_t, void*,
                           int, int, int, int, hipStream_t);
+int lds_linear_act_rows(int64_t, int64_t, int64_t, int);
 hipError_t lds_linear_act(const void*, int64_t, const void*, int64_t, void*,
-                          int, int, int, int, int, hipStream_t);
+                          int, int, int, int, int, int, hipStream_t);
 int lds_linear_split_plan(int64_t, int64_t, int64_t);
 hipError_t lds_linear_split(const void*, int64_t, const void*, int64_t, void*,
                             float*, int, int, int, int, hipStream_t);
@@ -74,27 +75,16 @@ inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
          rows_of_16_bytes(x) && rows_of_16_bytes(w);
 }
 
-// Whether a product of many rows and its activation are one kernel
-// (linear_act.hip): where its tiles fill 7/10 of their rounds over the compute
-// units. us, library and activation / here, behind it how full: 4096 -> [2 x
-// 14336], 600 rows 149 / 165 (51 %), 1000 202 / 197 (85 %), 2000 383 / 358 (85 %),
-// 8190 1415 / 1298; 2048 -> [2 x 8192], 4200 rows 249 / 239 (82 %), 1000 68 / 51 (98
-// %); 5120 -> [2 x 25600], 1000 rows 528 / 441 (76 %); 4096 -> 7168, 3000 rows 168 /
-// 163 (64 %), 8190 376 / 352 (87 %); 2048 -> 4096, 8533 rows 138 / 137 (69 %), 6000
-// 102 / 94 (73 %), 4200 74 / 87 (51 %).
-inline bool many_rows(const Tensor& x, const Tensor& w, bool gated) {
-  if (!plain_matrices(x, w)) return false;
-  const int64_t M = x.size(0), K = x.size(1), across = gated ? 128 : 256;
-  const int64_t N = gated ? w.size(0) / 2 : w.size(0);
-  const int64_t limit = 1ll << 31;       // elements: offsets stay under 4 GiB
-  if (M <= 256 || K < 128 || K % 64 || N < 8 || N % 8 ||
-      (gated && w.size(0) % 2) || M >= limit / K || w.size(0) >= limit / K ||
+// Rows of a tile where a product of many rows and its activation are one kernel
+// (linear_act.hip), else 0
+inline int many_rows(const Tensor& x, const Tensor& w, bool gated) {
+  if (!plain_matrices(x, w) || (gated && w.size(0) % 2)) return 0;
+  const int64_t M = x.size(0), K = x.size(1), limit = 1ll << 31;
+  if (K < 1 || M >= limit / K || w.size(0) >= limit / K ||
       !rows_of_16_bytes(x) || !rows_of_16_bytes(w) ||
       M * x.stride(0) >= limit || w.size(0) * w.stride(0) >= limit)
-    return false;
-  const int64_t tiles = (M + 255) / 256 * ((N + across - 1) / across);
-  const int64_t rounds = (tiles + 255) / 256;
-  return M * N * 10 >= rounds * 256 * 256 * across * 7;
+    return 0;               // offsets stay under 4 GiB
+  return lds_linear_act_rows(M, w.size(0) / (gated ? 2 : 1), K, gated);
 }
 
 // The plan of a product of many rows in parts of K (linear_split.hip), 0 where it
@@ -230,14 +220,14 @@ inline c10::optional<Tensor> linear32(const Tensor& x, const Tensor& w) {
 }
 
 inline Tensor linear_act(const Tensor& x, const Tensor& w, int64_t act,
-                         bool gated) {
+                         bool gated, int rows) {
   const c10::DeviceGuard guard(x.device());
   const int M = (int)x.size(0), K = (int)x.size(1);
   const int N = (int)w.size(0) / (gated ? 2 : 1);
   Tensor y = torch::empty({M, N}, x.options());
   check(lds_linear_act(
-      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), M, N,
-      K, (int)act, gated,
+      x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(), rows,
+      M, N, K, (int)act, gated,
       at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
   return y;
 }
@@ -246,7 +236,8 @@ inline Tensor linear_act(const Tensor& x, const Tensor& w, int64_t act,
 // and the activation have to be two calls
 inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
                                           int64_t act) {
-  if (many_rows(x, w, true)) return linear_act(x, w, act, true);
+  if (const int rows = many_rows(x, w, true))
+    return linear_act(x, w, act, true, rows);
   if (!few_rows(x, w, GATED)) return c10::nullopt;
   const c10::DeviceGuard guard(x.device());
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0) / 2;
@@ -260,8 +251,9 @@ inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
 // act(x w'), or None as above
 inline c10::optional<Tensor> activated_linear(const Tensor& x, const Tensor& w,
                                               int64_t act) {
-  if (!many_rows(x, w, false)) return c10::nullopt;
-  return linear_act(x, w, act, false);
+  const int rows = many_rows(x, w, false);
+  if (!rows) return c10::nullopt;
+  return linear_act(x, w, act, false, rows);
 }
 
 // drawn weights [in, out] in 32-bit -> [out, in] in bf16
@@ -292,6 +284,8 @@ inline void bind(pybind11::module& m) {
   m.def("few_rows",
         [](const Tensor& x, const Tensor& w) { return few_rows(x, w, PLAIN); },
         "whether x @ w' takes the streaming kernel");
+  m.def("act_rows", &lds_linear_act_rows,
+        "rows of a tile of a product and its activation in one kernel, or 0");
   m.def("split_plan", &lds_linear_split_plan,
         "rows of a tile | parts of K << 16 of such a product of many rows, or 0");
   m.def("whole_rounds", &whole_rounds,

@@ -254,13 +254,13 @@ struct TileCore {
     if (s < steps) step(integral_constant<int, 0>{});
   }
 
-  // Results of rows row(2 b) to row(2 b + 1) + 15 and of the first NC tiles of
+  // Results of 16 rows from row(2 b), 16 from row(2 b + 1) and the first NC tiles of
   // channels, f(c, t, x) for what acc[c][t][x] stands for, as bf16. The wave's share
   // of LDS behind the ring turns them round so that they leave in whole lines:
   // store(row of the 32, row of the tile, channel of the tile, 8 values).
   template <int NC, typename F, typename S>
   __device__ __forceinline__ void turn(short* lds, int b, F f, S store) const {
-    static_assert(QP % 2 == 0 && NC <= CT, "");
+    static_assert(PT % 2 == 0 && NC <= CT, "");
     constexpr int G = 2 * NC;            // pieces of 8 channels in a row
     static_assert(G == 16 || G == 8 || G == 4, "");
     short* mine = lds + RING + wave * TURN;
@@ -283,7 +283,8 @@ struct TileCore {
 #pragma unroll
     for (int j = 0; j < 32; j += WAVE / G) {
       const int r = j + lane / G;
-      store(r, row(2 * b) + r, channel(g / 2) + g % 2 * 8,
+      store(r, (j < 16 ? row(2 * b) : row(2 * b + 1) - 16) + r,
+            channel(g / 2) + g % 2 * 8,
             *(const short8*)(mine + place(r, g)));
     }
     asm volatile("" ::: "memory");

@@ -139,15 +139,17 @@ def test_split_of_what_is_left():
 
 @pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("gated", [True, False])
-@pytest.mark.parametrize("rows,n,k,one", [
-    (640, 10880, 128, True), (560, 10872, 192, True), (897, 8192, 320, True),
-    (1024, 8136, 256, True), (512, 16384, 64, False), (640, 10880, 136, False),
-    (512, 8192, 128, False)])
-def test_act_of_many_rows(name, gated, rows, n, k, one):
-    """Tiles of 256 rows and a last one of up to 128 or more, channels that end
-    inside a tile, even and odd numbers of steps, rows that lie apart; what does
+@pytest.mark.parametrize("rows,n,k,tile", [
+    (640, 10880, 128, 256), (560, 10872, 192, 192), (897, 8192, 320, 256),
+    (1024, 8136, 256, 256), (350, 14344, 128, 192), (300, 14344, 192, 192),
+    (1153, 8128, 128, 192), (512, 16384, 64, 0), (640, 10880, 136, 0),
+    (300, 8192, 128, 0)])
+def test_act_of_many_rows(name, gated, rows, n, k, tile):
+    """Tiles of 256 and 192 rows and a last one of up to 128 or more, channels that
+    end inside a tile, even and odd numbers of steps, rows that lie apart; what does
     not fill its rounds of tiles and other sizes of K stay apart."""
-    F, ext = torch.nn.functional, _ext(name)
+    F, ext, one = torch.nn.functional, _ext(name), tile > 0
+    assert ext.act_rows(rows, n if gated else 2 * n, k, gated) == tile
     n *= 1 if gated else 2
     x = _draw(rows, k + 8, seed=rows)[:, :k]
     w = _draw(2 * n if gated else n, k + 16, seed=n, scale=k ** -0.5)[:, 8:-8]
