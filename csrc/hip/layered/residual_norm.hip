@@ -75,7 +75,11 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
       if (i * NT * N < H) ldn<N>(xr + min(at(i), (int64_t)H - N), xk[i]);
 #pragma unroll
     for (int i = 0; i < KEEP; i += 2)
-      if (i * NT * N < H) {
+      if (i * NT * N < H && (i + 1) * NT * N >= H) {     // the last one alone
+        const float4v* const src[1] = {
+            (const float4v*)(s.yp + row * H + min(at(i), (int64_t)H - N))};
+        PartSums<1>(src, (int64_t)gridDim.x * H / 4, s.parts).get(0, keep[i]);
+      } else if (i * NT * N < H) {
         const float4v* src[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
