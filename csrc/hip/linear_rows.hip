@@ -150,16 +150,19 @@ __global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
   }
 }
 
-// sum of the parts; n4: float4s of one
+// sum of the parts, or (act >= 0) the activation of it; n4: float4s of one
 template <typename T>
 __global__ __launch_bounds__(256) void sum_parts_kernel(
     const float4v* __restrict__ part, T* __restrict__ y, int64_t n4,
-    int parts) {
+    int parts, int act) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n4) return;
   float4v s = part[i];
 #pragma unroll 8
   for (int k = 1; k < parts; ++k) s += part[k * n4 + i];
+  if (act >= 0)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s[j] = activate(act, s[j]);
   if constexpr (sizeof(T) == 4)
     ((float4v*)y)[i] = s;
   else
@@ -271,17 +274,20 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   return M <= 64 && N <= 4096;
 }
 
-// y [n] = the sum of part [parts, n], 16-byte aligned, n a multiple of 4
+// y [n] = the sum of part [parts, n], or (act >= 0) its activation; 16-byte aligned, n
+// a multiple of 4
 hipError_t lds_sum_parts(const float* part, void* y, int64_t n, int parts,
-                         int f32, hipStream_t stream) {
+                         int f32, int act, hipStream_t stream) {
+  if (n < 0 || n % 4 || act >= ACTS) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
   const int64_t n4 = n / 4;
   const dim3 grid((uint32_t)((n4 + 255) / 256));
   if (f32)
     hipLaunchKernelGGL(sum_parts_kernel<float>, grid, dim3(256), 0, stream,
-                       (const float4v*)part, (float*)y, n4, parts);
+                       (const float4v*)part, (float*)y, n4, parts, act);
   else
     hipLaunchKernelGGL(sum_parts_kernel<short>, grid, dim3(256), 0, stream,
-                       (const float4v*)part, (short*)y, n4, parts);
+                       (const float4v*)part, (short*)y, n4, parts, act);
   HIP_CHECK_LAST();
   return hipSuccess;
 }
@@ -311,7 +317,7 @@ hipError_t lds_linear_rows(const void* x, int64_t x_row, const void* w,
       e = two ? go<2, BF16>(p, 1, stream) : go<1, BF16>(p, 1, stream);
   }
   if (e != hipSuccess || !in_part || !y) return e;
-  return lds_sum_parts(part, y, (int64_t)M * N, parts, f32, stream);
+  return lds_sum_parts(part, y, (int64_t)M * N, parts, f32, -1, stream);
 }
 
 // in [R, C] 32-bit -> out [C, R] bf16

@@ -125,7 +125,7 @@ int lds_linear_split_plan(int64_t M, int64_t N, int64_t K) {
 }
 
 hipError_t lds_sum_parts(const float* part, void* y, int64_t n, int parts,
-                         int f32, hipStream_t stream);
+                         int f32, int act, hipStream_t stream);
 
 // x [M, K], w [N, K], rows x_row and w_row apart, 16-byte aligned, K a multiple of 64
 // with 128 per part at least, N one of 4; plan: of the function above. part [parts,
@@ -145,7 +145,7 @@ hipError_t lds_linear_split(const void* x, int64_t x_row, const void* w,
                   M, N, K, parts, (uint32_t)xb, (uint32_t)wb};
   const hipError_t e = rows == 192 ? go<6>(p, stream) : go<8>(p, stream);
   if (e != hipSuccess || !y) return e;
-  return lds_sum_parts(part, y, (int64_t)M * N, parts, 0, stream);
+  return lds_sum_parts(part, y, (int64_t)M * N, parts, 0, -1, stream);
 }
 
 }  // extern "C"

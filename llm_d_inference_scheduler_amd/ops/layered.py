@@ -49,7 +49,7 @@ def gated_linear(x, w, act):
 
 
 def activated_linear(x, w, act):
-    """act(x @ w'), one kernel for many rows."""
+    """act(x @ w'), one kernel for many rows, the sum of its parts for few."""
     if x.is_cuda:
         y = hip_layered().activated_linear(x, w, ACTS[act])
         if y is not None:

@@ -164,6 +164,22 @@ def test_act_of_many_rows(name, gated, rows, n, k, tile):
             _same(y, fn(g) * u, 8)
 
 
+@pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("rows,n,k", [(1, 8, 512), (16, 4096, 520), (17, 7168, 4096),
+                                      (64, 4088, 8192), (60, 30000, 264)])
+def test_act_of_few_rows(name, rows, n, k):
+    """The activation where the parts of K are summed; one part stays apart."""
+    F, ext = torch.nn.functional, _ext(name)
+    x, w = _draw(rows, k, seed=rows), _draw(n, k, seed=n, scale=k ** -0.5)
+    z = x.double() @ w.double().t()
+    for act, fn in enumerate([lambda z: F.gelu(z, approximate="tanh"), F.silu,
+                              lambda z: z.relu().square()]):
+        y = ext.activated_linear(x, w, act)
+        assert (y is None) == (n == 30000)
+        if y is not None:
+            _same(y, fn(z), 8)
+
+
 @pytest.mark.parametrize("act", [0, 1, 2])
 def test_act_of_large_sums(act):
     """Infinities and what overflows come out as they do apart."""
