@@ -34,6 +34,8 @@
 // merges partitions: m* = max m_p; o = sum o_p*exp(m_p-m*); l likewise.
 #include "hip_common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int D = 128;        // head_dim (Llama-3 family)
@@ -142,6 +144,16 @@ __device__ __forceinline__ void split3(const float4v* x, bf16x8* parts) {
   }
 }
 
+// values as they are, but infinite ones 0
+__device__ __forceinline__ uint4v finite(uint4v v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if ((v[i] & 0x7fffu) == 0x7f80u) v[i] &= 0xffff0000u;
+    if ((v[i] & 0x7fff0000u) == 0x7f800000u) v[i] &= 0xffffu;
+  }
+  return v;
+}
+
 // PAGE16: pages of 16 tokens and partitions that begin on a page, so half a
 // tile lies in one page; else every lane looks its tokens up one by one.
 template <typename CT, bool SPLIT, bool PAGE16, int NW>
@@ -245,81 +257,111 @@ __global__ __launch_bounds__(NW * WAVE, 3) void paged_attention_kernel(
       }
   };
 
-  int t0 = t_begin + wave * TILE;
-  if (t0 < t_end) {
-    find(t0);
-    fetch_k(t0);
-    fetch_v(t0);
-  }
-  for (; t0 < t_end; t0 += NW * TILE) {
-    const int next = t0 + NW * TILE;
-    const bool more = next < t_end;
-    if (more) find(next);
-    float4v sc[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      sc[h] = (float4v){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(C::key(kr[h], s),
-                                                        qf[s], sc[h], 0, 0, 0);
+  // ENDLESS: infinite values are no part of the lower products; no tile is read
+  // ahead, which would take more registers than there are
+  auto walk = [&](auto endless) {
+    constexpr bool ENDLESS = decltype(endless)::value;
+    int t0 = t_begin + wave * TILE;
+    if (!ENDLESS && t0 < t_end) {
+      find(t0);
+      fetch_k(t0);
+      fetch_v(t0);
     }
-    if (more) fetch_k(next);
+    for (; t0 < t_end; t0 += NW * TILE) {
+      const int next = t0 + NW * TILE;
+      const bool more = !ENDLESS && next < t_end;
+      if (ENDLESS) {
+        find(t0);
+        fetch_k(t0);
+        fetch_v(t0);
+      }
+      if (more) find(next);
+      float4v sc[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        sc[h] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          sc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(C::key(kr[h], s),
+                                                          qf[s], sc[h], 0, 0, 0);
+      }
+      if (more) fetch_k(next);
 
-    const bool tail = t0 + TILE > t_end;      // wave-uniform
-    float mx = NEG;
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sc[h][r] *= scale_log2;
-        if (tail && t0 + h * 16 + g * 4 + r >= t_end) sc[h][r] = -INFINITY;
-        mx = fmaxf(mx, sc[h][r]);
-      }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
-    const bool moved = mx > m + SLACK;
-    if (__any(moved)) {
-      const float to = moved ? mx : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - to);
-      m = to;
-      l *= alpha;
-      float4v a;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) a[r] = __shfl(alpha, g * 4 + r, WAVE);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] *= a;
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sc[h][r] = __builtin_amdgcn_exp2f(sc[h][r] - m);
-        l += sc[h][r];
-      }
-    if (tail) {      // a page's rows past the sequence may hold anything
+      const bool tail = t0 + TILE > t_end;      // wave-uniform
+      float mx = NEG;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (t0 + h * 16 + g * 4 + j >= t_end)
-            vr[h][j] = (typename C::VReg)(0u);
+        for (int r = 0; r < 4; ++r) {
+          sc[h][r] *= scale_log2;
+          if (tail && t0 + h * 16 + g * 4 + r >= t_end) sc[h][r] = -INFINITY;
+          mx = fmaxf(mx, sc[h][r]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      const bool moved = mx > m + SLACK;
+      if (__any(moved)) {
+        const float to = moved ? mx : m;
+        const float alpha = __builtin_amdgcn_exp2f(m - to);
+        m = to;
+        l *= alpha;
+        float4v a;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a[r] = __shfl(alpha, g * 4 + r, WAVE);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] *= a;
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sc[h][r] = __builtin_amdgcn_exp2f(sc[h][r] - m);
+          l += sc[h][r];
+        }
+      if (tail) {      // a page's rows past the sequence may hold anything
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (t0 + h * 16 + g * 4 + j >= t_end)
+              vr[h][j] = (typename C::VReg)(0u);
+      }
+      bf16x8 parts[3];
+      split3(sc, parts);
+#pragma unroll
+      for (int d = 0; d < 8 / C::CH; ++d) {
+        uint4v v[C::CH];
+        C::values(vr, d, v);
+#pragma unroll
+        for (int p = 2; p >= 0; --p)
+#pragma unroll
+          for (int c = 0; c < C::CH; ++c)
+            acc[d * C::CH + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                parts[p],
+                __builtin_bit_cast(bf16x8,
+                                   ENDLESS && p > 0 ? finite(v[c]) : v[c]),
+                acc[d * C::CH + c], 0, 0, 0);
+      }
+      if (more) fetch_v(next);
     }
-    bf16x8 parts[3];
-    split3(sc, parts);
+  };
+  walk(std::false_type{});
+  if constexpr (sizeof(CT) == 2) {
+    // A probability's lower parts, 0 or negative as often as not, make no number
+    // of an infinite value, where the whole one makes infinity: sums that are no
+    // number are taken anew, with infinite values in the first product only.
+    // (8-bit values have no infinities.)
+    float4v all = acc[0];
 #pragma unroll
-    for (int d = 0; d < 8 / C::CH; ++d) {
-      uint4v v[C::CH];
-      C::values(vr, d, v);
+    for (int i = 1; i < 8; ++i) all += acc[i];
+    const float sum = all[0] + all[1] + all[2] + all[3];
+    if (__any(sum != sum)) {
+      m = NEG;
+      l = 0.f;
 #pragma unroll
-      for (int p = 2; p >= 0; --p)
-#pragma unroll
-        for (int c = 0; c < C::CH; ++c)
-          acc[d * C::CH + c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              parts[p], __builtin_bit_cast(bf16x8, v[c]), acc[d * C::CH + c],
-              0, 0, 0);
+      for (int i = 0; i < 8; ++i) acc[i] = (float4v){0.f, 0.f, 0.f, 0.f};
+      walk(std::true_type{});
     }
-    if (more) fetch_v(next);
   }
   l += __shfl_xor(l, 16, WAVE);
   l += __shfl_xor(l, 32, WAVE);

@@ -115,6 +115,36 @@ def test_lengths_far_apart(batch, fp8):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("qpg,bs", [(1, 16), (8, 16), (4, 5)])
+@pytest.mark.parametrize("waves", [4, 8])
+def test_values_without_end(qpg, bs, waves):
+    """A probability times infinity is infinity, whichever parts the product is
+    taken in; two of either sign, or a value that is no number, leave none, and
+    other channels keep their sums."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    lens = [3, 31, 33, 256, 300, 700]
+    args, want = _case(lens, qpg, bs, False)
+    vc, bt = args[2], args[3].cpu()
+    inf = float("inf")
+    for i, n in enumerate(lens):
+        for t, channels in [(n // 2, {5: inf, 64: -inf, 100: inf}),
+                            (n - 1, {7: -inf, 100: -inf, 127: float("nan")})]:
+            for c, x in channels.items():
+                vc[int(bt[i, t // bs]), :, t % bs, c] = x
+    for c, x in {5: inf, 64: -inf, 7: -inf, 100: float("nan"),
+                 127: float("nan")}.items():
+        want[:, :, c] = x
+
+    def same(got):
+        torch.testing.assert_close(got.double().cpu(), want, rtol=2 ** -8,
+                                   atol=1e-4, equal_nan=True)
+    same(ext.paged_attention(*args, D ** -0.5, waves=waves))
+    for parts, part in [(3, 256), (8, 96)]:
+        same(ext.paged_attention_split(*args, parts, part, D ** -0.5,
+                                       waves=waves))
+
+
+@pytest.mark.gpu
 def test_running_maximum_far_apart():
     """Scores that grow along the context move the maximum at every tile."""
     args, _ = _case([600], 4, 16, False)
