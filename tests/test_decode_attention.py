@@ -28,6 +28,20 @@ def test_one_part_or_several(groups, max_len, elem, one, several):
     assert (parts > 1) == (several < one)
 
 
+@pytest.mark.parametrize("groups,max_len,mean,elem,one,several", [
+    (48, 742, 729, 1, 8.6, 11.1), (128, 1874, 1744, 1, 17.2, 21.0),
+    (160, 4076, 4076, 1, 34.7, 43.6), (160, 5504, 5168, 1, 43.9, 51.9),
+    (16, 835, 798, 1, 8.8, 11.0), (2, 697, 697, 1, 7.9, 11.0),
+    (48, 637, 294, 1, 7.4, 10.6), (176, 1205, 488, 1, 12.2, 15.5),
+    (80, 1316, 466, 2, 17.8, 14.4), (112, 4323, 3390, 2, 55.7, 42.9),
+    (132, 5262, 3223, 2, 67.0, 52.6), (4, 3300, 3300, 2, 32.2, 11.0)])
+def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
+    """All lengths alike, or most far below the longest: the bytes follow from the
+    mean. Against the times that both took, us."""
+    parts, _ = dispatch.decode_parts(groups, max_len, mean, elem)
+    assert (parts > 1) == (several < one)
+
+
 @pytest.mark.parametrize("batch", [2, 5, 17, 24, 25, 32, 64, 127, 256])
 @pytest.mark.parametrize("short", [1, 100, 300, 1000])
 @pytest.mark.parametrize("long", [1500, 3000, 8000, 131072])
