@@ -255,6 +255,8 @@ inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
 // left to the caller.
 inline c10::optional<Tensor> activated_linear(const Tensor& x, const Tensor& w,
                                               int64_t act) {
+  // (the sum of parts takes what is below 0 for no activation)
+  TORCH_CHECK(act >= 0 && act < 3, "activation ", act);
   if (const int rows = many_rows(x, w, false))
     return linear_act(x, w, act, false, rows);
   if (!few_rows(x, w, PLAIN)) return c10::nullopt;

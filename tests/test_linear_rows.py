@@ -180,6 +180,18 @@ def test_act_of_few_rows(name, rows, n, k):
             _same(y, fn(z), 8)
 
 
+@pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("rows,n", [(16, 4096), (8192, 8192)])
+@pytest.mark.parametrize("act", [-1, 3, 1 << 32])
+def test_no_such_act(name, rows, n, act):
+    """Refused ahead of any kernel, of few rows and of many."""
+    ext = _ext(name)
+    x, w = _draw(rows, 512, seed=1), _draw(n, 512, seed=2)
+    assert ext.activated_linear(x, w, 1) is not None
+    with pytest.raises(RuntimeError, match="activation"):
+        ext.activated_linear(x, w, act)
+
+
 @pytest.mark.parametrize("act", [0, 1, 2])
 def test_act_of_large_sums(act):
     """Infinities and what overflows come out as they do apart."""
