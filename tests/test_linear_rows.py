@@ -192,6 +192,25 @@ def test_no_such_act(name, rows, n, act):
         ext.activated_linear(x, w, act)
 
 
+@pytest.mark.parametrize("act,low,high", [(0, -10.0, -6.0), (1, -88.5, -60.0)])
+def test_act_of_small_results(act, low, high):
+    """Down to where the exponential overflows: the result's rounding (half a step of 7
+    bits behind the point, 2^-8) and the activation's own error, 2^-16 at most."""
+    ext = _ext("_hip_layered")
+    z = torch.linspace(low, high, 640, device="cuda").bfloat16()
+    x = torch.zeros(640, 128, device="cuda").bfloat16()
+    x[:, 0] = z
+    w = torch.zeros(2 * 10880, 128, device="cuda").bfloat16()
+    w[:, 0] = 1
+    a = z.double()
+    if act == 0:
+        a = 2 * 0.7978845608028654 * (a + 0.044715 * a ** 3)
+    want = z.double() / (1 + torch.exp(-a))
+    got = ext.activated_linear(x, w, act).double()
+    torch.testing.assert_close(got, want[:, None].expand_as(got),
+                               rtol=2 ** -8 + 2 ** -16, atol=0)
+
+
 @pytest.mark.parametrize("act", [0, 1, 2])
 def test_act_of_large_sums(act):
     """Infinities and what overflows come out as they do apart."""
