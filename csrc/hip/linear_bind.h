@@ -69,12 +69,15 @@ enum Use { PLAIN, GATED, PARTS };
 // library, as do odd layouts.
 inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
   if (!plain_matrices(x, w)) return false;
-  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0), limit = 1ll << 31;
+  // gated ones of more rows have one kernel, whose offsets stay under 4 GiB
+  const bool near = use != GATED || M <= 192;
   return M >= 1 && M <= 256 && K >= 8 && K % 8 == 0 && N >= 8 && N % 8 == 0 &&
          N <= (1 << 24) && K <= (1 << 24) && (use != GATED || N % 16 == 0) &&
          lds_linear_rows_takes((int)M, (int)(use == GATED ? N / 2 : N), (int)K,
                                use == GATED, use == PARTS) &&
-         rows_of_16_bytes(x) && rows_of_16_bytes(w);
+         rows_of_16_bytes(x) && rows_of_16_bytes(w) &&
+         (near || (M < limit / x.stride(0) && N < limit / w.stride(0)));
 }
 
 // Rows of a tile where a product of many rows and its activation are one kernel

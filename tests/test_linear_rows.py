@@ -90,6 +90,26 @@ def test_gated_of_many_steps(rows, n, k):
         assert torch.equal(y[-1:], _ext("_hip_ops").gated_linear(x[-1:], w, 1))
 
 
+@pytest.mark.parametrize("rows,one", [(192, True), (193, False), (256, False)])
+@pytest.mark.parametrize("of_x", [False, True])
+def test_gated_of_far_rows(rows, one, of_x):
+    """Rows spread over 4 GiB and more: up to 192 of x in one kernel, with offsets of
+    64 bits; more go to the library, as the kernel for them has 32."""
+    n, k = 14400, 1024
+
+    def far(t):
+        row = ((1 << 31) // len(t) + 8) // 8 * 8
+        out = torch.empty(len(t), row, dtype=t.dtype, device="cuda")[:, :k]
+        return out.copy_(t)
+    x, w = _draw(rows, k, seed=rows), _draw(2 * n, k, seed=n, scale=k ** -0.5)
+    assert _ext("_hip_ops").gated_linear(x, w, 1) is not None
+    y = _ext("_hip_ops").gated_linear(*((far(x), w) if of_x else (x, far(w))), 1)
+    assert (y is not None) == one
+    if one:
+        g, u = (x.double() @ w.double().t()).chunk(2, -1)
+        _same(y, torch.nn.functional.silu(g) * u, 8)
+
+
 @pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("rows,n,k", [
     (257, 1024, 5120), (384, 1288, 5184), (385, 1032, 8192), (512, 4088, 14336),
