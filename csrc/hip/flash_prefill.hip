@@ -4,13 +4,12 @@
 // Replaces the composed einsum+softmax prefill path (materialized S matrix,
 // ~6 HBM passes) with a flash-style kernel: per Q-tile, iterate KV tiles
 // computing QK^T -> online softmax -> P.V entirely on matrix cores
-// (v_mfma_f32_32x32x16_bf16), S never leaving registers (guide Appendix B
-// "Fused attention prefill").
+// (v_mfma_f32_32x32x16_bf16), S never leaving registers.
 //
 // The attention of a tile is flash_core.h's: S^T = K.Q^T, so that a lane owns
 // one query row and the online softmax is in-lane work. This kernel stages
 // through registers, converting fp8 to bf16 on the way, and also takes bf16
-// pools of contexts that flash_prefill_glds.hip's table does not hold.
+// pools of contexts that flash_prefill_bf16.hip's table does not hold.
 //
 // Work decomposition:
 //   grid = row tiles (128 "virtual rows" = (position, q-head-in-group)

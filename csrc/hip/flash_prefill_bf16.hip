@@ -1,4 +1,4 @@
-// flash_prefill_glds.hip — prefill attention of bf16 caches: tiles of keys and
+// flash_prefill_bf16.hip — prefill attention of bf16 caches: tiles of keys and
 // values go through registers into LDS, two of them there, a third on its way. The
 // attention of a tile is flash_core.h's; the tiles' loads and LDS writes stand
 // between its matrix instructions (in a row they hold a wave up for 1200 cycles of
@@ -27,7 +27,7 @@
 // GHz over long prompts.
 // Measured (groups of 4, 8 key heads, alone; before: operands of K waited for one
 // by one, tiles of 32 keys in a ring of loads to LDS): one prompt of 7900 tokens
-// 553 us, 924 TFLOP/s (652); 8 of 1000 109 us (127). By keys / by rows with 17 bits
+// 547 us, 934 TFLOP/s (652); 8 of 1000 110 us (127). By keys / by rows with 17 bits
 // (with 8): 150 tokens behind 1000 17 / 35 us (30; before 21 / 45); 500 behind 1000
 // 40 / 47 (38; 49 / 59); 600 behind 4000 139 / 127 (102; 183 / 168); 12 prompts of
 // 20 12 / 7 (7).
@@ -61,7 +61,7 @@ constexpr int lds_bytes(bool keys) {       // two tiles of keys and values
 // FINE: see attend. SHIFT: block size 1 << shift; else any
 template <int QPG, bool KEYS, bool FINE, bool SHIFT>
 __global__ __launch_bounds__(NW * WAVE, 2)
-void flash_prefill_glds_kernel(
+void flash_prefill_bf16_kernel(
     const short* __restrict__ q, const short* __restrict__ k_cache,
     const short* __restrict__ v_cache,
     const int32_t* __restrict__ block_tables,
@@ -290,7 +290,7 @@ hipError_t go(const void* q, const void* k_cache, const void* v_cache,
               const int32_t* block_tables, const int32_t* seq_meta,
               const int32_t* tiles, void* out, int n_tiles, int kvh, int bs,
               int shift, int max_blocks, float scale, hipStream_t stream) {
-  auto fn = flash_prefill_glds_kernel<QPG, KEYS, FINE, SHIFT>;
+  auto fn = flash_prefill_bf16_kernel<QPG, KEYS, FINE, SHIFT>;
   hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,
       lds_bytes(KEYS));
@@ -313,7 +313,7 @@ extern "C" {
 // else keys in one round of workgroups, or in two where prompts are long enough
 // to make up for the second (300 tokens behind 300 20 us by keys, 22 by rows; 4
 // x 100 13 and 10).
-hipError_t lds_flash_prefill_glds(
+hipError_t lds_flash_prefill_bf16(
     const void* q, const void* k_cache, const void* v_cache,
     const int32_t* block_tables, const int32_t* seq_meta,
     const int32_t* tiles, void* out, int n_tiles, int n_q_heads, int kvh,

@@ -58,7 +58,7 @@ hipError_t lds_flash_prefill(const void*, const void*, const void*,
                              const int32_t*, const int32_t*, const int32_t*,
                              void*, int, int, int, int, int, int, int, float,
                              hipStream_t);
-hipError_t lds_flash_prefill_glds(const void*, const void*, const void*,
+hipError_t lds_flash_prefill_bf16(const void*, const void*, const void*,
                                   const int32_t*, const int32_t*,
                                   const int32_t*, void*, int, int, int, int,
                                   int, int, float, int, int, int,
@@ -107,8 +107,8 @@ std::vector<torch::Tensor> hash_prompts(torch::Tensor tokens,
 }
 
 // A plain int of 32 bits, or false. Token ids have one digit, which is read where
-// it lies (a call for each took 1.2 ns, half of a burst's time); from Python 3.12 on
-// the digits lie elsewhere.
+// it lies (0.5 ns with all that is done for it, 0.6 more with a call for each); from
+// Python 3.12 on the digits lie elsewhere.
 inline bool int32_of(PyObject* x, int32_t* out) {
   if (!PyLong_CheckExact(x)) return false;
 #if PY_VERSION_HEX < 0x030C0000
@@ -428,15 +428,10 @@ torch::Tensor flash_prefill(torch::Tensor q, torch::Tensor k_cache,
   int qh = (int)q.size(1), d = (int)q.size(2);
   int kvh = (int)k_cache.size(1), bs = (int)k_cache.size(2);
   auto out = torch::empty_like(q);
-  // bf16 KV rides the glds staging pipeline; fp8 needs convert-on-stage.
-  // LLMD_NO_GLDS=1 forces the plain-VGPR kernel (bisect knob for the
-  // cross-stream wedge investigation, profiles/r02_notes.md).
-  static const bool no_glds = []() {
-    const char* e = getenv("LLMD_NO_GLDS");
-    return e && e[0] == '1';
-  }();
-  if (!no_glds && !kv_fp8_flag(k_cache) && block_tables.size(1) <= 1024) {
-    CHECK_HIP(lds_flash_prefill_glds(
+  // bf16 caches whose tables fit LDS have a kernel of their own; 8-bit values are
+  // widened on their way
+  if (!kv_fp8_flag(k_cache) && block_tables.size(1) <= 1024) {
+    CHECK_HIP(lds_flash_prefill_bf16(
         q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
         block_tables.data_ptr<int32_t>(), seq_meta.data_ptr<int32_t>(),
         tiles.data_ptr<int32_t>(), out.data_ptr(), (int)tiles.size(0), qh,

@@ -198,7 +198,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
 
 def prefill_shape(news: List[int], ctxs: List[int], group: int,
                   kv_heads: int) -> int:
-    """Shape of the prefill attention's workgroups (flash_prefill_glds.hip) for
+    """Shape of the prefill attention's workgroups (flash_prefill_bf16.hip) for
     prompts of `news` tokens that end contexts of `ctxs`: 0 by rows, 1 by keys,
     2 by rows with probabilities of 17 bits. From 256 workgroups by rows on the
     chip is full (1000 tokens behind 1000: 49 us by rows, 86 by keys). Below,

@@ -69,7 +69,7 @@ hip_ops = cpp_extension.CUDAExtension(
         "csrc/hip/kv_cache.hip",
         "csrc/hip/paged_attention.hip",
         "csrc/hip/flash_prefill.hip",
-        "csrc/hip/flash_prefill_glds.hip",
+        "csrc/hip/flash_prefill_bf16.hip",
     ],
     extra_compile_args=HIP_ARGS,
 )
