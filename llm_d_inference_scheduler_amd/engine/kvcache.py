@@ -163,7 +163,9 @@ class LayeredPool:
     def plan(config: LayeredConfig, budget_bytes: int, max_slots: int,
              block_size: int = BLOCK_SIZE, dtype_bytes: int = 2):
         """Split a budget -> (blocks, state slots): up to half of it for
-        state, the rest for pages."""
+        state, the rest for pages. What a pass needs for itself comes on top:
+        its activations and, with recurrent layers, up to 640 MB of workspace
+        (models/layered.py), 1.7 GB for 8000 tokens of width 4096."""
         per_seq = config.state_bytes_per_sequence(dtype_bytes)
         slots = max_slots
         if per_seq:

@@ -34,8 +34,10 @@ from . import feed_forward, rotary
 SHORT = 8
 CHUNK = 64                  # tokens per chunk of the chunked recurrence
 QUERY_TILE = 128            # query rows per workgroup of the prefill kernels
-# its workspace: a prompt of 8192 tokens of 32 heads in one group (28.6 ms a pass
-# of 7749 rows; in four groups that stay in the last-level cache 29.1)
+# Its workspace, taken beside the cache while a layer runs. Groups of 160 MB stay in
+# the last-level cache, but every group starts and drains once more. ms a pass of 8 layers by 160 / 640 / 1280 MB: 8000 tokens of
+# 32 heads 28.6 / 27.9 / 27.9 (one group from 640 on; at its peak 1380 and 1730 MB in
+# all), 16000 of them 58.9 / 56.3 / 55.8, 8000 of 64 heads 65.9 / 64.1 / 63.7.
 WORK_BYTES = 640 << 20
 
 

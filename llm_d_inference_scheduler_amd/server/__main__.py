@@ -33,7 +33,9 @@ def parse_args(argv=None):
                    help="EndpointPickerConfig YAML path")
     p.add_argument("--config-text", default="",
                    help="EndpointPickerConfig YAML inline")
-    p.add_argument("--kv-gb", type=float, default=160.0)
+    p.add_argument("--kv-gb", type=float, default=160.0,
+                   help="of cache; weights and what a pass needs (a few GB) "
+                        "come on top")
     p.add_argument("--kv-dtype", default="auto",
                    choices=["auto", "bf16", "fp8"])
     p.add_argument("--flow-control", action="store_true",
