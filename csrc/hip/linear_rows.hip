@@ -252,8 +252,12 @@ int lds_linear_rows_parts(int M, int N, int K) {
 //     fill at least 7/8 of their rounds, plain up to 128 rows. 4096 -> 32768: 32 rows
 //     46 / 62, 128 rows 55 / 64, 160 rows 66 / 67; -> 128256 (98 %): 64 rows
 //     182 / 208; 5120 -> 51200 (78 %): 64 rows 110 / 98. 4096 -> [2 x 14336]:
-//     64 rows 44 / 58, 128 rows 53 / 60, 192 rows 65 / 67, 256 rows 69 / 75 (by
-//     linear_wide, for K from 1024 on in whole steps);
+//     64 rows 44 / 58, 128 rows 53 / 60, 192 rows 65 / 67, 256 rows 69 / 75. From
+//     193 rows on by linear_wide, for K from 1024 on in whole steps, where the
+//     workgroups are one round and K is at most 8192: 1.01 to 1.25 times as fast
+//     over 25 sizes (232 rows, 1024 -> [2 x 14624]: 28 / 35). In two or three
+//     rounds it is 0.66 to 1.06 times (245 rows, 3584 -> [2 x 28744]: 132 / 118), by
+//     longer K 0.74 to 1.07 (15872 -> [2 x 15456]: 367 / 271);
 //     inside a 4-layer stack of about 180 rows the pass takes 790 / 835;
 //     2048 -> [2 x 4096] (25 %): 32 rows 18 / 16.
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
@@ -268,7 +272,8 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
   if (gated)
-    return full && (M <= 192 || (K >= 1024 && K % KS == 0));
+    return full && (M <= 192 || (groups <= 256 && K >= 1024 && K <= 8192 &&
+                                 K % KS == 0));
   if (N > 128 * 128) return full && M <= 128;
   if (full) return M <= 64 || K >= 4096;
   return M <= 64 && N <= 4096;

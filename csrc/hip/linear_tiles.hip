@@ -208,7 +208,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void linear_tiles_kernel(
 // From 193 rows on, K in parts of 1024 and more, multiples of 128: 128 rows of w by
 // all of x in four waves, by the loop of tile_core.h. The matrix cores are 75 %
 // busy, but they and the stream of weights together take the clock down to 1.25 to
-// 1.9 GHz: 4096 -> 28672, gated, 256 rows 69 us (78 above; library 65 to 69 and 6
+// 1.9 GHz: 4096 -> [2 x 14336], 256 rows 69 us (78 above; library 65 to 69 and 6
 // for the activation), 14336 -> 4096 37 (41), 4096 -> 12576 37 (42), of 5120 ->
 // 10240 38 (42). Shorter parts end sooner in eight waves (4096 -> 4096, 512 each:
 // 18 us for 20), as do 192 rows and fewer (a stack of 178: 795 us a pass for 814).

@@ -90,6 +90,20 @@ def test_gated_of_many_steps(rows, n, k):
         assert torch.equal(y[-1:], _ext("_hip_ops").gated_linear(x[-1:], w, 1))
 
 
+@pytest.mark.parametrize("rows", [193, 256])
+@pytest.mark.parametrize("n,k,one", [(16384, 1024, True), (14336, 8192, True),
+                                     (14336, 8320, False), (14336, 896, False),
+                                     (28744, 3584, False), (32768, 1024, False),
+                                     (46168, 2176, False)])
+def test_gated_of_one_round(rows, n, k, one):
+    """More than a round of workgroups, or longer K: the library and the activation
+    apart are faster."""
+    x = torch.zeros(rows, k, device="cuda").bfloat16()
+    w = torch.zeros(2 * n, k, dtype=torch.bfloat16, device="cuda")
+    for name in EXTENSIONS:
+        assert (_ext(name).gated_linear(x, w, 1) is not None) == one
+
+
 @pytest.mark.parametrize("rows,one", [(192, True), (193, False), (256, False)])
 @pytest.mark.parametrize("of_x", [False, True])
 def test_gated_of_far_rows(rows, one, of_x):
