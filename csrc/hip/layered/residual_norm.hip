@@ -65,9 +65,8 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
   // registers between the passes, the rest are read again
   float keep[KEEP][N];
   auto at = [&](int i) { return (int64_t)(threadIdx.x + i * NT) * N; };
-  // With parts the rows are few: all parts of what a thread keeps are asked for
-  // together, the stream's values ahead of them (8.5 us with the loads of a vector
-  // at a time).
+  // All parts of what a thread keeps are asked for together, the stream's values ahead
+  // of them (8.5 us with the loads of a vector at a time).
   float xk[PARTS ? KEEP : 1][N];
   if constexpr (PARTS) {
 #pragma unroll
@@ -239,7 +238,10 @@ hipError_t stream_norm_t(int mode, const void* const* p, int64_t rows,
     else if (mode == ADD) GO(N, ADD, false);                                  \
     else GO(N, LOOP, false);                                                  \
   } while (0)
-  if (parts && H % 8 == 0 && (mode == POST || mode == ADD)) {
+  // Past 256 rows enough is under way, and what is asked for ahead takes the registers
+  // of other rows (1300 rows of 4096 in 2 parts: 18.2 us with it, 16.1 without; 300 in 8
+  // parts 11.3 and 10.5; 256 rows of 3072 in 8 parts 5.9 and 6.5).
+  if (parts && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256) {
     if (mode == POST) GO(8, POST, true); else GO(8, ADD, true);
   } else if (H % 8 == 0) {
     GOM(8);

@@ -491,6 +491,36 @@ def test_norms_of_any_parts(rows, width, parts):
             _same(h, normed(s) * (wn.double() + 0.5), 8)
 
 
+@pytest.mark.parametrize("width", [1032, 2056, 4104, 8200])
+@pytest.mark.parametrize("few,many,parts", [(256, 257, 9), (512, 513, 2)])
+def test_norms_of_parts_of_many_rows(few, many, parts, width):
+    """A row comes out alike whichever way its parts are asked for: the same bits; of
+    the 32-bit stream, whose two forms join multiplications and additions otherwise,
+    32-bit sums within 1e-5 as above, and one step of bf16 in what follows."""
+    from llm_d_inference_scheduler_amd.ops import layered
+    hip = _ext("_hip_ops")
+    y = _draw(parts, many, width, seed=width).float()
+    gain, start = _draw(width, seed=3), _draw(many, width, seed=4)
+    outs = []
+    for n in (few, many):
+        mine, residual, x, z = y[:, :n].contiguous(), start[:n].clone(), *(
+            start[:n].float() for _ in range(2))
+        outs.append([hip.rmsnorm(mine, gain, 1e-5),
+                     hip.rmsnorm(mine, gain, 1e-5, residual), residual,
+                     layered.stream_norm(x, mine, gain.float(), gain.float(),
+                                         0.5, 1e-5, torch.bfloat16), x,
+                     layered.stream_norm(z, mine, None, gain.float(), 0.5,
+                                         1e-5, torch.bfloat16), z])
+    for i, (a, b) in enumerate(zip(*outs)):
+        if i < 3:
+            assert torch.equal(a, b[:few])
+        elif a.dtype == torch.float32:
+            torch.testing.assert_close(a, b[:few], rtol=1e-5, atol=1e-5)
+        else:
+            _same(a, b[:few].double(), 7)
+        assert b[few:].isfinite().all() and b[few:].any()
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("norm", [False, True])
 @pytest.mark.parametrize("T,qh,kvh,d,bs", [(1, 4, 1, 128, 16),
