@@ -131,15 +131,15 @@ def decode_parts(groups: int, max_len: int,
     average (None: 0.8 of that, lengths a quarter either way), of `elem` bytes a
     value. A workgroup of 8 waves takes 256 tokens a step, and about 512 of them
     fill the chip: parts make up for fewer groups as long as each has a step of its
-    own. They cost their sums and a second launch. In us: one part takes 2 and as
-    long as a workgroup walks (10.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
-    at 4.9 TB/s, several 9.5 and the bytes at 5.4 TB/s; over 340 batches, lengths
-    alike or down to a twentieth of the longest, the choice costs 0.5 % on average
-    and 19 % at most. From 200 groups on it is always one (groups, mean and longest
-    in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 44 in four; 132 of 3223,
-    5262: 67 and 53; 136 of 6800, 8190, 8-bit: 63 and 51; 80 of 466, 1316: 18 and 14;
-    160 of 1500, 1875: 27 and 34; 64 of 2000, 2500: 25 and 18; 240 of 1100: 27 and
-    35).
+    own. They cost their sums and a second launch. In us: one part takes 3 and as
+    long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
+    at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 320 batches, lengths
+    alike or down to a twentieth of the longest, the choice costs 0.4 % on average
+    and 22 % at most. From 200 groups on it is always one (groups, mean and longest
+    in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 43 in four; 136 of 3223,
+    5262: 71 and 56; 136 of 6800, 8190, 8-bit: 61 and 55; 80 of 466, 1316: 19 and 12;
+    160 of 1500, 1875: 30 and 37; 64 of 2000, 2500: 34 and 21; 8 of 777: 12 and 10, 8
+    of 450: 8.7 and 9.2; 240 of 1100, 1375: 28 and 38).
 
     One long sequence among short ones would hold the batch up: 14 us per 1000
     tokens that a workgroup walks alone. It is cut so that none walks more than
@@ -150,10 +150,10 @@ def decode_parts(groups: int, max_len: int,
     1000: 27 in one, 34 in two."""
     parts = 1
     if groups < 200:
-        walk = max_len * (10.5e-3 if elem > 1 else 6.8e-3)
+        walk = max_len * (12.5e-3 if elem > 1 else 6.8e-3)
         mean = 0.8 * max_len if mean_len is None else mean_len
         size = groups * mean * 256 * elem
-        if 2 + max(walk, size / 4.9e6) > 9.5 + size / 5.4e6:
+        if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
             parts = -(-512 // max(1, groups))
     if mean_len is not None and max_len > 1.4 * mean_len:
         # tokens that one workgroup may walk while each compute unit takes one

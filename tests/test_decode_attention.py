@@ -29,12 +29,13 @@ def test_one_part_or_several(groups, max_len, elem, one, several):
 
 
 @pytest.mark.parametrize("groups,max_len,mean,elem,one,several", [
-    (48, 742, 729, 1, 8.6, 11.1), (128, 1874, 1744, 1, 17.2, 21.0),
-    (160, 4076, 4076, 1, 34.7, 43.6), (160, 5504, 5168, 1, 43.9, 51.9),
-    (16, 835, 798, 1, 8.8, 11.0), (2, 697, 697, 1, 7.9, 11.0),
-    (48, 637, 294, 1, 7.4, 10.6), (176, 1205, 488, 1, 12.2, 15.5),
-    (80, 1316, 466, 2, 17.8, 14.4), (112, 4323, 3390, 2, 55.7, 42.9),
-    (132, 5262, 3223, 2, 67.0, 52.6), (4, 3300, 3300, 2, 32.2, 11.0)])
+    (48, 742, 729, 1, 8.7, 9.4), (128, 1874, 1744, 1, 17.3, 20.7),
+    (160, 4076, 4076, 1, 34.7, 43.0), (160, 5504, 5168, 1, 43.2, 49.9),
+    (8, 777, 777, 2, 11.9, 9.7), (8, 450, 450, 2, 8.7, 9.2),
+    (2, 697, 697, 1, 7.9, 8.4), (4, 3300, 3300, 2, 38.9, 10.5),
+    (48, 637, 294, 1, 7.5, 9.1), (176, 1205, 488, 1, 12.6, 16.8),
+    (80, 1316, 466, 2, 19.3, 12.2), (112, 4323, 3390, 2, 59.1, 43.5),
+    (136, 5262, 3223, 2, 70.6, 55.7)])
 def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
     """All lengths alike, or most far below the longest: the bytes follow from the
     mean. Against the times that both took, us."""
