@@ -240,8 +240,10 @@ hipError_t stream_norm_t(int mode, const void* const* p, int64_t rows,
   } while (0)
   // Past 256 rows enough is under way, and what is asked for ahead takes the registers
   // of other rows (1300 rows of 4096 in 2 parts: 18.2 us with it, 16.1 without; 300 in 8
-  // parts 11.3 and 10.5; 256 rows of 3072 in 8 parts 5.9 and 6.5).
-  if (parts && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256) {
+  // parts 11.3 and 10.5; 256 rows of 3072 in 8 parts 5.9 and 6.5), nor is there anything
+  // to ask for ahead in short rows (1024 in 8 parts: 3.7 and 3.5).
+  if (parts && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256 &&
+      H >= NT * 8) {
     if (mode == POST) GO(8, POST, true); else GO(8, ADD, true);
   } else if (H % 8 == 0) {
     GOM(8);

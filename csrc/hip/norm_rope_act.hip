@@ -27,9 +27,10 @@ namespace {
 constexpr int NT = 256;
 
 // EARLY: with parts, all that a thread keeps is asked for at once, pair by pair. Not
-// past 512 rows: other rows' loads are under way anyway, and what a pair reads past the
-// row's end costs more than the wait (600 rows of 5120 in 3 parts: 11.1 us, without
-// 10.1; 400 rows in 4 parts 8.2 and 8.6).
+// past 512 rows (256 where a thread has one vector): other rows' loads are under way
+// anyway, and what a pair reads past the row's end costs more than the wait (600 rows
+// of 5120 in 3 parts: 11.1 us, without 10.1; 400 rows in 4 parts 8.3 and 8.7; 257 rows of
+// 2048 in 14 parts 6.1 and 5.6).
 template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY>
 __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     const void* __restrict__ x, int parts, short* __restrict__ residual,
@@ -39,7 +40,10 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   const int nchunks = H / 8;
   short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
   auto source = [&](int c, float* f) {
-    if constexpr (PARTS) {
+    if constexpr (EARLY) {
+      const float4v* const p[1] = {(const float4v*)x + (row * H + c * 8) / 4};
+      PartSums<1>(p, (int64_t)gridDim.x * H / 4, parts).get(0, f);
+    } else if constexpr (PARTS) {
       const float4v* p = (const float4v*)x + (row * H + c * 8) / 4;
       const int64_t apart = (int64_t)gridDim.x * H / 4;
       float4v a = p[0], b = p[1];
@@ -60,9 +64,10 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     }
   };
   float vals[KEEP][8], ss = 0.f;
-  static_assert(!EARLY || (PARTS && KEEP % 2 == 0), "");
-  short8 rv[EARLY ? KEEP : 1], wk[EARLY ? KEEP : 1];
-  if constexpr (EARLY) {
+  static_assert(PARTS || !EARLY, "");
+  constexpr bool AHEAD = EARLY && KEEP > 1;
+  short8 rv[AHEAD ? KEEP : 1], wk[AHEAD ? KEEP : 1];
+  if constexpr (AHEAD) {
     const int64_t apart = (int64_t)gridDim.x * H / 4;
 #pragma unroll
     for (int i = 0; i < KEEP; ++i) {
@@ -83,9 +88,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
     }
   }
   auto first = [&](int c, float* f, int i) {
-    if (!EARLY || i < 0) source(c, f);
+    if (!AHEAD || i < 0) source(c, f);
     if constexpr (RESIDUAL) {
-      const short8 r = EARLY && i >= 0 ? rv[EARLY ? i : 0] : r8[c];
+      const short8 r = AHEAD && i >= 0 ? rv[AHEAD ? i : 0] : r8[c];
       short8 ro;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -110,7 +115,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
       rsqrtf(block_reduce_sum<NT / WAVE>(ss, red) / (float)H + eps);
   auto second = [&](int c, const float* f, int i) {
     const short8 wv =
-        EARLY && i >= 0 ? wk[EARLY ? i : 0] : ((const short8*)w)[c];
+        AHEAD && i >= 0 ? wk[AHEAD ? i : 0] : ((const short8*)w)[c];
     short8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
@@ -317,11 +322,12 @@ hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
                      (short*)residual, (const short*)w, (short*)y, H, eps)
 #define GO_K(RES, PARTS, EARLY)                                              \
   do {                                                                       \
-    if (H <= 1 * NT * 8) GO(1, RES, PARTS, false);                           \
+    if (H <= 1 * NT * 8) GO(1, RES, PARTS, EARLY);                           \
     else if (H <= 2 * NT * 8) GO(2, RES, PARTS, EARLY);                      \
     else GO(4, RES, PARTS, EARLY);                                           \
   } while (0)
-  if (parts > 0 && n_rows <= 512) {
+  const bool early = n_rows <= (H <= NT * 8 ? 256 : 512);
+  if (parts > 0 && early) {
     if (residual) GO_K(true, true, true); else GO_K(false, true, true);
   } else if (parts > 0) {
     if (residual) GO_K(true, true, false); else GO_K(false, true, false);
