@@ -133,7 +133,7 @@ def decode_parts(groups: int, max_len: int,
     fill the chip: parts make up for fewer groups as long as each has a step of its
     own. They cost their sums and a second launch. In us: one part takes 3 and as
     long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
-    at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 320 batches, lengths
+    at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 340 batches, lengths
     alike or down to a twentieth of the longest, the choice costs 0.4 % on average
     and 22 % at most. From 200 groups on it is always one (groups, mean and longest
     in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 43 in four; 136 of 3223,
