@@ -14,9 +14,12 @@
 
 extern "C" {
 int lds_linear_rows_parts(int M, int N, int K);
+int lds_linear_plain_parts(int M, int N, int K);
 int lds_linear_rows_takes(int M, int N, int K, int gated, int parts);
 hipError_t lds_linear_rows(const void*, int64_t, const void*, int64_t, void*,
                            float*, int, int, int, int, int, hipStream_t);
+hipError_t lds_activated_rows(const void*, int64_t, const void*, int64_t,
+                              void*, int, int, int, int, hipStream_t);
 hipError_t lds_gated_rows(const void*, int64_t, const void*, int64_t, void*,
                           int, int, int, int, hipStream_t);
 int lds_linear_act_rows(int64_t, int64_t, int64_t, int);
@@ -145,7 +148,7 @@ inline void linear_rows(const Tensor& x, const Tensor& w, const Tensor& y,
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
   const auto wide = x.options().dtype(at::kFloat);
   Tensor part;
-  const int parts = lds_linear_rows_parts(M, N, K);
+  const int parts = lds_linear_plain_parts(M, N, K);
   if (parts > 1) part = torch::empty({parts, M, N}, wide);
   check(lds_linear_rows(
       x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), y.data_ptr(),
@@ -254,8 +257,9 @@ inline c10::optional<Tensor> gated_linear(const Tensor& x, const Tensor& w,
 }
 
 // act(x w'), or None as above. Of few rows the kernel that sums the parts of K takes
-// the activation too (60 rows, 4096 -> 7168: a launch of 5 us of 24 less); one part is
-// left to the caller.
+// the activation too (60 rows, 4096 -> 7168: a launch of 5 us of 24 less), or that of
+// the product; one part of more than 64 rows or 128 x 128 channels is left to the
+// caller.
 inline c10::optional<Tensor> activated_linear(const Tensor& x, const Tensor& w,
                                               int64_t act) {
   // (the sum of parts takes what is below 0 for no activation)
@@ -264,13 +268,20 @@ inline c10::optional<Tensor> activated_linear(const Tensor& x, const Tensor& w,
     return linear_act(x, w, act, false, rows);
   if (!few_rows(x, w, PLAIN)) return c10::nullopt;
   const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
-  const int parts = lds_linear_rows_parts(M, N, K);
-  if (parts == 1) return c10::nullopt;
+  const int parts = lds_linear_plain_parts(M, N, K);
+  const bool one = parts == 1 && M <= 64 && N <= 128 * 128;
+  if (parts == 1 && !one) return c10::nullopt;
   const c10::DeviceGuard guard(x.device());
   const auto stream =
       at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
-  Tensor part = torch::empty({parts, M, N}, x.options().dtype(at::kFloat));
   Tensor y = torch::empty({M, N}, x.options());
+  if (one) {
+    check(lds_activated_rows(x.data_ptr(), x.stride(0), w.data_ptr(),
+                             w.stride(0), y.data_ptr(), M, N, K, (int)act,
+                             stream));
+    return y;
+  }
+  Tensor part = torch::empty({parts, M, N}, x.options().dtype(at::kFloat));
   check(lds_linear_rows(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                         nullptr, part.data_ptr<float>(), parts, M, N, K, 0,
                         stream));

@@ -1,23 +1,26 @@
 // linear_rows.hip — y = x w' for few rows of x (bf16, 32-bit sums): the kernel
-// for up to 16 rows, and which product goes where. Products of up to 256 rows
-// go to linear_tiles.hip.
+// for up to 64 rows, and which product goes where. Others of up to 256 rows go to
+// linear_tiles.hip.
 //
-// The weights' bytes are what counts, so they go straight from memory into
-// matrix-core operands, once, with plain loads (marked non-temporal they come
-// at three quarters of the rate). A workgroup owns 128 or 256 output channels
-// (8 waves of 16 CT) and walks K in steps of 128; a wave reads 256 bytes of 16
-// weight rows per step, two steps ahead. x goes through LDS: the waves share
-// it, since a workgroup that reads x for each wave spends as much of the
-// caches' rate on x as on weights. Loads retire in order, so x of a step is
-// asked for ahead of the weights of that step. Workgroups start at different
-// steps: in step they would hit the same few memory channels where rows are a
-// power of two apart. linear_tiles.hip adds up in the same order, so a row
-// comes out the same, to the bit, whichever of the two took it: as the one row
-// of a decode step or within a short prompt.
+// The weights' bytes are what counts. A workgroup has all rows of x against 128 rows
+// of w, or 64 where those of 128 leave compute units idle, and K is split until the
+// workgroups make up a round of the 256 compute units. Both operands go to LDS by
+// direct loads, 128 of K at a time, into a ring of three steps: 64 KB of w per compute
+// unit are under way. What the rate hangs on is the length of what is read of a row at
+// a time: 256 bytes of each by one instruction come at 5.9 TB/s, pieces of 128 take 10
+// to 20 % longer (14336 -> 4096 read and nothing else: 21.3 us, 23.8; 25600 -> 5120:
+// 45, 54). Workgroups start at different steps: in step they would hit the same few
+// memory channels where rows are a power of two apart (read and nothing else, 4096 ->
+// [2 x 14336], a start of 6 blocks: 41.5 us, 1: 63, none: 48). Where K is one part each
+// XCD has blocks that follow each other (39.9). linear_tiles.hip adds up in the same
+// order, so a row comes out the same, to the bit, whichever of the two took it: as the
+// one row of a decode step or within a short prompt.
 //
-// Measured, 1 row, cold weights, without the sum of the parts (library: its
-// time on the device): 4096 -> 28672: 43 us, 5.5 TB/s (58); 14336 -> 4096 22 us
-// (26); 25600 -> 5120: 47 us (134); 4096 -> 4096: 8.4 us (15).
+// Measured, cold weights, without the sum of the parts; before: up to 16 rows weights
+// straight to registers, x through LDS, above 128 bytes of a row at a time: 1 row,
+// 4096 -> [2 x 14336] 41.9 us, 5.6 TB/s (43.5; library 58 and the activation), 4096 ->
+// 6144 11.0 (11.9), 14336 -> 4096 21.9 (22.6), 4096 -> 4096 7.5 (8.0), 25600 -> 5120
+// 46.3 (47.9); 30 rows 42.5, 12.0, 23.0, 8.4, 48.4 (45.4, 12.0, 23.2, 8.7, 48.9).
 #include "layered/elem.h"
 
 namespace {
@@ -27,127 +30,244 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 struct Rows {
   const short *x, *w;        // [M, K], [N, K] (GATED: [2 N, K], gate first)
   int64_t x_row, w_row;      // strides in elements
-  void* y;                   // [M, N]; PARTS: [parts, M, N] 32-bit
+  void* y;                   // [M, N]; F32: [parts, M, N] 32-bit
   int M, N, K, k_part;       // k_part: K per part, a multiple of KS
-  int act;
+  int parts, act;
 };
 
-// what becomes of the sums: bf16, 32-bit (also of a part of K), or
+// what becomes of the sums: bf16, 32-bit (also of a part of K), act of them or
 // act(gate) * up as bf16
-enum Out { BF16, F32, GATED };
+enum Out { BF16, F32, ACT, GATED };
 
-constexpr int NW = 8, KS = 128, XS = KS + 8;   // XS: row of x in LDS
+constexpr int KS = 128, ROW = KS * 2;          // ROW: bytes of a row in LDS
+constexpr int ROUND = 256;       // compute units
+constexpr int RING = 3;          // 4 are no faster, 2 up to 15 % slower
 
-template <int CT, int OUT>
-__global__ __launch_bounds__(NW * WAVE) void linear_rows_kernel(const Rows p) {
-  __shared__ __align__(16) short xl[2][16 * XS];
-  constexpr int WI = KS / 32;
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int col = lane % 16, grp = lane / 16, M = p.M, N = p.N;
-  const int k_lo = blockIdx.y * p.k_part, k_hi = min(p.K, k_lo + p.k_part);
-  // GATED: waves 0 to 3 take gate's channels, 4 to 7 the same ones of up
-  constexpr int NC = OUT == GATED ? NW / 2 : NW;
-  const int n0 = (blockIdx.x * NC + wave % NC) * 16 * CT;
-  // channels past N and rows past M repeat the last one and are dropped
-  const short* wr[CT];
+// what is past the end of K
+__device__ const float4v zeros = {0.f, 0.f, 0.f, 0.f};
+
+// RT: rows of x / 16. BN rows of w; KG: groups of BN / 16 waves, each with its share of
+// K, whose sums meet at the end. A wave has CT tiles of 16 channels by MT of 16 rows.
+template <int RT, int BN, int KG, int OUT>
+__global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
+    const Rows p) {
+  extern __shared__ __align__(16) char lds[];
+  constexpr int NW = BN / 16, WM = RT == 1 ? 1 : 2, WC = NW / WM;
+  constexpr int CT = BN / 16 / WC, MT = RT / WM;
+  // a group's rings: RING steps of w, two of x, whose lines are near
+  constexpr int W_STEP = BN * ROW, X_STEP = 16 * RT * ROW;
+  constexpr int RINGS = RING * W_STEP + 2 * X_STEP;
+  // loads of a wave, 4 rows each (where x has fewer the last one is repeated)
+  constexpr int WL = BN / 4 / NW, XL = (4 * RT + NW - 1) / NW;
+  constexpr int CH = OUT == GATED ? BN / 2 : BN;       // channels
+  const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int group = all / NW, wave = all % NW;
+  const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
+  const int M = p.M, N = p.N;
+  const int part = blockIdx.x % p.parts;
+  // a round of the chip, in which an XCD has blocks that follow each other (65536 x 2048:
+  // 52.4 us, 59.6 in the order of the grid; over the whole grid 49.3, but 128256 x 4096
+  // 171.6, 168.7 and 175.9: eight far ends of a large matrix)
+  const int round = blockIdx.x / ROUND * ROUND, at = blockIdx.x - round;
+  const int blk = p.parts > 1 ? blockIdx.x / p.parts
+                              : round + at % 8 * (min(ROUND, int(gridDim.x) - round) / 8) +
+                                    at / 8;
+  if (blk * CH >= N) return;
+  // this group's K: steps of KS, the last ones past the end where they do not go round
+  const int p_lo = part * p.k_part, p_hi = min(p.K, p_lo + p.k_part);
+  const int steps = ((p_hi - p_lo + KS - 1) / KS + KG - 1) / KG;
+  const int k_lo = p_lo + group * steps * KS, k_hi = min(p_hi, k_lo + steps * KS);
+  // by blocks of 128 rows of w, as in linear_tiles.hip
+  const int first = (OUT == GATED    ? blk * BN / 128 * 6
+                     : N > 128 * 256 ? blk * BN / 256 * 3
+                                     : blk * BN / 128 * 3) %
+                    steps;
+  char* const w_ring = lds + group * RINGS;
+  char* const x_ring = w_ring + RING * W_STEP;
+
+  // A load takes 4 rows of KS, 16 pieces of 16 bytes each; the pieces of a row change
+  // places by XOR with its number, so that 16 lanes that read one piece of 16 rows
+  // find all banks. Rows that do not exist repeat the last one. GATED: of 32 rows of w
+  // 16 are of gate, 16 the same ones of up; with one tile per wave the halves are.
+  const int r4 = lane / 16;
+  const short *w_from[WL], *x_from[XL];
 #pragma unroll
-  for (int c = 0; c < CT; ++c)
-    wr[c] = p.w + (min(n0 + c * 16 + col, N - 1) + wave / NC * N) * p.w_row +
-            grp * 8;
-  // half of the threads bring 16 bytes of x each
-  const int xr = threadIdx.x / (KS / 8), xp = threadIdx.x % (KS / 8);
-  const bool x_mine = xr < 16;
-  const short* xg = p.x + min(xr, M - 1) * p.x_row + xp * 8;
-  float4v acc[CT];
+  for (int j = 0; j < WL; ++j) {
+    const int r = (wave * WL + j) * 4 + r4;            // row in LDS
+    const int n = OUT != GATED ? r : CT == 1 ? r % CH : r / 32 * 16 + r % 16;
+    const bool up = OUT == GATED && (CT == 1 ? r >= CH : r % 32 >= 16);
+    w_from[j] = p.w + (min(blk * CH + n, N - 1) + (up ? N : 0)) * p.w_row +
+                (lane % 16 ^ r % 16) * 8;
+  }
 #pragma unroll
-  for (int c = 0; c < CT; ++c) acc[c] = (float4v){0.f, 0.f, 0.f, 0.f};
-  const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  short8 w0[CT][WI], w1[CT][WI], xn = zero;
-  const int steps = (k_hi - k_lo + KS - 1) / KS;
-  // where rows are 8 KB apart, 1 of 4096 -> 28672: a start of 3 blockIdx.x 43
-  // us, 1: 44, 2: 72, 6: 51, none: 52; gated, with twice the streams, 6: 42.5,
-  // 3: 45, 1: 67, none: 52. Other sizes hardly mind.
-  const int first = blockIdx.x * (OUT == GATED ? 6u : 3u) % steps;
-  auto at = [&](int s) {
+  for (int j = 0; j < XL; ++j) {
+    const int r = min(wave * XL + j, 4 * RT - 1) * 4 + r4;
+    x_from[j] = p.x + min(r, M - 1) * p.x_row + (lane % 16 ^ r % 16) * 8;
+  }
+  typedef const __attribute__((address_space(1))) unsigned int gmem;
+  typedef __attribute__((address_space(3))) unsigned int smem;
+  auto k_of = [&](int s) {
     s += first;
     return k_lo + (s >= steps ? s - steps : s) * KS;
   };
-  auto fetch_w = [&](auto& r, int s) {
-    const int k0 = at(s);
-    const bool whole = k0 + KS <= k_hi;    // K is a multiple of 8
+  // 4 rows of K from k on, rows 4 q .. of their kind
+  auto load = [&](const short* from, char* to, int q, int k) {
+    const bool in = k + (lane % 16 ^ (q * 4 + r4) % 16) * 8 < k_hi;
+    __builtin_amdgcn_global_load_lds(
+        (gmem*)(in ? from + k : (const short*)&zeros), (smem*)(to + q * 1024),
+        16, 0, 0);
+  };
+  auto issue_w = [&](int s, int buf) {
+    const int k = k_of(s);
+#pragma unroll
+    for (int j = 0; j < WL; ++j)
+      load(w_from[j], w_ring + buf * W_STEP, wave * WL + j, k);
+  };
+  auto issue_x = [&](int s) {
+    const int k = k_of(s);
+#pragma unroll
+    for (int j = 0; j < XL; ++j)
+      load(x_from[j], x_ring + s % 2 * X_STEP, min(wave * XL + j, 4 * RT - 1), k);
+  };
+
+  float4v acc[CT][MT];
+#pragma unroll
+  for (int c = 0; c < CT; ++c)
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
+  const int wc = wave % WC, wm = wave / WC;
+  struct Operands {
+    bf16x8 w[CT], x[MT];
+  };
+  const int w_at = (wc * 16 * CT + col) * ROW, x_at = (wm * 16 * MT + col) * ROW;
+  auto read = [&](Operands& o, int buf, int s, int q) {       // q: 32 of K
+    const int piece = ((q * 4 + grp) ^ col) * 16;
+    const char* w = w_ring + buf * W_STEP + w_at + piece;
+    const char* x = x_ring + s % 2 * X_STEP + x_at + piece;
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+      o.w[c] = *(const bf16x8*)(w + c * 16 * ROW);
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+      o.x[t] = *(const bf16x8*)(x + t * 16 * ROW);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](const Operands& o) {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+        acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            o.w[c], o.x[t], acc[c][t], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // step s has landed, and so it has for the other waves, when only w of the next one
+  // is under way
+  auto landed = [&](int s) {
+    if (s + 1 < steps)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(WL) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // Operands are read 32 of K ahead of their products. At the barrier ahead of the
+  // last of step s all of its operands are in registers: its places take w of step
+  // s + RING and x of step s + 2.
+  static_assert(RING == 3, "");
+  issue_w(0, 0);
+  issue_x(0);
+  if (1 < steps) issue_w(1, 1);
+  Operands o0, o1;
+  landed(0);
+  if (1 < steps) issue_x(1);
+  if (2 < steps) issue_w(2, 2);
+  read(o0, 0, 0, 0);
+  int buf = 0;
+  for (int s = 0; s < steps; ++s) {
+    read(o1, buf, s, 1);
+    multiply(o0);
+    read(o0, buf, s, 2);
+    multiply(o1);
+    read(o1, buf, s, 3);
+    multiply(o0);
+    if (s + 1 < steps) {
+      landed(s + 1);
+      if (s + 2 < steps) issue_x(s + 2);
+      if (s + RING < steps) issue_w(s + RING, buf);
+      buf = buf + 1 == RING ? 0 : buf + 1;
+      read(o0, buf, s + 1, 0);
+    }
+    multiply(o1);
+  }
+
+  if constexpr (KG > 1) {                  // to the sums of the first group
+    static_assert(KG == 2 && CT * MT * NW * 1024 <= RINGS, "");
+    float4v* other = (float4v*)lds;
+    __syncthreads();                       // the rings are no longer read
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
-      for (int i = 0; i < WI; ++i) {
-        const int k = k0 + i * 32;
-        r[c][i] = whole || k + grp * 8 < k_hi ? *(const short8*)(wr[c] + k)
-                                               : zero;
-      }
-  };
-  auto fetch_x = [&](int s) {
-    const int k0 = at(s);
-    if (x_mine) xn = k0 + xp * 8 < k_hi ? *(const short8*)(xg + k0) : zero;
-  };
-  auto put_x = [&](int b) {
-    if (x_mine) *(short8*)(xl[b] + xr * XS + xp * 8) = xn;
-  };
-  auto step = [&](auto& r, int b, int s) {
-#pragma unroll
-    for (int i = 0; i < WI; ++i) {
-      const bf16x8 xf =
-          *(const bf16x8*)(xl[b] + col * XS + i * 32 + grp * 8);
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(bf16x8, r[c][i]), xf, acc[c], 0, 0, 0);
-    }
-    if (s + 1 < steps) put_x(b ^ 1);
-    if (s + 2 < steps) fetch_x(s + 2);
-    __builtin_amdgcn_sched_barrier(0);     // x ahead of the weights
-    if (s + 2 < steps) fetch_w(r, s + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    lds_barrier();
-  };
-  fetch_x(0);
-  fetch_w(w0, 0);
-  put_x(0);
-  if (1 < steps) fetch_x(1);
-  if (1 < steps) fetch_w(w1, 1);
-  lds_barrier();
-  for (int s = 0; s < steps; s += 2) {
-    step(w0, 0, s);
-    if (s + 1 < steps) step(w1, 1, s + 1);
-  }
-  float4v* up = (float4v*)xl;              // no longer read: the loop's end
-  if constexpr (OUT == GATED) {
-    static_assert(sizeof(xl) >= NC * CT * WAVE * sizeof(float4v));
-    if (wave >= NC) {
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        up[((wave - NC) * CT + c) * WAVE + lane] = acc[c];
-    }
+      for (int t = 0; t < MT; ++t)
+        if (group == 1)
+          other[((c * MT + t) * NW + wave) * WAVE + lane] = acc[c][t];
     __syncthreads();
-    if (wave >= NC) return;
-  }
-#pragma unroll
-  for (int c = 0; c < CT; ++c) {
-    const int n = n0 + c * 16 + grp * 4, m = col;
-    if (n >= N || m >= M) continue;        // N is a multiple of 4
-    const float4v a = acc[c];
-    const int64_t o = ((int64_t)blockIdx.y * M + m) * N + n;
-    if constexpr (OUT == F32) {
-      *(float4v*)((float*)p.y + o) = a;
+    if (group == 1) {
+      if (OUT != GATED || CT > 1) return;
     } else {
+#pragma unroll
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          acc[c][t] += other[((c * MT + t) * NW + wave) * WAVE + lane];
+    }
+  }
+  // lane: row `col` of a tile, channels 4 grp ..
+  if constexpr (OUT == GATED) {
+    if constexpr (CT == 1) {               // up is with the other half of the waves
+      static_assert(MT == 1, "");
+      float4v* other = (float4v*)lds;
+      __syncthreads();
+      if (group == 0 && wave >= NW / 2)
+        other[(wave - NW / 2) * WAVE + lane] = acc[0][0];
+      __syncthreads();
+      if (group > 0 || wave >= NW / 2) return;
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+      const int m = (wm * MT + t) * 16 + col, n = blk * CH + wc * 16 + grp * 4;
+      if (m >= M || n >= N) continue;      // N is a multiple of 4
+      const float4v u = CT == 1 ? ((const float4v*)lds)[wave * WAVE + lane]
+                                : acc[CT - 1][t];
       short4v v;
-      float4v u = a;
-      if constexpr (OUT == GATED) u = up[(wave * CT + c) * WAVE + lane];
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        v[r] = f32_to_bf16(OUT == GATED ? activate(p.act, a[r]) * u[r]
-                                        : a[r]);
-      *(short4v*)((short*)p.y + o) = v;
+        v[r] = f32_to_bf16(activate(p.act, acc[0][t][r]) * u[r]);
+      *(short4v*)((short*)p.y + (int64_t)m * N + n) = v;
     }
+    return;
   }
+#pragma unroll
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+      const int m = (wm * MT + t) * 16 + col;
+      const int n = blk * BN + (wc * CT + c) * 16 + grp * 4;
+      if (m >= M || n >= N) continue;
+      const int64_t o = ((int64_t)part * M + m) * N + n;
+      if constexpr (OUT == F32) {
+        *(float4v*)((float*)p.y + o) = acc[c][t];
+      } else {
+        short4v v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          v[r] = f32_to_bf16(OUT == ACT ? activate(p.act, acc[c][t][r])
+                                        : acc[c][t][r]);
+        *(short4v*)((short*)p.y + o) = v;
+      }
+    }
 }
 
 // sum of the parts, or (act >= 0) the activation of it; n4: float4s of one
@@ -199,26 +319,53 @@ __global__ __launch_bounds__(256) void lay_weights_kernel(
   }
 }
 
-// 16-channel tiles per wave: two where 128 channels per workgroup would make
-// more than one round of the 256 compute units
-int channel_tiles(int weight_rows) { return weight_rows > 128 * 256 ? 2 : 1; }
-
-template <int CT, int OUT>
-hipError_t go(const Rows& p, int parts, hipStream_t stream) {
-  constexpr int width = NW * 16 * CT / (OUT == GATED ? 2 : 1);
-  hipLaunchKernelGGL((linear_rows_kernel<CT, OUT>),
-                     dim3((p.N + width - 1) / width, parts), dim3(NW * WAVE),
-                     0, stream, p);
+template <int RT, int BN, int KG, int OUT>
+hipError_t go(const Rows& p, hipStream_t stream) {
+  constexpr int width = OUT == GATED ? BN / 2 : BN;
+  constexpr int bytes = KG * (RING * BN + 2 * 16 * RT) * ROW;
+  auto fn = linear_rows_kernel<RT, BN, KG, OUT>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (e != hipSuccess) return e;
+  int groups = (p.N + width - 1) / width * p.parts;
+  if (p.parts == 1) groups = (groups + 7) / 8 * 8;     // equal shares of the XCDs
+  hipLaunchKernelGGL(fn, dim3(groups), dim3(BN / 16 * KG * WAVE), bytes, stream,
+                     p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }
 
-// up to 16 rows come here, more go to linear_tiles.hip
-constexpr int ROWS = 16, TILE_ROWS = 256;
+// 64 rows of w per workgroup where 128 leave half of the chip idle, K in two halves
+// where 64 do as well (4096 -> [2 x 1024], 16 rows: 24.2 us by 128, 16.7 by 64, 14.8
+// with halves, [2 x 4096] 26.3, 19.6, 17.2; 2048 -> [2 x 8192] 16.6, 14.4, 16.3), and
+// for parts of a few steps: two workgroups per compute unit, whose ends overlap (4096 ->
+// 4096, parts of 512: 7.4 us, 7.6 by 128, 30 rows 8.3, 8.5; parts of 896 up: 22.1, 21.9).
+template <int RT, int OUT>
+hipError_t go_width(const Rows& p, hipStream_t stream) {
+  const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
+  if (p.parts == 1 && rows <= 64 * 128) return go<RT, 64, 2, OUT>(p, stream);
+  if (p.parts == 1 ? rows <= 128 * 128 : p.k_part <= 512)
+    return go<RT, 64, 1, OUT>(p, stream);
+  if constexpr (OUT == ACT) return hipErrorInvalidValue;
+  else return go<RT, 128, 1, OUT>(p, stream);
+}
 
-// of one part of K
+template <int OUT>
+hipError_t go_rows(const Rows& p, hipStream_t stream) {
+  return p.M <= 16   ? go_width<1, OUT>(p, stream)
+         : p.M <= 32 ? go_width<2, OUT>(p, stream)
+                     : go_width<4, OUT>(p, stream);
+}
+
+// Up to 64 rows come here, up to 32 where K is split, more go to linear_tiles.hip (60
+// rows, here / there: 4096 -> [2 x 14336] 43.6 us / 44.9, 4096 -> 6144 in 5 parts 13.5 /
+// 12.7, 14336 -> 4096 in 8 24.3 / 23.8).
+constexpr int ROWS = 64, SPLIT_ROWS = 32, TILE_ROWS = 256;
+
+// Of one part of K, by which the split and the rule below are reckoned: of 256 rows
+// of w for up to 16 of x where 128 are more than a round
 int workgroups(int M, int N) {
-  const int width = M <= ROWS ? 128 * channel_tiles(N) : 128;
+  const int width = M <= 16 && N > 128 * 256 ? 256 : 128;
   return (N + width - 1) / width;
 }
 
@@ -241,6 +388,19 @@ int lds_linear_rows_parts(int M, int N, int K) {
   return (K + k_part - 1) / k_part;
 }
 
+// The same where the sum of the parts is a launch of its own (3 to 5 us): one part of
+// short K, or of so many channels that it has few parts. Up to 64 rows, one part / parts
+// and their sum: 1024 -> 4096, 1 row 5.2 / 6.2, 64 rows 7.2 / 8.8; 2048 -> 8192 9.6 /
+// 11.8, 12.9 / 16.1, -> 2048 7.2 / 6.9, 10.5 / 9.2; 4096 -> 12576 23.6 / 26.0, -> 6144
+// 15.6 / 13.7.
+int lds_linear_plain_parts(int M, int N, int K) {
+  const int parts = lds_linear_rows_parts(M, N, K);
+  const bool one = M <= ROWS && N <= 128 * 128 &&
+                   (K <= 1024 || (K <= 2048 && N >= 4096) ||
+                    (K <= 8192 && N >= 96 * 128));
+  return one ? 1 : parts;
+}
+
 // Whether a product of M rows is faster here than in the library. Device
 // times, here / there, in us:
 //   parts the caller sums itself: always. 4096 -> 4096: 1 row 8 / 15, 96 rows
@@ -258,25 +418,37 @@ int lds_linear_rows_parts(int M, int N, int K) {
 //     over 25 sizes (232 rows, 1024 -> [2 x 14624]: 28 / 35). In two or three
 //     rounds it is 0.66 to 1.06 times (245 rows, 3584 -> [2 x 28744]: 132 / 118), by
 //     longer K 0.74 to 1.07 (15872 -> [2 x 15456]: 367 / 271);
-//     inside a 4-layer stack of about 180 rows the pass takes 790 / 835;
-//     2048 -> [2 x 4096] (25 %): 32 rows 18 / 16.
+//     inside a 4-layer stack of about 180 rows the pass takes 790 / 835. Up to 64
+//     rows need not fill their round, for K from 1024 to 8192, of longer K with so many
+//     channels that most compute units have some (16 rows, here / library with the
+//     activation: 1024 -> [2 x 1024] 5.8 / 14.1, 2048 -> [2 x 8192] 14.4 / 19.8, 64 rows
+//     18 / 21, 4096 -> [2 x 1024] 64 rows 20.0 / 16.4, [2 x 6144] 20.7 / 29.6, [2 x
+//     10240] 33 / 70, 8192 -> [2 x 4096] 33.7 / 31.6, [2 x 6144] 43 / 44); from 257 up to
+//     full rounds either is the faster (4096 -> [2 x 25600] 77 / 98, 5120 -> [2 x 25600]
+//     98 / 94).
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
 //     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
 //     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
 //     narrow ones up to 64 rows (4096 -> 1024: 64 rows 11 / 15, 96 rows
-//     13 / 12; 4096 -> 12576, 77 %: 64 rows 27 / 25).
+//     13 / 12; 4096 -> 12576, 77 %: 64 rows 27 / 25), or of one part (lds_linear_plain_
+//     parts), of more than 16384 / 4 channels and K past 2048 up to 16 rows (2048 ->
+//     8192: 64 rows 12.9 / 13.5; 1024 -> 6144: 8.2 / 11.6; 4096 -> 12576: 16 rows
+//     24.2 / 27.6, 48 rows 26.2 / 25.5).
 int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   if (M > TILE_ROWS) return 0;
-  const int n = gated ? 1 : lds_linear_rows_parts(M, N, K);
-  if (parts && n > 1) return 1;
+  if (!gated && parts && lds_linear_rows_parts(M, N, K) > 1) return 1;
+  const int n = gated ? 1 : lds_linear_plain_parts(M, N, K);
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
+  if (gated && M <= ROWS && groups <= 256 && K >= 1024 &&
+      (K <= 2048 || (K <= 4096 && groups >= 72) || (K <= 8192 && groups >= 96)))
+    return 1;
   if (gated)
     return full && (M <= 192 || (groups <= 256 && K >= 1024 && K <= 8192 &&
                                  K % KS == 0));
   if (N > 128 * 128) return full && M <= 128;
   if (full) return M <= 64 || K >= 4096;
-  return M <= 64 && N <= 4096;
+  return M <= 64 && (N <= 4096 || (n == 1 && (K <= 2048 || M <= 16)));
 }
 
 // y [n] = the sum of part [parts, n], or (act >= 0) its activation; 16-byte aligned, n
@@ -308,18 +480,15 @@ hipError_t lds_linear_rows(const void* x, int64_t x_row, const void* w,
     return hipErrorInvalidValue;
   const bool in_part = parts > 1 || !y;
   hipError_t e;
-  if (M > ROWS) {
+  if (M > ROWS || (M > SPLIT_ROWS && parts > 1)) {
     e = lds_linear_tiles(x, x_row, w, w_row, in_part ? part : y, parts, M, N,
                          K, in_part || f32, -1, stream);
   } else {
     Rows p{(const short*)x, (const short*)w, x_row, w_row,
-           in_part ? part : y, M, N, K, K, 0};
+           in_part ? part : y, M, N, K, K, parts, 0};
     p.k_part = ((K + parts - 1) / parts + KS - 1) / KS * KS;
-    const bool two = channel_tiles(N) == 2;
-    if (in_part || f32)
-      e = two ? go<2, F32>(p, parts, stream) : go<1, F32>(p, parts, stream);
-    else
-      e = two ? go<2, BF16>(p, 1, stream) : go<1, BF16>(p, 1, stream);
+    if ((K + p.k_part - 1) / p.k_part != parts) return hipErrorInvalidValue;
+    e = in_part || f32 ? go_rows<F32>(p, stream) : go_rows<BF16>(p, stream);
   }
   if (e != hipSuccess || !in_part || !y) return e;
   return lds_sum_parts(part, y, (int64_t)M * N, parts, f32, -1, stream);
@@ -346,10 +515,21 @@ hipError_t lds_gated_rows(const void* x, int64_t x_row, const void* w,
     return hipErrorInvalidValue;
   if (M > ROWS)
     return lds_linear_tiles(x, x_row, w, w_row, y, 1, M, N, K, 0, act, stream);
-  // 64 channels per workgroup: 128 rows of weights
   const Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K,
-               (K + KS - 1) / KS * KS, act};
-  return go<1, GATED>(p, 1, stream);
+               (K + KS - 1) / KS * KS, 1, act};
+  return go_rows<GATED>(p, stream);
+}
+
+// y [M, N] = act(x w') of one part, for up to 64 rows and 128 x 128 channels
+hipError_t lds_activated_rows(const void* x, int64_t x_row, const void* w,
+                              int64_t w_row, void* y, int M, int N, int K,
+                              int act, hipStream_t stream) {
+  if (M < 1 || M > ROWS || N < 1 || N % 4 || N > 128 * 128 || K < 8 || K % 8 ||
+      x_row % 8 || w_row % 8 || act < 0 || act >= ACTS)
+    return hipErrorInvalidValue;
+  const Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K,
+               (K + KS - 1) / KS * KS, 1, act};
+  return go_rows<ACT>(p, stream);
 }
 
 }  // extern "C"

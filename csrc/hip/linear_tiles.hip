@@ -1,4 +1,5 @@
-// linear_tiles.hip — y = x w' for 17 to 256 rows of x (bf16, 32-bit sums).
+// linear_tiles.hip — y = x w' for 65 to 256 rows of x, from 33 where K is split (bf16,
+// 32-bit sums).
 //
 // The weights should be read from memory once, at its rate, so one workgroup
 // has all rows of x (tiles of 64, up to four) against 128 rows of w, and K is
@@ -13,12 +14,12 @@
 // with 8 of them each XCD's L2 holds one part of x. Workgroups start at
 // different steps, as in linear_rows.hip.
 //
-// Measured, cold weights, without the sum of the parts; library / the kernel
-// that took weights to registers and x through LDS, up to 128 rows: 4096 ->
-// 28672: 64 rows 41 us, 5.7 TB/s (54 / 50); 14336 -> 4096: 64 rows 23 us (40 /
-// 28), 160 rows 35 (84), 256 rows 41 (63); 25600 -> 5120: 30 rows 47 us (145 /
-// 50), 256 rows 111 (260). Above 128 rows matrix cores and LDS bound it (with
-// one row of x and of w repeated, nothing to fetch, 256 rows 64 of 75 us).
+// Measured, cold weights, without the sum of the parts (library): 4096 -> [2 x 14336]:
+// 128 rows 53 us (60); 14336 -> 4096: 128 rows 28.4, 160 rows 35 (84), 256 rows 41
+// (63); 25600 -> 5120: 256 rows 111 (260). Above 128 rows matrix cores and LDS bound it
+// (with one row of x and of w repeated, nothing to fetch, 256 rows 64 of 75 us), and
+// both operands' way to LDS: 4096 -> [2 x 14336], 178 rows 57 to 62 us, the loads alone
+// 50, those of w 42, matrix cores and LDS without loads 30.
 #include "layered/elem.h"
 #include "tile_core.h"
 
@@ -53,7 +54,7 @@ typedef TileCore<4, 8, 2, 3> Wide;
 // what is past the end of K
 __device__ const float4v zeros = {0.f, 0.f, 0.f, 0.f};
 
-// steps in the ring of 64 MT rows (6 for 64 rows are no faster), and their LDS
+// steps in the ring of 64 MT rows, and their LDS
 constexpr int ring(int MT) { return MT <= 2 ? 4 : 3; }
 constexpr int stage_bytes(int MT) { return (BN + 64 * MT) * ROW; }
 
@@ -305,7 +306,7 @@ hipError_t go_rows(Tiles p, hipStream_t stream) {
     p.w_bytes = (uint32_t)wb;
     if constexpr (OUT != BF16) return go_wide<OUT>(p, stream);
   }
-  if (p.M <= 64) return go<1, OUT>(p, stream);
+  if (OUT == F32 && p.M <= 64) return go<OUT == F32 ? 1 : 2, OUT>(p, stream);
   if (p.M <= 128) return go<2, OUT>(p, stream);
   if (p.M <= 192) return go<3, OUT>(p, stream);
   if constexpr (OUT == GATED) return hipErrorInvalidValue;

@@ -214,6 +214,29 @@ def test_act_of_few_rows(name, rows, n, k):
             _same(y, fn(z), 8)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("rows_of_w,k", [
+    (8192, 1024), (8208, 1032), (4112, 2048), (16384, 1152), (16400, 1280),
+    (9232, 4104), (1024, 1064), (28672, 2080)])
+def test_width_of_workgroups(rows, rows_of_w, k):
+    """Ends of blocks of 64 and 128 rows of w, K in halves of which the second is shorter
+    or ends inside a step: one part, its activation, 32-bit, gated."""
+    F, ext = torch.nn.functional, _ext("_hip_layered")
+    x = _draw(rows, k, seed=rows)
+    w = _draw(rows_of_w, k, seed=rows_of_w, scale=k ** -0.5)
+    z = x.double() @ w.double().t()
+    _same(ext.linear(x, w), z, 8)
+    for y, want, bits in [(ext.linear32(x, w), z, 16),
+                          (ext.activated_linear(x, w, 1), F.silu(z), 8)]:
+        if y is not None:
+            _same(y, want, bits)
+    g, u = z.chunk(2, -1)
+    y = ext.gated_linear(x, w, 1)
+    assert y is not None or k > 4096 or rows_of_w == 1024 and k > 2048
+    if y is not None:
+        _same(y, F.silu(g) * u, 8)
+
+
 @pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("rows,n", [(16, 4096), (8192, 8192)])
 @pytest.mark.parametrize("act", [-1, 3, 1 << 32])
