@@ -53,63 +53,86 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
   if (wave == 0) take_top(z, E, top, ids + row * top, wt + row * top);
 }
 
-// 16 rows per workgroup, K split among NW waves; ET: 16-expert tiles
-template <int ET, int NW>
-__global__ __launch_bounds__(NW * WAVE) void route_kernel(
+// A wave's 16 rows by 128 columns, loaded by 256 bytes of a row (x[j]: row j * 4 + lane /
+// 16, columns lane % 16 * 8), as operands of four matrix instructions (x[f]: row lane %
+// 16, columns f * 32 + lane / 16 * 8), by way of the wave's 4 KB of LDS.
+__device__ __forceinline__ void to_operand(char* lds, int lane, short8* x) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = j * 4 + lane / 16;
+    *(short8*)(lds + r * 256 + (lane % 16 ^ r) * 16) = x[j];
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+    x[f] = *(const short8*)(lds + lane % 16 * 256 + ((f * 4 + lane / 16) ^ lane % 16) * 16);
+}
+
+// 16 rows per workgroup. EG groups of KW waves have 16 ET experts each and share K.
+// Bound by what a compute unit can load: the lanes of a load are to follow each other in
+// a row of memory, as operands they lie in 16 rows and a load took four times as long.
+// 32 experts of 4096, 60 rows 9.8 us (15.0), 7800 rows 20.4 (32.9); 64 experts 17.2
+// (26.8), 31.0 (48.0); 128 of 2048 23.8 (38.4), 43.8 (61.8). 16 waves in place of 8 are
+// no faster up to 64 experts (9.6 and 23.7 us for 32), above they are (27.3 and 40.6 by 8).
+template <int ET, int EG, int KW>
+__global__ __launch_bounds__(EG * KW * WAVE) void route_kernel(
     const short* __restrict__ h, const short* __restrict__ w,
     int32_t* __restrict__ ids, float* __restrict__ wt, int64_t rows, int K,
     int E, int top) {
-  extern __shared__ float lds[];       // [NW][16 rows][16 ET]
+  extern __shared__ __align__(16) float lds[];   // 4 KB of a wave; [KW][16 rows][16 ES]
+  constexpr int ES = ET * EG;
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane % 16, grp = lane / 16;
+  const int e0 = wave / KW * ET * 16, kw = wave % KW;
   const int64_t row0 = (int64_t)blockIdx.x * 16;
-  const int64_t row = row0 + col < rows ? row0 + col : rows - 1;
+  char* mine = (char*)lds + wave * 4096;
   const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   float4v acc[ET];
 #pragma unroll
   for (int t = 0; t < ET; ++t) acc[t] = (float4v){0.f, 0.f, 0.f, 0.f};
   // past the end of K the row counts as zero; experts past E are not looked at
-  const short* wr[ET];
+  const short* h0 = h + row0 * K;
+  const int last = min(rows - 1 - row0, (int64_t)15);
+  for (int k0 = kw * 128; k0 < K; k0 += KW * 128) {
+    short8 a[4], b[ET][4];
+    const int k = k0 + col * 8, kc = min(k, K - 8);
 #pragma unroll
-  for (int t = 0; t < ET; ++t)
-    wr[t] = w + (int64_t)min(t * 16 + col, E - 1) * K;
-  constexpr int AHEAD = ET <= 2 ? 4 : 2;     // steps whose loads go together
-  for (int k0 = wave * 64; k0 < K; k0 += AHEAD * NW * 64) {
-    short8 a[AHEAD][2], b[AHEAD][2][ET];
+    for (int j = 0; j < 4; ++j) {
+      const int r = j * 4 + grp;
+      a[j] = *(const short8*)(h0 + (uint32_t)(min(r, last) * K + kc));
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
+      for (int t = 0; t < ET; ++t)
+        b[t][j] =
+            *(const short8*)(w + (uint32_t)(min(e0 + t * 16 + r, E - 1) * K + kc));
+    }
+    __builtin_amdgcn_sched_barrier(0);       // all loads ahead of their first use
+    if (k >= K)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int k = k0 + u * NW * 64 + grp * 16 + s * 8, kc = min(k, K - 8);
-        a[u][s] = *(const short8*)(h + row * K + kc);
-        if (k >= K) a[u][s] = zero;
+      for (int j = 0; j < 4; ++j) a[j] = zero;
+    to_operand(mine, lane, a);
 #pragma unroll
-        for (int t = 0; t < ET; ++t)
-          b[u][s][t] = *(const short8*)(wr[t] + kc);
-      }
+    for (int t = 0; t < ET; ++t) {
+      to_operand(mine, lane, b[t]);
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u)
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int t = 0; t < ET; ++t)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, b[u][s][t]),
-              __builtin_bit_cast(bf16x8, a[u][s]), acc[t], 0, 0, 0);
+      for (int f = 0; f < 4; ++f)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, b[t][f]), __builtin_bit_cast(bf16x8, a[f]),
+            acc[t], 0, 0, 0);
+    }
   }
+  __syncthreads();
 #pragma unroll
   for (int t = 0; t < ET; ++t)
-    *(float4v*)(lds + (wave * 16 + col) * 16 * ET + t * 16 + grp * 4) = acc[t];
+    *(float4v*)(lds + (kw * 16 + col) * 16 * ES + e0 + t * 16 + grp * 4) = acc[t];
   __syncthreads();
-  for (int i = threadIdx.x; i < 256 * ET; i += NW * WAVE) {
+  for (int i = threadIdx.x; i < 256 * ES; i += EG * KW * WAVE) {
     float s = lds[i];
 #pragma unroll
-    for (int v = 1; v < NW; ++v) s += lds[v * 256 * ET + i];
+    for (int v = 1; v < KW; ++v) s += lds[v * 256 * ES + i];
     lds[i] = s;
   }
   __syncthreads();
-  for (int r = wave; r < 16 && row0 + r < rows; r += NW)
-    take_top(lds + r * 16 * ET, E, top, ids + (row0 + r) * top,
+  for (int r = wave; r < 16 && row0 + r < rows; r += EG * KW)
+    take_top(lds + r * 16 * ES, E, top, ids + (row0 + r) * top,
              wt + (row0 + r) * top);
 }
 
@@ -523,7 +546,7 @@ hipError_t lds_route(int f32, const void* h, const void* w, int32_t* ids,
                      hipStream_t stream) {
   if (rows == 0) return hipSuccess;
   if (top < 1 || top > E || E > 8192) return hipErrorInvalidValue;
-  if (f32 || K % 8 || E > 256) {
+  if (f32 || K % 8 || E > 256 || (int64_t)E * K >= 1ll << 31) {
     const size_t lds = E * sizeof(float);
     if (f32)
       hipLaunchKernelGGL(route_plain_kernel<float>, dim3((uint32_t)rows),
@@ -536,14 +559,14 @@ hipError_t lds_route(int f32, const void* h, const void* w, int32_t* ids,
     HIP_CHECK_LAST();
     return hipSuccess;
   }
-#define GO(ET, NW)                                                            \
-  hipLaunchKernelGGL((route_kernel<ET, NW>),                                  \
-                     dim3((uint32_t)((rows + 15) / 16)), dim3(NW * WAVE),     \
-                     NW * 256 * ET * sizeof(float), stream, (const short*)h,  \
-                     (const short*)w, ids, wt, rows, K, E, top)
-  if (E <= 16) GO(1, 16); else if (E <= 32) GO(2, 16);
-  else if (E <= 64) GO(4, 16); else if (E <= 128) GO(8, 8);
-  else GO(16, 4);
+#define GO(ET, EG, KW)                                                        \
+  hipLaunchKernelGGL((route_kernel<ET, EG, KW>),                              \
+                     dim3((uint32_t)((rows + 15) / 16)),                      \
+                     dim3(EG * KW * WAVE), EG * KW * 4096, stream,            \
+                     (const short*)h, (const short*)w, ids, wt, rows, K, E, top)
+  if (E <= 16) GO(1, 1, 8); else if (E <= 32) GO(2, 1, 8);
+  else if (E <= 64) GO(2, 2, 4); else if (E <= 128) GO(2, 4, 4);
+  else GO(2, 8, 2);
 #undef GO
   HIP_CHECK_LAST();
   return hipSuccess;

@@ -278,6 +278,25 @@ class TestRoute:
         assert (wt == 0.5).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 16, 31])
+@pytest.mark.parametrize("K,E,top", [
+    (1024, 16, 2), (2056, 7, 2), (1160, 17, 4), (1016, 32, 4), (640, 33, 8),
+    (520, 64, 8), (504, 65, 8), (1032, 128, 8), (264, 129, 3), (248, 255, 9)])
+def test_route_by_groups_of_experts(T, K, E, top):
+    """Each split of experts and K over waves: whole steps, remainders of 8, waves
+    without a step, rows and experts past the end."""
+    run = ("cuda", torch.bfloat16)
+    h, w = put(rnd(T, K), run), put(rnd(E, K, seed=1, scale=K ** -0.5), run)
+    ids, wt = ops.route(h, w, top)
+    want_ids, want = oracle.route(f64(h), f64(w), top)
+    # sums of K products of size K ** -0.5 in 32 bits, then a slope of at most 1/4:
+    # under K * 2 ** -24 * 8 / K ** 0.5 / 4 < 6e-6
+    assert (wt.cpu().double() - want).abs().max() < 6e-6
+    s = oracle.sigmoid(f64(h) @ f64(w).T)
+    assert (torch.gather(s, 1, ids.cpu().long()) - want).abs().max() < 6e-6
+
+
 SHAPES = [(38, 11, 5), (64, 24, 7), (64, 64, 4), (192, 320, 6), (128, 200, 3)]
 
 
