@@ -7,10 +7,10 @@
 // cut into tiles of one expert each; the product kernels take one tile and a
 // block of output channels per workgroup:
 //   expert_tiles   256 pairs and 256 channels through LDS, for many pairs
-//   expert_rows    up to 64 pairs, weights straight into registers, for few:
-//                  there the weights' bytes are what counts
+//   expert_rows    up to 64 pairs, for few: there the weights' bytes are what counts
 //   expert_plain   any size, bf16 or float
 #include "elem.h"
+#include "../rows_core.h"
 #include "../tile_core.h"
 
 namespace {
@@ -295,95 +295,84 @@ __global__ __launch_bounds__(256) void expert_plain_kernel(const Pairs p) {
   }
 }
 
-// grid (blocks of 64 channels, tiles of 16 MT pairs). The waves split K; a
-// lane reads 32 bytes of a row at a time, 16 rows and 128 bytes of each per
-// wave. The order of K inside a step is the same for both operands.
-template <int MT, bool UP>
-__global__ __launch_bounds__(256) void expert_rows_kernel(const Pairs p) {
-  __shared__ float4v red[4][4][MT][WAVE];   // [channel tile][wave]
+// grid (blocks of BN channels up to a multiple of 8, tiles of up to 16 RT pairs). The
+// weights stream as in linear_rows.hip; by 64 channels there are two workgroups to a
+// compute unit, whose ends overlap, by 128 the pairs' rows are read half as often. Both
+// products, 32 experts of 4096 x 3584, 4 each, in us; before: weights straight to
+// registers, by 32 bytes of a row (their bytes alone take 313 at 6.0 TB/s):
+//   rows         8    60   150   300
+//   before     238   344   414   518
+//   64         225   325   338   360
+//   128        225   328   334   350
+// and 64 experts of 2048 x 1408, 6 each, 250 rows 191, 149, 151. So tiles of 64 pairs
+// take 128.
+template <int RT, int BN, bool UP>
+__global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs p) {
+  extern __shared__ __align__(16) char ring[];
+  typedef rows_core::RowsCore<RT, BN> Core;
+  constexpr int WL = Core::WL, XL = Core::XL, CT = Core::CT, MT = Core::MT;
   if ((int)blockIdx.y >= p.tiles[0].x) return;
-  const int4 tile = p.tiles[1 + blockIdx.y];
-  const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  const int col = lane % 16, grp = lane / 16, N = p.N, K = p.K;
-  const int n0 = blockIdx.x * 64;
-  const short *wr[4], *ar[MT];
+  const int N = p.N, K = p.K, blocks = gridDim.x;
+  const int i = rows_core::along_xcd(blockIdx.y * blocks + blockIdx.x,
+                                     p.tiles[0].x * blocks, BN == 64 ? 512 : 256);
+  const int4 tile = p.tiles[1 + i / blocks];
+  const int n0 = i % blocks * BN;
+  if (n0 >= N) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
+  const short *w_from[WL], *x_from[XL];
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-    wr[c] = (const short*)p.w +
-            ((int64_t)tile.x * N + min(n0 + c * 16 + col, N - 1)) * K;
+  for (int j = 0; j < XL; ++j) {
+    const int r = Core::x_row(wave, j);    // uniform: places come by scalar loads
+    int64_t from = 0;
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
-    ar[t] = (const short*)p.a +
-            source<UP>(p, tile.y + min(t * 16 + col, tile.z - 1)) * K;
-  float4v acc[4][MT];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
-  const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  short8 wf[4][2], af[MT][2], wn[4][2], an[MT][2];
-  // past the end of K the pairs' rows count as zero
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int k = k0 + grp * 16 + s * 8, kc = min(k, K - 8);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) wn[c][s] = *(const short8*)(wr[c] + kc);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        if constexpr (MT > 2) {      // worth leaving absent pairs out
-          an[t][s] = k < K && t * 16 + col < tile.z
-                         ? *(const short8*)(ar[t] + k)
-                         : zero;
-        } else {
-          an[t][s] = *(const short8*)(ar[t] + kc);
-          if (k >= K) an[t][s] = zero;
-        }
-      }
+    for (int q = 0; q < 4; ++q) {
+      const int64_t f = source<UP>(p, tile.y + min(r + q, tile.z - 1));
+      from = grp == q ? f : from;
     }
-  };
-  fetch(wave * 64);
-  for (int k0 = wave * 64; k0 < K; k0 += 256) {
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) wf[c][s] = wn[c][s];
-#pragma unroll
-      for (int t = 0; t < MT; ++t) af[t][s] = an[t][s];
-    }
-    fetch(k0 + 256);
-#pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int t = 0; t < MT; ++t)
-          acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8, wf[c][s]),
-              __builtin_bit_cast(bf16x8, af[t][s]), acc[c][t], 0, 0, 0);
+    x_from[j] = (const short*)p.a + from * K + Core::piece(r + grp, lane);
   }
 #pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) red[c][wave][t][lane] = acc[c][t];
-  __syncthreads();
-  const int n = n0 + wave * 16 + grp * 4;    // this wave's channels
-  if (n >= N) return;
+  for (int j = 0; j < WL; ++j) {
+    const int r = Core::w_row(wave, j) + grp;
+    w_from[j] = (const short*)p.w +
+                ((int64_t)tile.x * N + min(n0 + r, N - 1)) * K + Core::piece(r, lane);
+  }
+  float4v acc[CT][MT];
+  const int steps = (K + rows_core::KS - 1) / rows_core::KS;
+  Core::run(ring, wave, lane, w_from, x_from, 0, K, steps,
+            uint32_t(i) * BN / 128 * 3 % uint32_t(steps), acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const int i = t * 16 + col;
-    if (i >= tile.z) continue;
-    const int pair = p.order[tile.y + i];
+    const int m = (wave / Core::WC * MT + t) * 16 + col;
+    if (m >= tile.z) continue;
+    const int pair = p.order[tile.y + m];
     const float wt = UP ? p.weights[pair] : 1.f;
-    float4v s = red[wave][0][t][lane];
 #pragma unroll
-    for (int v = 1; v < 4; ++v) s += red[wave][v][t][lane];
-    *(short4v*)((short*)p.out + (int64_t)(UP ? tile.y + i : pair) * N + n) =
-        (short4v){f32_to_bf16(finish<UP>(p, s[0], wt)),
-                  f32_to_bf16(finish<UP>(p, s[1], wt)),
-                  f32_to_bf16(finish<UP>(p, s[2], wt)),
-                  f32_to_bf16(finish<UP>(p, s[3], wt))};
+    for (int c = 0; c < CT; ++c) {
+      const int n = n0 + (wave % Core::WC * CT + c) * 16 + grp * 4;
+      if (n >= N) continue;
+      const float4v s = acc[c][t];
+      *(short4v*)((short*)p.out + (int64_t)(UP ? tile.y + m : pair) * N + n) =
+          (short4v){f32_to_bf16(finish<UP>(p, s[0], wt)),
+                    f32_to_bf16(finish<UP>(p, s[1], wt)),
+                    f32_to_bf16(finish<UP>(p, s[2], wt)),
+                    f32_to_bf16(finish<UP>(p, s[3], wt))};
+    }
   }
+}
+
+template <int RT, int BN, bool UP>
+hipError_t launch_rows(const Pairs& p, int max_tiles, hipStream_t stream) {
+  typedef rows_core::RowsCore<RT, BN> Core;
+  auto fn = expert_rows_kernel<RT, BN, UP>;
+  const hipError_t e = hipFuncSetAttribute(
+      (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, Core::RINGS);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(((p.N + BN - 1) / BN + 7) / 8 * 8, max_tiles),
+                     dim3(Core::NW * WAVE), Core::RINGS, stream, p);
+  HIP_CHECK_LAST();
+  return hipSuccess;
 }
 
 // 256 channels x 256 pairs, or 128 where a tile has no more (so nothing is lost by
@@ -528,9 +517,9 @@ hipError_t product(int f32, int plain, int tile, int max_tiles, const Pairs& p,
 #define K2(NAME, ARG) NAME<ARG, UP>
   if (f32) GO(K2(expert_plain_kernel, float));
   else if (plain || p.N % 8 || p.K % 8) GO(K2(expert_plain_kernel, short));
-  else if (tile <= 16) GO(K2(expert_rows_kernel, 1));
-  else if (tile <= 32) GO(K2(expert_rows_kernel, 2));
-  else GO(K2(expert_rows_kernel, 4));
+  else if (tile <= 16) return launch_rows<1, 64, UP>(p, max_tiles, stream);
+  else if (tile <= 32) return launch_rows<2, 64, UP>(p, max_tiles, stream);
+  else return launch_rows<4, 128, UP>(p, max_tiles, stream);
 #undef K2
 #undef GO
   HIP_CHECK_LAST();

@@ -3,29 +3,22 @@
 // linear_tiles.hip.
 //
 // The weights' bytes are what counts. A workgroup has all rows of x against 128 rows
-// of w, or 64 where those of 128 leave compute units idle, and K is split until the
-// workgroups make up a round of the 256 compute units. Both operands go to LDS by
-// direct loads, 128 of K at a time, into a ring of three steps: 64 KB of w per compute
-// unit are under way. What the rate hangs on is the length of what is read of a row at
-// a time: 256 bytes of each by one instruction come at 5.9 TB/s, pieces of 128 take 10
-// to 20 % longer (14336 -> 4096 read and nothing else: 21.3 us, 23.8; 25600 -> 5120:
-// 45, 54). Workgroups start at different steps: in step they would hit the same few
-// memory channels where rows are a power of two apart (read and nothing else, 4096 ->
-// [2 x 14336], a start of 6 blocks: 41.5 us, 1: 63, none: 48). Where K is one part each
-// XCD has blocks that follow each other (39.9). linear_tiles.hip adds up in the same
-// order, so a row comes out the same, to the bit, whichever of the two took it: as the
-// one row of a decode step or within a short prompt.
+// of w, or 64 where those of 128 leave compute units idle, by the loop of rows_core.h,
+// and K is split until the workgroups make up a round of the 256 compute units.
+// linear_tiles.hip adds up in the same order, so a row comes out the same, to the bit,
+// whichever of the two took it: as the one row of a decode step or within a short
+// prompt.
 //
 // Measured, cold weights, without the sum of the parts; before: up to 16 rows weights
 // straight to registers, x through LDS, above 128 bytes of a row at a time: 1 row,
 // 4096 -> [2 x 14336] 41.9 us, 5.6 TB/s (43.5; library 58 and the activation), 4096 ->
 // 6144 11.0 (11.9), 14336 -> 4096 21.9 (22.6), 4096 -> 4096 7.5 (8.0), 25600 -> 5120
 // 46.3 (47.9); 30 rows 42.5, 12.0, 23.0, 8.4, 48.4 (45.4, 12.0, 23.2, 8.7, 48.9).
-#include "layered/elem.h"
+#include "rows_core.h"
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+using namespace rows_core;
 
 struct Rows {
   const short *x, *w;        // [M, K], [N, K] (GATED: [2 N, K], gate first)
@@ -39,12 +32,7 @@ struct Rows {
 // act(gate) * up as bf16
 enum Out { BF16, F32, ACT, GATED };
 
-constexpr int KS = 128, ROW = KS * 2;          // ROW: bytes of a row in LDS
 constexpr int ROUND = 256;       // compute units
-constexpr int RING = 3;          // 4 are no faster, 2 up to 15 % slower
-
-// what is past the end of K
-__device__ const float4v zeros = {0.f, 0.f, 0.f, 0.f};
 
 // RT: rows of x / 16. BN rows of w; KG: groups of BN / 16 waves, each with its share of
 // K, whose sums meet at the end. A wave has CT tiles of 16 channels by MT of 16 rows.
@@ -52,26 +40,17 @@ template <int RT, int BN, int KG, int OUT>
 __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
     const Rows p) {
   extern __shared__ __align__(16) char lds[];
-  constexpr int NW = BN / 16, WM = RT == 1 ? 1 : 2, WC = NW / WM;
-  constexpr int CT = BN / 16 / WC, MT = RT / WM;
-  // a group's rings: RING steps of w, two of x, whose lines are near
-  constexpr int W_STEP = BN * ROW, X_STEP = 16 * RT * ROW;
-  constexpr int RINGS = RING * W_STEP + 2 * X_STEP;
-  // loads of a wave, 4 rows each (where x has fewer the last one is repeated)
-  constexpr int WL = BN / 4 / NW, XL = (4 * RT + NW - 1) / NW;
+  typedef RowsCore<RT, BN> Core;
+  constexpr int NW = Core::NW, WC = Core::WC, CT = Core::CT, MT = Core::MT;
+  constexpr int WL = Core::WL, XL = Core::XL;
   constexpr int CH = OUT == GATED ? BN / 2 : BN;       // channels
   const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int group = all / NW, wave = all % NW;
   const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
   const int M = p.M, N = p.N;
   const int part = blockIdx.x % p.parts;
-  // a round of the chip, in which an XCD has blocks that follow each other (65536 x 2048:
-  // 52.4 us, 59.6 in the order of the grid; over the whole grid 49.3, but 128256 x 4096
-  // 171.6, 168.7 and 175.9: eight far ends of a large matrix)
-  const int round = blockIdx.x / ROUND * ROUND, at = blockIdx.x - round;
   const int blk = p.parts > 1 ? blockIdx.x / p.parts
-                              : round + at % 8 * (min(ROUND, int(gridDim.x) - round) / 8) +
-                                    at / 8;
+                              : along_xcd(blockIdx.x, gridDim.x, ROUND);
   if (blk * CH >= N) return;
   // this group's K: steps of KS, the last ones past the end where they do not go round
   const int p_lo = part * p.k_part, p_hi = min(p.K, p_lo + p.k_part);
@@ -82,129 +61,29 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
                      : N > 128 * 256 ? blk * BN / 256 * 3
                                      : blk * BN / 128 * 3) %
                     steps;
-  char* const w_ring = lds + group * RINGS;
-  char* const x_ring = w_ring + RING * W_STEP;
-
-  // A load takes 4 rows of KS, 16 pieces of 16 bytes each; the pieces of a row change
-  // places by XOR with its number, so that 16 lanes that read one piece of 16 rows
-  // find all banks. Rows that do not exist repeat the last one. GATED: of 32 rows of w
-  // 16 are of gate, 16 the same ones of up; with one tile per wave the halves are.
-  const int r4 = lane / 16;
+  // Rows that do not exist repeat the last one. GATED: of 32 rows of w 16 are of gate, 16
+  // the same ones of up; with one tile per wave the halves are.
   const short *w_from[WL], *x_from[XL];
 #pragma unroll
   for (int j = 0; j < WL; ++j) {
-    const int r = (wave * WL + j) * 4 + r4;            // row in LDS
+    const int r = Core::w_row(wave, j) + grp;          // row in LDS
     const int n = OUT != GATED ? r : CT == 1 ? r % CH : r / 32 * 16 + r % 16;
     const bool up = OUT == GATED && (CT == 1 ? r >= CH : r % 32 >= 16);
     w_from[j] = p.w + (min(blk * CH + n, N - 1) + (up ? N : 0)) * p.w_row +
-                (lane % 16 ^ r % 16) * 8;
+                Core::piece(r, lane);
   }
 #pragma unroll
   for (int j = 0; j < XL; ++j) {
-    const int r = min(wave * XL + j, 4 * RT - 1) * 4 + r4;
-    x_from[j] = p.x + min(r, M - 1) * p.x_row + (lane % 16 ^ r % 16) * 8;
+    const int r = Core::x_row(wave, j) + grp;
+    x_from[j] = p.x + min(r, M - 1) * p.x_row + Core::piece(r, lane);
   }
-  typedef const __attribute__((address_space(1))) unsigned int gmem;
-  typedef __attribute__((address_space(3))) unsigned int smem;
-  auto k_of = [&](int s) {
-    s += first;
-    return k_lo + (s >= steps ? s - steps : s) * KS;
-  };
-  // 4 rows of K from k on, rows 4 q .. of their kind
-  auto load = [&](const short* from, char* to, int q, int k) {
-    const bool in = k + (lane % 16 ^ (q * 4 + r4) % 16) * 8 < k_hi;
-    __builtin_amdgcn_global_load_lds(
-        (gmem*)(in ? from + k : (const short*)&zeros), (smem*)(to + q * 1024),
-        16, 0, 0);
-  };
-  auto issue_w = [&](int s, int buf) {
-    const int k = k_of(s);
-#pragma unroll
-    for (int j = 0; j < WL; ++j)
-      load(w_from[j], w_ring + buf * W_STEP, wave * WL + j, k);
-  };
-  auto issue_x = [&](int s) {
-    const int k = k_of(s);
-#pragma unroll
-    for (int j = 0; j < XL; ++j)
-      load(x_from[j], x_ring + s % 2 * X_STEP, min(wave * XL + j, 4 * RT - 1), k);
-  };
-
   float4v acc[CT][MT];
-#pragma unroll
-  for (int c = 0; c < CT; ++c)
-#pragma unroll
-    for (int t = 0; t < MT; ++t) acc[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
-  const int wc = wave % WC, wm = wave / WC;
-  struct Operands {
-    bf16x8 w[CT], x[MT];
-  };
-  const int w_at = (wc * 16 * CT + col) * ROW, x_at = (wm * 16 * MT + col) * ROW;
-  auto read = [&](Operands& o, int buf, int s, int q) {       // q: 32 of K
-    const int piece = ((q * 4 + grp) ^ col) * 16;
-    const char* w = w_ring + buf * W_STEP + w_at + piece;
-    const char* x = x_ring + s % 2 * X_STEP + x_at + piece;
-#pragma unroll
-    for (int c = 0; c < CT; ++c)
-      o.w[c] = *(const bf16x8*)(w + c * 16 * ROW);
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-      o.x[t] = *(const bf16x8*)(x + t * 16 * ROW);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto multiply = [&](const Operands& o) {
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int c = 0; c < CT; ++c)
-        acc[c][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            o.w[c], o.x[t], acc[c][t], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  // step s has landed, and so it has for the other waves, when only w of the next one
-  // is under way
-  auto landed = [&](int s) {
-    if (s + 1 < steps)
-      asm volatile("s_waitcnt vmcnt(%0)" ::"i"(WL) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-  };
-
-  // Operands are read 32 of K ahead of their products. At the barrier ahead of the
-  // last of step s all of its operands are in registers: its places take w of step
-  // s + RING and x of step s + 2.
-  static_assert(RING == 3, "");
-  issue_w(0, 0);
-  issue_x(0);
-  if (1 < steps) issue_w(1, 1);
-  Operands o0, o1;
-  landed(0);
-  if (1 < steps) issue_x(1);
-  if (2 < steps) issue_w(2, 2);
-  read(o0, 0, 0, 0);
-  int buf = 0;
-  for (int s = 0; s < steps; ++s) {
-    read(o1, buf, s, 1);
-    multiply(o0);
-    read(o0, buf, s, 2);
-    multiply(o1);
-    read(o1, buf, s, 3);
-    multiply(o0);
-    if (s + 1 < steps) {
-      landed(s + 1);
-      if (s + 2 < steps) issue_x(s + 2);
-      if (s + RING < steps) issue_w(s + RING, buf);
-      buf = buf + 1 == RING ? 0 : buf + 1;
-      read(o0, buf, s + 1, 0);
-    }
-    multiply(o1);
-  }
+  Core::run(lds + group * Core::RINGS, wave, lane, w_from, x_from, k_lo, k_hi, steps,
+            first, acc);
+  const int wc = wave % WC, wm = wave / WC;      // its channels, its rows
 
   if constexpr (KG > 1) {                  // to the sums of the first group
-    static_assert(KG == 2 && CT * MT * NW * 1024 <= RINGS, "");
+    static_assert(KG == 2 && CT * MT * NW * 1024 <= Core::RINGS, "");
     float4v* other = (float4v*)lds;
     __syncthreads();                       // the rings are no longer read
 #pragma unroll
@@ -322,7 +201,7 @@ __global__ __launch_bounds__(256) void lay_weights_kernel(
 template <int RT, int BN, int KG, int OUT>
 hipError_t go(const Rows& p, hipStream_t stream) {
   constexpr int width = OUT == GATED ? BN / 2 : BN;
-  constexpr int bytes = KG * (RING * BN + 2 * 16 * RT) * ROW;
+  constexpr int bytes = KG * RowsCore<RT, BN>::RINGS;
   auto fn = linear_rows_kernel<RT, BN, KG, OUT>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);

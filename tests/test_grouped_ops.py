@@ -361,6 +361,28 @@ class TestExperts:
             close(one, f64(many[2 * t:2 * t + 2]), run, f32=1e-5, bf16=2e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,F", [(8, 8), (120, 136), (128, 64), (136, 1032), (520, 72),
+                                 (1024, 256)])
+@pytest.mark.parametrize("pairs", [1, 9, 12, 16, 17, 24, 33, 48])
+def test_experts_of_few_pairs(K, F, pairs):
+    """Each size of tiles: less than a step of K, remainders, channels past the end."""
+    run, E = ("cuda", torch.bfloat16), 5
+    up = put(rnd(E, F, K, seed=2, scale=K ** -0.5), run)
+    down = put(rnd(E, K, F, seed=3, scale=F ** -0.5), run)
+    g = torch.Generator().manual_seed(pairs)
+    # all experts but one, unevenly: up to twice the mean number of pairs
+    ids = torch.cat([torch.full((2 * pairs,), 4), torch.full((pairs,), 0),
+                     torch.full((max(1, pairs - 3),), 2), torch.full((1,), 3)])
+    ids = ids[torch.randperm(len(ids), generator=g)].int()[:, None]
+    h = put(rnd(len(ids), K), run)
+    wt = torch.rand(len(ids), 1, generator=g) * 0.9 + 0.05
+    out = ops.experts(h, ids.cuda(), wt.cuda(), up, down, "relu_squared")
+    want = TestExperts().want(h, ids, wt, up, down)
+    # the inner rows and the results are rounded to 8 bits, 32-bit sums beside that
+    close(out, want, run, bf16=2e-2)
+
+
 @GPU
 @pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (192, 128), (64, 256)])
 @pytest.mark.parametrize("bs", [1, 5, 64])
