@@ -26,6 +26,7 @@ struct Rows {
   void* y;                   // [M, N]; F32: [parts, M, N] 32-bit
   int M, N, K, k_part;       // k_part: K per part, a multiple of KS
   int parts, act;
+  int width;                 // rows of w of a workgroup, a multiple of 16
 };
 
 // what becomes of the sums: bf16, 32-bit (also of a part of K), act of them or
@@ -43,7 +44,6 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
   typedef RowsCore<RT, BN> Core;
   constexpr int NW = Core::NW, WC = Core::WC, CT = Core::CT, MT = Core::MT;
   constexpr int WL = Core::WL, XL = Core::XL;
-  constexpr int CH = OUT == GATED ? BN / 2 : BN;       // channels
   const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int group = all / NW, wave = all % NW;
   const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
@@ -51,26 +51,26 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
   const int part = blockIdx.x % p.parts;
   const int blk = p.parts > 1 ? blockIdx.x / p.parts
                               : along_xcd(blockIdx.x, gridDim.x, ROUND);
-  if (blk * CH >= N) return;
+  const int width = p.width, n0 = OUT == GATED ? blk * (width / 2) : blk * width;
+  if (n0 >= N) return;
   // this group's K: steps of KS, the last ones past the end where they do not go round
   const int p_lo = part * p.k_part, p_hi = min(p.K, p_lo + p.k_part);
   const int steps = ((p_hi - p_lo + KS - 1) / KS + KG - 1) / KG;
   const int k_lo = p_lo + group * steps * KS, k_hi = min(p_hi, k_lo + steps * KS);
   // by blocks of 128 rows of w, as in linear_tiles.hip
-  const int first = (OUT == GATED    ? blk * BN / 128 * 6
-                     : N > 128 * 256 ? blk * BN / 256 * 3
-                                     : blk * BN / 128 * 3) %
+  const int first = (OUT == GATED    ? blk * width / 128 * 6
+                     : N > 128 * 256 ? blk * width / 256 * 3
+                                     : blk * width / 128 * 3) %
                     steps;
-  // Rows that do not exist repeat the last one. GATED: of 32 rows of w 16 are of gate, 16
-  // the same ones of up; with one tile per wave the halves are.
+  // Rows that do not exist repeat the last one. GATED: of 16 rows of w 8 are of gate, 8
+  // the same ones of up.
   const short *w_from[WL], *x_from[XL];
 #pragma unroll
   for (int j = 0; j < WL; ++j) {
     const int r = Core::w_row(wave, j) + grp;          // row in LDS
-    const int n = OUT != GATED ? r : CT == 1 ? r % CH : r / 32 * 16 + r % 16;
-    const bool up = OUT == GATED && (CT == 1 ? r >= CH : r % 32 >= 16);
-    w_from[j] = p.w + (min(blk * CH + n, N - 1) + (up ? N : 0)) * p.w_row +
-                Core::piece(r, lane);
+    const int n = OUT == GATED ? r / 16 * 8 + r % 8 : r;
+    const bool up = OUT == GATED && r % 16 >= 8;
+    w_from[j] = p.w + (min(n0 + n, N - 1) + (up ? N : 0)) * p.w_row + Core::piece(r, lane);
   }
 #pragma unroll
   for (int j = 0; j < XL; ++j) {
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
   }
   float4v acc[CT][MT];
   Core::run(lds + group * Core::RINGS, wave, lane, w_from, x_from, k_lo, k_hi, steps,
-            first, acc);
+            first, wave * 16 < width, acc);
   const int wc = wave % WC, wm = wave / WC;      // its channels, its rows
 
   if constexpr (KG > 1) {                  // to the sums of the first group
@@ -93,57 +93,43 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
         if (group == 1)
           other[((c * MT + t) * NW + wave) * WAVE + lane] = acc[c][t];
     __syncthreads();
-    if (group == 1) {
-      if (OUT != GATED || CT > 1) return;
-    } else {
+    if (group == 1) return;
 #pragma unroll
-      for (int c = 0; c < CT; ++c)
+    for (int c = 0; c < CT; ++c)
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-          acc[c][t] += other[((c * MT + t) * NW + wave) * WAVE + lane];
-    }
+      for (int t = 0; t < MT; ++t)
+        acc[c][t] += other[((c * MT + t) * NW + wave) * WAVE + lane];
   }
-  // lane: row `col` of a tile, channels 4 grp ..
-  if constexpr (OUT == GATED) {
-    if constexpr (CT == 1) {               // up is with the other half of the waves
-      static_assert(MT == 1, "");
-      float4v* other = (float4v*)lds;
-      __syncthreads();
-      if (group == 0 && wave >= NW / 2)
-        other[(wave - NW / 2) * WAVE + lane] = acc[0][0];
-      __syncthreads();
-      if (group > 0 || wave >= NW / 2) return;
-    }
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int m = (wm * MT + t) * 16 + col, n = blk * CH + wc * 16 + grp * 4;
-      if (m >= M || n >= N) continue;      // N is a multiple of 4
-      const float4v u = CT == 1 ? ((const float4v*)lds)[wave * WAVE + lane]
-                                : acc[CT - 1][t];
-      short4v v;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        v[r] = f32_to_bf16(activate(p.act, acc[0][t][r]) * u[r]);
-      *(short4v*)((short*)p.y + (int64_t)m * N + n) = v;
-    }
-    return;
-  }
+  // lane: row `col` of a tile, channels 4 grp ..; GATED: gate with the lower half of the
+  // lanes, up with the other, and of two tiles each half takes one
 #pragma unroll
   for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int c = 0; c < CT; ++c) {
+    for (int c = 0; c < CT; c += OUT == GATED ? 2 : 1) {
       const int m = (wm * MT + t) * 16 + col;
-      const int n = blk * BN + (wc * CT + c) * 16 + grp * 4;
-      if (m >= M || n >= N) continue;
+      int tile = wc * CT + c, n = n0 + tile * 16 + grp * 4;
+      float4v s = acc[c][t];
+      if constexpr (OUT == GATED) {
+        tile += grp / 2;
+        n = n0 + tile * 8 + grp % 2 * 4;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const auto both = __builtin_amdgcn_permlane32_swap(
+              __float_as_uint(s[r]), __float_as_uint(acc[CT == 1 ? c : c + 1][t][r]),
+              false, false);
+          s[r] = activate(p.act, __uint_as_float(both[0])) * __uint_as_float(both[1]);
+        }
+        if (CT == 1 && grp >= 2) continue;
+      }
+      if (m >= M || n >= N || tile * 16 >= width) continue;    // N is a multiple of 4
       const int64_t o = ((int64_t)part * M + m) * N + n;
       if constexpr (OUT == F32) {
-        *(float4v*)((float*)p.y + o) = acc[c][t];
+        *(float4v*)((float*)p.y + o) = s;
       } else {
         short4v v;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          v[r] = f32_to_bf16(OUT == ACT ? activate(p.act, acc[c][t][r])
-                                        : acc[c][t][r]);
+          v[r] = f32_to_bf16(OUT == ACT ? activate(p.act, s[r]) : s[r]);
         *(short4v*)((short*)p.y + o) = v;
       }
     }
@@ -198,15 +184,28 @@ __global__ __launch_bounds__(256) void lay_weights_kernel(
   }
 }
 
+// Rows of w of a workgroup: as many rounds of the chip as by 128, each full, unless they
+// nearly are by 128 (16 rows, before / so: 8668 x 5640 gated 52.1 / 41.2 us, 17408 x 5120
+// 87.4 / 69.5, 25600 x 5120 99.4 / 94.0, 20480 x 2048 37.7 / 33.4; 36864 x 4096 plain 66.1
+// / 54.5, 41000 x 3072 54.2 / 48.5).
+int even_width(int rows) {
+  const int blocks = (rows + 127) / 128, slots = (blocks + ROUND - 1) / ROUND * ROUND;
+  if (blocks * 8 >= slots * 7) return 128;
+  return ((rows + slots - 1) / slots + 15) / 16 * 16;
+}
+
 template <int RT, int BN, int KG, int OUT>
-hipError_t go(const Rows& p, hipStream_t stream) {
-  constexpr int width = OUT == GATED ? BN / 2 : BN;
+hipError_t go(Rows p, hipStream_t stream) {
   constexpr int bytes = KG * RowsCore<RT, BN>::RINGS;
   auto fn = linear_rows_kernel<RT, BN, KG, OUT>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
-  int groups = (p.N + width - 1) / width * p.parts;
+  const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
+  p.width = BN;
+  if (p.parts == 1 && BN == 128) p.width = even_width(rows);
+  const int ch = OUT == GATED ? p.width / 2 : p.width;
+  int groups = (p.N + ch - 1) / ch * p.parts;
   if (p.parts == 1) groups = (groups + 7) / 8 * 8;     // equal shares of the XCDs
   hipLaunchKernelGGL(fn, dim3(groups), dim3(BN / 16 * KG * WAVE), bytes, stream,
                      p);
@@ -301,10 +300,8 @@ int lds_linear_plain_parts(int M, int N, int K) {
 //     rows need not fill their round, for K from 1024 to 8192, of longer K with so many
 //     channels that most compute units have some (16 rows, here / library with the
 //     activation: 1024 -> [2 x 1024] 5.8 / 14.1, 2048 -> [2 x 8192] 14.4 / 19.8, 64 rows
-//     18 / 21, 4096 -> [2 x 1024] 64 rows 20.0 / 16.4, [2 x 6144] 20.7 / 29.6, [2 x
-//     10240] 33 / 70, 8192 -> [2 x 4096] 33.7 / 31.6, [2 x 6144] 43 / 44); from 257 up to
-//     full rounds either is the faster (4096 -> [2 x 25600] 77 / 98, 5120 -> [2 x 25600]
-//     98 / 94).
+//     18 / 21, 4096 -> [2 x 1024] 64 rows 20.0 / 16.4, [2 x 6144] 20.7 / 29.6, 8192 ->
+//     [2 x 4096] 33.7 / 31.6, [2 x 6144] 43 / 44).
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
 //     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
 //     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
@@ -313,12 +310,17 @@ int lds_linear_plain_parts(int M, int N, int K) {
 //     parts), of more than 16384 / 4 channels and K past 2048 up to 16 rows (2048 ->
 //     8192: 64 rows 12.9 / 13.5; 1024 -> 6144: 8.2 / 11.6; 4096 -> 12576: 16 rows
 //     24.2 / 27.6, 48 rows 26.2 / 25.5).
+//   more than 16384 rows of w, in even rounds (even_width): up to 64 rows, K from 512 to
+//     10240. Over 76 sizes of 16384 to 130000 rows of w, gated and plain, 4 to 64 rows of
+//     x, 1.3 times as fast at the median; slower by 3 and 6 % at two (51200 x 5120 and
+//     49152 x 1024, plain, 64 rows), and past that range 53248 x 16384 649 / 622.
 int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   if (M > TILE_ROWS) return 0;
   if (!gated && parts && lds_linear_rows_parts(M, N, K) > 1) return 1;
   const int n = gated ? 1 : lds_linear_plain_parts(M, N, K);
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
+  if (M <= ROWS && (gated ? 2 : 1) * N > 128 * 128 && K >= 512 && K <= 10240) return 1;
   if (gated && M <= ROWS && groups <= 256 && K >= 1024 &&
       (K <= 2048 || (K <= 4096 && groups >= 72) || (K <= 8192 && groups >= 96)))
     return 1;

@@ -58,11 +58,12 @@ struct RowsCore {
 
   // K from k_lo to k_hi in `steps` of KS, from step `first` on and round; past k_hi it
   // counts as zero. w_from, x_from: the lane's piece at K = 0 of its row, w_row + lane /
-  // 16 and x_row + lane / 16, of each load; rows that do not exist repeat others.
+  // 16 and x_row + lane / 16, of each load; rows that do not exist repeat others. A wave
+  // without any of w (its 16 from w_row on) says so by `some`.
   static __device__ __forceinline__ void run(
       char* lds, int wave, int lane, const short* const (&w_from)[WL],
       const short* const (&x_from)[XL], int k_lo, int k_hi, int steps, int first,
-      float4v (&acc)[CT][MT]) {
+      bool some, float4v (&acc)[CT][MT]) {
     char* const w_ring = lds;
     char* const x_ring = lds + RING * W_STEP;
     const int col = lane % 16, grp = lane / 16;
@@ -80,6 +81,7 @@ struct RowsCore {
           16, 0, 0);
     };
     auto issue_w = [&](int s, int buf) {
+      if (!some) return;
       const int k = k_of(s);
 #pragma unroll
       for (int j = 0; j < WL; ++j)
@@ -125,7 +127,7 @@ struct RowsCore {
     // step s has landed, and so it has for the other waves, when only w of the next one
     // is under way
     auto landed = [&](int s) {
-      if (s + 1 < steps)
+      if (some && s + 1 < steps)
         asm volatile("s_waitcnt vmcnt(%0)" ::"i"(WL) : "memory");
       else
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

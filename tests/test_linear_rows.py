@@ -237,6 +237,21 @@ def test_width_of_workgroups(rows, rows_of_w, k):
         _same(y, F.silu(g) * u, 8)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("rows_of_w,k", [
+    (16400, 512), (16416, 520), (24576, 768), (28688, 640), (32784, 512), (41008, 1032),
+    (47120, 512), (57344, 520), (65552, 640), (70016, 512)])
+def test_even_rounds(rows, rows_of_w, k):
+    """Blocks of 80 to 128 rows of w: waves without rows, the last block's end."""
+    F, ext = torch.nn.functional, _ext("_hip_layered")
+    x = _draw(rows, k, seed=rows)
+    w = _draw(rows_of_w, k, seed=rows_of_w, scale=k ** -0.5)
+    z = x.double() @ w.double().t()
+    _same(ext.linear(x, w), z, 8)
+    g, u = z.chunk(2, -1)
+    _same(ext.gated_linear(x, w, 1), F.silu(g) * u, 8)
+
+
 @pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("rows,n", [(16, 4096), (8192, 8192)])
 @pytest.mark.parametrize("act", [-1, 3, 1 << 32])
