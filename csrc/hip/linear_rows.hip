@@ -26,7 +26,7 @@ struct Rows {
   void* y;                   // [M, N]; F32: [parts, M, N] 32-bit
   int M, N, K, k_part;       // k_part: K per part, a multiple of KS
   int parts, act;
-  int width;                 // rows of w of a workgroup, a multiple of 16
+  int width;                 // rows of w of a workgroup, a multiple of UNIT
 };
 
 // what becomes of the sums: bf16, 32-bit (also of a part of K), act of them or
@@ -34,6 +34,7 @@ struct Rows {
 enum Out { BF16, F32, ACT, GATED };
 
 constexpr int ROUND = 256;       // compute units
+constexpr int UNIT = 8;
 
 // RT: rows of x / 16. BN rows of w; KG: groups of BN / 16 waves, each with its share of
 // K, whose sums meet at the end. A wave has CT tiles of 16 channels by MT of 16 rows.
@@ -64,13 +65,14 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
                     steps;
   // Rows that do not exist repeat the last one. GATED: of 16 rows of w 8 are of gate, 8
   // the same ones of up.
+  const int n1 = min(N, n0 + (OUT == GATED ? width / 2 : width));
   const short *w_from[WL], *x_from[XL];
 #pragma unroll
   for (int j = 0; j < WL; ++j) {
     const int r = Core::w_row(wave, j) + grp;          // row in LDS
     const int n = OUT == GATED ? r / 16 * 8 + r % 8 : r;
     const bool up = OUT == GATED && r % 16 >= 8;
-    w_from[j] = p.w + (min(n0 + n, N - 1) + (up ? N : 0)) * p.w_row + Core::piece(r, lane);
+    w_from[j] = p.w + (min(n0 + n, n1 - 1) + (up ? N : 0)) * p.w_row + Core::piece(r, lane);
   }
 #pragma unroll
   for (int j = 0; j < XL; ++j) {
@@ -107,11 +109,10 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
 #pragma unroll
     for (int c = 0; c < CT; c += OUT == GATED ? 2 : 1) {
       const int m = (wm * MT + t) * 16 + col;
-      int tile = wc * CT + c, n = n0 + tile * 16 + grp * 4;
+      int n = n0 + (wc * CT + c) * 16 + grp * 4;
       float4v s = acc[c][t];
       if constexpr (OUT == GATED) {
-        tile += grp / 2;
-        n = n0 + tile * 8 + grp % 2 * 4;
+        n = n0 + (wc * CT + c + grp / 2) * 8 + grp % 2 * 4;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const auto both = __builtin_amdgcn_permlane32_swap(
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
         }
         if (CT == 1 && grp >= 2) continue;
       }
-      if (m >= M || n >= N || tile * 16 >= width) continue;    // N is a multiple of 4
+      if (m >= M || n >= n1) continue;     // n1 - n0 is a multiple of 4
       const int64_t o = ((int64_t)part * M + m) * N + n;
       if constexpr (OUT == F32) {
         *(float4v*)((float*)p.y + o) = s;
@@ -184,14 +185,16 @@ __global__ __launch_bounds__(256) void lay_weights_kernel(
   }
 }
 
-// Rows of w of a workgroup: as many rounds of the chip as by 128, each full, unless they
-// nearly are by 128 (16 rows, before / so: 8668 x 5640 gated 52.1 / 41.2 us, 17408 x 5120
-// 87.4 / 69.5, 25600 x 5120 99.4 / 94.0, 20480 x 2048 37.7 / 33.4; 36864 x 4096 plain 66.1
-// / 54.5, 41000 x 3072 54.2 / 48.5).
+// Rows of w of a workgroup where K is one part: as many rounds of the chip as by 128,
+// each full, unless they nearly are by 128 (16 rows, by 128 / so: 8668 x 5640 gated 52.1 /
+// 41.2 us, 17408 x 5120 87.4 / 69.0, 25600 x 5120 99.4 / 92.5, 20480 x 2048 37.7 / 33.4;
+// 36864 x 4096 plain 66.1 / 54.5, 41000 x 3072 54.2 / 48.5; by 64 / so: 1960 x 6160 gated
+// 27.5 / 17.6, 3072 x 1024 plain 5.8 / 4.8, 6720 x 6456 31.6 / 22.4).
 int even_width(int rows) {
   const int blocks = (rows + 127) / 128, slots = (blocks + ROUND - 1) / ROUND * ROUND;
   if (blocks * 8 >= slots * 7) return 128;
-  return ((rows + slots - 1) / slots + 15) / 16 * 16;
+  const int width = ((rows + slots - 1) / slots + UNIT - 1) / UNIT * UNIT;
+  return width < 16 ? 16 : width;
 }
 
 template <int RT, int BN, int KG, int OUT>
@@ -202,8 +205,7 @@ hipError_t go(Rows p, hipStream_t stream) {
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
   const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
-  p.width = BN;
-  if (p.parts == 1 && BN == 128) p.width = even_width(rows);
+  p.width = p.parts > 1 ? BN : even_width(rows);
   const int ch = OUT == GATED ? p.width / 2 : p.width;
   int groups = (p.N + ch - 1) / ch * p.parts;
   if (p.parts == 1) groups = (groups + 7) / 8 * 8;     // equal shares of the XCDs
@@ -213,17 +215,17 @@ hipError_t go(Rows p, hipStream_t stream) {
   return hipSuccess;
 }
 
-// 64 rows of w per workgroup where 128 leave half of the chip idle, K in two halves
-// where 64 do as well (4096 -> [2 x 1024], 16 rows: 24.2 us by 128, 16.7 by 64, 14.8
-// with halves, [2 x 4096] 26.3, 19.6, 17.2; 2048 -> [2 x 8192] 16.6, 14.4, 16.3), and
-// for parts of a few steps: two workgroups per compute unit, whose ends overlap (4096 ->
-// 4096, parts of 512: 7.4 us, 7.6 by 128, 30 rows 8.3, 8.5; parts of 896 up: 22.1, 21.9).
+// Up to 64 rows of w per workgroup have K in two halves, so that more is under way (16
+// rows, whole / halves: 10240 x 3072 15.5 us / 14.2, 3072 x 1024 5.7 / 4.8, 2760 x 8416
+// gated 32.6 / 25.4; 6344 x 1144 8.9 / 9.3). Parts of a few steps are taken by 64 too, two
+// workgroups per compute unit, whose ends overlap (4096 -> 4096, parts of 512: 7.4 us, 7.6
+// by 128, 30 rows 8.3, 8.5; parts of 896 up: 22.1, 21.9).
 template <int RT, int OUT>
 hipError_t go_width(const Rows& p, hipStream_t stream) {
   const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
-  if (p.parts == 1 && rows <= 64 * 128) return go<RT, 64, 2, OUT>(p, stream);
-  if (p.parts == 1 ? rows <= 128 * 128 : p.k_part <= 512)
-    return go<RT, 64, 1, OUT>(p, stream);
+  if (p.parts == 1 && rows <= 64 * ROUND) return go<RT, 64, 2, OUT>(p, stream);
+  if constexpr (OUT == F32)
+    if (p.parts > 1 && p.k_part <= 512) return go<RT, 64, 1, OUT>(p, stream);
   if constexpr (OUT == ACT) return hipErrorInvalidValue;
   else return go<RT, 128, 1, OUT>(p, stream);
 }
@@ -267,15 +269,17 @@ int lds_linear_rows_parts(int M, int N, int K) {
 }
 
 // The same where the sum of the parts is a launch of its own (3 to 5 us): one part of
-// short K, or of so many channels that it has few parts. Up to 64 rows, one part / parts
-// and their sum: 1024 -> 4096, 1 row 5.2 / 6.2, 64 rows 7.2 / 8.8; 2048 -> 8192 9.6 /
-// 11.8, 12.9 / 16.1, -> 2048 7.2 / 6.9, 10.5 / 9.2; 4096 -> 12576 23.6 / 26.0, -> 6144
-// 15.6 / 13.7.
+// short K, or of as many channels as K is long. Up to 64 rows, one part / parts and their
+// sum: 1536 -> 1024, 1 row 5.8 / 6.3, 50 rows 7.7 / 8.2; 2048 -> 2048 6.8 / 7.0, 9.3 / 9.8;
+// 3072 -> 3072 9.0 / 9.4, 12.6 / 12.1; 4096 -> 4096 11.6 / 11.8, 16.0 / 13.5, -> 6144 13.9
+// / 14.1, 18.0 / 16.3, -> 8192 16.7 / 17.8, 19.6 / 20.0, -> 2048 10.8 / 9.0; 6144 -> 8192
+// 21.8 / 23.3, 27.0 / 26.3; 8192 -> 8192 27.0 / 31.7, 33.8 / 34.7.
 int lds_linear_plain_parts(int M, int N, int K) {
   const int parts = lds_linear_rows_parts(M, N, K);
-  const bool one = M <= ROWS && N <= 128 * 128 &&
-                   (K <= 1024 || (K <= 2048 && N >= 4096) ||
-                    (K <= 8192 && N >= 96 * 128));
+  const bool one =
+      M <= ROWS && N <= 64 * ROUND &&
+      (K <= 1536 || (K <= 2048 && N >= 2048) ||
+       (K <= 8192 && N >= K && (M <= 32 || K <= 3072 || N >= 8192)));
   return one ? 1 : parts;
 }
 
@@ -297,19 +301,18 @@ int lds_linear_plain_parts(int M, int N, int K) {
 //     rounds it is 0.66 to 1.06 times (245 rows, 3584 -> [2 x 28744]: 132 / 118), by
 //     longer K 0.74 to 1.07 (15872 -> [2 x 15456]: 367 / 271);
 //     inside a 4-layer stack of about 180 rows the pass takes 790 / 835. Up to 64
-//     rows need not fill their round, for K from 1024 to 8192, of longer K with so many
+//     rows need not fill their round, for K from 256 to 4096, or to 8192 of so many
 //     channels that most compute units have some (16 rows, here / library with the
-//     activation: 1024 -> [2 x 1024] 5.8 / 14.1, 2048 -> [2 x 8192] 14.4 / 19.8, 64 rows
-//     18 / 21, 4096 -> [2 x 1024] 64 rows 20.0 / 16.4, [2 x 6144] 20.7 / 29.6, 8192 ->
-//     [2 x 4096] 33.7 / 31.6, [2 x 6144] 43 / 44).
+//     activation: 256 -> [2 x 2304] 4.0 / 12, 2048 -> [2 x 1024] 7.5 / 13, 4096 -> [2 x
+//     512] 11.3 / 17, 64 rows 16.1 / 16.9, 6144 -> [2 x 1536] 16.1 / 14.6, [2 x 2048] 16.9
+//     / 25, 8192 -> [2 x 2048] 21.5 / 18.6, [2 x 3072] 26.2 / 26.6).
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
 //     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
 //     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
 //     narrow ones up to 64 rows (4096 -> 1024: 64 rows 11 / 15, 96 rows
-//     13 / 12; 4096 -> 12576, 77 %: 64 rows 27 / 25), or of one part (lds_linear_plain_
-//     parts), of more than 16384 / 4 channels and K past 2048 up to 16 rows (2048 ->
-//     8192: 64 rows 12.9 / 13.5; 1024 -> 6144: 8.2 / 11.6; 4096 -> 12576: 16 rows
-//     24.2 / 27.6, 48 rows 26.2 / 25.5).
+//     13 / 12), or of one part (lds_linear_plain_parts; 2048 -> 8192: 50 rows 11.0 /
+//     13.5; 4096 -> 8192: 16 rows 16.8 / 16.4, 50 rows 19.6 / 18.6, -> 10240 19.9 / 26.0,
+//     22.1 / 27.5, -> 12576 23.4 / 28.4, 26.6 / 26.7; 8192 -> 8192 27.1 / 30.3).
 //   more than 16384 rows of w, in even rounds (even_width): up to 64 rows, K from 512 to
 //     10240. Over 76 sizes of 16384 to 130000 rows of w, gated and plain, 4 to 64 rows of
 //     x, 1.3 times as fast at the median; slower by 3 and 6 % at two (51200 x 5120 and
@@ -321,15 +324,15 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
   if (M <= ROWS && (gated ? 2 : 1) * N > 128 * 128 && K >= 512 && K <= 10240) return 1;
-  if (gated && M <= ROWS && groups <= 256 && K >= 1024 &&
-      (K <= 2048 || (K <= 4096 && groups >= 72) || (K <= 8192 && groups >= 96)))
+  if (gated && M <= ROWS && groups <= 256 && K >= 256 &&
+      (K <= 4096 || (K <= 6144 && groups >= 32) || (K <= 8192 && groups >= 48)))
     return 1;
   if (gated)
     return full && (M <= 192 || (groups <= 256 && K >= 1024 && K <= 8192 &&
                                  K % KS == 0));
   if (N > 128 * 128) return full && M <= 128;
   if (full) return M <= 64 || K >= 4096;
-  return M <= 64 && (N <= 4096 || (n == 1 && (K <= 2048 || M <= 16)));
+  return M <= ROWS && (N <= 4096 || n == 1);
 }
 
 // y [n] = the sum of part [parts, n], or (act >= 0) its activation; 16-byte aligned, n
