@@ -85,22 +85,26 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
   const int wc = wave % WC, wm = wave / WC;      // its channels, its rows
 
   if constexpr (KG > 1) {                  // to the sums of the first group
-    static_assert(KG == 2 && CT * MT * NW * 1024 <= Core::RINGS, "");
+    constexpr int ONE = CT * MT * NW * WAVE;
+    static_assert((KG - 1) * ONE * 16 <= KG * Core::RINGS, "");
     float4v* other = (float4v*)lds;
     __syncthreads();                       // the rings are no longer read
 #pragma unroll
     for (int c = 0; c < CT; ++c)
 #pragma unroll
       for (int t = 0; t < MT; ++t)
-        if (group == 1)
-          other[((c * MT + t) * NW + wave) * WAVE + lane] = acc[c][t];
+        if (group > 0)
+          other[(group - 1) * ONE + ((c * MT + t) * NW + wave) * WAVE + lane] =
+              acc[c][t];
     __syncthreads();
-    if (group == 1) return;
+    if (group > 0) return;
 #pragma unroll
-    for (int c = 0; c < CT; ++c)
+    for (int i = 0; i < KG - 1; ++i)
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
-        acc[c][t] += other[((c * MT + t) * NW + wave) * WAVE + lane];
+      for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+          acc[c][t] += other[i * ONE + ((c * MT + t) * NW + wave) * WAVE + lane];
   }
   // lane: row `col` of a tile, channels 4 grp ..; GATED: gate with the lower half of the
   // lanes, up with the other, and of two tiles each half takes one
@@ -215,15 +219,23 @@ hipError_t go(Rows p, hipStream_t stream) {
   return hipSuccess;
 }
 
-// Up to 64 rows of w per workgroup have K in two halves, so that more is under way (16
-// rows, whole / halves: 10240 x 3072 15.5 us / 14.2, 3072 x 1024 5.7 / 4.8, 2760 x 8416
-// gated 32.6 / 25.4; 6344 x 1144 8.9 / 9.3). Parts of a few steps are taken by 64 too, two
-// workgroups per compute unit, whose ends overlap (4096 -> 4096, parts of 512: 7.4 us, 7.6
-// by 128, 30 rows 8.3, 8.5; parts of 896 up: 22.1, 21.9).
+// Where few rows of w come to a workgroup K is shared out inside it, as far as the rings
+// fit, so that more is under way (1, 16 and 50 rows, in us: K whole by 64 rows of w; in
+// halves by 64; as it is here):
+//   4096 -> 1024           12.8, 13.6, 18.4    10.6, 10.8, 15.3     6.9,  7.6, 12.8
+//   4096 -> 6144           16.4, 17.0, 21      14.0, 14.3, 18.1    11.9, 12.5, 16.6
+//   8192 -> [2 x 2048]     30.1, 30.6, 42      21.7, 21.4, 30.4    15.2, 15.9, 25.2
+//   4096 -> 10240          21.0, 21.2, 23.9    19.7, 19.7, 22.4    19.2, 19.6, 23.9
+// Parts of a few steps are taken by 64 too, two workgroups per compute unit, whose ends
+// overlap (4096 -> 4096, parts of 512: 7.4 us, 7.6 by 128, 30 rows 8.3, 8.5; parts of 896
+// up: 22.1, 21.9).
 template <int RT, int OUT>
 hipError_t go_width(const Rows& p, hipStream_t stream) {
   const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
-  if (p.parts == 1 && rows <= 64 * ROUND) return go<RT, 64, 2, OUT>(p, stream);
+  if (p.parts == 1 && rows <= 32 * ROUND)
+    return go<RT, 32, RT == 1 ? 4 : 2, OUT>(p, stream);
+  if (p.parts == 1 && rows <= 64 * ROUND)
+    return go<RT, 64, RT == 4 ? 1 : 2, OUT>(p, stream);
   if constexpr (OUT == F32)
     if (p.parts > 1 && p.k_part <= 512) return go<RT, 64, 1, OUT>(p, stream);
   if constexpr (OUT == ACT) return hipErrorInvalidValue;

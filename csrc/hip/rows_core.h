@@ -37,9 +37,8 @@ template <int RT, int BN>
 struct RowsCore {
   static constexpr int NW = BN / 16, WM = RT == 1 ? 1 : 2, WC = NW / WM;
   static constexpr int CT = BN / 16 / WC, MT = RT / WM;
-  // RING steps of w, two of x, whose lines are near
   static constexpr int W_STEP = BN * ROW, X_STEP = 16 * RT * ROW;
-  static constexpr int RINGS = RING * W_STEP + 2 * X_STEP;
+  static constexpr int RINGS = RING * (W_STEP + X_STEP);
   // loads of a wave, 4 rows each (where x has fewer the last one is repeated)
   static constexpr int WL = BN / 4 / NW, XL = (4 * RT + NW - 1) / NW;
 
@@ -80,18 +79,15 @@ struct RowsCore {
           (gmem*)(in ? from + k : (const short*)&zeros), (smem*)(to + q * 1024),
           16, 0, 0);
     };
-    auto issue_w = [&](int s, int buf) {
-      if (!some) return;
+    auto issue = [&](int s, int buf) {
       const int k = k_of(s);
+      if (some)
 #pragma unroll
-      for (int j = 0; j < WL; ++j)
-        load(w_from[j], w_ring + buf * W_STEP, wave * WL + j, k);
-    };
-    auto issue_x = [&](int s) {
-      const int k = k_of(s);
+        for (int j = 0; j < WL; ++j)
+          load(w_from[j], w_ring + buf * W_STEP, wave * WL + j, k);
 #pragma unroll
       for (int j = 0; j < XL; ++j)
-        load(x_from[j], x_ring + s % 2 * X_STEP, x_row(wave, j) / 4, k);
+        load(x_from[j], x_ring + buf * X_STEP, x_row(wave, j) / 4, k);
     };
 
 #pragma unroll
@@ -103,10 +99,10 @@ struct RowsCore {
       bf16x8 w[CT], x[MT];
     };
     const int w_at = (wc * 16 * CT + col) * ROW, x_at = (wm * 16 * MT + col) * ROW;
-    auto read = [&](Operands& o, int buf, int s, int q) {       // q: 32 of K
+    auto read = [&](Operands& o, int buf, int q) {      // q: 32 of K
       const int at = ((q * 4 + grp) ^ col) * 16;
       const char* w = w_ring + buf * W_STEP + w_at + at;
-      const char* x = x_ring + s % 2 * X_STEP + x_at + at;
+      const char* x = x_ring + buf * X_STEP + x_at + at;
 #pragma unroll
       for (int c = 0; c < CT; ++c)
         o.w[c] = *(const bf16x8*)(w + c * 16 * ROW);
@@ -124,44 +120,43 @@ struct RowsCore {
               o.w[c], o.x[t], acc[c][t], 0, 0, 0);
       __builtin_amdgcn_sched_barrier(0);
     };
-    // step s has landed, and so it has for the other waves, when only w of the next one
-    // is under way
+    // step s has landed, and so it has for the other waves, when only the next one is
+    // under way
     auto landed = [&](int s) {
-      if (some && s + 1 < steps)
-        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(WL) : "memory");
-      else
+      if (s + 1 == steps)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      else if (some)
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(WL + XL) : "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(%0)" ::"i"(XL) : "memory");
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
     };
 
     // Operands are read 32 of K ahead of their products. At the barrier ahead of the
-    // last of step s all of its operands are in registers: its places take w of step
-    // s + RING and x of step s + 2.
+    // last of step s all of its operands are in registers: its places take step s +
+    // RING.
     static_assert(RING == 3, "");
-    issue_w(0, 0);
-    issue_x(0);
-    if (1 < steps) issue_w(1, 1);
+    issue(0, 0);
+    if (1 < steps) issue(1, 1);
     Operands o0, o1;
     landed(0);
-    if (1 < steps) issue_x(1);
-    if (2 < steps) issue_w(2, 2);
-    read(o0, 0, 0, 0);
+    if (2 < steps) issue(2, 2);
+    read(o0, 0, 0);
     int buf = 0;
     for (int s = 0; s < steps; ++s) {
-      read(o1, buf, s, 1);
+      read(o1, buf, 1);
       multiply(o0);
-      read(o0, buf, s, 2);
+      read(o0, buf, 2);
       multiply(o1);
-      read(o1, buf, s, 3);
+      read(o1, buf, 3);
       multiply(o0);
       if (s + 1 < steps) {
         landed(s + 1);
-        if (s + 2 < steps) issue_x(s + 2);
-        if (s + RING < steps) issue_w(s + RING, buf);
+        if (s + RING < steps) issue(s + RING, buf);
         buf = buf + 1 == RING ? 0 : buf + 1;
-        read(o0, buf, s + 1, 0);
+        read(o0, buf, 0);
       }
       multiply(o1);
     }
