@@ -2,8 +2,10 @@
 // (bf16). A tile is 128 rows of (query, head): all heads of a key/value head
 // share its tiles of keys. Keys and values come from
 //   pages        grouped heads: cache rows [key | value], found through the
-//                block table a tile ahead (block sizes that are powers of two
-//                without divisions, which took as long as the scores)
+//                block table a tile ahead. Where the rows of a wave's load lie in
+//                one page its address is a scalar's work; else each lane finds its
+//                row (block sizes that are powers of two without divisions, which
+//                took as long as the scores)
 //   context rows latent attention: keys and values expanded from the latents
 //                of everything a portion may see, the rotated key part shared
 //                by all heads; a sequence's context row 0 sits at ctx.pos0
@@ -16,10 +18,12 @@
 // run from the last to the first: under the causal mask the last of a sequence has
 // the most keys.
 //
-// 7800 rows of 7 prompts behind 100 tokens, 32 heads of 128 on 8 key heads: 190 us
-// (232 with one tile in LDS, divisions and operands of K waited for one by one; 231
-// in tiles of 32 keys); 7750 rows of 8 prompts, 32 heads of 192 and 128: 171 us (226;
-// 253 in tiles of 64 keys, whose scores do not fit the registers beside a tile).
+// 7800 rows of 7 prompts behind 100 tokens, 32 heads of 128 on 8 key heads: 148 us (196
+// with an address worked out per lane and row, 232 with one tile in LDS, divisions and
+// operands of K waited for one by one; 231 in tiles of 32 keys); one prompt of 7100 rows
+// 470 (620); 7750 rows of 8 prompts, 32 heads of 192 and 128: 157 us (178 with 64-bit
+// products per load; 253 in tiles of 64 keys, whose scores do not fit the registers beside
+// a tile).
 #include "../flash_core.h"
 #include "elem.h"
 
@@ -56,10 +60,14 @@ constexpr int tile_of(int DK, int DV) {       // in LDS (shorts)
   return keys_of(DK, DV) * (DK + 8 + DV + 32);
 }
 
+// where rows lie: context rows, pages, pages that hold the rows of a wave's load whole
+enum Rows { CONTEXT, PAGES, WHOLE };
+
 // grid (key/value heads, tiles)
-template <int DK, int DV, bool PAGED>
+template <int DK, int DV, int ROWS>
 __global__ __launch_bounds__(NT, DK + DV > 320 ? 1 : 2)
 void context_prefill_kernel(const Prefill a_) {
+  constexpr bool PAGED = ROWS != CONTEXT;
   constexpr int KS = DK + 8, VS = DV + 32;      // row strides in LDS (shorts)
   constexpr int KB = keys_of(DK, DV);
   constexpr int NK = DK * KB / 8 / NT, NV = DV * KB / 8 / NT;   // loads
@@ -121,13 +129,16 @@ void context_prefill_kernel(const Prefill a_) {
   // A tile goes through registers: rows past the last key that is seen repeat it
   // (they are masked), channels past the end are 0.
   short8 kn[NK], vn[NV];
-  int kp[PAGED ? NK : 1], vp[PAGED && DK != DV ? NV : 1];   // pages of a tile
+  // pages of a tile; WHOLE: those from its first key's on, one per lane
+  int kp[ROWS == PAGES ? NK : 1], vp[ROWS == PAGES && DK != DV ? NV : 1];
   const int shift = a_.shift, page_mask = bs - 1;
   auto row_of = [&](int t0, int i, int per) {
     return min(t0 + (tid + i * NT) / per, hi_wg - 1);
   };
   auto find = [&](int t0) {
-    if constexpr (PAGED) {
+    if constexpr (ROWS == WHOLE)
+      kp[0] = bt[min((t0 >> shift) + lane, (hi_wg - 1) >> shift)];
+    if constexpr (ROWS == PAGES) {
 #pragma unroll
       for (int i = 0; i < NK; ++i) {
         const int t = row_of(t0, i, DK / 8);
@@ -146,18 +157,51 @@ void context_prefill_kernel(const Prefill a_) {
     const uint32_t at = (shift < 0 ? t % bs : t & page_mask) * (D + V);
     return pages + ((uint64_t)(uint32_t)page * (uint64_t)a_.page + at);
   };
+  // WHOLE: the row of load i, in the page of the wave's first one
+  constexpr int PER = WAVE * 8 / DK;            // rows of a wave's load
+  const int first_row = __builtin_amdgcn_readfirstlane(wave) * PER;
+  auto whole_row = [&](int t0, int i) {
+    const int t = t0 + first_row + i * NW * PER, last = hi_wg - 1;
+    const int at = (min(t, last) >> shift) - (t0 >> shift);
+    const uint32_t page = __builtin_amdgcn_readlane(kp[0], max(at, 0));
+    const short* from = pages + (uint64_t)page * (uint32_t)a_.page;
+    return from + (uint32_t)((min(t + lane / (DK / 8), last) & page_mask) * (DK + DV) +
+                             lane % (DK / 8) * 8);
+  };
+  // CONTEXT: row 0 of each load's channels and the stride of its rows
+  constexpr bool CTX = ROWS == CONTEXT;
+  const short *k_from[CTX ? NK : 1], *v_from[CTX ? NV : 1];
+  uint32_t k_tok[CTX ? NK : 1];
+  if constexpr (CTX) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int d = (tid + i * NT) % (DK / 8) * 8;
+      k_from[i] = d < D ? a_.ka + ctx0 * a_.ka_tok + kvh * a_.ka_head + d
+                        : a_.kb + ctx0 * a_.kb_tok + (d - D);
+      k_tok[i] = d < D ? a_.ka_tok : a_.kb_tok;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      v_from[i] = a_.v + ctx0 * a_.v_tok + kvh * a_.v_head +
+                  (tid + i * NT) % (DV / 8) * 8;
+  }
   // load i of the keys, then of the values
   auto fetch = [&](int t0, int i) {
+    if constexpr (ROWS == WHOLE) {
+      static_assert(DK == DV, "");
+      if (i < NK) kn[i] = *(const short8*)whole_row(t0, i);
+      else vn[i - NK] = *(const short8*)(whole_row(t0, i - NK) + DK);
+      return;
+    }
     if (i < NK) {
       const int t = row_of(t0, i, DK / 8), d = (tid + i * NT) % (DK / 8) * 8;
       kn[i] = (short8){0, 0, 0, 0, 0, 0, 0, 0};
       if (d < QD) {
         if constexpr (PAGED)
-          kn[i] = *(const short8*)(page_row(kp[PAGED ? i : 0], t) + d);
+          kn[i] = *(const short8*)(page_row(kp[ROWS == PAGES ? i : 0], t) + d);
         else
-          kn[i] = *(const short8*)(
-              d < D ? a_.ka + (ctx0 + t) * a_.ka_tok + kvh * a_.ka_head + d
-                    : a_.kb + (ctx0 + t) * a_.kb_tok + (d - D));
+          kn[i] = *(const short8*)(k_from[CTX ? i : 0] +
+                                   (uint64_t)(uint32_t)t * k_tok[CTX ? i : 0]);
       }
     } else {
       i -= NK;
@@ -166,11 +210,12 @@ void context_prefill_kernel(const Prefill a_) {
       if (d < V) {
         if constexpr (PAGED)
           vn[i] = *(const short8*)(
-              page_row(DK == DV ? kp[PAGED ? i : 0]
-                                : vp[PAGED && DK != DV ? i : 0], t) + D + d);
+              page_row(DK == DV ? kp[ROWS == PAGES ? i : 0]
+                                : vp[ROWS == PAGES && DK != DV ? i : 0], t) +
+              D + d);
         else
-          vn[i] = *(const short8*)(a_.v + (ctx0 + t) * a_.v_tok +
-                                   kvh * a_.v_head + d);
+          vn[i] = *(const short8*)(v_from[CTX ? i : 0] +
+                                   (uint64_t)(uint32_t)t * (uint32_t)a_.v_tok);
       }
     }
   };
@@ -261,11 +306,11 @@ void context_prefill_kernel(const Prefill a_) {
   }
 }
 
-template <int DK, int DV, bool PAGED>
+template <int DK, int DV, int ROWS>
 hipError_t launch(const Prefill& a, int kv_heads, int n_tiles,
                   hipStream_t stream) {
   const int lds = 2 * tile_of(DK, DV) * (int)sizeof(short);
-  auto fn = context_prefill_kernel<DK, DV, PAGED>;
+  auto fn = context_prefill_kernel<DK, DV, ROWS>;
   hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   if (e != hipSuccess) return e;
@@ -316,8 +361,8 @@ hipError_t lds_latent_prefill(const void* q, const void* kv, const void* lat,
   a.scale = scale;
   const int qd = D + rot;
 #define GO(DK)                                                                \
-  return V <= 64 ? launch<DK, 64, false>(a, H, n_tiles, stream)               \
-                 : launch<DK, 128, false>(a, H, n_tiles, stream)
+  return V <= 64 ? launch<DK, 64, CONTEXT>(a, H, n_tiles, stream)               \
+                 : launch<DK, 128, CONTEXT>(a, H, n_tiles, stream)
   if (qd <= 64) GO(64);
   if (qd <= 96) GO(96);
   if (qd <= 128) GO(128);
@@ -362,10 +407,16 @@ hipError_t lds_grouped_prefill(const void* q, int64_t q_stride,
   a.scale = scale;
   a.has_sink = has_sink;
   a.sink = sink * LOG2E;
+  // rows of a load of 1 KB in one page: 8 of 64, 4 of 128, 2 of 256
+  if (D == V && a.shift >= 0 && bs * D >= 512 && a.page < 1ll << 32) {
+    if (D == 64) return launch<64, 64, WHOLE>(a, G, n_tiles, stream);
+    if (D == 128) return launch<128, 128, WHOLE>(a, G, n_tiles, stream);
+    if (D == 256) return launch<256, 256, WHOLE>(a, G, n_tiles, stream);
+  }
 #define GO(DK)                                                                \
-  return V <= 64    ? launch<DK, 64, true>(a, G, n_tiles, stream)             \
-         : V <= 128 ? launch<DK, 128, true>(a, G, n_tiles, stream)            \
-                    : launch<DK, 256, true>(a, G, n_tiles, stream)
+  return V <= 64    ? launch<DK, 64, PAGES>(a, G, n_tiles, stream)             \
+         : V <= 128 ? launch<DK, 128, PAGES>(a, G, n_tiles, stream)            \
+                    : launch<DK, 256, PAGES>(a, G, n_tiles, stream)
   if (D <= 64) GO(64);
   if (D <= 128) GO(128);
   if (D <= 192) GO(192);

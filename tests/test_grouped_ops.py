@@ -409,6 +409,15 @@ def test_prefill_in_other_pages(D, V, bs, monkeypatch):
 
 
 @GPU
+@pytest.mark.parametrize("D,bs", [(64, 8), (64, 4), (128, 4), (128, 2), (256, 2),
+                                  (256, 1), (256, 128)])
+def test_prefill_where_a_load_fits_a_page(D, bs, monkeypatch):
+    """The smallest pages that hold the rows of a load whole, and smaller ones."""
+    test_prefill_in_other_pages(D, D, bs, monkeypatch)
+
+
+
+@GPU
 def test_forms_agree_at_a_large_size():
     """The tiled products against the plain kernel."""
     dev, E, K, F, T, top = "cuda:0", 9, 512, 448, 1500, 3
