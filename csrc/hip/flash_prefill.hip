@@ -15,12 +15,21 @@
 //   grid = row tiles (128 "virtual rows" = (position, q-head-in-group)
 //          pairs, v = p*QPG + g), last first, times kv heads (fastest)
 //   workgroup = 4 waves; wave w owns v-rows [vrow0+32w, vrow0+32w+32)
-//   KV loop: 64-token tiles in LDS (XOR-swizzled rows), the next tile waits
-//            in registers
+//   KV loop: 64-token tiles in LDS (XOR-swizzled rows), two of them; a third is on
+//            its way in registers, and its loads and LDS writes stand between the
+//            matrix instructions. Where the rows of a wave's load lie in one page
+//            (WHOLE) the page's address is scalar work.
 //
 // GQA: q-heads of one group share the kv_head's K/V tiles; causal masking
 // is per-lane compares (kv <= prior + p), no divergence.
+//
+// Bound by vector work, of the softmax and of widening and moving tiles. 8-bit cache,
+// groups of 4, 8 key heads; before: one tile in LDS, a division and 64-bit products per
+// lane and row: one prompt of 7000 tokens 492 us (586), 8 of 1000 133 us (155), 4 of 1000
+// behind 1000 164 us (200), 150 behind 1000 44 us (55).
 #include "flash_core.h"
+
+#include <type_traits>
 
 namespace {
 
@@ -54,7 +63,7 @@ template <> struct Piece<unsigned char> {
   }
 };
 
-template <int QPG, typename CT>
+template <int QPG, typename CT, bool WHOLE>
 __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
     const short* __restrict__ q,        // [T, QH, D]
     const CT* __restrict__ k_cache,     // [NB, KVH, BS, D] bf16|fp8
@@ -63,7 +72,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
     const int32_t* __restrict__ seq_meta,      // [S, 3] start, chunk, prior
     const int32_t* __restrict__ tiles,         // [n_tiles, 2] seq, vrow0
     short* __restrict__ out,                   // [T, QH, D]
-    int kvh, int bs, int max_blocks, float scale) {
+    int kvh, int bs, int shift, int max_blocks, float scale) {
   const int kh = blockIdx.x % kvh;
   const int tile = (gridDim.x - 1 - blockIdx.x) / kvh;
   const int seq = tiles[2 * tile];
@@ -75,8 +84,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
   const int n_q_heads = kvh * QPG;
   const int32_t* bt = block_tables + (int64_t)seq * max_blocks;
 
-  __shared__ __align__(16) short k_lds[KVBLK * D];   // swizzled rows
-  __shared__ __align__(16) short v_lds[KVBLK * D];
+  __shared__ __align__(16) short lds[2][2][KVBLK * D];   // keys, values: swizzled rows
   static_assert(KVBLK * 16 % (NW * WAVE) == 0, "staging divides evenly");
 
   const int tid = threadIdx.x;
@@ -114,44 +122,76 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
   const int kv_end_wg = prior + last_wg + 1;
   const int kv_end_w = w0 < rows ? prior + last_w + 1 : 0;
 
+  // A tile goes through registers: rows past the last key that is seen repeat it (they
+  // are masked).
   typedef typename Piece<CT>::Raw Raw;
-  constexpr int REPS = KVBLK * 16 / (NW * WAVE);
+  constexpr int REPS = KVBLK * 16 / (NW * WAVE), PER = WAVE / 16;
+  const int last = kv_end_wg - 1;
+  const int first_row = __builtin_amdgcn_readfirstlane(wave) * PER;
   Raw kn[REPS], vn[REPS];
-  auto fetch = [&](int tile0) {
+  int pages[WHOLE ? 1 : REPS];   // of a tile; WHOLE: those from its first key's on, by lane
+  auto row_of = [&](int tile0, int r) {
+    return min(tile0 + r * NW * PER + first_row + lane / 16, last);
+  };
+  auto find = [&](int tile0) {
+    if constexpr (WHOLE) {
+      pages[0] = bt[min((tile0 >> shift) + lane, last >> shift)];
+    } else {
 #pragma unroll
-    for (int r = 0; r < REPS; ++r) {
-      const int ch = tid + r * (NW * WAVE);
-      const int t = tile0 + ch / 16, c = ch % 16 * 8;
-      kn[r] = vn[r] = Raw{};
-      if (t < kv_end_wg) {
-        const int pg = t / bs;
-        const int64_t base =
-            (((int64_t)bt[pg] * kvh + kh) * bs + (t - pg * bs)) * D + c;
-        kn[r] = *(const Raw*)(k_cache + base);
-        vn[r] = *(const Raw*)(v_cache + base);
-      }
+      for (int r = 0; r < REPS; ++r) pages[r] = bt[row_of(tile0, r) / bs];
     }
+  };
+  // load i of the keys, then of the values
+  auto fetch = [&](int tile0, int i) {
+    const int r = i % REPS, t = row_of(tile0, r), c = lane % 16 * 8;
+    const CT* from = i < REPS ? k_cache : v_cache;
+    if constexpr (WHOLE) {
+      const int first = min(tile0 + r * NW * PER + first_row, last);
+      const uint32_t page = __builtin_amdgcn_readlane(
+          pages[0], max((first >> shift) - (tile0 >> shift), 0));
+      from += ((uint64_t)page * kvh + kh) * (bs * D) +
+              (uint32_t)((t & (bs - 1)) * D + c);
+    } else {
+      from += (((int64_t)pages[WHOLE ? 0 : r] * kvh + kh) * bs + t % bs) * D + c;
+    }
+    (i < REPS ? kn : vn)[r] = *(const Raw*)from;
+  };
+  auto put = [&](int buf, int i) {
+    const int r = i % REPS, row = r * NW * PER + wave * PER + lane / 16;
+    const int at = row * 256 + (lane % 16 * 16 ^ swizzle(row));
+    *(short8*)((char*)lds[buf][i / REPS] + at) =
+        Piece<CT>::wide((i < REPS ? kn : vn)[r]);
   };
   const int i16 = lane % 16;
   const int v_col = (16 * ((lane & 31) >> 4) + (i16 % 4) * 4) * 2;
-  fetch(0);
-  for (int tile0 = 0; tile0 < kv_end_wg; tile0 += KVBLK) {
-    __syncthreads();  // previous tile's reads complete before overwrite
+  find(0);
 #pragma unroll
-    for (int r = 0; r < REPS; ++r) {
-      const int ch = tid + r * (NW * WAVE), row = ch / 16;
-      const int at = row * 256 + (ch % 16 * 16 ^ swizzle(row));
-      *(short8*)((char*)k_lds + at) = Piece<CT>::wide(kn[r]);
-      *(short8*)((char*)v_lds + at) = Piece<CT>::wide(vn[r]);
-    }
-    __syncthreads();
-    if (tile0 + KVBLK < kv_end_wg) fetch(tile0 + KVBLK);
-#pragma unroll 1
+  for (int i = 0; i < 2 * REPS; ++i) fetch(0, i);
+#pragma unroll
+  for (int i = 0; i < 2 * REPS; ++i) put(0, i);
+  if (KVBLK < kv_end_wg) {
+    find(KVBLK);
+#pragma unroll
+    for (int i = 0; i < 2 * REPS; ++i) fetch(KVBLK, i);
+    find(2 * KVBLK);
+  }
+  auto step = [&](int tile0, auto buf_) {
+    constexpr int buf = decltype(buf_)::value;
+    lds_barrier();
+#pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int sub0 = tile0 + 32 * half;
-      if (sub0 >= kv_end_w) break;          // beyond this wave's horizon
-      const char* kb = (const char*)k_lds + 32 * half * 256;
-      const char* vb = (const char*)v_lds + 32 * half * 256;
+      auto next = [&](int i) {
+        put(buf ^ 1, half * REPS + i);
+        fetch(tile0 + 2 * KVBLK, half * REPS + i);
+      };
+      if (sub0 >= kv_end_w) {               // beyond this wave's horizon
+#pragma unroll
+        for (int i = 0; i < REPS; ++i) next(i);
+        continue;
+      }
+      const char* kb = (const char*)lds[buf][0] + 32 * half * 256;
+      const char* vb = (const char*)lds[buf][1] + 32 * half * 256;
       attend<D / 16, D / 32, 1, false>(
           [&](int, int kk) {
             return *(const bf16x8*)(kb + qcol * 256 +
@@ -161,8 +201,17 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
             return vb + row * 256 + ((t * 64 + v_col) ^ swizzle(row));
           },
           qf, scale_log2, sub0 + 31 <= prior + first_w, 0, prior + p - sub0,
-          st, acc, [](int) {});
+          st, acc, [&](int m) {
+            static_assert(D / 16 == 2 * REPS, "");
+            if (m % 2 == 0) next(m / 2);
+          });
     }
+    find(tile0 + 3 * KVBLK);
+  };
+  for (int tile0 = 0; tile0 < kv_end_wg; tile0 += 2 * KVBLK) {
+    step(tile0, std::integral_constant<int, 0>{});
+    if (tile0 + KVBLK < kv_end_wg)
+      step(tile0 + KVBLK, std::integral_constant<int, 1>{});
   }
   st.l = st.join();
 
@@ -195,11 +244,19 @@ hipError_t lds_flash_prefill(const void* q, const void* k_cache,
     return hipErrorInvalidValue;
   const int qpg = n_q_heads / kvh;
   dim3 grid((uint32_t)n_tiles * kvh), block(NW * WAVE);
-#define LAUNCH_CT(QPG, CT)                                                    \
-  hipLaunchKernelGGL((flash_prefill_kernel<QPG, CT>), grid, block, 0, stream, \
+  const int shift = bs & bs - 1 ? -1 : __builtin_ctz(bs);
+#define LAUNCH_ROWS(QPG, CT, WHOLE)                                           \
+  hipLaunchKernelGGL((flash_prefill_kernel<QPG, CT, WHOLE>), grid, block, 0,  \
+                     stream,                                                  \
                      (const short*)q, (const CT*)k_cache,                     \
                      (const CT*)v_cache, block_tables, seq_meta, tiles,       \
-                     (short*)out, kvh, bs, max_blocks, scale)
+                     (short*)out, kvh, bs, shift, max_blocks, scale)
+  // a wave's load has 4 rows
+#define LAUNCH_CT(QPG, CT)                                                    \
+  do {                                                                        \
+    if (shift >= 2) LAUNCH_ROWS(QPG, CT, true);                               \
+    else LAUNCH_ROWS(QPG, CT, false);                                         \
+  } while (0)
 #define LAUNCH(QPG)                                                           \
   do {                                                                        \
     if (kv_fp8) LAUNCH_CT(QPG, unsigned char);                                \
@@ -213,6 +270,8 @@ hipError_t lds_flash_prefill(const void* q, const void* k_cache,
     default: return hipErrorInvalidValue;
   }
 #undef LAUNCH
+#undef LAUNCH_CT
+#undef LAUNCH_ROWS
   HIP_CHECK_LAST();
   return hipSuccess;
 }

@@ -155,3 +155,11 @@ struct PartSums {
       return e_;                                                       \
     }                                                                  \
   } while (0)
+
+// Workgroup barrier that orders LDS accesses only: global loads issued before
+// it stay in flight across it (__syncthreads waits for them)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}

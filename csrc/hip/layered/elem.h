@@ -87,14 +87,6 @@ __device__ __forceinline__ float softplus_f(float x) {
   return fmaf(2.f * s, p, fmaxf(x, 0.f));
 }
 
-// Workgroup barrier that orders LDS accesses only: global loads issued before
-// it stay in flight across it (__syncthreads waits for them)
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // sum over a block of NW waves; every thread gets it. Two calls in a row
 // need different scratch (NW floats each).
 template <int NW>

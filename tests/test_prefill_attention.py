@@ -101,6 +101,19 @@ def test_pages_in_fp8(seqs, qpg, kvh, bs):
     _close(ext.flash_prefill(*args), want)
 
 
+@pytest.mark.parametrize("bs", [1, 2, 4, 8, 64, 256])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_sizes_of_pages_through_registers(bs, fp8):
+    """As above; contexts of one to four tiles of keys and one key more or less, waves
+    that have seen all of theirs while others have not."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case([(65, 0), (40, 21), (3, 125), (30, 34), (1, 256), (128, 0),
+                        (191, 1)], 4, 2, bs, fp8, D ** -0.5)
+    wide = torch.zeros(7, 1025, dtype=torch.int32, device="cuda")
+    wide[:, :args[3].shape[1]] = args[3]
+    _close(ext.flash_prefill(*args[:3], wide, *args[4:]), want)
+
+
 @pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("keys", [0, 1, 2])
 @pytest.mark.parametrize("scale", [-0.1, 0.0, 2.0])
