@@ -10,7 +10,8 @@ int lds_grouped_decode_parts(int, int, int, int, int, int);
 hipError_t lds_grouped_decode(const void*, int64_t, const void*,
                               const int32_t*, const int32_t*, const int32_t*,
                               void*, float*, float*, int, int, int, int, int,
-                              int, int, int, float, int, float, hipStream_t);
+                              int, int, int, int, float, int, float,
+                              hipStream_t);
 int lds_grouped_prefill_ok(int, int, int, int64_t);
 hipError_t lds_grouped_prefill(const void*, int64_t, const void*,
                                const int32_t*, int, int, const int32_t*,
@@ -123,7 +124,8 @@ void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                 ip(positions), ip(row_seq), ip(block_tables), out.data_ptr(),
                 parts > 1 ? fp(po) : nullptr, parts > 1 ? fp(ml) : nullptr,
                 (int)n, (int)H, (int)s.G, (int)D, (int)s.V,
-                (int)block_tables.size(1), (int)s.bs, parts, (float)scale,
+                (int)block_tables.size(1), (int)s.bs, (int)max_ctx, parts,
+                (float)scale,
                 sink.has_value(), (float)sink.value_or(0.), cur_stream()),
             "grouped_decode");
 }

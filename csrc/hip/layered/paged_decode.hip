@@ -3,7 +3,8 @@
 // A cached token is one row of W elements per key/value head; its keys are the
 // first SW columns, its values R columns from v0 on. Two layouts use it: the
 // absorbed form of latent attention (one head for all queries, the latent
-// being key part and value at once) and grouped heads (rows [key | value]).
+// being key part and value at once) and grouped heads (rows [key | value]) of
+// sizes that decode_core.h does not take.
 //
 // One workgroup per (row, 16 or 32 query heads of one key/value head, part of
 // the context), 4 waves per 16 heads. Tiles of 64 tokens pass through LDS
@@ -12,6 +13,7 @@
 // O' = V' P' for all heads (a wave owns every NW-th 16 value channels; the
 // transposing LDS reads give V'). Memory-bound: the matrix work per token is
 // small beside its bytes.
+#include "../decode_core.h"
 #include "elem.h"
 
 namespace {
@@ -393,9 +395,25 @@ int lds_grouped_decode_ok(int D, int V, int64_t q_stride) {
          padded_width(D, D + V, D, V) <= 512;
 }
 
+// Heads of 128 in groups of up to 8 take decode_core.h's kernel, which neither stages
+// tiles in LDS nor waits at barriers for each of them: 60 rows of 1200 tokens, groups of
+// 4, 8 key heads 58.8 us (64.5), 32 rows 33.9 (37.9 in 3 parts), 8 rows 17.6 (19.3), 200
+// rows 185 (199), 60 of 300 18.2 (20.1), one of 777 9.3 (10.9).
+static bool in_core(int D, int V, int rep) { return D == 128 && V == 128 && rep <= 8; }
+
 int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx) {
   Decode d{};
   d.rep = H / G;
+  if (in_core(D, V, d.rep)) {
+    // As for the uniform decoder (decode_parts in ops/dispatch.py, where it was measured):
+    // one part takes 3 us and as long as a workgroup walks or its bytes take, several 8.5
+    // and their bytes; from 200 groups on it is one.
+    const int groups = n * G;
+    const float walk = max_ctx * 12.5e-3f, mb = groups * 0.8f * max_ctx * 512e-6f;
+    if (groups >= 200 || 3.f + fmaxf(walk, mb / 4.9f) <= 8.5f + mb / 5.2f) return 1;
+    const int parts = (511 + groups) / groups, most = (max_ctx + 255) / 256;
+    return parts < most ? parts < 64 ? parts : 64 : most < 64 ? most : 64;
+  }
   d.SW = d.v0 = D;
   d.W = D + V;
   d.R = V;
@@ -413,9 +431,23 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
                               const int32_t* block_tables, void* out,
                               float* part_o, float* part_ml, int n, int H,
                               int G, int D, int V, int max_blocks, int bs,
-                              int parts, float scale, int has_sink, float sink,
-                              hipStream_t stream) {
+                              int max_ctx, int parts, float scale, int has_sink,
+                              float sink, hipStream_t stream) {
   if (!lds_grouped_decode_ok(D, V, q_stride)) return hipErrorInvalidValue;
+  if (n == 0) return hipSuccess;
+  if (in_core(D, V, H / G)) {
+    const int64_t head = (int64_t)bs * (D + V);
+    const short* const keys = (const short*)cache;
+    const decode::Work<short> w{
+        (const short*)q, q_stride, keys, keys + D, G * head, head, block_tables,
+        positions, row_seq, 1, max_blocks, bs, (short*)out, part_o, part_ml, G,
+        H / G, 0, 0, scale, sink * LOG2E, has_sink};
+    // short rows leave half of 8 waves without a tile
+    const int waves = max_ctx <= 256 ? 4 : 8;
+    if (parts > 64) return hipErrorInvalidValue;
+    return parts > 1 ? decode::attend<true, 256>(w, n, parts, waves, stream)
+                     : decode::attend<false, 256>(w, n, 1, waves, stream);
+  }
   Decode d{};
   d.qa = (const short*)q;
   d.qa_row = q_stride;

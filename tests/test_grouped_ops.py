@@ -252,6 +252,33 @@ class TestGroupedAttention:
                 close(out[-1], want, run, f32=1e-5)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rep", [1, 3, 8])
+@pytest.mark.parametrize("bs", [16, 5])
+@pytest.mark.parametrize("sink", [0.0, None])
+@pytest.mark.parametrize("ctxs", [
+    [1, 31, 32, 33, 200, 256], [257, 1, 40], [3, 2000, 1025, 512], [130, 1] * 34])
+def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
+    """Four and eight waves, one part and several, of rows that have fewer tokens than
+    parts; tiles' and pages' ends."""
+    monkeypatch.setitem(globals(), "BS", bs)
+    run, G, D = ("cuda", torch.bfloat16), 3, 128
+    H, n = rep * G, len(ctxs)
+    cache, tables, kv = paged(run, G, D, D, ctxs)
+    proj = put(rnd(n, H * D + 2 * G * D, seed=3), run)
+    pos = torch.tensor([c - 1 for c in ctxs], dtype=torch.int32, device="cuda")
+    seq = torch.arange(n, dtype=torch.int32, device="cuda")
+    out = put(torch.full((n, H * D), 7.0), run)
+    scale = 1.2 * D ** -0.5
+    ops.grouped_decode(proj, cache, pos, seq, tables, n, H, D, scale, sink, max(ctxs),
+                       out)
+    q = f64(proj)[:, :H * D].view(n, H, D)
+    want = torch.stack([expected(q[i], *kv[i], c - 1, scale, sink)
+                        for i, c in enumerate(ctxs)])
+    # probabilities have 24 bits: 32-bit scores and sums, and the result's rounding
+    assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
+
+
 # ---- experts ----------------------------------------------------------------
 @pytest.mark.parametrize("run", RUNS)
 @pytest.mark.parametrize("T,K,E,top", [
