@@ -13,6 +13,8 @@
 #include "../rows_core.h"
 #include "../tile_core.h"
 
+#include <climits>
+
 namespace {
 
 // ---- router ----------------------------------------------------------------
@@ -262,6 +264,7 @@ struct Pairs {
   const int4* tiles;
   const float* weights;      // [P]
   int N, K, top, act;
+  int width;                 // expert_rows: channels of a workgroup
 };
 
 // input row of a place
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   const int i = rows_core::along_xcd(blockIdx.y * blocks + blockIdx.x,
                                      p.tiles[0].x * blocks, BN == 64 ? 512 : 256);
   const int4 tile = p.tiles[1 + i / blocks];
-  const int n0 = i % blocks * BN;
+  const int n0 = i % blocks * p.width, n1 = min(N, n0 + p.width);
   if (n0 >= N) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
   const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
@@ -336,12 +339,12 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   for (int j = 0; j < WL; ++j) {
     const int r = Core::w_row(wave, j) + grp;
     w_from[j] = (const short*)p.w +
-                ((int64_t)tile.x * N + min(n0 + r, N - 1)) * K + Core::piece(r, lane);
+                ((int64_t)tile.x * N + min(n0 + r, n1 - 1)) * K + Core::piece(r, lane);
   }
   float4v acc[CT][MT];
   const int steps = (K + rows_core::KS - 1) / rows_core::KS;
   Core::run(ring, wave, lane, w_from, x_from, 0, K, steps,
-            uint32_t(i) * BN / 128 * 3 % uint32_t(steps), true, acc);
+            uint32_t(i) * BN / 128 * 3 % uint32_t(steps), wave * 16 < p.width, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = (wave / Core::WC * MT + t) * 16 + col;
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       const int n = n0 + (wave % Core::WC * CT + c) * 16 + grp * 4;
-      if (n >= N) continue;
+      if (n >= n1) continue;
       const float4v s = acc[c][t];
       *(short4v*)((short*)p.out + (int64_t)(UP ? tile.y + m : pair) * N + n) =
           (short4v){f32_to_bf16(finish<UP>(p, s[0], wt)),
@@ -362,14 +365,28 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   }
 }
 
+// Channels of a workgroup, of BN at most, with which about `tiles` tiles take the least of
+// whole rounds of the chip (32 experts of 3584 channels: 3.5 rounds by 64, 4 by 56)
+int even_width(int N, int BN, int tiles) {
+  const int slots = BN == 64 ? 512 : 256;
+  int best = BN, least = INT_MAX;
+  for (int width = BN; width > BN / 2; width -= 8) {
+    const int64_t blocks = (int64_t)((N + width - 1) / width) * tiles;
+    const int64_t cost = (blocks + slots - 1) / slots * width;
+    if (cost < least) least = (int)cost, best = width;
+  }
+  return best;
+}
+
 template <int RT, int BN, bool UP>
-hipError_t launch_rows(const Pairs& p, int max_tiles, hipStream_t stream) {
+hipError_t launch_rows(Pairs p, int max_tiles, int tiles, hipStream_t stream) {
   typedef rows_core::RowsCore<RT, BN> Core;
   auto fn = expert_rows_kernel<RT, BN, UP>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, Core::RINGS);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(((p.N + BN - 1) / BN + 7) / 8 * 8, max_tiles),
+  p.width = even_width(p.N, BN, tiles);
+  hipLaunchKernelGGL(fn, dim3(((p.N + p.width - 1) / p.width + 7) / 8 * 8, max_tiles),
                      dim3(Core::NW * WAVE), Core::RINGS, stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
@@ -508,8 +525,8 @@ hipError_t launch_tiles(const Pairs& p, int max_tiles, hipStream_t stream) {
 }
 
 template <bool UP>
-hipError_t product(int f32, int plain, int tile, int max_tiles, const Pairs& p,
-                   hipStream_t stream) {
+hipError_t product(int f32, int plain, int tile, int max_tiles, int tiles,
+                   const Pairs& p, hipStream_t stream) {
   if (tile == TILE) return launch_tiles<UP>(p, max_tiles, stream);
   const dim3 grid((p.N + 63) / 64, max_tiles), block(256);
   if (max_tiles > 65535 || tile > 64) return hipErrorInvalidValue;
@@ -517,9 +534,9 @@ hipError_t product(int f32, int plain, int tile, int max_tiles, const Pairs& p,
 #define K2(NAME, ARG) NAME<ARG, UP>
   if (f32) GO(K2(expert_plain_kernel, float));
   else if (plain || p.N % 8 || p.K % 8) GO(K2(expert_plain_kernel, short));
-  else if (tile <= 16) return launch_rows<1, 64, UP>(p, max_tiles, stream);
-  else if (tile <= 32) return launch_rows<2, 64, UP>(p, max_tiles, stream);
-  else return launch_rows<4, 128, UP>(p, max_tiles, stream);
+  else if (tile <= 16) return launch_rows<1, 64, UP>(p, max_tiles, tiles, stream);
+  else if (tile <= 32) return launch_rows<2, 64, UP>(p, max_tiles, tiles, stream);
+  else return launch_rows<4, 128, UP>(p, max_tiles, tiles, stream);
 #undef K2
 #undef GO
   HIP_CHECK_LAST();
@@ -596,12 +613,13 @@ hipError_t lds_sort_pairs(const int32_t* ids, int32_t* order, void* tiles,
 hipError_t lds_expert_product(int f32, int plain, int up, const void* a,
                               const void* w, void* out, const int32_t* order,
                               const void* tiles, int max_tiles, int tile,
-                              const float* weights, int N, int K, int top,
+                              const float* weights, int E, int N, int K, int top,
                               int act, hipStream_t stream) {
   if (max_tiles == 0) return hipSuccess;
-  const Pairs p{a, w, out, order, (const int4*)tiles, weights, N, K, top, act};
-  return up ? product<true>(f32, plain, tile, max_tiles, p, stream)
-            : product<false>(f32, plain, tile, max_tiles, p, stream);
+  const Pairs p{a, w, out, order, (const int4*)tiles, weights, N, K, top, act, 0};
+  const int some = E < max_tiles ? E : max_tiles;      // a tile per expert, or so
+  return up ? product<true>(f32, plain, tile, max_tiles, some, p, stream)
+            : product<false>(f32, plain, tile, max_tiles, some, p, stream);
 }
 
 }  // extern "C"

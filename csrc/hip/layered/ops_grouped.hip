@@ -25,7 +25,7 @@ hipError_t lds_sort_pairs(const int32_t*, int32_t*, void*, int, int, int, int,
                           hipStream_t);
 hipError_t lds_expert_product(int, int, int, const void*, const void*, void*,
                               const int32_t*, const void*, int, int,
-                              const float*, int, int, int, int, hipStream_t);
+                              const float*, int, int, int, int, int, hipStream_t);
 }
 
 namespace {
@@ -223,13 +223,13 @@ Tensor experts(Tensor h, Tensor ids, Tensor weights, Tensor up, Tensor down,
       sort_pairs(ids, E, tile, E * F * K * h.element_size() > 512ll << 20);
   check_hip(lds_expert_product(f32, plain, 1, h.data_ptr(), up.data_ptr(),
                                inner.data_ptr(), ip(order), tiles.data_ptr(),
-                               max_tiles, tile, fp(weights), (int)F, (int)K,
-                               (int)top, (int)act_code, cur_stream()),
+                               max_tiles, tile, fp(weights), (int)E, (int)F,
+                               (int)K, (int)top, (int)act_code, cur_stream()),
             "expert_product");
   check_hip(lds_expert_product(f32, plain, 0, inner.data_ptr(),
                                down.data_ptr(), out.data_ptr(), ip(order),
                                tiles.data_ptr(), max_tiles, tile, fp(weights),
-                               (int)K, (int)F, (int)top, (int)act_code,
+                               (int)E, (int)K, (int)F, (int)top, (int)act_code,
                                cur_stream()),
             "expert_product");
   return out;
