@@ -212,6 +212,32 @@ __global__ __launch_bounds__(NT) void store_heads_kernel(
   }
 }
 
+// The same of rows [queries | keys | values] that are in parts of 32 bits (rows apart by P
+// channels, the parts by all of them): their sums, rounded to bf16; the queries, col
+// channels, go to q. A launch of its own for the sums took as long again (60 rows of 6144
+// in 5 parts: 4.7 + 4.2 us, so 5.2).
+__global__ __launch_bounds__(NT) void store_heads_parts_kernel(
+    const float* __restrict__ part, int parts, int P, int col,
+    const int64_t* __restrict__ slots, short* __restrict__ q,
+    short* __restrict__ cache, int64_t rows, int G, int bs, int D, int V) {
+  const int W = D + V, pieces = (col + G * W) / 8;
+  const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
+  if (i >= rows * pieces) return;
+  const int64_t row = i / pieces;
+  const int c = (int)(i % pieces) * 8;
+  const float4v* const src[1] = {(const float4v*)(part + row * P + c)};
+  float f[8];
+  PartSums<1>(src, rows * P / 4, parts).get(0, f);
+  short* to = q + row * col + c;
+  if (c >= col) {
+    const int64_t slot = slots[row];
+    const int x = c - col, v = x - G * D;       // of all heads' keys, of their values
+    const int g = v < 0 ? x / D : v / V, d = v < 0 ? x % D : D + v % V;
+    to = cache + ((slot / bs * G + g) * bs + slot % bs) * W + d;
+  }
+  stn<8>(to, f);
+}
+
 template <typename T>
 hipError_t attn_rows_t(const void* const* ptr, const int64_t* stride, int da,
                        int db, int dv, int rep, int has_sink, float sink,
@@ -348,6 +374,22 @@ hipError_t lds_store_heads(const void* kv, int64_t stride,
                      rows, G, bs, D / u, V / u)
   if (u > 1) GO(short8); else if (es == 4) GO(float); else GO(short);
 #undef GO
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
+// part [parts, rows, P]; q [rows, col]; bf16 cache. col, D and V in steps of 8.
+hipError_t lds_store_heads_parts(const float* part, int parts, int P, int col,
+                                 const int64_t* slots, void* q, void* cache,
+                                 int64_t rows, int G, int bs, int D, int V,
+                                 hipStream_t stream) {
+  if (rows == 0) return hipSuccess;
+  const int64_t blocks = (rows * ((col + G * (D + V)) / 8) + NT - 1) / NT;
+  if (col % 8 || D % 8 || V % 8 || P % 8 || blocks > 0x7fffffff)
+    return hipErrorInvalidValue;
+  hipLaunchKernelGGL(store_heads_parts_kernel, dim3((uint32_t)blocks), dim3(NT),
+                     0, stream, part, parts, P, col, slots, (short*)q,
+                     (short*)cache, rows, G, bs, D, V);
   HIP_CHECK_LAST();
   return hipSuccess;
 }

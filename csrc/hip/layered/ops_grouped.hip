@@ -5,6 +5,9 @@
 extern "C" {
 hipError_t lds_store_heads(const void*, int64_t, const int64_t*, void*,
                            int64_t, int, int, int, int, int, hipStream_t);
+hipError_t lds_store_heads_parts(const float*, int, int, int, const int64_t*,
+                                 void*, void*, int64_t, int, int, int, int,
+                                 hipStream_t);
 int lds_grouped_decode_ok(int, int, int64_t);
 int lds_grouped_decode_parts(int, int, int, int, int, int);
 hipError_t lds_grouped_decode(const void*, int64_t, const void*,
@@ -49,24 +52,39 @@ Heads heads(const Tensor& proj, const Tensor& cache, int64_t H, int64_t D) {
   return s;
 }
 
-// columns from `col` on: keys of all heads, then values of all heads
-void store_heads(Tensor proj, int64_t col, Tensor slots, Tensor cache,
-                 int64_t dim) {
+// columns from `col` on: keys of all heads, then values of all heads. -> proj, or where
+// it came in 32-bit parts [parts, rows, columns] the columns ahead of them in bf16
+Tensor store_heads(Tensor proj, int64_t col, Tensor slots, Tensor cache,
+                   int64_t dim) {
+  TORCH_CHECK((proj.dim() == 2 || proj.dim() == 3) && cache.dim() == 4,
+              "proj, cache");
+  const int64_t G = cache.size(1), W = cache.size(3), bs = cache.size(2);
+  const int64_t rows = proj.size(-2), P = proj.size(-1);
+  TORCH_CHECK(dim >= 0 && dim <= W && col >= 0 && col + G * W <= P, "columns");
+  check(slots, at::kLong, "slots");
+  sized(slots, {rows}, "slots");
+  if (proj.dim() == 3) {
+    check(proj, at::kFloat, "proj");
+    TORCH_CHECK(act(cache, "cache") == 0, "parts go to a bf16 cache");
+    TORCH_CHECK(col % 8 == 0 && dim % 8 == 0 && W % 8 == 0 && P % 8 == 0 &&
+                    dim > 0 && dim < W && P < (1 << 30), "columns of parts");
+    Tensor q = torch::empty({rows, col}, cache.options());
+    check_hip(lds_store_heads_parts(
+                  fp(proj), (int)proj.size(0), (int)P, (int)col,
+                  slots.data_ptr<int64_t>(), q.data_ptr(), cache.data_ptr(), rows,
+                  (int)G, (int)bs, (int)dim, (int)(W - dim), cur_stream()),
+              "store_heads");
+    return q;
+  }
   const int f32 = act(proj, "proj");
   same_act(cache, f32, "cache");
-  TORCH_CHECK(proj.dim() == 2 && cache.dim() == 4, "proj, cache");
-  const int64_t G = cache.size(1), W = cache.size(3);
-  TORCH_CHECK(dim >= 0 && dim <= W && col >= 0 &&
-                  col + G * W <= proj.size(1), "columns");
-  check(slots, at::kLong, "slots");
-  sized(slots, {proj.size(0)}, "slots");
   const int es = (int)proj.element_size();
-  check_hip(lds_store_heads((const char*)proj.data_ptr() + col * es,
-                            proj.size(1), slots.data_ptr<int64_t>(),
-                            cache.data_ptr(), proj.size(0), (int)G,
-                            (int)cache.size(2), (int)dim, (int)(W - dim), es,
+  check_hip(lds_store_heads((const char*)proj.data_ptr() + col * es, P,
+                            slots.data_ptr<int64_t>(), cache.data_ptr(), rows,
+                            (int)G, (int)bs, (int)dim, (int)(W - dim), es,
                             cur_stream()),
             "store_heads");
+  return proj;
 }
 
 // rows [base, base + n) one by one

@@ -183,8 +183,9 @@ def latent_prefill(q, kv, lat, positions, row_seq, base, seq_meta, ctx, tiles,
 
 def store_heads(proj, col, slots, cache, dim):
     """Keys of all heads, then values of all heads, from column `col` on ->
-    the cache pages [blocks, heads, tokens, key | value]."""
-    _impl(proj).store_heads(proj, col, slots, cache, dim)
+    the cache pages [blocks, heads, tokens, key | value]. Returns what leads a row,
+    the queries: proj, or of linear_parts' parts (sizes in steps of 8) their sums."""
+    return _impl(proj).store_heads(proj, col, slots, cache, dim)
 
 
 def grouped_decode(proj, cache, positions, row_seq, block_tables, n, heads,

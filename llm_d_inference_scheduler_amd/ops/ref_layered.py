@@ -189,6 +189,7 @@ def store_heads(proj, col, slots, cache, dim):
     new = torch.cat([k.unflatten(1, (G, dim)),
                      v.unflatten(1, (G, W - dim))], -1)
     cache[slots // bs, :, slots % bs] = new
+    return proj
 
 
 def _grouped(proj, cache, positions, row_seq, block_tables, lo, hi, heads,

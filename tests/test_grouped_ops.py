@@ -253,6 +253,28 @@ class TestGroupedAttention:
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("parts", [1, 2, 5, 8, 9])
+@pytest.mark.parametrize("rows,H,G,D,V,extra", [
+    (1, 4, 2, 128, 128, 0), (7, 3, 3, 8, 16, 8), (33, 2, 1, 40, 8, 0),
+    (60, 32, 8, 128, 128, 0)])
+def test_store_of_parts(parts, rows, H, G, D, V, extra):
+    """The sums in 32 bits, part by part, and one rounding: to the bit."""
+    run = ("cuda", torch.bfloat16)
+    part = rnd(parts, rows, H * D + G * (D + V) + extra, seed=parts).cuda()
+    total = part[0].clone()
+    for p in part[1:]:
+        total += p
+    want = put(torch.full((rows // BS + 2, G, BS, D + V), 9.0), run)
+    cache = want.clone()
+    slots = torch.randperm(rows + 3, generator=torch.Generator().manual_seed(rows))
+    slots = slots[:rows].cuda()
+    ops.store_heads(total.bfloat16(), H * D, slots, want, D)
+    q = ops.store_heads(part, H * D, slots, cache, D)
+    assert torch.equal(cache, want)
+    assert torch.equal(q, total.bfloat16()[:, :H * D])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("rep", [1, 3, 8])
 @pytest.mark.parametrize("bs", [16, 5])
 @pytest.mark.parametrize("sink", [0.0, None])
