@@ -15,6 +15,9 @@
 extern "C" {
 int lds_linear_rows_parts(int M, int N, int K);
 int lds_linear_plain_parts(int M, int N, int K);
+hipError_t lds_linear_pair(const void*, const void*, int64_t, const void*,
+                           const void*, int64_t, void*, void*, int, int, int,
+                           hipStream_t);
 int lds_linear_rows_takes(int M, int N, int K, int gated, int parts);
 hipError_t lds_linear_rows(const void*, int64_t, const void*, int64_t, void*,
                            float*, int, int, int, int, int, hipStream_t);
@@ -227,6 +230,28 @@ inline c10::optional<Tensor> linear32(const Tensor& x, const Tensor& w) {
   return linear_rows(x, w, true);
 }
 
+// x w' and x2 w2' of one shape in a launch, or None: for few rows of short K, whose
+// products are one part each
+inline c10::optional<std::tuple<Tensor, Tensor>> linear_pair(
+    const Tensor& x, const Tensor& w, const Tensor& x2, const Tensor& w2) {
+  if (!few_rows(x, w, PLAIN) || !few_rows(x2, w2, PLAIN) ||
+      x.sizes() != x2.sizes() || w.sizes() != w2.sizes() ||
+      x.stride(0) != x2.stride(0) || w.stride(0) != w2.stride(0) ||
+      x.device() != x2.device())
+    return c10::nullopt;
+  const int M = (int)x.size(0), K = (int)x.size(1), N = (int)w.size(0);
+  if (M > 64 || K > 1024 || lds_linear_plain_parts(M, N, K) != 1)
+    return c10::nullopt;
+  const c10::DeviceGuard guard(x.device());
+  Tensor y = torch::empty({M, N}, x.options());
+  Tensor y2 = torch::empty({M, N}, x.options());
+  check(lds_linear_pair(
+      x.data_ptr(), x2.data_ptr(), x.stride(0), w.data_ptr(), w2.data_ptr(),
+      w.stride(0), y.data_ptr(), y2.data_ptr(), M, N, K,
+      at::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()));
+  return std::make_tuple(y, y2);
+}
+
 inline Tensor linear_act(const Tensor& x, const Tensor& w, int64_t act,
                          bool gated, int rows) {
   const c10::DeviceGuard guard(x.device());
@@ -312,6 +337,7 @@ inline void bind(pybind11::module& m) {
   m.def("linear", &linear, "x @ w' of w [N, K]");
   m.def("linear_parts", &linear_parts, "the same, or its parts of K");
   m.def("linear32", &linear32, "the same with a 32-bit result, or None");
+  m.def("linear_pair", &linear_pair, "x @ w' and x2 @ w2' in a launch, or None");
   m.def("gated_linear", &gated_linear,
         "act(x gate') * (x up') of w = [gate; up], or None");
   m.def("activated_linear", &activated_linear, "act(x w'), or None");

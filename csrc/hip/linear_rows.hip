@@ -27,6 +27,9 @@ struct Rows {
   int M, N, K, k_part;       // k_part: K per part, a multiple of KS
   int parts, act;
   int width;                 // rows of w of a workgroup, a multiple of UNIT
+  int first;                 // blocks of the first of two products of one shape, or 0
+  const short *x2, *w2;
+  void* y2;
 };
 
 // what becomes of the sums: bf16, 32-bit (also of a part of K), act of them or
@@ -50,8 +53,16 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
   const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
   const int M = p.M, N = p.N;
   const int part = blockIdx.x % p.parts;
-  const int blk = p.parts > 1 ? blockIdx.x / p.parts
-                              : along_xcd(blockIdx.x, gridDim.x, ROUND);
+  int blk = p.parts > 1 ? blockIdx.x / p.parts
+                        : along_xcd(blockIdx.x, gridDim.x, ROUND);
+  const short *x = p.x, *w = p.w;
+  void* y = p.y;
+  if (p.first && blk >= p.first) {
+    blk -= p.first;
+    x = p.x2;
+    w = p.w2;
+    y = p.y2;
+  }
   const int width = p.width, n0 = OUT == GATED ? blk * (width / 2) : blk * width;
   if (n0 >= N) return;
   // this group's K: steps of KS, the last ones past the end where they do not go round
@@ -72,12 +83,12 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
     const int r = Core::w_row(wave, j) + grp;          // row in LDS
     const int n = OUT == GATED ? r / 16 * 8 + r % 8 : r;
     const bool up = OUT == GATED && r % 16 >= 8;
-    w_from[j] = p.w + (min(n0 + n, n1 - 1) + (up ? N : 0)) * p.w_row + Core::piece(r, lane);
+    w_from[j] = w + (min(n0 + n, n1 - 1) + (up ? N : 0)) * p.w_row + Core::piece(r, lane);
   }
 #pragma unroll
   for (int j = 0; j < XL; ++j) {
     const int r = Core::x_row(wave, j) + grp;
-    x_from[j] = p.x + min(r, M - 1) * p.x_row + Core::piece(r, lane);
+    x_from[j] = x + min(r, M - 1) * p.x_row + Core::piece(r, lane);
   }
   float4v acc[CT][MT];
   Core::run(lds + group * Core::RINGS, wave, lane, w_from, x_from, k_lo, k_hi, steps,
@@ -129,13 +140,13 @@ __global__ __launch_bounds__(BN / 16 * KG * WAVE) void linear_rows_kernel(
       if (m >= M || n >= n1) continue;     // n1 - n0 is a multiple of 4
       const int64_t o = ((int64_t)part * M + m) * N + n;
       if constexpr (OUT == F32) {
-        *(float4v*)((float*)p.y + o) = s;
+        *(float4v*)((float*)y + o) = s;
       } else {
         short4v v;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           v[r] = f32_to_bf16(OUT == ACT ? activate(p.act, s[r]) : s[r]);
-        *(short4v*)((short*)p.y + o) = v;
+        *(short4v*)((short*)y + o) = v;
       }
     }
 }
@@ -208,10 +219,14 @@ hipError_t go(Rows p, hipStream_t stream) {
   const hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
-  const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
+  const int rows = (OUT == GATED || p.x2 ? 2 : 1) * p.N;        // of w
   p.width = p.parts > 1 ? BN : even_width(rows);
   const int ch = OUT == GATED ? p.width / 2 : p.width;
   int groups = (p.N + ch - 1) / ch * p.parts;
+  if (p.x2) {
+    p.first = groups;
+    groups *= 2;
+  }
   if (p.parts == 1) groups = (groups + 7) / 8 * 8;     // equal shares of the XCDs
   hipLaunchKernelGGL(fn, dim3(groups), dim3(BN / 16 * KG * WAVE), bytes, stream,
                      p);
@@ -231,7 +246,7 @@ hipError_t go(Rows p, hipStream_t stream) {
 // up: 22.1, 21.9).
 template <int RT, int OUT>
 hipError_t go_width(const Rows& p, hipStream_t stream) {
-  const int rows = OUT == GATED ? 2 * p.N : p.N;       // of w
+  const int rows = (OUT == GATED || p.x2 ? 2 : 1) * p.N;        // of w
   if (p.parts == 1 && rows <= 32 * ROUND)
     return go<RT, 32, RT == 1 ? 4 : 2, OUT>(p, stream);
   if (p.parts == 1 && rows <= 64 * ROUND)
@@ -426,6 +441,20 @@ hipError_t lds_activated_rows(const void* x, int64_t x_row, const void* w,
   const Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K,
                (K + KS - 1) / KS * KS, 1, act};
   return go_rows<ACT>(p, stream);
+}
+
+// Two products of one shape and one part, y = x w' and y2 = x2 w2', in a launch, for up to
+// 64 rows (two of 128 -> 4096, 50 rows: 3.9 us each)
+hipError_t lds_linear_pair(const void* x, const void* x2, int64_t x_row,
+                           const void* w, const void* w2, int64_t w_row, void* y,
+                           void* y2, int M, int N, int K, hipStream_t stream) {
+  if (M < 1 || M > ROWS || N < 1 || N % 4 || N > 1 << 24 || K < 8 || K % 8 ||
+      x_row % 8 || w_row % 8 || !x2)
+    return hipErrorInvalidValue;
+  const Rows p{(const short*)x, (const short*)w, x_row, w_row, y, M, N, K,
+               (K + KS - 1) / KS * KS, 1, -1, 0, 0, (const short*)x2,
+               (const short*)w2, y2};
+  return go_rows<BF16>(p, stream);
 }
 
 }  // extern "C"

@@ -143,8 +143,9 @@ class ChannelDelta:
         s = self.spec
         conv_state, state = cache
         proj = linear(h, self.w_in)
-        decay = linear(proj[:, self.a_col:self.g_col], self.w_a2)
-        gate = linear(proj[:, self.g_col:], self.w_g2)
+        decay, gate = ops.linear_pair(
+            proj[:, self.a_col:self.g_col], self.w_a2,
+            proj[:, self.g_col:], self.w_g2)
         q, k, v = ops.delta_prep(
             proj, self.taps, conv_state, batch.row_seq, batch.seq_meta,
             batch.multi_row, s.kv_heads, s.heads, s.dim, s.vdim,

@@ -33,6 +33,15 @@ def linear(x, w):
     return hip_layered().linear(x, w) if x.is_cuda else x @ w.t()
 
 
+def linear_pair(x, w, x2, w2):
+    """x @ w' and x2 @ w2': of few rows and short K in one launch."""
+    if x.is_cuda:
+        pair = hip_layered().linear_pair(x, w, x2, w2)
+        if pair is not None:
+            return pair
+    return linear(x, w), linear(x2, w2)
+
+
 def linear_parts(x, w):
     """The same for stream_norm, which also takes the 32-bit partial sums
     [parts, rows, out] of a product that split K."""

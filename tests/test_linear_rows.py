@@ -252,6 +252,21 @@ def test_even_rounds(rows, rows_of_w, k):
     _same(ext.gated_linear(x, w, 1), F.silu(g) * u, 8)
 
 
+@pytest.mark.parametrize("rows", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(8, 8), (24, 128), (520, 136), (4096, 128), (4096, 520),
+                                 (4104, 1024)])
+def test_pair(rows, n, k):
+    """Two products in a launch: columns of one tensor, the last block of the first."""
+    ext = _ext("_hip_layered")
+    x = _draw(rows, 2 * k + 8, seed=rows)
+    w, w2 = (_draw(n, k, seed=n + i, scale=k ** -0.5) for i in range(2))
+    pair = ext.linear_pair(x[:, 8:k + 8], w, x[:, k + 8:], w2)
+    for y, a, b in zip(pair, (x[:, 8:k + 8], x[:, k + 8:]), (w, w2)):
+        _same(y, a.double() @ b.double().t(), 8)
+    assert ext.linear_pair(x[:, :k], w, x[:, :k], w2[:, :k - 8]) is None
+    assert ext.linear_pair(x[:, :k], w, x[:, :k].contiguous(), w2) is None or rows == 1
+
+
 @pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("rows,n", [(16, 4096), (8192, 8192)])
 @pytest.mark.parametrize("act", [-1, 3, 1 << 32])
