@@ -59,6 +59,70 @@ __global__ __launch_bounds__(NT) void latent_prep_kernel(
     rotate_pair(p + kv_rank + 2 * i, dst + kv_rank + 2 * i, cs + 2 * i);
 }
 
+// The same by pieces of 8 channels, PIECES per thread at most: both sums are of what is
+// then in registers (50 rows of 1536 + 512 + 64: 6.5 us a channel at a time).
+constexpr int PIECES = 4;
+__global__ __launch_bounds__(NT) void latent_prep_vec_kernel(
+    const short* __restrict__ proj, int64_t pstride,
+    const float* __restrict__ wq, const float* __restrict__ wkv,
+    const float* __restrict__ cos_sin, const int32_t* __restrict__ positions,
+    const int64_t* __restrict__ slots, short* __restrict__ cq,
+    short* __restrict__ cache, int q_rank, int kv_rank, int rot, float eps) {
+  __shared__ float red[2][NWV];
+  const int64_t row = blockIdx.x;
+  const short* p = proj + row * pstride;
+  const int all = (cache ? q_rank + kv_rank + rot : q_rank) / 8;
+  float x[PIECES][8], sq = 0.f, skv = 0.f;
+  const int64_t slot = cache ? slots[row] : 0;
+  const float* cs = cos_sin + (cache ? (int64_t)positions[row] * rot : 0);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int c = threadIdx.x + i * NT;
+    if (c < all) ldn<8>(p + c * 8, x[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int c = (threadIdx.x + i * NT) * 8;
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += x[i][j] * x[i][j];
+    if (c < q_rank) sq += ss;
+    else if (c < q_rank + kv_rank && c < all * 8) skv += ss;
+  }
+  const float iq =
+      1.f / sqrtf(block_sum<NWV>(sq, red[0]) / (float)q_rank + eps);
+  const float ikv =
+      cache ? 1.f / sqrtf(block_sum<NWV>(skv, red[1]) / (float)kv_rank + eps) : 0.f;
+  short* dst = cache + slot * (kv_rank + rot);
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    int c = (threadIdx.x + i * NT) * 8;
+    if (c >= all * 8) break;
+    float w[8], f[8];
+    if (c < q_rank) {
+      ldn<8>(wq + c, w);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = x[i][j] * iq * w[j];
+      stn<8>(cq + row * q_rank + c, f);
+      continue;
+    }
+    c -= q_rank;
+    if (c < kv_rank) {
+      ldn<8>(wkv + c, w);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = x[i][j] * ikv * w[j];
+    } else {
+      ldn<8>(cs + c - kv_rank, w);
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        f[j] = x[i][j] * w[j] - x[i][j + 1] * w[j + 1];
+        f[j + 1] = x[i][j + 1] * w[j] + x[i][j] * w[j + 1];
+      }
+    }
+    stn<8>(dst + c, f);
+  }
+}
+
 // In place on the rotated part of q [rows, H, D + rot]; the unrotated part
 // of the first n_abs rows is laid out by head for the absorbing product.
 template <typename T>
@@ -82,6 +146,38 @@ __global__ __launch_bounds__(NT) void rope_part_kernel(
           qr[(int64_t)h * (D + rot) + d];
     }
   }
+}
+
+// The same by pieces of 8 channels: those to be rotated, then those to be laid out (50
+// rows of 32 heads of 128 + 64: 6.5 us a row per workgroup, a channel at a time).
+__global__ __launch_bounds__(NT) void rope_part_vec_kernel(
+    short* __restrict__ q, short* __restrict__ by_head,
+    const float* __restrict__ cos_sin, const int32_t* __restrict__ positions,
+    int64_t rows, int64_t n_abs, int H, int D, int rot) {
+  const int turn = rot / 8, lay = D / 8;
+  const int64_t turned = rows * H * turn;
+  int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
+  if (i < turned) {
+    const int64_t rh = i / turn, row = rh / H;
+    const int d = (int)(i % turn) * 8;
+    short* p = q + rh * (D + rot) + D + d;
+    float x[8], w[8], f[8];
+    ldn<8>(p, x);
+    ldn<8>(cos_sin + (int64_t)positions[row] * rot + d, w);
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      f[j] = x[j] * w[j] - x[j + 1] * w[j + 1];
+      f[j + 1] = x[j + 1] * w[j] + x[j] * w[j + 1];
+    }
+    stn<8>(p, f);
+    return;
+  }
+  i -= turned;
+  if (i >= n_abs * H * lay) return;
+  const int64_t rh = i / lay, row = rh / H, h = rh % H;
+  const int d = (int)(i % lay) * 8;
+  *(short8*)(by_head + (h * n_abs + row) * D + d) =
+      *(const short8*)(q + rh * (D + rot) + d);
 }
 
 // [H, n_abs, V] -> rows of [.., H V]
@@ -284,6 +380,17 @@ hipError_t lds_latent_prep(int f32, const void* proj, int64_t pstride,
                            int rows, int q_rank, int kv_rank, int rot,
                            float eps, hipStream_t stream) {
   if (rows == 0) return hipSuccess;
+  const auto at16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  if (!f32 && pstride % 8 == 0 && q_rank % 8 == 0 && kv_rank % 8 == 0 &&
+      rot % 8 == 0 && q_rank + kv_rank + rot <= PIECES * NT * 8 && at16(proj) &&
+      at16(wq) && at16(wkv) && at16(cos_sin) && at16(cq) && at16(cache)) {
+    hipLaunchKernelGGL(latent_prep_vec_kernel, dim3(rows), dim3(NT), 0, stream,
+                       (const short*)proj, pstride, wq, wkv, cos_sin, positions,
+                       slots, (short*)cq, (short*)cache, q_rank, kv_rank, rot,
+                       eps);
+    HIP_CHECK_LAST();
+    return hipSuccess;
+  }
 #define GO(T)                                                                 \
   hipLaunchKernelGGL(latent_prep_kernel<T>, dim3(rows), dim3(NT), 0, stream,  \
                      (const T*)proj, pstride, wq, wkv, cos_sin, positions,    \
@@ -298,6 +405,18 @@ hipError_t lds_rope_part(int f32, void* q, void* by_head, const float* cos_sin,
                          const int32_t* positions, int rows, int n_abs, int H,
                          int D, int rot, hipStream_t stream) {
   if (rows == 0) return hipSuccess;
+  const int64_t pieces =
+      ((int64_t)rows * H * rot + (int64_t)n_abs * H * D) / 8, blocks = (pieces + NT - 1) / NT;
+  const auto at16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+  if (!f32 && D % 8 == 0 && rot % 8 == 0 && blocks <= 0x7fffffff && at16(q) &&
+      at16(by_head) && at16(cos_sin)) {
+    if (blocks)
+      hipLaunchKernelGGL(rope_part_vec_kernel, dim3((uint32_t)blocks), dim3(NT), 0,
+                         stream, (short*)q, (short*)by_head, cos_sin, positions,
+                         rows, n_abs, H, D, rot);
+    HIP_CHECK_LAST();
+    return hipSuccess;
+  }
 #define GO(T)                                                                 \
   hipLaunchKernelGGL(rope_part_kernel<T>, dim3(rows), dim3(NT), 0, stream,    \
                      (T*)q, (T*)by_head, cos_sin, positions, n_abs, H, D, rot)

@@ -272,12 +272,23 @@ __global__ __launch_bounds__(128) void combine_kernel(const Decode d_) {
   for (int p = 0; p < parts; ++p)
     l += ml[p * 2 + 1] * __builtin_amdgcn_exp2f(ml[p * 2] - m);
   const float inv = 1.f / l;
-  for (int d = threadIdx.x; d < R; d += 128) {
-    float o = 0.f;
-    for (int p = 0; p < parts; ++p)
-      o += d_.part_o[(pr + p) * R + d] *
-           __builtin_amdgcn_exp2f(ml[p * 2] - m);
-    d_.out[row * d_.o_row + h * d_.o_head + d] = f32_to_bf16(o * inv);
+  // R is a multiple of 4; four parts are asked for together (50 rows of 32 heads of 512
+  // in 5 parts, a channel at a time: 8.5 us)
+  for (int d = threadIdx.x * 4; d < R; d += 512) {
+    float4v o = {0.f, 0.f, 0.f, 0.f};
+    for (int p = 0; p < parts; p += 4) {
+      float4v x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        x[u] = *(const float4v*)(d_.part_o + (pr + min(p + u, parts - 1)) * R + d);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (p + u < parts) o += x[u] * __builtin_amdgcn_exp2f(ml[(p + u) * 2] - m);
+    }
+    o *= inv;
+    *(short4v*)(d_.out + row * d_.o_row + h * d_.o_head + d) =
+        (short4v){f32_to_bf16(o[0]), f32_to_bf16(o[1]), f32_to_bf16(o[2]),
+                  f32_to_bf16(o[3])};
   }
 }
 

@@ -420,6 +420,53 @@ class TestLatentPrep:
         assert not dst[4:].any()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("q_rank,kv_rank,rot", [
+    (8, 8, 8), (1536, 512, 64), (2040, 8, 16), (8000, 128, 64), (8008, 128, 64)])
+@pytest.mark.parametrize("rows,n_abs", [(1, 1), (9, 4), (70, 0), (70, 70)])
+def test_latent_prep_by_pieces(q_rank, kv_rank, rot, rows, n_abs):
+    """A row in one to four pieces per thread, the last that fits and more; queries
+    that are laid out and those that are not."""
+    run, H, D = ("cuda", torch.bfloat16), 3, 40
+    table = torch.randn(64, rot // 2, 2, generator=torch.Generator().manual_seed(1))
+    pos = torch.arange(rows, dtype=torch.int32) * 7 % 64
+    slots = torch.randperm(80, generator=torch.Generator().manual_seed(2))[:rows]
+    proj = put(rnd(rows, q_rank + kv_rank + rot), run)
+    wq, wkv = rnd(q_rank, seed=1), rnd(kv_rank, seed=2)
+    cache = put(torch.full((5, 16, kv_rank + rot), 9.0), run)
+
+    def turned(x):
+        cs = table.double()[pos.long()]
+        cs = cs.view(rows, *[1] * (x.dim() - 2), rot // 2, 2)
+        u, v = x[..., 0::2], x[..., 1::2]
+        return torch.stack([u * cs[..., 0] - v * cs[..., 1],
+                            v * cs[..., 0] + u * cs[..., 1]], -1).flatten(-2)
+
+    cq = ops.latent_prep(proj, wq.cuda(), wkv.cuda(), table.cuda(), pos.cuda(),
+                         slots.cuda(), cache, 1e-4)
+    p = f64(proj)
+    q_part, kv_part, turn = p.split([q_rank, kv_rank, rot], 1)
+    close(cq, oracle.rms(q_part, 1e-4) * wq.double(), run)
+    got = f64(cache).view(80, -1)
+    close(got[slots, :kv_rank], oracle.rms(kv_part, 1e-4) * wkv.double(), run)
+    # two products, each and their sum rounded in 32 bits, then to bf16
+    assert ((got[slots, kv_rank:] - turned(turn)).abs()
+            <= 2 ** -8 * turned(turn).abs() + 1e-5).all()
+    idle = torch.ones(80, dtype=torch.bool)
+    idle[slots] = False
+    assert (got[idle] == 9).all()
+    again = ops.latent_prep(proj[:, :q_rank].contiguous(), wq.cuda(), None,
+                            table.cuda(), pos.cuda(), slots.cuda(), None, 1e-4)
+    close(again, f64(cq), run)
+    q = put(rnd(rows, H, D + rot, seed=4), run)
+    old = f64(q)
+    plain = ops.rope_part(q, table.cuda(), pos.cuda(), n_abs)
+    assert torch.equal(f64(plain), old[:n_abs, :, :D].transpose(0, 1))
+    assert torch.equal(f64(q)[..., :D], old[..., :D])
+    want = turned(old[..., D:])
+    assert ((f64(q)[..., D:] - want).abs() <= 2 ** -8 * want.abs() + 1e-5).all()
+
+
 def stand_out(keys, pos, window, big):
     """For every row a direction on which one key stands out: in turn the
     oldest key it sees, the one just before that, itself, the next one and
