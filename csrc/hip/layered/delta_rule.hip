@@ -6,7 +6,8 @@
 // delta_prep     short causal convolutions + silu of q, k, v; unit norms
 // delta_conv     convolution inputs kept for the next step
 // delta_step     the recurrence itself, one workgroup per (head, sequence),
-//                with gates and the gated output norm (decode, short rows)
+//                with gates and the gated output norm (decode, short rows);
+//                of single rows with what the other two do (delta_single)
 // The chunked form for long rows is in delta_chunk.hip.
 #include "elem.h"
 
@@ -184,7 +185,21 @@ __global__ __launch_bounds__(NT) void delta_conv_kernel(
 // 14336 behind it: 56; 50 and 102 by the shorter chain; 47 and 103 with the
 // stores non-temporal; 42 (4.9 TB/s) and 88 with both. 200 sequences 186 -> 157,
 // 24 30 -> 17.5, 1 9.2 -> 8.7.
-template <typename T, int RPT, bool VEC>
+//
+// CONV: sequences of one row each, every head with q and k of its own; q, k and v are
+// what delta_prep makes of the row, made here while S is on its way (50 sequences of 32
+// heads of 128 x 128: 46.8 us, apart 6.4 and 44.0).
+template <typename T>
+struct Conv {
+  const T* proj;             // [rows, >= C]
+  int64_t pstride;
+  const float* taps;         // [n_taps, C], 2 to 4
+  T* state;                  // [slots, n_taps - 1, C]
+  int n_taps;
+  float q_scale, unit_eps;
+};
+
+template <typename T, int RPT, bool VEC, bool CONV>
 __global__ __launch_bounds__(NT, RPT <= 8    ? 4
                                  : RPT == 16 ? 3
                                              : 1) void delta_step_kernel(
@@ -198,7 +213,7 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
     const float* __restrict__ norm_w,            // [V]
     float* __restrict__ state,                   // [slots, H, K, V]
     const int32_t* __restrict__ seq_meta, T* __restrict__ out, int KH, int H,
-    int K, int V, int lanes_v, float eps) {
+    int K, int V, int lanes_v, float eps, const Conv<T> in_) {
   const int h = blockIdx.x;
   const Seq sq = load_seq(seq_meta, blockIdx.y);
   const int kh = h / (H / KH);
@@ -227,14 +242,16 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
 #pragma unroll
     for (int i = 0; i < KT; ++i) {
       const unsigned d = min(tid + i * NT, K - 1u);
-      qr[i] = qt[d];
-      kr[i] = kt[d];
+      if constexpr (!CONV) {
+        qr[i] = qt[d];
+        kr[i] = kt[d];
+      }
       dr[i] = dt[d];
     }
     br = beta[row * bstride + h];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      vr[j] = vt[channel(j)];
+      if constexpr (!CONV) vr[j] = vt[channel(j)];
       gr[j] = gt[channel(j)];
     }
   };
@@ -245,6 +262,30 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
 #pragma unroll
   for (int j = 0; j < 4; ++j) nw[j] = norm_w[channel(j)];
   if (sq.n > 0) fetch(0);
+  // the head's channels of q, k and v: a thread's inputs, oldest first, and taps
+  constexpr int CT = CONV ? 2 : 1, TAPS = 4;
+  __shared__ float conv[CONV ? 2 * NT : 1], unit[2];
+  T cx[CT][TAPS];
+  float cw[CT][TAPS];
+  const int QK = KH * K, all = 2 * K + V, C = 2 * QK + H * V;
+  auto column = [&](int i) {
+    const int d = min((int)tid + i * NT, all - 1);
+    return d < K ? kh * K + d : d < 2 * K ? QK + kh * K + d - K
+                                          : 2 * QK + h * V + d - 2 * K;
+  };
+  T* const kept = CONV ? in_.state + (int64_t)sq.slot * (in_.n_taps - 1) * C : nullptr;
+  if constexpr (CONV) {
+#pragma unroll
+    for (int i = 0; i < CT; ++i) {
+      const int c = column(i);
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        cw[i][j] = in_.taps[(int64_t)min(j, in_.n_taps - 1) * C + c];
+        cx[i][j] = j < in_.n_taps - 1 ? kept[(int64_t)j * C + c]
+                                     : in_.proj[sq.row0 * in_.pstride + c];
+      }
+    }
+  }
 
   float S[RPT][4];
   float* Sp = state + ((int64_t)sq.slot * H + h) * K * V;
@@ -270,7 +311,47 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
     }
   }
 
-  for (int t = 0; t < sq.n; ++t) {
+  if constexpr (CONV) {
+    if (sq.n > 0) {                                  // workgroup-uniform
+#pragma unroll
+      for (int i = 0; i < CT; ++i) {
+        const int d = tid + i * NT, c = column(i);
+        float x[TAPS], a = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+          x[j] = j < in_.n_taps - 1 && sq.prior <= 0 ? 0.f : ld(&cx[i][j]);
+          if (j < in_.n_taps) a += cw[i][j] * x[j];
+        }
+        if (d < all) {
+          conv[d] = a * sigmoid_f(a);
+#pragma unroll
+          for (int j = 0; j < TAPS - 1; ++j)
+            if (j < in_.n_taps - 1) st(kept + (int64_t)j * C + c, x[j + 1]);
+        }
+      }
+      lds_barrier();
+      if (tid < 2 * WAVE) {
+        float ss = 0.f;
+        for (int d = tid % WAVE; d < K; d += WAVE) {
+          const float x = conv[tid / WAVE * K + d];
+          ss += x * x;
+        }
+        ss = wave_reduce_sum(ss);
+        if (tid % WAVE == 0)
+          unit[tid / WAVE] = (tid < WAVE ? in_.q_scale : 1.f) / sqrtf(ss + in_.unit_eps);
+      }
+      lds_barrier();
+#pragma unroll
+      for (int i = 0; i < KT; ++i) {
+        const unsigned d = min(tid + i * NT, K - 1u);
+        qr[i] = conv[d] * unit[0];
+        kr[i] = conv[K + d] * unit[1];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) vr[j] = conv[2 * K + channel(j)];
+    }
+  }
+  for (int t = 0; t < (CONV ? min(sq.n, 1) : sq.n); ++t) {
     const int64_t row = sq.row0 + t;
     // readers of gkq and kq of the token before are past a barrier (block_sum)
 #pragma unroll
@@ -333,7 +414,7 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
     T gt[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) gt[j] = gr[j];
-    if (t + 1 < sq.n) fetch(t + 1);
+    if (!CONV && t + 1 < sq.n) fetch(t + 1);
     const float inv =
         1.f / sqrtf(block_sum<NWV>(ss, red) / (float)V + eps);
     T* ot = out + (row * H + h) * V;
@@ -431,10 +512,11 @@ hipError_t lds_delta_step(int f32, const float* q, const float* k,
   while (rpt < need) rpt *= 2;
   const dim3 grid(H, n_seqs);
 #define GO2(T, R, VEC)                                                        \
-  hipLaunchKernelGGL((delta_step_kernel<T, R, VEC>), grid, dim3(NT), 0,       \
-                     stream, q, k, v, (const T*)beta, bstride,                \
+  hipLaunchKernelGGL((delta_step_kernel<T, R, VEC, false>), grid, dim3(NT),   \
+                     0, stream, q, k, v, (const T*)beta, bstride,             \
                      (const T*)decay, dt_bias, neg_a, (const T*)gate, norm_w, \
-                     state, seq_meta, (T*)out, KH, H, K, V, lanes_v, eps)
+                     state, seq_meta, (T*)out, KH, H, K, V, lanes_v, eps,     \
+                     Conv<T>{})
 #define GO1(T, R)                                                             \
   do {                                                                        \
     if (V % 4 == 0) GO2(T, R, true); else GO2(T, R, false);                   \
@@ -456,6 +538,44 @@ hipError_t lds_delta_step(int f32, const float* q, const float* k,
 #undef GO
 #undef GO1
 #undef GO2
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
+// Whether lds_delta_single takes the sizes
+int lds_delta_single_ok(int f32, int KH, int H, int K, int V, int n_taps) {
+  return !f32 && KH == H && V % 4 == 0 && V >= 4 && 2 * K + V <= 2 * NT &&
+         n_taps >= 2 && n_taps <= 4;
+}
+
+// delta_prep and delta_step of sequences of one row each (bf16), in one kernel
+hipError_t lds_delta_single(const void* proj, int64_t pstride, const float* taps,
+                            void* conv_state, int n_taps, float q_scale,
+                            float unit_eps, const void* beta, const void* decay,
+                            const float* dt_bias, const float* neg_a,
+                            const void* gate, const float* norm_w, float* state,
+                            const int32_t* seq_meta, void* out, int n_seqs, int H,
+                            int K, int V, float eps, hipStream_t stream) {
+  if (n_seqs == 0) return hipSuccess;
+  if (!lds_delta_single_ok(0, H, H, K, V, n_taps)) return hipErrorInvalidValue;
+  int lanes_v = 1;
+  while (lanes_v * 4 < V) lanes_v *= 2;
+  const int groups = NT / lanes_v, need = (K + groups - 1) / groups;
+  const Conv<short> cv{(const short*)proj, pstride, taps, (short*)conv_state,
+                       n_taps, q_scale, unit_eps};
+#define GO(R)                                                                 \
+  hipLaunchKernelGGL((delta_step_kernel<short, R, true, true>),               \
+                     dim3(H, n_seqs), dim3(NT), 0, stream, nullptr, nullptr,  \
+                     nullptr, (const short*)beta, pstride,                    \
+                     (const short*)decay, dt_bias, neg_a, (const short*)gate, \
+                     norm_w, state, seq_meta, (short*)out, H, H, K, V,        \
+                     lanes_v, eps, cv)
+  if (need <= 4) GO(4);
+  else if (need <= 8) GO(8);
+  else if (need <= 16) GO(16);
+  else if (need <= 32) GO(32);
+  else return hipErrorInvalidValue;
+#undef GO
   HIP_CHECK_LAST();
   return hipSuccess;
 }

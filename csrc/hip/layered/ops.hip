@@ -11,6 +11,12 @@ hipError_t lds_delta_prep(int, const void*, int64_t, const float*, void*,
                           const int32_t*, const int32_t*, float*, float*,
                           float*, int, int, int, int, int, int, int, int,
                           float, float, hipStream_t);
+int lds_delta_single_ok(int, int, int, int, int, int);
+hipError_t lds_delta_single(const void*, int64_t, const float*, void*, int, float,
+                            float, const void*, const void*, const float*,
+                            const float*, const void*, const float*, float*,
+                            const int32_t*, void*, int, int, int, int, float,
+                            hipStream_t);
 hipError_t lds_delta_step(int, const float*, const float*, const float*,
                           const void*, int64_t, const void*, const float*,
                           const float*, const void*, const float*, float*,
@@ -248,6 +254,52 @@ void delta_step(Tensor q, Tensor k, Tensor v, Tensor proj, int64_t beta_col,
                            ip(seq_meta), out.data_ptr(), (int)n_seqs, (int)KH,
                            (int)H, (int)K, (int)V, (float)eps, cur_stream()),
             "delta_step");
+}
+
+// delta_prep and delta_step of a batch whose sequences have one row each, in one kernel;
+// false where the sizes have none
+bool delta_single(Tensor proj, Tensor taps, Tensor conv_state, double q_scale,
+                  double unit_eps, int64_t beta_col, Tensor decay, Tensor dt_bias,
+                  Tensor neg_a, Tensor gate, Tensor norm_w, Tensor state,
+                  Tensor seq_meta, int64_t KH, Tensor out, double eps) {
+  const int f32 = act(proj, "proj");
+  check(state, at::kFloat, "state");
+  TORCH_CHECK(state.dim() == 4 && proj.dim() == 2 && taps.dim() == 2, "state, proj");
+  const int64_t rows = proj.size(0), H = state.size(1), K = state.size(2);
+  const int64_t V = state.size(3), n_taps = taps.size(0);
+  if (!lds_delta_single_ok(f32, (int)KH, (int)H, (int)K, (int)V, (int)n_taps))
+    return false;
+  const int64_t C = 2 * KH * K + H * V;
+  check(taps, at::kFloat, "taps");
+  sized(taps, {n_taps, C}, "taps");
+  same_act(conv_state, f32, "conv_state");
+  sized(conv_state, {conv_state.size(0), n_taps - 1, C}, "conv_state");
+  TORCH_CHECK(proj.size(1) >= C && beta_col >= 0 && beta_col + H <= proj.size(1),
+              "columns of proj");
+  same_act(decay, f32, "decay");
+  sized(decay, {rows, H * K}, "decay");
+  check(dt_bias, at::kFloat, "dt_bias");
+  sized(dt_bias, {H * K}, "dt_bias");
+  check(neg_a, at::kFloat, "neg_a");
+  sized(neg_a, {H}, "neg_a");
+  same_act(gate, f32, "gate");
+  sized(gate, {rows, H * V}, "gate");
+  same_act(out, f32, "out");
+  sized(out, {rows, H * V}, "out");
+  check(norm_w, at::kFloat, "norm_w");
+  sized(norm_w, {V}, "norm_w");
+  check(seq_meta, at::kInt, "seq_meta");
+  sized(seq_meta, {seq_meta.size(0), 4}, "seq_meta");
+  check_hip(lds_delta_single(
+                proj.data_ptr(), proj.size(1), fp(taps), conv_state.data_ptr(),
+                (int)n_taps, (float)q_scale, (float)unit_eps,
+                (const char*)proj.data_ptr() + beta_col * proj.element_size(),
+                decay.data_ptr(), fp(dt_bias), fp(neg_a), gate.data_ptr(),
+                fp(norm_w), fp(state), ip(seq_meta), out.data_ptr(),
+                (int)seq_meta.size(0), (int)H, (int)K, (int)V, (float)eps,
+                cur_stream()),
+            "delta_single");
+  return true;
 }
 
 // chunks [n, 2] = first row, tokens (1..64); walk [s, 4] = first row, tokens,
@@ -500,6 +552,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("activate", &activate);
   m.def("delta_prep", &delta_prep);
   m.def("delta_step", &delta_step);
+  m.def("delta_single", &delta_single);
   m.def("delta_chunk_work", &lds_delta_chunk_work);
   m.def("delta_chunk", &delta_chunk);
   m.def("delta_gate", &delta_gate);

@@ -146,14 +146,19 @@ class ChannelDelta:
         decay, gate = ops.linear_pair(
             proj[:, self.a_col:self.g_col], self.w_a2,
             proj[:, self.g_col:], self.w_g2)
-        q, k, v = ops.delta_prep(
-            proj, self.taps, conv_state, batch.row_seq, batch.seq_meta,
-            batch.multi_row, s.kv_heads, s.heads, s.dim, s.vdim,
-            s.dim ** -0.5, s.unit_eps)
         T = h.shape[0]
         out = torch.empty((T, s.heads * s.vdim), dtype=h.dtype,
                           device=h.device)
         chunked = batch.long and self.work
+        if not (batch.multi_row or chunked) and ops.delta_single(
+                proj, self.taps, conv_state, s.dim ** -0.5, s.unit_eps,
+                self.beta_col, decay, self.dt_bias, self.neg_a, gate,
+                self.norm, state, batch.seq_meta, s.kv_heads, out, self.eps):
+            return ops.linear_parts(out, self.w_o)
+        q, k, v = ops.delta_prep(
+            proj, self.taps, conv_state, batch.row_seq, batch.seq_meta,
+            batch.multi_row, s.kv_heads, s.heads, s.dim, s.vdim,
+            s.dim ** -0.5, s.unit_eps)
         ops.delta_step(q, k, v, proj, self.beta_col, decay, self.dt_bias,
                        self.neg_a, gate, self.norm, state, batch.seq_meta,
                        batch.n_step_seqs if chunked

@@ -135,6 +135,16 @@ def delta_step(q, k, v, proj, beta_col, decay, dt_bias, neg_a, gate, norm_w,
                         norm_w, state, seq_meta, n_seqs, out, eps)
 
 
+def delta_single(proj, taps, conv_state, q_scale, unit_eps, beta_col, decay,
+                 dt_bias, neg_a, gate, norm_w, state, seq_meta, kv_heads, out,
+                 eps):
+    """delta_prep and delta_step of a batch whose sequences have one row each, in
+    one kernel; False where there is none for the sizes."""
+    return proj.is_cuda and hip_layered().delta_single(
+        proj, taps, conv_state, q_scale, unit_eps, beta_col, decay, dt_bias,
+        neg_a, gate, norm_w, state, seq_meta, kv_heads, out, eps)
+
+
 def delta_chunk_work(dim, vdim, device):
     """Floats of workspace per (chunk, head); 0 without a chunked form (then
     delta_step takes every sequence)."""

@@ -365,6 +365,38 @@ class TestRotary:
         assert (y - oracle.rotate_pairs(x, raw)).abs().max() < 1e-5
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,K,V,taps", [
+    (3, 64, 64, 4), (2, 128, 128, 4), (2, 8, 4, 2), (1, 192, 128, 3), (2, 100, 72, 4),
+    (5, 40, 300, 4), (2, 254, 4, 4)])
+@pytest.mark.parametrize("n", [1, 7])
+def test_single_rows_in_one_kernel(H, K, V, taps, n):
+    """Against convolutions and steps apart, which have the same inputs; sequences that
+    begin and others, slots that none has."""
+    run, C = ("cuda", torch.bfloat16), 2 * H * K + H * V
+    seqs = [(1, 0 if i % 3 == 2 else 5, (i * 3 + 1) % 8) for i in range(n)]
+    m, rows = meta(seqs, run)
+    proj = put(rnd(n, C + H + 8), run)
+    w = rnd(taps, C, seed=1).cuda()
+    conv = put(rnd(8, taps - 1, C, seed=2), run)
+    state = rnd(8, H, K, V, seed=3).cuda()
+    decay, gate = put(rnd(n, H * K, seed=4), run), put(rnd(n, H * V, seed=5), run)
+    bias, neg_a = rnd(H * K, seed=6).cuda(), -rnd(H, seed=7).abs().cuda()
+    norm = rnd(V, seed=8).cuda()
+    outs = [put(torch.full((n, H * V), 7.0), run) for _ in range(2)]
+    convs, states = [conv, conv.clone()], [state, state.clone()]
+    q, k, v = ops.delta_prep(proj, w, convs[0], rows, m, False, H, H, K, V, 0.3, 1e-6)
+    ops.delta_step(q, k, v, proj, C + 3, decay, bias, neg_a, gate, norm, states[0], m,
+                   n, outs[0], 1e-5)
+    assert ops.delta_single(proj, w, convs[1], 0.3, 1e-6, C + 3, decay, bias, neg_a,
+                            gate, norm, states[1], m, H, outs[1], 1e-5)
+    assert torch.equal(*convs)
+    # sums of K + V products in 32 bits in another order; then rounding to bf16
+    torch.testing.assert_close(states[1], states[0], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(outs[1].float(), outs[0].float(), rtol=2 ** -7,
+                               atol=1e-4)
+
+
 @pytest.mark.parametrize("run", RUNS)
 class TestLatentPrep:
     @pytest.mark.parametrize("q_rank,kv_rank,rot", [(14, 18, 4), (40, 48, 8),
