@@ -296,17 +296,24 @@ int lds_linear_rows_parts(int M, int N, int K) {
 }
 
 // The same where the sum of the parts is a launch of its own (3 to 5 us): one part of
-// short K, or of as many channels as K is long. Up to 64 rows, one part / parts and their
-// sum: 1536 -> 1024, 1 row 5.8 / 6.3, 50 rows 7.7 / 8.2; 2048 -> 2048 6.8 / 7.0, 9.3 / 9.8;
-// 3072 -> 3072 9.0 / 9.4, 12.6 / 12.1; 4096 -> 4096 11.6 / 11.8, 16.0 / 13.5, -> 6144 13.9
-// / 14.1, 18.0 / 16.3, -> 8192 16.7 / 17.8, 19.6 / 20.0, -> 2048 10.8 / 9.0; 6144 -> 8192
-// 21.8 / 23.3, 27.0 / 26.3; 8192 -> 8192 27.0 / 31.7, 33.8 / 34.7.
+// short K, or of many channels, the more of them the more rows there are. One part /
+// parts and their sum, in us:
+//                     1 row        16 rows      32 rows      50 rows
+//   1536 -> 1024      4.4 /  6.2    4.8 /  6.8   5.7 /  7.1   6.6 /  8.2
+//   2048 -> 4096      5.8 /  8.8    6.2 /  9.6   7.2 / 10.4   8.5 / 12.4
+//   3072 -> 2048      6.1 /  7.8    6.8 /  8.5   8.8 /  9.2  10.4 / 10.2
+//   4096 -> 1024      7.0 /  7.7    7.5 /  8.6  10.6 /  9.0  12.6 / 10.1
+//   4096 -> 4096      8.7 / 11.6    9.3 / 12.2  11.6 / 12.5  13.8 / 13.6
+//   4096 -> 8192     15.6 / 17.7   15.9 / 18.7  17.4 / 19.0  19.0 / 20.0
+//   8192 -> 2048     11.5 / 12.1   12.6 / 12.9  18.7 / 13.6  22.5 / 14.6
+//   8192 -> 8192     25.7 / 31.5   26.3 / 32.3  26.8 / 33.2  31.7 / 34.3
 int lds_linear_plain_parts(int M, int N, int K) {
   const int parts = lds_linear_rows_parts(M, N, K);
+  if (M > ROWS || N > 64 * ROUND || K > 8192) return parts;
   const bool one =
-      M <= ROWS && N <= 64 * ROUND &&
-      (K <= 1536 || (K <= 2048 && N >= 2048) ||
-       (K <= 8192 && N >= K && (M <= 32 || K <= 3072 || N >= 8192)));
+      K <= 2048 || (M <= 16   ? K <= 4096 || N >= 2048
+                    : M <= 32 ? N >= (K <= 4096 ? 2048 : 6144)
+                              : N >= (K <= 3072 ? 3072 : 8192));
   return one ? 1 : parts;
 }
 
