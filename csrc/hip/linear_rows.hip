@@ -2,12 +2,12 @@
 // for up to 64 rows, and which product goes where. Others of up to 256 rows go to
 // linear_tiles.hip.
 //
-// The weights' bytes are what counts. A workgroup has all rows of x against 128 rows
-// of w, or 64 where those of 128 leave compute units idle, by the loop of rows_core.h,
-// and K is split until the workgroups make up a round of the 256 compute units.
+// The weights' bytes are what counts. A workgroup has all rows of x against 128 rows of
+// w by the loop of rows_core.h, and K is split until the workgroups make up a round of
+// the 256 compute units; or K is one part, and the rows of w are dealt out in even
+// rounds, 16 to 128 to a workgroup. Where K is split, and by whole blocks of 128,
 // linear_tiles.hip adds up in the same order, so a row comes out the same, to the bit,
-// whichever of the two took it: as the one row of a decode step or within a short
-// prompt.
+// whichever of the two took it: as the one row of a decode step or within a short prompt.
 //
 // Measured, cold weights, without the sum of the parts; before: up to 16 rows weights
 // straight to registers, x through LDS, above 128 bytes of a row at a time: 1 row,
