@@ -445,6 +445,20 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
   }
 }
 
+// Threads along a row of the state, 4 channels each, and its rows per thread
+int state_lanes(int V) {
+  int lanes = 1;
+  while (lanes * 4 < V) lanes *= 2;
+  return lanes;
+}
+
+int state_rows(int K, int V) {
+  const int groups = NT / state_lanes(V);
+  return (K + groups - 1) / groups;
+}
+
+constexpr int SINGLE_ROWS = 32;      // of delta_single; delta_step has a form of 64
+
 }  // namespace
 
 extern "C" {
@@ -504,10 +518,8 @@ hipError_t lds_delta_step(int f32, const float* q, const float* k,
                           int KH, int H, int K, int V, float eps,
                           hipStream_t stream) {
   if (n_seqs == 0) return hipSuccess;
-  int lanes_v = 1;
-  while (lanes_v * 4 < V) lanes_v *= 2;
-  if (lanes_v > NT || K > 512) return hipErrorInvalidValue;
-  const int groups = NT / lanes_v, need = (K + groups - 1) / groups;
+  if (V > 4 * NT || K > 512) return hipErrorInvalidValue;
+  const int lanes_v = state_lanes(V), need = state_rows(K, V);
   int rpt = 1;
   while (rpt < need) rpt *= 2;
   const dim3 grid(H, n_seqs);
@@ -545,7 +557,7 @@ hipError_t lds_delta_step(int f32, const float* q, const float* k,
 // Whether lds_delta_single takes the sizes
 int lds_delta_single_ok(int f32, int KH, int H, int K, int V, int n_taps) {
   return !f32 && KH == H && V % 4 == 0 && V >= 4 && 2 * K + V <= 2 * NT &&
-         n_taps >= 2 && n_taps <= 4;
+         state_rows(K, V) <= SINGLE_ROWS && n_taps >= 2 && n_taps <= 4;
 }
 
 // delta_prep and delta_step of sequences of one row each (bf16), in one kernel
@@ -558,9 +570,7 @@ hipError_t lds_delta_single(const void* proj, int64_t pstride, const float* taps
                             int K, int V, float eps, hipStream_t stream) {
   if (n_seqs == 0) return hipSuccess;
   if (!lds_delta_single_ok(0, H, H, K, V, n_taps)) return hipErrorInvalidValue;
-  int lanes_v = 1;
-  while (lanes_v * 4 < V) lanes_v *= 2;
-  const int groups = NT / lanes_v, need = (K + groups - 1) / groups;
+  const int lanes_v = state_lanes(V), need = state_rows(K, V);
   const Conv<short> cv{(const short*)proj, pstride, taps, (short*)conv_state,
                        n_taps, q_scale, unit_eps};
 #define GO(R)                                                                 \
@@ -573,8 +583,7 @@ hipError_t lds_delta_single(const void* proj, int64_t pstride, const float* taps
   if (need <= 4) GO(4);
   else if (need <= 8) GO(8);
   else if (need <= 16) GO(16);
-  else if (need <= 32) GO(32);
-  else return hipErrorInvalidValue;
+  else GO(SINGLE_ROWS);
 #undef GO
   HIP_CHECK_LAST();
   return hipSuccess;

@@ -368,7 +368,7 @@ class TestRotary:
 @pytest.mark.gpu
 @pytest.mark.parametrize("H,K,V,taps", [
     (3, 64, 64, 4), (2, 128, 128, 4), (2, 8, 4, 2), (1, 192, 128, 3), (2, 100, 72, 4),
-    (5, 40, 300, 4), (2, 254, 4, 4)])
+    (5, 40, 300, 4), (2, 254, 4, 4), (2, 64, 384, 4), (2, 128, 256, 4)])
 @pytest.mark.parametrize("n", [1, 7])
 def test_single_rows_in_one_kernel(H, K, V, taps, n):
     """Against convolutions and steps apart, which have the same inputs; sequences that
@@ -395,6 +395,24 @@ def test_single_rows_in_one_kernel(H, K, V, taps, n):
     torch.testing.assert_close(states[1], states[0], rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(outs[1].float(), outs[0].float(), rtol=2 ** -7,
                                atol=1e-4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,K,V", [(2, 100, 300), (1, 160, 160), (2, 65, 260), (1, 96, 320)])
+def test_single_rows_of_other_sizes(H, K, V):
+    """More than 32 rows of the state per thread: left to the kernels apart, nothing
+    is written."""
+    run, C = ("cuda", torch.bfloat16), 2 * H * K + H * V
+    m, _ = meta([(1, 5, 0)], run)
+    proj, conv = put(rnd(1, C + H + 8), run), put(rnd(8, 3, C, seed=2), run)
+    state, out = rnd(8, H, K, V, seed=3).cuda(), put(torch.full((1, H * V), 7.0), run)
+    kept = conv.clone(), state.clone(), out.clone()
+    vecs = [rnd(i, seed=i).cuda() for i in (H * K, H, V)]
+    assert not ops.delta_single(
+        proj, rnd(4, C, seed=1).cuda(), conv, 0.3, 1e-6, C + 3,
+        put(rnd(1, H * K, seed=4), run), vecs[0], vecs[1],
+        put(rnd(1, H * V, seed=5), run), vecs[2], state, m, H, out, 1e-5)
+    assert all(torch.equal(a, b) for a, b in zip(kept, (conv, state, out)))
 
 
 @pytest.mark.parametrize("run", RUNS)

@@ -278,6 +278,23 @@ class TestRealisticSizes:
         close(torch.cat(out), models.expect("realistic", b), run[2], "b")
 
 
+@pytest.mark.parametrize("run", RUNS[2:])
+@pytest.mark.parametrize("dim,vdim", [(160, 160), (96, 320)])
+def test_decode_of_wide_states(models, run, dim, vdim):
+    """Heads whose single rows are convolved and stepped in kernels apart."""
+    name = f"wide-{dim}-{vdim}"
+    folder, cfg, _ = models(name, {
+        "architecture": "Rururax", "vocab": 128, "width": 256,
+        "embedding": {"scale": 16.0}, "norm": {"eps": 1e-6},
+        "layers": [
+            {"type": "channel_delta", "mlp": {"kind": "dense", "ff": 256},
+             "mixer": {"heads": 2, "kv_heads": 2, "dim": dim, "vdim": vdim,
+                       "conv": 4}}]})
+    toks = M.tokens(cfg, 20, 1)
+    close(feed(worker(folder, run), "a", toks, [12] + [1] * 8),
+          models.expect(name, toks), run[2])
+
+
 class TestChunkGroups:
     def test_groups_cover_every_portion_in_order(self):
         P = layered.Portion
