@@ -257,7 +257,7 @@ void delta_step(Tensor q, Tensor k, Tensor v, Tensor proj, int64_t beta_col,
 }
 
 // delta_prep and delta_step of a batch whose sequences have one row each, in one kernel;
-// false where the sizes have none
+// false where the sizes have none, or there are more rows than sequences or fewer
 bool delta_single(Tensor proj, Tensor taps, Tensor conv_state, double q_scale,
                   double unit_eps, int64_t beta_col, Tensor decay, Tensor dt_bias,
                   Tensor neg_a, Tensor gate, Tensor norm_w, Tensor state,
@@ -267,7 +267,8 @@ bool delta_single(Tensor proj, Tensor taps, Tensor conv_state, double q_scale,
   TORCH_CHECK(state.dim() == 4 && proj.dim() == 2 && taps.dim() == 2, "state, proj");
   const int64_t rows = proj.size(0), H = state.size(1), K = state.size(2);
   const int64_t V = state.size(3), n_taps = taps.size(0);
-  if (!lds_delta_single_ok(f32, (int)KH, (int)H, (int)K, (int)V, (int)n_taps))
+  if (!lds_delta_single_ok(f32, (int)KH, (int)H, (int)K, (int)V, (int)n_taps) ||
+      rows != seq_meta.size(0))
     return false;
   const int64_t C = 2 * KH * K + H * V;
   check(taps, at::kFloat, "taps");

@@ -139,7 +139,8 @@ def delta_single(proj, taps, conv_state, q_scale, unit_eps, beta_col, decay,
                  dt_bias, neg_a, gate, norm_w, state, seq_meta, kv_heads, out,
                  eps):
     """delta_prep and delta_step of a batch whose sequences have one row each, in
-    one kernel; False where there is none for the sizes."""
+    one kernel; False where there is none for the sizes or the numbers of rows and
+    sequences differ."""
     return proj.is_cuda and hip_layered().delta_single(
         proj, taps, conv_state, q_scale, unit_eps, beta_col, decay, dt_bias,
         neg_a, gate, norm_w, state, seq_meta, kv_heads, out, eps)

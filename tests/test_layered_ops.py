@@ -398,20 +398,22 @@ def test_single_rows_in_one_kernel(H, K, V, taps, n):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("H,K,V", [(2, 100, 300), (1, 160, 160), (2, 65, 260), (1, 96, 320)])
-def test_single_rows_of_other_sizes(H, K, V):
-    """More than 32 rows of the state per thread: left to the kernels apart, nothing
-    is written."""
-    run, C = ("cuda", torch.bfloat16), 2 * H * K + H * V
-    m, _ = meta([(1, 5, 0)], run)
-    proj, conv = put(rnd(1, C + H + 8), run), put(rnd(8, 3, C, seed=2), run)
-    state, out = rnd(8, H, K, V, seed=3).cuda(), put(torch.full((1, H * V), 7.0), run)
+@pytest.mark.parametrize("H,K,V,seqs", [
+    (2, 100, 300, [1]), (1, 160, 160, [1]), (2, 65, 260, [1]), (1, 96, 320, [1]),
+    (2, 128, 128, [2, 1]), (2, 64, 64, [3])])
+def test_single_rows_of_other_sizes(H, K, V, seqs):
+    """More than 32 rows of the state per thread, or sequences of several rows: left to
+    the kernels apart, nothing is written."""
+    run, C, n = ("cuda", torch.bfloat16), 2 * H * K + H * V, sum(seqs)
+    m, _ = meta([(r, 5, i) for i, r in enumerate(seqs)], run)
+    proj, conv = put(rnd(n, C + H + 8), run), put(rnd(8, 3, C, seed=2), run)
+    state, out = rnd(8, H, K, V, seed=3).cuda(), put(torch.full((n, H * V), 7.0), run)
     kept = conv.clone(), state.clone(), out.clone()
     vecs = [rnd(i, seed=i).cuda() for i in (H * K, H, V)]
     assert not ops.delta_single(
         proj, rnd(4, C, seed=1).cuda(), conv, 0.3, 1e-6, C + 3,
-        put(rnd(1, H * K, seed=4), run), vecs[0], vecs[1],
-        put(rnd(1, H * V, seed=5), run), vecs[2], state, m, H, out, 1e-5)
+        put(rnd(n, H * K, seed=4), run), vecs[0], vecs[1],
+        put(rnd(n, H * V, seed=5), run), vecs[2], state, m, H, out, 1e-5)
     assert all(torch.equal(a, b) for a, b in zip(kept, (conv, state, out)))
 
 
