@@ -275,14 +275,15 @@ __global__ __launch_bounds__(NT, RPT <= 8    ? 4
   };
   T* const kept = CONV ? in_.state + (int64_t)sq.slot * (in_.n_taps - 1) * C : nullptr;
   if constexpr (CONV) {
+    // a sequence without rows has no proj[row0]; a branch here cost 0.5 us of 8.4
+    const T* x = in_.proj + (sq.n > 0 ? sq.row0 : 0) * in_.pstride;
 #pragma unroll
     for (int i = 0; i < CT; ++i) {
       const int c = column(i);
 #pragma unroll
       for (int j = 0; j < TAPS; ++j) {
         cw[i][j] = in_.taps[(int64_t)min(j, in_.n_taps - 1) * C + c];
-        cx[i][j] = j < in_.n_taps - 1 ? kept[(int64_t)j * C + c]
-                                     : in_.proj[sq.row0 * in_.pstride + c];
+        cx[i][j] = j < in_.n_taps - 1 ? kept[(int64_t)j * C + c] : x[c];
       }
     }
   }

@@ -398,6 +398,32 @@ def test_single_rows_in_one_kernel(H, K, V, taps, n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("prior", [0, 5])
+def test_single_rows_beside_a_sequence_without(prior):
+    """A sequence without rows, first row past the end, is no part of it."""
+    run, H, K, V = ("cuda", torch.bfloat16), 3, 64, 64
+    C = 2 * H * K + H * V
+    proj, w = put(rnd(3, C + H + 5), run), rnd(4, C, seed=1).cuda()
+    conv, state = put(rnd(8, 3, C, seed=2), run), rnd(8, H, K, V, seed=3).cuda()
+    decay, gate = put(rnd(3, H * K, seed=4), run), put(rnd(3, H * V, seed=5), run)
+    vecs = [rnd(i, seed=i).cuda() for i in (H * K, H, V)]
+
+    def step(n, seqs):
+        c, s, out = conv.clone(), state.clone(), put(torch.full((n, H * V), 7.0), run)
+        m = torch.tensor(seqs, dtype=torch.int32, device="cuda")
+        assert ops.delta_single(proj[:n], w, c, 0.3, 1e-6, C, decay[:n], vecs[0], vecs[1],
+                                gate[:n], vecs[2], s, m, H, out, 1e-5)
+        return c, s, out
+    two = [[0, 1, 5, 3], [1, 1, 0, 6]]
+    want = step(2, two)
+    got = step(3, two + [[3, 0, prior, 1]])
+    if not prior:
+        want[1][1] = 0               # it begins: its state, as delta_step leaves it
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert torch.equal(got[2][:2], want[2]) and (got[2][2] == 7).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,K,V,seqs", [
     (2, 100, 300, [1]), (1, 160, 160, [1]), (2, 65, 260, [1]), (1, 96, 320, [1]),
     (2, 128, 128, [2, 1]), (2, 64, 64, [3])])
