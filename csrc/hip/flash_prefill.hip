@@ -178,6 +178,14 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
   auto step = [&](int tile0, auto buf_) {
     constexpr int buf = decltype(buf_)::value;
     lds_barrier();
+    // The last tile's values past the end count as 0: bf16 ones may be infinite, and a
+    // probability of 0 makes no 0 of that. (As they are put: 225 -> 234 us, 4000 rows.)
+    if (sizeof(CT) == 2 && tile0 + KVBLK > kv_end_wg) {
+      const int n = kv_end_wg - tile0;
+      for (int i = n * 16 + tid; i < KVBLK * 16; i += NW * WAVE)
+        *(short8*)((char*)lds[buf][1] + i * 16) = (short8){0, 0, 0, 0, 0, 0, 0, 0};
+      lds_barrier();
+    }
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       const int sub0 = tile0 + 32 * half;

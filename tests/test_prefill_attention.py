@@ -134,6 +134,29 @@ def test_long_tables_stage_through_registers():
     _close(ext.flash_prefill(*args[:3], wide, *args[4:]), want)
 
 
+@pytest.mark.parametrize("bs", [1, 16])
+@pytest.mark.parametrize("seqs", [[(1, 0)], [(3, 90), (64, 1)], [(150, 40), (1, 300)]])
+def test_an_infinite_value_through_registers(seqs, bs):
+    """The last key of each prompt has infinite values: infinity for its last query,
+    which sees it, however far the tile goes on behind it."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    args, want = _case(seqs, 4, 2, bs, False, D ** -0.5)
+    q, kc, vc, tables = args[:4]
+    last, at = [], 0
+    for i, (n, prior) in enumerate(seqs):
+        t = n + prior - 1
+        vc[tables[i, t // bs].long(), :, t % bs, 5] = torch.inf
+        vc[tables[i, t // bs].long(), :, t % bs, 100] = -torch.inf
+        at += n
+        last.append(at - 1)
+    wide = torch.zeros(len(seqs), 1025, dtype=torch.int32, device="cuda")
+    wide[:, :tables.shape[1]] = tables
+    got = ext.flash_prefill(q, kc, vc, wide, *args[4:])[last]
+    assert (got[..., 5] == torch.inf).all() and (got[..., 100] == -torch.inf).all()
+    rest = [c for c in range(D) if c not in (5, 100)]
+    _close(got[..., rest], [x[last][..., rest] for x in want])
+
+
 @pytest.mark.parametrize("seqs,qpg,kvh", [
     ([(300, 0)], 4, 8), ([(400, 300)], 4, 8), ([(100, 40)] * 4, 4, 8),
     ([(20, 300)] * 12, 4, 8), ([(250, 0)], 8, 8), ([(900, 0)], 4, 8),
