@@ -206,10 +206,11 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   const int col = lane % 16, g = lane / 16;
 
   if (SPLIT && t_begin >= seq_len) {
-    // empty partition: publish l=0 so the combiner skips it
+    // empty partition: the combiner skips what has this maximum (others have NEG at
+    // least)
     if (tid < qpg) {
       float* ml = part_ml + ((group * np + part) * qpg + tid) * 2;
-      ml[0] = NEG;
+      ml[0] = -INFINITY;
       ml[1] = 0.f;
     }
     return;
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
         ml[1] = sum;
       }
     } else {
-      w_.out[(group * qpg + h) * D + d] = f32_to_bf16(sum > 0.f ? s / sum : 0.f);
+      w_.out[(group * qpg + h) * D + d] = f32_to_bf16(seq_len > 0 ? s / sum : 0.f);
     }
   }
 }
@@ -453,11 +454,12 @@ __global__ __launch_bounds__(D) void decode_combine_kernel(
   const int64_t first = group * np * qpg + h;
   if (d < WAVE) {
     const float* ml = part_ml + (first + (int64_t)min(d, np - 1) * qpg) * 2;
-    const float m = d < np ? ml[0] : NEG, l = d < np ? ml[1] : 0.f;
+    const float m = d < np ? ml[0] : -INFINITY;
+    const bool empty = m == -INFINITY;
     const float top = wave_reduce_max(m);
-    const float w = l > 0.f ? __builtin_amdgcn_exp2f(m - top) : 0.f;
-    const float sum = wave_reduce_sum(w == 0.f ? 0.f : w * l);
-    weight[d] = w == 0.f ? 0.f : w / sum;
+    const float w = empty ? 0.f : __builtin_amdgcn_exp2f(m - top);
+    const float sum = wave_reduce_sum(empty ? 0.f : w * ml[1]);   // NaN stays NaN
+    weight[d] = empty ? 0.f : w / sum;
   }
   __syncthreads();
   float o = 0.f;

@@ -174,3 +174,25 @@ def test_running_maximum_far_apart():
     want = (s.softmax(-1) @ v).view(1, -1, D).cpu()
     _close(dispatch.paged_attention(*args, D ** -0.5, 600), want)
     _close(dispatch.paged_attention(*args, D ** -0.5), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("waves", [4, 8])
+def test_scores_that_are_no_numbers(fp8, waves):
+    """A key that is no number leaves none for the heads that see it, in one part and
+    in several; other sequences and heads keep theirs, and one without tokens has 0."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    lens, qpg, bs = [700, 3, 0, 257, 33], 4, 16
+    args, want = _case(lens, qpg, bs, fp8)
+    kc, bt = args[1], args[3].cpu()
+    for i, t in ((0, 650), (1, 1), (3, 256)):
+        kc[int(bt[i, t // bs]), 1, t % bs, 9] = float("nan")
+        want[i, qpg:2 * qpg] = float("nan")
+
+    def same(got):
+        torch.testing.assert_close(got.double().cpu(), want, rtol=2 ** -8,
+                                   atol=1e-4, equal_nan=True)
+    same(ext.paged_attention(*args, D ** -0.5, waves=waves))
+    for parts, part in [(3, 256), (8, 96)]:
+        same(ext.paged_attention_split(*args, parts, part, D ** -0.5, waves=waves))

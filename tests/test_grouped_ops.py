@@ -301,6 +301,45 @@ def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
     assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("sink", [0.0, None])
+@pytest.mark.parametrize("ctxs", [[40, 257, 1, 600], [3, 2000], [33] * 90])
+def test_scores_that_are_no_numbers(D, sink, ctxs):
+    """A key that is no number or infinite leaves no number for the heads that see it;
+    keys that are all infinitely far leave none, or a sink all. Other heads and rows
+    keep theirs."""
+    run, G, rep = ("cuda", torch.bfloat16), 3, 4
+    H, n = rep * G, len(ctxs)
+    cache, tables, kv = paged(run, G, D, D, ctxs)
+    proj = put(rnd(n, H * D + 2 * G * D, seed=3), run)
+    proj[:, 0:H * D:D] = 1.0                  # channel 0 of all queries
+    table = tables.cpu()
+
+    def key(i, t, g, x):
+        cache[int(table[i, t // BS]), g, t % BS, 0] = x
+    key(0, ctxs[0] // 2, 0, float("nan"))
+    key(1, ctxs[1] - 1, 1, float("inf"))
+    for t in range(ctxs[-1]):
+        key(n - 1, t, 2, -float("inf"))
+    pos = torch.tensor([c - 1 for c in ctxs], dtype=torch.int32, device="cuda")
+    seq = torch.arange(n, dtype=torch.int32, device="cuda")
+    out = put(torch.full((n, H * D), 7.0), run)
+    ops.grouped_decode(proj, cache, pos, seq, tables, n, H, D, D ** -0.5, sink, max(ctxs),
+                       out)
+    got, q = f64(out).view(n, G, rep, D), f64(proj)[:, :H * D].view(n, H, D)
+    assert got[0, 0].isnan().all() and got[1, 1].isnan().all()
+    if sink is not None:
+        assert (got[-1, 2] == 0).all()
+    elif D == 128:
+        assert got[-1, 2].isnan().all()
+    want = torch.stack([expected(q[i], *kv[i], c - 1, D ** -0.5, sink)
+                        for i, c in enumerate(ctxs)]).view(n, G, rep, D)
+    for i, g in ((0, 0), (1, 1), (n - 1, 2)):
+        got[i, g] = want[i, g] = 0
+    close(got, want, run, f32=1e-5)
+
+
 # ---- experts ----------------------------------------------------------------
 @pytest.mark.parametrize("run", RUNS)
 @pytest.mark.parametrize("T,K,E,top", [
