@@ -343,8 +343,10 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   }
   float4v acc[CT][MT];
   const int steps = (K + rows_core::KS - 1) / rows_core::KS;
-  Core::run(ring, wave, lane, w_from, x_from, 0, K, steps,
-            uint32_t(i) * BN / 128 * 3 % uint32_t(steps), wave * 16 < p.width, acc);
+  // by the expert, not its tile's rank: a row's sums do not hang on what others chose
+  const uint32_t first = uint32_t(tile.x * blocks + i % blocks) * BN / 128 * 3;
+  Core::run(ring, wave, lane, w_from, x_from, 0, K, steps, first % uint32_t(steps),
+            wave * 16 < p.width, acc);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = (wave / Core::WC * MT + t) * 16 + col;

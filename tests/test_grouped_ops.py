@@ -471,6 +471,24 @@ def test_experts_of_few_pairs(K, F, pairs):
     close(out, want, run, bf16=2e-2)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [8, 40, 90, 180])
+def test_experts_of_a_row_whatever_others_chose(T):
+    """Tiles of 16, 32 and 64 pairs: the first rows' bits, where the other rows have
+    all experts and where they have few."""
+    run, E, K, F = ("cuda", torch.bfloat16), 8, 1024, 776
+    up = put(rnd(E, F, K, seed=2, scale=K ** -0.5), run)
+    down = put(rnd(E, K, F, seed=3, scale=F ** -0.5), run)
+    h, wt = put(rnd(T, K), run), torch.full((T, 2), 0.5, device="cuda")
+    outs = []
+    for low in (0, 4, 6):
+        ids = torch.arange(T)[:, None] % (8 - low) + torch.tensor([low, low + 1])
+        ids[:4] = torch.tensor([5, 7])
+        out = ops.experts(h, (ids % 8).int().cuda(), wt, up, down, "relu_squared")
+        outs.append(out[:8])       # four rows of two pairs
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 @GPU
 @pytest.mark.parametrize("D,V", [(64, 64), (128, 128), (192, 128), (64, 256)])
 @pytest.mark.parametrize("bs", [1, 5, 64])
