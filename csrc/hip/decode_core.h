@@ -196,7 +196,8 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   const int share = w_.part_tokens ? w_.part_tokens
                                    : ((seq_len + np - 1) / np + 31) / 32 * 32;
   const int t_begin = SPLIT ? part * share : 0;
-  const int t_end = SPLIT ? min(seq_len, t_begin + share) : seq_len;
+  // (the last part takes what is left, whatever the longest was said to be)
+  const int t_end = SPLIT && part + 1 < np ? min(seq_len, t_begin + share) : seq_len;
   float* const part_o = w_.part_o;
   float* const part_ml = w_.part_ml;
 

@@ -9,11 +9,11 @@ hipError_t lds_store_heads_parts(const float*, int, int, int, const int64_t*,
                                  void*, void*, int64_t, int, int, int, int,
                                  hipStream_t);
 int lds_grouped_decode_ok(int, int, int64_t);
-int lds_grouped_decode_parts(int, int, int, int, int, int);
+int lds_grouped_decode_parts(int, int, int, int, int, int, int);
 hipError_t lds_grouped_decode(const void*, int64_t, const void*,
                               const int32_t*, const int32_t*, const int32_t*,
                               void*, float*, float*, int, int, int, int, int,
-                              int, int, int, int, float, int, float,
+                              int, int, int, int, int, float, int, float,
                               hipStream_t);
 int lds_grouped_prefill_ok(int, int, int, int64_t);
 hipError_t lds_grouped_prefill(const void*, int64_t, const void*,
@@ -111,17 +111,19 @@ void plain_rows(const Heads& s, const Tensor& proj, const Tensor& cache,
 
 // proj [rows, >= H D], queries first; cache [NB, G, bs, D + V]; the first n
 // rows of out [rows, H V]. bf16 in tiles where the sizes allow it, else (or
-// if `plain`) row by row.
+// if `plain`) row by row. core_parts, part_tokens: parts of heads that decode_core.h takes.
 void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                     Tensor row_seq, Tensor block_tables, int64_t n, int64_t H,
                     int64_t D, double scale, OptFloat sink, int64_t max_ctx,
-                    Tensor out, bool plain) {
+                    Tensor out, bool plain, int64_t core_parts,
+                    int64_t part_tokens) {
   const Heads s = heads(proj, cache, H, D);
   same_act(out, s.f32, "out");
   sized(out, {s.rows, H * s.V}, "out");
   check_rows(positions, row_seq, 0, n);
   check(block_tables, at::kInt, "block_tables");
-  TORCH_CHECK(n >= 0 && n <= s.rows, "n");
+  TORCH_CHECK(n >= 0 && n <= s.rows && part_tokens >= 0 && part_tokens % 32 == 0 &&
+                  part_tokens < (1 << 24), "n, part_tokens");
   if (s.f32 || plain ||
       !lds_grouped_decode_ok((int)D, (int)s.V, proj.size(1))) {
     plain_rows(s, proj, cache, positions, row_seq, block_tables, 0, n, scale,
@@ -130,7 +132,8 @@ void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
   }
   if (n == 0) return;
   const int parts = lds_grouped_decode_parts((int)n, (int)H, (int)s.G, (int)D,
-                                             (int)s.V, (int)max_ctx);
+                                             (int)s.V, (int)max_ctx,
+                                             (int)core_parts);
   auto f = proj.options().dtype(at::kFloat);
   Tensor po, ml;
   if (parts > 1) {
@@ -143,7 +146,7 @@ void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                 parts > 1 ? fp(po) : nullptr, parts > 1 ? fp(ml) : nullptr,
                 (int)n, (int)H, (int)s.G, (int)D, (int)s.V,
                 (int)block_tables.size(1), (int)s.bs, (int)max_ctx, parts,
-                (float)scale,
+                (int)part_tokens, (float)scale,
                 sink.has_value(), (float)sink.value_or(0.), cur_stream()),
             "grouped_decode");
 }

@@ -412,19 +412,13 @@ int lds_grouped_decode_ok(int D, int V, int64_t q_stride) {
 // rows 185 (199), 60 of 300 18.2 (20.1), one of 777 9.3 (10.9).
 static bool in_core(int D, int V, int rep) { return D == 128 && V == 128 && rep <= 8; }
 
-int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx) {
+// Parts of a row's context; core_parts: where decode_core.h takes the heads, by
+// decode_parts in ops/dispatch.py
+int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx,
+                             int core_parts) {
   Decode d{};
   d.rep = H / G;
-  if (in_core(D, V, d.rep)) {
-    // As for the uniform decoder (decode_parts in ops/dispatch.py, where it was measured):
-    // one part takes 3 us and as long as a workgroup walks or its bytes take, several 8.5
-    // and their bytes; from 200 groups on it is one.
-    const int groups = n * G;
-    const float walk = max_ctx * 12.5e-3f, mb = groups * 0.8f * max_ctx * 512e-6f;
-    if (groups >= 200 || 3.f + fmaxf(walk, mb / 4.9f) <= 8.5f + mb / 5.2f) return 1;
-    const int parts = (511 + groups) / groups, most = (max_ctx + 255) / 256;
-    return parts < most ? parts < 64 ? parts : 64 : most < 64 ? most : 64;
-  }
+  if (in_core(D, V, d.rep)) return core_parts < 1 ? 1 : core_parts < 64 ? core_parts : 64;
   d.SW = d.v0 = D;
   d.W = D + V;
   d.R = V;
@@ -435,15 +429,16 @@ int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx) {
 }
 
 // q: first query of row 0, rows q_stride apart; cache [NB, G, bs, D + V];
-// out [rows, H V]
+// out [rows, H V]; part_tokens (decode_core.h): 0 or a multiple of 32
 hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
                               const void* cache, const int32_t* positions,
                               const int32_t* row_seq,
                               const int32_t* block_tables, void* out,
                               float* part_o, float* part_ml, int n, int H,
                               int G, int D, int V, int max_blocks, int bs,
-                              int max_ctx, int parts, float scale, int has_sink,
-                              float sink, hipStream_t stream) {
+                              int max_ctx, int parts, int part_tokens,
+                              float scale, int has_sink, float sink,
+                              hipStream_t stream) {
   if (!lds_grouped_decode_ok(D, V, q_stride)) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
   if (in_core(D, V, H / G)) {
@@ -452,7 +447,8 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
     const decode::Work<short> w{
         (const short*)q, q_stride, keys, keys + D, G * head, head, block_tables,
         positions, row_seq, 1, max_blocks, bs, (short*)out, part_o, part_ml, G,
-        H / G, 0, 0, scale, sink * LOG2E, has_sink};
+        H / G, part_tokens, part_tokens > 0 && n % 2 == 0, scale, sink * LOG2E,
+        has_sink};
     // short rows leave half of 8 waves without a tile
     const int waves = max_ctx <= 256 ? 4 : 8;
     if (parts > 64) return hipErrorInvalidValue;

@@ -797,7 +797,7 @@ class EngineWorker:
         portions.sort(key=lambda p: len(p[1]) > SHORT)
         nd, T = len(decode_ids), len(decode_ids)
         parts = {k: [] for k in ("ids", "pos", "slot", "seq", "meta", "bt")}
-        max_ctx, rows_t = 0, None
+        max_ctx, sum_ctx, rows_t = 0, 0, None
         if nd:
             rows_t, ids, pos, slot, bt, _ = self._decode_rows(decode_ids)
             seq = torch.arange(nd, dtype=torch.int32, device=dev)
@@ -809,7 +809,8 @@ class EngineWorker:
             parts["meta"].append(torch.stack(
                 [seq, torch.ones_like(seq), pos,
                  self.dstate.state_slots.index_select(0, rows_t)], 1))
-            max_ctx = max(self.mgr.seq_lens[r] for r in decode_ids)
+            lens = [self.mgr.seq_lens[r] for r in decode_ids]
+            max_ctx, sum_ctx = max(lens), sum(lens)
         firsts, long, step_rows, step_seqs = [], [], nd, nd
         if portions:
             host = {k: [] for k in ("ids", "pos", "slot", "seq", "meta")}
@@ -834,6 +835,7 @@ class EngineWorker:
                 else:
                     step_rows, step_seqs = T + n, nd + i + 1
                     max_ctx = max(max_ctx, start + n)
+                    sum_ctx += n * start + n * (n + 1) // 2
                 T += n
             for k, arrays in host.items():
                 parts[k].append(torch.from_numpy(
@@ -849,7 +851,8 @@ class EngineWorker:
             slot_mapping=join("slot"), row_seq=join("seq"),
             seq_meta=join("meta"), block_tables=join("bt"),
             n_step_seqs=step_seqs, n_step_rows=step_rows,
-            multi_row=T > nd + len(portions), max_ctx=max_ctx, long=long,
+            multi_row=T > nd + len(portions), max_ctx=max_ctx,
+            mean_ctx=sum_ctx / max(1, step_rows), long=long,
             logit_rows=None if rows is None else torch.tensor(
                 rows, dtype=torch.int64).to(dev, non_blocking=True))
 

@@ -112,6 +112,7 @@ class LayeredBatch:
     max_ctx: int                    # longest context among the step rows
     long: List[Portion]
     logit_rows: Optional[torch.Tensor] = None   # None: every row
+    mean_ctx: Optional[float] = None            # mean context of step rows, if known
 
 
 class ChannelDelta:
@@ -258,7 +259,8 @@ class GroupedAttention:
         if n:
             ops.grouped_decode(proj, cache, batch.positions, batch.row_seq,
                                batch.block_tables, n, s.heads, s.dim,
-                               s.scale, s.sink, batch.max_ctx, out)
+                               s.scale, s.sink, batch.max_ctx, out,
+                               mean_ctx=batch.mean_ctx)
         if n < T:
             ops.grouped_prefill(proj, cache, batch.positions, batch.row_seq,
                                 batch.block_tables, n, batch.seq_meta,

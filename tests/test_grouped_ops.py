@@ -6,6 +6,7 @@ import torch
 
 import sezazen_oracle as oracle
 from llm_d_inference_scheduler_amd.ops import layered as ops
+from llm_d_inference_scheduler_amd.ops.dispatch import decode_parts
 from test_layered_ops import F64, GPU, RUNS, close, f64, meta, put, rnd
 
 F32 = ("", torch.float32)
@@ -299,6 +300,32 @@ def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
                         for i, c in enumerate(ctxs)])
     # probabilities have 24 bits: 32-bit scores and sums, and the result's rounding
     assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,rep,ctxs", [
+    (8, 2, [80 + 11 * i % 90 for i in range(14)] + [1421]),      # 5 parts
+    (4, 4, [9 + 7 * i % 300 for i in range(34)] + [1770]),       # 4
+    (2, 1, [1 + 37 * i % 90 for i in range(103)] + [2900])])     # 10: by the longest
+@pytest.mark.parametrize("sink", [0.0, None])
+def test_decode_of_rows_far_apart(G, rep, ctxs, sink):
+    """One long row among short ones is in parts where the mean is known."""
+    run, D = ("cuda", torch.bfloat16), 128
+    H, n, mean = rep * G, len(ctxs), sum(ctxs) / len(ctxs)
+    assert decode_parts(n * G, max(ctxs), mean)[0] > decode_parts(n * G, max(ctxs))[0]
+    cache, tables, kv = paged(run, G, D, D, ctxs)
+    proj = put(rnd(n, H * D, seed=3), run)
+    pos = torch.tensor([c - 1 for c in ctxs], dtype=torch.int32, device="cuda")
+    seq = torch.arange(n, dtype=torch.int32, device="cuda")
+    q = f64(proj).view(n, H, D)
+    want = torch.stack([expected(q[i], *kv[i], c - 1, D ** -0.5, sink)
+                        for i, c in enumerate(ctxs)])
+    for said in (max(ctxs), max(ctxs) - 300):      # the longest, or less
+        out = put(torch.full((n, H * D), 7.0), run)
+        ops.grouped_decode(proj, cache, pos, seq, tables, n, H, D, D ** -0.5, sink, said,
+                           out, mean_ctx=mean)
+        # as test_decode_of_heads_of_128
+        assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
 
 
 @pytest.mark.gpu

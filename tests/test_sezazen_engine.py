@@ -81,6 +81,28 @@ def best_by_oracle(cfg, weights, prompt, made, limit):
             8 * limit * float(row.pow(2).mean().sqrt()), i
 
 
+def test_mean_context_of_a_batch(models, monkeypatch):
+    """Of rows that decode and of short portions' rows, as attention is told it."""
+    from llm_d_inference_scheduler_amd.ops import layered as ops
+    w, told = worker(models("tiled")[0], CPU), []
+    real = ops.grouped_decode
+
+    def spy(proj, cache, positions, *args, mean_ctx=None, **kw):
+        n = args[2]
+        told.append((mean_ctx, float((positions[:n] + 1).double().mean())))
+        return real(proj, cache, positions, *args, mean_ctx=mean_ctx, **kw)
+    monkeypatch.setattr(ops, "grouped_decode", spy)
+    toks = M.tokens(models("tiled")[1], 150)
+    w.forward_spans([TokenSpan("a", toks[:100], [99])])
+    assert not told
+    w.forward_spans([TokenSpan("a", toks[100:101], [0]), TokenSpan("b", toks[:5], [4]),
+                     TokenSpan("c", toks, [149])])
+    assert told and all(mean == want for mean, want in told)
+    del told[:]
+    generate(w, {"d": toks[:40], "e": toks[:7]}, 4)
+    assert told and all(mean == pytest.approx(want) for mean, want in told)
+
+
 @pytest.mark.parametrize("run", RUNS)
 @pytest.mark.parametrize("name", list(CONFIGS))
 class TestAgainstOracle:
