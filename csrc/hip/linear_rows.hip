@@ -276,6 +276,35 @@ int workgroups(int M, int N) {
   return (N + width - 1) / width;
 }
 
+// Whether a gated product that fills no round of the chip is faster here, up to 64 rows,
+// than as a product and its activation, by the blocks of 64 channels that K takes: the
+// more rows, the fewer groups of waves share K out. own: that product is one of this
+// file, not the library's. Here / there:
+//                  16 rows   17     32     33     64
+//   2560 x  256     0.78    0.92   0.93   0.99   1.03
+//   2800 x  192     0.79    0.87   0.86   0.86   0.97
+//   3072 x  256     0.81    1.00   0.96   1.05   1.07
+//   3392 x  520     0.81    1.09   1.05   1.14   1.10
+//   3840 x 1296     0.82    0.83   0.84   1.03   0.94
+//   4096 x   64     0.83    1.15   1.10   1.22   1.24
+//   4096 x  768     0.80    0.92   0.87   1.05   1.00
+//   4712 x 2336     0.89    0.53   0.57   0.67   0.70 (library)
+//   5120 x 2048     0.87    0.84   0.86   1.00   1.06
+//   5120 x 4096     0.90    0.90   0.89   0.94   0.94
+//   7168 x 3072     0.92    0.91   0.92   1.00   1.03
+//   8192 x 4096     0.98    1.10   1.06   1.04   1.03
+bool enough_blocks(int M, int blocks, int K, bool own) {
+  if (M <= 16)
+    return K <= 4096 || (K <= 6144 && blocks >= 32) || (K <= 8192 && blocks >= 48);
+  if (M <= 32)
+    return K <= 3072 || (K <= 4096 && blocks >= 12) || (K <= 6144 && blocks >= 32) ||
+           (K < 8192 && blocks >= 48);
+  return K <= 2688 || (K < 3072 && blocks >= 2) || (K <= 3072 && blocks >= 8) ||
+         (K <= 4096 && blocks >= 16) || (K <= 4736 && blocks >= 32) ||
+         (K <= 6144 && ((blocks >= 48 && M <= 40) || (blocks >= 32 && !own))) ||
+         (K < 8192 && blocks >= 64);
+}
+
 }  // namespace
 
 extern "C" {
@@ -335,11 +364,7 @@ int lds_linear_plain_parts(int M, int N, int K) {
 //     rounds it is 0.66 to 1.06 times (245 rows, 3584 -> [2 x 28744]: 132 / 118), by
 //     longer K 0.74 to 1.07 (15872 -> [2 x 15456]: 367 / 271);
 //     inside a 4-layer stack of about 180 rows the pass takes 790 / 835. Up to 64
-//     rows need not fill their round, for K from 256 to 4096, or to 8192 of so many
-//     channels that most compute units have some (16 rows, here / library with the
-//     activation: 256 -> [2 x 2304] 4.0 / 12, 2048 -> [2 x 1024] 7.5 / 13, 4096 -> [2 x
-//     512] 11.3 / 17, 64 rows 16.1 / 16.9, 6144 -> [2 x 1536] 16.1 / 14.6, [2 x 2048] 16.9
-//     / 25, 8192 -> [2 x 2048] 21.5 / 18.6, [2 x 3072] 26.2 / 26.6).
+//     rows need not fill their round (enough_blocks; 16 rows, 256 -> [2 x 2304] 4.0 / 12).
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
 //     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
 //     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
@@ -359,7 +384,7 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
   if (M <= ROWS && (gated ? 2 : 1) * N > 128 * 128 && K >= 512 && K <= 10240) return 1;
   if (gated && M <= ROWS && groups <= 256 && K >= 256 &&
-      (K <= 4096 || (K <= 6144 && groups >= 32) || (K <= 8192 && groups >= 48)))
+      enough_blocks(M, groups, K, lds_linear_rows_takes(M, 2 * N, K, 0, 0)))
     return 1;
   if (gated)
     return full && (M <= 192 || (groups <= 256 && K >= 1024 && K <= 8192 &&
