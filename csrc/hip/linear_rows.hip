@@ -276,6 +276,11 @@ int workgroups(int M, int N) {
   return (N + width - 1) / width;
 }
 
+// Whether workgroups fill 7/8 of their rounds
+bool fills(int groups) {
+  return groups * 8 >= (groups + ROUND - 1) / ROUND * ROUND * 7;
+}
+
 // Whether a gated product that fills no round of the chip is faster here, up to 64 rows,
 // than as a product and its activation, by the blocks of 64 channels that K takes: the
 // more rows, the fewer groups of waves share K out. own: that product is one of this
@@ -325,7 +330,9 @@ int lds_linear_rows_parts(int M, int N, int K) {
 }
 
 // The same where the sum of the parts is a launch of its own (3 to 5 us): one part of
-// short K, or of many channels, the more of them the more rows there are. One part /
+// short K, or of many channels, the more of them the more rows there are. From 33 rows
+// on three parts or four that make up their round are faster still where K is long, but
+// four of a power of two, which begin at the same memory channels in every row. One part /
 // parts and their sum, in us:
 //                     1 row        16 rows      32 rows      50 rows
 //   1536 -> 1024      4.4 /  6.2    4.8 /  6.8   5.7 /  7.1   6.6 /  8.2
@@ -336,13 +343,22 @@ int lds_linear_rows_parts(int M, int N, int K) {
 //   4096 -> 8192     15.6 / 17.7   15.9 / 18.7  17.4 / 19.0  19.0 / 20.0
 //   8192 -> 2048     11.5 / 12.1   12.6 / 12.9  18.7 / 13.6  22.5 / 14.6
 //   8192 -> 8192     25.7 / 31.5   26.3 / 32.3  26.8 / 33.2  31.7 / 34.3
+// and their ratio:    17 rows  32 rows            33 rows  48 rows  64 rows
+//   4096 -> 2304       1.14     1.06    5120 ->  8192  1.06  1.08  1.05
+//   3840 -> 2560       1.10     1.00    7680 ->  8192  1.04  1.14  1.13
+//   4096 -> 3072       0.97     0.90    4096 -> 10240  1.07  1.07  1.09
+//   3072 -> 2048       1.02     0.94    6144 -> 10240  1.10  1.04  1.03
+// (8192 -> 9216, whose three parts do not fill their round, takes 42.4 us, 33 rows, the
+// library 38.6.)
 int lds_linear_plain_parts(int M, int N, int K) {
   const int parts = lds_linear_rows_parts(M, N, K);
   if (M > ROWS || N > 64 * ROUND || K > 8192) return parts;
+  const bool round = K >= 4096 && (parts == 3 || (parts == 4 && K % 4096)) &&
+                     (fills(workgroups(M, N) * parts) || (parts == 3 && K >= 8192));
   const bool one =
       K <= 2048 || (M <= 16   ? K <= 4096 || N >= 2048
-                    : M <= 32 ? N >= (K <= 4096 ? 2048 : 6144)
-                              : N >= (K <= 3072 ? 3072 : 8192));
+                    : M <= 32 ? N >= (K <= 3072 ? 2048 : K <= 4096 ? 2816 : 6144)
+                              : N >= (K <= 3072 ? 3072 : 8192) && !round);
   return one ? 1 : parts;
 }
 
@@ -381,7 +397,7 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   if (!gated && parts && lds_linear_rows_parts(M, N, K) > 1) return 1;
   const int n = gated ? 1 : lds_linear_plain_parts(M, N, K);
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
-  const bool full = groups * 8 >= (groups + 255) / 256 * 256 * 7;
+  const bool full = fills(groups);
   if (M <= ROWS && (gated ? 2 : 1) * N > 128 * 128 && K >= 512 && K <= 10240) return 1;
   if (gated && M <= ROWS && groups <= 256 && K >= 256 &&
       enough_blocks(M, groups, K, lds_linear_rows_takes(M, 2 * N, K, 0, 0)))

@@ -24,3 +24,17 @@ EVERY = (1, 16, 17, 24, 32, 33, 48, 64)
 def test_gated(n, k, rows):
     taken = [m for m in EVERY if RULES.lds_linear_rows_takes(m, n, k, 1, 0)]
     assert taken == list(rows)
+
+
+# rows of x by which parts and their sum are slower than one part
+@pytest.mark.parametrize("n,k,rows", [
+    (8, 2048, EVERY), (1024, 4096, (1, 16)), (2048, 3072, EVERY[:5]),
+    (2304, 4096, (1, 16)), (2560, 3840, (1, 16)), (3072, 3072, EVERY),
+    (3072, 4096, EVERY[:5]), (3000, 3992, EVERY[:5]), (2048, 8192, (1, 16)), (4096, 5120, (1, 16)),
+    (8192, 4096, EVERY), (10240, 3584, EVERY), (10240, 4096, EVERY[:5]),
+    (8192, 5120, EVERY[:5]), (8192, 7680, EVERY[:5]), (8192, 8192, EVERY),
+    (8192, 8184, EVERY[:5]),
+    (9216, 4608, EVERY), (9216, 7680, EVERY), (9216, 8192, EVERY[:5]), (10240, 6144, EVERY[:5]), (12800, 8192, EVERY),
+    (16384, 5120, EVERY)])
+def test_one_part(n, k, rows):
+    assert [m for m in EVERY if RULES.lds_linear_plain_parts(m, n, k) == 1] == list(rows)
