@@ -224,7 +224,7 @@ __global__ __launch_bounds__(NW * WAVE, 2) void flash_prefill_kernel(
   st.l = st.join();
 
   // ---- epilogue: out[seq_start+p][qh][dim] = acc / l ----
-  if (active && st.l > 0.f) {
+  if (active) {                             // it sees a key: l is above 0 or no number
     const float inv = 1.f / st.l;
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)

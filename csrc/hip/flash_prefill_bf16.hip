@@ -272,7 +272,7 @@ void flash_prefill_bf16_kernel(
       for (int r = 0; r < 16; ++r)
         o[r] += a * o_sh[((w * (D / 32) + wave) * 16 + r) * WAVE + lane];
     }
-    if (!active || !(l > 0.f)) return;
+    if (!active) return;                            // it sees a key: l > 0 or no number
     const float inv = 1.f / l;
     short* dst = out + q_row * D + wave * 32 + 4 * hi;
 #pragma unroll
@@ -280,7 +280,7 @@ void flash_prefill_bf16_kernel(
       *(uint2*)(dst + 8 * g) = make_uint2(
           pack2(o[4 * g] * inv, o[4 * g + 1] * inv),
           pack2(o[4 * g + 2] * inv, o[4 * g + 3] * inv));
-  } else if (active && st.l > 0.f) {
+  } else if (active) {
     const float inv = 1.f / st.l;
 #pragma unroll
     for (int t = 0; t < D / 32; ++t)

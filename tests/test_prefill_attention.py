@@ -134,6 +134,31 @@ def test_long_tables_stage_through_registers():
     _close(ext.flash_prefill(*args[:3], wide, *args[4:]), want)
 
 
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("keys", [0, 1, 2])
+@pytest.mark.parametrize("pages", [0, 1025])
+def test_scores_that_are_no_numbers(fp8, keys, pages):
+    """A key that is no number leaves none for the rows and heads that see it, and every
+    row is written."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    seqs = [(70, 300), (40, 0), (3, 65)]
+    args, (want, size) = _case(seqs, 4, 2, 16, fp8, D ** -0.5)
+    tables, row = args[3], 0
+    for i, ((n, prior), t) in enumerate(zip(seqs, (350, 0, 67))):
+        args[1][tables[i, t // 16].long(), 1, t % 16, 9] = float("nan")
+        want[row + max(0, t - prior):row + n, 4:] = float("nan")
+        row += n
+    if pages:
+        tables = torch.zeros(3, pages, dtype=torch.int32, device="cuda")
+        tables[:, :args[3].shape[1]] = args[3]
+    for _ in range(3):
+        torch.full_like(args[0], 3.0)          # what an unwritten row would hold
+        got = ext.flash_prefill(*args[:3], tables, *args[4:], keys=keys)
+        none = want.isnan()
+        assert got[none].isnan().all()
+        _close(got[~none], (want[~none], size[~none]))
+
+
 @pytest.mark.parametrize("bs", [1, 16])
 @pytest.mark.parametrize("seqs", [[(1, 0)], [(3, 90), (64, 1)], [(150, 40), (1, 300)]])
 def test_an_infinite_value_through_registers(seqs, bs):
