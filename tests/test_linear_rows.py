@@ -226,10 +226,11 @@ def test_width_of_workgroups(rows, rows_of_w, k):
     w = _draw(rows_of_w, k, seed=rows_of_w, scale=k ** -0.5)
     z = x.double() @ w.double().t()
     _same(ext.linear(x, w), z, 8)
-    for y, want, bits in [(ext.linear32(x, w), z, 16),
-                          (ext.activated_linear(x, w, 1), F.silu(z), 8)]:
-        if y is not None:
-            _same(y, want, bits)
+    _same(ext.linear32(x, w), z, 16)
+    y = ext.activated_linear(x, w, 1)
+    assert (y is not None) == (rows_of_w <= 16384)
+    if y is not None:
+        _same(y, F.silu(z), 8)
     g, u = z.chunk(2, -1)
     y = ext.gated_linear(x, w, 1)
     assert y is not None or k > 4096 or rows_of_w == 1024 and k > 2048
@@ -630,7 +631,10 @@ def test_rope_and_cache(T, qh, kvh, d, bs, norm, fp8, parts):
 @pytest.mark.parametrize("n,k", [(4096, 4096), (264, 1000), (30000, 200),
                                  (60008, 136)])
 def test_rows_come_out_alike(n, k):
-    """One row alone and the same row among up to 256 give the same bits."""
+    """One row alone and the same row among up to 256 give the same bits where K is in
+    parts for the caller to sum, and in gated products of whole blocks. Not so where K is
+    shared out inside a workgroup or parts are summed here (linear, linear32, an
+    activation, narrow gated products): there the shares hang on the number of rows."""
     ext = _ext("_hip_ops")
     x, w = _draw(256, k, seed=1), _draw(n, k, seed=2, scale=k ** -0.5)
     one = ext.linear_parts(x[:1], w)
