@@ -5,15 +5,17 @@
 // The weights' bytes are what counts. A workgroup has all rows of x against 128 rows of
 // w by the loop of rows_core.h, and K is split until the workgroups make up a round of
 // the 256 compute units; or K is one part, and the rows of w are dealt out in even
-// rounds, 16 to 128 to a workgroup. Where K is split, and by whole blocks of 128,
-// linear_tiles.hip adds up in the same order, so a row comes out the same, to the bit,
-// whichever of the two took it: as the one row of a decode step or within a short prompt.
+// rounds, 16 to 128 to a workgroup. Where the parts are left to the caller, and in gated
+// products by whole blocks of 128, linear_tiles.hip adds up in the same order, so a row
+// comes out the same, to the bit, whichever of the two took it: as the one row of a decode
+// step or within a short prompt. Elsewhere how K is shared out, over parts or over groups
+// of waves, hangs on the number of rows, and so do a row's last bits.
 //
 // Measured, cold weights, without the sum of the parts; before: up to 16 rows weights
 // straight to registers, x through LDS, above 128 bytes of a row at a time: 1 row,
-// 4096 -> [2 x 14336] 41.9 us, 5.6 TB/s (43.5; library 58 and the activation), 4096 ->
-// 6144 11.0 (11.9), 14336 -> 4096 21.9 (22.6), 4096 -> 4096 7.5 (8.0), 25600 -> 5120
-// 46.3 (47.9); 30 rows 42.5, 12.0, 23.0, 8.4, 48.4 (45.4, 12.0, 23.2, 8.7, 48.9).
+// 4096 -> [2 x 14336] 42.0 us, 5.6 TB/s (43.7; library 58 and the activation), 4096 ->
+// 6144 10.8 (11.4), 14336 -> 4096 21.7 (22.4), 4096 -> 4096 7.7 (8.4), 25600 -> 5120
+// 46.3 (47.6); 30 rows 42.3, 11.7, 22.7, 8.5, 48.4 (45.7, 11.7, 23.0, 9.1, 48.9).
 #include "rows_core.h"
 
 namespace {
@@ -265,8 +267,8 @@ hipError_t go_rows(const Rows& p, hipStream_t stream) {
 }
 
 // Up to 64 rows come here, up to 32 where K is split, more go to linear_tiles.hip (60
-// rows, here / there: 4096 -> [2 x 14336] 43.6 us / 44.9, 4096 -> 6144 in 5 parts 13.5 /
-// 12.7, 14336 -> 4096 in 8 24.3 / 23.8).
+// rows, here / there: 4096 -> [2 x 14336] 44.0 us / 50.2, 4096 -> 6144 in 5 parts 13.4 /
+// 12.7, 4096 -> 4096 in 8 11.4 / 10.1, 14336 -> 4096 in 8 24.8 / 24.7).
 constexpr int ROWS = 64, SPLIT_ROWS = 32, TILE_ROWS = 256;
 
 // Of one part of K, by which the split and the rule below are reckoned: of 256 rows
