@@ -11,11 +11,11 @@
 // step or within a short prompt. Elsewhere how K is shared out, over parts or over groups
 // of waves, hangs on the number of rows, and so do a row's last bits.
 //
-// Measured, cold weights, without the sum of the parts; before: up to 16 rows weights
-// straight to registers, x through LDS, above 128 bytes of a row at a time: 1 row,
-// 4096 -> [2 x 14336] 42.0 us, 5.6 TB/s (43.7; library 58 and the activation), 4096 ->
-// 6144 10.8 (11.4), 14336 -> 4096 21.7 (22.4), 4096 -> 4096 7.7 (8.4), 25600 -> 5120
-// 46.3 (47.6); 30 rows 42.3, 11.7, 22.7, 8.5, 48.4 (45.7, 11.7, 23.0, 9.1, 48.9).
+// Measured, cold weights, without the sum of the parts; before: weights by way of the L2
+// caches like x (and 128 bytes of a row at a time): 1 row, 4096 -> [2 x 14336] 38.3 us,
+// 6.1 TB/s (41.8, 43.7; library 58 and the activation), 4096 -> 6144 10.4 (11.1, 11.4),
+// 14336 -> 4096 20.2 (22.4, 22.4), 4096 -> 4096 7.5 (7.8, 8.4), 25600 -> 5120 42.1 (47.4,
+// 47.6); 30 rows 39.3, 11.4, 21.5, 8.5, 44.2 (42.3, 12.0, 23.4, 8.7, 49.3).
 #include "rows_core.h"
 
 namespace {

@@ -12,12 +12,21 @@
 #pragma once
 #include "layered/elem.h"
 
+#include <type_traits>
+
 namespace rows_core {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
 constexpr int KS = 128, ROW = KS * 2;          // ROW: bytes of a row in LDS
 constexpr int RING = 3;          // 4 are no faster, 2 up to 15 % slower
+
+// Cache policy (nt) of loads of weights. They are read once, and as other loads they push
+// x and each other's lines on their way out of the L2 caches: 1 row, 4096 -> [2 x 14336]
+// 41.8 us, so 38.3 (6.1 TB/s); 25600 -> 5120 47.4, 42.1; 30 rows 42.3 and 39.3, 49.3 and
+// 44.2. (sc0, or sc0 and sc1, gain a third of that. Weights that fit the 256 MB cache
+// from one pass to the next would lose by it; those of a model do not.)
+constexpr int ONCE = 2;
 
 // what is past the end of K
 __device__ const float4v zeros = {0.f, 0.f, 0.f, 0.f};
@@ -73,21 +82,23 @@ struct RowsCore {
       return k_lo + (s >= steps ? s - steps : s) * KS;
     };
     // 4 rows of K from k on, rows 4 q .. of their kind
-    auto load = [&](const short* from, char* to, int q, int k) {
+    auto load = [&](auto hint, const short* from, char* to, int q, int k) {
       const bool in = k + piece(q * 4 + grp, lane) < k_hi;
       __builtin_amdgcn_global_load_lds(
           (gmem*)(in ? from + k : (const short*)&zeros), (smem*)(to + q * 1024),
-          16, 0, 0);
+          16, 0, decltype(hint)::value);
     };
     auto issue = [&](int s, int buf) {
       const int k = k_of(s);
       if (some)
 #pragma unroll
         for (int j = 0; j < WL; ++j)
-          load(w_from[j], w_ring + buf * W_STEP, wave * WL + j, k);
+          load(std::integral_constant<int, ONCE>{}, w_from[j], w_ring + buf * W_STEP,
+               wave * WL + j, k);
 #pragma unroll
       for (int j = 0; j < XL; ++j)
-        load(x_from[j], x_ring + buf * X_STEP, x_row(wave, j) / 4, k);
+        load(std::integral_constant<int, 0>{}, x_from[j], x_ring + buf * X_STEP,
+             x_row(wave, j) / 4, k);
     };
 
 #pragma unroll
