@@ -371,18 +371,20 @@ int lds_linear_plain_parts(int M, int N, int K) {
 //     41 / 63; 4096 -> 12576: 64 rows 24 / 25, 256 rows 42 / 50. (Above 128 rows
 //     a K below 1600 takes up to 3 us more here, 688 -> 1680, 256 rows 13 / 10;
 //     that it comes out as a single row does is worth it.)
-//   one part, and gated ones (there with their activation): if the workgroups
-//     fill at least 7/8 of their rounds, plain up to 128 rows. 4096 -> 32768: 32 rows
-//     46 / 62, 128 rows 55 / 64, 160 rows 66 / 67; -> 128256 (98 %): 64 rows
-//     182 / 208; 5120 -> 51200 (78 %): 64 rows 110 / 98. 4096 -> [2 x 14336]:
-//     64 rows 44 / 58, 128 rows 53 / 60, 192 rows 65 / 67, 256 rows 69 / 75. From
-//     193 rows on by linear_wide, for K from 1024 on in whole steps, where the
-//     workgroups are one round and K is at most 8192: 1.01 to 1.25 times as fast
-//     over 25 sizes (232 rows, 1024 -> [2 x 14624]: 28 / 35). In two or three
-//     rounds it is 0.66 to 1.06 times (245 rows, 3584 -> [2 x 28744]: 132 / 118), by
-//     longer K 0.74 to 1.07 (15872 -> [2 x 15456]: 367 / 271);
-//     inside a 4-layer stack of about 180 rows the pass takes 790 / 835. Up to 64
-//     rows need not fill their round (enough_blocks; 16 rows, 256 -> [2 x 2304] 4.0 / 12).
+//   one part, and gated ones (there with their activation), up to 64 rows: if the
+//     workgroups fill at least 7/8 of their rounds. 4096 -> 32768: 32 rows 46 / 62; ->
+//     128256 (98 %): 64 rows 182 / 208; 5120 -> 51200 (78 %): 64 rows 110 / 98; 4096 ->
+//     [2 x 14336]: 64 rows 44 / 58. Gated ones need not fill their round (enough_blocks;
+//     16 rows, 256 -> [2 x 2304] 4.0 / 12).
+//   the same of 65 rows and more, ratio of the times over 140 sizes:
+//     one round, of which plain ones fill more than half: 0.63 to 1.0 but for three of
+//     1.05 to 1.08 (143 blocks, 128 rows, K of 5248 the most). 0.95 to 1.0 from a K of
+//     11392 on, so that longer ones stay away. Gated: from 5/8 of the round on 0.64 to
+//     0.97, 105 to 128 blocks 0.9 to 1.25; above 192 rows K of 15872 1.13.
+//     more rounds, 7/8 full: up to 128 rows 0.66 to 1.0, 192 rows 0.79 to 1.04 for K up to
+//     4096 and 0.83 to 1.11 for more; 256 rows 1.07 to 1.22 in two rounds, in three to
+//     five 0.85 to 1.02 for K up to 4224 (128256 x 4096 264 / 300 us), gated 0.88 to 1.13.
+//     Less full ones 1.02 to 1.34.
 //   parts and their sum (3 to 5 us): with full rounds (4096 -> 6144: 64 rows
 //     16 / 18, 160 rows 23 / 28; 8192 -> 5120: 256 rows 40 / 74) unless K is
 //     short (2048 -> 8192: 64 rows 13.3 / 14.0, 128 rows 17.7 / 16.8), else
@@ -400,14 +402,20 @@ int lds_linear_rows_takes(int M, int N, int K, int gated, int parts) {
   const int n = gated ? 1 : lds_linear_plain_parts(M, N, K);
   const int groups = gated ? (N + 63) / 64 : workgroups(M, N) * n;
   const bool full = fills(groups);
+  const bool one_round = M > ROWS && groups <= ROUND && groups * 8 >= ROUND * 5;
   if (M <= ROWS && (gated ? 2 : 1) * N > 128 * 128 && K >= 512 && K <= 10240) return 1;
   if (gated && M <= ROWS && groups <= 256 && K >= 256 &&
       enough_blocks(M, groups, K, lds_linear_rows_takes(M, 2 * N, K, 0, 0)))
     return 1;
   if (gated)
-    return full && (M <= 192 || (groups <= 256 && K >= 1024 && K <= 8192 &&
-                                 K % KS == 0));
-  if (N > 128 * 128) return full && M <= 128;
+    return M <= 192 ? full || one_round
+                    : one_round && K >= 1024 && K <= 8192 && K % KS == 0;
+  if (N > 128 * 128)
+    return M <= ROWS         ? full
+           : groups <= ROUND
+               ? K <= 12288
+               : full && (M <= 128 || (K <= 4096 && (M <= 192 || (groups > 2 * ROUND &&
+                                                                  K >= 1024))));
   if (full) return M <= 64 || K >= 4096;
   return M <= ROWS && (N <= 4096 || n == 1);
 }

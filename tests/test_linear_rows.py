@@ -78,6 +78,33 @@ def test_parts_of_many_steps(rows, n, k, parts):
     assert torch.equal(y[:, -1:], ext.linear_parts(x[-1:], w))
 
 
+@pytest.mark.parametrize("rows", [65, 128, 129, 192, 193, 256])
+@pytest.mark.parametrize("n,k,parts", [
+    (16392, 1024, 1), (20488, 1152, 1), (16392, 1032, 1), (4088, 14336, 8),
+    (9224, 5504, 3), (12576, 3968, 2)])
+def test_whole_lines(rows, n, k, parts):
+    """Ends of groups of 64 rows, of channels, and even and odd numbers of steps of
+    128 of K; a K that is none goes by halves. With parts, the bits of a row alone."""
+    ext = _ext("_hip_ops")
+    x, w = _draw(rows, k, seed=rows), _draw(n, k, seed=n, scale=k ** -0.5)
+    want = x.double() @ w.double().t()
+    assert ext.few_rows(x, w) or parts > 1
+    _same(ext.linear(x, w), want, 8)
+    got = ext.linear_parts(x, w)
+    if parts > 1:
+        assert got.shape == (parts, rows, n)
+        _same(got.sum(0), want, 16)
+        for at in (0, rows - 1):
+            assert torch.equal(got[:, at:at + 1],
+                               ext.linear_parts(x[at:at + 1], w))
+    half = n // 16 * 8
+    gate, up = want[:, :half], want[:, half:2 * half]
+    y = ext.gated_linear(x, w[:2 * half], 2)
+    assert (y is None) == (half <= 64 * 159)
+    if y is not None:
+        _same(y, gate.relu().square() * up, 8)
+
+
 @pytest.mark.parametrize("rows", [193, 256])
 @pytest.mark.parametrize("n,k", [(14400, 1024), (16368, 1152), (14400, 1096)])
 def test_gated_of_many_steps(rows, n, k):
