@@ -64,6 +64,8 @@ __device__ __forceinline__ int start(int blk, int N, int steps) {
 // 16-byte pieces of a row change places by XOR with its number. Past the caches: as other
 // stores they take their time at the end of the kernel, when all of the parts are
 // written back at once (4096 -> 6144, 178 rows 19.3 us, so 16.5; by whole lines only 17.9).
+// Up to 64 rows they are few, and whoever sums them finds them in the caches (a pass of
+// the delta design, 50 rows, 1372 us past them, 1356 so).
 template <int MT, int OUT>
 __device__ __forceinline__ void store(const Tiles& p, char* lds, int part, int blk,
                                       const float4v (&acc)[4][MT]) {
@@ -101,10 +103,13 @@ __device__ __forceinline__ void store(const Tiles& p, char* lds, int part, int b
 #pragma unroll
   for (int i = 0; i < 64 * MT; i += ROWS) {
     const int m = i + threadIdx.x / PIECES;
-    if (m < M)
-      __builtin_nontemporal_store(
-          *(const float4v*)(lds + (m * PIECES + (piece ^ m % PIECES)) * 16),
-          (float4v*)((Elem*)p.y + ((int64_t)part * M + m) * N + n));
+    if (m >= M) continue;
+    const float4v v = *(const float4v*)(lds + (m * PIECES + (piece ^ m % PIECES)) * 16);
+    float4v* const to = (float4v*)((Elem*)p.y + ((int64_t)part * M + m) * N + n);
+    if (MT == 1)
+      *to = v;
+    else
+      __builtin_nontemporal_store(v, to);
   }
 }
 
