@@ -22,6 +22,10 @@
 // a SIMD, so the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost
 // nothing.
 //
+// Values are read by whole rows and past the caches (256 sequences of 1500 tokens, the
+// pass 1818 us with both by way of them, so 1739, with both past them 1795: a load of keys
+// takes 64 bytes of 16 rows, whose other halves have to be found again).
+//
 // Measured alone, cold (8 key heads, ragged; before: P V on the 32-bit cores): 256
 // sequences of 1500 tokens, groups of 4: 269 us, 5.8 TB/s (279), fp8 156 us, 5.0 TB/s
 // (191); 30 of 1100, groups of 8: 27.5 us (31.5); 17 of 6800, fp8, in 4 partitions:
@@ -282,7 +286,9 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
           row = v_head + page[h] * w_.page + (g * 4 + j) * RS;
         else
           row = v_head + row_of(t0 + h * 16 + g * 4 + j);
-        vr[h][j] = *(const typename C::VReg*)(row + col * 8);
+        // past the caches, by whole rows
+        vr[h][j] =
+            __builtin_nontemporal_load((const typename C::VReg*)(row + col * 8));
       }
   };
 
