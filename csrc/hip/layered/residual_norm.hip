@@ -6,7 +6,17 @@
 namespace {
 
 constexpr int NT = 256;
-constexpr int KEEP = 4;  // vectors kept in registers per thread
+constexpr int PT = 512;  // of rows in parts
+
+template <typename T> struct Eight;
+template <> struct Eight<short> {
+  typedef short8 type;
+  static __device__ __forceinline__ float get(type v, int j) { return bf16_to_f32(v[j]); }
+};
+template <> struct Eight<float> {
+  typedef __attribute__((ext_vector_type(8))) float type;
+  static __device__ __forceinline__ float get(type v, int j) { return v[j]; }
+};
 
 enum Mode { EMBED, POST, ADD, LOOP };
 
@@ -35,17 +45,24 @@ struct Stream {
 //   ADD:   x += y + the token's rows (either may be missing)
 //   LOOP:  x = a + b + v
 //   h = x / rms(x) * (wn + offset)
-//   PARTS: y is in parts, 8 channels per vector
-template <typename T, int N, int MODE, bool PARTS>
-__global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
+//   PARTS: y is in parts, 8 channels per vector; so many of them stay in a thread's
+//   registers, the others' threads keep four. What a row takes is the time of its loads,
+//   one after the other: 512 threads with one vector each, everything that is known ahead
+//   asked for at once (50 rows of 4096 in 8 parts in a pass: 5.3 us; 256 threads, and
+//   weights and rows of experts when they are needed: 7.3).
+template <typename T, int N, int MODE, int PARTS>
+__global__ __launch_bounds__(PARTS ? PT : NT) void stream_norm_kernel(
+    const Stream<T> s) {
   static_assert(!PARTS || N == 8, "");
-  __shared__ float red[2][NT / WAVE];
+  constexpr int BT = PARTS ? PT : NT;
+  constexpr int KEEP = PARTS ? PARTS : 4;  // vectors kept in registers per thread
+  __shared__ float red[2][BT / WAVE];
   const int64_t row = blockIdx.x;
   const int H = s.H;
   float* xr = s.x + row * H;
   const T* yr = MODE == EMBED ? s.y + s.ids[row] * H : s.y + row * H;
   // the sublayer's output; its parts are summed here rather than by a launch
-  // of their own (50 rows of 4096 in 8 parts: 7.4 us, apart 10.5)
+  // of their own, one of 3 us
   auto load_y = [&](int64_t c, float* f) {
     if (!s.yp) {
       ldn<N>(yr + c, f);
@@ -64,21 +81,34 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
   // vector i of this thread starts at element at(i); the first KEEP stay in
   // registers between the passes, the rest are read again
   float keep[KEEP][N];
-  auto at = [&](int i) { return (int64_t)(threadIdx.x + i * NT) * N; };
-  // All parts of what a thread keeps are asked for together, the stream's values ahead
-  // of them (8.5 us with the loads of a vector at a time).
-  float xk[PARTS ? KEEP : 1][N];
+  auto at = [&](int i) { return (int64_t)(threadIdx.x + i * BT) * N; };
+  // All parts of what a thread keeps are asked for together, the stream's values, the
+  // weights and the first ROWS of the token's rows (with two vectors they have no room)
+  // ahead of them.
+  constexpr int ROWS = PARTS == 1 ? 4 : 0;
+  float xk[PARTS ? KEEP : 1][N], wbk[PARTS ? KEEP : 1][N], wnk[PARTS ? KEEP : 1][N];
+  typename Eight<T>::type rk[PARTS ? KEEP : 1][ROWS ? ROWS : 1];   // as in memory
   if constexpr (PARTS) {
 #pragma unroll
     for (int i = 0; i < KEEP; ++i)
-      if (i * NT * N < H) ldn<N>(xr + min(at(i), (int64_t)H - N), xk[i]);
+      if (i * BT * N < H) {
+        const int64_t c = min(at(i), (int64_t)H - N);
+        ldn<N>(xr + c, xk[i]);
+        if (MODE == POST) ldn<N>(s.wb + c, wbk[i]);
+        if (s.wn) ldn<N>(s.wn + c, wnk[i]);
+        if (s.n_rows)
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r)
+            rk[i][r] = *(const typename Eight<T>::type*)(
+                s.rows + (row * s.n_rows + min(r, s.n_rows - 1)) * H + c);
+      }
 #pragma unroll
     for (int i = 0; i < KEEP; i += 2)
-      if (i * NT * N < H && (i + 1) * NT * N >= H) {     // the last one alone
+      if (i * BT * N < H && (i + 1) * BT * N >= H) {     // the last one alone
         const float4v* const src[1] = {
             (const float4v*)(s.yp + row * H + min(at(i), (int64_t)H - N))};
         PartSums<1>(src, (int64_t)gridDim.x * H / 4, s.parts).get(0, keep[i]);
-      } else if (i * NT * N < H) {
+      } else if (i * BT * N < H) {
         const float4v* src[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -104,7 +134,7 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
       float f[N];
       square(i, f);
     }
-    inv_y = 1.f / sqrtf(block_sum<NT / WAVE>(ss, red[0]) / (float)H + s.eps);
+    inv_y = 1.f / sqrtf(block_sum<BT / WAVE>(ss, red[0]) / (float)H + s.eps);
   }
   float ss = 0.f;
   auto update = [&](int i, float* f) {  // POST: y's vector in; stream's out
@@ -135,7 +165,11 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
       for (int j = 0; j < N; ++j) d[j] = 0.f;
       if constexpr (MODE == POST) {
         float w[N];
-        ldn<N>(s.wb + c, w);
+        if (PARTS && i < KEEP)
+#pragma unroll
+          for (int j = 0; j < N; ++j) w[j] = wbk[PARTS ? i : 0][j];
+        else
+          ldn<N>(s.wb + c, w);
 #pragma unroll
         for (int j = 0; j < N; ++j) d[j] = f[j] * inv_y * (w[j] + s.offset);
       } else if (PARTS && i < KEEP) {
@@ -144,7 +178,14 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
       } else if (s.y || s.yp) {
         load_y(c, d);
       }
-      for (int r = 0; r < s.n_rows; ++r) {
+      int r = 0;
+      if (PARTS && i < KEEP)
+#pragma unroll
+        for (; r < ROWS; ++r)
+          if (r < s.n_rows)
+#pragma unroll
+            for (int j = 0; j < N; ++j) d[j] += Eight<T>::get(rk[PARTS ? i : 0][r], j);
+      for (; r < s.n_rows; ++r) {
         ldn<N>(s.rows + (row * s.n_rows + r) * H + c, g);
 #pragma unroll
         for (int j = 0; j < N; ++j) d[j] += g[j];
@@ -170,13 +211,17 @@ __global__ __launch_bounds__(NT) void stream_norm_kernel(const Stream<T> s) {
     if (MODE == POST) load_y(at(i), f);
     update(i, f);
   }
-  const float inv = s.wn ? 1.f / sqrtf(block_sum<NT / WAVE>(ss, red[1]) /
+  const float inv = s.wn ? 1.f / sqrtf(block_sum<BT / WAVE>(ss, red[1]) /
                                        (float)H + s.eps)
                          : 1.f;
   auto finish = [&](int i, float* f) {
     if (s.wn) {
       float w[N];
-      ldn<N>(s.wn + at(i), w);
+      if (PARTS && i < KEEP)
+#pragma unroll
+        for (int j = 0; j < N; ++j) w[j] = wnk[PARTS ? i : 0][j];
+      else
+        ldn<N>(s.wn + at(i), w);
 #pragma unroll
       for (int j = 0; j < N; ++j) f[j] *= inv * (w[j] + s.offset);
     }
@@ -227,16 +272,16 @@ hipError_t stream_norm_t(int mode, const void* const* p, int64_t rows,
                     (const float*)p[7], (const float*)p[8],
                     (const float*)p[9], (const float*)p[10], (T*)p[11], H,
                     scale, offset, eps};
-  const dim3 grid((uint32_t)rows), block(NT);
+  const dim3 grid((uint32_t)rows);
 #define GO(N, M, PARTS)                                                       \
-  hipLaunchKernelGGL((stream_norm_kernel<T, N, M, PARTS>), grid, block, 0,    \
-                     stream, s)
+  hipLaunchKernelGGL((stream_norm_kernel<T, N, M, PARTS>), grid,              \
+                     dim3(PARTS ? PT : NT), 0, stream, s)
 #define GOM(N)                                                                \
   do {                                                                        \
-    if (mode == EMBED) GO(N, EMBED, false);                                   \
-    else if (mode == POST) GO(N, POST, false);                                \
-    else if (mode == ADD) GO(N, ADD, false);                                  \
-    else GO(N, LOOP, false);                                                  \
+    if (mode == EMBED) GO(N, EMBED, 0);                                   \
+    else if (mode == POST) GO(N, POST, 0);                                \
+    else if (mode == ADD) GO(N, ADD, 0);                                  \
+    else GO(N, LOOP, 0);                                                  \
   } while (0)
   // Past 256 rows enough is under way, and what is asked for ahead takes the registers
   // of other rows (1300 rows of 4096 in 2 parts: 18.2 us with it, 16.1 without; 300 in 8
@@ -244,7 +289,10 @@ hipError_t stream_norm_t(int mode, const void* const* p, int64_t rows,
   // to ask for ahead in short rows (1024 in 8 parts: 3.7 and 3.5).
   if (parts && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256 &&
       H >= NT * 8) {
-    if (mode == POST) GO(8, POST, true); else GO(8, ADD, true);
+    if (mode == POST && H <= PT * 8) GO(8, POST, 1);
+    else if (mode == POST) GO(8, POST, 2);
+    else if (H <= PT * 8) GO(8, ADD, 1);
+    else GO(8, ADD, 2);
   } else if (H % 8 == 0) {
     GOM(8);
   } else {
