@@ -16,15 +16,18 @@ namespace {
 //   y = src * rsqrt(mean(src^2) + eps) * w
 // x is bf16, or the partial sums of a product that split K: [parts, rows, H]
 // 32-bit, summed here instead of by a launch of their own (8 parts, one row of
-// 4096: 4.5 us, 6.5 with few loads under way; sum and norm apart 8.7; 30 rows of
-// 5120 6.7, were 7.6, 256 of 4096 8.6, were 9.6).
-// One block (256 threads) per token row; row length H % 8 == 0. The first KEEP
+// 4096: 4.1 us, 6.5 with few loads under way; sum and norm apart 8.7; 30 rows of
+// 5120 4.9, were 7.6, 256 of 4096 8.7, were 9.6).
+// One block per token row, of 256 threads, or 512 where the row is in parts: most of
+// its time is the loads' way, and so each thread has half of them (30 rows of 5120 5.5
+// us by 256 threads). Row length H % 8 == 0. The first KEEP
 // vectors of a thread stay in registers between the two passes, the rest are
 // read again. Their number is known at compile time: an index that is not puts
 // the array into scratch memory (8013 rows of 4096 with residual: 84 us, now
 // 44, 5.9 TB/s).
 // ---------------------------------------------------------------------------
 constexpr int NT = 256;
+constexpr int PT = 512;        // of a row in parts
 
 // EARLY: with parts, all that a thread keeps is asked for at once, pair by pair. Not
 // past 512 rows (256 where a thread has one vector): other rows' loads are under way
@@ -32,10 +35,11 @@ constexpr int NT = 256;
 // of 5120 in 3 parts: 11.1 us, without 10.1; 400 rows in 4 parts 8.3 and 8.7; 257 rows of
 // 2048 in 14 parts 6.1 and 5.6).
 template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY>
-__global__ __launch_bounds__(NT) void rmsnorm_kernel(
+__global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
     const void* __restrict__ x, int parts, short* __restrict__ residual,
     const short* __restrict__ w, short* __restrict__ y, int H, float eps) {
-  __shared__ float red[NT / WAVE];
+  constexpr int BT = PARTS ? PT : NT;
+  __shared__ float red[BT / WAVE];
   const int64_t row = blockIdx.x;
   const int nchunks = H / 8;
   short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
@@ -65,26 +69,27 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   };
   float vals[KEEP][8], ss = 0.f;
   static_assert(PARTS || !EARLY, "");
-  constexpr bool AHEAD = EARLY && KEEP > 1;
+  constexpr bool AHEAD = EARLY;
   short8 rv[AHEAD ? KEEP : 1], wk[AHEAD ? KEEP : 1];
   if constexpr (AHEAD) {
     const int64_t apart = (int64_t)gridDim.x * H / 4;
 #pragma unroll
     for (int i = 0; i < KEEP; ++i) {
-      const int c = min((int)threadIdx.x + i * NT, nchunks - 1);
+      const int c = min((int)threadIdx.x + i * BT, nchunks - 1);
       if constexpr (RESIDUAL) rv[i] = r8[c];
       wk[i] = ((const short8*)w)[c];
     }
+    constexpr int W = KEEP > 1 ? 2 : 1;
 #pragma unroll
-    for (int i = 0; i < KEEP; i += 2) {
-      const float4v* p[2];
+    for (int i = 0; i < KEEP; i += W) {
+      const float4v* p[W];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < W; ++j)
         p[j] = (const float4v*)x + row * H / 4 +
-               min((int)threadIdx.x + (i + j) * NT, nchunks - 1) * 2;
-      const PartSums<2> sum(p, apart, parts);
-      sum.get(0, vals[i]);
-      sum.get(1, vals[i + 1]);
+               min((int)threadIdx.x + (i + j) * BT, nchunks - 1) * 2;
+      const PartSums<W> sum(p, apart, parts);
+#pragma unroll
+      for (int j = 0; j < W; ++j) sum.get(j, vals[i + j]);
     }
   }
   auto first = [&](int c, float* f, int i) {
@@ -104,15 +109,15 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   };
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int c = threadIdx.x + i * NT;
+    const int c = threadIdx.x + i * BT;
     if (c < nchunks) first(c, vals[i], i);
   }
-  for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
+  for (int c = threadIdx.x + KEEP * BT; c < nchunks; c += BT) {
     float f[8];
     first(c, f, -1);
   }
   const float inv =
-      rsqrtf(block_reduce_sum<NT / WAVE>(ss, red) / (float)H + eps);
+      rsqrtf(block_reduce_sum<BT / WAVE>(ss, red) / (float)H + eps);
   auto second = [&](int c, const float* f, int i) {
     const short8 wv =
         AHEAD && i >= 0 ? wk[AHEAD ? i : 0] : ((const short8*)w)[c];
@@ -124,10 +129,10 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(
   };
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
-    const int c = threadIdx.x + i * NT;
+    const int c = threadIdx.x + i * BT;
     if (c < nchunks) second(c, vals[i], i);
   }
-  for (int c = threadIdx.x + KEEP * NT; c < nchunks; c += NT) {
+  for (int c = threadIdx.x + KEEP * BT; c < nchunks; c += BT) {
     float f[8];
     if constexpr (RESIDUAL) {   // this thread's own store above
       const short8 v = r8[c];
@@ -318,12 +323,13 @@ hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
   if (n_rows == 0) return hipSuccess;
 #define GO(KEEP, RES, PARTS, EARLY)                                          \
   hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS, EARLY>),              \
-                     dim3((uint32_t)n_rows), dim3(NT), 0, stream, x, parts,  \
+                     dim3((uint32_t)n_rows), dim3(PARTS ? PT : NT), 0, stream, x, parts, \
                      (short*)residual, (const short*)w, (short*)y, H, eps)
 #define GO_K(RES, PARTS, EARLY)                                              \
   do {                                                                       \
-    if (H <= 1 * NT * 8) GO(1, RES, PARTS, EARLY);                           \
-    else if (H <= 2 * NT * 8) GO(2, RES, PARTS, EARLY);                      \
+    const int each = (PARTS ? PT : NT) * 8;                                  \
+    if (H <= each) GO(1, RES, PARTS, EARLY);                                 \
+    else if (H <= 2 * each) GO(2, RES, PARTS, EARLY);                        \
     else GO(4, RES, PARTS, EARLY);                                           \
   } while (0)
   const bool early = n_rows <= (H <= NT * 8 ? 256 : 512);
