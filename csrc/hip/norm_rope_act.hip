@@ -34,22 +34,36 @@ constexpr int PT = 512;        // of a row in parts
 // anyway, and what a pair reads past the row's end costs more than the wait (600 rows
 // of 5120 in 3 parts: 11.1 us, without 10.1; 400 rows in 4 parts 8.3 and 8.7; 257 rows of
 // 2048 in 14 parts 6.1 and 5.6).
-template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY>
+// ROWS: ALL of them; PICKED: the rows that `rows` names, of n_rows, without a word to
+// the residual; TABLE: rows of the table x that `rows` names (token ids), which become the
+// residual. As in an index, rows below 0 count from the end; others that do not exist are
+// the nearest that does.
+enum Rows { ALL, PICKED, TABLE };
+
+template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY, int ROWS>
 __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
     const void* __restrict__ x, int parts, short* __restrict__ residual,
-    const short* __restrict__ w, short* __restrict__ y, int H, float eps) {
+    const short* __restrict__ w, short* __restrict__ y, int H, float eps,
+    const int64_t* __restrict__ rows, int64_t n_rows) {
   constexpr int BT = PARTS ? PT : NT;
   __shared__ float red[BT / WAVE];
-  const int64_t row = blockIdx.x;
+  int64_t row = blockIdx.x;
+  if constexpr (ROWS != ALL) {
+    row = rows[row];
+    row += row < 0 ? n_rows : 0;
+    row = row < 0 ? 0 : row < n_rows ? row : n_rows - 1;
+  }
   const int nchunks = H / 8;
-  short8* r8 = RESIDUAL ? (short8*)(residual + row * H) : nullptr;
+  short8* r8 = RESIDUAL ? (short8*)(residual + row * H)
+               : ROWS == TABLE ? (short8*)(residual + (int64_t)blockIdx.x * H)
+                               : nullptr;
   auto source = [&](int c, float* f) {
     if constexpr (EARLY) {
       const float4v* const p[1] = {(const float4v*)x + (row * H + c * 8) / 4};
-      PartSums<1>(p, (int64_t)gridDim.x * H / 4, parts).get(0, f);
+      PartSums<1>(p, n_rows * H / 4, parts).get(0, f);
     } else if constexpr (PARTS) {
       const float4v* p = (const float4v*)x + (row * H + c * 8) / 4;
-      const int64_t apart = (int64_t)gridDim.x * H / 4;
+      const int64_t apart = n_rows * H / 4;
       float4v a = p[0], b = p[1];
 #pragma unroll 4
       for (int i = 1; i < parts; ++i) {
@@ -72,7 +86,7 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
   constexpr bool AHEAD = EARLY;
   short8 rv[AHEAD ? KEEP : 1], wk[AHEAD ? KEEP : 1];
   if constexpr (AHEAD) {
-    const int64_t apart = (int64_t)gridDim.x * H / 4;
+    const int64_t apart = n_rows * H / 4;
 #pragma unroll
     for (int i = 0; i < KEEP; ++i) {
       const int c = min((int)threadIdx.x + i * BT, nchunks - 1);
@@ -102,7 +116,12 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
         f[j] += bf16_to_f32(r[j]);
         ro[j] = f32_to_bf16(f[j]);
       }
-      r8[c] = ro;  // residual stream updated in place
+      if (ROWS == ALL) r8[c] = ro;  // residual stream updated in place
+    } else if constexpr (ROWS == TABLE) {
+      short8 ro;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) ro[j] = f32_to_bf16(f[j]);
+      r8[c] = ro;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss += f[j] * f[j];
@@ -125,7 +144,7 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       o[j] = f32_to_bf16(f[j] * inv * bf16_to_f32(wv[j]));
-    ((short8*)(y + row * H))[c] = o;
+    ((short8*)(y + (int64_t)blockIdx.x * H))[c] = o;
   };
 #pragma unroll
   for (int i = 0; i < KEEP; ++i) {
@@ -134,10 +153,16 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
   }
   for (int c = threadIdx.x + KEEP * BT; c < nchunks; c += BT) {
     float f[8];
-    if constexpr (RESIDUAL) {   // this thread's own store above
+    if constexpr (RESIDUAL && ROWS == ALL) {   // this thread's own store above
       const short8 v = r8[c];
 #pragma unroll
       for (int j = 0; j < 8; ++j) f[j] = bf16_to_f32(v[j]);
+    } else if constexpr (RESIDUAL) {           // what it would have been
+      const short8 v = r8[c];
+      source(c, f);
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        f[j] = bf16_to_f32(f32_to_bf16(f[j] + bf16_to_f32(v[j])));
     } else {
       source(c, f);
     }
@@ -316,29 +341,42 @@ __global__ void silu_mul_kernel(const short* __restrict__ gate_up,
 
 extern "C" {
 
-// parts > 0: x are that many partial sums in 32-bit
+// parts > 0: x are that many partial sums in 32-bit. rows: null, or n of the n_rows rows
+// of x and of the residual, or (table) of the table x, whose copies fill the residual.
 hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
                        void* y, int64_t n_rows, int H, float eps,
+                       const int64_t* rows, int64_t n, int table,
                        hipStream_t stream) {
-  if (n_rows == 0) return hipSuccess;
-#define GO(KEEP, RES, PARTS, EARLY)                                          \
-  hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS, EARLY>),              \
-                     dim3((uint32_t)n_rows), dim3(PARTS ? PT : NT), 0, stream, x, parts, \
-                     (short*)residual, (const short*)w, (short*)y, H, eps)
-#define GO_K(RES, PARTS, EARLY)                                              \
+  if (!rows) n = n_rows;
+  if (n == 0) return hipSuccess;
+  if (n > 0x7fffffff || n_rows < 1 || (table && (!rows || !residual || parts)))
+    return hipErrorInvalidValue;
+#define GO(KEEP, RES, PARTS, EARLY, ROWS)                                    \
+  hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS, EARLY, ROWS>),        \
+                     dim3((uint32_t)n), dim3(PARTS ? PT : NT), 0, stream, x, \
+                     parts, (short*)residual, (const short*)w, (short*)y, H, \
+                     eps, rows, n_rows)
+#define GO_K(RES, PARTS, EARLY, ROWS)                                        \
   do {                                                                       \
     const int each = (PARTS ? PT : NT) * 8;                                  \
-    if (H <= each) GO(1, RES, PARTS, EARLY);                                 \
-    else if (H <= 2 * each) GO(2, RES, PARTS, EARLY);                        \
-    else GO(4, RES, PARTS, EARLY);                                           \
+    if (H <= each) GO(1, RES, PARTS, EARLY, ROWS);                           \
+    else if (H <= 2 * each) GO(2, RES, PARTS, EARLY, ROWS);                  \
+    else GO(4, RES, PARTS, EARLY, ROWS);                                     \
   } while (0)
-  const bool early = n_rows <= (H <= NT * 8 ? 256 : 512);
-  if (parts > 0 && early) {
-    if (residual) GO_K(true, true, true); else GO_K(false, true, true);
+  const bool early = n <= (H <= NT * 8 ? 256 : 512);
+  if (table) {
+    GO_K(false, false, false, TABLE);
+  } else if (rows && parts > 0) {
+    if (residual) GO_K(true, true, true, PICKED); else GO_K(false, true, true, PICKED);
+  } else if (rows) {
+    if (residual) GO_K(true, false, false, PICKED);
+    else GO_K(false, false, false, PICKED);
+  } else if (parts > 0 && early) {
+    if (residual) GO_K(true, true, true, ALL); else GO_K(false, true, true, ALL);
   } else if (parts > 0) {
-    if (residual) GO_K(true, true, false); else GO_K(false, true, false);
+    if (residual) GO_K(true, true, false, ALL); else GO_K(false, true, false, ALL);
   } else {
-    if (residual) GO_K(true, false, false); else GO_K(false, false, false);
+    if (residual) GO_K(true, false, false, ALL); else GO_K(false, false, false, ALL);
   }
 #undef GO_K
 #undef GO

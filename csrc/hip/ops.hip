@@ -31,7 +31,7 @@ hipError_t lds_match_longest(const uint64_t*, const unsigned long long*,
                              uint32_t, const uint64_t*, const int32_t*, int,
                              int, int, int32_t*, hipStream_t);
 hipError_t lds_rmsnorm(const void*, int, void*, const void*, void*, int64_t,
-                       int, float, hipStream_t);
+                       int, float, const int64_t*, int64_t, int, hipStream_t);
 int lds_heads_ok(int, int);
 hipError_t lds_heads(const void*, int, int64_t, const void*, const void*,
                      const float*, const int32_t*, const int64_t*, void*,
@@ -195,28 +195,59 @@ torch::Tensor match_longest(torch::Tensor keys, torch::Tensor masks,
 // ---- engine kernels ----
 
 // x: bf16 rows, or 32-bit partial sums [parts, rows, H] of a product
+// rows: those of x that are wanted; the residual then stays as it is
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
-                      c10::optional<torch::Tensor> residual) {
+                      c10::optional<torch::Tensor> residual,
+                      c10::optional<torch::Tensor> rows) {
   CHECK_GPU(x); CHECK_GPU(w);
   const bool parts = x.dim() == 3 && x.dtype() == torch::kFloat32;
   TORCH_CHECK(parts || x.dtype() == torch::kBFloat16, "rmsnorm expects bf16");
   TORCH_CHECK(!parts || (x.size(0) > 0 && x.size(2) % 8 == 0 &&
                          w.numel() == x.size(2)), "rmsnorm parts");
-  auto y = parts ? torch::empty({x.size(1), x.size(2)},
-                                x.options().dtype(torch::kBFloat16))
-                 : torch::empty_like(x);
-  int H = (int)x.size(-1);
-  int64_t rows = y.numel() / H;
+  const int H = (int)x.size(-1);
+  const int64_t n_rows = parts ? x.size(1) : x.numel() / H;
+  auto opts = x.options().dtype(torch::kBFloat16);
+  torch::Tensor y;
+  if (rows.has_value()) {
+    CHECK_GPU(*rows);
+    TORCH_CHECK(rows->dtype() == torch::kInt64 && rows->dim() == 1 &&
+                    (n_rows > 0 || rows->numel() == 0) && w.numel() == H &&
+                    H % 8 == 0 && (parts || x.dim() == 2),
+                "rmsnorm rows");
+    y = torch::empty({rows->numel(), H}, opts);
+  } else {
+    y = parts ? torch::empty({n_rows, H}, opts) : torch::empty_like(x);
+  }
   void* res_ptr = nullptr;
   if (residual.has_value()) {
     CHECK_GPU(*residual);
-    TORCH_CHECK(!parts || residual->numel() == y.numel(), "residual");
+    TORCH_CHECK(!(parts || rows.has_value()) || residual->numel() == n_rows * H,
+                "residual");
     res_ptr = residual->data_ptr();
   }
   CHECK_HIP(lds_rmsnorm(x.data_ptr(), parts ? (int)x.size(0) : 0, res_ptr,
-                        w.data_ptr(), y.data_ptr(), rows, H, (float)eps,
-                        cur_stream()));
+                        w.data_ptr(), y.data_ptr(), n_rows, H, (float)eps,
+                        rows.has_value() ? rows->data_ptr<int64_t>() : nullptr,
+                        rows.has_value() ? rows->numel() : 0, 0, cur_stream()));
   return y;
+}
+
+// -> table[ids] and its norm
+std::tuple<torch::Tensor, torch::Tensor> embed_rmsnorm(torch::Tensor ids,
+                                                       torch::Tensor table,
+                                                       torch::Tensor w, double eps) {
+  CHECK_GPU(ids); CHECK_GPU(table); CHECK_GPU(w);
+  TORCH_CHECK(ids.dtype() == torch::kInt64 && ids.dim() == 1 && table.dim() == 2 &&
+                  table.dtype() == torch::kBFloat16 && table.size(1) % 8 == 0 &&
+                  (table.size(0) > 0 || ids.numel() == 0) &&
+                  w.dtype() == torch::kBFloat16 && w.numel() == table.size(1),
+              "embed_rmsnorm");
+  torch::Tensor x = torch::empty({ids.numel(), table.size(1)}, table.options());
+  torch::Tensor y = torch::empty_like(x);
+  CHECK_HIP(lds_rmsnorm(table.data_ptr(), 0, x.data_ptr(), w.data_ptr(),
+                        y.data_ptr(), table.size(0), (int)table.size(1), (float)eps,
+                        ids.data_ptr<int64_t>(), ids.numel(), 1, cur_stream()));
+  return {x, y};
 }
 
 // qkv [T, heads * D] bf16 or 32-bit partial sums [parts, T, heads * D]: q and
@@ -458,7 +489,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("table_update", &table_update, "device prefix table insert/remove");
   m.def("match_longest", &match_longest, "device longest-prefix match");
   m.def("rmsnorm", &rmsnorm, py::arg("x"), py::arg("w"), py::arg("eps"),
-        py::arg("residual") = py::none());
+        py::arg("residual") = py::none(), py::arg("rows") = py::none());
+  m.def("embed_rmsnorm", &embed_rmsnorm, "table[ids] and its norm");
   m.def("rope", &rope, "in-place NeoX RoPE");
   m.def("rope_and_cache", &rope_and_cache,
         "heads of a qkv product: normed, rotated, k and v into the cache",

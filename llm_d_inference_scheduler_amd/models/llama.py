@@ -128,10 +128,16 @@ class LlamaRunner:
         """Returns logits [n_logit_rows, vocab] (or final hidden states for
         embeddings_out). kv_pool: [L, 2, NB, KVH, BS, D]."""
         c = self.cfg
-        hidden = self.embed[batch.input_ids]
+        normed = residual = None
         if batch.embed_rows is not None and batch.embed_rows.numel():
+            hidden = self.embed[batch.input_ids]
             hidden[batch.embed_rows] = batch.embed_values.to(hidden.dtype)
-        residual = None
+        elif self.layers:
+            hidden, normed = ops.embed_rmsnorm(
+                batch.input_ids, self.embed, self.layers[0]["input_norm"],
+                c.rms_eps)
+        else:
+            hidden = self.embed[batch.input_ids]
         pos32 = batch.positions.to(torch.int32)
         shape = -1
         if batch.prefill_tiles is not None and batch.seq_starts and \
@@ -143,7 +149,9 @@ class LlamaRunner:
         for li, layer in enumerate(self.layers):
             if residual is None:
                 residual = hidden
-                normed = ops.rmsnorm(hidden, layer["input_norm"], c.rms_eps)
+                if normed is None:
+                    normed = ops.rmsnorm(hidden, layer["input_norm"],
+                                         c.rms_eps)
             else:
                 normed = ops.rmsnorm(hidden, layer["input_norm"], c.rms_eps,
                                      residual=residual)
@@ -170,13 +178,9 @@ class LlamaRunner:
             act = ops.gated_linear(normed2, layer["wgate_up"].t())
             hidden = ops.linear_parts(act, layer["wdown"].t())
         final = ops.rmsnorm(hidden, self.final_norm, c.rms_eps,
-                            residual=residual)
-        # `residual` now holds the pre-norm sum; `final` the normed states
-        if embeddings_out:
-            return final
-        rows = batch.logit_rows
-        sel = final if rows is None else final[rows]
-        return ops.linear(sel, self.lm_head)
+                            residual=residual,
+                            rows=None if embeddings_out else batch.logit_rows)
+        return final if embeddings_out else ops.linear(final, self.lm_head)
 
     def _prefill_attention(self, batch: ForwardBatch, q: torch.Tensor,
                            k_cache: torch.Tensor, v_cache: torch.Tensor,

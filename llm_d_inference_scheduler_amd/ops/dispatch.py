@@ -64,11 +64,32 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 _SILU = 1       # activation code of the kernels
 
 
+def _index(t: torch.Tensor) -> bool:
+    return t.dim() == 1 and t.dtype == torch.int64 and t.is_contiguous()
+
+
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
-            residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+            residual: Optional[torch.Tensor] = None,
+            rows: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """rows: the norms of these rows alone; what happens to the residual is
+    left open then."""
     if _use_hip(x):
-        return _ext.rmsnorm(x, w, eps, residual)
-    return ref.rmsnorm(x, w, eps, residual)
+        if rows is None or (rows.is_cuda and _index(rows) and
+                            x.shape[-1] % 8 == 0):
+            return _ext.rmsnorm(x, w, eps, residual, rows)
+        return _ext.rmsnorm(x, w, eps, residual)[rows]
+    y = ref.rmsnorm(x, w, eps, residual)
+    return y if rows is None else y[rows]
+
+
+def embed_rmsnorm(ids: torch.Tensor, table: torch.Tensor, w: torch.Tensor,
+                  eps: float):
+    """-> table[ids] and its norm."""
+    if _use_hip(table) and ids.is_cuda and _index(ids) and \
+            table.dtype == torch.bfloat16 and table.shape[1] % 8 == 0:
+        return _ext.embed_rmsnorm(ids, table, w, eps)
+    x = table[ids]
+    return x, rmsnorm(x, w, eps)
 
 
 def rope(q: torch.Tensor, k: torch.Tensor, cos_sin: torch.Tensor,

@@ -572,6 +572,31 @@ def test_norms_of_any_parts(rows, width, parts):
             _same(h, normed(s) * (wn.double() + 0.5), 8)
 
 
+@pytest.mark.parametrize("parts", [0, 1, 8])
+@pytest.mark.parametrize("rows,width", [(1, 8), (5, 2056), (300, 4096), (3, 4104),
+                                        (600, 1024), (2, 16400), (2, 32776)])
+def test_norms_of_some_rows(rows, width, parts):
+    """The rows asked for, twice or from the end, as they come out among all; of a
+    table, its rows and their norms. All the same bits: threads, sums and rounding are
+    the same."""
+    from llm_d_inference_scheduler_amd import ops
+    x = _draw(max(parts, 1), rows, width, seed=rows)
+    x = x.float() if parts else x[0]
+    gain, start = _draw(width, seed=3), _draw(rows, width, seed=4)
+    some = torch.tensor([rows - 1, 0, -1, rows // 2, 0], device="cuda")
+    for residual in (None, start):
+        want = ops.rmsnorm(x, gain, 1e-5,
+                           None if residual is None else residual.clone())
+        got = ops.rmsnorm(x, gain, 1e-5, residual, some)
+        assert torch.equal(got, want[some])
+        assert ops.rmsnorm(x, gain, 1e-5, residual, some[:0]).shape == (0, width)
+    assert torch.equal(start, _draw(rows, width, seed=4))
+    if not parts:
+        rows_of, normed = ops.embed_rmsnorm(some, x, gain, 1e-5)
+        assert torch.equal(rows_of, x[some])
+        assert torch.equal(normed, ops.rmsnorm(x[some], gain, 1e-5))
+
+
 @pytest.mark.parametrize("width", [1032, 2056, 4104, 8200])
 @pytest.mark.parametrize("few,many,parts", [(256, 257, 9), (512, 513, 2)])
 def test_norms_of_parts_of_many_rows(few, many, parts, width):
