@@ -6,7 +6,7 @@
 // Pairs are sorted by expert (stable, so results do not depend on timing) and
 // cut into tiles of one expert each; the product kernels take one tile and a
 // block of output channels per workgroup:
-//   expert_tiles   256 pairs and 256 channels through LDS, for many pairs
+//   expert_tiles   256, 192 or 128 pairs and 256 channels through LDS, for many pairs
 //   expert_rows    up to 64 pairs, for few: there the weights' bytes are what counts
 //   expert_plain   any size, bf16 or float
 #include "elem.h"
@@ -405,9 +405,12 @@ hipError_t launch_rows(Pairs p, int max_tiles, int tiles, hipStream_t stream) {
 constexpr int TC = 256, BK = TILE_K, HALF = 128;
 constexpr int TG = 4;                // tiles of pairs that run side by side
 typedef TileCore<8, 8, 2, 2> Whole;
+typedef TileCore<8, 6, 2, 2> Most;   // 192 pairs
 typedef TileCore<4, 8, 4, 2> Half;
-static_assert(Whole::CHANNELS == TC && Half::CHANNELS == TC &&
-                  Whole::ROWS == TILE && Half::ROWS == HALF,
+static_assert(Whole::CHANNELS == TC && Most::CHANNELS == TC && Half::CHANNELS == TC &&
+                  Whole::ROWS == TILE && Half::ROWS == HALF &&
+                  Most::LDS_TURN <= Whole::LDS_TURN &&
+                  Half::LDS_TURN <= Whole::LDS_TURN,
               "");
 
 template <bool UP, typename Core>
@@ -415,6 +418,7 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
                                              const int4 tile, int n0) {
   Core core;
   constexpr int LW = Core::LW, LP = Core::LP, PT = Core::ROWS / 16 / Core::WP;
+  constexpr int QP = Core::QP;
   const int N = p.N, K = p.K;
   // channels past the end and rows past the tile repeat the last one: they are
   // computed and dropped
@@ -438,9 +442,9 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
       asrc[h][j] = (asrc[h][j] * K + core.template piece<LP>(j)) * 2;
   }
   // what the results need is on its way while the products run: weights by row,
-  // or the places that 64 rows go to
+  // or the places that the rows of a quarter go to
   float wt[PT];
-  int32_t to[PT / 4];
+  int32_t to[2];
   if constexpr (UP) {
 #pragma unroll
     for (int t = 0; t < PT; ++t)
@@ -448,8 +452,8 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
                                              tile.z - 1)]];
   } else {
 #pragma unroll
-    for (int t = 0; t < PT / 4; ++t)
-      to[t] = p.order[tile.y + min(core.row(t * 4) + core.lane, tile.z - 1)];
+    for (int t = 0; t < 2; ++t)
+      to[t] = p.order[tile.y + min(core.row(t * QP) + core.lane, tile.z - 1)];
   }
   // offsets stay under 4 GiB (lds_expert_tile)
   core.run(lds, (const char*)p.w + (int64_t)tile.x * N * K * 2,
@@ -467,7 +471,13 @@ __device__ __forceinline__ void tile_product(const Pairs& p, short* lds,
           },
           [&](int row, int i, int c, short8 v) {
             int64_t at = tile.y + i;
-            if constexpr (!UP) at = __shfl(to[b / 2], b % 2 * 32 + row, WAVE);
+            if constexpr (!UP) {
+              at = __shfl(to[2 * b / QP], 2 * b % QP * 16 + row, WAVE);
+              if (2 * b % QP + 1 == QP) {        // its 32 rows lie in two quarters
+                const int next = __shfl(to[1], row - 16, WAVE);
+                if (row >= 16) at = next;
+              }
+            }
             if (i < tile.z && n0 + c < N)       // N is a multiple of 8
               *(short8*)((short*)p.out + at * N + n0 + c) = v;
           });
@@ -503,8 +513,13 @@ __global__ __launch_bounds__(256, 1) void expert_tiles_kernel(const Pairs p) {
   const int width = min(TG, n - g * TG);
   const int4 tile = p.tiles[base + g * TG + in % width];
   const int n0 = in / width * TC;
-  if (tile.z > HALF)
+  // What a tile's rows do without is left out: 32 experts of 4096 x 3584, 4 each, 1300
+  // rows 477 us with tiles of 256 and 128 alone, so 427; 1000 rows 416 and 397; 7821
+  // rows, the same.
+  if (tile.z > Most::ROWS)
     tile_product<UP, Whole>(p, tile_lds, tile, n0);
+  else if (tile.z > HALF)
+    tile_product<UP, Most>(p, tile_lds, tile, n0);
   else
     tile_product<UP, Half>(p, tile_lds, tile, n0);
 }

@@ -499,6 +499,26 @@ def test_experts_of_few_pairs(K, F, pairs):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,F", [(128, 128), (192, 320), (576, 448)])
+@pytest.mark.parametrize("counts", [(128, 129, 160), (192, 193, 0), (96, 145, 256),
+                                    (321, 400, 449)])
+def test_experts_of_many_pairs(K, F, counts):
+    """Tiles of 128, 192 and 256 pairs: the ends of each, channels past the end."""
+    run, E = ("cuda", torch.bfloat16), len(counts)
+    up = put(rnd(E, F, K, seed=2, scale=K ** -0.5), run)
+    down = put(rnd(E, K, F, seed=3, scale=F ** -0.5), run)
+    g = torch.Generator().manual_seed(sum(counts))
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    ids = ids[torch.randperm(len(ids), generator=g)].int()[:, None]
+    h = put(rnd(len(ids), K), run)
+    wt = torch.rand(len(ids), 1, generator=g) * 0.9 + 0.05
+    out = ops.experts(h, ids.cuda(), wt.cuda(), up, down, "relu_squared")
+    want = TestExperts().want(h, ids, wt, up, down)
+    # the inner rows and the results are rounded to 8 bits, 32-bit sums beside that
+    close(out, want, run, bf16=2e-2)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T", [8, 40, 90, 180])
 def test_experts_of_a_row_whatever_others_chose(T):
     """Tiles of 16, 32 and 64 pairs: the first rows' bits, where the other rows have
