@@ -26,6 +26,7 @@ struct Product {
   short* y;                  // [M, N]
   int M, N, K, act;
   uint32_t x_bytes, w_bytes;
+  int whole;                 // tiles ahead of those that are cut in two
 };
 
 // As activate() of elem.h, by the exponential and the reciprocal of the hardware. The
@@ -91,26 +92,48 @@ __global__ __launch_bounds__(256, 1) void linear_act_kernel(const Product p) {
   extern __shared__ __align__(16) short act_lds[];
   constexpr int BR = Whole<PT>::ROWS;
   // Workgroups go round the 8 XCDs in turn: each gets a contiguous share of the
-  // tiles, in which TG tiles of rows walk the channels together.
+  // whole tiles, then one of the others, in which TG tiles of rows walk the channels
+  // together.
   constexpr int width = GATED ? BC / 2 : BC;
   const int nx = (p.N + width - 1) / width, ny = (p.M + BR - 1) / BR;
-  const int id = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+  const bool cut = (int)blockIdx.x >= p.whole && p.whole > 0;
+  const int b = cut || p.whole == 0 ? blockIdx.x - p.whole : blockIdx.x;
+  const int share = (cut || p.whole == 0 ? gridDim.x - p.whole : p.whole) / 8;
+  const int at = b % 8 * share + b / 8;
+  const int id = cut ? p.whole + at / 2 : at;
   if (id >= nx * ny) return;
   const int g = id / (TG * nx), in = id % (TG * nx);
   const int side = min(TG, ny - g * TG);
-  const int m0 = (g * TG + in % side) * BR, blk = in / side;
-  if (p.M - m0 > Half::ROWS)
+  const int m0 = (g * TG + in % side) * BR + (cut ? at % 2 * Half::ROWS : 0);
+  const int blk = in / side;
+  if (m0 >= p.M) return;
+  if (!cut && p.M - m0 > Half::ROWS)
     tile<ACT, GATED, Whole<PT>>(p, act_lds, m0, blk);
   else
     tile<ACT, GATED, Half>(p, act_lds, m0, blk);
 }
 
+constexpr int CUS = 256;
+// Tiles behind whole rounds of the compute units, up to half a round of them, are cut
+// in two by rows: a half takes 0.65 of a round (4096 -> 7168, K = 4096: 42 us for 70 to
+// 88). us, whole / so: 4096 -> 7168, 5400 rows 248 / 226, 7000 334 / 307, 7821 343 / 325,
+// 8190 344 / 329; 2048 -> [2 x 8192], 8195 rows 430 / 414. More than half a round would
+// take two rounds of halves.
+bool cut_in_two(int64_t tiles) {
+  return tiles > CUS && tiles % CUS > 0 && tiles % CUS <= CUS / 2;
+}
+
 template <int ACT, bool GATED, int PT>
-hipError_t go(const Product& p, hipStream_t stream) {
+hipError_t go(Product p, hipStream_t stream) {
   constexpr int width = GATED ? BC / 2 : BC, BR = Whole<PT>::ROWS;
   constexpr int bytes = Whole<PT>::LDS_TURN;
-  const int64_t n = (int64_t)((p.N + width - 1) / width) * ((p.M + BR - 1) / BR);
+  int64_t n = (int64_t)((p.N + width - 1) / width) * ((p.M + BR - 1) / BR);
   if (n > 1 << 24) return hipErrorInvalidValue;
+  p.whole = 0;
+  if (BR == 2 * Half::ROWS && cut_in_two(n)) {
+    p.whole = (int)(n / CUS * CUS);
+    n += n - p.whole;
+  }
   auto fn = linear_act_kernel<ACT, GATED, PT>;
   const hipError_t e = hipFuncSetAttribute(
       (const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -134,14 +157,17 @@ extern "C" {
 // 1415 / 1298. 2048 -> [2 x 8192]: 565 rows 50 / 37 (192, 74 %), 1232 92 / 75 (192, 80
 // %). 5120 -> [2 x 25600]: 320 rows 205 / 176 (192, 65 %), 1005 528 / 429 (256, 77 %;
 // 192, 82 %: 468). 4096 -> 7168: 732 rows 61 / 66 (192, 42 %), 1047 69 / 62 (192, 60 %),
-// 8190 376 / 352 (256). 2048 -> 4096: 925 rows 31 / 33 (30 %), 2809 57 / 40 (192, 91 %).
-// 5120 -> 12800: 565 rows 89 / 87 (192, 57 %).
+// 8190 376 / 329 (256, the last 128 tiles cut). 2048 -> 4096: 925 rows 31 / 33 (30 %), 2809 57 / 40 (192, 91 %).
+// 5120 -> 12800: 565 rows 89 / 87 (192, 57 %). Cut tiles count as 0.65 of a round: by
+// 192 and by 256 rows, 4096 -> [2 x 14336] 2400 rows 418 / 405, 2900 504 / 487, 4700
+// 798 / 782, 2048 -> [2 x 8192] 4400 rows 234 / 226, 5120 -> 12800 5400 rows 508 / 491.
 int lds_linear_act_rows(int64_t M, int64_t N, int64_t K, int gated) {
   const int64_t width = gated ? BC / 2 : BC;
   if (M <= 256 || K < 2 * TILE_K || K % TILE_K || N < 8 || N % 8) return 0;
   auto cost = [&](int64_t rows) {
     const int64_t tiles = (M + rows - 1) / rows * ((N + width - 1) / width);
-    return (tiles + 255) / 256 * 256 * rows * width;
+    const int64_t last = rows == 2 * Half::ROWS && cut_in_two(tiles) ? CUS * 13 / 20 : CUS;
+    return (tiles / CUS * CUS + (tiles % CUS ? last : 0)) * rows * width;
   };
   const int rows = cost(192) * 108 < cost(256) * 100 ? 192 : 256;
   return M * N * 20 >= cost(rows) * 11 ? rows : 0;
@@ -160,7 +186,7 @@ hipError_t lds_linear_act(const void* x, int64_t x_row, const void* w,
       xb >= 1ll << 32 || wb >= 1ll << 32)
     return hipErrorInvalidValue;
   const Product p{(const short*)x, (const short*)w, x_row, w_row, (short*)y,
-              M, N, K, act, (uint32_t)xb, (uint32_t)wb};
+              M, N, K, act, (uint32_t)xb, (uint32_t)wb, 0};
 #define GO(A)                                                                \
   return rows == 192                                                         \
              ? gated ? go<A, true, 6>(p, stream) : go<A, false, 6>(p, stream) \

@@ -226,6 +226,25 @@ def test_act_of_many_rows(name, gated, rows, n, k, tile):
 
 
 @pytest.mark.parametrize("name", EXTENSIONS)
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("rows,n,tile", [
+    (385, 24576, 256), (400, 24568, 256), (512, 24576, 256), (3400, 10000, 256),
+    (5700, 4992, 256)])
+def test_act_of_cut_tiles(name, gated, rows, n, tile):
+    """Tiles behind whole rounds cut in two, up to half a round of them: a last row
+    alone, a second half without rows and with some, channels that end inside a tile;
+    a tile more than half a round, cut and whole."""
+    F, ext, k = torch.nn.functional, _ext(name), 128
+    n *= 1 if gated else 2
+    assert ext.act_rows(rows, n, k, gated) == tile
+    x, w = _draw(rows, k, seed=rows), _draw(n * (1 + gated), k, seed=n, scale=k ** -0.5)
+    y = (ext.gated_linear if gated else ext.activated_linear)(x, w, 1)
+    z = x.double() @ w.double().t()
+    g, u = z.chunk(2, -1) if gated else (z, 1)
+    _same(y, F.silu(g) * u, 8)
+
+
+@pytest.mark.parametrize("name", EXTENSIONS)
 @pytest.mark.parametrize("rows,n,k", [(1, 8, 512), (16, 4096, 520), (17, 7168, 4096),
                                       (64, 4088, 8192), (60, 30000, 264)])
 def test_act_of_few_rows(name, rows, n, k):
