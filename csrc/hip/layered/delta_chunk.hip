@@ -29,6 +29,7 @@
 
 namespace {
 
+constexpr int BUFFER_BYTES = 0x00027000;       // fourth word of a buffer: raw bytes
 constexpr int C = 64;       // tokens per chunk
 constexpr int B = 16;       // tokens per block
 constexpr int LT = 512;     // threads of delta_chunk_local
@@ -473,8 +474,11 @@ __global__ __launch_bounds__(LT, 4) void delta_chunk_local_kernel(
 // In 32-bit the matrix instructions bound it: 223 us of 297 for 16 chunks of 8
 // sequences, 32 heads of 128 x 128. With two tiles values are sums of three bf16
 // instead, six products of which take 3/8 of the time: 254 us, 172 of them with
-// operands that are in cache (now the splitting of operands, 2400 instructions per
-// chunk and wave, and the waits), the error of outputs 3.52e-7 instead of 4.18e-7.
+// operands that are in cache, the error of outputs 3.52e-7 instead of 4.18e-7. Vector
+// instructions bound it then, the splitting of operands first of them: with a rounded
+// pair taken out of one word, operands by way of a buffer and no masks around whole
+// chunks' stores it is 1500 instructions per chunk and wave (1970), 126 chunks of 8
+// prompts in a pass 287 -> 253 us, the same bits.
 // With one tile the splitting costs more than it saves (31 chunks of one sequence
 // 112 us, in 32-bit 91); four tiles do not fit the registers (+ 7 %).
 typedef __attribute__((ext_vector_type(8))) float float8v;
@@ -483,14 +487,26 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 template <int N> struct Vec;
 template <> struct Vec<4> { typedef float4v F; typedef bf16x4 H; };
 template <> struct Vec<8> { typedef float8v F; typedef bf16x8 H; };
-// 32-bit values as sums of three bf16 (high, middle, low): 24 bits of them
+// 32-bit values as sums of three bf16 (high, middle, low): 24 bits of them. Two at a
+// time, the rounded values taken out of the word that holds both (converted back as
+// vectors each is rounded once more by itself, 4 instructions of 15 per pair and part).
 template <int N>
 __device__ __forceinline__ void split(typename Vec<N>::F f,
                                       typename Vec<N>::H (&o)[3]) {
+  typedef __attribute__((ext_vector_type(N / 2))) unsigned int Words;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    o[i] = __builtin_convertvector(f, typename Vec<N>::H);
-    if (i < 2) f -= __builtin_convertvector(o[i], typename Vec<N>::F);
+    Words w;
+#pragma unroll
+    for (int x = 0; x < N; x += 2) {
+      const unsigned int two = __builtin_bit_cast(
+          unsigned int, __builtin_convertvector((float2v){f[x], f[x + 1]}, bf16x2));
+      w[x / 2] = two;
+      f[x] -= __builtin_bit_cast(float, two << 16);
+      f[x + 1] -= __builtin_bit_cast(float, two & 0xffff0000u);
+    }
+    o[i] = __builtin_bit_cast(typename Vec<N>::H, w);
   }
 }
 __device__ __forceinline__ void split2(float4v a, float4v b, bf16x8 (&o)[3]) {
@@ -521,7 +537,8 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
   constexpr int TILE = SPLIT ? WAVE * 3 / 2 : WAVE;
   __shared__ float4v s_lds[NC][KT * TILE], u_lds[NC][4 * TILE];
   const int h = blockIdx.x, lane = threadIdx.x % WAVE;
-  const int wave = threadIdx.x / WAVE, col = lane % 16, g4 = 4 * (lane / 16);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int col = lane % 16, g4 = 4 * (lane / 16);
   auto put = [&](float4v* to, int tile, float4v f) {
     if constexpr (SPLIT) {
       bf16x4 o[3];
@@ -565,50 +582,58 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
   const int tw = wave * B;            // this wave's 16 tokens
   const int64_t stride = (int64_t)H * work_size(KP, VP);
   const float* base = ws + (chunk0 * H + h) * work_size(KP, VP);
-  const unsigned at_w = wave * KT * 256 + lane * 4;
+  const unsigned at_w = wave * KT * 1024 + lane * 16;    // bytes
   unsigned at_u[NC];                  // past the last tile: that one's
 #pragma unroll
   for (int x = 0; x < NC; ++x)
-    at_u[x] = (min((int)blockIdx.y * NC + x, VP / 16 - 1) * 4 + wave) * 256 +
-              lane * 4;
-  const unsigned at_p = wave * 4 * 256 + lane * 4;
+    at_u[x] = (min((int)blockIdx.y * NC + x, VP / 16 - 1) * 4 + wave) * 1024 +
+              lane * 16;
+  const unsigned at_p = wave * 4 * 1024 + lane * 16;
   // of 32 channels, the third and fourth wave have no tile of their own
-  const unsigned at_k = wave % KT * 4 * 256 + lane * 4;
-  const unsigned at_g = wave % KT * B + g4;
+  const unsigned at_k = wave % KT * 4 * 1024 + lane * 16;
+  const unsigned at_g = (wave % KT * B + g4) * 4;
+  // by way of a buffer, whose offsets take no vector instructions
+  const int work_bytes = (int)work_size(KP, VP) * 4;
+  auto buffer = [&](const float* p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, work_bytes, BUFFER_BYTES);
+  };
+  auto load = [&](__amdgpu_buffer_rsrc_t b, unsigned lane_at, int at) {
+    return __builtin_bit_cast(float4v,
+                              __builtin_amdgcn_raw_buffer_load_b128(b, lane_at, at, 0));
+  };
+  const int off_w = C * VP * 4, off_q = off_w + C * KP * 4, off_k = off_q + C * KP * 4;
+  const int off_p = off_k + C * KP * 4, off_g = off_p + C * C * 4;
   float4v w[KT], qe[KT], u[NC];
   auto fetch = [&](const float* p) {  // in the order of their use
-    const float* pw = p + C * VP;
-    const float* pq = pw + C * KP;
+    const auto b = buffer(p);
 #pragma unroll
-    for (int x = 0; x < NC; ++x) u[x] = *(const float4v*)(p + at_u[x]);
+    for (int x = 0; x < NC; ++x) u[x] = load(b, at_u[x], 0);
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      w[t] = *(const float4v*)(pw + (at_w + 256 * t));
-      qe[t] = *(const float4v*)(pq + (at_w + 256 * t));
+      w[t] = load(b, at_w, off_w + 1024 * t);
+      qe[t] = load(b, at_w, off_q + 1024 * t);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
   fetch(base);
   float* oc = out + (row0 * H + h) * V;
   const unsigned at_o = (tw + g4) * (H * V) + c0, orow = H * V;
+  const bool all_columns = (int)(blockIdx.y + 1) * 16 * NC <= V;
   // No load of the loop is under a condition: the compiler could not count
   // what is under way, and would wait for all of it.
   for (int t0 = 0; t0 < n; t0 += C, oc += C * orow) {
     // operands of the state update and of P U, used after the first products
     float4v kt[MY][4], decay[MY], p[4];
-    const float* pk = base + C * VP + 2 * C * KP;
-    const float* pp = pk + C * KP;
-    const float* pg = pp + C * C;
+    const auto b = buffer(base);
 #pragma unroll
     for (int i = 0; i < MY; ++i) {
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
-        kt[i][x] = *(const float4v*)(pk + (at_k + i * 4096 + 256 * x));
-      decay[i] = *(const float4v*)(pg + (at_g + i * 4 * B));
+      for (int x = 0; x < 4; ++x) kt[i][x] = load(b, at_k, off_k + i * 16384 + 1024 * x);
+      decay[i] = load(b, at_g, off_g + i * 4 * B * 4);
     }
 #pragma unroll
     for (int x = 0; x < 4; ++x)       // those past the wave's own are not used
-      p[x] = *(const float4v*)(pp + (at_p + 256 * x));
+      p[x] = load(b, at_p, off_p + 1024 * x);
     __builtin_amdgcn_sched_barrier(0);    // now, not where they are used
     float4v o[NC];
 #pragma unroll
@@ -690,13 +715,20 @@ __global__ __launch_bounds__(ST, 2) void delta_chunk_scan_kernel(
     for (int x = 0; x < NC; ++x)
 #pragma unroll
       for (int i = 0; i < MY; ++i)
-        if (wave + 4 * i < KT) put(s_lds[x], wave + 4 * i, S[x][i]);
+        if (KT % 4 == 0 || wave + 4 * i < KT) put(s_lds[x], wave + 4 * i, S[x][i]);
+    if (t0 + C <= n && all_columns) {
 #pragma unroll
-    for (int x = 0; x < NC; ++x)
+      for (int x = 0; x < NC; ++x)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (t0 + tw + g4 + r < n && c0 + 16 * x < V)
-          oc[at_o + r * orow + 16 * x] = o[x][r];
+        for (int r = 0; r < 4; ++r) oc[at_o + r * orow + 16 * x] = o[x][r];
+    } else {
+#pragma unroll
+      for (int x = 0; x < NC; ++x)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (t0 + tw + g4 + r < n && c0 + 16 * x < V)
+            oc[at_o + r * orow + 16 * x] = o[x][r];
+    }
     lds_barrier();
   }
 
