@@ -189,6 +189,82 @@ __global__ __launch_bounds__(NT) void heads_to_rows_kernel(
     dst[row * H * V + i] = src[((int64_t)(i / V) * n_abs + row) * V + i % V];
 }
 
+// y[t][h] = x[t][h] w[h]' for few rows t of every head (bf16, 32-bit sums): the products
+// around latent decode attention. A head's weights are small, so what a launch takes is
+// one way of loads: workgroups of 16 rows by 64 channels, whose four waves share K in
+// steps of 128, or the channels where K is short, load everything of a step by 256 bytes
+// of a row at once.
+struct HeadProducts {
+  const short *x, *w;        // w [H, N, K]
+  short* y;
+  int64_t x_row, x_head, y_row, y_head;   // strides in elements
+  int T, N, K;
+};
+template <int KW>            // waves that share K: 1, 2 or 4
+__global__ __launch_bounds__(256) void head_products_kernel(const HeadProducts p) {
+  typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+  typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+  __shared__ __align__(16) char lds[4 * 4096];   // 4 KB of a wave; then the waves' sums
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int lane = threadIdx.x % WAVE, col = lane % 16, grp = lane / 16;
+  const int kw = wave % KW, c0 = wave / KW * KW;         // of the 64 channels, by 16
+  const int n0 = blockIdx.x * 64, h = blockIdx.y, t0 = blockIdx.z * 16;
+  const int N = p.N, K = p.K;
+  const short* const x = p.x + (int64_t)t0 * p.x_row + h * p.x_head;
+  const short* const w = p.w + (int64_t)h * N * K;
+  char* const mine = lds + wave * 4096;
+  const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  const int last = min(p.T - 1 - t0, 15);
+  float4v acc[KW];
+#pragma unroll
+  for (int c = 0; c < KW; ++c) acc[c] = (float4v){0.f, 0.f, 0.f, 0.f};
+  // past the end of K the rows count as zero; rows and channels past the end repeat the
+  // last one
+  for (int k0 = kw * 128; k0 < K; k0 += KW * 128) {
+    short8 a[4], b[KW][4];
+    const int k = k0 + col * 8, kc = min(k, K - 8);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int r = j * 4 + grp;
+      a[j] = *(const short8*)(x + min(r, last) * p.x_row + kc);
+#pragma unroll
+      for (int c = 0; c < KW; ++c)
+        b[c][j] = *(const short8*)(
+            w + (int64_t)min(n0 + (c0 + c) * 16 + r, N - 1) * K + kc);
+    }
+    __builtin_amdgcn_sched_barrier(0);       // all loads ahead of their first use
+    if (k >= K)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) a[j] = zero;
+    to_operand(mine, lane, a);
+#pragma unroll
+    for (int c = 0; c < KW; ++c) {
+      to_operand(mine, lane, b[c]);
+#pragma unroll
+      for (int f = 0; f < 4; ++f)
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(bf16x8, b[c][f]), __builtin_bit_cast(bf16x8, a[f]),
+            acc[c], 0, 0, 0);
+    }
+  }
+  // wave: 16 channels of the sums
+  float4v sum = acc[0];
+  if constexpr (KW > 1) {
+    float4v* const sums = (float4v*)lds;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < KW; ++c) sums[(kw * 4 + c0 + c) * WAVE + lane] = acc[c];
+    __syncthreads();
+    sum = sums[wave * WAVE + lane];
+#pragma unroll
+    for (int v = 1; v < KW; ++v) sum += sums[(v * 4 + wave) * WAVE + lane];
+  }
+  const int n = n0 + wave * 16 + grp * 4;
+  if (col <= last && n < N)
+    *(bf16x4*)(p.y + (int64_t)(t0 + col) * p.y_row + h * p.y_head + n) =
+        __builtin_convertvector(sum, bf16x4);
+}
+
 // rows of the cache at `slots`, contiguous; unit: bytes moved per lane
 template <typename U>
 __global__ __launch_bounds__(NT) void gather_rows_kernel(
@@ -434,6 +510,28 @@ hipError_t lds_heads_to_rows(int f32, const void* src, void* dst, int n_abs,
                      stream, (const T*)src, (T*)dst, n_abs, H, V)
   if (f32) GO(float); else GO(short);
 #undef GO
+  HIP_CHECK_LAST();
+  return hipSuccess;
+}
+
+// x, y: rows and heads apart by strides of 4 elements and more, 16 and 8 bytes aligned; N
+// and K multiples of 8
+hipError_t lds_head_products(const void* x, int64_t x_row, int64_t x_head, const void* w,
+                             void* y, int64_t y_row, int64_t y_head, int T, int H, int N,
+                             int K, hipStream_t stream) {
+  if (T == 0) return hipSuccess;
+  if (N < 8 || N % 8 || K < 8 || K % 8 || x_row % 8 || x_head % 8 || y_row % 4 ||
+      y_head % 4 || T > 16 * 65535 || H > 65535)
+    return hipErrorInvalidValue;
+  const HeadProducts p{(const short*)x, (const short*)w, (short*)y, x_row, x_head,
+                       y_row, y_head, T, N, K};
+  const dim3 grid((N + 63) / 64, H, (T + 15) / 16);
+  if (K <= 128)
+    hipLaunchKernelGGL(head_products_kernel<1>, grid, dim3(256), 0, stream, p);
+  else if (K <= 256)
+    hipLaunchKernelGGL(head_products_kernel<2>, grid, dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL(head_products_kernel<4>, grid, dim3(256), 0, stream, p);
   HIP_CHECK_LAST();
   return hipSuccess;
 }

@@ -108,3 +108,17 @@ __device__ __forceinline__ Seq load_seq(const int32_t* meta, int s) {
   const int4 m = ((const int4*)meta)[s];
   return {m.x, m.y, m.z, m.w};
 }
+
+// A wave's 16 rows by 128 columns, loaded by 256 bytes of a row (x[j]: row j * 4 + lane /
+// 16, columns lane % 16 * 8), as operands of four matrix instructions (x[f]: row lane %
+// 16, columns f * 32 + lane / 16 * 8), by way of the wave's 4 KB of LDS.
+__device__ __forceinline__ void to_operand(char* lds, int lane, short8* x) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int r = j * 4 + lane / 16;
+    *(short8*)(lds + r * 256 + (lane % 16 ^ r) * 16) = x[j];
+  }
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+    x[f] = *(const short8*)(lds + lane % 16 * 256 + ((f * 4 + lane / 16) ^ lane % 16) * 16);
+}

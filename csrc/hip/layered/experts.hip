@@ -55,20 +55,6 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
   if (wave == 0) take_top(z, E, top, ids + row * top, wt + row * top);
 }
 
-// A wave's 16 rows by 128 columns, loaded by 256 bytes of a row (x[j]: row j * 4 + lane /
-// 16, columns lane % 16 * 8), as operands of four matrix instructions (x[f]: row lane %
-// 16, columns f * 32 + lane / 16 * 8), by way of the wave's 4 KB of LDS.
-__device__ __forceinline__ void to_operand(char* lds, int lane, short8* x) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = j * 4 + lane / 16;
-    *(short8*)(lds + r * 256 + (lane % 16 ^ r) * 16) = x[j];
-  }
-#pragma unroll
-  for (int f = 0; f < 4; ++f)
-    x[f] = *(const short8*)(lds + lane % 16 * 256 + ((f * 4 + lane / 16) ^ lane % 16) * 16);
-}
-
 // 16 rows per workgroup. EG groups of KW waves have 16 ET experts each and share K.
 // Bound by what a compute unit can load: the lanes of a load are to follow each other in
 // a row of memory, as operands they lie in 16 rows and a load took four times as long.

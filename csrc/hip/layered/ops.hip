@@ -36,6 +36,8 @@ hipError_t lds_latent_prep(int, const void*, int64_t, const float*,
                            float, hipStream_t);
 hipError_t lds_rope_part(int, void*, void*, const float*, const int32_t*, int,
                          int, int, int, int, hipStream_t);
+hipError_t lds_head_products(const void*, int64_t, int64_t, const void*, void*, int64_t,
+                             int64_t, int, int, int, int, hipStream_t);
 hipError_t lds_heads_to_rows(int, const void*, void*, int, int, int,
                              hipStream_t);
 hipError_t lds_gather_rows(const void*, const int64_t*, void*, int64_t,
@@ -417,6 +419,29 @@ Tensor rope_part(Tensor q, Tensor cos_sin, Tensor positions, int64_t n_abs) {
   return by_head;
 }
 
+// y [T, H, N] = x [T, H, K] w [H, N, K]' by head, x and y with strides of their own; false
+// where there is no such form
+bool head_products(Tensor x, Tensor w, Tensor y) {
+  TORCH_CHECK(x.is_cuda() && y.is_cuda() && x.dim() == 3 && y.dim() == 3, "x, y");
+  const int64_t T = x.size(0), H = x.size(1), K = x.size(2), N = y.size(2);
+  TORCH_CHECK(w.is_cuda() && w.is_contiguous(), "w");
+  sized(w, {H, N, K}, "w");
+  sized(y, {T, H, N}, "y");
+  TORCH_CHECK(x.scalar_type() == y.scalar_type() && x.scalar_type() == w.scalar_type(),
+              "types");
+  if (x.scalar_type() != at::kBFloat16 || K % 8 || N % 8 || K < 8 || N < 8 ||
+      x.stride(2) != 1 || y.stride(2) != 1 || x.stride(0) % 8 || x.stride(1) % 8 ||
+      y.stride(0) % 4 || y.stride(1) % 4 || T > 16 * 65535 || H > 65535 ||
+      ((uintptr_t)x.data_ptr() | (uintptr_t)w.data_ptr()) % 16 ||
+      (uintptr_t)y.data_ptr() % 8)
+    return false;
+  check_hip(lds_head_products(x.data_ptr(), x.stride(0), x.stride(1), w.data_ptr(),
+                              y.data_ptr(), y.stride(0), y.stride(1), (int)T, (int)H,
+                              (int)N, (int)K, cur_stream()),
+            "head_products");
+  return true;
+}
+
 // src [H, n, V] -> the first n rows of dst [rows, H V]
 void heads_to_rows(Tensor src, Tensor dst) {
   const int f32 = act(src, "src");
@@ -560,6 +585,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_prep", &latent_prep);
   m.def("rope_part", &rope_part);
   m.def("heads_to_rows", &heads_to_rows);
+  m.def("head_products", &head_products);
   m.def("gather_rows", &gather_rows);
   m.def("latent_decode", &latent_decode);
   m.def("latent_prefill", &latent_prefill);

@@ -179,6 +179,12 @@ def rope_part(q, cos_sin, positions, n_abs):
     return _impl(q).rope_part(q, cos_sin, positions, n_abs)
 
 
+def head_products(x, w, y):
+    """y [T, H, N] = x [T, H, K] w [H, N, K]' by head (x and y may be views) for
+    few rows; False where there is no kernel for the types and sizes."""
+    return x.is_cuda and hip_layered().head_products(x, w, y)
+
+
 def heads_to_rows(src, dst):
     _impl(src).heads_to_rows(src, dst)
 

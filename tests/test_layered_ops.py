@@ -678,3 +678,29 @@ class TestLatentAttention:
                                tiles, rot, window, scale, out, plain)
             assert not out[:base].any()
             close(out[base:], want, run, f32=1e-5, bf16=1.2e-2)
+
+
+@GPU
+@pytest.mark.parametrize("T,H,N,K", [(1, 3, 8, 8), (15, 2, 64, 128), (16, 4, 72, 136),
+                                     (17, 1, 512, 128), (50, 5, 128, 512),
+                                     (33, 2, 200, 256), (256, 2, 56, 1032)])
+@pytest.mark.parametrize("by_head", [True, False])
+def test_head_products(T, H, N, K, by_head):
+    """Every split of K, ends of steps, rows and channels; operands in both orders of
+    rows and heads, the columns of wider rows."""
+    run = ("cuda:0", torch.bfloat16)
+    x = put(rnd(T, H, K + 16, seed=1), run)[:, :, 8:-8]
+    w = put(rnd(H, N, K, seed=2, scale=K ** -0.5), run)
+    y = put(torch.full((H, T, N), 9.), run).transpose(0, 1)
+    if by_head:
+        x = x.transpose(0, 1).contiguous().transpose(0, 1)
+    else:
+        y = put(torch.full((T, H, N), 9.), run)
+    assert ops.head_products(x, w, y)
+    want = (f64(x).transpose(0, 1) @ f64(w).transpose(1, 2)).transpose(0, 1)
+    # rounded to 8 bits, 32-bit sums beside that
+    close(y, want, run, bf16=2 ** -8)
+    if K % 16 == 8:                 # rows that are not 16 bytes apart
+        assert ops.head_products(put(rnd(T, H, K + 4), run)[:, :, :K], w, y) == (
+            (K + 4) % 8 == 0)
+    assert not ops.head_products(x.float(), w.float(), y.float())
