@@ -11,10 +11,13 @@
 // The chunked form for long rows is in delta_chunk.hip.
 #include "elem.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int NT = 256;
 constexpr int NWV = NT / WAVE;
+constexpr int AHEAD = 4;  // rows that delta_prep's threads ask for at once
 constexpr int MAXU = 8;  // unit norm over up to MAXU * 64 channels
 
 // grid (rows, y): waves share the units of one row. Units: KH of q, KH of k
@@ -99,53 +102,81 @@ __global__ __launch_bounds__(NT) void delta_prep_vec_kernel(
 #pragma unroll
   for (int j = 0; j < TAPS; ++j) ldn<8>(taps + (int64_t)j * C + cc, w[j]);
   const int r0 = blockIdx.y * RB, r1 = min(rows, r0 + RB);
-  for (int row = r0; row < r1; ++row) {
-    const Seq sq = load_seq(seq_meta, row_seq[row]);
-    const int pos = row - sq.row0;
-    T* state = conv_state + (int64_t)sq.slot * (TAPS - 1) * C + cc;
-    if (row == r0 || pos == 0) {
+  typedef typename std::conditional<
+      sizeof(T) == 2, short8, __attribute__((ext_vector_type(8))) float>::type Eight;
+  // a block's rows are of one sequence, as a rule: it is looked up once then
+  const int s0 = row_seq[r0];
+  const bool one = row_seq[r1 - 1] == s0;
+  Seq sq = load_seq(seq_meta, s0);
+  Eight raw[AHEAD];
+  auto ask = [&](int row) {
 #pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) {
-        const int p = pos - (TAPS - 1) + j;
-        if (p >= 0) {
-          ldn<8>(proj + (int64_t)(sq.row0 + p) * pstride + cc, x[j]);
-        } else if (sq.prior > 0) {
-          ldn<8>(state + (int64_t)(TAPS - 1 + p) * C, x[j]);
-        } else {
+    for (int i = 0; i < AHEAD; ++i)
+      raw[i] = *(const Eight*)(proj + (int64_t)min(row + i, r1 - 1) * pstride + cc);
+  };
+  ask(r0);
+  for (int first = r0; first < r1; first += AHEAD) {
+    Eight now[AHEAD];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[j][e] = 0.f;
+    for (int i = 0; i < AHEAD; ++i) now[i] = raw[i];
+    if (first + AHEAD < r1) ask(first + AHEAD);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int row = first + i;
+      if (row >= r1) break;
+      if (!one) sq = load_seq(seq_meta, row_seq[row]);
+      const int pos = row - sq.row0;
+      T* state = conv_state + (int64_t)sq.slot * (TAPS - 1) * C + cc;
+      if (row == r0 || pos == 0) {
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) {
+          const int p = pos - (TAPS - 1) + j;
+          if (p >= 0) {
+            ldn<8>(proj + (int64_t)(sq.row0 + p) * pstride + cc, x[j]);
+          } else if (sq.prior > 0) {
+            ldn<8>(state + (int64_t)(TAPS - 1 + p) * C, x[j]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[j][e] = 0.f;
+          }
         }
       }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if constexpr (sizeof(T) == 2)
+          x[TAPS - 1][e] = bf16_to_f32(now[i][e]);
+        else
+          x[TAPS - 1][e] = now[i][e];
+      }
+      if (sq.n == 1 && in) {
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) stn<8>(state + (int64_t)j * C, x[j + 1]);
+      }
+      float f[8], ss = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        float a = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) a += w[j][e] * x[j][e];
+        f[e] = a * sigmoid_f(a);
+        ss += f[e] * f[e];
+      }
+      for (int o = K / 16; o > 0; o /= 2) ss += __shfl_xor(ss, o, WAVE);
+      if (qk) {
+        const float m = (cc < QK ? q_scale : 1.f) / sqrtf(ss + unit_eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[e] *= m;
+      }
+      if (in)
+        stn<8>(cc < QK       ? q + (int64_t)row * QK + cc
+               : cc < 2 * QK ? k + (int64_t)row * QK + cc - QK
+                             : v + (int64_t)row * H * V + cc - 2 * QK,
+               f);
+#pragma unroll
+      for (int j = 0; j < TAPS - 1; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[j][e] = x[j + 1][e];
     }
-    ldn<8>(proj + (int64_t)row * pstride + cc, x[TAPS - 1]);
-    if (sq.n == 1 && in) {
-#pragma unroll
-      for (int j = 0; j < TAPS - 1; ++j) stn<8>(state + (int64_t)j * C, x[j + 1]);
-    }
-    float f[8], ss = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float a = 0.f;
-#pragma unroll
-      for (int j = 0; j < TAPS; ++j) a += w[j][e] * x[j][e];
-      f[e] = a * sigmoid_f(a);
-      ss += f[e] * f[e];
-    }
-    for (int o = K / 16; o > 0; o /= 2) ss += __shfl_xor(ss, o, WAVE);
-    if (qk) {
-      const float m = (cc < QK ? q_scale : 1.f) / sqrtf(ss + unit_eps);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) f[e] *= m;
-    }
-    if (in)
-      stn<8>(cc < QK       ? q + (int64_t)row * QK + cc
-             : cc < 2 * QK ? k + (int64_t)row * QK + cc - QK
-                           : v + (int64_t)row * H * V + cc - 2 * QK,
-             f);
-#pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) x[j][e] = x[j + 1][e];
   }
 }
 
