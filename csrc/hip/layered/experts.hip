@@ -55,13 +55,17 @@ __global__ __launch_bounds__(256) void route_plain_kernel(
   if (wave == 0) take_top(z, E, top, ids + row * top, wt + row * top);
 }
 
-// 16 rows per workgroup. EG groups of KW waves have 16 ET experts each and share K.
+// R rows per workgroup: 16 of a matrix instruction, or 4 where that is at most a round of
+// workgroups. EG groups of KW waves have 16 ET experts each and share K.
 // Bound by what a compute unit can load: the lanes of a load are to follow each other in
 // a row of memory, as operands they lie in 16 rows and a load took four times as long.
 // 32 experts of 4096, 60 rows 9.8 us (15.0), 7800 rows 20.4 (32.9); 64 experts 17.2
-// (26.8), 31.0 (48.0); 128 of 2048 23.8 (38.4), 43.8 (61.8). 16 waves in place of 8 are
+// (26.8), 31.0 (48.0); 128 of 2048 23.8 (38.4), 43.8 (61.8). By 4 rows a unit loads a
+// quarter less and a wave chooses for one: 60 rows again, warm, by 16 / by 4: 8.3 / 6.6 us,
+// 64 experts 13.6 / 10.6, 128 of 2048 19.5 / 15.7; 1000 rows 8.7 / 7.2, 14.2 / 11.1, 19.9 /
+// 17.6. Two steps of K asked for together are no faster. 16 waves in place of 8 are
 // no faster up to 64 experts (9.6 and 23.7 us for 32), above they are (27.3 and 40.6 by 8).
-template <int ET, int EG, int KW>
+template <int ET, int EG, int KW, int R>
 __global__ __launch_bounds__(EG * KW * WAVE) void route_kernel(
     const short* __restrict__ h, const short* __restrict__ w,
     int32_t* __restrict__ ids, float* __restrict__ wt, int64_t rows, int K,
@@ -71,7 +75,7 @@ __global__ __launch_bounds__(EG * KW * WAVE) void route_kernel(
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
   const int col = lane % 16, grp = lane / 16;
   const int e0 = wave / KW * ET * 16, kw = wave % KW;
-  const int64_t row0 = (int64_t)blockIdx.x * 16;
+  const int64_t row0 = (int64_t)blockIdx.x * R;
   char* mine = (char*)lds + wave * 4096;
   const short8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
   float4v acc[ET];
@@ -79,14 +83,14 @@ __global__ __launch_bounds__(EG * KW * WAVE) void route_kernel(
   for (int t = 0; t < ET; ++t) acc[t] = (float4v){0.f, 0.f, 0.f, 0.f};
   // past the end of K the row counts as zero; experts past E are not looked at
   const short* h0 = h + row0 * K;
-  const int last = min(rows - 1 - row0, (int64_t)15);
+  const int last = min(rows - 1 - row0, (int64_t)(R - 1));
   for (int k0 = kw * 128; k0 < K; k0 += KW * 128) {
     short8 a[4], b[ET][4];
     const int k = k0 + col * 8, kc = min(k, K - 8);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int r = j * 4 + grp;
-      a[j] = *(const short8*)(h0 + (uint32_t)(min(r, last) * K + kc));
+      a[j] = j * 4 < R ? *(const short8*)(h0 + (uint32_t)(min(r, last) * K + kc)) : zero;
 #pragma unroll
       for (int t = 0; t < ET; ++t)
         b[t][j] =
@@ -112,14 +116,14 @@ __global__ __launch_bounds__(EG * KW * WAVE) void route_kernel(
   for (int t = 0; t < ET; ++t)
     *(float4v*)(lds + (kw * 16 + col) * 16 * ES + e0 + t * 16 + grp * 4) = acc[t];
   __syncthreads();
-  for (int i = threadIdx.x; i < 256 * ES; i += EG * KW * WAVE) {
+  for (int i = threadIdx.x; i < 16 * R * ES; i += EG * KW * WAVE) {
     float s = lds[i];
 #pragma unroll
     for (int v = 1; v < KW; ++v) s += lds[v * 256 * ES + i];
     lds[i] = s;
   }
   __syncthreads();
-  for (int r = wave; r < 16 && row0 + r < rows; r += EG * KW)
+  for (int r = wave; r < R && row0 + r < rows; r += EG * KW)
     take_top(lds + r * 16 * ES, E, top, ids + (row0 + r) * top,
              wt + (row0 + r) * top);
 }
@@ -569,14 +573,20 @@ hipError_t lds_route(int f32, const void* h, const void* w, int32_t* ids,
     return hipSuccess;
   }
 #define GO(ET, EG, KW)                                                        \
-  hipLaunchKernelGGL((route_kernel<ET, EG, KW>),                              \
-                     dim3((uint32_t)((rows + 15) / 16)),                      \
+  do {                                                                        \
+    if (rows <= 4 * 256) GO_R(ET, EG, KW, 4);                                 \
+    else GO_R(ET, EG, KW, 16);                                                \
+  } while (0)
+#define GO_R(ET, EG, KW, R)                                                   \
+  hipLaunchKernelGGL((route_kernel<ET, EG, KW, R>),                           \
+                     dim3((uint32_t)((rows + R - 1) / R)),                    \
                      dim3(EG * KW * WAVE), EG * KW * 4096, stream,            \
                      (const short*)h, (const short*)w, ids, wt, rows, K, E, top)
   if (E <= 16) GO(1, 1, 8); else if (E <= 32) GO(2, 1, 8);
   else if (E <= 64) GO(2, 2, 4); else if (E <= 128) GO(2, 4, 4);
   else GO(2, 8, 2);
 #undef GO
+#undef GO_R
   HIP_CHECK_LAST();
   return hipSuccess;
 }

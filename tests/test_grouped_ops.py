@@ -412,6 +412,20 @@ def test_route_by_groups_of_experts(T, K, E, top):
     assert (torch.gather(s, 1, ids.cpu().long()) - want).abs().max() < 6e-6
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [3, 4, 5, 1023, 1024, 1025])
+@pytest.mark.parametrize("K,E,top", [(136, 32, 4), (512, 130, 8)])
+def test_route_by_4_and_16_rows(T, K, E, top):
+    run = ("cuda", torch.bfloat16)
+    h, w = put(rnd(T, K), run), put(rnd(E, K, seed=1, scale=K ** -0.5), run)
+    ids, wt = ops.route(h, w, top)
+    _, want = oracle.route(f64(h), f64(w), top)
+    # as above
+    assert (wt.cpu().double() - want).abs().max() < 6e-6
+    s = oracle.sigmoid(f64(h) @ f64(w).T)
+    assert (torch.gather(s, 1, ids.cpu().long()) - want).abs().max() < 6e-6
+
+
 SHAPES = [(38, 11, 5), (64, 24, 7), (64, 64, 4), (192, 320, 6), (128, 200, 3)]
 
 
