@@ -456,8 +456,14 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
         positions, row_seq, 1, max_blocks, bs, (short*)out, part_o, part_ml, G,
         H / G, part_tokens, part_tokens > 0 && n % 2 == 0, scale, sink * LOG2E,
         has_sink};
-    // short rows leave half of 8 waves without a tile
-    const int waves = max_ctx <= 256 ? 4 : 8;
+    // Short rows leave half of 8 waves without a tile; where a compute unit has several
+    // workgroups to do, three of 4 waves fit it and one of 8 (256 rows of 500 tokens, 8
+    // key heads, groups of 8: 102 us by 8, 95 by 4; of 1000 95 and 95; 20 rows of 7000 in
+    // parts: 106 and 103).
+    const int64_t groups = (int64_t)n * G;
+    const bool four = parts > 1 ? part_tokens == 0 && groups > 128 && groups < 200
+                                : groups > 256 && max_ctx <= 1024;
+    const int waves = max_ctx <= 256 || four ? 4 : 8;
     if (parts > 64) return hipErrorInvalidValue;
     return parts > 1 ? decode::attend<true, 256>(w, n, parts, waves, stream)
                      : decode::attend<false, 256>(w, n, 1, waves, stream);

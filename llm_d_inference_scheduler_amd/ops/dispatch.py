@@ -150,9 +150,13 @@ def decode_parts(groups: int, max_len: int,
     """-> (parts, tokens per part) of the decode attention of `groups`
     (sequence, key head) pairs of up to max_len tokens, and of mean_len on
     average (None: 0.8 of that, lengths a quarter either way), of `elem` bytes a
-    value. A workgroup of 8 waves takes 256 tokens a step, and about 512 of them
-    fill the chip: parts make up for fewer groups as long as each has a step of its
-    own. They cost their sums and a second launch. In us: one part takes 3 and as
+    value. A workgroup of 8 waves takes 256 tokens a step, and a compute unit has
+    registers for one of them or three of 4 waves: parts make up for fewer than 128
+    groups by one round of the former, from there on by a round of the latter, as long
+    as each has a step of its own (as many as make up 512, mostly two rounds and the
+    beginning of a third, / so, us, 8 key heads: 3 of 7000, 8-bit 20.7 / 15.7; 8 of
+    4000 33 / 29, 8-bit 22.6 / 19.9; 10 of 4000 45 / 33.5, 8-bit 30.5 / 22; 17 of 6800,
+    8-bit 56.6 / 50.6; 20 of 7000 121 / 103.6). They cost their sums and a second launch. In us: one part takes 3 and as
     long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
     at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 340 batches, lengths
     alike or down to a twentieth of the longest, the choice costs 0.4 % on average
@@ -175,7 +179,8 @@ def decode_parts(groups: int, max_len: int,
         mean = 0.8 * max_len if mean_len is None else mean_len
         size = groups * mean * 256 * elem
         if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
-            parts = -(-512 // max(1, groups))
+            parts = max(2, 256 // max(1, groups)) if groups <= 128 \
+                else -(-768 // groups)
     if mean_len is not None and max_len > 1.4 * mean_len:
         # tokens that one workgroup may walk while each compute unit takes one
         # and a half shares of the whole
@@ -188,6 +193,23 @@ def decode_parts(groups: int, max_len: int,
     return -(-max_len // part), part
 
 
+def decode_waves(groups: int, parts: int, max_len: int,
+                 mean_len: Optional[float] = None, elem: int = 2) -> int:
+    """Waves of a workgroup of the decode attention, 4 or 8. Short sequences leave
+    half of 8 without a tile (100 sequences of 120 tokens: 19 us with 8 waves, 15 with
+    4). Where a compute unit has several workgroups to do, three of 4 waves have more
+    under way than one of 8, which counts with few bytes a tile, and their ends overlap:
+    in parts as many as make that up (decode_parts), in one part from 257 groups on, in
+    8 bits or up to 1024 tokens (8 / 4 waves, us: 40 of 600, 28 / 27, 8-bit 18.8 / 16.6;
+    100 of 300 32.4 / 28.2, 24.2 / 18.6; 256 of 500 96 / 91, 71 / 53; 256 of 1500 252 /
+    257, 145 / 137; 32 of 300 11.9 / 12.1, 10.1 / 10.2)."""
+    if parts > 1:
+        alike = mean_len is None or max_len <= 1.4 * mean_len
+        return 4 if max_len <= 256 or (alike and 128 < groups < 200) else 8
+    return 4 if max_len <= 256 or (groups > 256 and
+                                   (elem == 1 or max_len <= 1024)) else 8
+
+
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
                     v_cache: torch.Tensor, block_tables: torch.Tensor,
                     seq_lens: torch.Tensor, scale: float,
@@ -198,12 +220,9 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,
         sl = seq_lens.to(torch.int32)
         waves = 8
         if max_seq_len is not None and max_seq_len > 0:
-            # short sequences leave half of 8 waves without a tile (100
-            # sequences of 120 tokens: 19 us with 8 waves, 15 with 4)
-            waves = 4 if max_seq_len <= 256 else 8
-            parts, part = decode_parts(q.shape[0] * k_cache.shape[1],
-                                       max_seq_len, mean_seq_len,
-                                       k_cache.element_size())
+            groups, elem = q.shape[0] * k_cache.shape[1], k_cache.element_size()
+            parts, part = decode_parts(groups, max_seq_len, mean_seq_len, elem)
+            waves = decode_waves(groups, parts, max_seq_len, mean_seq_len, elem)
             if parts > 1:
                 far_apart = mean_seq_len is not None and \
                     max_seq_len > 2 * mean_seq_len

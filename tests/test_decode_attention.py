@@ -43,6 +43,21 @@ def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
     assert (parts > 1) == (several < one)
 
 
+@pytest.mark.parametrize("groups,max_len,mean,elem,eight,four", [
+    (256, 374, None, 2, 11.9, 12.1), (256, 374, None, 1, 10.1, 10.2),
+    (272, 748, None, 2, 26.7, 25.9), (320, 748, 600, 1, 18.8, 16.6),
+    (320, 1871, 1500, 2, 57.0, 57.5), (320, 1871, None, 1, 33.0, 31.0),
+    (800, 374, None, 2, 32.4, 28.2), (2048, 624, None, 1, 70.6, 53.3),
+    (2048, 1871, None, 2, 252, 257), (800, 150, None, 2, 19, 15),
+    (136, 8190, None, 1, 56.5, 51.2), (160, 8700, 7000, 2, 112.9, 105.0),
+    (80, 5000, 4000, 2, 32.1, 36.0), (8, 5000, None, 1, 15.0, 15.3)])
+def test_waves_of_a_workgroup(groups, max_len, mean, elem, eight, four):
+    """Against the times of both, us, in as many parts as each is to have."""
+    parts, _ = dispatch.decode_parts(groups, max_len, mean, elem)
+    assert dispatch.decode_waves(groups, parts, max_len, mean, elem) == (
+        4 if four < eight else 8)
+
+
 @pytest.mark.parametrize("batch", [2, 5, 17, 24, 25, 32, 64, 127, 256])
 @pytest.mark.parametrize("short", [1, 100, 300, 1000])
 @pytest.mark.parametrize("long", [1500, 3000, 8000, 131072])
