@@ -193,7 +193,9 @@ __global__ __launch_bounds__(NT) void heads_to_rows_kernel(
 // around latent decode attention. A head's weights are small, so what a launch takes is
 // one way of loads: workgroups of 16 rows by 64 channels, whose four waves share K in
 // steps of 128, or the channels where K is short, load everything of a step by 256 bytes
-// of a row at once.
+// of a row at once. 32 heads, 128 -> 512 and 512 -> 128: 1 row 3.3 and 3.6 us, 50 rows 3.7
+// and 3.9 (the library's batched products 11.4 and 6.4), 256 rows 8.9 and 6.9, 512 rows
+// 16.8 and 11.7.
 struct HeadProducts {
   const short *x, *w;        // w [H, N, K]
   short* y;
