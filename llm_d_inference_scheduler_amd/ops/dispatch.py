@@ -144,6 +144,16 @@ def reshape_and_cache(k_new: torch.Tensor, v_new: torch.Tensor,
     ref.reshape_and_cache(k_new, v_new, k_cache, v_cache, slots)
 
 
+def _one_round(groups: int) -> bool:
+    """Whether parts of the decode attention can make up 5/6 of 256 workgroups, one
+    round of 8 waves. By that / by 768 of 4 waves, us, 8 key heads of 4000 tokens, 8-bit
+    and bf16: 9 sequences (84 %) 21.8 / 22.8, 32.4 / 32.8; 14 (88 %) 28.7 / 31.0, 47.2 /
+    48.3; 16 30.3 / 33.4, 50.0 / 52.8; 13 (81 %) 28.2 / 27.1, 45.5 / 42.6; 12 (75 %)
+    27.8 / 26.6, 44.4 / 42.0; 11 (69 %) 27.5 / 25.6, 44.0 / 38.5; 17 (53 %) 41.3 / 33.9,
+    64.2 / 50.8; 21 (66 %) 46.8 / 39.0, 78.8 / 65.7."""
+    return 256 // max(1, groups) * groups * 6 >= 256 * 5
+
+
 def decode_parts(groups: int, max_len: int,
                  mean_len: Optional[float] = None,
                  elem: int = 2) -> Tuple[int, int]:
@@ -151,12 +161,12 @@ def decode_parts(groups: int, max_len: int,
     (sequence, key head) pairs of up to max_len tokens, and of mean_len on
     average (None: 0.8 of that, lengths a quarter either way), of `elem` bytes a
     value. A workgroup of 8 waves takes 256 tokens a step, and a compute unit has
-    registers for one of them or three of 4 waves: parts make up for fewer than 128
-    groups by one round of the former, from there on by a round of the latter, as long
-    as each has a step of its own (as many as make up 512, mostly two rounds and the
-    beginning of a third, / so, us, 8 key heads: 3 of 7000, 8-bit 20.7 / 15.7; 8 of
-    4000 33 / 29, 8-bit 22.6 / 19.9; 10 of 4000 45 / 33.5, 8-bit 30.5 / 22; 17 of 6800,
-    8-bit 56.6 / 50.6; 20 of 7000 121 / 103.6). They cost their sums and a second launch. In us: one part takes 3 and as
+    registers for one of them or three of 4 waves: parts make up for fewer groups, by one
+    round of the former (_one_round) or of the latter, as long as each has a step of its
+    own (as many as make up 512, mostly two rounds and the beginning of a third, / so,
+    us, 8 key heads: 3 of 7000, 8-bit 20.7 / 15.7; 8 of 4000 33 / 29, 8-bit 22.6 / 19.9;
+    10 of 4000 45 / 33.5, 8-bit 30.5 / 22; 17 of 6800, 8-bit 56.6 / 50.6; 20 of 7000
+    121 / 103.6). They cost their sums and a second launch. In us: one part takes 3 and as
     long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
     at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 340 batches, lengths
     alike or down to a twentieth of the longest, the choice costs 0.4 % on average
@@ -179,7 +189,7 @@ def decode_parts(groups: int, max_len: int,
         mean = 0.8 * max_len if mean_len is None else mean_len
         size = groups * mean * 256 * elem
         if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
-            parts = max(2, 256 // max(1, groups)) if groups <= 128 \
+            parts = max(2, 256 // max(1, groups)) if _one_round(groups) \
                 else -(-768 // groups)
     if mean_len is not None and max_len > 1.4 * mean_len:
         # tokens that one workgroup may walk while each compute unit takes one
@@ -205,7 +215,8 @@ def decode_waves(groups: int, parts: int, max_len: int,
     257, 145 / 137; 32 of 300 11.9 / 12.1, 10.1 / 10.2)."""
     if parts > 1:
         alike = mean_len is None or max_len <= 1.4 * mean_len
-        return 4 if max_len <= 256 or (alike and 128 < groups < 200) else 8
+        few = alike and groups < 200 and not _one_round(groups)
+        return 4 if few or max_len <= 256 else 8
     return 4 if max_len <= 256 or (groups > 256 and
                                    (elem == 1 or max_len <= 1024)) else 8
 

@@ -50,7 +50,9 @@ def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
     (800, 374, None, 2, 32.4, 28.2), (2048, 624, None, 1, 70.6, 53.3),
     (2048, 1871, None, 2, 252, 257), (800, 150, None, 2, 19, 15),
     (136, 8190, None, 1, 56.5, 51.2), (160, 8700, 7000, 2, 112.9, 105.0),
-    (80, 5000, 4000, 2, 32.1, 36.0), (8, 5000, None, 1, 15.0, 15.3)])
+    (80, 5000, 4000, 2, 32.1, 36.0), (8, 5000, None, 1, 15.0, 15.3),
+    (72, 5000, None, 2, 32.4, 32.8), (112, 8700, 7000, 1, 41.6, 43.6),
+    (104, 5000, 4000, 2, 45.5, 42.6), (88, 8700, None, 1, 40.3, 36.9)])
 def test_waves_of_a_workgroup(groups, max_len, mean, elem, eight, four):
     """Against the times of both, us, in as many parts as each is to have."""
     parts, _ = dispatch.decode_parts(groups, max_len, mean, elem)
