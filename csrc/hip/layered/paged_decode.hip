@@ -461,8 +461,9 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
     // key heads, groups of 8: 102 us by 8, 95 by 4; of 1000 95 and 95; 20 rows of 7000 in
     // parts: 106 and 103).
     const int64_t groups = (int64_t)n * G;
-    const bool four = parts > 1 ? part_tokens == 0 && groups < 200 &&
-                                      256 / groups * groups * 6 < 256 * 5
+    const bool four = parts > 1 ? part_tokens == 0 &&
+                                      (groups < 200 ? 256 / groups * groups * 6 < 256 * 5
+                                                    : groups > 256 && groups <= 320)
                                 : groups > 256 && max_ctx <= 1024;
     const int waves = max_ctx <= 256 || four ? 4 : 8;
     if (parts > 64) return hipErrorInvalidValue;

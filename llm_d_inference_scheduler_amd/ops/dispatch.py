@@ -154,6 +154,20 @@ def _one_round(groups: int) -> bool:
     return 256 // max(1, groups) * groups * 6 >= 256 * 5
 
 
+def _past_a_round(groups: int, max_len: int, elem: int) -> bool:
+    """Whether the decode attention has up to a quarter more workgroups than compute
+    units, an eighth in 8 bits: some compute units then have two to do, and the others
+    wait. Three parts of 4 waves, which a compute unit takes three of, even that out
+    from where the sequences outweigh the second launch. One part / three, us, bf16:
+    264 of 1000 tokens 36.5 / 34.2, of 4000 125 / 106; 320 of 500 22.9 / 24.9, of 1000
+    37.6 / 36.3, of 4000 131 / 114, of 8000 272 / 235; 384 of 1500 58.0 / 58.3. 8-bit:
+    264 of 700 16.8 / 18.5; 288 of 1500 30.5 / 31.7, of 2000 40.2 / 37.1, of 8000 141 /
+    115; 320 of 4000 66.4 / 67.6."""
+    if elem > 1:
+        return 256 < groups <= 320 and max_len > 1024
+    return 256 < groups <= 288 and max_len > 2048
+
+
 def decode_parts(groups: int, max_len: int,
                  mean_len: Optional[float] = None,
                  elem: int = 2) -> Tuple[int, int]:
@@ -170,11 +184,11 @@ def decode_parts(groups: int, max_len: int,
     long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
     at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 340 batches, lengths
     alike or down to a twentieth of the longest, the choice costs 0.4 % on average
-    and 22 % at most. From 200 groups on it is always one (groups, mean and longest
-    in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 43 in four; 136 of 3223,
-    5262: 71 and 56; 136 of 6800, 8190, 8-bit: 61 and 55; 80 of 466, 1316: 19 and 12;
-    160 of 1500, 1875: 30 and 37; 64 of 2000, 2500: 34 and 21; 8 of 777: 12 and 10, 8
-    of 450: 8.7 and 9.2; 240 of 1100, 1375: 28 and 38).
+    and 22 % at most. From 200 groups on it is one, but for _past_a_round (groups, mean
+    and longest in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 43 in four;
+    136 of 3223, 5262: 71 and 56; 136 of 6800, 8190, 8-bit: 61 and 55; 80 of 466, 1316:
+    19 and 12; 160 of 1500, 1875: 30 and 37; 64 of 2000, 2500: 34 and 21; 8 of 777: 12
+    and 10, 8 of 450: 8.7 and 9.2; 240 of 1100, 1375: 28 and 38).
 
     One long sequence among short ones would hold the batch up: 14 us per 1000
     tokens that a workgroup walks alone. It is cut so that none walks more than
@@ -191,6 +205,9 @@ def decode_parts(groups: int, max_len: int,
         if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
             parts = max(2, 256 // max(1, groups)) if _one_round(groups) \
                 else -(-768 // groups)
+    elif _past_a_round(groups, max_len, elem) and \
+            (mean_len is None or max_len <= 1.4 * mean_len):
+        parts = 3
     if mean_len is not None and max_len > 1.4 * mean_len:
         # tokens that one workgroup may walk while each compute unit takes one
         # and a half shares of the whole
@@ -215,8 +232,9 @@ def decode_waves(groups: int, parts: int, max_len: int,
     257, 145 / 137; 32 of 300 11.9 / 12.1, 10.1 / 10.2)."""
     if parts > 1:
         alike = mean_len is None or max_len <= 1.4 * mean_len
-        few = alike and groups < 200 and not _one_round(groups)
-        return 4 if few or max_len <= 256 else 8
+        many = groups < 200 and not _one_round(groups) or \
+            _past_a_round(groups, max_len, elem)
+        return 4 if alike and many or max_len <= 256 else 8
     return 4 if max_len <= 256 or (groups > 256 and
                                    (elem == 1 or max_len <= 1024)) else 8
 

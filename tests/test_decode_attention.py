@@ -35,7 +35,10 @@ def test_one_part_or_several(groups, max_len, elem, one, several):
     (2, 697, 697, 1, 7.9, 8.4), (4, 3300, 3300, 2, 38.9, 10.5),
     (48, 637, 294, 1, 7.5, 9.1), (176, 1205, 488, 1, 12.6, 16.8),
     (80, 1316, 466, 2, 19.3, 12.2), (112, 4323, 3390, 2, 59.1, 43.5),
-    (136, 5262, 3223, 2, 70.6, 55.7)])
+    (136, 5262, 3223, 2, 70.6, 55.7), (264, 5000, 4000, 2, 125.3, 105.9),
+    (320, 625, 500, 2, 22.9, 24.9), (320, 10800, 8000, 2, 270, 241),
+    (384, 1875, 1500, 2, 58.0, 58.3), (288, 1250, 1000, 1, 20.6, 24.2),
+    (288, 2700, 2000, 1, 40.2, 37.1), (320, 4400, 4000, 1, 66.4, 67.6)])
 def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
     """All lengths alike, or most far below the longest: the bytes follow from the
     mean. Against the times that both took, us."""
@@ -46,7 +49,7 @@ def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
 @pytest.mark.parametrize("groups,max_len,mean,elem,eight,four", [
     (256, 374, None, 2, 11.9, 12.1), (256, 374, None, 1, 10.1, 10.2),
     (272, 748, None, 2, 26.7, 25.9), (320, 748, 600, 1, 18.8, 16.6),
-    (320, 1871, 1500, 2, 57.0, 57.5), (320, 1871, None, 1, 33.0, 31.0),
+    (320, 1871, 1500, 2, 57.0, 52.8), (320, 1871, None, 1, 33.0, 31.0),
     (800, 374, None, 2, 32.4, 28.2), (2048, 624, None, 1, 70.6, 53.3),
     (2048, 1871, None, 2, 252, 257), (800, 150, None, 2, 19, 15),
     (136, 8190, None, 1, 56.5, 51.2), (160, 8700, 7000, 2, 112.9, 105.0),
@@ -144,6 +147,22 @@ def test_lengths_far_apart(batch, fp8):
         for spread in (False, True):
             _close(ext.paged_attention_split(*args, parts, part, D ** -0.5,
                                              spread=spread), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("batch,long,fp8", [(129, 1025, False), (160, 1100, False),
+                                            (144, 2049, True)])
+def test_a_little_more_than_a_round(batch, long, fp8):
+    """In three parts, with the mean length and without, and shorter than said."""
+    lens = [long - 61 * i % (long // 4) for i in range(batch)]
+    args, want = _case(lens, 4, 16, fp8)
+    mean = sum(lens) / batch
+    elem = args[1].element_size()
+    for m in (mean, None):
+        assert dispatch.decode_parts(batch * KVH, long, m, elem)[0] == 3
+        assert dispatch.decode_waves(batch * KVH, 3, long, m, elem) == 4
+        for said in (long, 3 * long):
+            _close(dispatch.paged_attention(*args, D ** -0.5, said, m), want)
 
 
 @pytest.mark.gpu
