@@ -204,7 +204,7 @@ def decode_parts(groups: int, max_len: int,
         size = groups * mean * 256 * elem
         if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
             parts = max(2, 256 // max(1, groups)) if _one_round(groups) \
-                else -(-768 // groups)
+                else -(-768 // max(1, groups))
     elif _past_a_round(groups, max_len, elem) and \
             (mean_len is None or max_len <= 1.4 * mean_len):
         parts = 3

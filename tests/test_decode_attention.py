@@ -17,6 +17,15 @@ def test_parts_cover_the_context(groups, max_len):
     assert (parts - 1) * part < max_len <= parts * part
 
 
+@pytest.mark.parametrize("max_len", [1, 441, 1000, 131072])
+@pytest.mark.parametrize("mean", [None, 0.0, 400.0])
+@pytest.mark.parametrize("elem", [1, 2])
+def test_no_rows(max_len, mean, elem):
+    parts, part = dispatch.decode_parts(0, max_len, mean, elem)
+    assert 1 <= parts <= 64 and part % 32 == 0
+    assert dispatch.decode_waves(0, parts, max_len, mean, elem) in (4, 8)
+
+
 @pytest.mark.parametrize("groups,max_len,elem,one,several", [
     (136, 8190, 1, 63, 51), (136, 8190, 2, 108, 87), (160, 1875, 2, 27, 34),
     (176, 3750, 2, 54, 58), (96, 1000, 2, 13, 16), (64, 2500, 2, 25, 18),
@@ -147,6 +156,15 @@ def test_lengths_far_apart(batch, fp8):
         for spread in (False, True):
             _close(ext.paged_attention_split(*args, parts, part, D ** -0.5,
                                              spread=spread), want)
+
+
+@pytest.mark.gpu
+def test_attention_of_no_rows():
+    (q, *cache, tables, lens), _ = _case([40], 4, 16, False)
+    for longest in (None, 40, 1000):
+        out = dispatch.paged_attention(q[:0], *cache, tables[:0], lens[:0], D ** -0.5,
+                                       longest)
+        assert out.shape == (0, KVH * 4, D)
 
 
 @pytest.mark.gpu

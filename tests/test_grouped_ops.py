@@ -302,6 +302,20 @@ def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
     assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
 
 
+@pytest.mark.parametrize("run", RUNS)
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mean", [None, 100.0])
+def test_decode_of_no_rows(run, D, mean):
+    cache, tables, _ = paged(run, 2, D, D, [40])
+    for rows in (0, 3):                 # of them none of one token
+        out = put(torch.full((rows, 4 * D), 7.0), run)
+        seq = torch.zeros(rows, dtype=torch.int32, device=run[0])
+        ops.grouped_decode(put(rnd(rows, 4 * D, seed=3), run), cache, seq, seq,
+                           tables if rows else tables[:0], 0, 4, D, D ** -0.5, None,
+                           1000, out, mean_ctx=mean)
+        assert (out == 7.0).all()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("G,rep,ctxs", [
     (8, 2, [80 + 11 * i % 90 for i in range(14)] + [1421]),      # 5 parts
