@@ -36,8 +36,8 @@ constexpr int PT = 512;        // of a row in parts
 // 2048 in 14 parts 6.1 and 5.6).
 // ROWS: ALL of them; PICKED: the rows that `rows` names, of n_rows, without a word to
 // the residual; TABLE: rows of the table x that `rows` names (token ids), which become the
-// residual. As in an index, rows below 0 count from the end; others that do not exist are
-// the nearest that does.
+// residual. As in an index, rows below 0 count from the end. Rows that do not exist are
+// NaN throughout: never another row's values.
 enum Rows { ALL, PICKED, TABLE };
 
 template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY, int ROWS>
@@ -51,12 +51,21 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
   if constexpr (ROWS != ALL) {
     row = rows[row];
     row += row < 0 ? n_rows : 0;
-    row = row < 0 ? 0 : row < n_rows ? row : n_rows - 1;
   }
   const int nchunks = H / 8;
   short8* r8 = RESIDUAL ? (short8*)(residual + row * H)
                : ROWS == TABLE ? (short8*)(residual + (int64_t)blockIdx.x * H)
                                : nullptr;
+  if (ROWS != ALL && (row < 0 || row >= n_rows)) {
+    short8 nan;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) nan[j] = 0x7fc0;
+    for (int c = threadIdx.x; c < nchunks; c += BT) {
+      ((short8*)(y + (int64_t)blockIdx.x * H))[c] = nan;
+      if (ROWS == TABLE) r8[c] = nan;
+    }
+    return;
+  }
   auto source = [&](int c, float* f) {
     if constexpr (EARLY) {
       const float4v* const p[1] = {(const float4v*)x + (row * H + c * 8) / 4};

@@ -72,7 +72,8 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
             residual: Optional[torch.Tensor] = None,
             rows: Optional[torch.Tensor] = None) -> torch.Tensor:
     """rows: the norms of these rows alone; what happens to the residual is
-    left open then."""
+    left open then. A row that x does not have raises IndexError on the CPU and
+    comes out as NaN on the GPU."""
     if _use_hip(x):
         if rows is None or (rows.is_cuda and _index(rows) and
                             x.shape[-1] % 8 == 0):
@@ -84,7 +85,8 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
 
 def embed_rmsnorm(ids: torch.Tensor, table: torch.Tensor, w: torch.Tensor,
                   eps: float):
-    """-> table[ids] and its norm."""
+    """-> table[ids] and its norm. An id that the table does not have raises
+    IndexError on the CPU; on the GPU both of its rows come out as NaN."""
     if _use_hip(table) and ids.is_cuda and _index(ids) and \
             table.dtype == torch.bfloat16 and table.shape[1] % 8 == 0:
         return _ext.embed_rmsnorm(ids, table, w, eps)

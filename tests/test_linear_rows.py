@@ -616,6 +616,29 @@ def test_norms_of_some_rows(rows, width, parts):
         assert torch.equal(normed, ops.rmsnorm(x[some], gain, 1e-5))
 
 
+@pytest.mark.parametrize("parts", [0, 3])
+@pytest.mark.parametrize("rows,width", [(1, 8), (7, 2056), (3, 4104), (2, 32776)])
+def test_norms_of_rows_that_do_not_exist(rows, width, parts):
+    """They are no other row's, whatever stands beside the first and the last."""
+    from llm_d_inference_scheduler_amd import ops
+    x = _draw(max(parts, 1), rows, width, seed=rows)
+    x = x.float() if parts else x[0]
+    gain, start = _draw(width, seed=3), _draw(rows, width, seed=4)
+    some = torch.tensor([0, rows, -rows - 1, rows - 1, 1 << 40, -(1 << 40), -rows],
+                        device="cuda")
+    there = torch.tensor([0, 3, 6], device="cuda")
+    gone = torch.tensor([1, 2, 4, 5], device="cuda")
+    for residual in (None, start):
+        got = ops.rmsnorm(x, gain, 1e-5, residual, some)
+        want = ops.rmsnorm(x, gain, 1e-5, residual, some[there])
+        assert torch.equal(got[there], want) and got[gone].isnan().all()
+    assert torch.equal(start, _draw(rows, width, seed=4))
+    if not parts:
+        for got, want in zip(ops.embed_rmsnorm(some, x, gain, 1e-5),
+                             ops.embed_rmsnorm(some[there], x, gain, 1e-5)):
+            assert torch.equal(got[there], want) and got[gone].isnan().all()
+
+
 @pytest.mark.parametrize("width", [1032, 2056, 4104, 8200])
 @pytest.mark.parametrize("few,many,parts", [(256, 257, 9), (512, 513, 2)])
 def test_norms_of_parts_of_many_rows(few, many, parts, width):
