@@ -13,7 +13,7 @@ int lds_grouped_decode_parts(int, int, int, int, int, int, int);
 hipError_t lds_grouped_decode(const void*, int64_t, const void*,
                               const int32_t*, const int32_t*, const int32_t*,
                               void*, float*, float*, int, int, int, int, int,
-                              int, int, int, int, int, float, int, float,
+                              int, int, int, int, int, int, float, int, float,
                               hipStream_t);
 int lds_grouped_prefill_ok(int, int, int, int64_t);
 hipError_t lds_grouped_prefill(const void*, int64_t, const void*,
@@ -111,19 +111,21 @@ void plain_rows(const Heads& s, const Tensor& proj, const Tensor& cache,
 
 // proj [rows, >= H D], queries first; cache [NB, G, bs, D + V]; the first n
 // rows of out [rows, H V]. bf16 in tiles where the sizes allow it, else (or
-// if `plain`) row by row. core_parts, part_tokens: parts of heads that decode_core.h takes.
+// if `plain`) row by row. core_parts, part_tokens, waves: parts and workgroups of heads
+// that decode_core.h takes.
 void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                     Tensor row_seq, Tensor block_tables, int64_t n, int64_t H,
                     int64_t D, double scale, OptFloat sink, int64_t max_ctx,
                     Tensor out, bool plain, int64_t core_parts,
-                    int64_t part_tokens) {
+                    int64_t part_tokens, int64_t waves) {
   const Heads s = heads(proj, cache, H, D);
   same_act(out, s.f32, "out");
   sized(out, {s.rows, H * s.V}, "out");
   check_rows(positions, row_seq, 0, n);
   check(block_tables, at::kInt, "block_tables");
   TORCH_CHECK(n >= 0 && n <= s.rows && part_tokens >= 0 && part_tokens % 32 == 0 &&
-                  part_tokens < (1 << 24), "n, part_tokens");
+                  part_tokens < (1 << 24) && (waves == 4 || waves == 8),
+              "n, part_tokens, waves");
   if (s.f32 || plain ||
       !lds_grouped_decode_ok((int)D, (int)s.V, proj.size(1))) {
     plain_rows(s, proj, cache, positions, row_seq, block_tables, 0, n, scale,
@@ -146,7 +148,7 @@ void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                 parts > 1 ? fp(po) : nullptr, parts > 1 ? fp(ml) : nullptr,
                 (int)n, (int)H, (int)s.G, (int)D, (int)s.V,
                 (int)block_tables.size(1), (int)s.bs, (int)max_ctx, parts,
-                (int)part_tokens, (float)scale,
+                (int)part_tokens, (int)waves, (float)scale,
                 sink.has_value(), (float)sink.value_or(0.), cur_stream()),
             "grouped_decode");
 }

@@ -436,14 +436,15 @@ int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx,
 }
 
 // q: first query of row 0, rows q_stride apart; cache [NB, G, bs, D + V];
-// out [rows, H V]; part_tokens (decode_core.h): 0 or a multiple of 32
+// out [rows, H V]; part_tokens (decode_core.h): 0 or a multiple of 32; waves of its
+// workgroups: 4 or 8, by decode_waves in ops/dispatch.py
 hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
                               const void* cache, const int32_t* positions,
                               const int32_t* row_seq,
                               const int32_t* block_tables, void* out,
                               float* part_o, float* part_ml, int n, int H,
                               int G, int D, int V, int max_blocks, int bs,
-                              int max_ctx, int parts, int part_tokens,
+                              int max_ctx, int parts, int part_tokens, int waves,
                               float scale, int has_sink, float sink,
                               hipStream_t stream) {
   if (!lds_grouped_decode_ok(D, V, q_stride)) return hipErrorInvalidValue;
@@ -456,17 +457,7 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
         positions, row_seq, 1, max_blocks, bs, (short*)out, part_o, part_ml, G,
         H / G, part_tokens, part_tokens > 0 && n % 2 == 0, scale, sink * LOG2E,
         has_sink};
-    // Short rows leave half of 8 waves without a tile; where a compute unit has several
-    // workgroups to do, three of 4 waves fit it and one of 8 (256 rows of 500 tokens, 8
-    // key heads, groups of 8: 102 us by 8, 95 by 4; of 1000 95 and 95; 20 rows of 7000 in
-    // parts: 106 and 103).
-    const int64_t groups = (int64_t)n * G;
-    const bool four = parts > 1 ? part_tokens == 0 &&
-                                      (groups < 200 ? 256 / groups * groups * 6 < 256 * 5
-                                                    : groups > 256 && groups <= 320)
-                                : groups > 256 && max_ctx <= 1024;
-    const int waves = max_ctx <= 256 || four ? 4 : 8;
-    if (parts > 64) return hipErrorInvalidValue;
+    if (parts > 64 || (waves != 4 && waves != 8)) return hipErrorInvalidValue;
     return parts > 1 ? decode::attend<true, 256>(w, n, parts, waves, stream)
                      : decode::attend<false, 256>(w, n, 1, waves, stream);
   }

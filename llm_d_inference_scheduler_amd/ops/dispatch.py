@@ -223,22 +223,37 @@ def decode_parts(groups: int, max_len: int,
 
 
 def decode_waves(groups: int, parts: int, max_len: int,
-                 mean_len: Optional[float] = None, elem: int = 2) -> int:
-    """Waves of a workgroup of the decode attention, 4 or 8. Short sequences leave
-    half of 8 without a tile (100 sequences of 120 tokens: 19 us with 8 waves, 15 with
-    4). Where a compute unit has several workgroups to do, three of 4 waves have more
-    under way than one of 8, which counts with few bytes a tile, and their ends overlap:
-    in parts as many as make that up (decode_parts), in one part from 257 groups on, in
-    8 bits or up to 1024 tokens (8 / 4 waves, us: 40 of 600, 28 / 27, 8-bit 18.8 / 16.6;
-    100 of 300 32.4 / 28.2, 24.2 / 18.6; 256 of 500 96 / 91, 71 / 53; 256 of 1500 252 /
-    257, 145 / 137; 32 of 300 11.9 / 12.1, 10.1 / 10.2)."""
+                 mean_len: Optional[float] = None, elem: int = 2,
+                 apart: float = 2.) -> int:
+    """Waves of a workgroup of the decode attention, 4 or 8; apart: how many times the
+    mean the longest sequence may have where parts are shares of each sequence
+    (else all have one length). Short sequences leave half of 8 without a tile (100
+    sequences of 120 tokens: 19 us with 8 waves, 15 with 4). Where a compute unit has
+    several workgroups to do, three of 4 waves have more under way than one of 8, which
+    counts with few bytes a tile, and their ends overlap.
+
+    In parts: as many as make that up (decode_parts), 0.88 of the time in geometric
+    mean up to 1.4 times the mean (22 batches) and 0.92 up to 2 (23); past that 1.02.
+
+    In one part: from 257 groups on, in 8 bits up to a mean of 1600 or up to 1024 tokens
+    (8 / 4 waves, us: 40 of 600, 28 / 27, 8-bit 18.8 / 16.6; 100 of 300 32.4 / 28.2, 24.2
+    / 18.6; 256 of 500 96 / 91, 71 / 53; 256 of 1500 252 / 257, 145 / 137; 32 of 300
+    11.9 / 12.1, 10.1 / 10.2; 149 of 1640, 8-bit 98 / 104). But 4 waves walk the longest
+    sequence twice as long as 8, and it is to end with the rest: with a compute unit's
+    share of the tokens, and 400 (a launch and the first loads) beside it. 8-bit: 33
+    sequences of 470 and one of 2494 20.5 / 29.5; 36 of 100 to 2100 25.0 / 29.6; 76 of
+    up to 8190, 2800 on average 106 / 151; 106 of up to 3130, 770 on average 49 / 45. Over
+    156 batches the choice costs 0.9 % on average and 14 % at most."""
+    mean = 0.8 * max_len if mean_len is None else mean_len
+    if max_len <= 256:
+        return 4
     if parts > 1:
-        alike = mean_len is None or max_len <= 1.4 * mean_len
         many = groups < 200 and not _one_round(groups) or \
             _past_a_round(groups, max_len, elem)
-        return 4 if alike and many or max_len <= 256 else 8
-    return 4 if max_len <= 256 or (groups > 256 and
-                                   (elem == 1 or max_len <= 1024)) else 8
+        return 4 if many and (mean_len is None or max_len <= apart * mean) else 8
+    few = mean <= 1600 if elem == 1 else max_len <= 1024
+    return 4 if groups > 256 and few and \
+        max_len <= 400 + 1.1 * groups * mean / 256 else 8
 
 
 def paged_attention(q: torch.Tensor, k_cache: torch.Tensor,

@@ -3,7 +3,7 @@
 import torch
 
 from . import ref_layered as ref
-from .dispatch import decode_parts
+from .dispatch import decode_parts, decode_waves
 
 try:
     from .. import _hip_layered as _ext
@@ -221,13 +221,16 @@ def grouped_decode(proj, cache, positions, row_seq, block_tables, n, heads,
     paged keys and values; sink: score of a key without a value, or None.
     max_ctx: tokens of the longest row; mean_ctx: of the mean one, if known."""
     max_ctx = max(1, max_ctx)
-    parts, part = decode_parts(n * cache.shape[1], max_ctx, mean_ctx)
+    groups = n * cache.shape[1]
+    parts, part = decode_parts(groups, max_ctx, mean_ctx)
     # A row is shared out over all parts; rows far apart have parts of one length (one
     # of 8260 tokens among 7 of 500, 8 key heads: 18 us, 40 shared out).
-    far_apart = mean_ctx is not None and max_ctx > 2.5 * mean_ctx
+    apart = 2.5
+    waves = decode_waves(groups, parts, max_ctx, mean_ctx, apart=apart)
+    far_apart = mean_ctx is not None and max_ctx > apart * mean_ctx
     _impl(proj).grouped_decode(proj, cache, positions, row_seq, block_tables,
                                n, heads, dim, scale, sink, max_ctx, out,
-                               plain, parts, part if far_apart else 0)
+                               plain, parts, part if far_apart else 0, waves)
 
 
 def grouped_prefill(proj, cache, positions, row_seq, block_tables, base,

@@ -209,7 +209,7 @@ def _grouped(proj, cache, positions, row_seq, block_tables, lo, hi, heads,
 
 def grouped_decode(proj, cache, positions, row_seq, block_tables, n, heads,
                    dim, scale, sink, max_ctx, out, plain, parts,
-                   part_tokens):
+                   part_tokens, waves):
     _grouped(proj, cache, positions, row_seq, block_tables, 0, n, heads, dim,
              scale, sink, out)
 

@@ -72,6 +72,19 @@ def test_waves_of_a_workgroup(groups, max_len, mean, elem, eight, four):
         4 if four < eight else 8)
 
 
+@pytest.mark.parametrize("groups,max_len,mean,elem,eight,four", [
+    (288, 2107, 1062, 1, 25.0, 29.6), (608, 8190, 2809, 1, 106, 151),
+    (352, 1909, 646, 1, 23.5, 26.4), (424, 1614, 288, 1, 18.7, 22.0),
+    (1192, 2412, 1637, 1, 98, 104), (848, 3128, 768, 1, 49.2, 44.8),
+    (2072, 2641, 1312, 1, 146, 140), (280, 1348, 296, 2, 20.6, 22.2),
+    (408, 672, 378, 2, 21.5, 20.4), (96, 4378, 2855, 2, 36.8, 33.2)])
+def test_waves_by_the_mean(groups, max_len, mean, elem, eight, four):
+    """Lengths from half as much again as the mean to far apart, as above."""
+    parts, _ = dispatch.decode_parts(groups, max_len, mean, elem)
+    assert dispatch.decode_waves(groups, parts, max_len, mean, elem) == (
+        4 if four < eight else 8)
+
+
 @pytest.mark.parametrize("batch", [2, 5, 17, 24, 25, 32, 64, 127, 256])
 @pytest.mark.parametrize("short", [1, 100, 300, 1000])
 @pytest.mark.parametrize("long", [1500, 3000, 8000, 131072])

@@ -6,7 +6,7 @@ import torch
 
 import sezazen_oracle as oracle
 from llm_d_inference_scheduler_amd.ops import layered as ops
-from llm_d_inference_scheduler_amd.ops.dispatch import decode_parts
+from llm_d_inference_scheduler_amd.ops.dispatch import decode_parts, decode_waves
 from test_layered_ops import F64, GPU, RUNS, close, f64, meta, put, rnd
 
 F32 = ("", torch.float32)
@@ -300,6 +300,24 @@ def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
                         for i, c in enumerate(ctxs)])
     # probabilities have 24 bits: 32-bit scores and sums, and the result's rounding
     assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
+
+
+@pytest.mark.parametrize("n,longest,mean", [
+    (12, 5000, None), (12, 5000, 3400.0), (12, 5000, 2100.0), (12, 5000, 1900.0),
+    (33, 900, None), (33, 900, 300.0), (33, 3000, 2500.0), (16, 3000, 2800.0)])
+def test_waves_of_decode(monkeypatch, n, longest, mean):
+    """The kernel is told what the rule says; shares of every row up to 2.5 times the
+    mean."""
+    told = []
+    monkeypatch.setattr(ops.ref, "grouped_decode",
+                        lambda *a: told.append(a[-3:]))
+    cache = torch.zeros(1, 8, 16, 256)
+    ops.grouped_decode(torch.zeros(n, 32 * 128), cache, None, None, None, n, 32, 128,
+                       1.0, None, longest, None, mean_ctx=mean)
+    parts, tokens = decode_parts(n * 8, longest, mean)
+    far = mean is not None and longest > 2.5 * mean
+    assert told == [(parts, tokens if far else 0, decode_waves(
+        n * 8, parts, longest, mean, apart=2.5))]
 
 
 @pytest.mark.parametrize("run", RUNS)
