@@ -178,19 +178,22 @@ def decode_parts(groups: int, max_len: int,
     average (None: 0.8 of that, lengths a quarter either way), of `elem` bytes a
     value. A workgroup of 8 waves takes 256 tokens a step, and a compute unit has
     registers for one of them or three of 4 waves: parts make up for fewer groups, by one
-    round of the former (_one_round) or of the latter, as long as each has a step of its
-    own (as many as make up 512, mostly two rounds and the beginning of a third, / so,
-    us, 8 key heads: 3 of 7000, 8-bit 20.7 / 15.7; 8 of 4000 33 / 29, 8-bit 22.6 / 19.9;
-    10 of 4000 45 / 33.5, 8-bit 30.5 / 22; 17 of 6800, 8-bit 56.6 / 50.6; 20 of 7000
-    121 / 103.6). They cost their sums and a second launch. In us: one part takes 3 and as
-    long as a workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take
-    at 4.9 TB/s, several 8.5 and the bytes at 5.2 TB/s; over 340 batches, lengths
-    alike or down to a twentieth of the longest, the choice costs 0.4 % on average
-    and 22 % at most. From 200 groups on it is one, but for _past_a_round (groups, mean
-    and longest in tokens: 160 of 4076, all alike, 8-bit: 35 in one part, 43 in four;
-    136 of 3223, 5262: 71 and 56; 136 of 6800, 8190, 8-bit: 61 and 55; 80 of 466, 1316:
-    19 and 12; 160 of 1500, 1875: 30 and 37; 64 of 2000, 2500: 34 and 21; 8 of 777: 12
-    and 10, 8 of 450: 8.7 and 9.2; 240 of 1100, 1375: 28 and 38).
+    round of the former (_one_round), or by at least one of the latter, as long as each
+    has a step of its own. That is 768 workgroups, rounded up: the few of a second round
+    cost less than the units that one part less leaves with two (us, up / down: 104
+    groups of 2500 27.5 / 30.6, of 4000 39.2 / 42.6; 168 of 7000 109 / 119; 8-bit 58 /
+    64; at the worst 176 of 7000 127 / 123).
+
+    Parts cost their sums and a second launch. In us: one part takes 3 and as long as a
+    workgroup walks (12.5 per 1000 tokens, 6.8 in 8 bits) or the bytes take at 5.2 TB/s,
+    several 9 and the bytes at 5.8 TB/s. Over 264 batches of 1 to 24 sequences of like
+    lengths, 8 key heads, the choice costs 0.2 % on average and 9 % at most; over 140,
+    lengths alike to far apart, 0.4 and 24 %. One part / several, us, by groups and mean:
+    8 of 400 6.7 / 8.3, of 800 11.2 / 9.1; 96 of 400 9.9 / 11.2, of 1500 24.9 / 21.6; 128
+    of 1500 25.9 / 23.3; 136 of 2500 41.9 / 37.6; 152 of 1500 27.1 / 27.2, of 4000 72 /
+    55; 168 of 1500 28.2 / 29.1, of 4000 76 / 67; 8-bit 136 of 2500 24.3 / 24.4, of 4000
+    35.9 / 32.9; 168 of 4000 37.8 / 38.2, of 7000 66 / 58. From 200 groups on it is one
+    (192 of 4000 80 / 80), but for _past_a_round.
 
     One long sequence among short ones would hold the batch up: 14 us per 1000
     tokens that a workgroup walks alone. It is cut so that none walks more than
@@ -204,7 +207,7 @@ def decode_parts(groups: int, max_len: int,
         walk = max_len * (12.5e-3 if elem > 1 else 6.8e-3)
         mean = 0.8 * max_len if mean_len is None else mean_len
         size = groups * mean * 256 * elem
-        if 3 + max(walk, size / 4.9e6) > 8.5 + size / 5.2e6:
+        if 3 + max(walk, size / 5.2e6) > 9 + size / 5.8e6:
             parts = max(2, 256 // max(1, groups)) if _one_round(groups) \
                 else -(-768 // max(1, groups))
     elif _past_a_round(groups, max_len, elem) and \

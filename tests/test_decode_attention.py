@@ -55,6 +55,17 @@ def test_parts_by_the_mean(groups, max_len, mean, elem, one, several):
     assert (parts > 1) == (several < one)
 
 
+@pytest.mark.parametrize("groups,max_len,elem,one,several", [
+    (152, 4993, 2, 72.2, 55.2), (168, 4995, 2, 75.8, 67.2), (136, 3075, 2, 41.9, 37.6),
+    (128, 1842, 2, 25.9, 23.3), (128, 3070, 1, 23.9, 20.9), (168, 8741, 1, 66.3, 57.6),
+    (160, 8728, 1, 67.7, 62.4), (152, 4993, 1, 37.0, 34.0), (192, 4996, 1, 40.1, 43.2),
+    (168, 1873, 2, 28.2, 29.1), (160, 1870, 2, 28.5, 30.1), (136, 1845, 1, 16.3, 18.3)])
+def test_one_part_or_several_rounds(groups, max_len, elem, one, several):
+    """Lengths a quarter either way. Against the times that both took, us."""
+    parts, _ = dispatch.decode_parts(groups, max_len, None, elem)
+    assert (parts > 1) == (several < one)
+
+
 @pytest.mark.parametrize("groups,max_len,mean,elem,eight,four", [
     (256, 374, None, 2, 11.9, 12.1), (256, 374, None, 1, 10.1, 10.2),
     (272, 748, None, 2, 26.7, 25.9), (320, 748, 600, 1, 18.8, 16.6),
