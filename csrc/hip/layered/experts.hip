@@ -299,6 +299,15 @@ __global__ __launch_bounds__(256) void expert_plain_kernel(const Pairs p) {
 //   128        225   328   334   350
 // and 64 experts of 2048 x 1408, 6 each, 250 rows 191, 149, 151. So tiles of 64 pairs
 // take 128.
+//
+// Weights that one tile reads go past the L2 caches (rows_core.h), not those that the
+// next tile in the list reads too, which finds them there. Both products as above, by how
+// uneven the loads are (standard deviation of the choice's logits), all weights by way of
+// the caches / all past them / so:
+//   rows         60                100               180               380
+//   0     325 / 292 / 290   328 / 293 / 298   353 / 328 / 327   352 / 342 / 345
+//   0.5   328 / 302 / 295   337 / 308 / 306   372 / 371 / 353   400 / 422 / 402
+//   1.5   302 / 294 / 285   319 / 317 / 305   395 / 418 / 387   437 / 472 / 423
 template <int RT, int BN, bool UP>
 __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs p) {
   extern __shared__ __align__(16) char ring[];
@@ -308,7 +317,10 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   const int N = p.N, K = p.K, blocks = gridDim.x;
   const int i = rows_core::along_xcd(blockIdx.y * blocks + blockIdx.x,
                                      p.tiles[0].x * blocks, BN == 64 ? 512 : 256);
-  const int4 tile = p.tiles[1 + i / blocks];
+  const int at = i / blocks, tiles = p.tiles[0].x;
+  const int4 tile = p.tiles[1 + at];
+  const bool several = (at > 0 && p.tiles[at].x == tile.x) ||
+                       (at + 1 < tiles && p.tiles[2 + at].x == tile.x);
   const int n0 = i % blocks * p.width, n1 = min(N, n0 + p.width);
   if (n0 >= N) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
@@ -335,8 +347,14 @@ __global__ __launch_bounds__(BN / 16 * WAVE) void expert_rows_kernel(const Pairs
   const int steps = (K + rows_core::KS - 1) / rows_core::KS;
   // by the expert, not its tile's rank: a row's sums do not hang on what others chose
   const uint32_t first = uint32_t(tile.x * blocks + i % blocks) * BN / 128 * 3;
-  Core::run(ring, wave, lane, w_from, x_from, 0, K, steps, first % uint32_t(steps),
-            wave * 16 < p.width, acc);
+  auto run = [&](auto core) {
+    decltype(core)::run(ring, wave, lane, w_from, x_from, 0, K, steps,
+                        first % uint32_t(steps), wave * 16 < p.width, acc);
+  };
+  if (several)
+    run(rows_core::RowsCore<RT, BN, 0>{});
+  else
+    run(Core{});
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const int m = (wave / Core::WC * MT + t) * 16 + col;

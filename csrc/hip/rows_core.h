@@ -12,8 +12,6 @@
 #pragma once
 #include "layered/elem.h"
 
-#include <type_traits>
-
 namespace rows_core {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -21,11 +19,14 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 constexpr int KS = 128, ROW = KS * 2;          // ROW: bytes of a row in LDS
 constexpr int RING = 3;          // 4 are no faster, 2 up to 15 % slower
 
-// Cache policy (nt) of loads of weights. They are read once, and as other loads they push
+// Cache policy (nt) of loads of weights that one workgroup reads. As other loads they push
 // x and each other's lines on their way out of the L2 caches: 1 row, 4096 -> [2 x 14336]
 // 41.8 us, so 38.3 (6.1 TB/s); 25600 -> 5120 47.4, 42.1; 30 rows 42.3 and 39.3, 49.3 and
-// 44.2. (sc0, or sc0 and sc1, gain a third of that. Weights that fit the 256 MB cache
-// from one pass to the next would lose by it; those of a model do not.)
+// 44.2. (sc0, or sc0 and sc1, gain a third of that.) Weights that stay in the 256 MB
+// cache from one pass to the next lose by it, which only those of a model of less than
+// 100 million parameters do, and a matrix does not tell: 4096 -> 4096, 1 and 64 rows, of
+// 64 MB in turn 4.7 and 7.9 us, so 5.1 and 8.6; of 700 MB 8.4 and 11.2, 7.7 and 10.0.
+// Those that several workgroups read at a time are to be loaded without (experts.hip).
 constexpr int ONCE = 2;
 
 // what is past the end of K
@@ -41,8 +42,8 @@ __device__ __forceinline__ int along_xcd(int i, int n, int round) {
 }
 
 // RT: rows of x / 16. BN rows of w for BN / 16 waves. A wave has CT tiles of 16 channels
-// by MT of 16 rows.
-template <int RT, int BN>
+// by MT of 16 rows. HINT: cache policy of the loads of w.
+template <int RT, int BN, int HINT = ONCE>
 struct RowsCore {
   static constexpr int NW = BN / 16, WM = RT == 1 ? 1 : 2, WC = NW / WM;
   static constexpr int CT = BN / 16 / WC, MT = RT / WM;
@@ -64,6 +65,17 @@ struct RowsCore {
     return (lane % 16 ^ row % 16) * 8;
   }
 
+  // 4 rows of K from k on, rows 4 q .. of their kind
+  template <int POLICY>
+  static __device__ __forceinline__ void load(const short* from, char* to, int q,
+                                              int lane, int k, int k_hi) {
+    typedef const __attribute__((address_space(1))) unsigned int gmem;
+    typedef __attribute__((address_space(3))) unsigned int smem;
+    const bool in = k + piece(q * 4 + lane / 16, lane) < k_hi;
+    __builtin_amdgcn_global_load_lds((gmem*)(in ? from + k : (const short*)&zeros),
+                                     (smem*)(to + q * 1024), 16, 0, POLICY);
+  }
+
   // K from k_lo to k_hi in `steps` of KS, from step `first` on and round; past k_hi it
   // counts as zero. w_from, x_from: the lane's piece at K = 0 of its row, w_row + lane /
   // 16 and x_row + lane / 16, of each load; rows that do not exist repeat others. A wave
@@ -75,30 +87,19 @@ struct RowsCore {
     char* const w_ring = lds;
     char* const x_ring = lds + RING * W_STEP;
     const int col = lane % 16, grp = lane / 16;
-    typedef const __attribute__((address_space(1))) unsigned int gmem;
-    typedef __attribute__((address_space(3))) unsigned int smem;
     auto k_of = [&](int s) {
       s += first;
       return k_lo + (s >= steps ? s - steps : s) * KS;
-    };
-    // 4 rows of K from k on, rows 4 q .. of their kind
-    auto load = [&](auto hint, const short* from, char* to, int q, int k) {
-      const bool in = k + piece(q * 4 + grp, lane) < k_hi;
-      __builtin_amdgcn_global_load_lds(
-          (gmem*)(in ? from + k : (const short*)&zeros), (smem*)(to + q * 1024),
-          16, 0, decltype(hint)::value);
     };
     auto issue = [&](int s, int buf) {
       const int k = k_of(s);
       if (some)
 #pragma unroll
         for (int j = 0; j < WL; ++j)
-          load(std::integral_constant<int, ONCE>{}, w_from[j], w_ring + buf * W_STEP,
-               wave * WL + j, k);
+          load<HINT>(w_from[j], w_ring + buf * W_STEP, wave * WL + j, lane, k, k_hi);
 #pragma unroll
       for (int j = 0; j < XL; ++j)
-        load(std::integral_constant<int, 0>{}, x_from[j], x_ring + buf * X_STEP,
-             x_row(wave, j) / 4, k);
+        load<0>(x_from[j], x_ring + buf * X_STEP, x_row(wave, j) / 4, lane, k, k_hi);
     };
 
 #pragma unroll
