@@ -22,9 +22,20 @@
 // a SIMD, so the 12 to 15 columns that a group of 1 to 4 heads leaves idle cost
 // nothing.
 //
-// Values are read by whole rows and past the caches (256 sequences of 1500 tokens, the
-// pass 1818 us with both by way of them, so 1739, with both past them 1795: a load of keys
-// takes 64 bytes of 16 rows, whose other halves have to be found again).
+// Values are read by whole rows and, where no other row reads them too, past the caches:
+// as other loads they push keys out of them, a load of which takes 64 bytes of 16 rows,
+// whose other halves have to be found again. Where sequences share blocks it is what one
+// of them leaves in the caches that the others find. By way of them / past them / as the
+// rows' tables say (shared), us, 8 key heads:
+//   256 of 1500 tokens, none shared     271 / 251 / 252.5    8-bit 150 / 138 / 142
+//   17 of 6800, none shared             95 / 87.5 / 87.8    56 / 52 / 52
+//   30 of 1100, none shared             29.1 / 27.5 / 27.7    17.1 / 16.2 / 16.7
+//   256 of 1500, 1000 of one prefix     166 / 182 / 169    95 / 104 / 97
+//   256 of 1500, 1000 of 8 prefixes     170 / 196 / 173    96 / 112 / 99
+//   256 of 1500, 500 of 8 prefixes      217 / 218 / 221    123 / 127 / 129
+//   64 of 4100, 4000 of one prefix      82 / 101 / 82    54 / 59 / 56
+// Chosen tile by tile the branch around the loads costs more than it gives (fp8, 64 of
+// 4100, 4000 shared: 73).
 //
 // Measured alone, cold (8 key heads, ragged; before: P V on the 32-bit cores): 256
 // sequences of 1500 tokens, groups of 4: 269 us, 5.8 TB/s (279), fp8 156 us, 5.0 TB/s
@@ -177,6 +188,8 @@ struct Work {
   int kvh, qpg;
   int part_tokens;            // 0: each row's own share, in steps of 32
   int spread;
+  int probe;                  // page by whose readers values are read: below max_blocks,
+                              // or -1
   float scale, sink;          // sink: score (log2) of a key without a value
   int has_sink;
 };
@@ -198,6 +211,23 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   const int part = SPLIT ? blockIdx.z : 0;
   const int np = SPLIT ? gridDim.z : 1;
   const int64_t group = (int64_t)b * kvh + kh;
+  const int tid = threadIdx.x;
+  // Whether another row reads the page `probe` too: one of the 64 behind this one, a lane
+  // each, is found wherever more than a few share a prefix. Asked for ahead of all else,
+  // so that the answer comes little later than the first pages (a page that hangs on the
+  // row's length 0.2 us later).
+  const int32_t* bt =
+      w_.tables + (int64_t)(w_.seq ? w_.seq[b] : b) * w_.max_blocks;
+  bool shared = false;
+  {
+    const int rows = gridDim.x, others = w_.probe < 0 ? 0 : min(rows - 1, WAVE);
+    int r = b + 1 + tid % WAVE;
+    r -= r >= rows ? rows : 0;
+    if (tid % WAVE < others) {
+      const int64_t table = w_.seq ? w_.seq[r] : r;
+      shared = w_.tables[table * w_.max_blocks + w_.probe] == bt[w_.probe];
+    }
+  }
   const int seq_len = w_.lens[b] + w_.more;
   const int share = w_.part_tokens ? w_.part_tokens
                                    : ((seq_len + np - 1) / np + 31) / 32 * 32;
@@ -207,7 +237,6 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   float* const part_o = w_.part_o;
   float* const part_ml = w_.part_ml;
 
-  const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int lane = tid % WAVE;
   const int col = lane % 16, g = lane / 16;
@@ -245,8 +274,6 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   };
   begin();
 
-  const int32_t* bt =
-      w_.tables + (int64_t)(w_.seq ? w_.seq[b] : b) * w_.max_blocks;
   const CT* const k_head = w_.k + kh * w_.head;
   const CT* const v_head = w_.v + kh * w_.head;
   uint4v kr[2][C::KL];
@@ -278,7 +305,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
         kr[h][i] = *(const uint4v*)((const char*)row + i * 64 + g * 16);
     }
   };
-  auto fetch_v = [&](int t0) {
+  auto fetch_v = [&](auto past, int t0) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -288,21 +315,24 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
           row = v_head + page[h] * w_.page + (g * 4 + j) * RS;
         else
           row = v_head + row_of(t0 + h * 16 + g * 4 + j);
-        // past the caches, by whole rows
-        vr[h][j] =
-            __builtin_nontemporal_load((const typename C::VReg*)(row + col * 8));
+        const auto* const v = (const typename C::VReg*)(row + col * 8);
+        if constexpr (decltype(past)::value)
+          vr[h][j] = __builtin_nontemporal_load(v);
+        else
+          vr[h][j] = *v;
       }
   };
 
   // ENDLESS: infinite values are no part of the lower products; no tile is read
-  // ahead, which would take more registers than there are
-  auto walk = [&](auto endless) {
+  // ahead, which would take more registers than there are. PAST: values are read past the
+  // caches.
+  const int t_first = t_begin + wave * TILE;
+  auto walk = [&](auto endless, auto past) {       // !ENDLESS: with the first tile's pages
     constexpr bool ENDLESS = decltype(endless)::value;
-    int t0 = t_begin + wave * TILE;
+    int t0 = t_first;
     if (!ENDLESS && t0 < t_end) {
-      find(t0);
       fetch_k(t0);
-      fetch_v(t0);
+      fetch_v(past, t0);
     }
     for (; t0 < t_end; t0 += NW * TILE) {
       const int next = t0 + NW * TILE;
@@ -310,7 +340,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
       if (ENDLESS) {
         find(t0);
         fetch_k(t0);
-        fetch_v(t0);
+        fetch_v(past, t0);
       }
       if (more) find(next);
       float4v sc[2];
@@ -379,10 +409,14 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
                                    ENDLESS && p > 0 ? finite(v[c]) : v[c]),
                 acc[d * C::CH + c], 0, 0, 0);
       }
-      if (more) fetch_v(next);
+      if (more) fetch_v(past, next);
     }
   };
-  walk(std::false_type{});
+  if (t_first < t_end) find(t_first);
+  if (w_.probe * bs < seq_len && __any(shared))
+    walk(std::false_type{}, std::false_type{});
+  else
+    walk(std::false_type{}, std::true_type{});
   if constexpr (sizeof(CT) == 2) {
     // A probability's lower parts, 0 or negative as often as not, make no number
     // of an infinite value, where the whole one makes infinity: sums that are no
@@ -396,7 +430,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
       begin();
 #pragma unroll
       for (int i = 0; i < 8; ++i) acc[i] = (float4v){0.f, 0.f, 0.f, 0.f};
-      walk(std::true_type{});
+      walk(std::true_type{}, std::false_type{});
     }
   }
   l += __shfl_xor(l, 16, WAVE);

@@ -13,8 +13,8 @@ int lds_grouped_decode_parts(int, int, int, int, int, int, int);
 hipError_t lds_grouped_decode(const void*, int64_t, const void*,
                               const int32_t*, const int32_t*, const int32_t*,
                               void*, float*, float*, int, int, int, int, int,
-                              int, int, int, int, int, int, float, int, float,
-                              hipStream_t);
+                              int, int, int, int, int, int, int, float, int,
+                              float, hipStream_t);
 int lds_grouped_prefill_ok(int, int, int, int64_t);
 hipError_t lds_grouped_prefill(const void*, int64_t, const void*,
                                const int32_t*, int, int, const int32_t*,
@@ -111,12 +111,12 @@ void plain_rows(const Heads& s, const Tensor& proj, const Tensor& cache,
 
 // proj [rows, >= H D], queries first; cache [NB, G, bs, D + V]; the first n
 // rows of out [rows, H V]. bf16 in tiles where the sizes allow it, else (or
-// if `plain`) row by row. core_parts, part_tokens, waves: parts and workgroups of heads
-// that decode_core.h takes.
+// if `plain`) row by row. probe, core_parts, part_tokens, waves: the page that is
+// compared, parts and workgroups of heads that decode_core.h takes.
 void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                     Tensor row_seq, Tensor block_tables, int64_t n, int64_t H,
                     int64_t D, double scale, OptFloat sink, int64_t max_ctx,
-                    Tensor out, bool plain, int64_t core_parts,
+                    Tensor out, bool plain, int64_t probe, int64_t core_parts,
                     int64_t part_tokens, int64_t waves) {
   const Heads s = heads(proj, cache, H, D);
   same_act(out, s.f32, "out");
@@ -148,7 +148,7 @@ void grouped_decode(Tensor proj, Tensor cache, Tensor positions,
                 parts > 1 ? fp(po) : nullptr, parts > 1 ? fp(ml) : nullptr,
                 (int)n, (int)H, (int)s.G, (int)D, (int)s.V,
                 (int)block_tables.size(1), (int)s.bs, (int)max_ctx, parts,
-                (int)part_tokens, (int)waves, (float)scale,
+                (int)part_tokens, (int)waves, (int)probe, (float)scale,
                 sink.has_value(), (float)sink.value_or(0.), cur_stream()),
             "grouped_decode");
 }

@@ -437,7 +437,7 @@ int lds_grouped_decode_parts(int n, int H, int G, int D, int V, int max_ctx,
 
 // q: first query of row 0, rows q_stride apart; cache [NB, G, bs, D + V];
 // out [rows, H V]; part_tokens (decode_core.h): 0 or a multiple of 32; waves of its
-// workgroups: 4 or 8, by decode_waves in ops/dispatch.py
+// workgroups: 4 or 8, by decode_waves in ops/dispatch.py; probe: a page or -1
 hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
                               const void* cache, const int32_t* positions,
                               const int32_t* row_seq,
@@ -445,7 +445,7 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
                               float* part_o, float* part_ml, int n, int H,
                               int G, int D, int V, int max_blocks, int bs,
                               int max_ctx, int parts, int part_tokens, int waves,
-                              float scale, int has_sink, float sink,
+                              int probe, float scale, int has_sink, float sink,
                               hipStream_t stream) {
   if (!lds_grouped_decode_ok(D, V, q_stride)) return hipErrorInvalidValue;
   if (n == 0) return hipSuccess;
@@ -455,8 +455,8 @@ hipError_t lds_grouped_decode(const void* q, int64_t q_stride,
     const decode::Work<short> w{
         (const short*)q, q_stride, keys, keys + D, G * head, head, block_tables,
         positions, row_seq, 1, max_blocks, bs, (short*)out, part_o, part_ml, G,
-        H / G, part_tokens, part_tokens > 0 && n % 2 == 0, scale, sink * LOG2E,
-        has_sink};
+        H / G, part_tokens, part_tokens > 0 && n % 2 == 0,
+        probe < max_blocks ? probe : max_blocks - 1, scale, sink * LOG2E, has_sink};
     if (parts > 64 || (waves != 4 && waves != 8)) return hipErrorInvalidValue;
     return parts > 1 ? decode::attend<true, 256>(w, n, parts, waves, stream)
                      : decode::attend<false, 256>(w, n, 1, waves, stream);

@@ -47,12 +47,12 @@ hipError_t lds_gather_blocks(const void*, void*, const int32_t*, int, int,
                              int64_t, int64_t, int, hipStream_t);
 hipError_t lds_paged_attention(const void*, const void*, const void*,
                                const int32_t*, const int32_t*, void*, int, int,
-                               int, int, int, int, int, int, float,
+                               int, int, int, int, int, int, int, float,
                                hipStream_t);
 hipError_t lds_paged_attention_split(const void*, const void*, const void*,
                                      const int32_t*, const int32_t*, void*,
                                      float*, float*, int, int, int, int, int,
-                                     int, int, int, int, int, int, float,
+                                     int, int, int, int, int, int, int, float,
                                      hipStream_t);
 hipError_t lds_flash_prefill(const void*, const void*, const void*,
                              const int32_t*, const int32_t*, const int32_t*,
@@ -410,7 +410,7 @@ torch::Tensor paged_attention(torch::Tensor q, torch::Tensor k_cache,
                               torch::Tensor v_cache,
                               torch::Tensor block_tables,
                               torch::Tensor seq_lens, double scale,
-                              int64_t waves) {
+                              int64_t waves, int64_t probe) {
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -420,7 +420,7 @@ torch::Tensor paged_attention(torch::Tensor q, torch::Tensor k_cache,
       q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
       out.data_ptr(), B, qh, kvh, bs, d, (int)block_tables.size(1),
-      kv_fp8_flag(k_cache), (int)waves, (float)scale, cur_stream()));
+      (int)probe, kv_fp8_flag(k_cache), (int)waves, (float)scale, cur_stream()));
   return out;
 }
 
@@ -429,7 +429,7 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
                                     torch::Tensor block_tables,
                                     torch::Tensor seq_lens, int64_t n_parts,
                                     int64_t part_tokens, double scale,
-                                    int64_t waves, bool spread) {
+                                    int64_t waves, bool spread, int64_t probe) {
   CHECK_GPU(q); CHECK_GPU(k_cache); CHECK_GPU(v_cache);
   CHECK_GPU(block_tables); CHECK_GPU(seq_lens);
   int B = (int)q.size(0), qh = (int)q.size(1), d = (int)q.size(2);
@@ -444,8 +444,8 @@ torch::Tensor paged_attention_split(torch::Tensor q, torch::Tensor k_cache,
       block_tables.data_ptr<int32_t>(), seq_lens.data_ptr<int32_t>(),
       out.data_ptr(), part_o.data_ptr<float>(), part_ml.data_ptr<float>(), B,
       qh, kvh, bs, d, (int)block_tables.size(1), (int)n_parts,
-      (int)part_tokens, spread, kv_fp8_flag(k_cache), (int)waves, (float)scale,
-      cur_stream()));
+      (int)part_tokens, spread, (int)probe, kv_fp8_flag(k_cache), (int)waves,
+      (float)scale, cur_stream()));
   return out;
 }
 
@@ -511,13 +511,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_attention", &paged_attention,
         "GQA decode attention over paged KV", py::arg("q"),
         py::arg("k_cache"), py::arg("v_cache"), py::arg("block_tables"),
-        py::arg("seq_lens"), py::arg("scale"), py::arg("waves") = 8);
+        py::arg("seq_lens"), py::arg("scale"), py::arg("waves") = 8,
+        py::arg("probe") = 0);
   m.def("paged_attention_split", &paged_attention_split,
         "flash-decoding GQA attention with sequence partitioning",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),
         py::arg("block_tables"), py::arg("seq_lens"), py::arg("n_parts"),
         py::arg("part_tokens"), py::arg("scale"), py::arg("waves") = 8,
-        py::arg("spread") = false);
+        py::arg("spread") = false, py::arg("probe") = 0);
   m.def("flash_prefill", &flash_prefill,
         "fused MFMA causal varlen prefill attention over paged KV",
         py::arg("q"), py::arg("k_cache"), py::arg("v_cache"),

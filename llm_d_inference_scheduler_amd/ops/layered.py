@@ -3,7 +3,7 @@
 import torch
 
 from . import ref_layered as ref
-from .dispatch import decode_parts, decode_waves
+from .dispatch import decode_parts, decode_probe, decode_waves
 
 try:
     from .. import _hip_layered as _ext
@@ -230,7 +230,8 @@ def grouped_decode(proj, cache, positions, row_seq, block_tables, n, heads,
     far_apart = mean_ctx is not None and max_ctx > apart * mean_ctx
     _impl(proj).grouped_decode(proj, cache, positions, row_seq, block_tables,
                                n, heads, dim, scale, sink, max_ctx, out,
-                               plain, parts, part if far_apart else 0, waves)
+                               plain, decode_probe(max_ctx, mean_ctx, cache.shape[2]),
+                               parts, part if far_apart else 0, waves)
 
 
 def grouped_prefill(proj, cache, positions, row_seq, block_tables, base,

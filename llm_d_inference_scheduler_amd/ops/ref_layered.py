@@ -208,7 +208,7 @@ def _grouped(proj, cache, positions, row_seq, block_tables, lo, hi, heads,
 
 
 def grouped_decode(proj, cache, positions, row_seq, block_tables, n, heads,
-                   dim, scale, sink, max_ctx, out, plain, parts,
+                   dim, scale, sink, max_ctx, out, plain, probe, parts,
                    part_tokens, waves):
     _grouped(proj, cache, positions, row_seq, block_tables, 0, n, heads, dim,
              scale, sink, out)

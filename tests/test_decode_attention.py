@@ -207,6 +207,50 @@ def test_a_little_more_than_a_round(batch, long, fp8):
             _close(dispatch.paged_attention(*args, D ** -0.5, said, m), want)
 
 
+@pytest.mark.parametrize("longest,mean,block,page", [
+    (1500, None, 16, 25), (1500, 1100.0, 16, 22), (8190, 300.0, 16, 6), (40, None, 16, 0),
+    (1500, 1500.0, 5, 100), (1000, 0.0, 16, 0)])
+def test_probe(longest, mean, block, page):
+    assert dispatch.decode_probe(longest, mean, block) == page
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("bs", [16, 5])
+@pytest.mark.parametrize("batch,prefixes", [(2, 1), (7, 3), (65, 64), (66, 65), (150, 4)])
+def test_shared_prefixes(batch, prefixes, bs, fp8):
+    """However values are read, by the page that is looked at, the sums are the same to
+    the bit: rows next to each other that share it, up to 64 and more apart, or none;
+    rows that end before it, and one without tokens."""
+    from llm_d_inference_scheduler_amd import _hip_ops as ext
+    lens = [240 + 37 * i % 90 for i in range(batch)]
+    lens[batch // 2] = 0
+    lens[-1] = 33
+    (q, kc, vc, bt, sl), _ = _case(lens, 4, bs, fp8)
+    kc, vc = (c.float().nan_to_num().to(c.dtype) for c in (kc, vc))
+    for i in range(prefixes, batch):            # the first 180 tokens
+        n = 180 // bs
+        bt[i, :n] = bt[i % prefixes, :n]
+    args, want = (q, kc, vc, bt, sl, D ** -0.5), []
+    for i, n in enumerate(lens):
+        k, v = (c[bt[i].long()].double().permute(1, 0, 2, 3).reshape(KVH, -1, D)[:, :n]
+                for c in (kc, vc))
+        s = q[i].double().view(KVH, 4, D) @ k.transpose(1, 2).contiguous() * D ** -0.5
+        want.append((s.softmax(-1) @ v).view(-1, D).cpu())
+    want = torch.stack(want)
+    for waves in (4, 8):
+        whole = ext.paged_attention(*args, waves=waves, probe=-1)
+        parted = ext.paged_attention_split(*args[:5], 3, 96, args[5], waves=waves,
+                                           spread=True, probe=-1)
+        _close(whole, want)
+        _close(parted, want)
+        for probe in (0, 80 // bs, 180 // bs, 230 // bs, 1 << 20):
+            assert torch.equal(whole, ext.paged_attention(*args, waves=waves,
+                                                          probe=probe))
+            assert torch.equal(parted, ext.paged_attention_split(
+                *args[:5], 3, 96, args[5], waves=waves, spread=True, probe=probe))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("qpg,bs", [(1, 16), (8, 16), (4, 5)])
 @pytest.mark.parametrize("waves", [4, 8])

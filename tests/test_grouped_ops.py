@@ -302,6 +302,32 @@ def test_decode_of_heads_of_128(rep, bs, sink, ctxs, monkeypatch):
     assert ((f64(out) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 4, 70])
+def test_rows_of_one_sequence(rows, monkeypatch):
+    """They read one table: the same bits by whichever page that is found, if at all."""
+    run, G, D, H = ("cuda", torch.bfloat16), 3, 128, 6
+    ctxs = [300, 120]
+    cache, tables, kv = paged(run, G, D, D, ctxs)
+    n = 2 * rows
+    proj = put(rnd(n, H * D, seed=4), run)
+    pos = torch.tensor([c - rows + i for c in ctxs for i in range(rows)],
+                       dtype=torch.int32, device="cuda")
+    seq = torch.tensor([i for i in (0, 1) for _ in range(rows)], dtype=torch.int32,
+                       device="cuda")
+    outs = []
+    for probe in (-1, 0, 6, 9, 1 << 20):
+        monkeypatch.setattr(ops, "decode_probe", lambda *a: probe)
+        outs.append(put(torch.zeros(n, H * D), run))
+        ops.grouped_decode(proj, cache, pos, seq, tables, n, H, D, D ** -0.5, None, 300,
+                           outs[-1])
+    q = f64(proj).view(n, H, D)
+    want = torch.stack([expected(q[i], *kv[i // rows], int(pos[i]), D ** -0.5, None)
+                        for i in range(n)]).view(n, -1)
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    assert ((f64(outs[0]) - want).abs() <= 2 ** -8 * want.abs() + 2e-5).all()
+
+
 @pytest.mark.parametrize("n,longest,mean", [
     (12, 5000, None), (12, 5000, 3400.0), (12, 5000, 2100.0), (12, 5000, 1900.0),
     (33, 900, None), (33, 900, 300.0), (33, 3000, 2500.0), (16, 3000, 2800.0)])
