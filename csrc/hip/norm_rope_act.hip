@@ -358,7 +358,7 @@ hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
                        hipStream_t stream) {
   if (!rows) n = n_rows;
   if (n == 0) return hipSuccess;
-  if (n > 0x7fffffff || n_rows < 1 || (table && (!rows || !residual || parts)))
+  if (n > 0x7fffffff || n_rows < 1 || H < 1 || (table && (!rows || !residual || parts)))
     return hipErrorInvalidValue;
 #define GO(KEEP, RES, PARTS, EARLY, ROWS)                                    \
   hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS, EARLY, ROWS>),        \

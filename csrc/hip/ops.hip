@@ -204,6 +204,7 @@ torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
   TORCH_CHECK(parts || x.dtype() == torch::kBFloat16, "rmsnorm expects bf16");
   TORCH_CHECK(!parts || (x.size(0) > 0 && x.size(2) % 8 == 0 &&
                          w.numel() == x.size(2)), "rmsnorm parts");
+  TORCH_CHECK(x.dim() > 0 && x.size(-1) > 0, "rmsnorm of no channels");
   const int H = (int)x.size(-1);
   const int64_t n_rows = parts ? x.size(1) : x.numel() / H;
   auto opts = x.options().dtype(torch::kBFloat16);
@@ -238,7 +239,7 @@ std::tuple<torch::Tensor, torch::Tensor> embed_rmsnorm(torch::Tensor ids,
                                                        torch::Tensor w, double eps) {
   CHECK_GPU(ids); CHECK_GPU(table); CHECK_GPU(w);
   TORCH_CHECK(ids.dtype() == torch::kInt64 && ids.dim() == 1 && table.dim() == 2 &&
-                  table.dtype() == torch::kBFloat16 && table.size(1) % 8 == 0 &&
+                  table.dtype() == torch::kBFloat16 && table.size(1) > 0 && table.size(1) % 8 == 0 &&
                   (table.size(0) > 0 || ids.numel() == 0) &&
                   w.dtype() == torch::kBFloat16 && w.numel() == table.size(1),
               "embed_rmsnorm");

@@ -591,6 +591,21 @@ def test_norms_of_any_parts(rows, width, parts):
             _same(h, normed(s) * (wn.double() + 0.5), 8)
 
 
+@pytest.mark.parametrize("parts", [0, 2])
+@pytest.mark.parametrize("some", [None, [2, 0]])
+def test_norms_of_no_channels(parts, some):
+    from llm_d_inference_scheduler_amd import ops
+    x = torch.empty(*[parts] * (parts > 0), 3, 0, device="cuda")
+    x, gain = x if parts else x.bfloat16(), torch.empty(0, device="cuda").bfloat16()
+    some = None if some is None else torch.tensor(some, device="cuda")
+    for residual in (None, torch.empty(3, 0, device="cuda").bfloat16()):
+        with pytest.raises(RuntimeError, match="no channels"):
+            ops.rmsnorm(x, gain, 1e-5, residual, some)
+    if some is not None and not parts:
+        with pytest.raises(RuntimeError):
+            ops.embed_rmsnorm(some, x, gain, 1e-5)
+
+
 @pytest.mark.parametrize("parts", [0, 1, 8])
 @pytest.mark.parametrize("rows,width", [(1, 8), (5, 2056), (300, 4096), (3, 4104),
                                         (600, 1024), (2, 16400), (2, 32776)])
