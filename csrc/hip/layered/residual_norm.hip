@@ -6,7 +6,7 @@
 namespace {
 
 constexpr int NT = 256;
-constexpr int PT = 512;  // of rows in parts
+constexpr int PT = 512;  // of rows in parts of more than 256 vectors
 
 template <typename T> struct Eight;
 template <> struct Eight<short> {
@@ -47,14 +47,12 @@ struct Stream {
 //   h = x / rms(x) * (wn + offset)
 //   PARTS: y is in parts, 8 channels per vector; so many of them stay in a thread's
 //   registers, the others' threads keep four. What a row takes is the time of its loads,
-//   one after the other: 512 threads with one vector each, everything that is known ahead
-//   asked for at once (50 rows of 4096 in 8 parts in a pass: 5.3 us; 256 threads, and
-//   weights and rows of experts when they are needed: 7.3).
-template <typename T, int N, int MODE, int PARTS>
-__global__ __launch_bounds__(PARTS ? PT : NT) void stream_norm_kernel(
-    const Stream<T> s) {
+//   one after the other: everything that is known ahead is asked for at once, by as many
+//   threads as there are vectors, up to 512 (50 rows of 4096 in 8 parts in a pass: 5.3 us;
+//   256 threads, and weights and rows of experts when they are needed: 7.3).
+template <typename T, int N, int MODE, int PARTS, int BT>
+__global__ __launch_bounds__(BT) void stream_norm_kernel(const Stream<T> s) {
   static_assert(!PARTS || N == 8, "");
-  constexpr int BT = PARTS ? PT : NT;
   constexpr int KEEP = PARTS ? PARTS : 4;  // vectors kept in registers per thread
   __shared__ float red[2][BT / WAVE];
   const int64_t row = blockIdx.x;
@@ -104,7 +102,7 @@ __global__ __launch_bounds__(PARTS ? PT : NT) void stream_norm_kernel(
       }
 #pragma unroll
     for (int i = 0; i < KEEP; i += 2)
-      if (i * BT * N < H && (i + 1) * BT * N >= H) {     // the last one alone
+      if (KEEP == 1 || (i * BT * N < H && (i + 1) * BT * N >= H)) {  // the last one alone
         const float4v* const src[1] = {
             (const float4v*)(s.yp + row * H + min(at(i), (int64_t)H - N))};
         PartSums<1>(src, (int64_t)gridDim.x * H / 4, s.parts).get(0, keep[i]);
@@ -273,31 +271,38 @@ hipError_t stream_norm_t(int mode, const void* const* p, int64_t rows,
                     (const float*)p[9], (const float*)p[10], (T*)p[11], H,
                     scale, offset, eps};
   const dim3 grid((uint32_t)rows);
-#define GO(N, M, PARTS)                                                       \
-  hipLaunchKernelGGL((stream_norm_kernel<T, N, M, PARTS>), grid,              \
-                     dim3(PARTS ? PT : NT), 0, stream, s)
+#define GO(N, M, PARTS, BT)                                                   \
+  hipLaunchKernelGGL((stream_norm_kernel<T, N, M, PARTS, BT>), grid, dim3(BT), \
+                     0, stream, s)
 #define GOM(N)                                                                \
   do {                                                                        \
-    if (mode == EMBED) GO(N, EMBED, 0);                                   \
-    else if (mode == POST) GO(N, POST, 0);                                \
-    else if (mode == ADD) GO(N, ADD, 0);                                  \
-    else GO(N, LOOP, 0);                                                  \
+    if (mode == EMBED) GO(N, EMBED, 0, NT);                                   \
+    else if (mode == POST) GO(N, POST, 0, NT);                                \
+    else if (mode == ADD) GO(N, ADD, 0, NT);                                  \
+    else GO(N, LOOP, 0, NT);                                                  \
   } while (0)
-  // Past 256 rows enough is under way, and what is asked for ahead takes the registers
-  // of other rows (1300 rows of 4096 in 2 parts: 18.2 us with it, 16.1 without; 300 in 8
-  // parts 11.3 and 10.5; 256 rows of 3072 in 8 parts 5.9 and 6.5), nor is there anything
-  // to ask for ahead in short rows (1024 in 8 parts: 3.7 and 3.5).
-  if (parts && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256 &&
-      H >= NT * 8) {
-    if (mode == POST && H <= PT * 8) GO(8, POST, 1);
-    else if (mode == POST) GO(8, POST, 2);
-    else if (H <= PT * 8) GO(8, ADD, 1);
-    else GO(8, ADD, 2);
+#define GOP(PARTS, BT)                                                        \
+  do {                                                                        \
+    if (mode == POST) GO(8, POST, PARTS, BT); else GO(8, ADD, PARTS, BT);     \
+  } while (0)
+  // Ahead, up to 256 rows: past them enough is under way, and of two vectors what is
+  // asked for takes the registers of other rows. us, not ahead / by 512 threads / by 256
+  // threads, 8 parts, with a norm of the sum and four rows of experts:
+  //              1 row              50 rows             256 rows            300 rows
+  //   1024   4.2 / 4.2 / 3.6     4.7 / 4.5 / 3.9     6.8 / 5.8 / 5.1     7.2 / 7.2 / 5.8
+  //   2048   4.5 / 4.2 / 3.6     6.1 / 5.0 / 4.3     7.9 / 7.3 / 6.7     8.6 / 9.0 / 7.7
+  //   4096   6.6 / 4.4 / 5.8     9.9 / 5.8 / 8.3    12.6 /10.4 /12.0    14.1 /12.7 /13.9
+  //   5120   8.4 / 6.7          13.5 / 9.0          16.1 /13.5          18.1 /20.4
+  if (parts && H > 0 && H % 8 == 0 && (mode == POST || mode == ADD) && rows <= 256) {
+    if (H <= NT * 8) GOP(1, NT);
+    else if (H <= PT * 8) GOP(1, PT);
+    else GOP(2, PT);
   } else if (H % 8 == 0) {
     GOM(8);
   } else {
     GOM(1);
   }
+#undef GOP
 #undef GOM
 #undef GO
   HIP_CHECK_LAST();

@@ -16,36 +16,46 @@ namespace {
 //   y = src * rsqrt(mean(src^2) + eps) * w
 // x is bf16, or the partial sums of a product that split K: [parts, rows, H]
 // 32-bit, summed here instead of by a launch of their own (8 parts, one row of
-// 4096: 4.1 us, 6.5 with few loads under way; sum and norm apart 8.7; 30 rows of
-// 5120 4.9, were 7.6, 256 of 4096 8.7, were 9.6).
-// One block per token row, of 256 threads, or 512 where the row is in parts: most of
-// its time is the loads' way, and so each thread has half of them (30 rows of 5120 5.5
-// us by 256 threads). Row length H % 8 == 0. The first KEEP
+// 4096: sum and norm apart 8.7 us, so 4.1).
+// One block per token row, of 256 threads, or 512 where the row is in parts and has
+// more than 256 vectors of 8: most of its time is the loads' way, and so each thread has
+// half of them. Row length H % 8 == 0. The first KEEP
 // vectors of a thread stay in registers between the two passes, the rest are
 // read again. Their number is known at compile time: an index that is not puts
 // the array into scratch memory (8013 rows of 4096 with residual: 84 us, now
 // 44, 5.9 TB/s).
 // ---------------------------------------------------------------------------
 constexpr int NT = 256;
-constexpr int PT = 512;        // of a row in parts
+constexpr int PT = 512;
 
-// EARLY: with parts, all that a thread keeps is asked for at once, pair by pair. Not
-// past 512 rows (256 where a thread has one vector): other rows' loads are under way
-// anyway, and what a pair reads past the row's end costs more than the wait (600 rows
-// of 5120 in 3 parts: 11.1 us, without 10.1; 400 rows in 4 parts 8.3 and 8.7; 257 rows of
-// 2048 in 14 parts 6.1 and 5.6).
+// EARLY: with parts, all that a thread keeps is asked for at once, pair by pair. Up to
+// 2048 channels always; above up to 512 rows where a thread has one vector, 256 where it
+// has two, the second of which reads past the row's end. us, with residual, parts and
+// residual in the caches, 512 threads early / not, 256 early / not:
+//             rows      2 parts                   8 parts
+//   1024         1   2.2  2.3  2.2  2.3      2.9  2.7  2.5  2.7
+//              256   2.6  2.7  2.5  2.7      4.3  4.6  3.9  4.6
+//              640   4.8  4.1  3.9  4.0      7.3  6.3  5.9  6.2
+//   2048         1   2.3  2.4  2.2  2.3      3.0  2.8  2.6  2.8
+//              256   3.5  3.7  3.4  3.7      5.5  5.6  5.1  5.6
+//              640   5.6  5.2  4.9  5.2      9.4  9.5  9.0  9.5
+//   4096         1   2.4  2.5  2.7  3.0      3.2  3.2  3.6  4.0
+//              256   4.4  4.6  4.7  5.1      7.8  8.0  8.0  8.6
+//              512   6.4  6.6  6.8  6.8     13.2 13.2 13.3 13.6
+//   5120         1   3.0  3.1  3.2  3.7      4.4  4.1  4.9  5.1
+//              256   5.3  5.5  5.6  6.2      9.3  9.9  9.8 10.7
+//              400   7.8  7.1  7.0  7.5     14.3 13.5 13.7 13.8
 // ROWS: ALL of them; PICKED: the rows that `rows` names, of n_rows, without a word to
 // the residual; TABLE: rows of the table x that `rows` names (token ids), which become the
 // residual. As in an index, rows below 0 count from the end. Rows that do not exist are
 // NaN throughout: never another row's values.
 enum Rows { ALL, PICKED, TABLE };
 
-template <int KEEP, bool RESIDUAL, bool PARTS, bool EARLY, int ROWS>
-__global__ __launch_bounds__(PARTS ? PT : NT) void rmsnorm_kernel(
+template <int BT, int KEEP, bool RESIDUAL, bool PARTS, bool EARLY, int ROWS>
+__global__ __launch_bounds__(BT) void rmsnorm_kernel(
     const void* __restrict__ x, int parts, short* __restrict__ residual,
     const short* __restrict__ w, short* __restrict__ y, int H, float eps,
     const int64_t* __restrict__ rows, int64_t n_rows) {
-  constexpr int BT = PARTS ? PT : NT;
   __shared__ float red[BT / WAVE];
   int64_t row = blockIdx.x;
   if constexpr (ROWS != ALL) {
@@ -360,33 +370,37 @@ hipError_t lds_rmsnorm(const void* x, int parts, void* residual, const void* w,
   if (n == 0) return hipSuccess;
   if (n > 0x7fffffff || n_rows < 1 || H < 1 || (table && (!rows || !residual || parts)))
     return hipErrorInvalidValue;
-#define GO(KEEP, RES, PARTS, EARLY, ROWS)                                    \
-  hipLaunchKernelGGL((rmsnorm_kernel<KEEP, RES, PARTS, EARLY, ROWS>),        \
-                     dim3((uint32_t)n), dim3(PARTS ? PT : NT), 0, stream, x, \
-                     parts, (short*)residual, (const short*)w, (short*)y, H, \
-                     eps, rows, n_rows)
-#define GO_K(RES, PARTS, EARLY, ROWS)                                        \
+#define GO(BT, KEEP, RES, PARTS, EARLY, ROWS)                                \
+  hipLaunchKernelGGL((rmsnorm_kernel<BT, KEEP, RES, PARTS, EARLY, ROWS>),    \
+                     dim3((uint32_t)n), dim3(BT), 0, stream, x, parts,       \
+                     (short*)residual, (const short*)w, (short*)y, H, eps,   \
+                     rows, n_rows)
+#define GO_K(BT, RES, PARTS, EARLY, ROWS)                                    \
   do {                                                                       \
-    const int each = (PARTS ? PT : NT) * 8;                                  \
-    if (H <= each) GO(1, RES, PARTS, EARLY, ROWS);                           \
-    else if (H <= 2 * each) GO(2, RES, PARTS, EARLY, ROWS);                  \
-    else GO(4, RES, PARTS, EARLY, ROWS);                                     \
+    if (H <= BT * 8) GO(BT, 1, RES, PARTS, EARLY, ROWS);                     \
+    else if (H <= 2 * BT * 8) GO(BT, 2, RES, PARTS, EARLY, ROWS);            \
+    else GO(BT, 4, RES, PARTS, EARLY, ROWS);                                 \
   } while (0)
-  const bool early = n <= (H <= NT * 8 ? 256 : 512);
+#define GO_P(RES, ROWS)                                                      \
+  do {                                                                       \
+    if (H <= NT * 8) GO(NT, 1, RES, true, true, ROWS);                       \
+    else if (n <= (H <= PT * 8 ? 512 : 256)) GO_K(PT, RES, true, true, ROWS); \
+    else GO_K(PT, RES, true, false, ROWS);                                   \
+  } while (0)
   if (table) {
-    GO_K(false, false, false, TABLE);
+    GO_K(NT, false, false, false, TABLE);
   } else if (rows && parts > 0) {
-    if (residual) GO_K(true, true, true, PICKED); else GO_K(false, true, true, PICKED);
+    if (residual) GO_P(true, PICKED); else GO_P(false, PICKED);
   } else if (rows) {
-    if (residual) GO_K(true, false, false, PICKED);
-    else GO_K(false, false, false, PICKED);
-  } else if (parts > 0 && early) {
-    if (residual) GO_K(true, true, true, ALL); else GO_K(false, true, true, ALL);
+    if (residual) GO_K(NT, true, false, false, PICKED);
+    else GO_K(NT, false, false, false, PICKED);
   } else if (parts > 0) {
-    if (residual) GO_K(true, true, false, ALL); else GO_K(false, true, false, ALL);
+    if (residual) GO_P(true, ALL); else GO_P(false, ALL);
   } else {
-    if (residual) GO_K(true, false, false, ALL); else GO_K(false, false, false, ALL);
+    if (residual) GO_K(NT, true, false, false, ALL);
+    else GO_K(NT, false, false, false, ALL);
   }
+#undef GO_P
 #undef GO_K
 #undef GO
   HIP_CHECK_LAST();

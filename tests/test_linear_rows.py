@@ -654,6 +654,21 @@ def test_norms_of_rows_that_do_not_exist(rows, width, parts):
             assert torch.equal(got[there], want) and got[gone].isnan().all()
 
 
+@pytest.mark.parametrize("width", [8, 1032, 2040, 2048])
+@pytest.mark.parametrize("rows", [1, 300])
+def test_norm_of_one_part(rows, width):
+    """Rows of up to 256 vectors have 256 threads in parts too: to the bit what rows in
+    bf16 come out as."""
+    hip = _ext("_hip_ops")
+    x, gain, start = (_draw(rows, width, seed=2), _draw(width, seed=3),
+                      _draw(rows, width, seed=4))
+    for residual in (None, start):
+        a, b = (None if residual is None else residual.clone() for _ in range(2))
+        assert torch.equal(hip.rmsnorm(x.float()[None], gain, 1e-5, a),
+                           hip.rmsnorm(x, gain, 1e-5, b))
+        assert residual is None or torch.equal(a, b)
+
+
 @pytest.mark.parametrize("width", [1032, 2056, 4104, 8200])
 @pytest.mark.parametrize("few,many,parts", [(256, 257, 9), (512, 513, 2)])
 def test_norms_of_parts_of_many_rows(few, many, parts, width):
