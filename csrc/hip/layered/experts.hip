@@ -412,9 +412,9 @@ hipError_t launch_rows(Pairs p, int max_tiles, int tiles, hipStream_t stream) {
 // us, 1366 with 3).
 constexpr int TC = 256, BK = TILE_K, HALF = 128;
 constexpr int TG = 4;                // tiles of pairs that run side by side
-typedef TileCore<8, 8, 2, 2> Whole;
-typedef TileCore<8, 6, 2, 2> Most;   // 192 pairs
-typedef TileCore<4, 8, 4, 2> Half;
+typedef TileCore<8, 8, 2> Whole;
+typedef TileCore<8, 6, 2> Most;   // 192 pairs
+typedef TileCore<4, 8, 4> Half;
 static_assert(Whole::CHANNELS == TC && Most::CHANNELS == TC && Half::CHANNELS == TC &&
                   Whole::ROWS == TILE && Half::ROWS == HALF &&
                   Most::LDS_TURN <= Whole::LDS_TURN &&

@@ -12,8 +12,8 @@
 
 namespace {
 
-template <int PT> using Whole = TileCore<8, PT, 2, 2>;    // 32 PT rows
-typedef TileCore<4, 8, 4, 2> Half;       // the last tile, of up to 128
+template <int PT> using Whole = TileCore<8, PT, 2>;    // 32 PT rows
+typedef TileCore<4, 8, 4> Half;       // the last tile, of up to 128
 constexpr int BC = Whole<8>::CHANNELS;
 static_assert(Half::CHANNELS == BC && Half::CH == Whole<8>::CH &&
                   Half::LDS_TURN <= Whole<6>::LDS_TURN,

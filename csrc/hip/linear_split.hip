@@ -25,7 +25,7 @@ struct Product {
 
 template <int PT>
 __global__ __launch_bounds__(256, 1) void linear_split_kernel(const Product p) {
-  typedef TileCore<8, PT, 2, 2> Core;
+  typedef TileCore<8, PT, 2> Core;
   constexpr int LW = Core::LW, LP = Core::LP, BR = Core::ROWS;
   static_assert(Core::CHANNELS == BC, "");
   extern __shared__ __align__(16) short split_lds[];
@@ -74,7 +74,7 @@ __global__ __launch_bounds__(256, 1) void linear_split_kernel(const Product p) {
 
 template <int PT>
 hipError_t go(const Product& p, hipStream_t stream) {
-  typedef TileCore<8, PT, 2, 2> Core;
+  typedef TileCore<8, PT, 2> Core;
   const int64_t n = (int64_t)((p.N + BC - 1) / BC) *
                     ((p.M + Core::ROWS - 1) / Core::ROWS) * p.parts;
   if (n > 1 << 24) return hipErrorInvalidValue;

@@ -37,8 +37,8 @@ constexpr int BUFFER_BYTES = 0x00027000;
 constexpr int TILE_K = 64;              // K of a step
 
 // CT x PT results of 16 x 16 per wave, WC waves across the channels, the others
-// across the rows; a ring of RS steps.
-template <int CT, int PT, int WC, int RS>
+// across the rows.
+template <int CT, int PT, int WC>
 struct TileCore {
   static constexpr int QC = CT / 2, QP = PT / 2;   // of a quarter
   static constexpr int WP = 4 / WC;
@@ -46,9 +46,9 @@ struct TileCore {
   static constexpr int CH = CHANNELS / 2, RH = ROWS / 2;   // of a half
   // 8 rows per load; loads of a wave and half
   static constexpr int LW = CH / 32, LP = RH / 32;
-  static_assert(CH % 32 == 0 && RH % 32 == 0 && RS >= 2, "");
+  static_assert(CH % 32 == 0 && RH % 32 == 0, "");
   static constexpr int STEP = (CHANNELS + ROWS) * TILE_K;
-  static constexpr int RING = RS * STEP;
+  static constexpr int RING = 2 * STEP;
   // results that a wave turns round at a time: 32 rows
   static constexpr int TURN = 32 * 16 * CT;
   static constexpr int LDS = RING * (int)sizeof(short);
@@ -116,8 +116,9 @@ struct TileCore {
                                                       BUFFER_BYTES),
                     __builtin_amdgcn_readfirstlane(in ? at(s) : 0)};
     };
-    // load j of half i of a step of parity par to the step at `base`
-    auto load = [&](const Source& s, int par, int i, int base, int j) {
+    // load j of half i of a step of parity par
+    auto load = [&](const Source& s, int par, int i, int j) {
+      const int base = par * STEP;
       if (i % 3 == 0)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
             s.w, (smem*)(wdst + base + place[i] + j * 8 * TILE_K), 16,
@@ -128,13 +129,13 @@ struct TileCore {
             asrc[i == 1 ? par : 1 - par][j], s.k, 0, 0);
     };
 #pragma unroll
-    for (int s = 0; s < RS; ++s) {
+    for (int s = 0; s < 2; ++s) {
       const Source from = source(s);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < (i % 3 ? LP : LW); ++j)
-          load(from, s % 2, i, s * STEP, j);
+          load(from, s, i, j);
     }
 
 #pragma unroll
@@ -142,43 +143,38 @@ struct TileCore {
 #pragma unroll
       for (int t = 0; t < PT; ++t) acc[c][t] = (float4v){0.f, 0.f, 0.f, 0.f};
     bf16x8 wf[2][2][QC], af[2][2][QP];     // [half][32 of K][16 rows]
-    // pieces 4 kk + grp; the second step of a ring of two from addresses of its
-    // own (an LDS read has 16 bits of offset)
-    constexpr int U = RS == 2 ? 2 : 1;
-    const short *wl[U][2], *al[U][2];
+    // pieces 4 kk + grp; the second step of the ring from addresses of its own (an
+    // LDS read has 16 bits of offset)
+    const short *wl[2][2], *al[2][2];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       const int p = ((kk * 4 + grp) ^ (col / 2 & 7)) * 8;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
+      for (int u = 0; u < 2; ++u) {
         wl[u][kk] = lds + u * STEP + (wc * 16 * QC + col) * TILE_K + p;
         al[u][kk] = lds + u * STEP + (wp * 16 * QP + col) * TILE_K + p;
       }
     }
-    // read x of half i of the step at `base` (of a ring of two: step u)
-    auto read_w = [&](int h, int u, int base, int x) {
+    // read x of half i of step u of the ring
+    auto read_w = [&](int h, int u, int x) {
       wf[h][x / QC][x % QC] = *(const bf16x8*)(
-          wl[U == 2 ? u : 0][x / QC] + (U == 2 ? 0 : base) + place[h * 3] +
-          x % QC * 16 * TILE_K);
+          wl[u][x / QC] + place[h * 3] + x % QC * 16 * TILE_K);
     };
-    auto read_a = [&](int h, int i, int u, int base, int x) {
+    auto read_a = [&](int h, int i, int u, int x) {
       af[h][x / QP][x % QP] = *(const bf16x8*)(
-          al[U == 2 ? u : 0][x / QP] + (U == 2 ? 0 : base) + place[i] +
-          x % QP * 16 * TILE_K);
+          al[u][x / QP] + place[i] + x % QP * 16 * TILE_K);
     };
     // the first two halves into registers
-    asm volatile("s_waitcnt vmcnt(%0)" ::"i"((2 * RS - 1) * (LW + LP))
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"(3 * (LW + LP))
                  : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int x = 0; x < 2 * QC; ++x) read_w(0, 0, 0, x);
+    for (int x = 0; x < 2 * QC; ++x) read_w(0, 0, x);
 #pragma unroll
-    for (int x = 0; x < 2 * QP; ++x) read_a(0, 1, 0, 0, x);
+    for (int x = 0; x < 2 * QP; ++x) read_a(0, 1, 0, x);
 
-    // base, next: where this step and the one after it lie
-    auto phase = [&](auto par_, auto i_, const Source& from, int base,
-                     int next) {
+    auto phase = [&](auto par_, auto i_, const Source& from) {
       constexpr int par = decltype(par_)::value, i = decltype(i_)::value;
       constexpr int hw = i / 2, ha = i % 3 ? 1 - par : par;
       constexpr int n = 2 * QC * QP;                   // matrix instructions
@@ -186,8 +182,8 @@ struct TileCore {
       constexpr int reads = channels ? 2 * QC : 2 * QP;
       constexpr int loads = i % 3 ? LP : LW;
       // The barrier of phases 0 and 2 lets this and the next one read and load:
-      // every wave has what the loads of halves i + 2 and i + 3 brought in (the
-      // others of a ring are on their way), and has read halves i and i + 1. It
+      // every wave has what the loads of halves i + 2 and i + 3 brought in (those
+      // after them are on their way), and has read halves i and i + 1. It
       // comes after some instructions, which wait for the last reads piece by
       // piece.
       constexpr int ahead = i % 2 ? 0 : n / 4;
@@ -199,7 +195,7 @@ struct TileCore {
       for (int m = 0; m < n; ++m) {
         if (i % 2 == 0 && m == ahead) {
           asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(
-                           (2 * RS - 2) * (LW + LP))
+                           2 * (LW + LP))
                        : "memory");
           __builtin_amdgcn_s_barrier();
           asm volatile("" ::: "memory");
@@ -224,27 +220,23 @@ struct TileCore {
                        : "+a"(d) : "v"(w), "v"(a));
         const int x = m - ahead;
         if (x >= 0 && x % every == 0 && x / every < reads) {
-          if (i == 0) read_a(1 - par, 2, par, base, x / every);
-          if (i == 1) read_w(1, par, base, x / every);
-          if (i == 2) read_w(0, 1 - par, next, x / every);
-          if (i == 3) read_a(1 - par, 1, 1 - par, next, x / every);
+          if (i == 0) read_a(1 - par, 2, par, x / every);
+          if (i == 1) read_w(1, par, x / every);
+          if (i == 2) read_w(0, 1 - par, x / every);
+          if (i == 3) read_a(1 - par, 1, 1 - par, x / every);
         }
         if (x >= 0 && x % apart == apart - 1 && x / apart < loads)
-          load(from, (par + RS) % 2, i, base, x / apart);
+          load(from, par, i, x / apart);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    int s = 0, base = 0;
+    int s = 0;
     auto step = [&](auto par) {
-      const Source from = source(s + RS);
-      const int here = RS == 2 ? par * STEP : base;
-      const int next = RS == 2 ? STEP - here : here + STEP == RING ? 0
-                                                                   : here + STEP;
-      phase(par, integral_constant<int, 0>{}, from, here, next);
-      phase(par, integral_constant<int, 1>{}, from, here, next);
-      phase(par, integral_constant<int, 2>{}, from, here, next);
-      phase(par, integral_constant<int, 3>{}, from, here, next);
-      base = next;
+      const Source from = source(s + 2);
+      phase(par, integral_constant<int, 0>{}, from);
+      phase(par, integral_constant<int, 1>{}, from);
+      phase(par, integral_constant<int, 2>{}, from);
+      phase(par, integral_constant<int, 3>{}, from);
       ++s;
     };
     while (s + 1 < steps) {
