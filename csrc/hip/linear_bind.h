@@ -76,7 +76,8 @@ enum Use { PLAIN, GATED, PARTS };
 inline bool few_rows(const Tensor& x, const Tensor& w, Use use) {
   if (!plain_matrices(x, w)) return false;
   const int64_t M = x.size(0), K = x.size(1), N = w.size(0), limit = 1ll << 31;
-  // gated ones of more rows have one kernel, whose offsets stay under 4 GiB
+  // gated ones of more rows have one kernel, which goes by lines: its offsets stay
+  // under 4 GiB
   const bool near = use != GATED || M <= 192;
   return M >= 1 && M <= 256 && K >= 8 && K % 8 == 0 && N >= 8 && N % 8 == 0 &&
          N <= (1 << 24) && K <= (1 << 24) && (use != GATED || N % 16 == 0) &&

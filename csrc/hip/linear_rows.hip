@@ -438,13 +438,14 @@ hipError_t lds_sum_parts(const float* part, void* y, int64_t n, int parts,
   return hipSuccess;
 }
 
-// x [M, K], w [N, K], rows x_row and w_row apart and 16-byte aligned; y [M, N]
+// x [M, K], w [N, K], rows x_row and w_row apart and 16-byte aligned, N a multiple of 8; y
+// [M, N]
 // bf16 or (f32) 32-bit. part: [parts, M, N] floats if parts > 1; without y
 // the result stays there.
 hipError_t lds_linear_rows(const void* x, int64_t x_row, const void* w,
                            int64_t w_row, void* y, float* part, int parts,
                            int M, int N, int K, int f32, hipStream_t stream) {
-  if (M < 1 || M > TILE_ROWS || N < 1 || N % 4 || K < 8 || K % 8 ||
+  if (M < 1 || M > TILE_ROWS || N < 1 || N % 8 || K < 8 || K % 8 ||
       x_row % 8 || w_row % 8 || parts < 1 || (!part && (parts > 1 || !y)))
     return hipErrorInvalidValue;
   const bool in_part = parts > 1 || !y;
@@ -475,11 +476,11 @@ hipError_t lds_lay_weights(const float* in, void* out, int R, int C,
   return hipSuccess;
 }
 
-// y [M, N] = act(x gate') * (x up'), w [2 N, K] = [gate; up]
+// y [M, N] = act(x gate') * (x up'), w [2 N, K] = [gate; up], N a multiple of 8
 hipError_t lds_gated_rows(const void* x, int64_t x_row, const void* w,
                           int64_t w_row, void* y, int M, int N, int K, int act,
                           hipStream_t stream) {
-  if (M < 1 || M > TILE_ROWS || N < 1 || N % 4 || K < 8 || K % 8 ||
+  if (M < 1 || M > TILE_ROWS || N < 1 || N % 8 || K < 8 || K % 8 ||
       x_row % 8 || w_row % 8 || act < 0 || act >= ACTS)
     return hipErrorInvalidValue;
   if (M > ROWS)

@@ -508,14 +508,16 @@ hipError_t go_rows(Tiles p, hipStream_t stream) {
     if (p.M <= 64) return go<1, OUT, false>(p, stream);
   if (p.M <= 128) return go<2, OUT, false>(p, stream);
   if (p.M <= 192) return go<3, OUT, false>(p, stream);
-  return go<4, OUT, false>(p, stream);
+  if constexpr (OUT == GATED) return hipErrorInvalidValue;
+  else return go<4, OUT, false>(p, stream);
 }
 
 }  // namespace
 
 // x [M, K], w [N, K], rows x_row and w_row apart and 16-byte aligned, up
 // to 256 rows, N a multiple of 8; y [M, N] bf16, or (f32) [parts, M, N]
-// 32-bit. act >= 0: y [M, N] = act(x gate') * (x up'), w [2 N, K].
+// 32-bit. act >= 0: y [M, N] = act(x gate') * (x up'), w [2 N, K]; of more than 192
+// rows for K in whole steps of 128 from 1024 on and operands of less than 4 GiB.
 extern "C" hipError_t lds_linear_tiles(const void* x, int64_t x_row,
                                        const void* w, int64_t w_row, void* y,
                                        int parts, int M, int N, int K, int f32,
