@@ -220,8 +220,8 @@ __global__ __launch_bounds__(256) void head_products_kernel(const HeadProducts p
   float4v acc[KW];
 #pragma unroll
   for (int c = 0; c < KW; ++c) acc[c] = (float4v){0.f, 0.f, 0.f, 0.f};
-  // past the end of K the rows count as zero; rows and channels past the end repeat the
-  // last one
+  // past the end of K both count as zero (a weight may be infinite); rows and channels
+  // past the end repeat the last one
   for (int k0 = kw * 128; k0 < K; k0 += KW * 128) {
     short8 a[4], b[KW][4];
     const int k = k0 + col * 8, kc = min(k, K - 8);
@@ -237,7 +237,11 @@ __global__ __launch_bounds__(256) void head_products_kernel(const HeadProducts p
     __builtin_amdgcn_sched_barrier(0);       // all loads ahead of their first use
     if (k >= K)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a[j] = zero;
+      for (int j = 0; j < 4; ++j) {
+        a[j] = zero;
+#pragma unroll
+        for (int c = 0; c < KW; ++c) b[c][j] = zero;
+      }
     to_operand(mine, lane, a);
 #pragma unroll
     for (int c = 0; c < KW; ++c) {

@@ -704,3 +704,20 @@ def test_head_products(T, H, N, K, by_head):
         assert ops.head_products(put(rnd(T, H, K + 4), run)[:, :, :K], w, y) == (
             (K + 4) % 8 == 0)
     assert not ops.head_products(x.float(), w.float(), y.float())
+
+
+@GPU
+@pytest.mark.parametrize("K", [8, 72, 136, 200, 264, 1032])
+def test_head_products_without_end(K):
+    """Infinite weights and rows at the end of K, where a step has nothing left: infinity
+    in what they reach and nowhere else."""
+    run, T, H, N, inf = ("cuda:0", torch.bfloat16), 17, 2, 72, float("inf")
+    x = put(rnd(T, H, K, seed=1), run)
+    w = put(rnd(H, N, K, seed=2, scale=K ** -0.5), run)
+    w[0, 3, K - 1] = w[0, N - 1, K - 8] = inf
+    w[1, 40, K - 1] = -inf
+    x[5, 1, K - 2] = x[T - 1, 0, K - 3] = inf
+    y = put(torch.zeros(T, H, N), run)
+    assert ops.head_products(x, w, y)
+    want = torch.stack([f64(x)[:, h] @ f64(w)[h].T for h in range(H)], 1)
+    torch.testing.assert_close(f64(y), want, rtol=2 ** -8, atol=1e-5, equal_nan=True)
