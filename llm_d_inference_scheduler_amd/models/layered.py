@@ -202,7 +202,8 @@ class LatentAttention:
             1, 2).contiguous()
         # and with a channel's weights together, for few rows
         self.rows_uk = self.w_uk.transpose(1, 2).contiguous()
-        self.rows_uv = uv.view(spec.heads, spec.vdim, spec.kv_rank)
+        self.rows_uv = self.w_ukv[uk.shape[0]:].view(spec.heads, spec.vdim,
+                                                     spec.kv_rank)
 
     def __call__(self, h: torch.Tensor, batch: LayeredBatch, cache,
                  ctx) -> torch.Tensor:
