@@ -211,7 +211,8 @@ torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor w, double eps,
   torch::Tensor y;
   if (rows.has_value()) {
     CHECK_GPU(*rows);
-    TORCH_CHECK(rows->dtype() == torch::kInt64 && rows->dim() == 1 &&
+    TORCH_CHECK(rows->device() == x.device() && rows->dtype() == torch::kInt64 &&
+                    rows->dim() == 1 &&
                     (n_rows > 0 || rows->numel() == 0) && w.numel() == H &&
                     H % 8 == 0 && (parts || x.dim() == 2),
                 "rmsnorm rows");
@@ -238,7 +239,8 @@ std::tuple<torch::Tensor, torch::Tensor> embed_rmsnorm(torch::Tensor ids,
                                                        torch::Tensor table,
                                                        torch::Tensor w, double eps) {
   CHECK_GPU(ids); CHECK_GPU(table); CHECK_GPU(w);
-  TORCH_CHECK(ids.dtype() == torch::kInt64 && ids.dim() == 1 && table.dim() == 2 &&
+  TORCH_CHECK(ids.device() == table.device() && w.device() == table.device() &&
+                  ids.dtype() == torch::kInt64 && ids.dim() == 1 && table.dim() == 2 &&
                   table.dtype() == torch::kBFloat16 && table.size(1) > 0 && table.size(1) % 8 == 0 &&
                   (table.size(0) > 0 || ids.numel() == 0) &&
                   w.dtype() == torch::kBFloat16 && w.numel() == table.size(1),

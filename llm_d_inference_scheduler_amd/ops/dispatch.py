@@ -64,8 +64,10 @@ def gated_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 _SILU = 1       # activation code of the kernels
 
 
-def _index(t: torch.Tensor) -> bool:
-    return t.dim() == 1 and t.dtype == torch.int64 and t.is_contiguous()
+def _index(t: torch.Tensor, of: torch.Tensor) -> bool:
+    """Whether the kernels take t as an index into rows of `of`."""
+    return t.device == of.device and t.dim() == 1 and \
+        t.dtype == torch.int64 and t.is_contiguous()
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
@@ -75,8 +77,7 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float,
     left open then. A row that x does not have raises IndexError on the CPU and
     comes out as NaN on the GPU."""
     if _use_hip(x):
-        if rows is None or (rows.is_cuda and _index(rows) and
-                            x.shape[-1] % 8 == 0):
+        if rows is None or (_index(rows, x) and x.shape[-1] % 8 == 0):
             return _ext.rmsnorm(x, w, eps, residual, rows)
         return _ext.rmsnorm(x, w, eps, residual)[rows]
     y = ref.rmsnorm(x, w, eps, residual)
@@ -87,7 +88,7 @@ def embed_rmsnorm(ids: torch.Tensor, table: torch.Tensor, w: torch.Tensor,
                   eps: float):
     """-> table[ids] and its norm. An id that the table does not have raises
     IndexError on the CPU; on the GPU both of its rows come out as NaN."""
-    if _use_hip(table) and ids.is_cuda and _index(ids) and \
+    if _use_hip(table) and _index(ids, table) and table.is_contiguous() and \
             table.dtype == torch.bfloat16 and table.shape[1] % 8 == 0:
         return _ext.embed_rmsnorm(ids, table, w, eps)
     x = table[ids]

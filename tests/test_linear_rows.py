@@ -772,3 +772,14 @@ def test_rows_come_out_alike(n, k):
             y = ext.gated_linear(x[:rows], w, 1)
             assert (y is None) == (one is None)
             assert y is None or torch.equal(y[:1], one)
+
+
+def test_rows_of_a_table_that_is_a_view():
+    """As an index takes them."""
+    from llm_d_inference_scheduler_amd import ops
+    table, gain = _draw(50, 64)[::2, :40], _draw(40, seed=3)
+    ids = torch.tensor([24, 0, -1], device="cuda")
+    for some in (ids, ids.int(), ids.repeat(2)[::2]):
+        rows, normed = ops.embed_rmsnorm(some, table, gain, 1e-5)
+        assert torch.equal(rows, table[some])
+        assert torch.equal(normed, ops.rmsnorm(table[some], gain, 1e-5))

@@ -38,3 +38,12 @@ def test_gated(n, k, rows):
     (16384, 5120, EVERY)])
 def test_one_part(n, k, rows):
     assert [m for m in EVERY if RULES.lds_linear_plain_parts(m, n, k) == 1] == list(rows)
+
+
+def test_an_index_of_another_device_is_no_index():
+    """The kernels read one by its address; torch's own says what is wrong with it."""
+    from llm_d_inference_scheduler_amd.ops.dispatch import _index
+    table, ids = torch.zeros(4, 8), torch.zeros(6, dtype=torch.int64)
+    assert _index(ids, table)
+    for other in (ids.to("meta"), ids.int(), ids[::2], ids.view(2, 3)):
+        assert not _index(other, table)
