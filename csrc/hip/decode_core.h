@@ -38,8 +38,8 @@
 // 4100, 4000 shared: 73).
 //
 // Measured alone, cold (8 key heads, ragged; before: P V on the 32-bit cores): 256
-// sequences of 1500 tokens, groups of 4: 269 us, 5.8 TB/s (279), fp8 156 us, 5.0 TB/s
-// (191), 137 by 4 waves; 30 of 1100, groups of 8: 27.5 us (31.5); 17 of 6800, fp8, in 4
+// sequences of 1500 tokens, groups of 4: 252 us, 6.2 TB/s (279), fp8 156 us (191), by 4
+// waves 142, 5.5 TB/s; 30 of 1100, groups of 8: 27.5 us (31.5); 17 of 6800, fp8, in 4
 // partitions by 8 waves: 51 us, 4.5 TB/s (66.5; with its sum 56.6, in 6 by 4 waves 50.6);
 // 60 of 300: 15.7 us (19.9); one of 777: 9.3 us (10.3). Registers let a compute unit have
 // 12 waves: one workgroup of 8 or three of 4. One of 12 is no faster.
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(NW * WAVE, 3) void decode_attention_kernel(
   };
 
   // ENDLESS: infinite values are no part of the lower products; no tile is read
-  // ahead, which would take more registers than there are. PAST: values are read past the
+  // ahead, which would take more registers than there are. past: values are read past the
   // caches.
   const int t_first = t_begin + wave * TILE;
   auto walk = [&](auto endless, auto past) {       // !ENDLESS: with the first tile's pages
